@@ -260,6 +260,11 @@ int mmf_hgrn_gate_bwd(const void* i_in, int64_t ldi, const void* f_in, int64_t l
  *   exp(g_t) and dg_t = dh h_{t-1} exp(g_t).  As in the reference the gradient of the final state is not propagated. */
 int mmf_hgrn_recurrent_bwd(const void* g, const void* o, const void* grad_o, const float* h0, void* dx, void* dg, int64_t BH,
                            int64_t T, int64_t D, int log_gates, int dtype, void* stream);
+/* The same with a workspace of mmf_hgrn_recurrent_bwd_workspace_bytes(BH, T, D) bytes (fp32, 0 bytes: may be NULL): a long
+ *   sequence of few channels is then cut into time segments that run in parallel. */
+int64_t mmf_hgrn_recurrent_bwd_workspace_bytes(int64_t BH, int64_t T, int64_t D);
+int mmf_hgrn_recurrent_bwd_split(const void* g, const void* o, const void* grad_o, const float* h0, void* dx, void* dg, int64_t BH,
+                                 int64_t T, int64_t D, int log_gates, int dtype, void* workspace, void* stream);
 /* mmf_cross_entropy_train_fwd / _bwd replace cross_entropy_fwd_kernel / cross_entropy_bwd_kernel,
  *   mmfreelm/modules/fused_cross_entropy.py:26-98 / :98-160 (CrossEntropyLossFunction :163-310, one device): per row, with
  *   l = logit_scale * logits, lse = logsumexp(l):

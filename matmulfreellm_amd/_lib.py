@@ -67,6 +67,8 @@ SIGNATURES = {
     "mmf_hgrn_gate_bwd": (_i32, [_ptr, _i64, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _ptr, _i64, _ptr, _ptr, _i64, _i64, _i32,
                                  _ptr]),
     "mmf_hgrn_recurrent_bwd": (_i32, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _i32, _i32, _ptr]),
+    "mmf_hgrn_recurrent_bwd_workspace_bytes": (_i64, [_i64, _i64, _i64]),
+    "mmf_hgrn_recurrent_bwd_split": (_i32, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _i32, _i32, _ptr, _ptr]),
     "mmf_cross_entropy_train_fwd": (_i32, [_ptr, _i64, _ptr, _i64, _f32, _f32, _f32, _ptr, _ptr, _ptr, _i64, _i64, _i32, _ptr]),
     "mmf_cross_entropy_train_bwd": (_i32, [_ptr, _i64, _ptr, _i64, _ptr, _ptr, _f32, _f32, _f32, _ptr, _i64, _i64, _i64, _i32, _ptr]),
     "mmf_short_conv_max_kernel_size": (_i32, []),

@@ -211,10 +211,12 @@ def _scan_bwd(g, o, do, h0, log_gates):
     gc, oc, dc = g.contiguous(), o.contiguous(), do.to(g.dtype).contiguous()
     dx, dg = torch.empty_like(gc), torch.empty_like(gc)
     h0f = h0.detach().reshape(b * h, d).float().contiguous() if h0 is not None else None
+    nws = lib.mmf_hgrn_recurrent_bwd_workspace_bytes(b * h, t, d)
+    ws = torch.empty(nws // 4, dtype=torch.float32, device=g.device) if nws else None    # per-segment carries (few KB)
     with torch.cuda.device(g.device):
-        L.check(lib.mmf_hgrn_recurrent_bwd(gc.data_ptr(), oc.data_ptr(), dc.data_ptr(), L.ptr(h0f), dx.data_ptr(), dg.data_ptr(),
-                                           b * h, t, d, 1 if log_gates else 0, L.dtype_id(g.dtype), L.stream()),
-                "mmf_hgrn_recurrent_bwd")
+        L.check(lib.mmf_hgrn_recurrent_bwd_split(gc.data_ptr(), oc.data_ptr(), dc.data_ptr(), L.ptr(h0f), dx.data_ptr(),
+                                                 dg.data_ptr(), b * h, t, d, 1 if log_gates else 0, L.dtype_id(g.dtype),
+                                                 L.ptr(ws), L.stream()), "mmf_hgrn_recurrent_bwd_split")
     return dx, dg
 
 

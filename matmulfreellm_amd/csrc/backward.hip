@@ -6,8 +6,6 @@
 //                            the gradient through both quantisers unchanged)
 //   mmf_swiglu_bwd           mmfreelm/modules/activations.py:121-126
 //   mmf_hgrn_gate_bwd        autograd of mmfreelm/layers/hgrn_bit.py:113-120 (sigmoid, lower bound, swiglu(i, 1 - f), mask)
-//   mmf_hgrn_recurrent_bwd   mmfreelm/ops/hgrn/recurrent_fuse.py:89-133 (and, with log gates, the gradient that
-//                            mmfreelm/ops/hgrn/chunk.py:137-220 computes chunk-wise)
 //   mmf_cross_entropy_train_fwd / _bwd   mmfreelm/modules/fused_cross_entropy.py:26-98 / :98-160 (label smoothing, logit
 //                            scale, z-loss)
 //
@@ -288,83 +286,6 @@ __global__ __launch_bounds__(256) void hgrn_gate_bwd_kernel(const T* __restrict_
     }
 }
 
-// ------------------------------------------------------------------------------------------ recurrence
-// dh += do_t; dx_t = dh; dg_t = dh * h_{t-1} (* exp(g_t) for log gates); dh *= g_t (exp(g_t)).  A lane owns a channel and a
-// workgroup 64 channels of one sequence; its NW waves split the time axis.  Every wave first walks its segment from a zero carry
-// and keeps the carry L it would hand to the earlier segment and the product P of its gates, then folds the (L, P) of the later
-// segments (carry = L + P * carry, last segment first) into the carry it really starts from, and walks its segment again to
-// write the gradients.  Time runs backwards in register blocks of 32 steps whose loads are issued together.
-constexpr int kScanBwdBlock = 32, kScanBwdMaxWaves = 8;
-template <typename T, bool LOG>
-__global__ __launch_bounds__(64 * kScanBwdMaxWaves) void hgrn_recurrent_bwd_kernel(const T* __restrict__ g, const T* __restrict__ o,
-                                                                                   const T* __restrict__ dout,
-                                                                                   const float* __restrict__ h0, T* __restrict__ dx,
-                                                                                   T* __restrict__ dg, int64_t Tlen, int64_t D,
-                                                                                   int64_t seg) {
-    constexpr int BL = kScanBwdBlock;
-    __shared__ float carry_l[kScanBwdMaxWaves][64], carry_p[kScanBwdMaxWaves][64];
-    const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6, nw = (int)blockDim.x >> 6;
-    const int64_t d = (int64_t)blockIdx.x * 64 + lane, bh = blockIdx.y;
-    const bool live = d < D;
-    const int64_t base = bh * Tlen * D + (live ? d : 0);
-    const int64_t ta = (int64_t)wave * seg, tb = ta + seg < Tlen ? ta + seg : Tlen;   // this wave's steps ta .. tb - 1 (may be none)
-    float dh = 0.0f;
-    if (nw > 1) {
-        float prod = 1.0f;
-        if (live)
-            for (int64_t t1 = tb; t1 > ta; t1 -= BL) {
-                const int64_t t0 = t1 - BL;
-                float gv[BL], dv[BL];
-#pragma unroll
-                for (int j = 0; j < BL; ++j) {
-                    const int64_t t = t0 + j;
-                    if (t >= ta) {
-                        gv[j] = mmf_to_float(g[base + t * D]);
-                        dv[j] = mmf_to_float(dout[base + t * D]);
-                    }
-                }
-#pragma unroll
-                for (int j = BL - 1; j >= 0; --j)
-                    if (t0 + j >= ta) {
-                        const float gl = LOG ? __expf(gv[j]) : gv[j];
-                        dh = (dh + dv[j]) * gl;
-                        prod *= gl;
-                    }
-            }
-        carry_l[wave][lane] = dh;
-        carry_p[wave][lane] = prod;
-        __syncthreads();
-        dh = 0.0f;
-        for (int w = nw - 1; w > wave; --w) dh = carry_l[w][lane] + carry_p[w][lane] * dh;
-    }
-    if (!live) return;
-    const float hinit = h0 ? h0[bh * D + d] : 0.0f;
-    for (int64_t t1 = tb; t1 > ta; t1 -= BL) {
-        const int64_t t0 = t1 - BL;                              // block covers steps max(t0, ta) .. t1 - 1
-        float gv[BL], dv[BL], hv[BL];
-#pragma unroll
-        for (int j = 0; j < BL; ++j) {
-            const int64_t t = t0 + j;
-            if (t >= ta) {
-                gv[j] = mmf_to_float(g[base + t * D]);
-                dv[j] = mmf_to_float(dout[base + t * D]);
-                hv[j] = t > 0 ? mmf_to_float(o[base + (t - 1) * D]) : hinit;
-            }
-        }
-#pragma unroll
-        for (int j = BL - 1; j >= 0; --j) {
-            const int64_t t = t0 + j;
-            if (t >= ta) {
-                const float gl = LOG ? __expf(gv[j]) : gv[j];
-                dh += dv[j];
-                dx[base + t * D] = mmf_from_float<T>(dh);
-                dg[base + t * D] = mmf_from_float<T>(LOG ? dh * hv[j] * gl : dh * hv[j]);
-                dh *= gl;
-            }
-        }
-    }
-}
-
 // ------------------------------------------------------------------------------------------ cross entropy (training)
 // forward: lse, the loss with label smoothing and z-loss, and the z-loss alone, per row (fp32); 512 threads per row.
 template <typename T>
@@ -532,30 +453,6 @@ int mmf_hgrn_gate_bwd(const void* i_in, int64_t ldi, const void* f_in, int64_t l
         launch_colsum(part, groups, D, dlb, stream);
         MMF_CHECK_LAUNCH();
     }
-    return 0;
-}
-
-int mmf_hgrn_recurrent_bwd(const void* g, const void* o, const void* grad_o, const float* h0, void* dx, void* dg, int64_t BH,
-                           int64_t T, int64_t D, int log_gates, int dtype, void* stream_) {
-    hipStream_t stream = static_cast<hipStream_t>(stream_);
-    if (BH < 0 || T < 0 || D <= 0 || BH > 65535) return MMF_ERR_ARG;
-    if (BH == 0 || T == 0) return 0;
-    if (!g || !o || !grad_o || !dx || !dg) return MMF_ERR_ARG;
-    dim3 grid((unsigned)mmf_ceil_div(D, 64), (unsigned)BH);
-    // segments of at least 64 steps, a whole number of register blocks each, at most 8 waves
-    int64_t nw = T / 64 < 1 ? 1 : T / 64 > kScanBwdMaxWaves ? kScanBwdMaxWaves : T / 64;
-    const int64_t seg = mmf_ceil_div(mmf_ceil_div(T, nw), kScanBwdBlock) * kScanBwdBlock;
-    nw = mmf_ceil_div(T, seg);
-#define MMF_RB(T_, L_) hgrn_recurrent_bwd_kernel<T_, L_><<<grid, (unsigned)(64 * nw), 0, stream>>>(static_cast<const T_*>(g), \
-        static_cast<const T_*>(o), static_cast<const T_*>(grad_o), h0, static_cast<T_*>(dx), static_cast<T_*>(dg), T, D, seg)
-    switch (dtype) {
-        case MMF_F32: if (log_gates) MMF_RB(float, true); else MMF_RB(float, false); break;
-        case MMF_BF16: if (log_gates) MMF_RB(bf16_t, true); else MMF_RB(bf16_t, false); break;
-        case MMF_F16: if (log_gates) MMF_RB(f16_t, true); else MMF_RB(f16_t, false); break;
-        default: return MMF_ERR_ARG;
-    }
-#undef MMF_RB
-    MMF_CHECK_LAUNCH();
     return 0;
 }
 

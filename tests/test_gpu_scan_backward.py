@@ -1,0 +1,31 @@
+"""The scan backward at the edges of its split: block and segment remainders, halved columns (fewer than 256 of 64 channels),
+whole columns, time segments with their carries, lanes past the last channel -- against autograd through the CPU
+restatement, linear and log gates, with and without an initial state."""
+import pytest
+import torch
+
+from oracle import hgrn as oh
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("log", [False, True])
+@pytest.mark.parametrize("bhtd", [(1, 1, 1, 64), (1, 1, 24, 33), (1, 1, 25, 64), (1, 1, 48, 64), (1, 1, 49, 100), (1, 3, 431, 100),
+                                  (1, 140, 50, 40), (1, 2, 23, 8200), (2, 1, 25, 8192), (1, 1, 2100, 96), (1, 2, 2497, 64)])
+def test_scan_backward_split(dev, bhtd, log):
+    import matmulfreellm_amd as mm
+    torch.manual_seed(11)
+    b, h, t, d = bhtd
+    g = torch.randn(b, h, t, d) + 2
+    g = torch.nn.functional.logsigmoid(g) if log else torch.sigmoid(g)
+    x, do = torch.randn(b, h, t, d), torch.randn(b, h, t, d)
+    h0 = torch.randn(b, h, d) if t % 2 else None
+    leaves = [v.clone().requires_grad_() for v in (x, g)]
+    o, _ = oh.naive_recurrent_hgrn_literal(leaves[0], leaves[1].exp() if log else leaves[1], h0, False)
+    want = torch.autograd.grad(o, leaves, do)
+    mine = [v.to(dev).requires_grad_() for v in (x, g)]
+    o2, _ = (mm.chunk_hgrn if log else mm.fused_recurrent_hgrn)(*mine, h0.to(dev) if h0 is not None else None)
+    got = torch.autograd.grad(o2, mine, do.to(dev))
+    for name, a, r in zip(("dx", "dg"), got, want):
+        err = ((a.cpu() - r).abs().max() / r.abs().max().clamp_min(1e-30)).item()
+        assert err < 2e-5, (name, err)
