@@ -356,6 +356,49 @@ int mmf_decode_layers(const void* phases, int n_layers, const void* table, const
                       void* h_out, const void* head, void* logits, uint64_t* am_words, int64_t* tok_out, uint32_t* epoch, int* err,
                       int H, int D, int I, int spin, int dtype, void* stream);
 
+/* ---- stacked projections whose inner norms differ (a trained checkpoint's i, f and g): one row, three norm weights
+ * mmf_rmsnorm_quant_multi: mmf_rmsnorm_quant_fused with the norm prologue (w1, eps1), quantised under three norm weights:
+ *   q receives three tiled code matrices, mmf_codes_bytes(M, K, 1) bytes apart, deq and qsum [3, M].
+ * mmf_bitlinear_mfma_multi: the contraction on a weight stacked from segments of seg_rows rows, segment s with the codes at
+ *   codes_tiled + s * codes_stride, deq + s * M, qsum + s * M (codes_stride 0: all with the same).
+ * mmf_bitlinear_gemv_multi: the one-launch form for few rows, N = 3 * seg_rows; epilogue 0 (plain) or 1 (gate math +
+ *   recurrence step, as mmf_bitlinear_gemv_fused). */
+int mmf_rmsnorm_quant_multi(const void* x, int64_t ldx, const void* w1, float eps1, const void* norm_weight0, const void* norm_weight1,
+                            const void* norm_weight2, float eps, int8_t* q, float* deq, int* qsum, int64_t M, int64_t K, int x_dtype,
+                            int weight_dtype, void* stream);
+int mmf_bitlinear_mfma_multi(const int8_t* codes_tiled, int64_t codes_stride, const float* deq, const int* qsum, const void* packed,
+                             const float* wdeq, int64_t seg_rows, void* out, int64_t ldo, int64_t M, int64_t K, int64_t N,
+                             int out_dtype, int config, void* stream);
+int mmf_bitlinear_gemv_multi(int epilogue, const void* x, int64_t ldx, const void* w1, float eps1, const void* norm_weight0,
+                             const void* norm_weight1, const void* norm_weight2, float eps, const void* packed, const float* wdeq,
+                             int64_t seg_rows, void* out, void* g_out, const float* lower_bound, float* state, int64_t M, int64_t K,
+                             int64_t N, int x_dtype, int weight_dtype, void* stream);
+
+/* ---- a whole block (mmfreelm/models/hgrn_bit/modeling_hgrn_bit.py:97-111) as one host call: the launches above in the order
+ * of the model, bit for bit what they give one by one.  out [B, T, H] = block(x [B, T, H]); mask: null or [B, T] bytes;
+ * h0 / ht: recurrent state [B, D] fp32 in / out, each may be null, h0 == ht updates in place.  f_norm == null: i_norm serves
+ * all three projections.  lower_bound: null in the first layer.  *_seg_rows: rows per weight scale (i/f/g: D).  The struct lives in
+ * HOST memory and is read before the call returns.  workspace: 256-byte aligned, mmf_block_workspace_bytes(p, B * T) bytes.
+ * D and I must be multiples of 32. */
+typedef struct {
+    const void *attn_norm, *i_norm, *f_norm, *g_proj_norm, *ifg_packed;
+    const float* ifg_wdeq;
+    const void *g_norm, *o_norm, *o_packed;
+    const float* o_wdeq;
+    const void *mlp_norm, *gate_norm, *gate_packed;
+    const float* gate_wdeq;
+    const void *down_norm, *down_packed;
+    const float* down_wdeq;
+    int64_t o_seg_rows, gate_seg_rows, down_seg_rows;
+    int64_t H, D, I;
+    float attn_eps, ifg_eps, g_eps, o_eps, mlp_eps, gate_eps, down_eps;
+    int dtype, weight_dtype;
+} mmf_block;
+int64_t mmf_block_struct_bytes(void);
+int64_t mmf_block_workspace_bytes(const mmf_block* p, int64_t rows);
+int mmf_block_forward(const mmf_block* p, const void* x, void* out, int64_t B, int64_t T, const float* lower_bound,
+                      const uint8_t* mask, const float* h0, float* ht, void* workspace, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -76,6 +76,13 @@ SIGNATURES = {
     "mmf_short_conv_step": (_i32, [_ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i32, _i32, _i32, _ptr]),
     "mmf_short_conv_bwd_groups": (_i32, [_i64]),
     "mmf_short_conv_bwd": (_i32, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _i32, _i32, _i32, _ptr]),
+    "mmf_rmsnorm_quant_multi": (_i32, [_ptr, _i64, _ptr, _f32, _ptr, _ptr, _ptr, _f32, _ptr, _ptr, _ptr, _i64, _i64, _i32, _i32, _ptr]),
+    "mmf_bitlinear_mfma_multi": (_i32, [_ptr, _i64, _ptr, _ptr, _ptr, _ptr, _i64, _ptr, _i64, _i64, _i64, _i64, _i32, _i32, _ptr]),
+    "mmf_bitlinear_gemv_multi": (_i32, [_i32, _ptr, _i64, _ptr, _f32, _ptr, _ptr, _ptr, _f32, _ptr, _ptr, _i64, _ptr, _ptr, _ptr, _ptr,
+                                        _i64, _i64, _i64, _i32, _i32, _ptr]),
+    "mmf_block_struct_bytes": (_i64, []),
+    "mmf_block_workspace_bytes": (_i64, [_ptr, _i64]),
+    "mmf_block_forward": (_i32, [_ptr, _ptr, _ptr, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr]),
     "mmf_sample_top_p_max_vocab": (_i64, []),
     "mmf_sample_top_p": (_i32, [_ptr, _i64, _i64, _i64, _f32, _f32, _i64, _ptr, _ptr, _i32, _ptr]),
 }
@@ -138,4 +145,20 @@ def ptr(t):
 
 
 def stream():
-    return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
+class _NoSwitch:
+    def __enter__(self):
+        pass
+
+    def __exit__(self, *exc):
+        return False
+
+
+_NO_SWITCH = _NoSwitch()
+
+
+def on(dev):
+    """``torch.cuda.device(dev)``, without its work when ``dev`` is the current device already."""
+    return _NO_SWITCH if torch._C._cuda_getDevice() == dev.index else torch.cuda.device(dev)

@@ -64,6 +64,7 @@ class HGRNBitAttention(nn.Module):
         self.o_proj = BitLinear(self.input_dim, hidden_size, bias=False, fused_eps=bitlinear_eps)
         self.apply(self._initialize_weights)
         self._ifg_key, self._ifg = None, None
+        self._stack_key, self._stack = None, None
 
     def _initialize_weights(self, module):
         if getattr(module, "_is_hf_initialized", False):
@@ -75,6 +76,15 @@ class HGRNBitAttention(nn.Module):
         module._is_hf_initialized = True
 
     # ---- stacked i/f/g projection ------------------------------------------------------
+    def _stacked_weight(self):
+        """PackedWeight of [i; f; g], whatever their inner norms hold."""
+        parts = [p.packed_weight() for p in (self.i_proj, self.f_proj, self.g_proj)]
+        key = tuple(id(pw) for pw in parts)
+        if key != self._stack_key:
+            # (the parts stay alive with the projections' pack caches; kept here too, so that an id is not reused)
+            self._stack_key, self._stack = key, (F_.stack_packed(parts), parts)
+        return self._stack[0]
+
     def _stacked_ifg(self):
         """PackedWeight of [i; f; g] if the three inner norms are identical, else None."""
         projs = (self.i_proj, self.f_proj, self.g_proj)
@@ -86,7 +96,7 @@ class HGRNBitAttention(nn.Module):
                     and all(p.norm.eps == projs[0].norm.eps and p.fused_eps == projs[0].fused_eps for p in projs)
                     and torch.equal(self.i_proj.norm.weight, self.f_proj.norm.weight)
                     and torch.equal(self.i_proj.norm.weight, self.g_proj.norm.weight))
-            self._ifg = F_.stack_packed([p.packed_weight() for p in projs]) if same else None
+            self._ifg = self._stacked_weight() if same else None
         return self._ifg
 
     def forward(self, hidden_states: torch.Tensor, attention_mask: Optional[torch.Tensor] = None,

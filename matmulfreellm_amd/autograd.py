@@ -61,7 +61,7 @@ def _norm_bwd(mode, xs, gate, weight, dy, dres, eps, want_y=False):
         w = w.float()
     dw = torch.empty_like(w) if w is not None else None
     part = torch.empty(lib.mmf_backward_groups(m), k, dtype=torch.float32, device=dev) if w is not None else None
-    with torch.cuda.device(dev):
+    with L.on(dev):
         L.check(lib.mmf_rmsnorm_bwd(mode, x2.data_ptr(), ldx, L.ptr(g2), ldg, L.ptr(w), dy2.data_ptr(), lddy, L.ptr(dr2),
                                     dx.data_ptr(), L.ptr(dgate), L.ptr(yq), L.ptr(part), L.ptr(dw), m, k, eps,
                                     L.dtype_id(x2.dtype), L.dtype_id(w.dtype) if w is not None else 0, L.stream()),
@@ -165,7 +165,7 @@ class SwiGLUFn(torch.autograd.Function):
         rows, cols = x2.shape
         dx = torch.empty(rows, cols, dtype=x.dtype, device=x.device)
         dy = torch.empty(rows, cols, dtype=x.dtype, device=x.device)
-        with torch.cuda.device(x.device):
+        with L.on(x.device):
             L.check(lib.mmf_swiglu_bwd(x2.data_ptr(), ldx, y2.data_ptr(), ldy, g2.data_ptr(), ldg, dx.data_ptr(), cols,
                                        dy.data_ptr(), cols, rows, cols, L.dtype_id(x.dtype), L.stream()), "mmf_swiglu_bwd")
         return dx.reshape(x.shape), dy.reshape(y.shape)
@@ -198,7 +198,7 @@ class HGRNGateFn(torch.autograd.Function):
         dlb = torch.empty(d, dtype=torch.float32, device=dev) if lb is not None else None
         part = torch.empty(lib.mmf_backward_groups(rows), d, dtype=torch.float32, device=dev) if lb is not None else None
         mk = F_._mask_rows(mask, rows, dev) if mask is not None else None
-        with torch.cuda.device(dev):
+        with L.on(dev):
             L.check(lib.mmf_hgrn_gate_bwd(i2.data_ptr(), ldi, f2.data_ptr(), ldf, L.ptr(lbf), L.ptr(mk), gx2.data_ptr(),
                                           gg2.data_ptr(), di.data_ptr(), d, df.data_ptr(), d, L.ptr(part), L.ptr(dlb), rows, d,
                                           L.dtype_id(i.dtype), L.stream()), "mmf_hgrn_gate_bwd")
@@ -213,7 +213,7 @@ def _scan_bwd(g, o, do, h0, log_gates):
     h0f = h0.detach().reshape(b * h, d).float().contiguous() if h0 is not None else None
     nws = lib.mmf_hgrn_recurrent_bwd_workspace_bytes(b * h, t, d)
     ws = torch.empty(nws // 4, dtype=torch.float32, device=g.device) if nws else None    # per-segment carries (few KB)
-    with torch.cuda.device(g.device):
+    with L.on(g.device):
         L.check(lib.mmf_hgrn_recurrent_bwd_split(gc.data_ptr(), oc.data_ptr(), dc.data_ptr(), L.ptr(h0f), dx.data_ptr(),
                                                  dg.data_ptr(), b * h, t, d, 1 if log_gates else 0, L.dtype_id(g.dtype),
                                                  L.ptr(ws), L.stream()), "mmf_hgrn_recurrent_bwd_split")
@@ -269,7 +269,7 @@ class CrossEntropyFn(torch.autograd.Function):
         loss = torch.empty(rows, dtype=torch.float32, device=dev)
         lse = torch.empty(rows, dtype=torch.float32, device=dev)
         z = torch.empty(rows, dtype=torch.float32, device=dev)
-        with torch.cuda.device(dev):
+        with L.on(dev):
             L.check(lib.mmf_cross_entropy_train_fwd(lg.data_ptr(), lg.stride(0), lab.data_ptr(), int(ignore_index), float(smoothing),
                                                     float(logit_scale), float(lse_square_scale), loss.data_ptr(), lse.data_ptr(),
                                                     z.data_ptr(), rows, v, L.dtype_id(lg.dtype), L.stream()),
@@ -287,7 +287,7 @@ class CrossEntropyFn(torch.autograd.Function):
         rows, v = lg.shape
         dlogits = lg if inplace else torch.empty_like(lg)
         dl = dloss.to(torch.float32).contiguous()
-        with torch.cuda.device(lg.device):
+        with L.on(lg.device):
             L.check(lib.mmf_cross_entropy_train_bwd(lg.data_ptr(), lg.stride(0), lab.data_ptr(), ignore_index, lse.data_ptr(),
                                                     dl.data_ptr(), smoothing, logit_scale, lse_square_scale, dlogits.data_ptr(),
                                                     dlogits.stride(0), rows, v, L.dtype_id(lg.dtype), L.stream()),

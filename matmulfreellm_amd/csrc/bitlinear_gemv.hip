@@ -52,6 +52,8 @@ struct GemvArgs {
     void* res_out;        // PRO_RESNORM: summed residual stream [M, K] (written by the first workgroup of a row)
     const void* w1;       // weight of the prologue's own norm [K]
     const void* norm_w;   // BitLinear's inner norm weight [K] or null
+    const void* norm_w2;  // null, or the inner norm weights of the second and third stacked segment (norm_w: the first)
+    const void* norm_w3;
     const uint4* packed;  // [Np/32][Kp/128][64] uint4
     const float* wdeq;    // one scale per segment of seg_rows output rows
     const void* bias;     // [N] or null
@@ -77,8 +79,12 @@ struct GemvArgs {
 // grid of as many workgroups as are resident at once; workgroup b of a row of x takes the n-blocks b, b + grid, ... behind ONE
 // prologue, the next block's packed weights in flight while the current one is contracted -- otherwise every 16 KiB of
 // weights would wait behind a re-quantisation of the whole row.
-template <typename T, typename TW, int NW, int NV, int PRO, int EPI, bool VEC, int S, bool WALK = false>
+// NN = 3 (EPI_STEP): the i, f and g rows have inner norms of their own, so the row is normalised once and quantised three
+// times -- three maxima in one exchange, three code rows in LDS.  (With the plain epilogue a workgroup's rows lie in one
+// segment and it just picks that segment's norm weight.)
+template <typename T, typename TW, int NW, int NV, int PRO, int EPI, bool VEC, int S, bool WALK = false, int NN = 1>
 __global__ __launch_bounds__(64 * NW) void bitlinear_gemv_kernel(GemvArgs a) {
+    static_assert(NN == 1 || (NN == 3 && EPI == EPI_STEP), "one code row per stacked segment");
     static_assert(!WALK || (S == 1 && EPI == EPI_PLAIN), "the n-block walk is built for whole n-blocks and the plain epilogue");
     constexpr int kGemvWaves = NW, kGemvThreads = 64 * NW;
     constexpr int R = EPI == EPI_STEP ? 3 : EPI == EPI_SWIGLU ? 2 : 1;
@@ -89,11 +95,11 @@ __global__ __launch_bounds__(64 * NW) void bitlinear_gemv_kernel(GemvArgs a) {
     constexpr bool HAS_AUX = PRO >= PRO_RESNORM;
     constexpr bool HAS_W1 = PRO >= PRO_NORM && PRO <= PRO_GATEDNORM;
     extern __shared__ __align__(16) unsigned char smem[];
-    int8_t* q_lds = reinterpret_cast<int8_t*>(smem);            // Kp bytes
+    int8_t* q_lds = reinterpret_cast<int8_t*>(smem);            // NN x Kp bytes
     // one slot array per reduction, so each costs a single barrier
     __shared__ double red_a[kGemvWaves], red_b[kGemvWaves];
-    __shared__ float red_f[kGemvWaves];
-    __shared__ int red_q[kGemvWaves];
+    __shared__ float red_f[NN][kGemvWaves];
+    __shared__ int red_q[NN][kGemvWaves];
     __shared__ int2 part[S == 1 ? R * kGemvWaves * 32 : R * GMAX * 8];   // S = 1: [r][wave][row], S = 4: [item][row8]; .x/.y: lane halves
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -107,16 +113,28 @@ __global__ __launch_bounds__(64 * NW) void bitlinear_gemv_kernel(GemvArgs a) {
     const T* x = static_cast<const T*>(a.x) + (int64_t)row * a.ldx;
     const T* aux = static_cast<const T*>(a.aux) + (int64_t)row * a.ldaux;
     const TW* w1 = static_cast<const TW*>(a.w1);
-    const TW* nw = static_cast<const TW*>(a.norm_w);
+    const TW* nws[3] = {static_cast<const TW*>(a.norm_w), static_cast<const TW*>(a.norm_w2), static_cast<const TW*>(a.norm_w3)};
+    const TW* nw = nws[0];
+    if constexpr (EPI == EPI_PLAIN) {
+        if (a.norm_w2) {
+            const uint32_t seg = (uint32_t)(nb * 32) / (uint32_t)a.seg_rows;
+            nw = seg == 0 ? nw : seg == 1 ? nws[1] : nws[2];
+        }
+    }
     Raw4<T> xraw[NV], araw[HAS_AUX ? NV : 1];
-    Raw4<TW> w1raw[HAS_W1 ? NV : 1], nwraw[NV];
+    Raw4<TW> w1raw[HAS_W1 ? NV : 1], nwraw[NN][NV];
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
         const int k0 = (v * kGemvThreads + (int)threadIdx.x) * kGemvEl;
         xraw[v] = raw4_load<T, VEC>(x, k0, K);
         if constexpr (HAS_AUX) araw[v] = raw4_load<T, VEC>(aux, k0, K);
         if constexpr (HAS_W1) w1raw[v] = raw4_load<TW, VEC>(w1, k0, K);
-        if (nw) nwraw[v] = raw4_load<TW, VEC>(nw, k0, K);
+        if constexpr (NN == 1) {
+            if (nw) nwraw[0][v] = raw4_load<TW, VEC>(nw, k0, K);
+        } else {
+#pragma unroll
+            for (int j = 0; j < NN; ++j) nwraw[j][v] = raw4_load<TW, VEC>(nws[j], k0, K);
+        }
     }
     constexpr int NWREG = S == 1 ? R * BPW : ITEMS;
     uint4 wreg[NWREG];
@@ -224,48 +242,86 @@ __global__ __launch_bounds__(64 * NW) void bitlinear_gemv_kernel(GemvArgs a) {
         for (int i = 0; i < 4; ++i) ss = mmf_add_square(ss, xv[v][i]);
     ss = mmf_block_sum_once<kGemvWaves>(ss, red_b);
     const float rstd = mmf_rstd(ss, K, a.inv_K, a.eps);
-    float amax = 0.0f;
+    float amax[NN];
+#pragma unroll
+    for (int j = 0; j < NN; ++j) amax[j] = 0.0f;
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-        float wv[4];
-        if (nw) raw4_unpack<TW>(nwraw[v], wv);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float y = __fmul_rn(xv[v][i], rstd);
-            if (nw) y = __fmul_rn(y, wv[i]);
-            xv[v][i] = y;                                       // elements past K are exact zeros and stay so
-            amax = fmaxf(amax, fabsf(y));
+        for (int i = 0; i < 4; ++i) xv[v][i] = __fmul_rn(xv[v][i], rstd);   // elements past K are exact zeros and stay so
+#pragma unroll
+        for (int j = 0; j < NN; ++j) {
+            float wv[4];
+            if (NN > 1 || nw) raw4_unpack<TW>(nwraw[j][v], wv);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float y = xv[v][i];
+                if (NN > 1 || nw) y = __fmul_rn(y, wv[i]);
+                if constexpr (NN == 1) xv[v][i] = y;
+                amax[j] = fmaxf(amax[j], fabsf(y));
+            }
         }
     }
-    amax = mmf_block_max_once<kGemvWaves>(amax, red_f);
-    const float scale = mmf_127_over(fmaxf(amax, 1e-5f));
-    const float deq = mmf_rcp_pos(scale);                 // needed by the epilogue only: computed here, in the shadow of the barriers
-    int qs = 0;
+    if constexpr (NN == 1) {
+        amax[0] = mmf_block_max_once<kGemvWaves>(amax[0], red_f[0]);
+    } else {
+#pragma unroll
+        for (int j = 0; j < NN; ++j) {
+            amax[j] = mmf_wave_max(amax[j]);
+            if (lane == 0) red_f[j][wave] = amax[j];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < NN; ++j) {
+            amax[j] = red_f[j][0];
+#pragma unroll
+            for (int i = 1; i < kGemvWaves; ++i) amax[j] = fmaxf(amax[j], red_f[j][i]);
+        }
+    }
+    float scale[NN], deq[NN];                                   // deq is needed by the epilogue only: computed here, in the shadow of the barriers
+    int qs[NN];
+#pragma unroll
+    for (int j = 0; j < NN; ++j) {
+        scale[j] = mmf_127_over(fmaxf(amax[j], 1e-5f));
+        deq[j] = mmf_rcp_pos(scale[j]);
+        qs[j] = 0;
+    }
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
         const int k0 = (v * kGemvThreads + (int)threadIdx.x) * kGemvEl;
         if (k0 < Kp) {
-            uint32_t packed4 = 0;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int c = (k0 + i < K) ? mmf_code(xv[v][i], scale) : 0;
-                qs += c;
-                packed4 |= (uint32_t)(c & 0xff) << (8 * i);
+            for (int j = 0; j < NN; ++j) {
+                float wv[4];
+                if constexpr (NN > 1) raw4_unpack<TW>(nwraw[j][v], wv);
+                uint32_t packed4 = 0;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float y = NN > 1 ? __fmul_rn(xv[v][i], wv[i]) : xv[v][i];
+                    const int c = (k0 + i < K) ? mmf_code(y, scale[j]) : 0;
+                    qs[j] += c;
+                    packed4 |= (uint32_t)(c & 0xff) << (8 * i);
+                }
+                *reinterpret_cast<uint32_t*>(q_lds + j * Kp + k0) = packed4;
             }
-            *reinterpret_cast<uint32_t*>(q_lds + k0) = packed4;
         }
     }
     __syncthreads();                                            // publishes q_lds
     // the code sum is only needed by the epilogue: fold it after the barrier, off the critical path
     // (red_q is read behind the next barrier)
-    qs = mmf_wave_sum(qs);
-    if (lane == 0) red_q[wave] = qs;
+#pragma unroll
+    for (int j = 0; j < NN; ++j) {
+        qs[j] = mmf_wave_sum(qs[j]);
+        if (lane == 0) red_q[j][wave] = qs[j];
+    }
 
     // ---- main + epilogue of one n-block (R stacked ones): weights `wr`, epilogue operands as loaded for that block
     auto contract = [&](const uint4 (&wr)[NWREG], int nbc, const float (&wdq)[R], float bias_v, float add_v) {
         const int chc = nbc * 32 + sub * CHN + (lane & (CHN - 1));
         const bool epl = wave == 0 && lane < CHN && chc < Nseg;
-        auto dot_block = [&](const uint4& wq, int kb, int acc) { return mmf_dot_block(q_lds, wq, kb, half, acc); };
+        auto dot_block = [&](const uint4& wq, int r, int kb, int acc) {
+            return mmf_dot_block(q_lds + (NN > 1 ? r * Kp : 0), wq, kb, half, acc);
+        };
         if constexpr (S == 1) {
             int acc[R];
 #pragma unroll
@@ -275,7 +331,7 @@ __global__ __launch_bounds__(64 * NW) void bitlinear_gemv_kernel(GemvArgs a) {
                 const int kb = wave + i * kGemvWaves;
                 if (kb < KB) {
 #pragma unroll
-                    for (int r = 0; r < R; ++r) acc[r] = dot_block(wr[r * BPW + i], kb, acc[r]);
+                    for (int r = 0; r < R; ++r) acc[r] = dot_block(wr[r * BPW + i], r, kb, acc[r]);
                 }
             }
 #pragma unroll
@@ -286,7 +342,7 @@ __global__ __launch_bounds__(64 * NW) void bitlinear_gemv_kernel(GemvArgs a) {
                 const int item = wave + i * kGemvWaves;
                 if (item < R * G) {
                     const int kb = (item % G) * 4 + kbi;
-                    int acc = dot_block(wr[i], kb < KB ? kb : 0, 0);   // blocks past the end carry zero codes
+                    int acc = dot_block(wr[i], item / G, kb < KB ? kb : 0, 0);   // blocks past the end carry zero codes
                     acc += mmf_dpp<0x128>(acc);                      // row_ror:8 -> the other k-half
                     acc += __builtin_amdgcn_ds_swizzle(acc, 0x401F);   // xor 16 -> the neighbouring k-block
                     if ((lane & 31) < 8) reinterpret_cast<int*>(&part[item * 8 + (lane & 7)])[lane >> 5] = acc;
@@ -295,9 +351,13 @@ __global__ __launch_bounds__(64 * NW) void bitlinear_gemv_kernel(GemvArgs a) {
         }
         __syncthreads();
         if (epl) {
-            int qtot = 0;
+            int qtot[NN];
 #pragma unroll
-            for (int w = 0; w < kGemvWaves; ++w) qtot += red_q[w];
+            for (int j = 0; j < NN; ++j) {
+                qtot[j] = 0;
+#pragma unroll
+                for (int w = 0; w < kGemvWaves; ++w) qtot[j] += red_q[j][w];
+            }
             float res[R];
 #pragma unroll
             for (int r = 0; r < R; ++r) {
@@ -315,7 +375,7 @@ __global__ __launch_bounds__(64 * NW) void bitlinear_gemv_kernel(GemvArgs a) {
                         tot += gi < G ? pr.x + pr.y : 0;
                     }
                 }
-                res[r] = __fmul_rn(__fmul_rn((float)(tot - qtot), deq), wdq[r]);
+                res[r] = __fmul_rn(__fmul_rn((float)(tot - qtot[NN > 1 ? r : 0]), deq[NN > 1 ? r : 0]), wdq[r]);
             }
             if constexpr (EPI == EPI_PLAIN) {
                 float o = res[0];
@@ -370,7 +430,7 @@ __global__ __launch_bounds__(64 * NW) void bitlinear_gemv_kernel(GemvArgs a) {
     }
 }
 
-template <typename T, typename TW, int PRO, int EPI, int NW, int NV>
+template <typename T, typename TW, int PRO, int EPI, int NW, int NV, int NN>
 void launch_gemv_shape(const GemvArgs& a, dim3 grid, bool split, bool walk, hipStream_t s) {
     if constexpr (EPI == EPI_PLAIN) {
         if (walk) {
@@ -378,8 +438,8 @@ void launch_gemv_shape(const GemvArgs& a, dim3 grid, bool split, bool walk, hipS
             return;
         }
     }
-    if (split) bitlinear_gemv_kernel<T, TW, NW, NV, PRO, EPI, true, 4><<<grid, dim3(64 * NW), (size_t)a.Kp, s>>>(a);
-    else bitlinear_gemv_kernel<T, TW, NW, NV, PRO, EPI, true, 1><<<grid, dim3(64 * NW), (size_t)a.Kp, s>>>(a);
+    if (split) bitlinear_gemv_kernel<T, TW, NW, NV, PRO, EPI, true, 4, false, NN><<<grid, dim3(64 * NW), (size_t)a.Kp * NN, s>>>(a);
+    else bitlinear_gemv_kernel<T, TW, NW, NV, PRO, EPI, true, 1, false, NN><<<grid, dim3(64 * NW), (size_t)a.Kp * NN, s>>>(a);
 }
 
 // Workgroups that a launch keeps resident at once on this build's target (256 CUs, 2048 threads each): the n-block walk
@@ -392,7 +452,7 @@ inline int gemv_walk_slots(int threads) {
     return env >= 0 ? env : 256 * (2048 / threads);
 }
 
-template <typename T, typename TW, int PRO, int EPI>
+template <typename T, typename TW, int PRO, int EPI, int NN = 1>
 int launch_gemv(const GemvArgs& a, int64_t M, bool vec, hipStream_t s) {
     constexpr int R = EPI == EPI_STEP ? 3 : EPI == EPI_SWIGLU ? 2 : 1;
     const int64_t nblocks = mmf_ceil_div(a.N / R, 32);
@@ -402,14 +462,14 @@ int launch_gemv(const GemvArgs& a, int64_t M, bool vec, hipStream_t s) {
     const int nw = a.Kp <= 2048 ? 8 : a.Kp <= 3072 ? 12 : a.Kp <= 4096 ? 16 : a.Kp <= 6144 ? 12 : 16;
     // many more n-blocks than resident workgroups (vocabulary-sized N): a grid of resident workgroups walks them
     const int64_t per_row = gemv_walk_slots(64 * nw) / M;
-    const bool walk = vec && EPI == EPI_PLAIN && per_row >= 32 && nblocks > per_row;
+    const bool walk = vec && EPI == EPI_PLAIN && !a.norm_w2 && per_row >= 32 && nblocks > per_row;
     dim3 grid((unsigned)(walk ? per_row : nblocks * (split ? 4 : 1)), (unsigned)M);
-    if (!vec) bitlinear_gemv_kernel<T, TW, 8, 4, PRO, EPI, false, 1><<<grid, dim3(512), (size_t)a.Kp, s>>>(a);   // ragged shapes: one generic build
-    else if (a.Kp <= 2048) launch_gemv_shape<T, TW, PRO, EPI, 8, 1>(a, grid, split, walk, s);
-    else if (a.Kp <= 3072) launch_gemv_shape<T, TW, PRO, EPI, 12, 1>(a, grid, split, walk, s);
-    else if (a.Kp <= 4096) launch_gemv_shape<T, TW, PRO, EPI, 16, 1>(a, grid, split, walk, s);
-    else if (a.Kp <= 6144) launch_gemv_shape<T, TW, PRO, EPI, 12, 2>(a, grid, split, walk, s);
-    else launch_gemv_shape<T, TW, PRO, EPI, 16, 2>(a, grid, split, walk, s);
+    if (!vec) bitlinear_gemv_kernel<T, TW, 8, 4, PRO, EPI, false, 1, false, NN><<<grid, dim3(512), (size_t)a.Kp * NN, s>>>(a);   // ragged shapes: one generic build
+    else if (a.Kp <= 2048) launch_gemv_shape<T, TW, PRO, EPI, 8, 1, NN>(a, grid, split, walk, s);
+    else if (a.Kp <= 3072) launch_gemv_shape<T, TW, PRO, EPI, 12, 1, NN>(a, grid, split, walk, s);
+    else if (a.Kp <= 4096) launch_gemv_shape<T, TW, PRO, EPI, 16, 1, NN>(a, grid, split, walk, s);
+    else if (a.Kp <= 6144) launch_gemv_shape<T, TW, PRO, EPI, 12, 2, NN>(a, grid, split, walk, s);
+    else launch_gemv_shape<T, TW, PRO, EPI, 16, 2, NN>(a, grid, split, walk, s);
     MMF_CHECK_LAUNCH();
     return 0;
 }
@@ -426,6 +486,7 @@ int dispatch_gemv_kind(const GemvArgs& a, int64_t M, int pro, int epi, bool vec,
             case PRO_SWIGLU: return launch_gemv<T, TW, PRO_SWIGLU, EPI_PLAIN>(a, M, vec, s);
         }
     } else if (epi == EPI_STEP) {
+        if (pro == PRO_NORM && a.norm_w2) return launch_gemv<T, TW, PRO_NORM, EPI_STEP, 3>(a, M, vec, s);
         if (pro == PRO_NORM) return launch_gemv<T, TW, PRO_NORM, EPI_STEP>(a, M, vec, s);
         if (pro == PRO_PLAIN) return launch_gemv<T, TW, PRO_PLAIN, EPI_STEP>(a, M, vec, s);
     } else if (epi == EPI_SWIGLU) {
@@ -444,13 +505,7 @@ int dispatch_gemv_w(const GemvArgs& a, int64_t M, int pro, int epi, int x_dtype,
 
 bool aligned(const void* p, size_t n) { return (reinterpret_cast<uintptr_t>(p) % n) == 0; }
 
-}  // namespace
-
-extern "C" {
-
-int64_t mmf_bitlinear_gemv_max_k(void) { return kGemvMaxK; }
-
-int mmf_bitlinear_gemv_fused(int prologue, int epilogue, const void* x, int64_t ldx, const void* aux, int64_t ldaux,
+int run_gemv(const void* norm_weight2, const void* norm_weight3, int prologue, int epilogue, const void* x, int64_t ldx, const void* aux, int64_t ldaux,
                              void* res_out, const void* w1, float eps1, const void* norm_weight, float eps,
                              const void* packed, const float* wdeq, int64_t seg_rows, const void* bias,
                              const void* addend, void* out, void* g_out, const float* lower_bound, float* state,
@@ -468,6 +523,7 @@ int mmf_bitlinear_gemv_fused(int prologue, int epilogue, const void* x, int64_t 
     if (seg_rows % 32 != 0 && seg_rows < N) return MMF_ERR_ARG;   // stacked segments are whole n-blocks
     GemvArgs a{};
     a.x = x; a.aux = aux ? aux : x; a.res_out = res_out; a.w1 = w1; a.norm_w = norm_weight;
+    a.norm_w2 = norm_weight2; a.norm_w3 = norm_weight3;
     a.packed = static_cast<const uint4*>(packed); a.wdeq = wdeq; a.bias = bias; a.addend = addend; a.out = out;
     a.g_out = g_out; a.lb = lower_bound; a.state = state;
     a.K = (int)K; a.Kp = (int)mmf_round_up(K, 128); a.N = (int)N; a.seg_rows = (int)seg_rows; a.ldx = ldx;
@@ -478,7 +534,8 @@ int mmf_bitlinear_gemv_fused(int prologue, int epilogue, const void* x, int64_t 
     if (!norm_weight && !w1) weight_dtype = MMF_F32;
     const size_t xa = 4 * (x_dtype == MMF_F32 ? 4 : 2), wa = 4 * (weight_dtype == MMF_F32 ? 4 : 2);
     const bool vec = K % 4 == 0 && ldx % 4 == 0 && a.ldaux % 4 == 0;
-    if (vec && !(aligned(x, xa) && aligned(a.aux, xa) && aligned(res_out, xa) && aligned(w1, wa) && aligned(norm_weight, wa)))
+    if (vec && !(aligned(x, xa) && aligned(a.aux, xa) && aligned(res_out, xa) && aligned(w1, wa) && aligned(norm_weight, wa) && aligned(norm_weight2, wa) &&
+                 aligned(norm_weight3, wa)))
         return MMF_ERR_ALIGN;
     switch (x_dtype) {
         case MMF_F32: return dispatch_gemv_w<float>(a, M, prologue, epilogue, x_dtype, weight_dtype, vec, stream);
@@ -486,6 +543,31 @@ int mmf_bitlinear_gemv_fused(int prologue, int epilogue, const void* x, int64_t 
         case MMF_F16: return dispatch_gemv_w<f16_t>(a, M, prologue, epilogue, x_dtype, weight_dtype, vec, stream);
     }
     return MMF_ERR_ARG;
+}
+
+}  // namespace
+
+extern "C" {
+
+int64_t mmf_bitlinear_gemv_max_k(void) { return kGemvMaxK; }
+
+int mmf_bitlinear_gemv_fused(int prologue, int epilogue, const void* x, int64_t ldx, const void* aux, int64_t ldaux,
+                             void* res_out, const void* w1, float eps1, const void* norm_weight, float eps,
+                             const void* packed, const float* wdeq, int64_t seg_rows, const void* bias,
+                             const void* addend, void* out, void* g_out, const float* lower_bound, float* state,
+                             int64_t M, int64_t K, int64_t N, int x_dtype, int weight_dtype, void* stream) {
+    return run_gemv(nullptr, nullptr, prologue, epilogue, x, ldx, aux, ldaux, res_out, w1, eps1, norm_weight, eps, packed, wdeq, seg_rows,
+                    bias, addend, out, g_out, lower_bound, state, M, K, N, x_dtype, weight_dtype, stream);
+}
+
+int mmf_bitlinear_gemv_multi(int epilogue, const void* x, int64_t ldx, const void* w1, float eps1, const void* norm_weight0,
+                             const void* norm_weight1, const void* norm_weight2, float eps, const void* packed, const float* wdeq,
+                             int64_t seg_rows, void* out, void* g_out, const float* lower_bound, float* state, int64_t M, int64_t K,
+                             int64_t N, int x_dtype, int weight_dtype, void* stream) {
+    if (epilogue != EPI_PLAIN && epilogue != EPI_STEP) return MMF_ERR_ARG;
+    if (M > 0 && (!norm_weight0 || !norm_weight1 || !norm_weight2 || N != 3 * seg_rows)) return MMF_ERR_ARG;
+    return run_gemv(norm_weight1, norm_weight2, PRO_NORM, epilogue, x, ldx, nullptr, 0, nullptr, w1, eps1, norm_weight0, eps, packed, wdeq,
+                    seg_rows, nullptr, nullptr, out, g_out, lower_bound, state, M, K, N, x_dtype, weight_dtype, stream);
 }
 
 int mmf_bitlinear_gemv(const void* x, const void* norm_weight, const void* packed, const float* wdeq,

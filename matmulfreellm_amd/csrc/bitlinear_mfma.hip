@@ -41,6 +41,8 @@ struct MfmaArgs {
     const void* addend;   // [M, N] (leading dimension ldo) or null: out = T(T(o) + addend)
     void* out;            // [M, N]
     int64_t M, N, Kp, seg_rows, ldo;
+    int64_t a_seg;        // 0, or the bytes from one weight segment's codes to the next's (deq, qsum: M entries): stacked
+                          // projections whose inner norms differ contract each its own codes of the same rows
     int tiles_m, tiles_n;
     int rows_per_xcd;     // tile rows an XCD keeps in its L2 while it walks the columns (0: row-major tile order)
     int vec_store;        // outputs can be written as aligned 16-byte vectors
@@ -51,6 +53,15 @@ struct MfmaArgs {
 // Where the tiled kernel notes its clocks (mmf_bitlinear_mfma_clock_sink); null: nothing is noted.
 long long* g_clock_sink = nullptr;
 int64_t g_clock_cap = 0;
+
+// The operands of the weight segment that n-block nb0 lies in (wave-uniform; a workgroup's tile lies in one segment).
+__device__ __forceinline__ void mfma_select_segment(MfmaArgs& p, int64_t nb0) {
+    if (p.a_seg == 0) return;
+    const int64_t seg = (int64_t)((uint32_t)(nb0 * 32) / (uint32_t)p.seg_rows);
+    p.a += seg * p.a_seg;
+    p.deq += seg * p.M;
+    p.qsum += seg * p.M;
+}
 
 // Pack rounded outputs: two floats -> one dword of bf16/f16 (round to nearest even).
 template <typename T>
@@ -477,6 +488,7 @@ void bitlinear_mfma_dma3_kernel(MfmaArgs p) {
         if constexpr (SWI) return (nb0 < NBs ? nb0 : NBs - 1) + j * NBs;
         else return nb0 + j < NB ? nb0 + j : NB - 1;
     };
+    if constexpr (!SWI) mfma_select_segment(p, tile_n * BNB);
     EpiScales<WM, WN> sc;
     mfma_prefetch_scales<WM, WN>(p, sc, lane, wm, mb0, nb0);
     if constexpr (SWI) {
@@ -691,6 +703,7 @@ __global__ __launch_bounds__(512) void bitlinear_mfma_skinny_kernel(MfmaArgs p) 
     __shared__ int red[NWV][MB][16][64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform: keep it in a scalar register
     const int64_t nb = blockIdx.x, mbase = (int64_t)blockIdx.y * MB;   // this workgroup's first m-block
+    mfma_select_segment(p, nb);
     const int64_t KB = p.Kp >> 7, KG = p.Kp >> 4;
     const int64_t MBtot = (p.M + 31) >> 5;
 
@@ -832,6 +845,24 @@ int dispatch_mfma(const MfmaArgs& a, int config, hipStream_t s) {
         else config = a.N >= 512 ? 17 : 16;
     }
     if (config == 5 && (a.Kp > 8192 || a.M > 65535 * 32)) return MMF_ERR_ARG;
+    const int64_t tile_cols = config == 5 ? 32 : config == 16 ? 256 : config == 17 ? 512 : 0;
+    if (a.a_seg != 0 && a.N > a.seg_rows && (tile_cols == 0 || a.seg_rows % tile_cols != 0)) {
+        // tiles that would straddle two segments (or tiles of the kernels that take one set of codes): a launch per segment
+        for (int64_t n0 = 0; n0 < a.N; n0 += a.seg_rows) {
+            const int64_t seg = n0 / a.seg_rows;
+            MfmaArgs b = a;
+            b.a += seg * a.a_seg;
+            b.deq += seg * a.M;
+            b.qsum += seg * a.M;
+            b.a_seg = 0;
+            b.b += (n0 >> 5) * (a.Kp >> 7) * 64;
+            b.wdeq += seg;
+            b.N = a.N - n0 < a.seg_rows ? a.N - n0 : a.seg_rows;
+            b.out = static_cast<T*>(a.out) + n0;
+            if (const int rc = dispatch_mfma<T>(b, config, s)) return rc;
+        }
+        return 0;
+    }
     switch (config) {
         case 5: return launch_skinny<T, 1>(a, s);
         case 0: return launch_mfma<T, 1, 8, 1, 1>(a, s);
@@ -911,6 +942,26 @@ int mmf_bitlinear_mfma(const int8_t* codes_tiled, const float* deq, const int* q
     if ((reinterpret_cast<uintptr_t>(codes_tiled) & 15u) || (reinterpret_cast<uintptr_t>(packed) & 15u)) return MMF_ERR_ALIGN;
     MfmaArgs a{};
     a.a = codes_tiled; a.b = static_cast<const uint4*>(packed); a.deq = deq; a.qsum = qsum; a.wdeq = wdeq; a.bias = bias; a.addend = addend;
+    a.out = out; a.M = M; a.N = N; a.Kp = mmf_round_up(K, 128); a.seg_rows = seg_rows; a.ldo = ldo;
+    switch (out_dtype) {
+        case MMF_F32: return dispatch_mfma<float>(a, config, stream);
+        case MMF_BF16: return dispatch_mfma<bf16_t>(a, config, stream);
+        case MMF_F16: return dispatch_mfma<f16_t>(a, config, stream);
+    }
+    return MMF_ERR_ARG;
+}
+
+int mmf_bitlinear_mfma_multi(const int8_t* codes_tiled, int64_t codes_stride, const float* deq, const int* qsum, const void* packed,
+                             const float* wdeq, int64_t seg_rows, void* out, int64_t ldo, int64_t M, int64_t K, int64_t N,
+                             int out_dtype, int config, void* stream_) {
+    hipStream_t stream = static_cast<hipStream_t>(stream_);
+    if (M < 0 || K <= 0 || N <= 0 || seg_rows <= 0 || seg_rows % 32 != 0 || ldo < N || N > 0x7fffffff) return MMF_ERR_ARG;
+    if (M == 0) return 0;
+    if (!codes_tiled || !deq || !qsum || !packed || !wdeq || !out || codes_stride < 0) return MMF_ERR_ARG;
+    if ((reinterpret_cast<uintptr_t>(codes_tiled) & 15u) || (codes_stride & 15) || (reinterpret_cast<uintptr_t>(packed) & 15u))
+        return MMF_ERR_ALIGN;
+    MfmaArgs a{};
+    a.a = codes_tiled; a.a_seg = codes_stride; a.b = static_cast<const uint4*>(packed); a.deq = deq; a.qsum = qsum; a.wdeq = wdeq;
     a.out = out; a.M = M; a.N = N; a.Kp = mmf_round_up(K, 128); a.seg_rows = seg_rows; a.ldo = ldo;
     switch (out_dtype) {
         case MMF_F32: return dispatch_mfma<float>(a, config, stream);

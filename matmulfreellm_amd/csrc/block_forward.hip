@@ -1,0 +1,151 @@
+// One HGRNBit block (mmfreelm/models/hgrn_bit/modeling_hgrn_bit.py:97-111) over B sequences of T tokens as ONE host call: the
+// launches of the module path, in its order, with every elementwise op folded into the BitLinear next to it.
+//
+// Host code only.  Short prompts are bound by what it costs to issue a launch: through nn.Module calls, output allocations and
+// one foreign-function call per kernel a 24-layer forward of 77 tokens spent 8.9 ms on the host and 1.6 ms on the GPU.  Here a
+// layer costs one foreign-function call, and its buffers are offsets into one workspace.
+#include "mmf_common.h"
+
+namespace {
+
+constexpr int64_t kGemvRows = 8;      // rows up to which every workgroup of a BitLinear redoes the row's prologue (one launch)
+constexpr int64_t kSwigluRows = 512;  // rows from which the gate/up contraction runs tiled and carries the swiglu in its epilogue
+
+// prologue / epilogue ids of mmf_bitlinear_gemv_fused and mmf_rmsnorm_quant_fused
+enum { G_PLAIN = 0, G_NORM = 1, G_RESNORM = 2, G_GATEDNORM = 3, E_PLAIN = 0, E_STEP = 1, E_SWIGLU = 2 };
+enum { Q_PLAIN = 0, Q_NORM = 1, Q_RESNORM = 2, Q_STEP_GATE = 3, Q_SWIGLU = 4, Q_GATEDNORM = 5 };
+
+int64_t esize(const mmf_block* p) { return p->dtype == MMF_F32 ? 4 : 2; }
+bool few_rows(const mmf_block* p, int64_t M) {
+    const int64_t k = p->H > p->I ? p->H : p->I;
+    return M <= kGemvRows && (k > p->D ? k : p->D) <= mmf_bitlinear_gemv_max_k();
+}
+
+// Offsets of the intermediates in the workspace (each 256-byte aligned).
+struct Layout {
+    int64_t ifg, o, attn, res, big, q, deq, qsum, bytes;
+    Layout(const mmf_block* p, int64_t M) {
+        const int64_t e = esize(p);
+        bytes = 0;
+        auto take = [&](int64_t n) {
+            const int64_t at = bytes;
+            bytes += mmf_round_up(n, 256);
+            return at;
+        };
+        ifg = take(M * 3 * p->D * e);
+        o = take(M * p->D * e);
+        attn = take(M * p->H * e);
+        res = take(M * p->H * e);
+        big = take(M * 2 * (p->I > p->D ? p->I : p->D) * e);    // the scan's x and g, later gate/up
+        int64_t codes = 3 * mmf_codes_bytes(M, p->H, 1);
+        for (int64_t k : {(int64_t)p->D, (int64_t)p->I})
+            if (mmf_codes_bytes(M, k, 1) > codes) codes = mmf_codes_bytes(M, k, 1);
+        q = take(codes);
+        deq = take(3 * M * 4);
+        qsum = take(3 * M * 4);
+    }
+};
+
+}  // namespace
+
+extern "C" {
+
+int64_t mmf_block_struct_bytes(void) { return (int64_t)sizeof(mmf_block); }
+
+int64_t mmf_block_workspace_bytes(const mmf_block* p, int64_t rows) {
+    if (!p || rows <= 0) return 0;
+    return Layout(p, rows).bytes;
+}
+
+int mmf_block_forward(const mmf_block* p, const void* x, void* out, int64_t B, int64_t T, const float* lower_bound,
+                      const uint8_t* mask, const float* h0, float* ht, void* workspace, void* stream) {
+    if (!p || B < 0 || T < 0 || p->H <= 0 || p->D <= 0 || p->I <= 0 || p->D % 32 || p->I % 32) return MMF_ERR_ARG;
+    const int64_t M = B * T, H = p->H, D = p->D, I = p->I, e = esize(p);
+    if (M == 0) return 0;
+    if (!x || !out || x == out || !workspace) return MMF_ERR_ARG;
+    if (reinterpret_cast<uintptr_t>(workspace) & 255u) return MMF_ERR_ALIGN;
+    const Layout L(p, M);
+    char* w = static_cast<char*>(workspace);
+    char* ifg = w + L.ifg;
+    char *i = ifg, *f = ifg + D * e, *g = ifg + 2 * D * e;     // columns of the stacked projection, row stride 3 D
+    void *o = w + L.o, *attn = w + L.attn, *res = w + L.res;
+    char* big = w + L.big;
+    int8_t* q = reinterpret_cast<int8_t*>(w + L.q);
+    float* deq = reinterpret_cast<float*>(w + L.deq);
+    int* qsum = reinterpret_cast<int*>(w + L.qsum);
+    const int dt = p->dtype, wt = p->weight_dtype;
+    const bool multi = p->f_norm != nullptr;                   // i, f and g have inner norms of their own
+    const bool step = T == 1 && h0 && h0 == ht;                // one token on a kept state: gate math + recurrence step in one kernel
+    int rc = 0;
+#define MMF_DO(call)                \
+    do {                            \
+        if ((rc = (call))) return rc; \
+    } while (0)
+    auto scan = [&]() -> int {                                 // gate math, then the recurrence: o [M, D] contiguous
+        if (step) return mmf_hgrn_step(i, 3 * D, f, 3 * D, lower_bound, mask, ht, o, M, D, dt, stream);
+        void *xs = big, *gs = big + M * D * e;
+        if (const int r = mmf_hgrn_gate(i, 3 * D, f, 3 * D, lower_bound, mask, xs, gs, M, D, dt, stream)) return r;
+        return mmf_hgrn_recurrent(xs, gs, h0, o, ht, B, T, D, dt, stream);
+    };
+    if (few_rows(p, M)) {
+        const int epi = step && !mask ? E_STEP : E_PLAIN;
+        void* first = epi == E_STEP ? o : ifg;
+        void* g_row = epi == E_STEP ? ifg : (void*)g;           // the raw g projection, row stride D or 3 D
+        if (multi)
+            MMF_DO(mmf_bitlinear_gemv_multi(epi, x, H, p->attn_norm, p->attn_eps, p->i_norm, p->f_norm, p->g_proj_norm, p->ifg_eps,
+                                            p->ifg_packed, p->ifg_wdeq, D, first, ifg, lower_bound, ht, M, H, 3 * D, dt, wt,
+                                            stream));
+        else
+            MMF_DO(mmf_bitlinear_gemv_fused(G_NORM, epi, x, H, nullptr, 0, nullptr, p->attn_norm, p->attn_eps, p->i_norm, p->ifg_eps,
+                                            p->ifg_packed, p->ifg_wdeq, D, nullptr, nullptr, first, ifg, lower_bound, ht, M, H,
+                                            3 * D, dt, wt, stream));
+        if (epi != E_STEP) MMF_DO(scan());
+        MMF_DO(mmf_bitlinear_gemv_fused(G_GATEDNORM, E_PLAIN, g_row, epi == E_STEP ? D : 3 * D, o, D, nullptr, p->g_norm, p->g_eps,
+                                        p->o_norm, p->o_eps, p->o_packed, p->o_wdeq, p->o_seg_rows, nullptr, nullptr, attn, nullptr,
+                                        nullptr, nullptr, M, D, H, dt, wt, stream));
+        MMF_DO(mmf_bitlinear_gemv_fused(G_RESNORM, E_SWIGLU, attn, H, x, H, res, p->mlp_norm, p->mlp_eps, p->gate_norm, p->gate_eps,
+                                        p->gate_packed, p->gate_wdeq, p->gate_seg_rows, nullptr, nullptr, big, nullptr, nullptr,
+                                        nullptr, M, H, 2 * I, dt, wt, stream));
+        MMF_DO(mmf_bitlinear_gemv_fused(G_PLAIN, E_PLAIN, big, I, nullptr, 0, nullptr, nullptr, 0.0f, p->down_norm, p->down_eps,
+                                        p->down_packed, p->down_wdeq, p->down_seg_rows, nullptr, res, out, nullptr, nullptr, nullptr,
+                                        M, I, H, dt, wt, stream));
+        return 0;
+    }
+    if (multi) {
+        MMF_DO(mmf_rmsnorm_quant_multi(x, H, p->attn_norm, p->attn_eps, p->i_norm, p->f_norm, p->g_proj_norm, p->ifg_eps, q, deq, qsum,
+                                       M, H, dt, wt, stream));
+        MMF_DO(mmf_bitlinear_mfma_multi(q, mmf_codes_bytes(M, H, 1), deq, qsum, p->ifg_packed, p->ifg_wdeq, D, ifg, 3 * D, M, H, 3 * D,
+                                        dt, -1, stream));
+    } else {
+        MMF_DO(mmf_rmsnorm_quant_fused(Q_NORM, x, H, nullptr, 0, nullptr, 0, nullptr, p->attn_norm, p->attn_eps, p->i_norm, p->ifg_eps,
+                                       nullptr, nullptr, q, deq, qsum, M, H, dt, wt, stream));
+        MMF_DO(mmf_bitlinear_mfma(q, deq, qsum, p->ifg_packed, p->ifg_wdeq, D, nullptr, nullptr, ifg, 3 * D, M, H, 3 * D, dt, -1,
+                                  stream));
+    }
+    if (step && !mask) {
+        MMF_DO(mmf_rmsnorm_quant_fused(Q_STEP_GATE, i, 3 * D, f, 3 * D, g, 3 * D, nullptr, p->g_norm, p->g_eps, p->o_norm, p->o_eps,
+                                       lower_bound, ht, q, deq, qsum, M, D, dt, wt, stream));
+    } else {
+        MMF_DO(scan());
+        MMF_DO(mmf_rmsnorm_quant_fused(Q_GATEDNORM, g, 3 * D, o, D, nullptr, 0, nullptr, p->g_norm, p->g_eps, p->o_norm, p->o_eps,
+                                       nullptr, nullptr, q, deq, qsum, M, D, dt, wt, stream));
+    }
+    MMF_DO(mmf_bitlinear_mfma(q, deq, qsum, p->o_packed, p->o_wdeq, p->o_seg_rows, nullptr, nullptr, attn, H, M, D, H, dt, -1, stream));
+    MMF_DO(mmf_rmsnorm_quant_fused(Q_RESNORM, attn, H, x, H, nullptr, 0, res, p->mlp_norm, p->mlp_eps, p->gate_norm, p->gate_eps, nullptr,
+                                   nullptr, q, deq, qsum, M, H, dt, wt, stream));
+    if (M >= kSwigluRows) {
+        MMF_DO(mmf_bitlinear_mfma_swiglu(q, deq, qsum, p->gate_packed, p->gate_wdeq, p->gate_seg_rows, big, I, M, H, 2 * I, dt, stream));
+        MMF_DO(mmf_rmsnorm_quant_fused(Q_PLAIN, big, I, nullptr, 0, nullptr, 0, nullptr, nullptr, 0.0f, p->down_norm, p->down_eps, nullptr,
+                                       nullptr, q, deq, qsum, M, I, dt, wt, stream));
+    } else {
+        MMF_DO(mmf_bitlinear_mfma(q, deq, qsum, p->gate_packed, p->gate_wdeq, p->gate_seg_rows, nullptr, nullptr, big, 2 * I, M, H, 2 * I,
+                                  dt, -1, stream));
+        MMF_DO(mmf_rmsnorm_quant_fused(Q_SWIGLU, big, 2 * I, big + I * e, 2 * I, nullptr, 0, nullptr, nullptr, 0.0f, p->down_norm,
+                                       p->down_eps, nullptr, nullptr, q, deq, qsum, M, I, dt, wt, stream));
+    }
+    MMF_DO(mmf_bitlinear_mfma(q, deq, qsum, p->down_packed, p->down_wdeq, p->down_seg_rows, nullptr, res, out, H, M, I, H, dt, -1, stream));
+#undef MMF_DO
+    return 0;
+}
+
+}  // extern "C"

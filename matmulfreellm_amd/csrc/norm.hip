@@ -226,6 +226,8 @@ struct FusedQuantArgs {
     int64_t ldx, ldaux, ldaux2;
     void* res_out;
     const void* w1; const void* norm_w;
+    const void* norm_w2; const void* norm_w3;   // NN = 3: the second and third norm weight
+    int64_t q_stride;                           // NN = 3: bytes from one norm's codes to the next's (deq, qsum: M entries)
     const float* lb; float* state;
     int8_t* q; float* deq; int* qsum;
     int64_t M, K, Kp;
@@ -241,12 +243,14 @@ constexpr int kQWaves = 8, kQThreads = kQWaves * 64;
 //   RPW = 8 : prefill has thousands of rows and the kernel should stream: one wave per row, whose
 //             reductions are DPP folds only - no LDS exchange and no barrier anywhere.
 // VEC: K, the strides and every pointer allow 4-element accesses.
-template <typename T, typename TW, int NV, int PRO, bool VEC, int RPW>
+// NN = 3: the row is normalised once and quantised under three norm weights (the projections of a trained layer share their
+// input, not their inner norm): one read of the row and one rstd instead of three, the three maxima in one exchange.
+template <typename T, typename TW, int NV, int PRO, bool VEC, int RPW, int NN = 1>
 __global__ __launch_bounds__(kQThreads) void row_quant_fused_kernel(FusedQuantArgs a) {
     constexpr int TPR = kQThreads / RPW, WPR = TPR / 64;        // threads / waves per row
     __shared__ double red_a[kQWaves], red_b[kQWaves];
-    __shared__ float red_f[kQWaves];
-    __shared__ int red_i[kQWaves];
+    __shared__ float red_f[NN][kQWaves];
+    __shared__ int red_i[NN][kQWaves];
     constexpr bool HAS_AUX = PRO >= QPRO_RESNORM, STEP = PRO == QPRO_STEP_GATE, HAS_W1 = PRO != QPRO_SWIGLU && PRO != QPRO_PLAIN;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int w0 = (wave / WPR) * WPR;                          // first wave of this row
@@ -261,13 +265,14 @@ __global__ __launch_bounds__(kQThreads) void row_quant_fused_kernel(FusedQuantAr
     const T* aux = static_cast<const T*>(a.aux) + row * a.ldaux;
     const T* aux2 = static_cast<const T*>(a.aux2) + row * a.ldaux2;
     const TW* w1 = static_cast<const TW*>(a.w1);
-    const TW* nw = static_cast<const TW*>(a.norm_w);
+    const TW* const nws[3] = {static_cast<const TW*>(a.norm_w), static_cast<const TW*>(a.norm_w2), static_cast<const TW*>(a.norm_w3)};
+    const TW* nw = nws[0];
     float* st = a.state + row * K;
 
     // every load of the kernel first, raw; conversions only after the last one is issued
     Raw4<T> xraw[NV], araw[HAS_AUX ? NV : 1], graw[STEP ? NV : 1];
     Raw4<float> straw[STEP ? NV : 1], lbraw[STEP ? NV : 1];
-    Raw4<TW> w1raw[HAS_W1 ? NV : 1], nwraw[NV];
+    Raw4<TW> w1raw[HAS_W1 ? NV : 1], nwraw[NN][NV];
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
         const int k0 = (v * TPR + tr) * 4;
@@ -279,7 +284,10 @@ __global__ __launch_bounds__(kQThreads) void row_quant_fused_kernel(FusedQuantAr
             if (a.lb) lbraw[v] = raw4_load<float, VEC>(a.lb, k0, K);
         }
         if constexpr (HAS_W1) w1raw[v] = raw4_load<TW, VEC>(w1, k0, K);
-        if (nw) nwraw[v] = raw4_load<TW, VEC>(nw, k0, K);
+        if (NN > 1 || nw) {
+#pragma unroll
+            for (int j = 0; j < NN; ++j) nwraw[j][v] = raw4_load<TW, VEC>(nws[j], k0, K);
+        }
     }
     float xv[NV][4], av[HAS_AUX ? NV : 1][4];
 #pragma unroll
@@ -379,106 +387,140 @@ __global__ __launch_bounds__(kQThreads) void row_quant_fused_kernel(FusedQuantAr
         for (int w = 1; w < WPR; ++w) ss += red_b[w0 + w];
     }
     const float rstd = mmf_rstd(ss, K, a.inv_K, a.eps);
-    float amax = 0.0f;
+    float amax[NN];
+#pragma unroll
+    for (int j = 0; j < NN; ++j) amax[j] = 0.0f;
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-        float wv[4];
-        if (nw) raw4_unpack<TW>(nwraw[v], wv);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float y = __fmul_rn(xv[v][i], rstd);
-            if (nw) y = __fmul_rn(y, wv[i]);
-            xv[v][i] = y;                                       // elements past K are exact zeros and stay so
-            amax = fmaxf(amax, fabsf(y));
+        for (int i = 0; i < 4; ++i) xv[v][i] = __fmul_rn(xv[v][i], rstd);   // elements past K are exact zeros and stay so
+#pragma unroll
+        for (int j = 0; j < NN; ++j) {
+            float wv[4];
+            if (NN > 1 || nw) raw4_unpack<TW>(nwraw[j][v], wv);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float y = xv[v][i];
+                if (NN > 1 || nw) y = __fmul_rn(y, wv[i]);
+                if constexpr (NN == 1) xv[v][i] = y;
+                amax[j] = fmaxf(amax[j], fabsf(y));
+            }
         }
     }
-    amax = mmf_wave_max(amax);
-    if constexpr (WPR > 1) {
-        if ((threadIdx.x & 63) == 0) red_f[wave] = amax;
-        __syncthreads();
-        amax = red_f[w0];
 #pragma unroll
-        for (int w = 1; w < WPR; ++w) amax = fmaxf(amax, red_f[w0 + w]);
+    for (int j = 0; j < NN; ++j) amax[j] = mmf_wave_max(amax[j]);
+    if constexpr (WPR > 1) {
+#pragma unroll
+        for (int j = 0; j < NN; ++j)
+            if ((threadIdx.x & 63) == 0) red_f[j][wave] = amax[j];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < NN; ++j) {
+            amax[j] = red_f[j][w0];
+#pragma unroll
+            for (int w = 1; w < WPR; ++w) amax[j] = fmaxf(amax[j], red_f[j][w0 + w]);
+        }
     }
-    const float scale = mmf_127_over(fmaxf(amax, 1e-5f));
-    int qs = 0;
+    float scale[NN];
+    int qs[NN];
+#pragma unroll
+    for (int j = 0; j < NN; ++j) {
+        scale[j] = mmf_127_over(fmaxf(amax[j], 1e-5f));
+        qs[j] = 0;
+    }
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
         const int k0 = (v * TPR + tr) * 4;
         if (k0 < Kp) {
-            uint32_t packed4 = 0;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int c = inb(k0, i) ? mmf_code(xv[v][i], scale) : 0;
-                qs += c;
-                packed4 |= (uint32_t)(c & 0xff) << (8 * i);
-            }
             const int64_t off = ((row >> 5) * (Kp >> 4) + (k0 >> 4)) * 512 + (row & 31) * 16 + (k0 & 15);
-            if (live) *reinterpret_cast<uint32_t*>(a.q + off) = packed4;
+#pragma unroll
+            for (int j = 0; j < NN; ++j) {
+                float wv[4];
+                if constexpr (NN > 1) raw4_unpack<TW>(nwraw[j][v], wv);
+                uint32_t packed4 = 0;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float y = NN > 1 ? __fmul_rn(xv[v][i], wv[i]) : xv[v][i];
+                    const int c = inb(k0, i) ? mmf_code(y, scale[j]) : 0;
+                    qs[j] += c;
+                    packed4 |= (uint32_t)(c & 0xff) << (8 * i);
+                }
+                if (live) *reinterpret_cast<uint32_t*>(a.q + j * a.q_stride + off) = packed4;
+            }
         }
     }
-    qs = mmf_wave_sum(qs);
-    if constexpr (WPR > 1) {
-        if ((threadIdx.x & 63) == 0) red_i[wave] = qs;
-        __syncthreads();
-        qs = 0;
 #pragma unroll
-        for (int w = 0; w < WPR; ++w) qs += red_i[w0 + w];
+    for (int j = 0; j < NN; ++j) qs[j] = mmf_wave_sum(qs[j]);
+    if constexpr (WPR > 1) {
+#pragma unroll
+        for (int j = 0; j < NN; ++j)
+            if ((threadIdx.x & 63) == 0) red_i[j][wave] = qs[j];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < NN; ++j) {
+            qs[j] = 0;
+#pragma unroll
+            for (int w = 0; w < WPR; ++w) qs[j] += red_i[j][w0 + w];
+        }
     }
     if (tr == 0 && live) {
-        a.deq[row] = mmf_rcp_pos(scale);
-        a.qsum[row] = qs;
+#pragma unroll
+        for (int j = 0; j < NN; ++j) {
+            a.deq[j * a.M + row] = mmf_rcp_pos(scale[j]);
+            a.qsum[j * a.M + row] = qs[j];
+        }
     }
 }
 
-template <typename T, typename TW, int PRO, int RPW>
+template <typename T, typename TW, int PRO, int RPW, int NN>
 int launch_fused_quant_rpw(const FusedQuantArgs& a, hipStream_t s) {
     constexpr int TPR = kQThreads / RPW;
     const int64_t nv = mmf_ceil_div(a.Kp, (int64_t)TPR * 4);
     dim3 grid((unsigned)mmf_ceil_div(a.M, (int64_t)RPW)), block(kQThreads);
-    if (nv <= 1) row_quant_fused_kernel<T, TW, 1, PRO, true, RPW><<<grid, block, 0, s>>>(a);
-    else if (nv <= 2) row_quant_fused_kernel<T, TW, 2, PRO, true, RPW><<<grid, block, 0, s>>>(a);
-    else if (nv <= 3) row_quant_fused_kernel<T, TW, 3, PRO, true, RPW><<<grid, block, 0, s>>>(a);
-    else if (nv <= 4) row_quant_fused_kernel<T, TW, 4, PRO, true, RPW><<<grid, block, 0, s>>>(a);
-    else if (nv <= 6) row_quant_fused_kernel<T, TW, 6, PRO, true, RPW><<<grid, block, 0, s>>>(a);
-    else if (nv <= 8) row_quant_fused_kernel<T, TW, 8, PRO, true, RPW><<<grid, block, 0, s>>>(a);
+    if (nv <= 1) row_quant_fused_kernel<T, TW, 1, PRO, true, RPW, NN><<<grid, block, 0, s>>>(a);
+    else if (nv <= 2) row_quant_fused_kernel<T, TW, 2, PRO, true, RPW, NN><<<grid, block, 0, s>>>(a);
+    else if (nv <= 3) row_quant_fused_kernel<T, TW, 3, PRO, true, RPW, NN><<<grid, block, 0, s>>>(a);
+    else if (nv <= 4) row_quant_fused_kernel<T, TW, 4, PRO, true, RPW, NN><<<grid, block, 0, s>>>(a);
+    else if (nv <= 6) row_quant_fused_kernel<T, TW, 6, PRO, true, RPW, NN><<<grid, block, 0, s>>>(a);
+    else if (nv <= 8) row_quant_fused_kernel<T, TW, 8, PRO, true, RPW, NN><<<grid, block, 0, s>>>(a);
     else if constexpr (PRO == QPRO_PLAIN && RPW == 4) {
         if (nv > 12) return MMF_ERR_WIDE;
-        row_quant_fused_kernel<T, TW, 12, PRO, true, RPW><<<grid, block, 0, s>>>(a);
+        row_quant_fused_kernel<T, TW, 12, PRO, true, RPW, NN><<<grid, block, 0, s>>>(a);
     } else return MMF_ERR_WIDE;
     MMF_CHECK_LAUNCH();
     return 0;
 }
 
-template <typename T, typename TW, int PRO>
+template <typename T, typename TW, int PRO, int NN = 1>
 int launch_fused_quant(const FusedQuantArgs& a, bool vec, hipStream_t s) {
     if (mmf_ceil_div(a.Kp, (int64_t)kQThreads * 4) > 8) return MMF_ERR_WIDE;
     if (!vec) {                                                 // ragged rows: one generic build
-        row_quant_fused_kernel<T, TW, 8, PRO, false, 1><<<dim3((unsigned)a.M), dim3(kQThreads), 0, s>>>(a);
+        row_quant_fused_kernel<T, TW, 8, PRO, false, 1, NN><<<dim3((unsigned)a.M), dim3(kQThreads), 0, s>>>(a);
         MMF_CHECK_LAUNCH();
         return 0;
     }
     // decode: latency (the recurrence-step prologue only exists there: one token per row)
-    if (a.M <= 256 || PRO == QPRO_STEP_GATE) return launch_fused_quant_rpw<T, TW, PRO, 1>(a, s);
+    if (a.M <= 256 || PRO == QPRO_STEP_GATE) return launch_fused_quant_rpw<T, TW, PRO, 1, NN>(a, s);
     // prefill: as many rows per workgroup as 8 passes of 4 elements per thread allow
     if constexpr (PRO != QPRO_STEP_GATE) {
-        if (a.Kp <= 64 * 4 * 8) return launch_fused_quant_rpw<T, TW, PRO, 8>(a, s);
-        if (a.Kp <= 128 * 4 * 8) return launch_fused_quant_rpw<T, TW, PRO, 4>(a, s);
+        if (a.Kp <= 64 * 4 * 8) return launch_fused_quant_rpw<T, TW, PRO, 8, NN>(a, s);
+        if (a.Kp <= 128 * 4 * 8) return launch_fused_quant_rpw<T, TW, PRO, 4, NN>(a, s);
         // the 5632- and 6912-wide rows in front of down_proj (nothing folded in: few registers per element): two waves
         // per row and 12 passes measured 12 % faster than four waves and 6
         if constexpr (PRO == QPRO_PLAIN) {
-            if (a.Kp <= 128 * 4 * 12) return launch_fused_quant_rpw<T, TW, PRO, 4>(a, s);
+            if (a.Kp <= 128 * 4 * 12) return launch_fused_quant_rpw<T, TW, PRO, 4, NN>(a, s);
         }
-        if (a.Kp <= 256 * 4 * 8) return launch_fused_quant_rpw<T, TW, PRO, 2>(a, s);
+        if (a.Kp <= 256 * 4 * 8) return launch_fused_quant_rpw<T, TW, PRO, 2, NN>(a, s);
     }
-    return launch_fused_quant_rpw<T, TW, PRO, 1>(a, s);
+    return launch_fused_quant_rpw<T, TW, PRO, 1, NN>(a, s);
 }
 
 template <typename T, typename TW>
 int dispatch_fused_quant(const FusedQuantArgs& a, int pro, bool vec, hipStream_t s) {
     switch (pro) {
         case QPRO_PLAIN: return launch_fused_quant<T, TW, QPRO_PLAIN>(a, vec, s);
-        case QPRO_NORM: return launch_fused_quant<T, TW, QPRO_NORM>(a, vec, s);
+        case QPRO_NORM:
+            return a.norm_w2 ? launch_fused_quant<T, TW, QPRO_NORM, 3>(a, vec, s) : launch_fused_quant<T, TW, QPRO_NORM>(a, vec, s);
         case QPRO_RESNORM: return launch_fused_quant<T, TW, QPRO_RESNORM>(a, vec, s);
         case QPRO_STEP_GATE: return launch_fused_quant<T, TW, QPRO_STEP_GATE>(a, vec, s);
         case QPRO_SWIGLU: return launch_fused_quant<T, TW, QPRO_SWIGLU>(a, vec, s);
@@ -488,6 +530,26 @@ int dispatch_fused_quant(const FusedQuantArgs& a, int pro, bool vec, hipStream_t
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+
+// Checks the accesses the kernel will make and picks the instance for the types.
+int run_fused_quant(const FusedQuantArgs& a, int prologue, int x_dtype, int weight_dtype, hipStream_t stream) {
+    const uintptr_t xa = 4 * (x_dtype == MMF_F32 ? 4 : 2), wa = 4 * (weight_dtype == MMF_F32 ? 4 : 2);
+    auto al = [](const void* ptr, uintptr_t n) { return (reinterpret_cast<uintptr_t>(ptr) % n) == 0; };
+    const bool vec = a.K % 4 == 0 && a.ldx % 4 == 0 && a.ldaux % 4 == 0 && a.ldaux2 % 4 == 0;
+    if (vec && !(al(a.x, xa) && al(a.aux, xa) && al(a.aux2, xa) && al(a.res_out, xa) && al(a.w1, wa) && al(a.norm_w, wa) && al(a.norm_w2, wa) && al(a.norm_w3, wa) &&
+                 al(a.lb, 16) && al(a.state, 16)))
+        return MMF_ERR_ALIGN;
+    const bool wf32 = weight_dtype == MMF_F32;
+    if (!wf32 && weight_dtype != x_dtype) return MMF_ERR_ARG;
+    switch (x_dtype) {
+        case MMF_F32: return dispatch_fused_quant<float, float>(a, prologue, vec, stream);
+        case MMF_BF16: return wf32 ? dispatch_fused_quant<bf16_t, float>(a, prologue, vec, stream)
+                                   : dispatch_fused_quant<bf16_t, bf16_t>(a, prologue, vec, stream);
+        case MMF_F16: return wf32 ? dispatch_fused_quant<f16_t, float>(a, prologue, vec, stream)
+                                  : dispatch_fused_quant<f16_t, f16_t>(a, prologue, vec, stream);
+    }
+    return MMF_ERR_ARG;
+}
 
 // ---------------------------------------------------------------- swiglu (elementwise)
 template <typename T>
@@ -624,22 +686,22 @@ int mmf_rmsnorm_quant_fused(int prologue, const void* x, int64_t ldx, const void
     a.q = q; a.deq = deq; a.qsum = qsum; a.M = M; a.K = K; a.inv_K = 1.0 / (double)K; a.Kp = mmf_round_up(K, 128); a.eps1 = eps1; a.eps = eps;
     if (!aligned16(q)) return MMF_ERR_ALIGN;
     if (!norm_weight && !w1) weight_dtype = MMF_F32;
-    const uintptr_t xa = 4 * (x_dtype == MMF_F32 ? 4 : 2), wa = 4 * (weight_dtype == MMF_F32 ? 4 : 2);
-    auto al = [](const void* ptr, uintptr_t n) { return (reinterpret_cast<uintptr_t>(ptr) % n) == 0; };
-    const bool vec = K % 4 == 0 && ldx % 4 == 0 && a.ldaux % 4 == 0 && a.ldaux2 % 4 == 0;
-    if (vec && !(al(x, xa) && al(a.aux, xa) && al(a.aux2, xa) && al(res_out, xa) && al(w1, wa) && al(norm_weight, wa) &&
-                 al(lower_bound, 16) && al(state, 16)))
-        return MMF_ERR_ALIGN;
-    const bool wf32 = weight_dtype == MMF_F32;
-    if (!wf32 && weight_dtype != x_dtype) return MMF_ERR_ARG;
-    switch (x_dtype) {
-        case MMF_F32: return dispatch_fused_quant<float, float>(a, prologue, vec, stream);
-        case MMF_BF16: return wf32 ? dispatch_fused_quant<bf16_t, float>(a, prologue, vec, stream)
-                                   : dispatch_fused_quant<bf16_t, bf16_t>(a, prologue, vec, stream);
-        case MMF_F16: return wf32 ? dispatch_fused_quant<f16_t, float>(a, prologue, vec, stream)
-                                  : dispatch_fused_quant<f16_t, f16_t>(a, prologue, vec, stream);
-    }
-    return MMF_ERR_ARG;
+    return run_fused_quant(a, prologue, x_dtype, weight_dtype, stream);
+}
+
+int mmf_rmsnorm_quant_multi(const void* x, int64_t ldx, const void* w1, float eps1, const void* norm_weight0, const void* norm_weight1,
+                            const void* norm_weight2, float eps, int8_t* q, float* deq, int* qsum, int64_t M, int64_t K, int x_dtype,
+                            int weight_dtype, void* stream_) {
+    hipStream_t stream = static_cast<hipStream_t>(stream_);
+    if (M < 0 || K <= 0 || ldx < K) return MMF_ERR_ARG;
+    if (M == 0) return 0;
+    if (!x || !w1 || !norm_weight0 || !norm_weight1 || !norm_weight2 || !q || !deq || !qsum) return MMF_ERR_ARG;
+    if (!aligned16(q)) return MMF_ERR_ALIGN;
+    FusedQuantArgs a{};
+    a.x = a.aux = a.aux2 = x; a.ldx = a.ldaux = a.ldaux2 = ldx; a.w1 = w1; a.norm_w = norm_weight0; a.norm_w2 = norm_weight1;
+    a.norm_w3 = norm_weight2; a.q_stride = mmf_codes_bytes(M, K, 1); a.q = q; a.deq = deq; a.qsum = qsum; a.M = M; a.K = K;
+    a.inv_K = 1.0 / (double)K; a.Kp = mmf_round_up(K, 128); a.eps1 = eps1; a.eps = eps;
+    return run_fused_quant(a, QPRO_NORM, x_dtype, weight_dtype, stream);
 }
 
 int mmf_swiglu(const void* x, int64_t ldx, const void* y, int64_t ldy, void* out, int64_t rows, int64_t cols,

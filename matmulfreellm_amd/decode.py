@@ -429,7 +429,7 @@ class DecodeEngine:
     def advance(self):
         """One decode step from the token buffer; leaves logits in self.logits and the greedy
         next token in the token buffer (no host synchronisation)."""
-        with torch.cuda.device(self.dev):
+        with L.on(self.dev):
             if not self.use_graph:
                 self._launch_step()
                 return

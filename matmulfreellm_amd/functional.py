@@ -44,7 +44,7 @@ def ternarize_pack(weight):
     packed = torch.empty(lib.mmf_packed_bytes(n, k), dtype=torch.uint8, device=w.device)
     wdeq = torch.empty(1, dtype=torch.float32, device=w.device)
     ws = _workspace(w.device, lib.mmf_ternarize_workspace_bytes(), "tern")
-    with torch.cuda.device(w.device):
+    with L.on(w.device):
         L.check(lib.mmf_ternarize_pack(w.data_ptr(), L.dtype_id(w.dtype), n, k, packed.data_ptr(), wdeq.data_ptr(),
                                        ws.data_ptr(), L.stream()), "mmf_ternarize_pack")
     return PackedWeight(packed, wdeq, n, k, -(-n // 32) * 32)
@@ -61,7 +61,7 @@ def stack_packed(parts):
 def unpack_ternary(pw):
     lib = L.load()
     codes = torch.empty(pw.n, pw.k, dtype=torch.int8, device=pw.packed.device)
-    with torch.cuda.device(codes.device):
+    with L.on(codes.device):
         L.check(lib.mmf_unpack_ternary(pw.packed.data_ptr(), pw.n, pw.k, codes.data_ptr(), L.stream()), "mmf_unpack_ternary")
     return codes
 
@@ -92,7 +92,7 @@ def rmsnorm(x, weight, residual=None, eps=1e-6, prenorm=False, residual_in_fp32=
     dev, shp, x2, r2, res_dtype, res_out, w = _norm_common(x, residual, weight, prenorm, residual_in_fp32)
     y = torch.empty_like(x2)
     m, k = x2.shape
-    with torch.cuda.device(dev):
+    with L.on(dev):
         L.check(lib.mmf_rmsnorm(x2.data_ptr(), L.ptr(r2), L.ptr(w), y.data_ptr(), L.ptr(res_out), m, k, eps,
                                 L.dtype_id(x2.dtype), L.dtype_id(res_dtype), L.dtype_id(w.dtype) if w is not None else 0,
                                 L.stream()), "mmf_rmsnorm")
@@ -116,7 +116,7 @@ def rmsnorm_swishgate(x, o, weight, residual=None, eps=1e-6, prenorm=False, resi
     o2 = _as_2d(o)
     m = x2.shape[0]
     y = torch.empty(m, k, dtype=x.dtype, device=dev)
-    with torch.cuda.device(dev):
+    with L.on(dev):
         L.check(lib.mmf_rmsnorm_swishgate(x2.data_ptr(), ldx, o2.data_ptr(), L.ptr(r2), L.ptr(w), y.data_ptr(), L.ptr(res_out),
                                           m, k, eps, L.dtype_id(x2.dtype), L.dtype_id(res_dtype),
                                           L.dtype_id(w.dtype) if w is not None else 0, L.stream()), "mmf_rmsnorm_swishgate")
@@ -152,7 +152,7 @@ def swiglu(x, y):
     x2, ldx = view2d(x)
     y2, ldy = view2d(y)
     out = torch.empty(x.shape, dtype=x.dtype, device=dev)
-    with torch.cuda.device(dev):
+    with L.on(dev):
         L.check(lib.mmf_swiglu(x2.data_ptr(), ldx, y2.data_ptr(), ldy, out.data_ptr(), rows, cols, L.dtype_id(x.dtype),
                                L.stream()), "mmf_swiglu")
     return out
@@ -178,7 +178,7 @@ def rmsnorm_quant(x, weight, residual=None, eps=1e-8, tiled=False, prenorm=False
         q = torch.empty(lib.mmf_codes_bytes(m, k, 1), dtype=torch.int8, device=dev)
         deq = torch.empty(m, dtype=torch.float32, device=dev)
         qsum = torch.empty(m, dtype=torch.int32, device=dev)
-        with torch.cuda.device(dev):
+        with L.on(dev):
             L.check(lib.mmf_rmsnorm_quant_fused(0, x2.data_ptr(), x2.stride(0), None, 0, None, 0, None, None, 0.0, L.ptr(w), eps,
                                                 None, None, q.data_ptr(), deq.data_ptr(), qsum.data_ptr(), m, k,
                                                 L.dtype_id(x2.dtype), L.dtype_id(w.dtype) if w is not None else 0, L.stream()),
@@ -189,7 +189,7 @@ def rmsnorm_quant(x, weight, residual=None, eps=1e-8, tiled=False, prenorm=False
     q = torch.empty(nbytes, dtype=torch.int8, device=dev)
     deq = torch.empty(m, dtype=torch.float32, device=dev)
     qsum = torch.empty(m, dtype=torch.int32, device=dev)
-    with torch.cuda.device(dev):
+    with L.on(dev):
         L.check(lib.mmf_rmsnorm_quant(x2.data_ptr(), L.ptr(r2), L.ptr(w), q.data_ptr(), deq.data_ptr(), qsum.data_ptr(),
                                       L.ptr(res_out), m, k, eps, L.dtype_id(x2.dtype), L.dtype_id(res_dtype),
                                       L.dtype_id(w.dtype) if w is not None else 0, 1 if tiled else 0, L.stream()),
@@ -213,7 +213,7 @@ def _layernorm_quant(lib, dev, shp, x, x2, r2, res_dtype, res_out, w, bias, eps,
     q = torch.empty(lib.mmf_codes_bytes(m, k, 1 if tiled else 0), dtype=torch.int8, device=dev)
     deq = torch.empty(m, dtype=torch.float32, device=dev)
     qsum = torch.empty(m, dtype=torch.int32, device=dev)
-    with torch.cuda.device(dev):
+    with L.on(dev):
         L.check(lib.mmf_layernorm_quant(x2.data_ptr(), L.ptr(r2), L.ptr(w), L.ptr(bias), q.data_ptr(), deq.data_ptr(),
                                         qsum.data_ptr(), L.ptr(res_out), m, k, eps, L.dtype_id(x2.dtype),
                                         L.dtype_id(res_dtype), L.dtype_id(w.dtype) if w is not None else 0,
@@ -246,7 +246,7 @@ def bitlinear_mfma(q_tiled, deq, qsum, pw, m, out_dtype, bias=None, config=-1, o
         addend = addend.reshape(m, pw.n)
         if addend.dtype != out_dtype or not addend.is_contiguous() or ldo != pw.n:
             raise ValueError("addend must be a contiguous [M, N] tensor of the output dtype")
-    with torch.cuda.device(dev):
+    with L.on(dev):
         L.check(lib.mmf_bitlinear_mfma(q_tiled.data_ptr(), deq.data_ptr(), qsum.data_ptr(), pw.packed.data_ptr(),
                                        pw.wdeq.data_ptr(), pw.seg_rows, L.ptr(bias), L.ptr(addend), out.data_ptr(), ldo, m, pw.k, pw.n,
                                        L.dtype_id(out_dtype), config, L.stream()), "mmf_bitlinear_mfma")
@@ -259,7 +259,7 @@ def bitlinear_mfma_swiglu(q_tiled, deq, qsum, pw, m, out_dtype):
     dev = L.require_gpu(q_tiled, deq, qsum, pw.packed)
     inter = pw.n // 2
     out = torch.empty(m, inter, dtype=out_dtype, device=dev)
-    with torch.cuda.device(dev):
+    with L.on(dev):
         L.check(lib.mmf_bitlinear_mfma_swiglu(q_tiled.data_ptr(), deq.data_ptr(), qsum.data_ptr(), pw.packed.data_ptr(),
                                               pw.wdeq.data_ptr(), pw.seg_rows, out.data_ptr(), inter, m, pw.k, pw.n,
                                               L.dtype_id(out_dtype), L.stream()), "mmf_bitlinear_mfma_swiglu")
@@ -285,7 +285,7 @@ def bitlinear_gemv(x2, norm_weight, pw, eps, bias=None, addend=None):
         addend = addend.reshape(m, pw.n)
         if addend.dtype != x2.dtype or not addend.is_contiguous():
             raise ValueError("addend must be a contiguous [M, N] tensor of the input dtype")
-    with torch.cuda.device(dev):
+    with L.on(dev):
         L.check(lib.mmf_bitlinear_gemv(x2.data_ptr(), L.ptr(nw), pw.packed.data_ptr(), pw.wdeq.data_ptr(), pw.seg_rows,
                                        L.ptr(bias), L.ptr(addend), out.data_ptr(), m, k, pw.n, eps, L.dtype_id(x2.dtype),
                                        L.dtype_id(nw.dtype) if nw is not None else 0, L.stream()), "mmf_bitlinear_gemv")
@@ -339,7 +339,7 @@ def _bitlinear_prologue(x, norm_weight, pw, bias, eps, addend, prologue, epilogu
             raise ValueError("addend must be a contiguous [M, N] tensor of the input dtype")
     ldx = x2.stride(0) if m > 1 else k
     lda = (a2.stride(0) if m > 1 else k) if a2 is not None else 0
-    with torch.cuda.device(dev):
+    with L.on(dev):
         if m <= GEMV_MAX_M and k <= lib.mmf_bitlinear_gemv_max_k():
             L.check(lib.mmf_bitlinear_gemv_fused(gid, 0, x2.data_ptr(), ldx, L.ptr(a2), lda, L.ptr(res_out), L.ptr(w1c), eps1,
                                                  L.ptr(nw), eps, pw.packed.data_ptr(), pw.wdeq.data_ptr(), pw.seg_rows,
@@ -430,7 +430,7 @@ def hgrn_recurrent(x, g, initial_state=None, output_final_state=False):
     o = torch.empty_like(xc)
     h0 = _state32(initial_state, b * h, d, dev)
     ht = torch.empty(b, h, d, dtype=torch.float32, device=dev) if output_final_state else None
-    with torch.cuda.device(dev):
+    with L.on(dev):
         L.check(lib.mmf_hgrn_recurrent(xc.data_ptr(), gc.data_ptr(), L.ptr(h0), o.data_ptr(), L.ptr(ht), b * h, t, d,
                                        L.dtype_id(x.dtype), L.stream()), "mmf_hgrn_recurrent")
     return o, ht
@@ -451,7 +451,7 @@ def hgrn_chunk(x, g, initial_state=None, output_final_state=False, chunk_size=64
         raise ValueError("chunk_size must lie in [1, 64]")
     nws = lib.mmf_hgrn_chunk_workspace_bytes(b * h, t, d, chunk_size)
     ws = torch.empty(nws // 4, dtype=torch.float32, device=dev) if nws else None    # per-segment carries (few KB)
-    with torch.cuda.device(dev):
+    with L.on(dev):
         L.check(lib.mmf_hgrn_chunk(xc.data_ptr(), gc.data_ptr(), L.ptr(h0), o.data_ptr(), L.ptr(ht), b * h, t, d,
                                    chunk_size, L.dtype_id(x.dtype), L.ptr(ws), L.stream()), "mmf_hgrn_chunk")
     return o, ht
@@ -490,7 +490,7 @@ def hgrn_gate(i, f, lower_bound=None, attention_mask=None):
     mk = _mask_rows(attention_mask, rows, dev)
     xo = torch.empty(i.shape, dtype=i.dtype, device=dev)
     go = torch.empty(i.shape, dtype=i.dtype, device=dev)
-    with torch.cuda.device(dev):
+    with L.on(dev):
         L.check(lib.mmf_hgrn_gate(i2.data_ptr(), ldi, f2.data_ptr(), ldf, L.ptr(lb), L.ptr(mk), xo.data_ptr(),
                                   go.data_ptr(), rows, d, L.dtype_id(i.dtype), L.stream()), "mmf_hgrn_gate")
     return xo, go
@@ -508,7 +508,7 @@ def hgrn_step(i, f, state, lower_bound=None, attention_mask=None):
     lb = lower_bound.detach().to(torch.float32).contiguous() if lower_bound is not None else None
     mk = _mask_rows(attention_mask, rows, dev)
     o = torch.empty(i.shape, dtype=i.dtype, device=dev)
-    with torch.cuda.device(dev):
+    with L.on(dev):
         L.check(lib.mmf_hgrn_step(i2.data_ptr(), ldi, f2.data_ptr(), ldf, L.ptr(lb), L.ptr(mk), state.data_ptr(),
                                   o.data_ptr(), rows, d, L.dtype_id(i.dtype), L.stream()), "mmf_hgrn_step")
     return o
@@ -522,7 +522,7 @@ def embedding(table, ids):
     idc = ids.reshape(-1).to(torch.int64).contiguous()
     tb = table.detach().contiguous()
     out = torch.empty(idc.numel(), tb.shape[1], dtype=tb.dtype, device=dev)
-    with torch.cuda.device(dev):
+    with L.on(dev):
         L.check(lib.mmf_embedding(tb.data_ptr(), idc.data_ptr(), out.data_ptr(), idc.numel(), tb.shape[1], tb.shape[0],
                                   L.dtype_id(tb.dtype), L.stream()), "mmf_embedding")
     return out.reshape(*ids.shape, tb.shape[1])
@@ -535,7 +535,7 @@ def argmax(logits):
     v = logits.shape[-1]
     l2 = _as_2d(logits)
     out = torch.empty(l2.shape[0], dtype=torch.int64, device=dev)
-    with torch.cuda.device(dev):
+    with L.on(dev):
         L.check(lib.mmf_argmax(l2.data_ptr(), v, l2.shape[0], v, out.data_ptr(), L.dtype_id(l2.dtype), L.stream()),
                 "mmf_argmax")
     return out.reshape(logits.shape[:-1])
@@ -562,7 +562,7 @@ def sample_top_p(logits, top_p, temperature, u, out=None, top_k=0):
         out = torch.empty(rows, dtype=torch.int64, device=dev)
     elif not (out.dtype == torch.int64 and out.device == dev and out.numel() == rows and out.is_contiguous()):
         raise L.MMFError("sample_top_p: out must be a contiguous int64 tensor with one element per row")
-    with torch.cuda.device(dev):
+    with L.on(dev):
         L.check(lib.mmf_sample_top_p(l2.data_ptr(), l2.stride(0), rows, v, float(temperature), float(top_p), int(top_k),
                                      u.data_ptr(), out.data_ptr(), L.dtype_id(l2.dtype), L.stream()), "mmf_sample_top_p")
     return out.reshape(logits.shape[:-1])
@@ -585,7 +585,7 @@ def cross_entropy(logits, labels, ignore_index=-100):
     if lab.numel() != l2.shape[0]:
         raise ValueError("one label per row of logits")
     rows = torch.empty(l2.shape[0], dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with L.on(dev):
         L.check(lib.mmf_cross_entropy_fwd(l2.data_ptr(), l2.stride(0), lab.data_ptr(), int(ignore_index), rows.data_ptr(),
                                           l2.shape[0], v, L.dtype_id(l2.dtype), L.stream()), "mmf_cross_entropy_fwd")
     counted = ((lab != ignore_index) & (lab >= 0) & (lab < v)).sum()
@@ -616,7 +616,7 @@ def short_conv(x, weight, bias=None, activation=True, cache=None):
     if cache is not None and not (cache.shape == (b, d, w2.shape[1]) and cache.dtype == x.dtype and cache.is_contiguous()
                                   and cache.device == dev):
         raise L.MMFError(f"short_conv: the cache must be a contiguous [{b}, {d}, {w2.shape[1]}] {x.dtype} tensor on {dev}")
-    with torch.cuda.device(dev):
+    with L.on(dev):
         L.check(lib.mmf_short_conv_fwd(xc.data_ptr(), w2.data_ptr(), L.ptr(b1), y.data_ptr(), L.ptr(cache), b, t, d, w2.shape[1],
                                        1 if activation else 0, L.dtype_id(x.dtype), L.stream()), "mmf_short_conv_fwd")
     return y
@@ -631,7 +631,7 @@ def short_conv_step(x, weight, bias, cache, activation=True):
         raise L.MMFError(f"short_conv_step: the cache must be a contiguous [{b}, {d}, {w2.shape[1]}] {x.dtype} tensor on {dev}")
     xc = x.contiguous()
     y = torch.empty_like(xc)
-    with torch.cuda.device(dev):
+    with L.on(dev):
         L.check(lib.mmf_short_conv_step(xc.data_ptr(), w2.data_ptr(), L.ptr(b1), cache.data_ptr(), y.data_ptr(), b, d, w2.shape[1],
                                         1 if activation else 0, L.dtype_id(x.dtype), L.stream()), "mmf_short_conv_step")
     return y
@@ -648,7 +648,7 @@ def short_conv_bwd(x, weight, bias, dy, activation=True):
     dpre = torch.empty(b, t, d, dtype=torch.float32, device=dev)
     part = torch.empty(lib.mmf_short_conv_bwd_groups(b * t), (w + 1) * d, dtype=torch.float32, device=dev)
     dwb = torch.empty((w + 1) * d, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with L.on(dev):
         L.check(lib.mmf_short_conv_bwd(xc.data_ptr(), w2.data_ptr(), L.ptr(b1), dyc.data_ptr(), dx.data_ptr(), dpre.data_ptr(),
                                        part.data_ptr(), dwb.data_ptr(), b, t, d, w, 1 if activation else 0, L.dtype_id(x.dtype),
                                        L.stream()), "mmf_short_conv_bwd")

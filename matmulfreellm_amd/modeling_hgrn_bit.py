@@ -25,6 +25,8 @@ from transformers.generation import GenerationMixin
 from transformers.modeling_outputs import BaseModelOutputWithPast, CausalLMOutputWithPast
 from transformers.modeling_utils import PreTrainedModel
 
+from . import _lib as L
+from . import block as native
 from . import functional as F_
 from .activations import swiglu
 from .attention import HGRNBitAttention
@@ -194,7 +196,8 @@ class HGRNBitModel(HGRNBitPreTrainedModel):
                                  output_attentions, output_hidden_states, return_dict)
 
     def _forward(self, train, input_ids, attention_mask, inputs_embeds, past_key_values, use_cache, output_attentions,
-                 output_hidden_states, return_dict):
+                 output_hidden_states, return_dict, final_norm=True):
+        """final_norm=False leaves the last norm to the caller (inference only: it folds it into the head)."""
         if output_attentions:
             warnings.warn("`HGRNBitModel` does not `output_attentions` now, setting it to `False`.")
         output_attentions = False
@@ -218,6 +221,13 @@ class HGRNBitModel(HGRNBitPreTrainedModel):
         if train:
             use_cache = False                                    # whole sequences, no recurrent-state cache
 
+        if not train:
+            done = self._forward_native(hidden_states, attention_mask, past_key_values, use_cache, output_hidden_states)
+            if done is not None:
+                hidden_states, past_key_values, all_hidden_states = done
+                return self._finish(hidden_states, past_key_values if use_cache else None, all_hidden_states, output_hidden_states,
+                                    return_dict, final_norm)
+
         if use_cache:
             if past_key_values is None:
                 past_key_values = [layer.attn.init_state(batch_size) for layer in self.layers]
@@ -240,11 +250,70 @@ class HGRNBitModel(HGRNBitPreTrainedModel):
                 hidden_states, attention_mask=attention_mask, past_key_values=past_key_values, use_cache=use_cache,
                 output_attentions=False, lower_bound=lower_bound)
 
-        hidden_states = self.norm(hidden_states)
+        return self._finish(hidden_states, past_key_values if use_cache else None, all_hidden_states, output_hidden_states,
+                            return_dict, final_norm)
+
+    def _forward_native(self, x, attention_mask, past_key_values, use_cache, output_hidden_states):
+        """All blocks through block.py's native calls: (hidden states, cache, per-layer hidden states), or None where the
+        first block has no native form.  A later block that has none runs as a module, on the same cache."""
+        if x.dim() != 3 or not x.is_cuda or x.numel() == 0 or native.global_hooks() or (past_key_values is not None and not use_cache):
+            return None
+        plan = native.BlockPlan.of(self.layers[0]) if len(self.layers) else None
+        B, T, H = x.shape
+        if plan is None or plan.dtype != x.dtype or plan.device != x.device or H != plan.H or (T > 1 and plan.mode != "fused_recurrent"):
+            return None
+        dev, fresh = x.device, None
+        if use_cache and past_key_values is None:
+            # one allocation for all layers' states; the first scan starts from zero without reading them
+            fresh = torch.empty(len(self.layers), B, plan.heads, plan.head_dim, dtype=torch.float32, device=dev)
+            past_key_values = RecurrentCache()
+            past_key_values.states = [(s,) for s in fresh.unbind(0)]
+        elif use_cache and not isinstance(past_key_values, RecurrentCache):
+            past_key_values = RecurrentCache.from_legacy_cache(past_key_values)
+        lbs = self.lower_bound_rows() if self.config.use_lower_bound else None
+        mask = F_._mask_rows(attention_mask, B * T, dev)
+        all_hidden_states = () if output_hidden_states else None
+        x = x.contiguous()
+        with L.on(dev):
+            stream, ws = L.stream(), native.workspace(plan, B * T)
+            spare, dims = None, plan.dims
+            for i, layer in enumerate(self.layers):
+                if output_hidden_states:
+                    all_hidden_states += (x,)
+                if i > 0:
+                    plan = native.BlockPlan.of(layer)
+                state = past_key_values[i][-1] if use_cache else None
+                fits = (plan is not None and plan.dtype == x.dtype and plan.device == dev and plan.dims == dims and plan.layer_idx == i
+                        and (T == 1 or plan.mode == "fused_recurrent"))
+                if fits and state is not None:
+                    fits = (state.dtype == torch.float32 and state.device == dev and state.is_contiguous()
+                            and state.numel() == B * plan.D)
+                lb = lbs[i] if lbs is not None else None
+                if not fits:
+                    if fresh is not None:
+                        state.zero_()
+                    seen = past_key_values._seen_tokens if use_cache else 0
+                    x = layer(x, attention_mask=attention_mask, past_key_values=past_key_values, use_cache=use_cache,
+                              output_attentions=False, lower_bound=lb)[0].contiguous()
+                    if use_cache:
+                        past_key_values._seen_tokens = seen
+                    continue
+                out = spare if spare is not None else torch.empty_like(x)
+                ht = state.data_ptr() if state is not None else None
+                native.forward(plan, x.data_ptr(), out.data_ptr(), B, T, lb.data_ptr() if lb is not None and i > 0 else None,
+                               L.ptr(mask), ht if fresh is None else None, ht, ws.data_ptr(), stream)
+                # the input's buffer serves the next block, unless somebody else holds it
+                spare = x if i > 0 and not output_hidden_states else None
+                x = out
+        if use_cache:
+            past_key_values._seen_tokens += 1
+        return x, past_key_values, all_hidden_states
+
+    def _finish(self, hidden_states, next_cache, all_hidden_states, output_hidden_states, return_dict, final_norm):
+        if final_norm:
+            hidden_states = self.norm(hidden_states)
         if output_hidden_states:
             all_hidden_states += (hidden_states,)
-
-        next_cache = past_key_values if use_cache else None
         if not return_dict:
             return tuple(x for x in [hidden_states, next_cache, all_hidden_states] if x is not None)
         return BaseModelOutputWithPast(last_hidden_state=hidden_states, past_key_values=next_cache,
@@ -333,14 +402,18 @@ class HGRNBitForCausalLM(HGRNBitPreTrainedModel, GenerationMixin):
         if labels is not None:
             logits_to_keep = 0                           # the loss scores every position
         return_dict = return_dict if return_dict is not None else bool(getattr(self.config, "return_dict", True))
-        outputs = self.model(input_ids=input_ids, attention_mask=attention_mask, inputs_embeds=inputs_embeds,
-                             past_key_values=past_key_values, use_cache=use_cache,
-                             output_attentions=output_attentions, output_hidden_states=output_hidden_states,
-                             return_dict=True)
+        fold = not train and self._folds_final_norm(output_hidden_states)
+        args = dict(input_ids=input_ids, attention_mask=attention_mask, inputs_embeds=inputs_embeds, past_key_values=past_key_values,
+                    use_cache=use_cache, output_attentions=output_attentions, output_hidden_states=output_hidden_states, return_dict=True)
+        outputs = self.model._forward(False, **args, final_norm=False) if fold else self.model(**args)
         hidden_states = outputs.last_hidden_state
         if logits_to_keep:
             hidden_states = hidden_states[:, -logits_to_keep:, :]
-        logits = self.lm_head(hidden_states)
+        if fold:
+            norm = self.model.norm
+            logits = self.lm_head.forward_fused(hidden_states, ("norm", norm.weight, norm.eps))
+        else:
+            logits = self.lm_head(hidden_states)
         loss = None
         if labels is not None:
             # as mmfreelm/models/hgrn_bit/modeling_hgrn_bit.py:388-397: position t is scored against token t + 1
@@ -356,6 +429,16 @@ class HGRNBitForCausalLM(HGRNBitPreTrainedModel, GenerationMixin):
             return tuple(x for x in (loss, logits, outputs.past_key_values, outputs.hidden_states) if x is not None)
         return CausalLMOutputWithPast(loss=loss, logits=logits, past_key_values=outputs.past_key_values,
                                       hidden_states=outputs.hidden_states, attentions=None)
+
+    def _folds_final_norm(self, output_hidden_states):
+        """Whether the last norm runs inside the head's quantiser, on the kept positions only: nobody else sees its output
+        (no hidden states asked for, no hook or replaced module in between) and the two norm weights share a dtype."""
+        norm, head = self.model.norm, self.lm_head
+        return (not output_hidden_states and not getattr(self.config, "output_hidden_states", False)
+                and type(self.model) is HGRNBitModel and type(norm) is RMSNorm and type(head) is BitLinear and type(head.norm) is RMSNorm
+                and not native.global_hooks() and all(native.hook_free(m) for m in (self.model, norm, head, head.norm))
+                and norm.weight is not None and head.norm.weight is not None and norm.weight.dtype == head.norm.weight.dtype
+                and head.in_features <= 8192)
 
     # ------------------------------------------------------------------ generation
     @torch.no_grad()

@@ -1,0 +1,66 @@
+"""The native block call against the module path it stands for, bit for bit: row counts on both sides of every switch (one
+launch per BitLinear, quantiser + contraction, swiglu epilogue), one token on a kept state, masks, inner norms that agree
+or differ, stacked segments that no tile width divides.  A hook anywhere in a block makes the model take the module path."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def build(dev, dtype, hidden, trained):
+    import matmulfreellm_amd as mm
+    torch.manual_seed(3)
+    model = mm.HGRNBitForCausalLM(mm.HGRNBitConfig(vocab_size=500, hidden_size=hidden, num_hidden_layers=3, bos_token_id=None,
+                                                   eos_token_id=None))
+    with torch.no_grad():
+        for name, p in model.named_parameters():
+            if trained and "norm" in name:
+                p.copy_(0.5 + torch.rand(p.shape))
+            if name.endswith("lower_bounds"):
+                p.copy_(torch.randn(p.shape))
+    return model.to(dev, dtype).eval()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("hidden,trained", [(160, True), (512, True), (160, False)])
+def test_native_block_equals_the_module_path(dev, dtype, hidden, trained):
+    model = build(dev, dtype, hidden, trained)
+    with torch.no_grad():
+        for b, t, masked in [(1, 1, False), (1, 5, False), (2, 4, True), (3, 3, False), (1, 77, False), (3, 100, True), (2, 257, False)]:
+            ids = torch.randint(0, 500, (b, t), device=dev)
+            mask = (torch.arange(t, device=dev) >= torch.arange(b, device=dev).view(-1, 1) % t).long() if masked else None
+            step = torch.randint(0, 500, (b, 1), device=dev)
+            got = {}
+            for path in ("native", "modules"):
+                hooks = [layer.attn.g_norm.register_forward_hook(lambda *a: None) for layer in model.model.layers] \
+                    if path == "modules" else []
+                out = model(input_ids=ids, attention_mask=mask, use_cache=True, output_hidden_states=masked)
+                first = [s[-1].clone() for s in out.past_key_values]
+                nxt = model(input_ids=step, past_key_values=out.past_key_values, use_cache=True)
+                keep = torch.ones_like(step)
+                keep[0] = 0
+                last = model(input_ids=step, attention_mask=keep, past_key_values=nxt.past_key_values, use_cache=True)
+                got[path] = [out.logits, *first, nxt.logits, last.logits, *(s[-1] for s in last.past_key_values),
+                             *(out.hidden_states or ())]
+                for h in hooks:
+                    h.remove()
+            for i, (a, r) in enumerate(zip(got["native"], got["modules"])):
+                assert torch.equal(a, r), (b, t, masked, i)
+
+
+def test_a_written_or_replaced_parameter_is_seen(dev):
+    model = build(dev, torch.bfloat16, 160, True)
+    ids = torch.randint(0, 500, (1, 20), device=dev)
+    attn = model.model.layers[1].attn
+    with torch.no_grad():
+        logits = [model(input_ids=ids).logits]
+        attn.f_proj.norm.weight.mul_(1.5)
+        logits.append(model(input_ids=ids).logits)
+        attn.o_proj.weight = torch.nn.Parameter(torch.randn_like(attn.o_proj.weight))
+        logits.append(model(input_ids=ids).logits)
+        attn.g_norm.eps = 0.5
+        logits.append(model(input_ids=ids).logits)
+        hook = attn.g_norm.register_forward_hook(lambda *a: None)
+        assert torch.equal(logits[-1], model(input_ids=ids).logits)
+        hook.remove()
+    assert not any(torch.equal(a, b) for a, b in zip(logits, logits[1:]))
