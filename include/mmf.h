@@ -355,6 +355,11 @@ int64_t mmf_decode_layers_words(int H, int D, int I);
 int mmf_decode_layers(const void* phases, int n_layers, const void* table, const int64_t* tok, int64_t vocab, uint32_t* words,
                       void* h_out, const void* head, void* logits, uint64_t* am_words, int64_t* tok_out, uint32_t* epoch, int* err,
                       int H, int D, int I, int spin, int dtype, void* stream);
+/* The same with the number of inner norms behind an i/f/g record: 1, or 3 when i, f and g have norms of their own (norm_w of
+ * those records then points to [3, K] weights). */
+int mmf_decode_layers_norms(int norms, const void* phases, int n_layers, const void* table, const int64_t* tok, int64_t vocab,
+                            uint32_t* words, void* h_out, const void* head, void* logits, uint64_t* am_words, int64_t* tok_out,
+                            uint32_t* epoch, int* err, int H, int D, int I, int spin, int dtype, void* stream);
 
 /* ---- stacked projections whose inner norms differ (a trained checkpoint's i, f and g): one row, three norm weights
  * mmf_rmsnorm_quant_multi: mmf_rmsnorm_quant_fused with the norm prologue (w1, eps1), quantised under three norm weights:

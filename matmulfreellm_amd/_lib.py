@@ -40,6 +40,8 @@ SIGNATURES = {
     "mmf_decode_layers_words": (_i64, [_i32, _i32, _i32]),
     "mmf_decode_layers": (_i32, [_ptr, _i32, _ptr, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr,
                                  _i32, _i32, _i32, _i32, _i32, _ptr]),
+    "mmf_decode_layers_norms": (_i32, [_i32, _ptr, _i32, _ptr, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr,
+                                       _i32, _i32, _i32, _i32, _i32, _ptr]),
     "mmf_decode_layers_trace_words": (_i32, []),
     "mmf_decode_layers_traced": (_i32, [_ptr, _i32, _ptr, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr,
                                         _i32, _i32, _i32, _i32, _i32, _i32, _ptr]),

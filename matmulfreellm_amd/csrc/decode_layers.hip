@@ -61,7 +61,7 @@ constexpr int kItems = 8;                      // (row-group, segment) items of 
 
 struct Phase {                // one fused BitLinear; four per layer: i/f/g, o, gate, down
     const void* w1;           // weight of the norm in front of the BitLinear (null for down)
-    const void* norm_w;       // the BitLinear's own norm weight
+    const void* norm_w;       // the BitLinear's own norm weight (i/f/g of a kernel built with three: [3, K])
     const uint4* packed;
     const float* wdeq;
     const float* lb;          // i/f/g: lower bound [D] or null
@@ -137,8 +137,8 @@ __device__ __forceinline__ void best_take(Best& b, float v, uint32_t i) {
 
 struct Small {
     double sum1[kNW], sum2[kNW];             // per-wave partial sums of squares
-    float amax[kNW];
-    int qs[kNW];                             // per-wave sums of codes
+    float amax[3][kNW];                      // (i/f/g with three norms: one row of partials each)
+    int qs[3][kNW];                          // per-wave sums of codes
     int part[kItems][8][2 * kNW];            // [row-group x segment][row][wave x lane half] partial dot products
     float best_v[kNW];
     uint32_t best_i[kNW];
@@ -224,7 +224,10 @@ __device__ __forceinline__ Geo make_geo(int K, int N, int kind, int wave) {
     return g;
 }
 
-template <typename T, class S, bool TRACE>
+// NORMS = 3: the i, f and g projections have inner norms of their own, as in a trained checkpoint.  The i/f/g link then
+// scales its row by three norm weights behind one rstd, exchanges three maxima where it exchanged one, and keeps three rows of
+// codes; its weights, hand-offs and barriers are the same.  Measured at the 1.3B shape: MULTI_NORM_US.
+template <typename T, class S, bool TRACE, int NORMS>
 __global__ __launch_bounds__(kNT) void decode_layers_kernel(LayersArgs a) {
     extern __shared__ __align__(16) unsigned char dyn[];
     __shared__ Small sm;
@@ -359,7 +362,10 @@ __global__ __launch_bounds__(kNT) void decode_layers_kernel(LayersArgs a) {
                 const int el = q * 512 + lane * 8;
                 const uint32_t off = (uint32_t)(g.kb0 * 128 + (g.even || el < g.nkb * 128 ? el : 0)) * 2u;
                 if constexpr (KIND != K_DOWN) dma16(reinterpret_cast<const void*>(uni64(rc)), off, nrm_w1 + (wave * a.nqmax + q) * 1024);
-                dma16(reinterpret_cast<const void*>(uni64(rc + 8)), off, nrm_nw + (wave * a.nqmax + q) * 1024);
+#pragma unroll
+                for (int n = 0; n < (KIND == K_IFG ? NORMS : 1); ++n)
+                    dma16(reinterpret_cast<const void*>(uni64(rc + 8)), off + (uint32_t)(n * Hh) * 2u,
+                          nrm_nw + (wave * a.nqmax + n * g.nq + q) * 1024);
             }
         }
     };
@@ -419,10 +425,10 @@ __global__ __launch_bounds__(kNT) void decode_layers_kernel(LayersArgs a) {
     };
 
     // the integer result of item `it`, row `row`: the waves' partial sums less the row's code sum (weights are stored as t + 1)
-    auto total = [&](int it, int row) -> int {
+    auto total = [&](int it, int row, int n = 0) -> int {
         const int4 p0 = *reinterpret_cast<const int4*>(&sm.part[it][row][0]);
         const int4 p1 = *reinterpret_cast<const int4*>(&sm.part[it][row][4]);
-        const int4 qv = *reinterpret_cast<const int4*>(&sm.qs[0]);
+        const int4 qv = *reinterpret_cast<const int4*>(&sm.qs[n][0]);
         return ((p0.x + p0.y) + (p0.z + p0.w)) + ((p1.x + p1.y) + (p1.z + p1.w)) - ((qv.x + qv.y) + (qv.z + qv.w));
     };
     // Two neighbouring rows' words become one 8-byte store by the even row (fewer, wider stores travel faster); `even_active`:
@@ -456,6 +462,7 @@ __global__ __launch_bounds__(kNT) void decode_layers_kernel(LayersArgs a) {
         };
         constexpr bool HAS_AUX = KIND == K_O || KIND == K_GATE, HAS_W1 = KIND != K_DOWN;
         constexpr int NPK = KIND == K_DOWN ? NP : NPH;                       // passes this link's row can take
+        constexpr int NN = KIND == K_IFG ? NORMS : 1;                        // inner norms, and so rows of codes
         const int l = ln >> 2;
         const Geo g = geo(kc, ln);
         stamp(ln, 0);
@@ -616,44 +623,59 @@ __global__ __launch_bounds__(kNT) void decode_layers_kernel(LayersArgs a) {
         const double tot2 = (sm.sum2[0] + sm.sum2[1]) + (sm.sum2[2] + sm.sum2[3]);
         const float rstd = mmf_rstd(tot2, g.K, inv_K, __uint_as_float(uni32(rc + 56)));
         stamp(ln, 3);
-        float amax = 0.0f;
+        float amax[NN], yv[NN][NPK][4];
+#pragma unroll
+        for (int n = 0; n < NN; ++n) amax[n] = 0.0f;
 #pragma unroll
         for (int v = 0; v < NPK; ++v) {
             if (v < g.np) {
-                Raw4<T> raw;
-                raw.v = *reinterpret_cast<const uint2*>(my_nw + v * 512);
-                float wv[4];
-                raw4_unpack<T>(raw, wv);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float y = has[v] ? __fmul_rn(__fmul_rn(xv[v][i], rstd), wv[i]) : 0.0f;
-                    xv[v][i] = y;
-                    amax = fmaxf(amax, fabsf(y));
+                for (int n = 0; n < NN; ++n) {
+                    Raw4<T> raw;
+                    raw.v = *reinterpret_cast<const uint2*>(my_nw + (NN > 1 ? n * g.nq * 1024 : 0) + v * 512);
+                    float wv[4];
+                    raw4_unpack<T>(raw, wv);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float y = has[v] ? __fmul_rn(__fmul_rn(xv[v][i], rstd), wv[i]) : 0.0f;
+                        yv[n][v][i] = y;
+                        amax[n] = fmaxf(amax[n], fabsf(y));
+                    }
                 }
             }
         }
         // this wave is done with its norm-weight regions: the next link's may come in
         if (more) dma_norm_next();
-        amax = mmf_wave_max(amax);
-        if (pl == 0) sm.amax[wave] = amax;
-        lds_barrier();
-        amax = fmaxf(fmaxf(sm.amax[0], sm.amax[1]), fmaxf(sm.amax[2], sm.amax[3]));
-        stamp(ln, 4);
-        const float scale = mmf_127_over(fmaxf(amax, 1e-5f));
-        int qs = 0;
 #pragma unroll
-        for (int v = 0; v < NPK; ++v) {
-            if (v < g.np) {
-                uint32_t packed4 = 0;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) packed4 |= (uint32_t)(mmf_code(xv[v][i], scale) & 0xff) << (8 * i);
-                qs = __builtin_amdgcn_sdot4((int)packed4, 0x01010101, qs, false);      // the sum of the four codes
-                if (has[v]) *reinterpret_cast<uint32_t*>(qbuf + k0[v]) = packed4;
-            }
+        for (int n = 0; n < NN; ++n) {
+            amax[n] = mmf_wave_max(amax[n]);
+            if (pl == 0) sm.amax[n][wave] = amax[n];
         }
-        qs = mmf_wave_sum(qs);
-        if (pl == 0) sm.qs[wave] = qs;
-        const float deq = mmf_rcp_pos(scale);       // needed by the epilogue only
+        lds_barrier();
+        float scale[NN], deq[NN];                   // deq is needed by the epilogue only
+        stamp(ln, 4);
+#pragma unroll
+        for (int n = 0; n < NN; ++n) {
+            amax[n] = fmaxf(fmaxf(sm.amax[n][0], sm.amax[n][1]), fmaxf(sm.amax[n][2], sm.amax[n][3]));
+            scale[n] = mmf_127_over(fmaxf(amax[n], 1e-5f));
+        }
+#pragma unroll
+        for (int n = 0; n < NN; ++n) {
+            int qs = 0;
+#pragma unroll
+            for (int v = 0; v < NPK; ++v) {
+                if (v < g.np) {
+                    uint32_t packed4 = 0;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) packed4 |= (uint32_t)(mmf_code(yv[n][v][i], scale[n]) & 0xff) << (8 * i);
+                    qs = __builtin_amdgcn_sdot4((int)packed4, 0x01010101, qs, false);      // the sum of the four codes
+                    if (has[v]) *reinterpret_cast<uint32_t*>(qbuf + (NN > 1 ? n * Hh : 0) + k0[v]) = packed4;
+                }
+            }
+            qs = mmf_wave_sum(qs);
+            if (pl == 0) sm.qs[n][wave] = qs;
+            deq[n] = mmf_rcp_pos(scale[n]);
+        }
         stamp(ln, 5);
 
         const uint32_t tag = tag_of(ln);
@@ -691,13 +713,16 @@ __global__ __launch_bounds__(kNT) void decode_layers_kernel(LayersArgs a) {
                 const unsigned char* src = wbuf_of(kc, pass) + lane * 16;
                 const int nit = ng * g.R;
                 uint4 wq[MAXIT][NQ];
-                int4 qv[NQ][4];
+                int4 qv[NN][NQ][4];
 #pragma unroll
                 for (int q = 0; q < NQ; ++q) {
                     const int kraw = 4 * q + slot;
                     const int kb = g.kb0 + (g.even || kraw < g.nkb ? kraw : g.nkb - 1);
 #pragma unroll
-                    for (int s4 = 0; s4 < 4; ++s4) qv[q][s4] = *reinterpret_cast<const int4*>(qbuf + kb * 128 + s4 * 32 + half * 16);
+                    for (int n = 0; n < NN; ++n)
+#pragma unroll
+                        for (int s4 = 0; s4 < 4; ++s4)
+                            qv[n][q][s4] = *reinterpret_cast<const int4*>(qbuf + (NN > 1 ? n * Hh : 0) + kb * 128 + s4 * 32 + half * 16);
                 }
 #pragma unroll
                 for (int it = 0; it < MAXIT; ++it)
@@ -711,7 +736,7 @@ __global__ __launch_bounds__(kNT) void decode_layers_kernel(LayersArgs a) {
                 for (int it = 0; it < MAXIT; ++it) {
                     acc[it] = 0;
 #pragma unroll
-                    for (int q = 0; q < NQ; ++q) acc[it] = mmf_dot_block_regs(qv[q], wq[it][q], acc[it]);
+                    for (int q = 0; q < NQ; ++q) acc[it] = mmf_dot_block_regs(qv[NN > 1 ? it % 3 : 0][q], wq[it][q], acc[it]);
                     acc[it] += mmf_dpp<0x128>(acc[it]);                      // the other half of the 16 lanes (rotate by 8)
                 }
 #pragma unroll
@@ -732,7 +757,7 @@ __global__ __launch_bounds__(kNT) void decode_layers_kernel(LayersArgs a) {
                             const int kb = g.kb0 + (live ? kraw : g.nkb - 1);
                             uint4 wq = *reinterpret_cast<const uint4*>(src + (it * g.nq + q) * 1024);
                             if (!live) wq = make_uint4(0u, 0u, 0u, 0u);
-                            acc = mmf_dot_block(qbuf, wq, kb, half, acc);
+                            acc = mmf_dot_block(qbuf + (NN > 1 ? (it % 3) * Hh : 0), wq, kb, half, acc);
                         }
                     }
                     acc += mmf_dpp<0x128>(acc);                              // the other half of the 16 lanes (rotate by 8)
@@ -756,9 +781,10 @@ __global__ __launch_bounds__(kNT) void decode_layers_kernel(LayersArgs a) {
                     if (gl >= ng) break;
                     const int ch = ((int)blockIdx.x + kWGs * (g0 + gl)) * 8 + row;
                     const float lbv = g0 + gl == 0 ? lb[0] : lb[1], stv = g0 + gl == 0 ? st[0] : st[1];
-                    const int tot = total(gl * 3 + (r3 < 3 ? r3 : 0), row);
+                    const int tot = total(gl * 3 + (r3 < 3 ? r3 : 0), row, NN > 1 && r3 < 3 ? r3 : 0);
+                    const float dq = NN == 1 || r3 == 0 ? deq[0] : r3 == 1 ? deq[NN > 1 ? 1 : 0] : deq[NN > 1 ? 2 : 0];
                     const float wdv = r3 == 0 ? wdk[KIND][0] : r3 == 1 ? wdk[KIND][1] : wdk[KIND][2];
-                    const float res = __fmul_rn(__fmul_rn((float)tot, deq), wdv);
+                    const float res = __fmul_rn(__fmul_rn((float)tot, dq), wdv);
                     const float v16 = mmf_round_to<T>(res);                       // iv on the i lanes, fv on the f lanes
                     const float ex = __fadd_rn(1.0f, mmf_exp(-v16));
                     float sgm = mmf_rcp_pos(ex);                                 // sigmoid(fv) on the f lanes
@@ -776,7 +802,7 @@ __global__ __launch_bounds__(kNT) void decode_layers_kernel(LayersArgs a) {
                 for (int gl = wave * 8 + (pl >> 3); gl < ng; gl += 8 * kNW) {
                     const int ch = ((int)blockIdx.x + kWGs * (g0 + gl)) * 8 + row;
                     if (ch < g.Nseg) {
-                        const float o = __fmul_rn(__fmul_rn((float)total(gl, row), deq), wdk[KIND][0]);
+                        const float o = __fmul_rn(__fmul_rn((float)total(gl, row), deq[0]), wdk[KIND][0]);
                         static_cast<T*>(a.logits)[ch] = mmf_from_float<T>(o);
                         const float ov = mmf_round_to<T>(o);
                         if (ov == ov) best_take(best, ov, (uint32_t)ch);
@@ -790,9 +816,9 @@ __global__ __launch_bounds__(kNT) void decode_layers_kernel(LayersArgs a) {
                 for (int gl = wave; gl < ng; gl += kNW) {
                     const int ch = ((int)blockIdx.x + kWGs * (g0 + gl)) * 8 + row;
                     const bool live = ch < g.Nseg;
-                    float o = __fmul_rn(__fmul_rn((float)total(gl * g.R, row), deq), wdk[KIND][0]);
+                    float o = __fmul_rn(__fmul_rn((float)total(gl * g.R, row), deq[0]), wdk[KIND][0]);
                     if constexpr (KIND == K_GATE) {
-                        const float u = mmf_round_to<T>(__fmul_rn(__fmul_rn((float)total(gl * 2 + 1, row), deq), wdk[KIND][1]));
+                        const float u = mmf_round_to<T>(__fmul_rn(__fmul_rn((float)total(gl * 2 + 1, row), deq[0]), wdk[KIND][1]));
                         const float gt = mmf_round_to<T>(o);
                         o = __fdiv_rn(__fmul_rn(gt, u), __fadd_rn(1.0f, mmf_exp(-gt)));
                     }
@@ -870,9 +896,9 @@ __global__ __launch_bounds__(kNT) void decode_layers_kernel(LayersArgs a) {
     if (blockIdx.x == 0 && threadIdx.x == 0) *a.epoch = e + 4u * (uint32_t)a.n_layers + 2u;
 }
 
-template <typename T, class S, bool TRACE>
+template <typename T, class S, bool TRACE, int NORMS>
 int launch_one(const LayersArgs& a, size_t lds, hipStream_t s) {
-    auto kern = decode_layers_kernel<T, S, TRACE>;
+    auto kern = decode_layers_kernel<T, S, TRACE, NORMS>;
     static size_t allowed = 0;                                   // per instantiation; the attribute only ever grows
     if (lds > allowed) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -884,10 +910,10 @@ int launch_one(const LayersArgs& a, size_t lds, hipStream_t s) {
     return 0;
 }
 
-template <typename T, bool TRACE>
+template <typename T, bool TRACE, int NORMS>
 int launch_layers(LayersArgs a, hipStream_t s) {
     const int kmax = a.H > a.I ? a.H : a.I;
-    a.nqmax = quads_of(kmax);
+    a.nqmax = quads_of(kmax) > NORMS * quads_of(a.H) ? quads_of(kmax) : NORMS * quads_of(a.H);
     // weight loads (1 KiB each) per wave a link kind needs when all its row-groups are resident: buffer A serves i/f/g
     // and gate/up, buffer B o_proj and down_proj; the lm_head takes what they hold, pass by pass
     const int nqh = quads_of(a.H), nqi = quads_of(a.I);
@@ -898,17 +924,18 @@ int launch_layers(LayersArgs a, hipStream_t s) {
     if (a.itemsA > 16 || a.itemsB > 16 || ngh > 2 || ngi * 2 > kItems) return MMF_ERR_WIDE;
     const uint32_t tab = (uint32_t)mmf_round_up((4 * a.n_layers + 1) * (int64_t)sizeof(Phase), 16);
     a.off_q = tab;
-    a.off_nrm = a.off_q + (uint32_t)mmf_round_up(kmax, 16);
+    a.off_nrm = a.off_q + (uint32_t)mmf_round_up(kmax > NORMS * a.H ? kmax : NORMS * a.H, 16);
     a.off_w = a.off_nrm + 2u * kNW * (uint32_t)a.nqmax * 1024u;
     const size_t lds = a.off_w + (size_t)kNW * (a.itemsA + a.itemsB) * 1024u;
-    if (a.H == 2048 && a.I == 5632) return launch_one<T, StaticShape<2048, 5632>, TRACE>(a, lds, s);
-    if (a.H == 2560 && a.I == 6912) return launch_one<T, StaticShape<2560, 6912>, TRACE>(a, lds, s);
-    return launch_one<T, DynShape, TRACE>(a, lds, s);
+    if (a.H == 2048 && a.I == 5632) return launch_one<T, StaticShape<2048, 5632>, TRACE, NORMS>(a, lds, s);
+    if (a.H == 1024 && a.I == 2816) return launch_one<T, StaticShape<1024, 2816>, TRACE, NORMS>(a, lds, s);
+    if (a.H == 2560 && a.I == 6912) return launch_one<T, StaticShape<2560, 6912>, TRACE, NORMS>(a, lds, s);
+    return launch_one<T, DynShape, TRACE, NORMS>(a, lds, s);
 }
 
 int decode_layers_entry(const void* phases, int n_layers, const void* table, const int64_t* tok, int64_t vocab, uint32_t* words,
                         void* h_out, const void* head, void* logits, uint64_t* am_words, int64_t* tok_out, uint32_t* epoch, int* err,
-                        int64_t* trace, int H, int D, int I, int spin, const int* delay, int dtype, void* stream_) {
+                        int64_t* trace, int norms, int H, int D, int I, int spin, const int* delay, int dtype, void* stream_) {
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     if (!phases || n_layers <= 0 || !table || !tok || vocab <= 0 || !words || !h_out || !epoch || !err || H <= 0 || D <= 0 || I <= 0 ||
         spin <= 0 || !delay)
@@ -933,13 +960,13 @@ int decode_layers_entry(const void* phases, int n_layers, const void* table, con
     for (int k = 0; k < 5; ++k) a.delay[k] = delay[k];
     if (trace) {
         switch (dtype) {
-            case MMF_BF16: return launch_layers<bf16_t, true>(a, stream);
-            case MMF_F16: return launch_layers<f16_t, true>(a, stream);
+            case MMF_BF16: return launch_layers<bf16_t, true, 1>(a, stream);
+            case MMF_F16: return launch_layers<f16_t, true, 1>(a, stream);
         }
     } else {
         switch (dtype) {
-            case MMF_BF16: return launch_layers<bf16_t, false>(a, stream);
-            case MMF_F16: return launch_layers<f16_t, false>(a, stream);
+            case MMF_BF16: return norms == 3 ? launch_layers<bf16_t, false, 3>(a, stream) : launch_layers<bf16_t, false, 1>(a, stream);
+            case MMF_F16: return norms == 3 ? launch_layers<f16_t, false, 3>(a, stream) : launch_layers<f16_t, false, 1>(a, stream);
         }
     }
     return MMF_ERR_ARG;
@@ -955,9 +982,10 @@ int64_t mmf_decode_layers_words(int H, int D, int I) { return (int64_t)kRep * (3
 
 int mmf_decode_layers_copies(void) { return kRep; }
 
-int mmf_decode_layers(const void* phases, int n_layers, const void* table, const int64_t* tok, int64_t vocab, uint32_t* words,
+int mmf_decode_layers_norms(int norms, const void* phases, int n_layers, const void* table, const int64_t* tok, int64_t vocab, uint32_t* words,
                       void* h_out, const void* head, void* logits, uint64_t* am_words, int64_t* tok_out, uint32_t* epoch, int* err,
                       int H, int D, int I, int spin, int dtype, void* stream) {
+    if (norms != 1 && norms != 3) return MMF_ERR_ARG;
     // hold-back of the first poll per kind of link (i/f/g, o_proj, gate/up, down_proj, lm_head); MMF_DECODE_POLL_DELAY
     // ("a" or "a,b,c,d,e") overrides the tuned values
     static const struct Delays {
@@ -977,7 +1005,14 @@ int mmf_decode_layers(const void* phases, int n_layers, const void* table, const
     } delays;
     const int* delay = delays.d;
     return decode_layers_entry(phases, n_layers, table, tok, vocab, words, h_out, head, logits, am_words, tok_out, epoch, err, nullptr,
-                               H, D, I, spin, delay, dtype, stream);
+                               norms, H, D, I, spin, delay, dtype, stream);
+}
+
+int mmf_decode_layers(const void* phases, int n_layers, const void* table, const int64_t* tok, int64_t vocab, uint32_t* words,
+                      void* h_out, const void* head, void* logits, uint64_t* am_words, int64_t* tok_out, uint32_t* epoch, int* err,
+                      int H, int D, int I, int spin, int dtype, void* stream) {
+    return mmf_decode_layers_norms(1, phases, n_layers, table, tok, vocab, words, h_out, head, logits, am_words, tok_out, epoch, err, H, D,
+                                   I, spin, dtype, stream);
 }
 
 int mmf_decode_layers_trace_words(void) { return kTraceWGs * kTraceLinks * kTraceStamps; }
@@ -987,7 +1022,7 @@ int mmf_decode_layers_traced(const void* phases, int n_layers, const void* table
                              int64_t* trace, int H, int D, int I, int spin, int delay, int dtype, void* stream) {
     if (!trace) return MMF_ERR_ARG;
     const int d[5] = {delay, delay, delay, delay, delay};
-    return decode_layers_entry(phases, n_layers, table, tok, vocab, words, h_out, head, logits, am_words, tok_out, epoch, err, trace, H, D,
+    return decode_layers_entry(phases, n_layers, table, tok, vocab, words, h_out, head, logits, am_words, tok_out, epoch, err, trace, 1, H, D,
                                I, spin, d, dtype, stream);
 }
 

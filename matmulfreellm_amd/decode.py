@@ -80,7 +80,9 @@ class DecodeEngine:
             ent = {
                 "attn_norm": blk.attn_norm.weight.detach(), "mlp_norm": blk.mlp_norm.weight.detach(),
                 "g_norm": a.g_norm.weight.detach(), "g_eps": float(a.g_norm.eps),
-                "ifg": a._stacked_ifg(),
+                "ifg": a._stacked_weight() if self._stackable(a) else None,
+                # None where the three inner norms agree (one row of codes serves i, f and g), else the three weights
+                "norms": None if a._stacked_ifg() is not None else [p.norm.weight.detach() for p in (a.i_proj, a.f_proj, a.g_proj)],
                 "projs": [(p.packed_weight(), p.norm.weight.detach(), self._eps_of(p)) for p in (a.i_proj, a.f_proj, a.g_proj)],
                 "o": (a.o_proj.packed_weight(), a.o_proj.norm.weight.detach(), self._eps_of(a.o_proj)),
                 "gate": (m.gate_proj.packed_weight(), m.gate_proj.norm.weight.detach(), self._eps_of(m.gate_proj)),
@@ -109,9 +111,11 @@ class DecodeEngine:
         self.zb = z(B, I)
         self.logits = z(B, self.V)
         kmax = max(H, D, I)
-        self.q = torch.zeros(self.lib.mmf_codes_bytes(B, kmax, 1), dtype=torch.int8, device=dev)
-        self.deq = z(B, dtype=torch.float32)
-        self.qsum = torch.zeros(B, dtype=torch.int32, device=dev)
+        # codes, scales and code sums of one row block, or of the three that i, f and g with norms of their own take
+        nbytes = max(self.lib.mmf_codes_bytes(B, kmax, 1), 3 * self.lib.mmf_codes_bytes(B, H, 1))
+        self.q = torch.zeros(nbytes, dtype=torch.int8, device=dev)
+        self.deq = z(3 * B, dtype=torch.float32)
+        self.qsum = torch.zeros(3 * B, dtype=torch.int32, device=dev)
         self.gemv = B <= F_.GEMV_MAX_M
         self.fused = fuse and self._can_fuse()
         self.fused_mfma = fuse and self._can_fuse_mfma()
@@ -122,6 +126,12 @@ class DecodeEngine:
         if self.resident:
             self._build_resident()
         self.graph = None
+
+    @classmethod
+    def _stackable(cls, attn):
+        projs = (attn.i_proj, attn.f_proj, attn.g_proj)
+        return (attn.input_dim % 32 == 0 and all(p.bias is None and p.norm.weight is not None for p in projs)
+                and len({cls._eps_of(p) for p in projs}) == 1)
 
     @staticmethod
     def _eps_of(p):
@@ -173,19 +183,24 @@ class DecodeEngine:
     def _build_resident(self):
         H, D, I = self.H, self.D, self.I
         assert self.lib.mmf_decode_layers_phase_bytes() == ctypes.sizeof(_Phase)
+        # a layer whose i, f and g have inner norms of their own: every layer then runs with three (equal ones repeated)
+        self.norms = 3 if any(ent["norms"] is not None for ent in self.layers) else 1
         table = (_Phase * (4 * self.L + 1))()            # the last record is the final norm + lm_head
 
         def fill(rec, w1, eps1, pw_nw_eps, k, n, lb=None, state=None):
             pw, nw, eps = pw_nw_eps
             rec.w1 = w1.data_ptr() if w1 is not None else None
             rec.norm_w, rec.packed, rec.wdeq = nw.data_ptr(), pw.packed.data_ptr(), pw.wdeq.data_ptr()
+            assert nw.is_contiguous() and (w1 is None or w1.is_contiguous())
             rec.lb = lb.data_ptr() if lb is not None else None
             rec.state = state.data_ptr() if state is not None else None
             rec.inv_K, rec.eps, rec.eps1, rec.K, rec.N, rec.seg_rows = 1.0 / k, eps, eps1, k, n, pw.seg_rows
 
         for li, ent in enumerate(self.layers):
-            fill(table[4 * li], ent["attn_norm"], self.eps, (ent["ifg"], ent["projs"][0][1], ent["projs"][0][2]), H, 3 * D,
-                 ent["lb"], ent["state"])
+            nw = ent["projs"][0][1]
+            if self.norms == 3:
+                nw = ent["norm3"] = torch.stack(ent["norms"] or [nw] * 3)
+            fill(table[4 * li], ent["attn_norm"], self.eps, (ent["ifg"], nw, ent["projs"][0][2]), H, 3 * D, ent["lb"], ent["state"])
             fill(table[4 * li + 1], ent["g_norm"], ent["g_eps"], ent["o"], D, H)
             fill(table[4 * li + 2], ent["mlp_norm"], self.eps, ent["gate"], H, 2 * I)
             fill(table[4 * li + 3], None, 0.0, ent["down"], I, H)
@@ -212,8 +227,10 @@ class DecodeEngine:
                 self.h.data_ptr(), head, self.logits.data_ptr(), self.am_words.data_ptr(), self.tok.data_ptr(),
                 self.epoch.data_ptr(), self.err.data_ptr())
         if trace is None:
-            L.check(self.lib.mmf_decode_layers(*args, self.H, self.D, self.I, self.SPIN, self.dt_id, L.stream()), "mmf_decode_layers")
+            L.check(self.lib.mmf_decode_layers_norms(self.norms, *args, self.H, self.D, self.I, self.SPIN, self.dt_id, L.stream()),
+                    "mmf_decode_layers_norms")
         else:
+            assert self.norms == 1, "the traced kernel is built for shared inner norms"
             L.check(self.lib.mmf_decode_layers_traced(*args, trace.data_ptr(), self.H, self.D, self.I, self.SPIN, delay, self.dt_id,
                                                       L.stream()), "mmf_decode_layers_traced")
 
@@ -263,9 +280,17 @@ class DecodeEngine:
                                       self.dt_id, s), "mmf_embedding")
         g_buf = self.ifg.view(-1)[:B * D].view(B, D)
         for ent in self.layers:
-            self._fused(self.NORM, self.E_STEP, self.h, H, None, 0, None, ent["attn_norm"], self.eps,
-                        (ent["ifg"], ent["projs"][0][1], ent["projs"][0][2]), self.o, g_buf, ent["lb"], ent["state"],
-                        3 * D, H)
+            if ent["norms"] is not None:
+                pw, n = ent["ifg"], ent["norms"]
+                L.check(lib.mmf_bitlinear_gemv_multi(
+                    self.E_STEP, self.h.data_ptr(), H, ent["attn_norm"].data_ptr(), self.eps, n[0].data_ptr(), n[1].data_ptr(),
+                    n[2].data_ptr(), ent["projs"][0][2], pw.packed.data_ptr(), pw.wdeq.data_ptr(), pw.seg_rows, self.o.data_ptr(),
+                    g_buf.data_ptr(), L.ptr(ent["lb"]), ent["state"].data_ptr(), B, H, 3 * D, self.dt_id, L.dtype_id(n[0].dtype), s),
+                    "mmf_bitlinear_gemv_multi")
+            else:
+                self._fused(self.NORM, self.E_STEP, self.h, H, None, 0, None, ent["attn_norm"], self.eps,
+                            (ent["ifg"], ent["projs"][0][1], ent["projs"][0][2]), self.o, g_buf, ent["lb"], ent["state"],
+                            3 * D, H)
             self._fused(self.GATEDNORM, self.E_PLAIN, g_buf, D, self.o, D, None, ent["g_norm"], ent["g_eps"], ent["o"],
                         self.a, None, None, None, H, D)
             self._fused(self.RESNORM, self.E_SWIGLU, self.a, H, self.h, H, self.res, ent["mlp_norm"], self.eps,
@@ -311,8 +336,19 @@ class DecodeEngine:
         ifg, y = self.ifg.data_ptr(), self.y.data_ptr()
         for ent in self.layers:
             nw, eps = ent["projs"][0][1], ent["projs"][0][2]
-            self._qfused(1, self.h.data_ptr(), H, None, 0, None, 0, None, ent["attn_norm"], self.eps, nw, eps, None, None, H)
-            self._mfma(ent["ifg"], self.ifg, 3 * D, H)
+            if ent["norms"] is not None:
+                pw, n = ent["ifg"], ent["norms"]
+                L.check(lib.mmf_rmsnorm_quant_multi(
+                    self.h.data_ptr(), H, ent["attn_norm"].data_ptr(), self.eps, n[0].data_ptr(), n[1].data_ptr(), n[2].data_ptr(), eps,
+                    self.q.data_ptr(), self.deq.data_ptr(), self.qsum.data_ptr(), B, H, self.dt_id, L.dtype_id(nw.dtype), s),
+                    "mmf_rmsnorm_quant_multi")
+                L.check(lib.mmf_bitlinear_mfma_multi(
+                    self.q.data_ptr(), lib.mmf_codes_bytes(B, H, 1), self.deq.data_ptr(), self.qsum.data_ptr(), pw.packed.data_ptr(),
+                    pw.wdeq.data_ptr(), pw.seg_rows, self.ifg.data_ptr(), 3 * D, B, H, 3 * D, self.dt_id, -1, s),
+                    "mmf_bitlinear_mfma_multi")
+            else:
+                self._qfused(1, self.h.data_ptr(), H, None, 0, None, 0, None, ent["attn_norm"], self.eps, nw, eps, None, None, H)
+                self._mfma(ent["ifg"], self.ifg, 3 * D, H)
             self._qfused(3, ifg, 3 * D, ifg + D * esz, 3 * D, ifg + 2 * D * esz, 3 * D, None, ent["g_norm"], ent["g_eps"],
                          ent["o"][1], ent["o"][2], ent["lb"], ent["state"], D)
             self._mfma(ent["o"][0], self.a, H, D)
@@ -329,7 +365,7 @@ class DecodeEngine:
     def _can_fuse_mfma(self):
         same_dt = all(t.dtype == self.final_norm.dtype for e in self.layers
                       for t in (e["attn_norm"], e["mlp_norm"], e["g_norm"], e["o"][1], e["gate"][1], e["down"][1],
-                                e["projs"][0][1])) and self.head[1].dtype == self.final_norm.dtype
+                                *(p[1] for p in e["projs"]))) and self.head[1].dtype == self.final_norm.dtype
         return (not self.gemv and same_dt and all(e["ifg"] is not None for e in self.layers)
                 and max(self.H, self.D, self.I) <= 8192 and (3 * self.D) % 8 == 0 and (2 * self.I) % 8 == 0)
 
@@ -337,7 +373,7 @@ class DecodeEngine:
         kmax = self.lib.mmf_bitlinear_gemv_max_k()
         same_dt = all(t.dtype == self.final_norm.dtype for e in self.layers
                       for t in (e["attn_norm"], e["mlp_norm"], e["g_norm"], e["o"][1], e["gate"][1], e["down"][1],
-                                e["projs"][0][1])) and self.head[1].dtype == self.final_norm.dtype
+                                *(p[1] for p in e["projs"]))) and self.head[1].dtype == self.final_norm.dtype
         return (self.gemv and same_dt and all(e["ifg"] is not None for e in self.layers)
                 and max(self.H, self.D, self.I) <= kmax and self.D % 32 == 0 and self.I % 32 == 0)
 
@@ -356,7 +392,7 @@ class DecodeEngine:
         for ent in self.layers:
             L.check(lib.mmf_rmsnorm(self.h.data_ptr(), None, ent["attn_norm"].data_ptr(), self.hn.data_ptr(), None, B, H,
                                     self.eps, dt, dt, wid, s), "mmf_rmsnorm")
-            if ent["ifg"] is not None:
+            if ent["norms"] is None:
                 self._bitlinear(self.hn, (ent["ifg"], ent["projs"][0][1], ent["projs"][0][2]), self.ifg, (3 * D, H))
                 ip, fp, gp, ld = self.ifg.data_ptr(), self.ifg.data_ptr() + D * esz, self.ifg.data_ptr() + 2 * D * esz, 3 * D
             else:
