@@ -82,8 +82,14 @@ SIGNATURES = {
     "mmf_bitlinear_mfma_multi": (_i32, [_ptr, _i64, _ptr, _ptr, _ptr, _ptr, _i64, _ptr, _i64, _i64, _i64, _i64, _i32, _i32, _ptr]),
     "mmf_bitlinear_gemv_multi": (_i32, [_i32, _ptr, _i64, _ptr, _f32, _ptr, _ptr, _ptr, _f32, _ptr, _ptr, _i64, _ptr, _ptr, _ptr, _ptr,
                                         _i64, _i64, _i64, _i32, _i32, _ptr]),
+    "mmf_chain_bwd_groups": (_i32, [_i64]),
+    "mmf_chain_bwd": (_i32, [_i32, _ptr, _i64, _ptr, _i64, _ptr, _f32, _i32, _ptr, _f32, _ptr, _i64, _ptr, _ptr, _i64, _ptr, _i64,
+                             _ptr, _ptr, _ptr, _i64, _i64, _i32, _i32, _ptr]),
+    "mmf_unpack_dequant": (_i32, [_ptr, _ptr, _i64, _i64, _i64, _ptr, _i32, _ptr]),
     "mmf_block_struct_bytes": (_i64, []),
     "mmf_block_workspace_bytes": (_i64, [_ptr, _i64]),
+    "mmf_block_train_workspace_bytes": (_i64, [_ptr, _i64]),
+    "mmf_block_train_forward": (_i32, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _ptr, _ptr, _ptr, _ptr]),
     "mmf_block_forward": (_i32, [_ptr, _ptr, _ptr, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr]),
     "mmf_sample_top_p_max_vocab": (_i64, []),
     "mmf_sample_top_p": (_i32, [_ptr, _i64, _i64, _i64, _f32, _f32, _i64, _ptr, _ptr, _i32, _ptr]),

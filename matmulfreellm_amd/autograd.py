@@ -7,6 +7,7 @@ Each Function mirrors one of the reference's autograd Functions:
   SwiGLUFn                 SwiGLUFunction                mmfreelm/modules/activations.py:143-175
   FusedRecurrentHGRNFn     FusedRecurrentHGRNFunction    mmfreelm/ops/hgrn/recurrent_fuse.py:136-173
   ChunkHGRNFn              ChunkHGRNFunction             mmfreelm/ops/hgrn/chunk.py:223-284
+  BlockFn, NormHeadFn      a whole block / final norm + head of mmfreelm/models/hgrn_bit/modeling_hgrn_bit.py:97-111, 262, 386
   HGRNGateFn               the elementwise ops of mmfreelm/layers/hgrn_bit.py:113-120, differentiated as one op
   CrossEntropyFn           CrossEntropyLossFunction      mmfreelm/modules/fused_cross_entropy.py:163-310
 
@@ -15,6 +16,8 @@ The two dense products of a BitLinear's backward (dout @ W_q and dout^T @ y_q, f
 library GEMMs (torch.matmul).  Modules pick these Functions when gradients are enabled and an input or parameter
 requires one (`needs_grad`); otherwise they keep the fused inference launches.
 """
+import ctypes
+
 import torch
 
 from . import _lib as L
@@ -252,6 +255,139 @@ class ChunkHGRNFn(torch.autograd.Function):
         g, o, h0 = ctx.saved_tensors
         dx, dg = _scan_bwd(g, o, do, h0, True)
         return dx, dg, None, None, None
+
+
+CHAIN_NORM, CHAIN_GATED, CHAIN_SWIGLU = 0, 1, 2
+
+
+def _chain_bwd(kind, x, aux, w1, eps1, w2, eps2, dy, dres=None, dx=None, daux=None):
+    """mmf_chain_bwd over [M, K] operands (column slices keep their row stride; dy [norms, M, K]):
+    (dx, daux, y_quant [norms, M, K], weight gradients [(w1) + norms, K])."""
+    lib = L.load()
+    m, k = x.shape
+    n = len(w2)
+    dx = torch.empty(m, k, dtype=x.dtype, device=x.device) if dx is None else dx
+    rows = n + (kind != CHAIN_SWIGLU)
+    y = torch.empty(n, m, k, dtype=x.dtype, device=x.device)
+    part = torch.empty(lib.mmf_chain_bwd_groups(m) * rows * k, dtype=torch.float32, device=x.device)
+    dw = torch.empty(rows, k, dtype=w2[0].dtype, device=x.device)
+    w2p = (ctypes.c_void_p * 3)(*[w.data_ptr() for w in w2])
+    dyp = (ctypes.c_void_p * 3)(*[d.data_ptr() for d in dy])
+    L.check(lib.mmf_chain_bwd(kind, x.data_ptr(), x.stride(0), L.ptr(aux), aux.stride(0) if aux is not None else 0, L.ptr(w1), eps1, n, w2p,
+                              eps2, dyp, k, L.ptr(dres), dx.data_ptr(), dx.stride(0), L.ptr(daux),
+                              daux.stride(0) if daux is not None else 0, y.data_ptr(), part.data_ptr(), dw.data_ptr(), m, k,
+                              L.dtype_id(x.dtype), L.dtype_id(dw.dtype), L.stream()), "mmf_chain_bwd")
+    return dx, daux, y, dw
+
+
+def _dequantised(pw, dtype):
+    """t * wdeq of a packed weight as a dense [N, K] matrix (fusedbitnet.py:456-458)."""
+    w = torch.empty(pw.n, pw.k, dtype=dtype, device=pw.packed.device)
+    L.check(L.load().mmf_unpack_dequant(pw.packed.data_ptr(), pw.wdeq.data_ptr(), pw.seg_rows, pw.n, pw.k, w.data_ptr(), L.dtype_id(dtype),
+                                        L.stream()), "mmf_unpack_dequant")
+    return w
+
+
+class BlockFn(torch.autograd.Function):
+    """A whole HGRNBitBlock (mmfreelm/models/hgrn_bit/modeling_hgrn_bit.py:97-111) as one differentiable op.
+
+    The forward is one native call that gives the bits of the op-by-op composition.  The backward runs the same dense
+    products as that composition's (dout @ W_q and dout^T @ y_q per BitLinear) and one row kernel between them where the
+    composition had a norm behind a norm, three norms added up, or sliced tensors to put together.
+    ``params``: the nine norm weights (block.py's order), then the six BitLinear weights i, f, g, o, gate, down."""
+
+    @staticmethod
+    def forward(ctx, plan, x, lower_bound, mask, *params):
+        lib = L.load()
+        H, D, I = plan.dims
+        b, t, _ = x.shape
+        m = b * t
+        x = x.contiguous()
+        dev, dt = x.device, x.dtype
+        with L.on(dev):
+            empty = lambda *shape: torch.empty(*shape, dtype=dt, device=dev)
+            out, ifg, xg, o, res, y = torch.empty_like(x), empty(m, 3 * D), empty(2, m, D), empty(m, D), empty(m, H), empty(m, 2 * I)
+            lb = lower_bound.detach().float().contiguous() if lower_bound is not None else None
+            mk = F_._mask_rows(mask, m, dev)
+            ws = torch.empty(lib.mmf_block_train_workspace_bytes(plan.ref, m), dtype=torch.uint8, device=dev)
+            L.check(lib.mmf_block_train_forward(plan.ref, x.data_ptr(), out.data_ptr(), ifg.data_ptr(), xg.data_ptr(), o.data_ptr(),
+                                                res.data_ptr(), y.data_ptr(), b, t, L.ptr(lb), L.ptr(mk), ws.data_ptr(), L.stream()),
+                    "mmf_block_train_forward")
+        ctx.save_for_backward(x, lb, mk, ifg, xg, o, res, y, *params[:9])
+        ctx.plan, ctx.lb_dtype = plan, lower_bound.dtype if lower_bound is not None else None
+        return out
+
+    @staticmethod
+    def backward(ctx, dout):
+        x, lb, mk, ifg, xg, o, res, y, *nw = ctx.saved_tensors
+        attn_norm, mlp_norm, g_norm, i_n, f_n, gp_n, o_n, gate_n, down_n = nw
+        plan, need = ctx.plan, ctx.needs_input_grad[4:]
+        H, D, I = plan.dims
+        eps, dt, dev = plan.eps, x.dtype, x.device
+        lib = L.load()
+        b, t, _ = x.shape
+        m = b * t
+        with L.on(dev):
+            d2 = dout.to(dt).reshape(m, H).contiguous()
+            o_pw, gate_pw, down_pw = plan.pws[3:]
+            # down_proj behind the swiglu: the gradients of gate and up land side by side
+            dz = d2 @ _dequantised(down_pw, dt)
+            dy = torch.empty_like(y)
+            _, _, yq, dw_down = _chain_bwd(CHAIN_SWIGLU, y[:, :I], y[:, I:], None, 0.0, [down_n], eps["down_eps"], [dz], dx=dy[:, :I],
+                                           daux=dy[:, I:])
+            d_down = d2.t() @ yq[0] if need[14] else None
+            # gate_proj behind mlp_norm, the residual's gradient joining
+            dh = dy @ _dequantised(gate_pw, dt)
+            dres, _, yq, dw_gate = _chain_bwd(CHAIN_NORM, res, None, mlp_norm, eps["mlp_eps"], [gate_n], eps["gate_eps"], [dh], dres=d2)
+            d_gate = dy.t() @ yq[0] if need[13] else None
+            # o_proj behind the gated norm: the g columns of the stacked projection's gradient, and the scan's output
+            do2 = dres @ _dequantised(o_pw, dt)
+            difg, do = torch.empty_like(ifg), torch.empty_like(o)
+            _, _, yq, dw_o = _chain_bwd(CHAIN_GATED, ifg[:, 2 * D:], o, g_norm, eps["g_eps"], [o_n], eps["o_eps"], [do2],
+                                        dx=difg[:, 2 * D:], daux=do)
+            d_o = dres.t() @ yq[0] if need[12] else None
+            # scan and gate math
+            dxs, dgs = _scan_bwd(xg[1].view(b, 1, t, D), o.view(b, 1, t, D), do.view(b, 1, t, D), None, False)
+            dlb = torch.empty(D, dtype=torch.float32, device=dev) if lb is not None else None
+            part = torch.empty(lib.mmf_backward_groups(m), D, dtype=torch.float32, device=dev) if lb is not None else None
+            e = x.element_size()
+            L.check(lib.mmf_hgrn_gate_bwd(ifg.data_ptr(), 3 * D, ifg.data_ptr() + D * e, 3 * D, L.ptr(lb), L.ptr(mk), dxs.data_ptr(),
+                                          dgs.data_ptr(), difg.data_ptr(), 3 * D, difg.data_ptr() + D * e, 3 * D, L.ptr(part), L.ptr(dlb),
+                                          m, D, L.dtype_id(dt), L.stream()), "mmf_hgrn_gate_bwd")
+            # i, f, g behind attn_norm: three products, one pass over the rows, the residual's gradient joining
+            w3, dh3 = _dequantised(plan.stacked, dt), torch.empty(3, m, H, dtype=dt, device=dev)
+            cols = [difg[:, j * D:(j + 1) * D] for j in range(3)]
+            for j in range(3):
+                torch.mm(cols[j], w3[j * D:(j + 1) * D], out=dh3[j])
+            dx, _, yq, dw_ifg = _chain_bwd(CHAIN_NORM, x.view(m, H), None, attn_norm, eps["attn_eps"], [i_n, f_n, gp_n], eps["ifg_eps"],
+                                           dh3, dres=dres)
+            d_ifg = [cols[j].t() @ yq[j] if need[9 + j] else None for j in range(3)]
+        grads = [dw_ifg[0], dw_gate[0], dw_o[0], dw_ifg[1], dw_ifg[2], dw_ifg[3], dw_o[1], dw_gate[1], dw_down[0]]
+        if dlb is not None:
+            dlb = dlb.to(ctx.lb_dtype)
+        return (None, dx.view(x.shape), dlb, None, *grads, *d_ifg, d_o, d_gate, d_down)
+
+
+class NormHeadFn(torch.autograd.Function):
+    """The final norm and the head's BitLinear (mmfreelm/models/hgrn_bit/modeling_hgrn_bit.py:262, 386) as one op."""
+
+    @staticmethod
+    def forward(ctx, x, norm_weight, head_norm_weight, weight, pw, eps1, eps2):
+        with torch.no_grad():
+            out = F_.bitlinear(x, head_norm_weight, pw, eps=eps2, prologue=("norm", norm_weight, eps1))
+        ctx.save_for_backward(x, norm_weight, head_norm_weight)
+        ctx.pw, ctx.eps1, ctx.eps2 = pw, eps1, eps2
+        return out
+
+    @staticmethod
+    def backward(ctx, dout):
+        x, norm_weight, head_norm_weight = ctx.saved_tensors
+        with L.on(x.device):
+            x2, d2 = _2d(x).contiguous(), _2d(dout).to(x.dtype).contiguous()
+            dh = d2 @ _dequantised(ctx.pw, x.dtype)
+            dx, _, yq, dw = _chain_bwd(CHAIN_NORM, x2, None, norm_weight, ctx.eps1, [head_norm_weight], ctx.eps2, [dh])
+            d_weight = d2.t() @ yq[0] if ctx.needs_input_grad[3] else None
+        return dx.view(x.shape), dw[0], dw[1], d_weight, None, None, None
 
 
 class CrossEntropyFn(torch.autograd.Function):

@@ -26,24 +26,20 @@ class _Block(ctypes.Structure):
 
 def global_hooks():
     """Hooks registered for every module of the process: the module path runs them, the native call does not."""
-    return bool(nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks)
+    return bool(nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks or nn_module._global_backward_hooks
+                or nn_module._global_backward_pre_hooks)
 
 
 def hook_free(module):
-    d = module.__dict__
-    return not (d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d)
+    return _untouched(module.__dict__)
 
 
-class BlockPlan:
-    """The native form of one block: ``None`` from ``of`` where there is none."""
+def _untouched(d):
+    return not (d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"] or "forward" in d)
 
-    @classmethod
-    def of(cls, block):
-        plan = block.__dict__.get("_native_plan")
-        if plan is not None and plan.current():
-            return plan if plan.fits else None
-        plan = block.__dict__["_native_plan"] = cls(block)
-        return plan if plan.fits else None
+
+class _Structure:
+    """The modules of a block and the numbers they carry: what a native call takes for granted besides the parameters."""
 
     def __init__(self, block):
         from .attention import HGRNBitAttention
@@ -52,69 +48,35 @@ class BlockPlan:
         from .layernorm import RMSNorm
         from .modeling_hgrn_bit import HGRNBitBlock, HGRNBitMLP
         self.fits = False
-        self.modules = list(block.modules())
-        self.dicts = [m.__dict__ for m in self.modules]
-        # what the plan depends on: children, parameters (object, version, address), the numbers it copies
+        self.dicts = [m.__dict__ for m in block.modules()]
         self.children = [(d["_modules"], k, c) for d in self.dicts for k, c in d["_modules"].items()]
-        self.params = [(d["_parameters"], k, p, p._version, p.data_ptr()) for d in self.dicts
-                       for k, p in d["_parameters"].items() if p is not None]
         self.absent = [(d["_parameters"], k) for d in self.dicts for k, p in d["_parameters"].items() if p is None]
-        self.numbers, self.packed = [], []
+        self.numbers = []
         attn, mlp = block.attn, block.mlp
         if (type(block) is not HGRNBitBlock or type(attn) is not HGRNBitAttention or type(mlp) is not HGRNBitMLP
-                or attn.use_short_conv or any("forward" in d for d in self.dicts)):
+                or attn.use_short_conv or not all(_untouched(d) for d in self.dicts)):
             return
         projs = (attn.i_proj, attn.f_proj, attn.g_proj, attn.o_proj, mlp.gate_proj, mlp.down_proj)
-        norms = (block.attn_norm, block.mlp_norm)
+        norms = (block.attn_norm, block.mlp_norm, attn.g_norm)
         if (any(type(p) is not FusedBitLinear or p.bias is not None or type(p.norm) is not RMSNorm for p in projs)
-                or any(type(n) is not RMSNorm for n in norms) or type(attn.g_norm) is not FusedRMSNormSwishGate):
+                or any(type(n) is not RMSNorm for n in norms[:2]) or type(norms[2]) is not FusedRMSNormSwishGate
+                or any(n.weight is None for n in norms) or any(p.norm.weight is None for p in projs)):
             return
-        norm_ws = [m.weight for m in norms + (attn.g_norm,)] + [p.norm.weight for p in projs]
-        if any(w is None or not w.is_cuda or not w.is_contiguous() or w.dtype != norm_ws[0].dtype for w in norm_ws):
-            return
-        dt, wdt, dev = projs[0].weight.dtype, norm_ws[0].dtype, norm_ws[0].device
         H, D, I = attn.hidden_size, attn.input_dim, mlp.intermediate_size
-        shapes = [(D, H)] * 3 + [(H, D), (2 * I, H), (H, I)]
-        if (dt not in L._DTYPE_IDS or any(p.weight.dtype != dt or tuple(p.weight.shape) != s for p, s in zip(projs, shapes))
-                or wdt not in (dt, torch.float32) or any(w.device != dev for w in norm_ws)
-                or [w.numel() for w in norm_ws] != [H, H, D, H, H, H, D, H, I]
-                or D % 32 or I % 32 or H % 8 or max(H, D, I) > 8192 or attn.num_heads * attn.head_dim != D):
+        if (D % 32 or I % 32 or H % 8 or max(H, D, I) > 8192 or attn.num_heads * attn.head_dim != D
+                or any(p.run_eps() != projs[0].run_eps() for p in projs[:3])):
             return
-        eps = [block.attn_norm.eps, projs[0].run_eps(), attn.g_norm.eps, projs[3].run_eps(), block.mlp_norm.eps,
-               projs[4].run_eps(), projs[5].run_eps()]
-        if any(p.run_eps() != projs[0].run_eps() for p in projs[:3]):
-            return
-        same = all(torch.equal(projs[0].norm.weight, p.norm.weight) for p in projs[1:3])
-        pws = [p.packed_weight() for p in projs]
-        if any(pw.packed.device != dev for pw in pws):
-            return
-        ifg = attn._stacked_weight()
-        self.numbers = ([(m, "eps", m.eps) for m in norms + (attn.g_norm,) + tuple(p.norm for p in projs)]
+        self.numbers = ([(m, "eps", m.eps) for m in norms + tuple(p.norm for p in projs)]
                         + [(p, "fused_eps", p.fused_eps) for p in projs])
-        self.packed = [(p._pack, pw) for p, pw in zip(projs, pws)]
-        self.keep = ifg
-        self.dtype, self.device, self.H, self.D, self.I = dt, dev, H, D, I
-        self.dims, self.heads, self.head_dim, self.mode = (H, D, I), attn.num_heads, attn.head_dim, attn.mode
-        o, gate, down = pws[3:]
-        nw = [w.data_ptr() for w in norm_ws]
-        self.struct = _Block(
-            attn_norm=nw[0], i_norm=nw[3], f_norm=None if same else nw[4], g_proj_norm=None if same else nw[5],
-            ifg_packed=ifg.packed.data_ptr(), ifg_wdeq=ifg.wdeq.data_ptr(), g_norm=nw[2], o_norm=nw[6], o_packed=o.packed.data_ptr(),
-            o_wdeq=o.wdeq.data_ptr(), mlp_norm=nw[1], gate_norm=nw[7], gate_packed=gate.packed.data_ptr(),
-            gate_wdeq=gate.wdeq.data_ptr(), down_norm=nw[8], down_packed=down.packed.data_ptr(), down_wdeq=down.wdeq.data_ptr(),
-            o_seg_rows=o.seg_rows, gate_seg_rows=gate.seg_rows, down_seg_rows=down.seg_rows, H=H, D=D, I=I,
-            attn_eps=eps[0], ifg_eps=eps[1], g_eps=eps[2], o_eps=eps[3], mlp_eps=eps[4], gate_eps=eps[5], down_eps=eps[6],
-            dtype=L.dtype_id(dt), weight_dtype=L.dtype_id(wdt))
-        self.ref = ctypes.addressof(self.struct)
-        self.layer_idx = attn.layer_idx
+        self.eps = dict(zip(("attn_eps", "mlp_eps", "g_eps", "ifg_eps", "o_eps", "gate_eps", "down_eps"),
+                            [m.eps for m in norms] + [p.run_eps() for p in projs[:1] + projs[3:]]))
+        self.attn, self.projs, self.norms = attn, projs, norms
+        self.dims, self.heads, self.head_dim, self.mode, self.layer_idx = (H, D, I), attn.num_heads, attn.head_dim, attn.mode, attn.layer_idx
         self.fits = True
 
     def current(self):
         for d in self.dicts:
-            if d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d:
-                return False
-        for d, k, p, version, address in self.params:
-            if d.get(k) is not p or p._version != version or p.data_ptr() != address:
+            if not _untouched(d):
                 return False
         for d, k, c in self.children:
             if d.get(k) is not c:
@@ -125,10 +87,111 @@ class BlockPlan:
         for m, k, v in self.numbers:
             if getattr(m, k) != v:
                 return False
+        return True
+
+    def norm_weights(self):
+        """attn_norm, mlp_norm, g_norm, then the inner norms of i, f, g, o, gate, down."""
+        return [m.weight for m in self.norms] + [p.norm.weight for p in self.projs]
+
+    def fits_tensors(self):
+        """(dtype, device) of the block's parameters if the native calls take them, else None."""
+        H, D, I = self.dims
+        ws, nws = [p.weight for p in self.projs], self.norm_weights()
+        dt, wdt, dev = ws[0].dtype, nws[0].dtype, nws[0].device
+        if (dt not in L._DTYPE_IDS or wdt not in (dt, torch.float32) or dev.type != "cuda"
+                or any(w.dtype != dt or w.shape != s for w, s in zip(ws, [(D, H)] * 3 + [(H, D), (2 * I, H), (H, I)]))
+                or any(w.dtype != wdt or w.device != dev or not w.is_contiguous() or w.numel() != n
+                       for w, n in zip(nws, (H, H, D, H, H, H, D, H, I)))):
+            return None
+        return dt, dev
+
+    def struct(self, nws, pws, stacked, same, dtype):
+        """The native struct over these norm weights and packed weights."""
+        H, D, I = self.dims
+        o, gate, down = pws[3:]
+        return _Block(
+            attn_norm=nws[0].data_ptr(), mlp_norm=nws[1].data_ptr(), g_norm=nws[2].data_ptr(), i_norm=nws[3].data_ptr(),
+            f_norm=None if same else nws[4].data_ptr(), g_proj_norm=None if same else nws[5].data_ptr(), o_norm=nws[6].data_ptr(),
+            gate_norm=nws[7].data_ptr(), down_norm=nws[8].data_ptr(), ifg_packed=stacked.packed.data_ptr(),
+            ifg_wdeq=stacked.wdeq.data_ptr(), o_packed=o.packed.data_ptr(), o_wdeq=o.wdeq.data_ptr(), gate_packed=gate.packed.data_ptr(),
+            gate_wdeq=gate.wdeq.data_ptr(), down_packed=down.packed.data_ptr(), down_wdeq=down.wdeq.data_ptr(), o_seg_rows=o.seg_rows,
+            gate_seg_rows=gate.seg_rows, down_seg_rows=down.seg_rows, H=H, D=D, I=I, dtype=L.dtype_id(dtype),
+            weight_dtype=L.dtype_id(nws[0].dtype), **self.eps)
+
+
+def _structure(block):
+    s = block.__dict__.get("_native_structure")
+    if s is None or not s.current():
+        s = block.__dict__["_native_structure"] = _Structure(block)
+    return s
+
+
+class BlockPlan:
+    """The native form of one block for inference: ``None`` from ``of`` where there is none."""
+
+    @classmethod
+    def of(cls, block):
+        plan = block.__dict__.get("_native_plan")
+        if plan is None or not plan.current():
+            plan = block.__dict__["_native_plan"] = cls(block)
+        return plan if plan.fits else None
+
+    def __init__(self, block):
+        self.fits = False
+        s = self.structure = _structure(block)
+        self.params = [(d["_parameters"], k, p, p._version, p.data_ptr()) for d in s.dicts
+                       for k, p in d["_parameters"].items() if p is not None]
+        self.packed = []
+        where = s.fits_tensors() if s.fits else None
+        if where is None:
+            return
+        self.dtype, self.device = where
+        nws, pws = s.norm_weights(), [p.packed_weight() for p in s.projs]
+        if any(pw.packed.device != self.device for pw in pws):
+            return
+        self.packed = [(p._pack, pw) for p, pw in zip(s.projs, pws)]
+        self.stacked = s.attn._stacked_weight()
+        same = all(torch.equal(nws[3], w) for w in nws[4:6])
+        self.native = s.struct(nws, pws, self.stacked, same, self.dtype)
+        self.ref = ctypes.addressof(self.native)
+        self.dims, self.heads, self.head_dim, self.mode, self.layer_idx = s.dims, s.heads, s.head_dim, s.mode, s.layer_idx
+        self.H, self.D = s.dims[:2]
+        self.fits = True
+
+    def current(self):
+        if not self.structure.current():
+            return False
+        for d, k, p, version, address in self.params:
+            if d.get(k) is not p or p._version != version or p.data_ptr() != address:
+                return False
         for pack, pw in self.packed:
             if pack.pw is not pw:
                 return False
         return True
+
+
+class TrainPlan:
+    """One training forward of a block: its struct over today's parameters (an optimizer step changes them all)."""
+
+    @classmethod
+    def of(cls, block, x):
+        s = _structure(block)
+        if not s.fits or max(s.dims[:2]) > 4096 or s.mode != "fused_recurrent":
+            return None
+        where = s.fits_tensors()
+        if where is None or where != (x.dtype, x.device) or any(p.weight.is_meta for p in s.projs):
+            return None
+        return cls(s, where[0])
+
+    def __init__(self, s, dtype):
+        self.dims, self.layer_idx = s.dims, s.layer_idx
+        self.pws = [p.packed_weight() for p in s.projs]
+        self.stacked = s.attn._stacked_weight()
+        self.eps = s.eps
+        self.norm_params = s.norm_weights()
+        self.weight_params = [p.weight for p in s.projs]
+        self.native = s.struct(self.norm_params, self.pws, self.stacked, False, dtype)
+        self.ref = ctypes.addressof(self.native)
 
 
 def workspace(plan, rows):

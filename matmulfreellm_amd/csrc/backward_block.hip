@@ -1,0 +1,400 @@
+// Backward of an HGRNBit block between its dense products: the row kernels that carry a gradient through a BitLinear's norm
+// AND the elementwise op in front of it in one pass, and the ternary weights as a dense matrix.
+//
+//   mmf_chain_bwd        CHAIN_NORM    norm(x; w1) -> 1 or 3 BitLinears' norms (block norm in front of i/f/g, of gate/up, of the head)
+//                        CHAIN_GATED   norm(x; w1) * a * sigmoid(a) -> a BitLinear's norm (g_norm in front of o_proj)
+//                        CHAIN_SWIGLU  swiglu(x, a) -> a BitLinear's norm (the MLP activation in front of down_proj)
+//     i.e. mmfreelm/ops/fusedbitnet.py:209-317 followed by mmfreelm/modules/layernorm.py:245-330,
+//     mmfreelm/modules/fused_norm_gate.py:210-300 or mmfreelm/modules/activations.py:121-126.
+//   mmf_unpack_dequant   the de-quantised weight of fusedbitnet.py:456-458 for the product dout @ W_q.
+//
+// HBM is the bound: a step read and wrote every row of gradient between these ops (norm behind norm, three norms and two
+// additions behind i/f/g); here the row stays in registers from the products' output to the next products' input.  The
+// quantised activations that the weight gradient contracts with are recomputed in the forward's arithmetic, bit for bit;
+// gradients are fp32 between the stages.
+#include "mmf_common.h"
+
+namespace {
+
+enum Chain : int { CHAIN_NORM = 0, CHAIN_GATED = 1, CHAIN_SWIGLU = 2 };
+constexpr int kT = 512, kW = kT / 64;
+
+struct ChainArgs {
+    const void* x; const void* aux;     // the op's inputs, row strides ldx, ldaux
+    const void* w1;                     // NORM, GATED: weight of the norm in front
+    const void* w2[3];                  // the BitLinears' norm weights
+    const void* dy[3];                  // gradients of their normalised inputs (dout @ W_q), row stride lddy
+    const void* dres;                   // NORM: null, or a gradient that joins dx (the residual branch), row stride K
+    void* dx; void* daux;               // gradients of x and aux, row strides lddx, lddaux
+    void* y;                            // [NN][M, K]: the de-quantised codes of the BitLinears' inputs
+    float* part;                        // [gridDim.x][W1 + NN][K]: sums for w1, then for the w2
+    int64_t M, ldx, ldaux, lddy, lddx, lddaux;
+    int K;
+    float eps1, eps2;
+    double inv_K;
+};
+
+// One row per workgroup and turn, 4 elements per thread and pass, the next row's loads in flight under this row's arithmetic;
+// four exchanges of per-wave partials a row, each with slots of its own and one barrier.
+template <typename T, typename TW, int NV, int ST, int NN>
+__global__ __launch_bounds__(kT) void chain_bwd_kernel(ChainArgs a) {
+    constexpr bool W1 = ST != CHAIN_SWIGLU, AUX = ST != CHAIN_NORM, RES = ST == CHAIN_NORM;
+    __shared__ double s_sum1[kW], s_sum2[kW];
+    __shared__ float s_max[NN][kW], s_dot2[kW], s_dot1[kW];
+    const int K = a.K, lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    float acc1[W1 ? NV : 1][4], acc2[NN][NV][4];
+    Raw4<TW> w1r[W1 ? NV : 1], w2r[NN][NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+        const int k0 = (v * kT + (int)threadIdx.x) * 4;
+        if constexpr (W1) w1r[v] = raw4_load<TW, true>(static_cast<const TW*>(a.w1), k0, K);
+#pragma unroll
+        for (int n = 0; n < NN; ++n) w2r[n][v] = raw4_load<TW, true>(static_cast<const TW*>(a.w2[n]), k0, K);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if constexpr (W1) acc1[v][i] = 0.0f;
+#pragma unroll
+            for (int n = 0; n < NN; ++n) acc2[n][v][i] = 0.0f;
+        }
+    }
+    Raw4<T> xr[NV], ar[AUX ? NV : 1], rr[RES ? NV : 1], dr[NN][NV];
+    auto load = [&](int64_t row) __attribute__((always_inline)) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const int k0 = (v * kT + (int)threadIdx.x) * 4;
+            xr[v] = raw4_load<T, true>(static_cast<const T*>(a.x) + row * a.ldx, k0, K);
+            if constexpr (AUX) ar[v] = raw4_load<T, true>(static_cast<const T*>(a.aux) + row * a.ldaux, k0, K);
+#pragma unroll
+            for (int n = 0; n < NN; ++n) dr[n][v] = raw4_load<T, true>(static_cast<const T*>(a.dy[n]) + row * a.lddy, k0, K);
+            if constexpr (RES) {
+                if (a.dres) rr[v] = raw4_load<T, true>(static_cast<const T*>(a.dres) + row * (int64_t)K, k0, K);
+            }
+        }
+    };
+    auto fold = [&](float v) __attribute__((always_inline)) {
+        v += mmf_dpp<kDppXor1>(v);
+        v += mmf_dpp<kDppXor2>(v);
+        v += mmf_dpp<kDppHalfMirror>(v);
+        v += mmf_dpp<kDppMirror>(v);
+        return (mmf_readlane(v, 0) + mmf_readlane(v, 16)) + (mmf_readlane(v, 32) + mmf_readlane(v, 48));
+    };
+    auto total = [&](const float* s) __attribute__((always_inline)) {
+        float t = s[0];
+#pragma unroll
+        for (int w = 1; w < kW; ++w) t += s[w];
+        return t;
+    };
+    auto in_row = [&](int v) __attribute__((always_inline)) { return (v * kT + (int)threadIdx.x) * 4 < K; };   // K is a multiple of 4
+
+    load((int64_t)blockIdx.x < a.M ? blockIdx.x : 0);
+    for (int64_t row = blockIdx.x; row < a.M; row += gridDim.x) {
+        float x[NV][4], av[AUX ? NV : 1][4], res[RES ? NV : 1][4], dy[NN][NV][4];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            raw4_unpack<T>(xr[v], x[v]);
+            if constexpr (AUX) raw4_unpack<T>(ar[v], av[v]);
+#pragma unroll
+            for (int n = 0; n < NN; ++n) raw4_unpack<T>(dr[n][v], dy[n][v]);
+            if constexpr (RES) raw4_unpack<T>(rr[v], res[v]);
+            const bool in = in_row(v);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                x[v][i] = in ? x[v][i] : 0.0f;
+                if constexpr (AUX) av[v][i] = in ? av[v][i] : 0.0f;
+#pragma unroll
+                for (int n = 0; n < NN; ++n) dy[n][v][i] = in ? dy[n][v][i] : 0.0f;
+                if constexpr (RES) res[v][i] = a.dres ? res[v][i] : 0.0f;
+            }
+        }
+        load(row + gridDim.x < a.M ? row + gridDim.x : row);
+
+        // ---- the op in front, as the forward rounds it: s = what the BitLinear saw
+        float s[NV][4], sg[AUX ? NV : 1][4];
+        float rstd1 = 0.0f;
+        if constexpr (W1) {
+            double q = 0.0;
+#pragma unroll
+            for (int v = 0; v < NV; ++v)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) q = mmf_add_square(q, x[v][i]);
+            rstd1 = mmf_rstd(mmf_block_sum_once<kW>(q, s_sum1), K, a.inv_K, a.eps1);
+        }
+        double q2 = 0.0;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            float w1[4];
+            if constexpr (W1) raw4_unpack<TW>(w1r[v], w1);
+            if constexpr (ST == CHAIN_GATED) mmf_sigmoid_n<4>(av[v], sg[v]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if constexpr (ST == CHAIN_SWIGLU) {
+                    const float e = __fadd_rn(1.0f, mmf_exp(-x[v][i]));
+                    s[v][i] = mmf_round_to<T>(__fdiv_rn(__fmul_rn(x[v][i], av[v][i]), e));
+                    sg[v][i] = __builtin_amdgcn_rcpf(e);
+                } else {
+                    float y = __fmul_rn(__fmul_rn(x[v][i], rstd1), w1[i]);
+                    if constexpr (ST == CHAIN_GATED) y = __fmul_rn(__fmul_rn(y, av[v][i]), sg[v][i]);
+                    s[v][i] = in_row(v) ? mmf_round_to<T>(y) : 0.0f;
+                }
+                q2 = mmf_add_square(q2, s[v][i]);
+            }
+        }
+        // ---- the BitLinears' norms: codes, and the gradient through them
+        const float rstd2 = mmf_rstd(mmf_block_sum_once<kW>(q2, s_sum2), K, a.inv_K, a.eps2);
+        float amax[NN], dot2 = 0.0f, wd[NV][4];
+#pragma unroll
+        for (int n = 0; n < NN; ++n) amax[n] = 0.0f;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                s[v][i] = __fmul_rn(s[v][i], rstd2);
+                wd[v][i] = 0.0f;
+            }
+#pragma unroll
+            for (int n = 0; n < NN; ++n) {
+                float w2[4];
+                raw4_unpack<TW>(w2r[n][v], w2);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    amax[n] = fmaxf(amax[n], fabsf(__fmul_rn(s[v][i], w2[i])));
+                    wd[v][i] += w2[i] * dy[n][v][i];
+                    acc2[n][v][i] += dy[n][v][i] * s[v][i];
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) dot2 += s[v][i] * wd[v][i];
+        }
+        dot2 = fold(dot2);
+#pragma unroll
+        for (int n = 0; n < NN; ++n) {
+            amax[n] = mmf_wave_max(amax[n]);
+            if (lane == 0) s_max[n][wave] = amax[n];
+        }
+        if (lane == 0) s_dot2[wave] = dot2;
+        __syncthreads();
+        const float c2 = total(s_dot2) / (float)K;
+        float scale[NN], deq[NN];
+#pragma unroll
+        for (int n = 0; n < NN; ++n) {
+            amax[n] = s_max[n][0];
+#pragma unroll
+            for (int w = 1; w < kW; ++w) amax[n] = fmaxf(amax[n], s_max[n][w]);
+            scale[n] = mmf_127_over(fmaxf(amax[n], 1e-5f));
+            deq[n] = mmf_rcp_pos(scale[n]);
+        }
+        float dot1 = 0.0f;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const int k0 = (v * kT + (int)threadIdx.x) * 4;
+#pragma unroll
+            for (int n = 0; n < NN; ++n) {
+                float w2[4], o[4];
+                raw4_unpack<TW>(w2r[n][v], w2);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[i] = __fmul_rn((float)mmf_code(__fmul_rn(s[v][i], w2[i]), scale[n]), deq[n]);
+                raw4_store<T, true>(static_cast<T*>(a.y) + ((int64_t)n * a.M + row) * K, k0, K, o);
+            }
+            float w1[4], o[4];
+            if constexpr (W1) raw4_unpack<TW>(w1r[v], w1);
+            // ---- back through the op in front: wd = gradient of s
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float d = (wd[v][i] - s[v][i] * c2) * rstd2;
+                if constexpr (ST == CHAIN_SWIGLU) {
+                    const float g = x[v][i];
+                    o[i] = d * g * sg[v][i];
+                    x[v][i] = sg[v][i] * (1.0f + g * (1.0f - sg[v][i])) * d * av[v][i];
+                } else {
+                    const float xh = x[v][i] * rstd1;
+                    if constexpr (ST == CHAIN_GATED) {
+                        o[i] = d * xh * w1[i] * sg[v][i] * (1.0f + av[v][i] * (1.0f - sg[v][i]));
+                        d *= av[v][i] * sg[v][i];
+                    }
+                    acc1[v][i] += d * xh;
+                    wd[v][i] = d * w1[i];
+                    x[v][i] = xh;
+                    dot1 += xh * wd[v][i];
+                }
+            }
+            if constexpr (AUX) raw4_store<T, true>(static_cast<T*>(a.daux) + row * a.lddaux, k0, K, o);
+            if constexpr (ST == CHAIN_SWIGLU) raw4_store<T, true>(static_cast<T*>(a.dx) + row * a.lddx, k0, K, x[v]);
+        }
+        if constexpr (W1) {
+            dot1 = fold(dot1);
+            if (lane == 0) s_dot1[wave] = dot1;
+            __syncthreads();
+            const float c1 = total(s_dot1) / (float)K;
+#pragma unroll
+            for (int v = 0; v < NV; ++v) {
+                float o[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[i] = (wd[v][i] - x[v][i] * c1) * rstd1 + (RES ? res[v][i] : 0.0f);
+                raw4_store<T, true>(static_cast<T*>(a.dx) + row * a.lddx, (v * kT + (int)threadIdx.x) * 4, K, o);
+            }
+        } else {
+            __syncthreads();                                     // the slots are free for the next row
+        }
+    }
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+        const int k0 = (v * kT + (int)threadIdx.x) * 4;
+        float* p = a.part + (int64_t)blockIdx.x * ((W1 ? 1 : 0) + NN) * K;
+        if constexpr (W1) raw4_store<float, true>(p, k0, K, acc1[v]);
+#pragma unroll
+        for (int n = 0; n < NN; ++n) raw4_store<float, true>(p + (int64_t)((W1 ? 1 : 0) + n) * K, k0, K, acc2[n][v]);
+    }
+}
+
+// out[k] = T(sum_g part[g, k]).  A workgroup owns 32 columns; its 32 lanes per column each add every 32nd group in index order and
+// the 32 lane sums are then added in lane order, so the result depends on the shape only.
+constexpr int kCols = 32, kLanes = 32;
+template <typename T>
+__global__ __launch_bounds__(kCols * kLanes) void colsum_rows_kernel(const float* __restrict__ part, int groups, int K, T* __restrict__ out) {
+    __shared__ float lane_sum[kLanes][kCols + 1];
+    const int c = (int)threadIdx.x % kCols, l = (int)threadIdx.x / kCols;
+    const int k = (int)blockIdx.x * kCols + c;
+    float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
+    if (k < K) {
+        int g = l;
+        for (; g + 3 * kLanes < groups; g += 4 * kLanes) {
+            s0 += part[(int64_t)g * K + k];
+            s1 += part[(int64_t)(g + kLanes) * K + k];
+            s2 += part[(int64_t)(g + 2 * kLanes) * K + k];
+            s3 += part[(int64_t)(g + 3 * kLanes) * K + k];
+        }
+        for (; g < groups; g += kLanes) s0 += part[(int64_t)g * K + k];
+    }
+    lane_sum[l][c] = (s0 + s1) + (s2 + s3);
+    __syncthreads();
+    if (l == 0 && k < K) {
+        float s = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kLanes; ++i) s += lane_sum[i][c];
+        out[k] = mmf_from_float<T>(s);
+    }
+}
+
+template <typename T, typename TW, int ST, int NN>
+int launch_chain(const ChainArgs& a, int groups, void* dw, hipStream_t s) {
+    const int nv = (int)mmf_ceil_div(a.K, kT * 4);
+    if (nv <= 1) chain_bwd_kernel<T, TW, 1, ST, NN><<<groups, kT, 0, s>>>(a);
+    else if (nv <= 2) chain_bwd_kernel<T, TW, 2, ST, NN><<<groups, kT, 0, s>>>(a);
+    else if constexpr (NN == 1) {                                // (three norms: a wider row would not fit the registers)
+        if (nv <= 3) chain_bwd_kernel<T, TW, 3, ST, NN><<<groups, kT, 0, s>>>(a);
+        else if (nv <= 4) chain_bwd_kernel<T, TW, 4, ST, NN><<<groups, kT, 0, s>>>(a);
+        else return MMF_ERR_WIDE;
+    } else return MMF_ERR_WIDE;
+    MMF_CHECK_LAUNCH();
+    const int cols = ((ST != CHAIN_SWIGLU ? 1 : 0) + NN) * a.K;
+    colsum_rows_kernel<TW><<<(unsigned)mmf_ceil_div(cols, kCols), kCols * kLanes, 0, s>>>(a.part, groups, cols, static_cast<TW*>(dw));
+    MMF_CHECK_LAUNCH();
+    return 0;
+}
+template <typename T, typename TW>
+int dispatch_chain(const ChainArgs& a, int kind, int n, int groups, void* dw, hipStream_t s) {
+    switch (kind) {
+        case CHAIN_NORM: return n == 3 ? launch_chain<T, TW, CHAIN_NORM, 3>(a, groups, dw, s) : launch_chain<T, TW, CHAIN_NORM, 1>(a, groups, dw, s);
+        case CHAIN_GATED: return launch_chain<T, TW, CHAIN_GATED, 1>(a, groups, dw, s);
+        case CHAIN_SWIGLU: return launch_chain<T, TW, CHAIN_SWIGLU, 1>(a, groups, dw, s);
+    }
+    return MMF_ERR_ARG;
+}
+
+// ------------------------------------------------------------------------------------------ weights
+// One thread per 16 inputs of a row: its dword of codes becomes 32 (64) bytes of the row, so consecutive threads write a row of
+// the block's 128 inputs side by side.  Bound by the write, 2 (4) bytes a weight.
+template <typename T>
+__global__ __launch_bounds__(256) void unpack_dequant_kernel(const uint32_t* __restrict__ packed, const float* __restrict__ wdeq,
+                                                             int64_t seg_rows, int64_t N, int64_t K, int64_t KB, T* __restrict__ out) {
+    const int64_t groups = mmf_ceil_div(K, 16);
+    const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (gid >= N * groups) return;
+    const int64_t n = gid / groups, kg = gid % groups;
+    const int64_t k0 = kg * 16, nb = n >> 5, kb = k0 >> 7;
+    const int s = (int)((k0 >> 5) & 3), half = (int)((k0 >> 4) & 1), lane = half * 32 + (int)(n & 31);
+    const uint32_t v = packed[((nb * KB + kb) * 64 + lane) * 4 + s];
+    const float wd = wdeq[n / seg_rows];
+    T* row = out + n * K + k0;
+    const bool whole = K % 8 == 0 && k0 + 16 <= K;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        float e[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int i = h * 8 + j;
+            e[j] = (float)((int)((v >> (8 * (i & 3) + 2 * (i >> 2))) & 3u) - 1) * wd;
+        }
+        mmf_store8<T>(row, h * 8, K - k0, whole, e);
+    }
+}
+
+}  // namespace
+
+extern "C" {
+
+int mmf_chain_bwd_groups(int64_t rows) { return (int)(rows < 1 ? 1 : rows < 1024 ? rows : 1024); }
+
+int mmf_chain_bwd(int kind, const void* x, int64_t ldx, const void* aux, int64_t ldaux, const void* w1, float eps1, int norms,
+                  const void* const* w2, float eps2, const void* const* dy, int64_t lddy, const void* dres, void* dx, int64_t lddx,
+                  void* daux, int64_t lddaux, void* y, float* part, void* dweights, int64_t M, int64_t K, int x_dtype, int weight_dtype,
+                  void* stream_) {
+    hipStream_t stream = static_cast<hipStream_t>(stream_);
+    if (kind < CHAIN_NORM || kind > CHAIN_SWIGLU || M < 0 || K <= 0 || ldx < K || lddy < K || lddx < K) return MMF_ERR_ARG;
+    if (M == 0) return 0;
+    if (!(norms == 1 || (norms == 3 && kind == CHAIN_NORM)) || !x || !w2 || !dy || !dx || !y || !part || !dweights) return MMF_ERR_ARG;
+    if (kind != CHAIN_SWIGLU && !w1) return MMF_ERR_ARG;
+    if (kind != CHAIN_NORM && (!aux || !daux || ldaux < K || lddaux < K || dres)) return MMF_ERR_ARG;
+    if (K % 4 != 0 || K > kT * 4 * 4) return MMF_ERR_WIDE;
+    ChainArgs a{};
+    a.x = x; a.aux = aux; a.w1 = w1; a.dres = dres; a.dx = dx; a.daux = daux; a.y = y; a.part = part;
+    for (int n = 0; n < norms; ++n) {
+        if (!w2[n] || !dy[n]) return MMF_ERR_ARG;
+        a.w2[n] = w2[n];
+        a.dy[n] = dy[n];
+    }
+    a.M = M; a.ldx = ldx; a.ldaux = ldaux; a.lddy = lddy; a.lddx = lddx; a.lddaux = lddaux; a.K = (int)K;
+    a.eps1 = eps1; a.eps2 = eps2; a.inv_K = 1.0 / (double)K;
+    const uintptr_t xm = 4 * (x_dtype == MMF_F32 ? 4 : 2) - 1, wm = 4 * (weight_dtype == MMF_F32 ? 4 : 2) - 1;
+    auto off = [](const void* p, uintptr_t m) { return (reinterpret_cast<uintptr_t>(p) & m) != 0; };
+    for (int64_t ld : {ldx, kind != CHAIN_NORM ? ldaux : 0, lddy, lddx, kind != CHAIN_NORM ? lddaux : 0})
+        if (ld % 4 != 0) return MMF_ERR_ALIGN;
+    for (const void* p : {x, aux, dres, (const void*)dx, (const void*)daux, (const void*)y, a.dy[0], a.dy[1], a.dy[2]})
+        if (off(p, xm)) return MMF_ERR_ALIGN;
+    for (const void* p : {w1, a.w2[0], a.w2[1], a.w2[2]})
+        if (off(p, wm)) return MMF_ERR_ALIGN;
+    if (off(part, 15)) return MMF_ERR_ALIGN;
+    const bool wf32 = weight_dtype == MMF_F32;
+    if (!wf32 && weight_dtype != x_dtype) return MMF_ERR_ARG;
+    const int groups = mmf_chain_bwd_groups(M);
+    switch (x_dtype) {
+        case MMF_F32: return dispatch_chain<float, float>(a, kind, norms, groups, dweights, stream);
+        case MMF_BF16: return wf32 ? dispatch_chain<bf16_t, float>(a, kind, norms, groups, dweights, stream)
+                                   : dispatch_chain<bf16_t, bf16_t>(a, kind, norms, groups, dweights, stream);
+        case MMF_F16: return wf32 ? dispatch_chain<f16_t, float>(a, kind, norms, groups, dweights, stream)
+                                  : dispatch_chain<f16_t, f16_t>(a, kind, norms, groups, dweights, stream);
+    }
+    return MMF_ERR_ARG;
+}
+
+int mmf_unpack_dequant(const void* packed, const float* wdeq, int64_t seg_rows, int64_t N, int64_t K, void* out, int dtype,
+                       void* stream_) {
+    hipStream_t stream = static_cast<hipStream_t>(stream_);
+    if (N <= 0 || K <= 0 || seg_rows <= 0 || !packed || !wdeq || !out) return MMF_ERR_ARG;
+    if (K % 8 == 0 && (reinterpret_cast<uintptr_t>(out) & 15u)) return MMF_ERR_ALIGN;
+    const int64_t KB = mmf_ceil_div(K, 128), blocks = mmf_ceil_div(N * mmf_ceil_div(K, 16), 256);
+    if (blocks > 0x7fffffff) return MMF_ERR_WIDE;
+#define MMF_UD(T) unpack_dequant_kernel<T><<<(unsigned)blocks, 256, 0, stream>>>(static_cast<const uint32_t*>(packed), wdeq, seg_rows, N, K, \
+                                                                                KB, static_cast<T*>(out))
+    switch (dtype) {
+        case MMF_F32: MMF_UD(float); break;
+        case MMF_BF16: MMF_UD(bf16_t); break;
+        case MMF_F16: MMF_UD(f16_t); break;
+        default: return MMF_ERR_ARG;
+    }
+#undef MMF_UD
+    MMF_CHECK_LAUNCH();
+    return 0;
+}
+
+}  // extern "C"

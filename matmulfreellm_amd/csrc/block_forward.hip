@@ -21,22 +21,40 @@ bool few_rows(const mmf_block* p, int64_t M) {
     return M <= kGemvRows && (k > p->D ? k : p->D) <= mmf_bitlinear_gemv_max_k();
 }
 
+// What the i/f/g projections contract: codes of x under the block norm and their inner norm(s), q [1 or 3], deq, qsum.
+int project_ifg(const mmf_block* p, const void* x, int64_t M, int8_t* q, float* deq, int* qsum, void* ifg, void* stream) {
+    const int64_t H = p->H, D = p->D;
+    const int dt = p->dtype, wt = p->weight_dtype;
+    if (p->f_norm) {
+        if (const int rc = mmf_rmsnorm_quant_multi(x, H, p->attn_norm, p->attn_eps, p->i_norm, p->f_norm, p->g_proj_norm, p->ifg_eps, q, deq,
+                                                   qsum, M, H, dt, wt, stream))
+            return rc;
+        return mmf_bitlinear_mfma_multi(q, mmf_codes_bytes(M, H, 1), deq, qsum, p->ifg_packed, p->ifg_wdeq, D, ifg, 3 * D, M, H, 3 * D, dt,
+                                        -1, stream);
+    }
+    if (const int rc = mmf_rmsnorm_quant_fused(Q_NORM, x, H, nullptr, 0, nullptr, 0, nullptr, p->attn_norm, p->attn_eps, p->i_norm, p->ifg_eps,
+                                               nullptr, nullptr, q, deq, qsum, M, H, dt, wt, stream))
+        return rc;
+    return mmf_bitlinear_mfma(q, deq, qsum, p->ifg_packed, p->ifg_wdeq, D, nullptr, nullptr, ifg, 3 * D, M, H, 3 * D, dt, -1, stream);
+}
+
 // Offsets of the intermediates in the workspace (each 256-byte aligned).
 struct Layout {
-    int64_t ifg, o, attn, res, big, q, deq, qsum, bytes;
-    Layout(const mmf_block* p, int64_t M) {
+    int64_t ifg = 0, o = 0, attn, res = 0, big = 0, q, deq, qsum, bytes = 0;
+    Layout(const mmf_block* p, int64_t M, bool train) {
         const int64_t e = esize(p);
-        bytes = 0;
         auto take = [&](int64_t n) {
             const int64_t at = bytes;
             bytes += mmf_round_up(n, 256);
             return at;
         };
-        ifg = take(M * 3 * p->D * e);
-        o = take(M * p->D * e);
         attn = take(M * p->H * e);
-        res = take(M * p->H * e);
-        big = take(M * 2 * (p->I > p->D ? p->I : p->D) * e);    // the scan's x and g, later gate/up
+        if (!train) {                                            // training keeps these in tensors of the caller's
+            ifg = take(M * 3 * p->D * e);
+            o = take(M * p->D * e);
+            res = take(M * p->H * e);
+            big = take(M * 2 * (p->I > p->D ? p->I : p->D) * e);    // the scan's x and g, later gate/up
+        }
         int64_t codes = 3 * mmf_codes_bytes(M, p->H, 1);
         for (int64_t k : {(int64_t)p->D, (int64_t)p->I})
             if (mmf_codes_bytes(M, k, 1) > codes) codes = mmf_codes_bytes(M, k, 1);
@@ -54,7 +72,50 @@ int64_t mmf_block_struct_bytes(void) { return (int64_t)sizeof(mmf_block); }
 
 int64_t mmf_block_workspace_bytes(const mmf_block* p, int64_t rows) {
     if (!p || rows <= 0) return 0;
-    return Layout(p, rows).bytes;
+    return Layout(p, rows, false).bytes;
+}
+
+int64_t mmf_block_train_workspace_bytes(const mmf_block* p, int64_t rows) {
+    if (!p || rows <= 0) return 0;
+    return Layout(p, rows, true).bytes;
+}
+
+int mmf_block_train_forward(const mmf_block* p, const void* x, void* out, void* ifg, void* xg, void* o, void* res, void* y, int64_t B,
+                            int64_t T, const float* lower_bound, const uint8_t* mask, void* workspace, void* stream) {
+    if (!p || B < 0 || T < 0 || p->H <= 0 || p->D <= 0 || p->I <= 0 || p->D % 32 || p->I % 32) return MMF_ERR_ARG;
+    const int64_t M = B * T, H = p->H, D = p->D, I = p->I, e = esize(p);
+    if (M == 0) return 0;
+    if (!x || !out || !ifg || !xg || !o || !res || !y || !workspace) return MMF_ERR_ARG;
+    if (reinterpret_cast<uintptr_t>(workspace) & 255u) return MMF_ERR_ALIGN;
+    const Layout L(p, M, true);
+    char* w = static_cast<char*>(workspace);
+    void* attn = w + L.attn;
+    int8_t* q = reinterpret_cast<int8_t*>(w + L.q);
+    float* deq = reinterpret_cast<float*>(w + L.deq);
+    int* qsum = reinterpret_cast<int*>(w + L.qsum);
+    char *i = static_cast<char*>(ifg), *f = i + D * e, *g = i + 2 * D * e, *gs = static_cast<char*>(xg) + M * D * e;
+    char* up = static_cast<char*>(y) + I * e;
+    const int dt = p->dtype, wt = p->weight_dtype;
+    int rc = 0;
+#define MMF_DO(call)                \
+    do {                            \
+        if ((rc = (call))) return rc; \
+    } while (0)
+    MMF_DO(project_ifg(p, x, M, q, deq, qsum, ifg, stream));
+    MMF_DO(mmf_hgrn_gate(i, 3 * D, f, 3 * D, lower_bound, mask, xg, gs, M, D, dt, stream));
+    MMF_DO(mmf_hgrn_recurrent(xg, gs, nullptr, o, nullptr, B, T, D, dt, stream));
+    MMF_DO(mmf_rmsnorm_quant_fused(Q_GATEDNORM, g, 3 * D, o, D, nullptr, 0, nullptr, p->g_norm, p->g_eps, p->o_norm, p->o_eps, nullptr,
+                                   nullptr, q, deq, qsum, M, D, dt, wt, stream));
+    MMF_DO(mmf_bitlinear_mfma(q, deq, qsum, p->o_packed, p->o_wdeq, p->o_seg_rows, nullptr, nullptr, attn, H, M, D, H, dt, -1, stream));
+    MMF_DO(mmf_rmsnorm_quant_fused(Q_RESNORM, attn, H, x, H, nullptr, 0, res, p->mlp_norm, p->mlp_eps, p->gate_norm, p->gate_eps, nullptr,
+                                   nullptr, q, deq, qsum, M, H, dt, wt, stream));
+    MMF_DO(mmf_bitlinear_mfma(q, deq, qsum, p->gate_packed, p->gate_wdeq, p->gate_seg_rows, nullptr, nullptr, y, 2 * I, M, H, 2 * I, dt, -1,
+                              stream));
+    MMF_DO(mmf_rmsnorm_quant_fused(Q_SWIGLU, y, 2 * I, up, 2 * I, nullptr, 0, nullptr, nullptr, 0.0f, p->down_norm, p->down_eps, nullptr,
+                                   nullptr, q, deq, qsum, M, I, dt, wt, stream));
+    MMF_DO(mmf_bitlinear_mfma(q, deq, qsum, p->down_packed, p->down_wdeq, p->down_seg_rows, nullptr, res, out, H, M, I, H, dt, -1, stream));
+#undef MMF_DO
+    return 0;
 }
 
 int mmf_block_forward(const mmf_block* p, const void* x, void* out, int64_t B, int64_t T, const float* lower_bound,
@@ -64,7 +125,7 @@ int mmf_block_forward(const mmf_block* p, const void* x, void* out, int64_t B, i
     if (M == 0) return 0;
     if (!x || !out || x == out || !workspace) return MMF_ERR_ARG;
     if (reinterpret_cast<uintptr_t>(workspace) & 255u) return MMF_ERR_ALIGN;
-    const Layout L(p, M);
+    const Layout L(p, M, false);
     char* w = static_cast<char*>(workspace);
     char* ifg = w + L.ifg;
     char *i = ifg, *f = ifg + D * e, *g = ifg + 2 * D * e;     // columns of the stacked projection, row stride 3 D
@@ -111,17 +172,7 @@ int mmf_block_forward(const mmf_block* p, const void* x, void* out, int64_t B, i
                                         M, I, H, dt, wt, stream));
         return 0;
     }
-    if (multi) {
-        MMF_DO(mmf_rmsnorm_quant_multi(x, H, p->attn_norm, p->attn_eps, p->i_norm, p->f_norm, p->g_proj_norm, p->ifg_eps, q, deq, qsum,
-                                       M, H, dt, wt, stream));
-        MMF_DO(mmf_bitlinear_mfma_multi(q, mmf_codes_bytes(M, H, 1), deq, qsum, p->ifg_packed, p->ifg_wdeq, D, ifg, 3 * D, M, H, 3 * D,
-                                        dt, -1, stream));
-    } else {
-        MMF_DO(mmf_rmsnorm_quant_fused(Q_NORM, x, H, nullptr, 0, nullptr, 0, nullptr, p->attn_norm, p->attn_eps, p->i_norm, p->ifg_eps,
-                                       nullptr, nullptr, q, deq, qsum, M, H, dt, wt, stream));
-        MMF_DO(mmf_bitlinear_mfma(q, deq, qsum, p->ifg_packed, p->ifg_wdeq, D, nullptr, nullptr, ifg, 3 * D, M, H, 3 * D, dt, -1,
-                                  stream));
-    }
+    MMF_DO(project_ifg(p, x, M, q, deq, qsum, ifg, stream));
     if (step && !mask) {
         MMF_DO(mmf_rmsnorm_quant_fused(Q_STEP_GATE, i, 3 * D, f, 3 * D, g, 3 * D, nullptr, p->g_norm, p->g_eps, p->o_norm, p->o_eps,
                                        lower_bound, ht, q, deq, qsum, M, D, dt, wt, stream));

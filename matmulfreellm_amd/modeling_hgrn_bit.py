@@ -30,7 +30,7 @@ from . import block as native
 from . import functional as F_
 from .activations import swiglu
 from .attention import HGRNBitAttention
-from .autograd import module_needs_grad
+from .autograd import BlockFn, NormHeadFn, module_needs_grad
 from .bitlinear import FusedBitLinear as BitLinear
 from .cache import RecurrentCache
 from .configuration_hgrn_bit import HGRNBitConfig
@@ -239,13 +239,21 @@ class HGRNBitModel(HGRNBitPreTrainedModel):
             lower_bounds = None
         elif train:                                              # differentiable (modeling_hgrn_bit.py:231-233)
             lower_bounds = self.lower_bounds.float().softmax(0)
-            lower_bounds = lower_bounds.cumsum(0) - lower_bounds[0]
+            lower_bounds = (lower_bounds.cumsum(0) - lower_bounds[0]).unbind(0)
         else:
             lower_bounds = self.lower_bound_rows()
+        # training: a block whose modules nobody hooks into is one autograd op
+        blocks = (hidden_states.dim() == 3 and hidden_states.is_cuda and hidden_states.numel() > 0 and not native.global_hooks()
+                  and not torch.is_autocast_enabled())
         for i, layer in enumerate(self.layers):
             if output_hidden_states:
                 all_hidden_states += (hidden_states,)
             lower_bound = lower_bounds[i] if lower_bounds is not None else None
+            plan = native.TrainPlan.of(layer, hidden_states) if train and blocks else None
+            if plan is not None and plan.dims[0] == hidden_states.shape[-1] and past_key_values is None:
+                lb = lower_bound if plan.layer_idx > 0 else None
+                hidden_states = BlockFn.apply(plan, hidden_states, lb, attention_mask, *plan.norm_params, *plan.weight_params)
+                continue
             hidden_states, _, past_key_values = layer(
                 hidden_states, attention_mask=attention_mask, past_key_values=past_key_values, use_cache=use_cache,
                 output_attentions=False, lower_bound=lower_bound)
@@ -402,16 +410,22 @@ class HGRNBitForCausalLM(HGRNBitPreTrainedModel, GenerationMixin):
         if labels is not None:
             logits_to_keep = 0                           # the loss scores every position
         return_dict = return_dict if return_dict is not None else bool(getattr(self.config, "return_dict", True))
-        fold = not train and self._folds_final_norm(output_hidden_states)
+        fold = self._folds_final_norm(output_hidden_states, train)
         args = dict(input_ids=input_ids, attention_mask=attention_mask, inputs_embeds=inputs_embeds, past_key_values=past_key_values,
                     use_cache=use_cache, output_attentions=output_attentions, output_hidden_states=output_hidden_states, return_dict=True)
-        outputs = self.model._forward(False, **args, final_norm=False) if fold else self.model(**args)
+        outputs = self.model._forward(train, **args, final_norm=False) if fold else self.model(**args)
         hidden_states = outputs.last_hidden_state
         if logits_to_keep:
             hidden_states = hidden_states[:, -logits_to_keep:, :]
         if fold:
-            norm = self.model.norm
-            logits = self.lm_head.forward_fused(hidden_states, ("norm", norm.weight, norm.eps))
+            norm, head = self.model.norm, self.lm_head
+            if train and hidden_states.dtype != head.weight.dtype:
+                logits = head(norm(hidden_states))
+            elif train:
+                logits = NormHeadFn.apply(hidden_states, norm.weight, head.norm.weight, head.weight, head.packed_weight(), norm.eps,
+                                          head.run_eps())
+            else:
+                logits = head.forward_fused(hidden_states, ("norm", norm.weight, norm.eps))
         else:
             logits = self.lm_head(hidden_states)
         loss = None
@@ -430,7 +444,7 @@ class HGRNBitForCausalLM(HGRNBitPreTrainedModel, GenerationMixin):
         return CausalLMOutputWithPast(loss=loss, logits=logits, past_key_values=outputs.past_key_values,
                                       hidden_states=outputs.hidden_states, attentions=None)
 
-    def _folds_final_norm(self, output_hidden_states):
+    def _folds_final_norm(self, output_hidden_states, train):
         """Whether the last norm runs inside the head's quantiser, on the kept positions only: nobody else sees its output
         (no hidden states asked for, no hook or replaced module in between) and the two norm weights share a dtype."""
         norm, head = self.model.norm, self.lm_head
@@ -438,7 +452,11 @@ class HGRNBitForCausalLM(HGRNBitPreTrainedModel, GenerationMixin):
                 and type(self.model) is HGRNBitModel and type(norm) is RMSNorm and type(head) is BitLinear and type(head.norm) is RMSNorm
                 and not native.global_hooks() and all(native.hook_free(m) for m in (self.model, norm, head, head.norm))
                 and norm.weight is not None and head.norm.weight is not None and norm.weight.dtype == head.norm.weight.dtype
-                and head.in_features <= 8192)
+                and head.in_features <= 8192 and (not train or (
+                    head.bias is None and not head.weight.is_meta and head.in_features % 8 == 0
+                    and head.weight.dtype == self.model.embeddings.weight.dtype and norm.weight.dtype in (head.weight.dtype, torch.float32)
+                    and all(p.is_cuda and p.is_contiguous() for p in (norm.weight, head.norm.weight, head.weight))
+                    and not torch.is_autocast_enabled())))
 
     # ------------------------------------------------------------------ generation
     @torch.no_grad()
