@@ -692,60 +692,63 @@ int launch_mfma_dma3(MfmaArgs a, hipStream_t s) {
 // ------------------------------------------------------------------------------------------
 // Small problems (decode batches, short prompts): the contraction is a weight stream, not a
 // GEMM, and the enemy is latency, so nothing is staged and nothing waits on a barrier until the
-// very end.  One workgroup of 8 waves owns MB 32x32 output blocks of one 32-row n-block (grid.y
-// walks M); wave w takes the k-blocks w, w+8, ...
+// very end.  One workgroup of NWV waves owns a 32x32 output block (grid.y walks M); wave w takes the k-blocks
+// w, w + NWV, ...: at most ITER of them, with the loads of PF in flight.
 // A fragments (1 KiB each, L2 resident: the whole A is M x K bytes) and the packed B block
-// are loaded straight into registers, three k-blocks in flight per wave; the 8 partial
-// accumulators meet in LDS and all 512 threads run the epilogue.
-template <typename T, int MB>
-__global__ __launch_bounds__(512) void bitlinear_mfma_skinny_kernel(MfmaArgs p) {
-    constexpr int NWV = 8, PF = 3, MAXK = 8;            // Kp <= 8 * 8 * 128
-    __shared__ int red[NWV][MB][16][64];
+// are loaded straight into registers; the partial accumulators meet in LDS and all threads run the epilogue.
+// NWV = 16 where that still leaves a CU per workgroup: half the k-blocks in a wave's chain.  NWV = 8 otherwise, in few enough
+// registers for three workgroups a CU when the row is short (a gate/up projection of 704 blocks took two rounds at two a
+// CU).  Measured at 64 rows, 1.3B shape: gate/up 7.9 -> 6.6 us, down_proj 7.2 -> 6.1 us against 8 waves and three k-blocks in
+// flight for every shape.
+// SWI: the weight is stacked [gate; up] (N = 2 I) and a workgroup contracts the gate and the up rows of the same 32 channels with
+// shared A fragments, half of their traffic; the epilogue writes swiglu(gate, up), so the exp and divide of the MLP activation
+// run spread over all workgroups instead of in the next quantiser's one workgroup per row: 6.6 + 5.9 -> 6.4 + 4.2 us for the two.
+// (Two plain n-blocks per workgroup measured no faster than one.)
+template <typename T, int NWV, int ITER, bool SWI>
+__global__ __launch_bounds__(64 * NWV, NWV == 8 && ITER <= 2 && !SWI ? 6 : 4) void bitlinear_mfma_skinny_kernel(MfmaArgs p) {
+    constexpr int NB = SWI ? 2 : 1, PF = ITER < 3 ? ITER : 3, NT = 64 * NWV, EL = 1024 / NT;   // outputs per thread
+    __shared__ int red[NWV][NB][16][64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform: keep it in a scalar register
-    const int64_t nb = blockIdx.x, mbase = (int64_t)blockIdx.y * MB;   // this workgroup's first m-block
+    const int64_t nb = blockIdx.x, nb1 = nb + (p.N >> 6), mb = blockIdx.y;           // SWI: nb1 holds the up rows
     mfma_select_segment(p, nb);
-    const int64_t KB = p.Kp >> 7, KG = p.Kp >> 4;
-    const int64_t MBtot = (p.M + 31) >> 5;
+    const int KB = (int)(p.Kp >> 7);
+    const int8_t* abase = p.a + mb * (p.Kp >> 4) * 512;
+    const uint4* const bbase[2] = {p.b + nb * KB * 64, p.b + nb1 * KB * 64};
 
-    v16i acc[MB];
+    v16i acc[NB];
 #pragma unroll
-    for (int i = 0; i < MB; ++i)
+    for (int i = 0; i < NB; ++i)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[i][r] = 0;
-
-    uint4 breg[PF];
-    v4i areg[PF][MB][4];
-    auto load_stage = [&](int st, int64_t kb) {
+    uint4 breg[PF][NB];
+    v4i areg[PF][4];
+    auto load_stage = [&](int st, int kb) __attribute__((always_inline)) {
         if (kb < KB) {
-            breg[st] = p.b[(nb * KB + kb) * 64 + lane];
 #pragma unroll
-            for (int i = 0; i < MB; ++i)
+            for (int i = 0; i < NB; ++i) breg[st][i] = bbase[i][kb * 64 + lane];
 #pragma unroll
-                for (int ks = 0; ks < 4; ++ks) {
-                    areg[st][i][ks] = (v4i){0, 0, 0, 0};
-                    if (mbase + i < MBtot)
-                        areg[st][i][ks] = *reinterpret_cast<const v4i*>(p.a + ((mbase + i) * KG + kb * 8 + ks * 2) * 512 + lane * 16);
-                }
+            for (int ks = 0; ks < 4; ++ks) areg[st][ks] = *reinterpret_cast<const v4i*>(abase + (kb * 8 + ks * 2) * 512 + lane * 16);
         }
     };
 #pragma unroll
-    for (int st = 0; st < PF; ++st) load_stage(st, wave + (int64_t)st * NWV);
+    for (int st = 0; st < PF; ++st) load_stage(st, wave + st * NWV);
 
     // the epilogue's operands, requested now so that the end of the kernel waits for nothing
     const T* bias = static_cast<const T*>(p.bias);
     const T* addend = static_cast<const T*>(p.addend);
     T* out = static_cast<T*>(p.out);
     const int64_t n_ep = nb * 32 + (lane & 31);
-    const bool n_ok = n_ep < p.N;
-    const float ep_wdeq = p.wdeq[(uint32_t)(nb * 32) / (uint32_t)p.seg_rows];   // an n-block never straddles a segment
-    const float ep_bias = (bias && n_ok) ? mmf_to_float(bias[n_ep]) : 0.0f;
-    int ep_qsum[MB * 2];
-    float ep_deq[MB * 2], ep_add[MB * 2];
+    const bool n_ok = SWI || n_ep < p.N;
+    float ep_wdeq[NB];                                   // an n-block never straddles a segment
 #pragma unroll
-    for (int j = 0; j < MB * 2; ++j) {
-        const int e = threadIdx.x + j * 512;             // (mb, r, lane) flattened
-        const int r = (e >> 6) & 15, mb = e >> 10;
-        const int64_t m = (mbase + mb) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+    for (int i = 0; i < NB; ++i) ep_wdeq[i] = p.wdeq[(uint32_t)((i ? nb1 : nb) * 32) / (uint32_t)p.seg_rows];
+    const float ep_bias = (bias && n_ok) ? mmf_to_float(bias[n_ep]) : 0.0f;
+    int ep_qsum[EL];
+    float ep_deq[EL], ep_add[EL];
+#pragma unroll
+    for (int j = 0; j < EL; ++j) {
+        const int r = wave + j * NWV;                    // accumulator register of this thread's j-th output
+        const int64_t m = mb * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
         const int64_t mc = m < p.M ? m : 0;
         ep_qsum[j] = p.qsum[mc];
         ep_deq[j] = p.deq[mc];
@@ -753,51 +756,78 @@ __global__ __launch_bounds__(512) void bitlinear_mfma_skinny_kernel(MfmaArgs p) 
     }
 
 #pragma unroll
-    for (int it = 0; it < MAXK; ++it) {
-        const int st = it % PF;
-        const int64_t kb = wave + (int64_t)it * NWV;
+    for (int it = 0; it < ITER; ++it) {
+        const int st = it % PF, kb = wave + it * NWV;
         if (kb < KB) {
 #pragma unroll
-            for (int ks = 0; ks < 4; ++ks) {
-                const uint32_t w = ks == 0 ? breg[st].x : ks == 1 ? breg[st].y : ks == 2 ? breg[st].z : breg[st].w;
-                v4i bf;
-                bf[0] = (int)(w & 0x03030303u);
-                bf[1] = (int)((w >> 2) & 0x03030303u);
-                bf[2] = (int)((w >> 4) & 0x03030303u);
-                bf[3] = (int)((w >> 6) & 0x03030303u);
+            for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
-                for (int i = 0; i < MB; ++i)
-                    acc[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(areg[st][i][ks], bf, acc[i], 0, 0, 0);
-            }
+                for (int i = 0; i < NB; ++i) {
+                    const uint4 bq = breg[st][i];
+                    const uint32_t w = ks == 0 ? bq.x : ks == 1 ? bq.y : ks == 2 ? bq.z : bq.w;
+                    v4i bf;
+                    bf[0] = (int)(w & 0x03030303u);
+                    bf[1] = (int)((w >> 2) & 0x03030303u);
+                    bf[2] = (int)((w >> 4) & 0x03030303u);
+                    bf[3] = (int)((w >> 6) & 0x03030303u);
+                    acc[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(areg[st][ks], bf, acc[i], 0, 0, 0);
+                }
         }
-        if (it + PF < MAXK) load_stage(st, wave + (int64_t)(it + PF) * NWV);
+        if (it + PF < ITER) load_stage(st, wave + (it + PF) * NWV);
     }
 #pragma unroll
-    for (int i = 0; i < MB; ++i)
+    for (int i = 0; i < NB; ++i)
 #pragma unroll
         for (int r = 0; r < 16; ++r) red[wave][i][r][lane] = acc[i][r];
     __syncthreads();
 
 #pragma unroll
-    for (int j = 0; j < MB * 2; ++j) {
-        const int e = threadIdx.x + j * 512;             // (mb, r, lane) flattened
-        const int r = (e >> 6) & 15, mb = e >> 10;
-        int tot = 0;
+    for (int j = 0; j < EL; ++j) {
+        const int r = wave + j * NWV;
+        const int64_t m = mb * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+        float o[NB];
 #pragma unroll
-        for (int w = 0; w < NWV; ++w) tot += red[w][mb][r][lane];
-        const int64_t m = (mbase + mb) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (m < p.M && n_ok) {
-            float o = __fmul_rn(__fmul_rn((float)(tot - ep_qsum[j]), ep_deq[j]), ep_wdeq);
-            if (bias) o = __fadd_rn(o, ep_bias);
-            if (addend) o = __fadd_rn(mmf_round_to<T>(o), ep_add[j]);
-            out[m * p.ldo + n_ep] = mmf_from_float<T>(o);
+        for (int i = 0; i < NB; ++i) {
+            int tot = 0;
+#pragma unroll
+            for (int w = 0; w < NWV; ++w) tot += red[w][i][r][lane];
+            o[i] = __fmul_rn(__fmul_rn((float)(tot - ep_qsum[j]), ep_deq[j]), ep_wdeq[i]);
+        }
+        if constexpr (SWI) {
+            const float g = mmf_round_to<T>(o[0]), u = mmf_round_to<T>(o[1]);
+            if (m < p.M) out[m * p.ldo + n_ep] = mmf_from_float<T>(__fdiv_rn(__fmul_rn(g, u), __fadd_rn(1.0f, mmf_exp(-g))));
+        } else if (m < p.M && n_ok) {
+            if (bias) o[0] = __fadd_rn(o[0], ep_bias);
+            if (addend) o[0] = __fadd_rn(mmf_round_to<T>(o[0]), ep_add[j]);
+            out[m * p.ldo + n_ep] = mmf_from_float<T>(o[0]);
         }
     }
 }
 
-template <typename T, int MB>
+template <typename T, int NWV, bool SWI>
+void launch_skinny_waves(const MfmaArgs& a, dim3 grid, hipStream_t s) {
+    const int64_t it = mmf_ceil_div(a.Kp >> 7, (int64_t)NWV);
+    if (it <= 1) bitlinear_mfma_skinny_kernel<T, NWV, 1, SWI><<<grid, dim3(64 * NWV), 0, s>>>(a);
+    else if (it <= 2) bitlinear_mfma_skinny_kernel<T, NWV, 2, SWI><<<grid, dim3(64 * NWV), 0, s>>>(a);
+    else if (it <= 3) bitlinear_mfma_skinny_kernel<T, NWV, 3, SWI><<<grid, dim3(64 * NWV), 0, s>>>(a);
+    else if (it <= 4) bitlinear_mfma_skinny_kernel<T, NWV, 4, SWI><<<grid, dim3(64 * NWV), 0, s>>>(a);
+    else if constexpr (NWV == 8) {
+        if (it <= 6) bitlinear_mfma_skinny_kernel<T, NWV, 6, SWI><<<grid, dim3(64 * NWV), 0, s>>>(a);
+        else bitlinear_mfma_skinny_kernel<T, NWV, 8, SWI><<<grid, dim3(64 * NWV), 0, s>>>(a);
+    }
+}
+// Kp <= 8192: at most 64 k-blocks, four per wave of 16 or eight per wave of 8
+template <typename T>
 int launch_skinny(const MfmaArgs& a, hipStream_t s) {
-    bitlinear_mfma_skinny_kernel<T, MB><<<dim3((unsigned)mmf_ceil_div(a.N, 32), (unsigned)mmf_ceil_div(a.M, 32 * MB)), dim3(512), 0, s>>>(a);
+    const dim3 grid((unsigned)mmf_ceil_div(a.N, 32), (unsigned)mmf_ceil_div(a.M, 32));
+    if ((int64_t)grid.x * grid.y <= 256) launch_skinny_waves<T, 16, false>(a, grid, s);
+    else launch_skinny_waves<T, 8, false>(a, grid, s);
+    MMF_CHECK_LAUNCH();
+    return 0;
+}
+template <typename T>
+int launch_skinny_swiglu(const MfmaArgs& a, hipStream_t s) {
+    launch_skinny_waves<T, 8, true>(a, dim3((unsigned)(a.N / 64), (unsigned)mmf_ceil_div(a.M, 32)), s);
     MMF_CHECK_LAUNCH();
     return 0;
 }
@@ -824,6 +854,17 @@ int launch_mfma(MfmaArgs a, hipStream_t s) {
     return 0;
 }
 
+// Whether the weight-stream kernel is the faster one.  Measured on MI355X: it costs ~3 us + 0.33 ns per (output block x k-block); a
+// round of tiles of the DMA kernel ~0.9 us per k-block whatever the problem size.
+inline bool mfma_streams(const MfmaArgs& a) {
+    const int64_t KB = a.Kp >> 7;
+    const double wgs = (double)mmf_ceil_div(a.M, 32) * (double)mmf_ceil_div(a.N, 32);
+    const double tiles = (double)mmf_ceil_div(a.M, 128) * (double)mmf_ceil_div(a.N, 256);
+    const double t_stream = 3.0 + wgs * (double)KB * 0.00033;
+    const double t_tiled = (double)KB * 0.9 * (double)mmf_ceil_div((int64_t)tiles, 256);
+    return a.Kp <= 8192 && (a.M <= 64 || t_stream < t_tiled);
+}
+
 template <typename T>
 int dispatch_mfma(const MfmaArgs& a, int config, hipStream_t s) {
     // config < 0: pick by shape.
@@ -832,14 +873,7 @@ int dispatch_mfma(const MfmaArgs& a, int config, hipStream_t s) {
     //   15 / 16 / 17  256x256 / 128x256 / 64x512 tiles, A staged by DMA (17: every wave reads the whole activation
     //            tile from LDS and owns its own weight columns, so no weight block is fetched twice)
     if (config < 0) {
-        const int64_t KB = a.Kp >> 7;
-        const double wgs = (double)mmf_ceil_div(a.M, 32) * (double)mmf_ceil_div(a.N, 32);
-        const double tiles = (double)mmf_ceil_div(a.M, 128) * (double)mmf_ceil_div(a.N, 256);
-        // measured on MI355X: the stream kernel costs ~3 us + 0.33 ns per (output block x k-block); a round of
-        // tiles of the DMA kernel ~0.9 us per k-block whatever the problem size
-        const double t_stream = 3.0 + wgs * (double)KB * 0.00033;
-        const double t_tiled = (double)KB * 0.9 * (double)mmf_ceil_div((int64_t)tiles, 256);
-        if (a.Kp <= 8192 && (a.M <= 64 || t_stream < t_tiled)) config = 5;
+        if (mfma_streams(a)) config = 5;
         else if (a.M <= 32) config = 0;
         else if (a.M <= 64) config = 1;
         else config = a.N >= 512 ? 17 : 16;
@@ -864,7 +898,7 @@ int dispatch_mfma(const MfmaArgs& a, int config, hipStream_t s) {
         return 0;
     }
     switch (config) {
-        case 5: return launch_skinny<T, 1>(a, s);
+        case 5: return launch_skinny<T>(a, s);
         case 0: return launch_mfma<T, 1, 8, 1, 1>(a, s);
         case 1: return launch_mfma<T, 1, 8, 2, 1>(a, s);
         case 15: return launch_mfma_dma3<T, 2, 4, 4, 2>(a, s);
@@ -987,9 +1021,9 @@ int mmf_bitlinear_mfma_swiglu(const int8_t* codes_tiled, const float* deq, const
     a.a = codes_tiled; a.b = static_cast<const uint4*>(packed); a.deq = deq; a.qsum = qsum; a.wdeq = wdeq;
     a.out = out; a.M = M; a.N = N; a.Kp = mmf_round_up(K, 128); a.seg_rows = seg_rows; a.ldo = ldo;
     switch (out_dtype) {
-        case MMF_F32: return launch_mfma_dma3_swiglu<float>(a, stream);
-        case MMF_BF16: return launch_mfma_dma3_swiglu<bf16_t>(a, stream);
-        case MMF_F16: return launch_mfma_dma3_swiglu<f16_t>(a, stream);
+        case MMF_F32: return mfma_streams(a) ? launch_skinny_swiglu<float>(a, stream) : launch_mfma_dma3_swiglu<float>(a, stream);
+        case MMF_BF16: return mfma_streams(a) ? launch_skinny_swiglu<bf16_t>(a, stream) : launch_mfma_dma3_swiglu<bf16_t>(a, stream);
+        case MMF_F16: return mfma_streams(a) ? launch_skinny_swiglu<f16_t>(a, stream) : launch_mfma_dma3_swiglu<f16_t>(a, stream);
     }
     return MMF_ERR_ARG;
 }

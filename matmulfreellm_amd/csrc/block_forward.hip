@@ -9,7 +9,6 @@
 namespace {
 
 constexpr int64_t kGemvRows = 8;      // rows up to which every workgroup of a BitLinear redoes the row's prologue (one launch)
-constexpr int64_t kSwigluRows = 512;  // rows from which the gate/up contraction runs tiled and carries the swiglu in its epilogue
 
 // prologue / epilogue ids of mmf_bitlinear_gemv_fused and mmf_rmsnorm_quant_fused
 enum { G_PLAIN = 0, G_NORM = 1, G_RESNORM = 2, G_GATEDNORM = 3, E_PLAIN = 0, E_STEP = 1, E_SWIGLU = 2 };
@@ -184,16 +183,9 @@ int mmf_block_forward(const mmf_block* p, const void* x, void* out, int64_t B, i
     MMF_DO(mmf_bitlinear_mfma(q, deq, qsum, p->o_packed, p->o_wdeq, p->o_seg_rows, nullptr, nullptr, attn, H, M, D, H, dt, -1, stream));
     MMF_DO(mmf_rmsnorm_quant_fused(Q_RESNORM, attn, H, x, H, nullptr, 0, res, p->mlp_norm, p->mlp_eps, p->gate_norm, p->gate_eps, nullptr,
                                    nullptr, q, deq, qsum, M, H, dt, wt, stream));
-    if (M >= kSwigluRows) {
-        MMF_DO(mmf_bitlinear_mfma_swiglu(q, deq, qsum, p->gate_packed, p->gate_wdeq, p->gate_seg_rows, big, I, M, H, 2 * I, dt, stream));
-        MMF_DO(mmf_rmsnorm_quant_fused(Q_PLAIN, big, I, nullptr, 0, nullptr, 0, nullptr, nullptr, 0.0f, p->down_norm, p->down_eps, nullptr,
-                                       nullptr, q, deq, qsum, M, I, dt, wt, stream));
-    } else {
-        MMF_DO(mmf_bitlinear_mfma(q, deq, qsum, p->gate_packed, p->gate_wdeq, p->gate_seg_rows, nullptr, nullptr, big, 2 * I, M, H, 2 * I,
-                                  dt, -1, stream));
-        MMF_DO(mmf_rmsnorm_quant_fused(Q_SWIGLU, big, 2 * I, big + I * e, 2 * I, nullptr, 0, nullptr, nullptr, 0.0f, p->down_norm,
-                                       p->down_eps, nullptr, nullptr, q, deq, qsum, M, I, dt, wt, stream));
-    }
+    MMF_DO(mmf_bitlinear_mfma_swiglu(q, deq, qsum, p->gate_packed, p->gate_wdeq, p->gate_seg_rows, big, I, M, H, 2 * I, dt, stream));
+    MMF_DO(mmf_rmsnorm_quant_fused(Q_PLAIN, big, I, nullptr, 0, nullptr, 0, nullptr, nullptr, 0.0f, p->down_norm, p->down_eps, nullptr,
+                                   nullptr, q, deq, qsum, M, I, dt, wt, stream));
     MMF_DO(mmf_bitlinear_mfma(q, deq, qsum, p->down_packed, p->down_wdeq, p->down_seg_rows, nullptr, res, out, H, M, I, H, dt, -1, stream));
 #undef MMF_DO
     return 0;

@@ -333,7 +333,7 @@ class DecodeEngine:
         esz = self.h.element_size()
         L.check(lib.mmf_embedding(self.table.data_ptr(), self.tok.data_ptr(), self.h.data_ptr(), B, H, self.V,
                                   self.dt_id, s), "mmf_embedding")
-        ifg, y = self.ifg.data_ptr(), self.y.data_ptr()
+        ifg = self.ifg.data_ptr()
         for ent in self.layers:
             nw, eps = ent["projs"][0][1], ent["projs"][0][2]
             if ent["norms"] is not None:
@@ -354,8 +354,11 @@ class DecodeEngine:
             self._mfma(ent["o"][0], self.a, H, D)
             self._qfused(2, self.a.data_ptr(), H, self.h.data_ptr(), H, None, 0, self.res, ent["mlp_norm"], self.eps,
                          ent["gate"][1], ent["gate"][2], None, None, H)
-            self._mfma(ent["gate"][0], self.y, 2 * I, H)
-            self._qfused(4, y, 2 * I, y + I * esz, 2 * I, None, 0, None, None, 0.0, ent["down"][1], ent["down"][2], None, None, I)
+            gate = ent["gate"][0]
+            L.check(lib.mmf_bitlinear_mfma_swiglu(self.q.data_ptr(), self.deq.data_ptr(), self.qsum.data_ptr(), gate.packed.data_ptr(),
+                                                  gate.wdeq.data_ptr(), gate.seg_rows, self.zb.data_ptr(), I, B, H, 2 * I, self.dt_id, s),
+                    "mmf_bitlinear_mfma_swiglu")
+            self._qfused(0, self.zb.data_ptr(), I, None, 0, None, 0, None, None, 0.0, ent["down"][1], ent["down"][2], None, None, I)
             self._mfma(ent["down"][0], self.h, H, I, addend=self.res)
         self._qfused(1, self.h.data_ptr(), H, None, 0, None, 0, None, self.final_norm, self.eps, self.head[1], self.head[2],
                      None, None, H)
@@ -367,7 +370,7 @@ class DecodeEngine:
                       for t in (e["attn_norm"], e["mlp_norm"], e["g_norm"], e["o"][1], e["gate"][1], e["down"][1],
                                 *(p[1] for p in e["projs"]))) and self.head[1].dtype == self.final_norm.dtype
         return (not self.gemv and same_dt and all(e["ifg"] is not None for e in self.layers)
-                and max(self.H, self.D, self.I) <= 8192 and (3 * self.D) % 8 == 0 and (2 * self.I) % 8 == 0)
+                and max(self.H, self.D, self.I) <= 8192 and (3 * self.D) % 8 == 0 and self.I % 32 == 0)
 
     def _can_fuse(self):
         kmax = self.lib.mmf_bitlinear_gemv_max_k()
