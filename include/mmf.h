@@ -215,6 +215,10 @@ int mmf_hgrn_step(const void* i_in, int64_t ldi, const void* f_in, int64_t ldf, 
  *   (modeling_hgrn_bit.py:386): out[r] = lowest index of the row maximum (int64). */
 int mmf_embedding(const void* table, const int64_t* ids, void* out, int64_t rows, int64_t H, int64_t vocab,
                   int dtype, void* stream);
+/* The same, and row r's id goes to history[pos[r] * rows + r]; pos[r] then advances, modulo cap.  history null: not recorded.  A
+ * decode loop replayed as a graph keeps its tokens this way without a copy per step. */
+int mmf_embedding_record(const void* table, const int64_t* ids, void* out, int64_t rows, int64_t H, int64_t vocab, int64_t* history,
+                         int* pos, int cap, int dtype, void* stream);
 int mmf_argmax(const void* logits, int64_t ld, int64_t rows, int64_t V, int64_t* out, int dtype, void* stream);
 
 /* ---- next-token loss (forward only) -----------------------------------------------------------
@@ -356,10 +360,11 @@ int mmf_decode_layers(const void* phases, int n_layers, const void* table, const
                       void* h_out, const void* head, void* logits, uint64_t* am_words, int64_t* tok_out, uint32_t* epoch, int* err,
                       int H, int D, int I, int spin, int dtype, void* stream);
 /* The same with the number of inner norms behind an i/f/g record: 1, or 3 when i, f and g have norms of their own (norm_w of
- * those records then points to [3, K] weights). */
+ * those records then points to [3, K] weights), and with the token fed recorded as mmf_embedding_record does (history null: not). */
 int mmf_decode_layers_norms(int norms, const void* phases, int n_layers, const void* table, const int64_t* tok, int64_t vocab,
                             uint32_t* words, void* h_out, const void* head, void* logits, uint64_t* am_words, int64_t* tok_out,
-                            uint32_t* epoch, int* err, int H, int D, int I, int spin, int dtype, void* stream);
+                            uint32_t* epoch, int* err, int64_t* history, int* pos, int cap, int H, int D, int I, int spin, int dtype,
+                            void* stream);
 
 /* ---- stacked projections whose inner norms differ (a trained checkpoint's i, f and g): one row, three norm weights
  * mmf_rmsnorm_quant_multi: mmf_rmsnorm_quant_fused with the norm prologue (w1, eps1), quantised under three norm weights:

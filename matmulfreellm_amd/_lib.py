@@ -41,7 +41,7 @@ SIGNATURES = {
     "mmf_decode_layers": (_i32, [_ptr, _i32, _ptr, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr,
                                  _i32, _i32, _i32, _i32, _i32, _ptr]),
     "mmf_decode_layers_norms": (_i32, [_i32, _ptr, _i32, _ptr, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr,
-                                       _i32, _i32, _i32, _i32, _i32, _ptr]),
+                                       _ptr, _ptr, _i32, _i32, _i32, _i32, _i32, _i32, _ptr]),
     "mmf_decode_layers_trace_words": (_i32, []),
     "mmf_decode_layers_traced": (_i32, [_ptr, _i32, _ptr, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr,
                                         _i32, _i32, _i32, _i32, _i32, _i32, _ptr]),
@@ -60,6 +60,7 @@ SIGNATURES = {
     "mmf_hgrn_gate": (_i32, [_ptr, _i64, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i32, _ptr]),
     "mmf_hgrn_step": (_i32, [_ptr, _i64, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i32, _ptr]),
     "mmf_embedding": (_i32, [_ptr, _ptr, _ptr, _i64, _i64, _i64, _i32, _ptr]),
+    "mmf_embedding_record": (_i32, [_ptr, _ptr, _ptr, _i64, _i64, _i64, _ptr, _ptr, _i32, _i32, _ptr]),
     "mmf_argmax": (_i32, [_ptr, _i64, _i64, _i64, _ptr, _i32, _ptr]),
     "mmf_cross_entropy_fwd": (_i32, [_ptr, _i64, _ptr, _i64, _ptr, _i64, _i64, _i32, _ptr]),
     "mmf_backward_groups": (_i32, [_i64]),

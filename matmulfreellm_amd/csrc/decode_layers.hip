@@ -85,6 +85,9 @@ struct LayersArgs {
     int64_t* tok_out;         // head: the greedy token
     uint32_t* epoch;          // tag base; advanced by 4 * n_layers + 2 at the end of the launch
     int* err;                 // set to 1 when a poll ran out of rounds
+    int64_t* history;         // null, or where the token fed is recorded: history[*pos], *pos advancing modulo cap
+    int* pos;
+    int cap;
     long long* trace;         // TRACE builds: kTraceWGs * kTraceLinks * kTraceStamps cycle stamps
     int n_layers, H, D, I, spin;
     int delay[5];             // hold-back of a link's first poll, per kind of link, in units of about 64 cycles
@@ -233,6 +236,11 @@ __global__ __launch_bounds__(kNT) void decode_layers_kernel(LayersArgs a) {
     __shared__ Small sm;
     const uint32_t e = *a.epoch;
     int64_t id = *a.tok;
+    if (a.history && blockIdx.x == 0 && threadIdx.x == 0) {
+        const int at = *a.pos;
+        a.history[at] = id;
+        *a.pos = at + 1 < a.cap ? at + 1 : 0;
+    }
     if (id < 0 || id >= a.vocab) id = 0;
     const int L = a.n_layers;
     const T* emb_row = static_cast<const T*>(a.table) + id * (S::kStatic ? S::H : a.H);
@@ -935,11 +943,13 @@ int launch_layers(LayersArgs a, hipStream_t s) {
 
 int decode_layers_entry(const void* phases, int n_layers, const void* table, const int64_t* tok, int64_t vocab, uint32_t* words,
                         void* h_out, const void* head, void* logits, uint64_t* am_words, int64_t* tok_out, uint32_t* epoch, int* err,
-                        int64_t* trace, int norms, int H, int D, int I, int spin, const int* delay, int dtype, void* stream_) {
+                        int64_t* trace, int norms, int64_t* history, int* pos, int cap, int H, int D, int I, int spin, const int* delay, int dtype,
+                        void* stream_) {
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     if (!phases || n_layers <= 0 || !table || !tok || vocab <= 0 || !words || !h_out || !epoch || !err || H <= 0 || D <= 0 || I <= 0 ||
         spin <= 0 || !delay)
         return MMF_ERR_ARG;
+    if (history && (!pos || cap <= 0)) return MMF_ERR_ARG;
     for (int k = 0; k < 5; ++k)
         if (delay[k] < 0 || delay[k] > 64) return MMF_ERR_ARG;
     if (head && (!logits || !am_words || !tok_out)) return MMF_ERR_ARG;
@@ -957,6 +967,7 @@ int decode_layers_entry(const void* phases, int n_layers, const void* table, con
     a.words = words; a.h_out = h_out; a.head = static_cast<const Phase*>(head); a.logits = logits; a.am_words = am_words;
     a.tok_out = tok_out; a.epoch = epoch; a.err = err; a.trace = reinterpret_cast<long long*>(trace);
     a.H = H; a.D = D; a.I = I; a.spin = spin;
+    a.history = history; a.pos = pos; a.cap = cap;
     for (int k = 0; k < 5; ++k) a.delay[k] = delay[k];
     if (trace) {
         switch (dtype) {
@@ -984,7 +995,7 @@ int mmf_decode_layers_copies(void) { return kRep; }
 
 int mmf_decode_layers_norms(int norms, const void* phases, int n_layers, const void* table, const int64_t* tok, int64_t vocab, uint32_t* words,
                       void* h_out, const void* head, void* logits, uint64_t* am_words, int64_t* tok_out, uint32_t* epoch, int* err,
-                      int H, int D, int I, int spin, int dtype, void* stream) {
+                      int64_t* history, int* pos, int cap, int H, int D, int I, int spin, int dtype, void* stream) {
     if (norms != 1 && norms != 3) return MMF_ERR_ARG;
     // hold-back of the first poll per kind of link (i/f/g, o_proj, gate/up, down_proj, lm_head); MMF_DECODE_POLL_DELAY
     // ("a" or "a,b,c,d,e") overrides the tuned values
@@ -1005,14 +1016,14 @@ int mmf_decode_layers_norms(int norms, const void* phases, int n_layers, const v
     } delays;
     const int* delay = delays.d;
     return decode_layers_entry(phases, n_layers, table, tok, vocab, words, h_out, head, logits, am_words, tok_out, epoch, err, nullptr,
-                               norms, H, D, I, spin, delay, dtype, stream);
+                               norms, history, pos, cap, H, D, I, spin, delay, dtype, stream);
 }
 
 int mmf_decode_layers(const void* phases, int n_layers, const void* table, const int64_t* tok, int64_t vocab, uint32_t* words,
                       void* h_out, const void* head, void* logits, uint64_t* am_words, int64_t* tok_out, uint32_t* epoch, int* err,
                       int H, int D, int I, int spin, int dtype, void* stream) {
-    return mmf_decode_layers_norms(1, phases, n_layers, table, tok, vocab, words, h_out, head, logits, am_words, tok_out, epoch, err, H, D,
-                                   I, spin, dtype, stream);
+    return mmf_decode_layers_norms(1, phases, n_layers, table, tok, vocab, words, h_out, head, logits, am_words, tok_out, epoch, err, nullptr,
+                                   nullptr, 0, H, D, I, spin, dtype, stream);
 }
 
 int mmf_decode_layers_trace_words(void) { return kTraceWGs * kTraceLinks * kTraceStamps; }
@@ -1022,7 +1033,7 @@ int mmf_decode_layers_traced(const void* phases, int n_layers, const void* table
                              int64_t* trace, int H, int D, int I, int spin, int delay, int dtype, void* stream) {
     if (!trace) return MMF_ERR_ARG;
     const int d[5] = {delay, delay, delay, delay, delay};
-    return decode_layers_entry(phases, n_layers, table, tok, vocab, words, h_out, head, logits, am_words, tok_out, epoch, err, trace, 1, H, D,
+    return decode_layers_entry(phases, n_layers, table, tok, vocab, words, h_out, head, logits, am_words, tok_out, epoch, err, trace, 1, nullptr, nullptr, 0, H, D,
                                I, spin, d, dtype, stream);
 }
 

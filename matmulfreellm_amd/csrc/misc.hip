@@ -11,9 +11,15 @@ namespace {
 
 template <typename T>
 __global__ __launch_bounds__(256) void embedding_kernel(const T* __restrict__ table, const int64_t* __restrict__ ids,
-                                                        T* __restrict__ out, int64_t rows, int64_t H, int64_t vocab) {
+                                                        T* __restrict__ out, int64_t rows, int64_t H, int64_t vocab,
+                                                        int64_t* __restrict__ history, int* __restrict__ pos, int cap) {
     const int64_t r = blockIdx.x;
     int64_t id = ids[r];
+    if (history && threadIdx.x == 0) {   // a decode loop's record of what it fed: row r counts its own steps
+        const int at = pos[r];
+        history[(int64_t)at * rows + r] = id;
+        pos[r] = at + 1 < cap ? at + 1 : 0;
+    }
     if (id < 0 || id >= vocab) id = 0;   // out-of-range ids read row 0 instead of faulting
     const T* src = table + id * H;
     T* dst = out + r * H;
@@ -104,20 +110,27 @@ __global__ __launch_bounds__(256) void exact_forms_kernel(unsigned long long* co
 
 extern "C" {
 
-int mmf_embedding(const void* table, const int64_t* ids, void* out, int64_t rows, int64_t H, int64_t vocab, int dtype,
-                  void* stream_) {
+int mmf_embedding_record(const void* table, const int64_t* ids, void* out, int64_t rows, int64_t H, int64_t vocab, int64_t* history,
+                         int* pos, int cap, int dtype, void* stream_) {
     hipStream_t stream = static_cast<hipStream_t>(stream_);
-    if (rows < 0 || H <= 0 || vocab <= 0) return MMF_ERR_ARG;
+    if (rows < 0 || H <= 0 || vocab <= 0 || (history && (!pos || cap <= 0))) return MMF_ERR_ARG;
     if (rows == 0) return 0;
     if (!table || !ids || !out) return MMF_ERR_ARG;
+#define MMF_EM(T) embedding_kernel<T><<<(unsigned)rows, 256, 0, stream>>>(static_cast<const T*>(table), ids, static_cast<T*>(out), rows, H, \
+                                                                         vocab, history, pos, cap)
     switch (dtype) {
-        case MMF_F32: embedding_kernel<float><<<(unsigned)rows, 256, 0, stream>>>(static_cast<const float*>(table), ids, static_cast<float*>(out), rows, H, vocab); break;
-        case MMF_BF16: embedding_kernel<bf16_t><<<(unsigned)rows, 256, 0, stream>>>(static_cast<const bf16_t*>(table), ids, static_cast<bf16_t*>(out), rows, H, vocab); break;
-        case MMF_F16: embedding_kernel<f16_t><<<(unsigned)rows, 256, 0, stream>>>(static_cast<const f16_t*>(table), ids, static_cast<f16_t*>(out), rows, H, vocab); break;
+        case MMF_F32: MMF_EM(float); break;
+        case MMF_BF16: MMF_EM(bf16_t); break;
+        case MMF_F16: MMF_EM(f16_t); break;
         default: return MMF_ERR_ARG;
     }
+#undef MMF_EM
     MMF_CHECK_LAUNCH();
     return 0;
+}
+
+int mmf_embedding(const void* table, const int64_t* ids, void* out, int64_t rows, int64_t H, int64_t vocab, int dtype, void* stream) {
+    return mmf_embedding_record(table, ids, out, rows, H, vocab, nullptr, nullptr, 0, dtype, stream);
 }
 
 int mmf_argmax(const void* logits, int64_t ld, int64_t rows, int64_t V, int64_t* out, int dtype, void* stream_) {

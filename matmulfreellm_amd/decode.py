@@ -34,6 +34,7 @@ class _Phase(ctypes.Structure):
 
 
 class DecodeEngine:
+    CHUNK = 32          # steps whose input tokens the recorded graph keeps before the host has to fetch them
     SPIN = 1 << 15      # polling rounds a resident workgroup waits for its input before it gives up (mmf_decode_layers)
 
     @classmethod
@@ -63,7 +64,10 @@ class DecodeEngine:
         self.L = len(model.model.layers)
         self.eps = float(cfg.rms_norm_eps)
         self.use_graph = use_graph
-        self._version_key = self._param_versions()
+        # what the operands below were taken from: modules, parameters (object, version, address)
+        self._children = [(d["_modules"], k, c) for d in (m.__dict__ for m in model.modules()) for k, c in d["_modules"].items()]
+        self._parameters = [(d["_parameters"], k, p, p._version, p.data_ptr()) for d in (m.__dict__ for m in model.modules())
+                            for k, p in d["_parameters"].items() if p is not None]
 
         attn0 = model.model.layers[0].attn
         self.D = D = attn0.input_dim
@@ -100,6 +104,9 @@ class DecodeEngine:
 
         # ---- static activation buffers
         self.tok = torch.zeros(B, dtype=torch.int64, device=dev)
+        # every step records the token it was fed: row t of the history is step t's, modulo CHUNK, counted per batch row
+        self.history = torch.zeros(self.CHUNK, B, dtype=torch.int64, device=dev)
+        self.pos = torch.zeros(B, dtype=torch.int32, device=dev)
         self.h = z(B, H)            # residual stream
         self.hn = z(B, H)
         self.ifg = z(B, 3 * D)
@@ -137,11 +144,15 @@ class DecodeEngine:
     def _eps_of(p):
         return float(p.norm.eps if getattr(p, "fused_eps", None) is None else p.fused_eps)
 
-    def _param_versions(self):
-        return tuple((p.data_ptr(), p._version) for p in self.model.parameters())
-
     def stale(self):
-        return self._param_versions() != self._version_key
+        """Whether a module or parameter the engine was built on has been replaced or written since."""
+        for d, k, p, version, address in self._parameters:
+            if d.get(k) is not p or p._version != version or p.data_ptr() != address:
+                return True
+        for d, k, c in self._children:
+            if d.get(k) is not c:
+                return True
+        return False
 
     # ------------------------------------------------------------------ launches
     def _bitlinear(self, x, pw_nw_eps, out, n_k, addend=None):
@@ -226,8 +237,9 @@ class DecodeEngine:
         args = (self.phases.data_ptr(), self.L, self.table.data_ptr(), self.tok.data_ptr(), self.V, self._words.data_ptr(),
                 self.h.data_ptr(), head, self.logits.data_ptr(), self.am_words.data_ptr(), self.tok.data_ptr(),
                 self.epoch.data_ptr(), self.err.data_ptr())
+        record = (self.history.data_ptr(), self.pos.data_ptr(), self.CHUNK)
         if trace is None:
-            L.check(self.lib.mmf_decode_layers_norms(self.norms, *args, self.H, self.D, self.I, self.SPIN, self.dt_id, L.stream()),
+            L.check(self.lib.mmf_decode_layers_norms(self.norms, *args, *record, self.H, self.D, self.I, self.SPIN, self.dt_id, L.stream()),
                     "mmf_decode_layers_norms")
         else:
             assert self.norms == 1, "the traced kernel is built for shared inner norms"
@@ -271,13 +283,17 @@ class DecodeEngine:
                              "on this device?); the tokens of this generation are invalid. Build the engine with "
                              "resident=False to decode with one launch per BitLinear.")
 
+    def _embed(self):
+        L.check(self.lib.mmf_embedding_record(self.table.data_ptr(), self.tok.data_ptr(), self.h.data_ptr(), self.B, self.H, self.V,
+                                              self.history.data_ptr(), self.pos.data_ptr(), self.CHUNK, self.dt_id, L.stream()),
+                "mmf_embedding_record")
+
     def _launch_step_fused(self, ends=True):
         """Batch <= GEMV_MAX_M: four launches per layer, every elementwise op folded into a GEMV.
         ends=False leaves out the embedding gather and the argmax (the 4L+1 GEMV launches only)."""
         lib, s, B, H, D, I = self.lib, L.stream(), self.B, self.H, self.D, self.I
         if ends:
-            L.check(lib.mmf_embedding(self.table.data_ptr(), self.tok.data_ptr(), self.h.data_ptr(), B, H, self.V,
-                                      self.dt_id, s), "mmf_embedding")
+            self._embed()
         g_buf = self.ifg.view(-1)[:B * D].view(B, D)
         for ent in self.layers:
             if ent["norms"] is not None:
@@ -331,8 +347,7 @@ class DecodeEngine:
         (norm / recurrence step + gated norm / residual norm / swiglu folded in) and a matrix-core contraction."""
         lib, s, B, H, D, I = self.lib, L.stream(), self.B, self.H, self.D, self.I
         esz = self.h.element_size()
-        L.check(lib.mmf_embedding(self.table.data_ptr(), self.tok.data_ptr(), self.h.data_ptr(), B, H, self.V,
-                                  self.dt_id, s), "mmf_embedding")
+        self._embed()
         ifg = self.ifg.data_ptr()
         for ent in self.layers:
             nw, eps = ent["projs"][0][1], ent["projs"][0][2]
@@ -390,8 +405,7 @@ class DecodeEngine:
         lib, s, B, H, D, I = self.lib, L.stream(), self.B, self.H, self.D, self.I
         dt, esz = self.dt_id, self.h.element_size()
         wid = L.dtype_id(self.final_norm.dtype)
-        L.check(lib.mmf_embedding(self.table.data_ptr(), self.tok.data_ptr(), self.h.data_ptr(), B, H, self.V, dt, s),
-                "mmf_embedding")
+        self._embed()
         for ent in self.layers:
             L.check(lib.mmf_rmsnorm(self.h.data_ptr(), None, ent["attn_norm"].data_ptr(), self.hn.data_ptr(), None, B, H,
                                     self.eps, dt, dt, wid, s), "mmf_rmsnorm")
@@ -424,7 +438,7 @@ class DecodeEngine:
     def _capture(self):
         # warm-up launches on a side stream (module loading, attribute setting), then record
         saved = [e["state"].clone() for e in self.layers]
-        tok = self.tok.clone()
+        tok, pos = self.tok.clone(), self.pos.clone()
         side = torch.cuda.Stream(device=self.dev)
         side.wait_stream(torch.cuda.current_stream(self.dev))
         with torch.cuda.stream(side):
@@ -451,16 +465,18 @@ class DecodeEngine:
         for e, sv in zip(self.layers, saved):     # undo the warm-up step's state update
             e["state"].copy_(sv)
         self.tok.copy_(tok)
+        self.pos.copy_(pos)
         self.graph = g
 
     # ------------------------------------------------------------------ public
     def load_state(self, states: Optional[List[torch.Tensor]]):
         """Set the per-layer recurrent states ([B, *, D] tensors, or None for zeros)."""
-        for i, e in enumerate(self.layers):
-            if states is None:
-                e["state"].zero_()
-            else:
-                e["state"].copy_(states[i].reshape(self.B, self.D).to(torch.float32))
+        if states is None:
+            torch._foreach_zero_([e["state"] for e in self.layers])
+        else:
+            # one launch for all layers (a copy per layer costs more than a decode step's layer)
+            torch._foreach_copy_([e["state"] for e in self.layers],
+                                 [s.reshape(self.B, self.D).to(device=self.dev, dtype=torch.float32) for s in states])
 
     def export_state(self):
         return [e["state"].clone() for e in self.layers]
@@ -482,13 +498,33 @@ class DecodeEngine:
         self.advance()
         return self.logits
 
+    def run(self, n_steps: int, pick=None, seen=None) -> torch.Tensor:
+        """n_steps self-feeding steps from the token buffer; returns the [n_steps + 1, B] tokens: what the buffer held, then what
+        it held after each step.  pick(t), when given, replaces the token step t chose.  seen(tokens [t + 1, B]), when given, is
+        asked every CHUNK steps whether to stop there.  No host synchronisation of its own."""
+        out = torch.empty(n_steps + 1, self.B, dtype=torch.int64, device=self.dev)
+        self.pos.zero_()
+        done = 0
+        while done < n_steps:
+            n = min(self.CHUNK, n_steps - done)
+            for t in range(done, done + n):
+                self.advance()
+                if pick is not None:
+                    pick(t)
+            out[done:done + n].copy_(self.history[:n])
+            done += n
+            if seen is not None or done == n_steps:
+                out[done].copy_(self.tok)
+            if seen is not None and seen(out[:done + 1]):
+                break
+        if n_steps == 0:
+            out[0].copy_(self.tok)
+        return out[:done + 1]
+
     def greedy(self, first_tokens: torch.Tensor, n_steps: int) -> torch.Tensor:
         """Run n_steps self-feeding greedy steps starting from first_tokens [B]; returns the
         [B, n_steps] tokens chosen after each step.  One host synchronisation at the end."""
-        out = torch.empty(n_steps, self.B, dtype=torch.int64, device=self.dev)
         self.tok.copy_(first_tokens.reshape(self.B))
-        for t in range(n_steps):
-            self.advance()
-            out[t].copy_(self.tok)
+        out = self.run(n_steps)[1:]
         self.check()
         return out.t().contiguous()

@@ -528,13 +528,16 @@ def embedding(table, ids):
     return out.reshape(*ids.shape, tb.shape[1])
 
 
-def argmax(logits):
-    """Lowest index of the maximum over the last dim; logits [..., V] -> int64 [...]."""
+def argmax(logits, out=None):
+    """Lowest index of the maximum over the last dim; logits [..., V] -> int64 [...] (written to `out` [rows], when given)."""
     lib = L.load()
     dev = L.require_gpu(logits)
     v = logits.shape[-1]
     l2 = _as_2d(logits)
-    out = torch.empty(l2.shape[0], dtype=torch.int64, device=dev)
+    if out is None:
+        out = torch.empty(l2.shape[0], dtype=torch.int64, device=dev)
+    elif not (out.dtype == torch.int64 and out.device == dev and out.numel() == l2.shape[0] and out.is_contiguous()):
+        raise L.MMFError("argmax: out must be a contiguous int64 tensor with one element per row")
     with L.on(dev):
         L.check(lib.mmf_argmax(l2.data_ptr(), v, l2.shape[0], v, out.data_ptr(), L.dtype_id(l2.dtype), L.stream()),
                 "mmf_argmax")

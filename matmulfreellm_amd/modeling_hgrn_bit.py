@@ -530,10 +530,11 @@ class HGRNBitForCausalLM(HGRNBitPreTrainedModel, GenerationMixin):
             else:
                 choose = lambda lg, step, out=None: _sample_top_p(lg.float(), top_p, temperature, uniforms[step], out,
                                                                   top_k=top_k)
-        first = choose(logits, 0) if do_sample else F_.argmax(logits)
+        tok = engine.tok if engine is not None else None         # the engine's own buffer: its first step embeds it
+        first = choose(logits, 0, tok) if do_sample else F_.argmax(logits, tok)
         if engine is not None:
-            pick = (lambda step: choose(engine.logits, step, engine.tok)) if do_sample else None
-            new = _self_feeding(engine, first, max_new_tokens, eos_token_id, pad_token_id, pick=pick)
+            pick = (lambda step: choose(engine.logits, step + 1, engine.tok)) if do_sample else None
+            new = _self_feeding(engine, max_new_tokens, eos_token_id, pad_token_id, pick=pick)
             engine.check()
             return torch.cat([input_ids, new], dim=1)
         nxt = first
@@ -552,28 +553,14 @@ class HGRNBitForCausalLM(HGRNBitPreTrainedModel, GenerationMixin):
         return torch.cat(tokens, dim=1)
 
 
-def _self_feeding(engine, first, max_new_tokens, eos_token_id, pad_token_id, chunk=32, pick=None):
-    """Decoding without a host round trip per token: every replay of the engine's graph leaves its argmax in the
-    token buffer the next replay embeds; pick(step), when given, replaces that token by one drawn from the step's
-    logits (sampling) before it is recorded.  The end-of-sequence test looks at a whole chunk of steps at a time;
+def _self_feeding(engine, max_new_tokens, eos_token_id, pad_token_id, pick=None):
+    """Decoding from the engine's token buffer without a host round trip per token: every replay of its graph leaves its
+    argmax in the buffer the next replay embeds and records; pick(step), when given, replaces that token by one drawn
+    from the step's logits (sampling).  The end-of-sequence test looks at a whole chunk of steps at a time;
     the steps decoded past the point where every row had finished are cut off, and a finished row's later tokens
     are replaced by the padding id, so the result is the one of the token-by-token loop."""
-    B = first.shape[0]
-    buf = torch.empty(max_new_tokens, B, dtype=torch.int64, device=first.device)
-    buf[0].copy_(first)
-    engine.tok.copy_(first.reshape(B))
-    produced = 1
-    while produced < max_new_tokens:
-        n = min(chunk, max_new_tokens - produced)
-        for _ in range(n):
-            engine.advance()
-            if pick is not None:
-                pick(produced)
-            buf[produced].copy_(engine.tok)
-            produced += 1
-        if eos_token_id is not None and bool((buf[:produced] == eos_token_id).any(0).all()):
-            break
-    seq = buf[:produced].t()                                                    # [B, produced]
+    seen = (lambda toks: bool((toks == eos_token_id).any(0).all())) if eos_token_id is not None else None
+    seq = engine.run(max_new_tokens - 1, pick, seen).t()                        # [B, produced]
     if eos_token_id is None:
         return seq.contiguous()
     is_eos = seq == eos_token_id
