@@ -442,21 +442,25 @@ __device__ __forceinline__ void mfma_barrier_vm() {
 // FAST (chosen by the launcher): 16-byte stores possible and no bias -> lean epilogue, accumulators start at -qsum.
 // SWI: the weight is the stacked [gate; up] projection (N = 2 * I): a wave's two n-blocks are the gate and the up rows
 // of the same 32 channels, a workgroup tile covers WGN such channel blocks, and the epilogue writes swiglu(gate, up).
-template <typename T, int WGM, int WGN, int WM, int WN, bool FAST, bool SWI = false>
-__global__ __launch_bounds__(64 * WGM * WGN, (WM * WN <= 4 ? 4 : 1))   // small wave tiles: 4 waves per SIMD = two workgroups per CU
+// KS > 1: the workgroup's waves form KS groups that take every KS-th k-block of the same (KS times narrower) tile: a mid-sized
+// problem then has KS times as many tiles at the same work per wave, and each wave's chain is KS times shorter.  The groups
+// exchange partial sums through LDS at the end (integers: exact), each finishing its share of the wave tile.
+template <typename T, int WGM, int WGN, int WM, int WN, int KS, bool FAST, bool SWI = false>
+__global__ __launch_bounds__(64 * WGM * WGN * KS, (WM * WN <= 4 ? 4 : 1))   // small wave tiles: 4 waves per SIMD = two workgroups per CU
 void bitlinear_mfma_dma3_kernel(MfmaArgs p) {
-    constexpr int NW = WGM * WGN;
+    constexpr int NT = WGM * WGN;                  // waves that cover the tile once
+    constexpr int NW = NT * KS;
     constexpr int BMB = WGM * WM;
     constexpr int BNB = WGN * WN;
     constexpr int CH = 4096;                       // bytes of one m-block's k-block
-    constexpr int BUF = BMB * CH;
-    constexpr int WPIECES = BMB * CH / 1024;       // 1 KiB wave-loads per k-block
+    constexpr int BUF = BMB * CH * KS;             // one step: a k-block for each group
+    constexpr int WPIECES = BUF / 1024;            // 1 KiB wave-loads per step
     constexpr int NDMA = (WPIECES + NW - 1) / NW;  // per wave
     static_assert(WPIECES % NW == 0, "every wave issues the same number of DMA pieces");
     extern __shared__ __align__(16) unsigned char smem[];
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wm = wave / WGN, wn = wave % WGN;
+    const int wk = wave / NT, wm = wave % NT / WGN, wn = wave % WGN;
     long long clk0 = 0, wall0 = 0;
     if (p.clocks) { clk0 = __builtin_amdgcn_s_memtime(); wall0 = __builtin_amdgcn_s_memrealtime(); }
     // Workgroup ids are dealt round-robin to the 8 XCDs.  The tile rows are cut into bands of 8 * RB rows; inside a band
@@ -478,7 +482,7 @@ void bitlinear_mfma_dma3_kernel(MfmaArgs p) {
         tile_n = wg % p.tiles_n;
     }
     const int64_t MB = (p.M + 31) >> 5, NB = (p.N + 31) >> 5;
-    const int KB = (int)(p.Kp >> 7);
+    const int KB = (int)(p.Kp >> 7), KBs = KB / KS;               // k-blocks of the row, steps (the launcher: KB % KS == 0)
     const int64_t KG = p.Kp >> 4;
     static_assert(!SWI || (WN == 2 && FAST), "the swiglu epilogue pairs a gate and an up n-block per wave");
     const int64_t NBs = NB >> 1;                                  // SWI: n-blocks per stacked segment
@@ -500,10 +504,10 @@ void bitlinear_mfma_dma3_kernel(MfmaArgs p) {
 #pragma unroll
         for (int i = 0; i < NDMA; ++i) {
             const int w = i * NW + wave;
-            const int chunk = w >> 2, within = w & 3;             // 4 pieces per m-block
+            const int sub = w / (BMB * 4), chunk = (w >> 2) % BMB, within = w & 3;   // 4 pieces per m-block
             int64_t mb = mb0 + chunk;
             if (mb >= MB) mb = MB - 1;                            // rows past M are never stored: any valid data will do
-            const int kbc = kb < KB ? kb : KB - 1;                // past the end: harmless re-read, never consumed
+            const int kbc = (kb < KBs ? kb : KBs - 1) * KS + sub; // past the end: harmless re-read, never consumed
             const unsigned char* g = reinterpret_cast<const unsigned char*>(p.a) + (mb * KG + kbc * 8 + within * 2) * 512;
             mfma_dma_1k(g, (uint32_t)lane * 16u, smem + boff + w * 1024);
         }
@@ -512,7 +516,7 @@ void bitlinear_mfma_dma3_kernel(MfmaArgs p) {
 #pragma unroll
         for (int j = 0; j < WN; ++j) {
             const int64_t nb = nblock(j);
-            const int kbc = kb < KB ? kb : KB - 1;                // past the end: never consumed
+            const int kbc = (kb < KBs ? kb : KBs - 1) * KS + wk;  // past the end: never consumed
             // wave-uniform block address + a 32-bit lane offset: the load then takes its base from scalar registers and
             // no 64-bit per-lane address is kept alive
             const unsigned char* blk = reinterpret_cast<const unsigned char*>(p.b + (nb * KB + kbc) * 64);
@@ -546,13 +550,13 @@ void bitlinear_mfma_dma3_kernel(MfmaArgs p) {
     v16i acc[WM][WN];
 #pragma unroll
     for (int i = 0; i < WM; ++i) {
-        const int init = FAST ? -sc.qs[i] : 0;
+        const int init = FAST && wk == 0 ? -sc.qs[i] : 0;
 #pragma unroll
         for (int j = 0; j < WN; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = init;
     }
-    const int aoff = (wm * WM) * CH + lane * 16;
+    const int aoff = (wk * BMB + wm * WM) * CH + lane * 16;
     int cur = 0, nxt = BUF, fre = 2 * BUF;         // byte offsets of the buffers of k-blocks s, s+1, s+2
     v4i af[2][WM];
 #pragma unroll
@@ -605,20 +609,66 @@ void bitlinear_mfma_dma3_kernel(MfmaArgs p) {
         const int t = cur; cur = nxt; nxt = fre; fre = t;
     };
     int kb = 0;
-    for (; kb + 3 <= KB; kb += 3) {
+    for (; kb + 3 <= KBs; kb += 3) {
         kblock(kb, bset0, bset1, bset2);
         kblock(kb + 1, bset1, bset2, bset0);
         kblock(kb + 2, bset2, bset0, bset1);
     }
-    if (kb < KB) {
+    if (kb < KBs) {
         kblock(kb, bset0, bset1, bset2);
-        if (kb + 1 < KB) kblock(kb + 1, bset1, bset2, bset0);
+        if (kb + 1 < KBs) kblock(kb + 1, bset1, bset2, bset0);
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);            // the trailing DMA must not land in the epilogue's staging area
     __syncthreads();
-    if constexpr (SWI) mfma_epilogue_swiglu<T, WM>(p, acc, sc, smem, lane, wave, wm, mb0, nb0);
-    else if constexpr (FAST) mfma_epilogue_fast<T, WM, WN>(p, acc, sc, smem, lane, wave, wm, mb0, nb0);
-    else mfma_epilogue<T, WM, WN>(p, acc, sc, smem, lane, wave, wm, mb0, nb0);
+    if constexpr (KS == 1) {
+        if constexpr (SWI) mfma_epilogue_swiglu<T, WM>(p, acc, sc, smem, lane, wave, wm, mb0, nb0);
+        else if constexpr (FAST) mfma_epilogue_fast<T, WM, WN>(p, acc, sc, smem, lane, wave, wm, mb0, nb0);
+        else mfma_epilogue<T, WM, WN>(p, acc, sc, smem, lane, wave, wm, mb0, nb0);
+    } else {
+        // group g finishes row block g of the wave tile: it takes the other groups' partial sums of that block
+        static_assert(KS == WM, "a row block of the wave tile per group");
+        int* const ex = reinterpret_cast<int*>(smem);            // [source wave][KS - 1 blocks][WN][16][64]
+        constexpr int BLK = WN * 16 * 64;
+#pragma unroll
+        for (int i = 0; i < WM; ++i) {
+            if (i != wk) {
+                int* dst = ex + (wave * (KS - 1) + (i > wk ? i - 1 : i)) * BLK + lane;
+#pragma unroll
+                for (int j = 0; j < WN; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) dst[(j * 16 + r) * 64] = acc[i][j][r];
+            }
+        }
+        __syncthreads();
+        v16i mine[1][WN];
+        EpiScales<1, WN> sc1;
+#pragma unroll
+        for (int i = 0; i < WM; ++i) {
+            if (i == wk) {
+                sc1.dq[0] = sc.dq[i];
+                sc1.qs[0] = sc.qs[i];
+#pragma unroll
+                for (int j = 0; j < WN; ++j) mine[0][j] = acc[i][j];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < WN; ++j) sc1.wdq[j] = sc.wdq[j];
+#pragma unroll
+        for (int o = 0; o < KS; ++o) {
+            if (o != wk) {
+                const int* src = ex + ((o * NT + wave % NT) * (KS - 1) + (wk > o ? wk - 1 : wk)) * BLK + lane;
+#pragma unroll
+                for (int j = 0; j < WN; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) mine[0][j][r] += src[(j * 16 + r) * 64];
+            }
+        }
+        __syncthreads();                                         // the exchange area becomes the epilogue's staging area
+        const int wm1 = wm * WM + wk;
+        if constexpr (SWI) mfma_epilogue_swiglu<T, 1>(p, mine, sc1, smem, lane, wave, wm1, mb0, nb0);
+        else if constexpr (FAST) mfma_epilogue_fast<T, 1, WN>(p, mine, sc1, smem, lane, wave, wm1, mb0, nb0);
+        else mfma_epilogue<T, 1, WN>(p, mine, sc1, smem, lane, wave, wm1, mb0, nb0);
+    }
     if (p.clocks && threadIdx.x == 0 && (int64_t)blockIdx.x < p.clock_cap) {
         p.clocks[2 * blockIdx.x] = __builtin_amdgcn_s_memtime() - clk0;
         p.clocks[2 * blockIdx.x + 1] = __builtin_amdgcn_s_memrealtime() - wall0;
@@ -641,50 +691,32 @@ inline int mfma_rows_per_xcd(int tiles_m, int tile_rows, int64_t Kp) {
     return best;
 }
 
-// The 64 x 512 tile on the stacked [gate; up] weight with the swiglu epilogue: a tile is 64 rows x 256 channels.
-template <typename T>
-int launch_mfma_dma3_swiglu(MfmaArgs a, hipStream_t s) {
-    constexpr int WGM = 1, WGN = 8, WM = 2, WN = 2;
-    a.clocks = g_clock_sink; a.clock_cap = g_clock_cap;
-    a.tiles_m = (int)mmf_ceil_div(a.M, WGM * WM * 32);
-    a.tiles_n = (int)mmf_ceil_div(a.N / 2, WGN * 32);
-    a.rows_per_xcd = mfma_rows_per_xcd(a.tiles_m, WGM * WM * 32, a.Kp);
-    size_t lds = 3u * (WGM * WM) * 4096u;
-    const size_t lds_epi = (size_t)(WGM * WGN) * 32u * (32u * sizeof(T) + 16u);
-    if (lds_epi > lds) lds = lds_epi;
-    a.vec_store = 1;
-    auto kern = bitlinear_mfma_dma3_kernel<T, WGM, WGN, WM, WN, true, true>;
-    if (lds > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)lds);
-        if (e != hipSuccess) return (int)e;
-    }
-    kern<<<dim3((unsigned)((int64_t)a.tiles_m * a.tiles_n)), dim3(64 * WGM * WGN), lds, s>>>(a);
-    MMF_CHECK_LAUNCH();
-    return 0;
-}
-
-template <typename T, int WGM, int WGN, int WM, int WN>
+template <typename T, int WGM, int WGN, int WM, int WN, int KS, bool SWI>
 int launch_mfma_dma3(MfmaArgs a, hipStream_t s) {
-    constexpr int BM = WGM * WM * 32, BN = WGN * WN * 32;
+    constexpr int BM = WGM * WM * 32, BN = WGN * WN * 32;        // SWI: BN rows of the stacked weight, BN / 2 channels
     a.clocks = g_clock_sink; a.clock_cap = g_clock_cap;
     a.tiles_m = (int)mmf_ceil_div(a.M, BM);
-    a.tiles_n = (int)mmf_ceil_div(a.N, BN);
+    a.tiles_n = SWI ? (int)mmf_ceil_div(a.N / 2, BN / 2) : (int)mmf_ceil_div(a.N, BN);
     a.rows_per_xcd = mfma_rows_per_xcd(a.tiles_m, BM, a.Kp);
-    size_t lds = 3u * (WGM * WM) * 4096u;
-    const size_t lds_epi = (size_t)(WGM * WGN) * 32u * (WN * 32u * sizeof(T) + 16u);
+    size_t lds = 3u * (WGM * WM) * 4096u * KS;
+    constexpr int waves = WGM * WGN * KS;
+    const size_t lds_epi = (size_t)waves * 32u * ((SWI ? 1 : WN) * 32u * sizeof(T) + 16u);
+    const size_t lds_ex = KS > 1 ? (size_t)waves * (KS - 1) * WN * 4096u : 0;
     if (lds_epi > lds) lds = lds_epi;
+    if (lds_ex > lds) lds = lds_ex;
     const int per_vec = 16 / (int)sizeof(T);
-    a.vec_store = (a.N % per_vec == 0) && (a.ldo % per_vec == 0) && ((reinterpret_cast<uintptr_t>(a.out) & 15u) == 0) &&
-                  ((reinterpret_cast<uintptr_t>(a.addend) & 15u) == 0);
-    const bool fast = a.vec_store && !a.bias;
-    auto kern = fast ? bitlinear_mfma_dma3_kernel<T, WGM, WGN, WM, WN, true> : bitlinear_mfma_dma3_kernel<T, WGM, WGN, WM, WN, false>;
+    a.vec_store = SWI || ((a.N % per_vec == 0) && (a.ldo % per_vec == 0) && ((reinterpret_cast<uintptr_t>(a.out) & 15u) == 0) &&
+                          ((reinterpret_cast<uintptr_t>(a.addend) & 15u) == 0));
+    auto kern = bitlinear_mfma_dma3_kernel<T, WGM, WGN, WM, WN, KS, true, SWI>;
+    if constexpr (!SWI) {
+        if (!a.vec_store || a.bias) kern = bitlinear_mfma_dma3_kernel<T, WGM, WGN, WM, WN, KS, false, false>;
+    }
     if (lds > 48 * 1024) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                            (int)lds);
         if (e != hipSuccess) return (int)e;
     }
-    kern<<<dim3((unsigned)((int64_t)a.tiles_m * a.tiles_n)), dim3(64 * WGM * WGN), lds, s>>>(a);
+    kern<<<dim3((unsigned)((int64_t)a.tiles_m * a.tiles_n)), dim3(64 * waves), lds, s>>>(a);
     MMF_CHECK_LAUNCH();
     return 0;
 }
@@ -854,15 +886,26 @@ int launch_mfma(MfmaArgs a, hipStream_t s) {
     return 0;
 }
 
-// Whether the weight-stream kernel is the faster one.  Measured on MI355X: it costs ~3 us + 0.33 ns per (output block x k-block); a
-// round of tiles of the DMA kernel ~0.9 us per k-block whatever the problem size.
-inline bool mfma_streams(const MfmaArgs& a) {
+// Which kernel is the fastest, from its measured time on MI355X (us, N from 1024 to 11264, K from 1024 to 5632, M from 77 to 8192):
+//   weight stream  3 + 0.7 ns per output block + 0.18 ns per output block and k-block, as long as the row fits its LDS;
+//   split tiles    (64 x 256, two groups of waves on every second k-block) one round of at most one tile per CU: a chain of
+//                  0.29 us per k-block, and what a fuller chip adds.  Beyond one round they only add traffic: 2048 over
+//                  6144 columns at M 777 (312 tiles) 17.0 us against 15.3 -- except where two rounds of whole tiles would leave
+//                  the second one more than half empty: the same columns at M 1377 (528 against 264 tiles) 26.1 against 27.5;
+//   tiles          (64 x 512) 4 + 0.6 us per k-block and round.
+// 2002 x 5632 -> 2048: stream 37 us, split 23, tiles 31; 1377 x 2048 -> 2048: 12.2 / 10.5 / 14.3.
+enum class MfmaPick { kStream, kSplit, kTiles };
+inline MfmaPick mfma_pick(const MfmaArgs& a) {
     const int64_t KB = a.Kp >> 7;
-    const double wgs = (double)mmf_ceil_div(a.M, 32) * (double)mmf_ceil_div(a.N, 32);
-    const double tiles = (double)mmf_ceil_div(a.M, 128) * (double)mmf_ceil_div(a.N, 256);
-    const double t_stream = 3.0 + wgs * (double)KB * 0.00033;
-    const double t_tiled = (double)KB * 0.9 * (double)mmf_ceil_div((int64_t)tiles, 256);
-    return a.Kp <= 8192 && (a.M <= 64 || t_stream < t_tiled);
+    const double kb = (double)KB, blocks = (double)mmf_ceil_div(a.M, 32) * (double)mmf_ceil_div(a.N, 32);
+    const int64_t half = mmf_ceil_div(a.M, 64) * mmf_ceil_div(a.N, 256), full = mmf_ceil_div(a.M, 64) * mmf_ceil_div(a.N, 512);
+    const double t_stream = 3.0 + blocks * (0.0007 + 0.00018 * (double)((KB + 7) / 8 * 8));
+    const double t_tiles = (double)mmf_ceil_div(full, 256) * (4.0 + 0.6 * kb);
+    double t_split = 1e30;
+    if (KB % 2 == 0 && half <= 256) t_split = 4.4 + 0.29 * kb + (double)half / 256.0 * (1.0 + 0.1 * kb);
+    if (KB % 2 == 0 && KB >= 16 && half > 512 && half <= 768) t_split = 0.95 * t_tiles;
+    if (a.Kp <= 8192 && a.M <= 65535 * 32 && (a.M <= 64 || (t_stream <= t_split && t_stream <= t_tiles))) return MfmaPick::kStream;
+    return t_split < t_tiles ? MfmaPick::kSplit : MfmaPick::kTiles;
 }
 
 template <typename T>
@@ -870,16 +913,20 @@ int dispatch_mfma(const MfmaArgs& a, int config, hipStream_t s) {
     // config < 0: pick by shape.
     //   5        weight-stream kernel: one 32x32 output block per workgroup, 8 waves split K (needs Kp <= 8192)
     //   0 / 1    32x256 / 64x256 tiles, A staged through registers (small M with Kp > 8192)
+    //   18       64x256 tiles, two groups of waves on every second k-block (needs an even number of k-blocks)
     //   15 / 16 / 17  256x256 / 128x256 / 64x512 tiles, A staged by DMA (17: every wave reads the whole activation
     //            tile from LDS and owns its own weight columns, so no weight block is fetched twice)
     if (config < 0) {
-        if (mfma_streams(a)) config = 5;
+        const MfmaPick pick = mfma_pick(a);
+        if (pick == MfmaPick::kStream) config = 5;
         else if (a.M <= 32) config = 0;
         else if (a.M <= 64) config = 1;
+        else if (pick == MfmaPick::kSplit) config = 18;
         else config = a.N >= 512 ? 17 : 16;
     }
+    if (config == 18 && (a.Kp >> 7) % 2 != 0) return MMF_ERR_ARG;
     if (config == 5 && (a.Kp > 8192 || a.M > 65535 * 32)) return MMF_ERR_ARG;
-    const int64_t tile_cols = config == 5 ? 32 : config == 16 ? 256 : config == 17 ? 512 : 0;
+    const int64_t tile_cols = config == 5 ? 32 : config == 16 || config == 18 ? 256 : config == 17 ? 512 : 0;
     if (a.a_seg != 0 && a.N > a.seg_rows && (tile_cols == 0 || a.seg_rows % tile_cols != 0)) {
         // tiles that would straddle two segments (or tiles of the kernels that take one set of codes): a launch per segment
         for (int64_t n0 = 0; n0 < a.N; n0 += a.seg_rows) {
@@ -901,9 +948,20 @@ int dispatch_mfma(const MfmaArgs& a, int config, hipStream_t s) {
         case 5: return launch_skinny<T>(a, s);
         case 0: return launch_mfma<T, 1, 8, 1, 1>(a, s);
         case 1: return launch_mfma<T, 1, 8, 2, 1>(a, s);
-        case 15: return launch_mfma_dma3<T, 2, 4, 4, 2>(a, s);
-        case 16: return launch_mfma_dma3<T, 2, 4, 2, 2>(a, s);
-        case 17: return launch_mfma_dma3<T, 1, 8, 2, 2>(a, s);
+        case 15: return launch_mfma_dma3<T, 2, 4, 4, 2, 1, false>(a, s);
+        case 16: return launch_mfma_dma3<T, 2, 4, 2, 2, 1, false>(a, s);
+        case 17: return launch_mfma_dma3<T, 1, 8, 2, 2, 1, false>(a, s);
+        case 18: return launch_mfma_dma3<T, 1, 4, 2, 2, 2, false>(a, s);
+    }
+    return MMF_ERR_ARG;
+}
+
+template <typename T>
+int dispatch_mfma_swiglu(const MfmaArgs& a, hipStream_t s) {
+    switch (mfma_pick(a)) {
+        case MfmaPick::kStream: return launch_skinny_swiglu<T>(a, s);
+        case MfmaPick::kSplit: return launch_mfma_dma3<T, 1, 4, 2, 2, 2, true>(a, s);
+        case MfmaPick::kTiles: return launch_mfma_dma3<T, 1, 8, 2, 2, 1, true>(a, s);
     }
     return MMF_ERR_ARG;
 }
@@ -1021,9 +1079,9 @@ int mmf_bitlinear_mfma_swiglu(const int8_t* codes_tiled, const float* deq, const
     a.a = codes_tiled; a.b = static_cast<const uint4*>(packed); a.deq = deq; a.qsum = qsum; a.wdeq = wdeq;
     a.out = out; a.M = M; a.N = N; a.Kp = mmf_round_up(K, 128); a.seg_rows = seg_rows; a.ldo = ldo;
     switch (out_dtype) {
-        case MMF_F32: return mfma_streams(a) ? launch_skinny_swiglu<float>(a, stream) : launch_mfma_dma3_swiglu<float>(a, stream);
-        case MMF_BF16: return mfma_streams(a) ? launch_skinny_swiglu<bf16_t>(a, stream) : launch_mfma_dma3_swiglu<bf16_t>(a, stream);
-        case MMF_F16: return mfma_streams(a) ? launch_skinny_swiglu<f16_t>(a, stream) : launch_mfma_dma3_swiglu<f16_t>(a, stream);
+        case MMF_F32: return dispatch_mfma_swiglu<float>(a, stream);
+        case MMF_BF16: return dispatch_mfma_swiglu<bf16_t>(a, stream);
+        case MMF_F16: return dispatch_mfma_swiglu<f16_t>(a, stream);
     }
     return MMF_ERR_ARG;
 }

@@ -1,0 +1,47 @@
+"""The tiles whose two groups of waves take alternate k-blocks, at the edges: two k-blocks (one step), a step count off the ring of
+three, ragged rows and columns, the slow epilogue (bias, unaligned rows), an addend, segments, the swiglu form."""
+import pytest
+import torch
+
+from test_gpu_stream_contraction import exact, operands
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 256, 32), (65, 512, 256), (77, 768, 264), (200, 1024, 515), (1377, 2048, 2048), (2002, 5632, 1000)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_split_tiles_are_exact(dev, m, k, n, dtype):
+    F, lib, pw, q, codes, deq, qsum = operands(dev, m, k, n)
+    out = F.bitlinear_mfma(q[0], deq[0], qsum[0], pw, m, dtype, config=18)
+    assert torch.equal(out.cpu(), exact(F, pw, codes[0], deq[0], dtype))
+    bias, add = torch.randn(n, device=dev).to(dtype), torch.randn(m, n, device=dev).to(dtype)
+    for kw in ({"bias": bias}, {"addend": add}):
+        assert torch.equal(F.bitlinear_mfma(q[0], deq[0], qsum[0], pw, m, dtype, config=18, **kw),
+                           F.bitlinear_mfma(q[0], deq[0], qsum[0], pw, m, dtype, config=16, **kw)), tuple(kw)
+
+
+def test_odd_number_of_k_blocks_is_refused(dev):
+    F, lib, pw, q, codes, deq, qsum = operands(dev, 70, 384, 256)
+    with pytest.raises(RuntimeError):
+        F.bitlinear_mfma(q[0], deq[0], qsum[0], pw, 70, torch.bfloat16, config=18)
+
+
+@pytest.mark.parametrize("m,k,inter", [(300, 2048, 1056), (333, 1024, 2816), (385, 1024, 2816), (66, 8448, 96)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_swiglu_equals_contraction_then_swiglu(dev, m, k, inter, dtype):
+    F, lib, pw, q, codes, deq, qsum = operands(dev, m, k, 2 * inter, seed=2)
+    y = F.bitlinear_mfma(q[0], deq[0], qsum[0], pw, m, dtype)
+    assert torch.equal(F.bitlinear_mfma_swiglu(q[0], deq[0], qsum[0], pw, m, dtype), F.swiglu(y[:, :inter], y[:, inter:]))
+
+
+@pytest.mark.parametrize("seg", [512, 160])
+def test_segments_contract_their_own_codes(dev, seg):
+    m, k = 300, 512
+    F, lib, pw, q, codes, deq, qsum = operands(dev, m, k, 3 * seg, sets=3, seed=3)
+    pw.wdeq, pw.seg_rows = pw.wdeq.repeat(3) * torch.tensor([1.0, 2.0, 0.5], device=dev), seg
+    out = torch.empty(m, 3 * seg, dtype=torch.bfloat16, device=dev)
+    F.L.check(lib.mmf_bitlinear_mfma_multi(q.data_ptr(), q.stride(0), deq.data_ptr(), qsum.data_ptr(), pw.packed.data_ptr(),
+                                           pw.wdeq.data_ptr(), seg, out.data_ptr(), 3 * seg, m, k, 3 * seg, 1, 18, F.L.stream()), "multi")
+    for s in range(3):
+        alone = F.bitlinear_mfma(q[s], deq[s], qsum[s], pw, m, torch.bfloat16, config=5)
+        assert torch.equal(out[:, s * seg:(s + 1) * seg], alone[:, s * seg:(s + 1) * seg]), s
