@@ -17,7 +17,6 @@
 namespace {
 
 enum Chain : int { CHAIN_NORM = 0, CHAIN_GATED = 1, CHAIN_SWIGLU = 2 };
-constexpr int kT = 512, kW = kT / 64;
 
 struct ChainArgs {
     const void* x; const void* aux;     // the op's inputs, row strides ldx, ldaux
@@ -36,9 +35,15 @@ struct ChainArgs {
 
 // One row per workgroup and turn, 4 elements per thread and pass, the next row's loads in flight under this row's arithmetic;
 // four exchanges of per-wave partials a row, each with slots of its own and one barrier.
-template <typename T, typename TW, int NV, int ST, int NN>
-__global__ __launch_bounds__(kT) void chain_bwd_kernel(ChainArgs a) {
+// The vector units are the bound next to HBM: a wave spends ~300 instructions a row whatever it carries (addresses, exchanges, the
+// roots) on top of ~45 to 100 an element, so rows go to few waves with 8 elements a thread, as long as the registers still leave
+// two rows on a CU.  8192 rows of 2048 in bf16: 4 waves with 8 elements 45 us (norm) and 57 us (gated) where 8 waves with 4 took
+// 52 and 70; three norms keep 8 waves (194 registers otherwise).  5632 wide (swiglu): 12 waves with 8, 153 us; 8 waves with 12,
+// one to two on a SIMD, 159 us.
+template <typename T, typename TW, int KT, int NV, int ST, int NN>
+__global__ __launch_bounds__(KT) void chain_bwd_kernel(ChainArgs a) {
     constexpr bool W1 = ST != CHAIN_SWIGLU, AUX = ST != CHAIN_NORM, RES = ST == CHAIN_NORM;
+    constexpr int kW = KT / 64;
     __shared__ double s_sum1[kW], s_sum2[kW];
     __shared__ float s_max[NN][kW], s_dot2[kW], s_dot1[kW];
     const int K = a.K, lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -46,7 +51,7 @@ __global__ __launch_bounds__(kT) void chain_bwd_kernel(ChainArgs a) {
     Raw4<TW> w1r[W1 ? NV : 1], w2r[NN][NV];
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-        const int k0 = (v * kT + (int)threadIdx.x) * 4;
+        const int k0 = (v * KT + (int)threadIdx.x) * 4;
         if constexpr (W1) w1r[v] = raw4_load<TW, true>(static_cast<const TW*>(a.w1), k0, K);
 #pragma unroll
         for (int n = 0; n < NN; ++n) w2r[n][v] = raw4_load<TW, true>(static_cast<const TW*>(a.w2[n]), k0, K);
@@ -61,7 +66,7 @@ __global__ __launch_bounds__(kT) void chain_bwd_kernel(ChainArgs a) {
     auto load = [&](int64_t row) __attribute__((always_inline)) {
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-            const int k0 = (v * kT + (int)threadIdx.x) * 4;
+            const int k0 = (v * KT + (int)threadIdx.x) * 4;
             xr[v] = raw4_load<T, true>(static_cast<const T*>(a.x) + row * a.ldx, k0, K);
             if constexpr (AUX) ar[v] = raw4_load<T, true>(static_cast<const T*>(a.aux) + row * a.ldaux, k0, K);
 #pragma unroll
@@ -84,7 +89,7 @@ __global__ __launch_bounds__(kT) void chain_bwd_kernel(ChainArgs a) {
         for (int w = 1; w < kW; ++w) t += s[w];
         return t;
     };
-    auto in_row = [&](int v) __attribute__((always_inline)) { return (v * kT + (int)threadIdx.x) * 4 < K; };   // K is a multiple of 4
+    auto in_row = [&](int v) __attribute__((always_inline)) { return (v * KT + (int)threadIdx.x) * 4 < K; };   // K is a multiple of 4
 
     load((int64_t)blockIdx.x < a.M ? blockIdx.x : 0);
     for (int64_t row = blockIdx.x; row < a.M; row += gridDim.x) {
@@ -186,7 +191,7 @@ __global__ __launch_bounds__(kT) void chain_bwd_kernel(ChainArgs a) {
         float dot1 = 0.0f;
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-            const int k0 = (v * kT + (int)threadIdx.x) * 4;
+            const int k0 = (v * KT + (int)threadIdx.x) * 4;
 #pragma unroll
             for (int n = 0; n < NN; ++n) {
                 float w2[4], o[4];
@@ -230,7 +235,7 @@ __global__ __launch_bounds__(kT) void chain_bwd_kernel(ChainArgs a) {
                 float o[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) o[i] = (wd[v][i] - x[v][i] * c1) * rstd1 + (RES ? res[v][i] : 0.0f);
-                raw4_store<T, true>(static_cast<T*>(a.dx) + row * a.lddx, (v * kT + (int)threadIdx.x) * 4, K, o);
+                raw4_store<T, true>(static_cast<T*>(a.dx) + row * a.lddx, (v * KT + (int)threadIdx.x) * 4, K, o);
             }
         } else {
             __syncthreads();                                     // the slots are free for the next row
@@ -238,7 +243,7 @@ __global__ __launch_bounds__(kT) void chain_bwd_kernel(ChainArgs a) {
     }
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-        const int k0 = (v * kT + (int)threadIdx.x) * 4;
+        const int k0 = (v * KT + (int)threadIdx.x) * 4;
         float* p = a.part + (int64_t)blockIdx.x * ((W1 ? 1 : 0) + NN) * K;
         if constexpr (W1) raw4_store<float, true>(p, k0, K, acc1[v]);
 #pragma unroll
@@ -277,13 +282,15 @@ __global__ __launch_bounds__(kCols * kLanes) void colsum_rows_kernel(const float
 
 template <typename T, typename TW, int ST, int NN>
 int launch_chain(const ChainArgs& a, int groups, void* dw, hipStream_t s) {
-    const int nv = (int)mmf_ceil_div(a.K, kT * 4);
-    if (nv <= 1) chain_bwd_kernel<T, TW, 1, ST, NN><<<groups, kT, 0, s>>>(a);
-    else if (nv <= 2) chain_bwd_kernel<T, TW, 2, ST, NN><<<groups, kT, 0, s>>>(a);
+    if (a.K <= 1024) chain_bwd_kernel<T, TW, 256, 1, ST, NN><<<groups, 256, 0, s>>>(a);
+    else if (a.K <= 2048) {
+        if constexpr (NN == 1) chain_bwd_kernel<T, TW, 256, 2, ST, NN><<<groups, 256, 0, s>>>(a);
+        else chain_bwd_kernel<T, TW, 512, 1, ST, NN><<<groups, 512, 0, s>>>(a);
+    }
+    else if (a.K <= 4096) chain_bwd_kernel<T, TW, 512, 2, ST, NN><<<groups, 512, 0, s>>>(a);
     else if constexpr (NN == 1) {                                // (three norms: a wider row would not fit the registers)
-        if (nv <= 3) chain_bwd_kernel<T, TW, 3, ST, NN><<<groups, kT, 0, s>>>(a);
-        else if (nv <= 4) chain_bwd_kernel<T, TW, 4, ST, NN><<<groups, kT, 0, s>>>(a);
-        else return MMF_ERR_WIDE;
+        if (a.K <= 6144) chain_bwd_kernel<T, TW, 768, 2, ST, NN><<<groups, 768, 0, s>>>(a);
+        else chain_bwd_kernel<T, TW, 512, 4, ST, NN><<<groups, 512, 0, s>>>(a);
     } else return MMF_ERR_WIDE;
     MMF_CHECK_LAUNCH();
     const int cols = ((ST != CHAIN_SWIGLU ? 1 : 0) + NN) * a.K;
@@ -302,30 +309,37 @@ int dispatch_chain(const ChainArgs& a, int kind, int n, int groups, void* dw, hi
 }
 
 // ------------------------------------------------------------------------------------------ weights
-// One thread per 16 inputs of a row: its dword of codes becomes 32 (64) bytes of the row, so consecutive threads write a row of
-// the block's 128 inputs side by side.  Bound by the write, 2 (4) bytes a weight.
+// Bound by the write, 2 (4) bytes a weight.  A thread owns one 16-byte vector of kUdRows consecutive rows, so a wave's store is 1 KiB
+// of one row and the rows of a workgroup use up the lines of the packed blocks (a row's codes of 128 inputs are two 16-byte pieces
+// 512 bytes apart, the next row's follow each).  The 32000 x 2048 head in bf16: one thread per dword of codes, 64-byte strides
+// between the lanes' stores and a 64-bit division took 44 us.
+constexpr int kUdRows = 8;
 template <typename T>
 __global__ __launch_bounds__(256) void unpack_dequant_kernel(const uint32_t* __restrict__ packed, const float* __restrict__ wdeq,
-                                                             int64_t seg_rows, int64_t N, int64_t K, int64_t KB, T* __restrict__ out) {
-    const int64_t groups = mmf_ceil_div(K, 16);
-    const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (gid >= N * groups) return;
-    const int64_t n = gid / groups, kg = gid % groups;
-    const int64_t k0 = kg * 16, nb = n >> 5, kb = k0 >> 7;
-    const int s = (int)((k0 >> 5) & 3), half = (int)((k0 >> 4) & 1), lane = half * 32 + (int)(n & 31);
-    const uint32_t v = packed[((nb * KB + kb) * 64 + lane) * 4 + s];
-    const float wd = wdeq[n / seg_rows];
-    T* row = out + n * K + k0;
-    const bool whole = K % 8 == 0 && k0 + 16 <= K;
+                                                             uint32_t seg_rows, int N, int K, int KB, bool whole, T* __restrict__ out) {
+    constexpr int VE = 16 / (int)sizeof(T);
+    const int k0 = ((int)blockIdx.y * 256 + (int)threadIdx.x) * VE;
+    if (k0 >= K) return;
+    const int n0 = (int)blockIdx.x * kUdRows, part = (k0 & 15) >> 2;     // VE is 4 or 8: one or two groups of 4 codes
+    const uint32_t* src = packed + ((((int64_t)(n0 >> 5) * KB + (k0 >> 7)) * 64 + ((k0 >> 4) & 1) * 32 + (n0 & 31)) * 4 + ((k0 >> 5) & 3));
+    uint32_t code[kUdRows];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        float e[8];
+    for (int r = 0; r < kUdRows; ++r) code[r] = src[r * 4];              // (rows are padded to 32 there)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int i = h * 8 + j;
-            e[j] = (float)((int)((v >> (8 * (i & 3) + 2 * (i >> 2))) & 3u) - 1) * wd;
+    for (int r = 0; r < kUdRows; ++r) {
+        if (n0 + r >= N) break;
+        const float wd = wdeq[(uint32_t)(n0 + r) / seg_rows];
+        float e[VE];
+#pragma unroll
+        for (int j = 0; j < VE; ++j) e[j] = (float)((int)((code[r] >> (8 * (j & 3) + 2 * (part + (j >> 2)))) & 3u) - 1) * wd;
+        T* row = out + (int64_t)(n0 + r) * K + k0;
+        if (whole) {
+            if constexpr (VE == 8) mmf_store8<T>(row, 0, VE, true, e);
+            else *reinterpret_cast<float4*>(row) = make_float4(e[0], e[1], e[2], e[3]);
+        } else {
+            for (int j = 0; j < VE; ++j)
+                if (k0 + j < K) row[j] = mmf_from_float<T>(e[j]);
         }
-        mmf_store8<T>(row, h * 8, K - k0, whole, e);
     }
 }
 
@@ -345,7 +359,7 @@ int mmf_chain_bwd(int kind, const void* x, int64_t ldx, const void* aux, int64_t
     if (!(norms == 1 || (norms == 3 && kind == CHAIN_NORM)) || !x || !w2 || !dy || !dx || !y || !part || !dweights) return MMF_ERR_ARG;
     if (kind != CHAIN_SWIGLU && !w1) return MMF_ERR_ARG;
     if (kind != CHAIN_NORM && (!aux || !daux || ldaux < K || lddaux < K || dres)) return MMF_ERR_ARG;
-    if (K % 4 != 0 || K > kT * 4 * 4) return MMF_ERR_WIDE;
+    if (K % 4 != 0 || K > 8192) return MMF_ERR_WIDE;
     ChainArgs a{};
     a.x = x; a.aux = aux; a.w1 = w1; a.dres = dres; a.dx = dx; a.daux = daux; a.y = y; a.part = part;
     for (int n = 0; n < norms; ++n) {
@@ -382,10 +396,12 @@ int mmf_unpack_dequant(const void* packed, const float* wdeq, int64_t seg_rows, 
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     if (N <= 0 || K <= 0 || seg_rows <= 0 || !packed || !wdeq || !out) return MMF_ERR_ARG;
     if (K % 8 == 0 && (reinterpret_cast<uintptr_t>(out) & 15u)) return MMF_ERR_ALIGN;
-    const int64_t KB = mmf_ceil_div(K, 128), blocks = mmf_ceil_div(N * mmf_ceil_div(K, 16), 256);
-    if (blocks > 0x7fffffff) return MMF_ERR_WIDE;
-#define MMF_UD(T) unpack_dequant_kernel<T><<<(unsigned)blocks, 256, 0, stream>>>(static_cast<const uint32_t*>(packed), wdeq, seg_rows, N, K, \
-                                                                                KB, static_cast<T*>(out))
+    if (N > 0x7fffffff || K > 0x7fffffff || seg_rows > 0x7fffffff) return MMF_ERR_WIDE;
+    const int64_t KB = mmf_ceil_div(K, 128), columns = mmf_ceil_div(K, 256 * (dtype == MMF_F32 ? 4 : 8));
+    if (columns > 65535) return MMF_ERR_WIDE;
+    const bool whole = K % (dtype == MMF_F32 ? 4 : 8) == 0 && (reinterpret_cast<uintptr_t>(out) & 15u) == 0;
+#define MMF_UD(T) unpack_dequant_kernel<T><<<dim3((unsigned)mmf_ceil_div(N, kUdRows), (unsigned)columns), 256, 0, stream>>>( \
+        static_cast<const uint32_t*>(packed), wdeq, (uint32_t)seg_rows, (int)N, (int)K, (int)KB, whole, static_cast<T*>(out))
     switch (dtype) {
         case MMF_F32: MMF_UD(float); break;
         case MMF_BF16: MMF_UD(bf16_t); break;

@@ -1,0 +1,35 @@
+"""The ternary weights as a dense matrix, at the edges of the vectors, the row groups, the packed blocks and the segments."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,k,seg", [(1, 4, 1), (7, 100, 7), (33, 131, 33), (96, 1024, 32), (40, 2056, 20), (64, 4100, 64)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_dense_weights_equal_unpacked_codes_times_scale(dev, n, k, seg, dtype):
+    import matmulfreellm_amd.functional as F
+    from matmulfreellm_amd.autograd import _dequantised
+    torch.manual_seed(n + k)
+    pw = F.ternarize_pack(torch.randn(n, k, device=dev))
+    codes = F.unpack_ternary(pw).float()
+    pw.wdeq, pw.seg_rows = torch.rand(-(-n // seg), device=dev) + 0.5, seg
+    scale = pw.wdeq.repeat_interleave(seg)[:n].view(n, 1)
+    assert torch.equal(_dequantised(pw, dtype), (codes * scale).to(dtype))
+
+
+@pytest.mark.parametrize("rows,k,norms", [(3, 1024, 1), (5, 1028, 3), (2, 2048, 3), (1100, 260, 1), (3, 4096, 3), (3, 4100, 1), (2, 6148, 1), (2, 8192, 1)])
+def test_chained_norm_backward_equals_autograd(dev, rows, k, norms):
+    """norm behind norm against torch autograd of the same ops in fp64 (straight through the quantiser), for each split of a row."""
+    from matmulfreellm_amd.autograd import CHAIN_NORM, _chain_bwd
+    torch.manual_seed(k)
+    x, dres = torch.randn(rows, k, device=dev), torch.randn(rows, k, device=dev)
+    w1, w2 = torch.rand(k, device=dev) + 0.5, [torch.rand(k, device=dev) + 0.5 for _ in range(norms)]
+    dy = [torch.randn(rows, k, device=dev) for _ in range(norms)]
+    dx, _, _, dw = _chain_bwd(CHAIN_NORM, x, None, w1, 1e-6, w2, 1e-6, dy, dres=dres)
+    leaf = [t.double().requires_grad_() for t in (x, w1, *w2)]
+    norm = lambda v, w: v * torch.rsqrt(v.square().mean(-1, keepdim=True) + 1e-6) * w
+    s = norm(leaf[0], leaf[1])
+    ref = torch.autograd.grad([norm(s, w) for w in leaf[2:]], leaf, [d.double() for d in dy])
+    for got, want in zip((dx - dres, *dw), ref):
+        assert (got.double() - want).norm() <= 2e-6 * want.norm()
