@@ -4,12 +4,15 @@ There is no CPU implementation behind these calls: if the shared library is miss
 first use raises, it never falls back to another code path.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libmmf_hip.so")
+NATIVE_PATH = os.path.join(_HERE, "lib", "mmf_torch.so")
 
 MMF_F32, MMF_BF16, MMF_F16 = 0, 1, 2
 _DTYPE_IDS = {torch.float32: MMF_F32, torch.bfloat16: MMF_BF16, torch.float16: MMF_F16}
@@ -97,6 +100,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_native = None
 
 
 class MMFError(RuntimeError):
@@ -116,6 +120,18 @@ def load():
             fn.restype, fn.argtypes = res, args
         _lib = lib
     return _lib
+
+
+def native():
+    """The calls that take tensors themselves (csrc/torch_ops.cpp); loaded once, raises if it has not been built."""
+    global _native
+    if _native is None:
+        load()
+        if not os.path.exists(NATIVE_PATH):
+            raise MMFError(f"{NATIVE_PATH} is missing: build it with `python -m matmulfreellm_amd.build` (there is no fallback path)")
+        loader = importlib.machinery.ExtensionFileLoader("mmf_torch", NATIVE_PATH)
+        _native = importlib.util.module_from_spec(importlib.util.spec_from_loader("mmf_torch", loader))
+    return _native
 
 
 def check(rc, what):

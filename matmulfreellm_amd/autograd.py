@@ -5,8 +5,6 @@ Each Function mirrors one of the reference's autograd Functions:
   RMSNormFn                LayerNormFn (RMS form)        mmfreelm/modules/layernorm.py:445-531
   RMSNormSwishGateFn       LayerNormFn (gated)           mmfreelm/modules/fused_norm_gate.py:420-500
   SwiGLUFn                 SwiGLUFunction                mmfreelm/modules/activations.py:143-175
-  FusedRecurrentHGRNFn     FusedRecurrentHGRNFunction    mmfreelm/ops/hgrn/recurrent_fuse.py:136-173
-  ChunkHGRNFn              ChunkHGRNFunction             mmfreelm/ops/hgrn/chunk.py:223-284
   BlockFn, NormHeadFn      a whole block / final norm + head of mmfreelm/models/hgrn_bit/modeling_hgrn_bit.py:97-111, 262, 386
   HGRNGateFn               the elementwise ops of mmfreelm/layers/hgrn_bit.py:113-120, differentiated as one op
   CrossEntropyFn           CrossEntropyLossFunction      mmfreelm/modules/fused_cross_entropy.py:163-310
@@ -14,7 +12,8 @@ Each Function mirrors one of the reference's autograd Functions:
 The forward values are those of the inference kernels (same launches); the backward kernels live in csrc/backward.hip.
 The two dense products of a BitLinear's backward (dout @ W_q and dout^T @ y_q, fusedbitnet.py:474, :498) are plain
 library GEMMs (torch.matmul).  Modules pick these Functions when gradients are enabled and an input or parameter
-requires one (`needs_grad`); otherwise they keep the fused inference launches.
+requires one (`needs_grad`); otherwise they keep the fused inference launches.  The scans differentiate in native code
+(csrc/torch_ops.cpp).
 """
 import ctypes
 
@@ -221,40 +220,6 @@ def _scan_bwd(g, o, do, h0, log_gates):
                                                  dg.data_ptr(), b * h, t, d, 1 if log_gates else 0, L.dtype_id(g.dtype),
                                                  L.ptr(ws), L.stream()), "mmf_hgrn_recurrent_bwd_split")
     return dx, dg
-
-
-class FusedRecurrentHGRNFn(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, g, initial_state, output_final_state):
-        with torch.no_grad():
-            o, ht = F_.hgrn_recurrent(x, g, initial_state, output_final_state)
-        ctx.save_for_backward(g, o, initial_state)
-        if ht is not None:
-            ctx.mark_non_differentiable(ht)
-        return o, ht
-
-    @staticmethod
-    def backward(ctx, do, dht=None):
-        g, o, h0 = ctx.saved_tensors
-        dx, dg = _scan_bwd(g, o, do, h0, False)
-        return dx, dg, None, None
-
-
-class ChunkHGRNFn(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, g, initial_state, output_final_state, chunk_size):
-        with torch.no_grad():
-            o, ht = F_.hgrn_chunk(x, g, initial_state, output_final_state, chunk_size)
-        ctx.save_for_backward(g, o, initial_state)
-        if ht is not None:
-            ctx.mark_non_differentiable(ht)
-        return o, ht
-
-    @staticmethod
-    def backward(ctx, do, dht=None):
-        g, o, h0 = ctx.saved_tensors
-        dx, dg = _scan_bwd(g, o, do, h0, True)
-        return dx, dg, None, None, None
 
 
 CHAIN_NORM, CHAIN_GATED, CHAIN_SWIGLU = 0, 1, 2

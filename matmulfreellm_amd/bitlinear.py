@@ -7,7 +7,9 @@ reference re-quantises it on every forward, fusedbitnet.py:456).
 import torch
 import torch.nn as nn
 
+from . import _lib as L
 from . import functional as F_
+from .autograd import BitLinearFn, needs_grad
 from .layernorm import RMSNorm
 
 
@@ -38,7 +40,7 @@ class _PackCache:
             if not weight.is_meta:
                 raise RuntimeError("this BitLinear holds packed codes only; assigning a latent weight to it is not supported")
             return self.pw
-        key = (weight.data_ptr(), weight._version, weight.dtype, weight.device, tuple(weight.shape))
+        key = (weight.data_ptr(), weight._version, weight.dtype, weight.device, weight.shape)
         if key != self.key:
             self.pw = F_.ternarize_pack(weight)
             self.key = key
@@ -53,7 +55,6 @@ def layer_norm_linear_quant_fn(x, norm_weight, norm_bias, linear_weight, linear_
     MatMul-free LM never takes it (FusedBitLinear passes is_rms_norm=True, fusedbitnet.py:602-610).  A norm bias on the
     RMSNorm form raises.  ``packed`` (a functional.PackedWeight) skips the ternarise+pack pass.
     """
-    from .autograd import BitLinearFn, needs_grad
     if not is_rms_norm:
         if needs_grad(x, norm_weight, norm_bias, linear_weight, linear_bias, residual):
             raise NotImplementedError("the LayerNorm form of layer_norm_linear_quant_fn has no backward here "
@@ -96,9 +97,23 @@ class BitLinear(nn.Linear):
         return F_.bitlinear(x, self.norm.weight, self.packed_weight(), bias=self.bias, eps=self.run_eps(), addend=addend,
                             prologue=prologue, epilogue=epilogue)
 
+    def _few_rows(self, x, eps):
+        """forward() without gradients on a few rows, past everything that is the same on each call; None if it is not that."""
+        own, norm = self._parameters, self.norm._parameters
+        weight, norm_weight = own.get("weight"), norm.get("weight")
+        if weight is None or norm_weight is None or own.get("bias") is not None or norm.get("bias") is not None:
+            return None
+        pw = self._pack.get(weight)
+        return L.native().bitlinear_few_rows(x, norm_weight, pw.packed, pw.wdeq, pw.seg_rows, pw.n, pw.k, eps, F_.GEMV_MAX_M)
+
     def forward(self, x):
-        return layer_norm_linear_quant_fn(x, self.norm.weight, self.norm.bias, self.weight, self.bias,
-                                          eps=self.norm.eps, is_rms_norm=True, packed=self.packed_weight())
+        eps = self.run_eps()
+        if not torch.is_grad_enabled():
+            out = self._few_rows(x, eps)
+            if out is not None:
+                return out
+        return layer_norm_linear_quant_fn(x, self.norm.weight, self.norm.bias, self.weight, self.bias, eps=eps,
+                                          is_rms_norm=True, packed=self.packed_weight())
 
 
 class FusedBitLinear(BitLinear):
@@ -113,8 +128,3 @@ class FusedBitLinear(BitLinear):
     def __init__(self, in_features, out_features, bias=False, fused_eps=1e-6):
         super().__init__(in_features, out_features, bias=bias)
         self.fused_eps = fused_eps
-
-    def forward(self, x):
-        eps = self.norm.eps if self.fused_eps is None else self.fused_eps
-        return layer_norm_linear_quant_fn(x, self.norm.weight, self.norm.bias, self.weight, self.bias, eps=eps,
-                                          is_rms_norm=True, packed=self.packed_weight())

@@ -1,16 +1,18 @@
-"""Compile the HIP sources in csrc/ into lib/libmmf_hip.so for gfx950.
+"""Compile the HIP sources in csrc/ into lib/libmmf_hip.so for gfx950, and csrc/torch_ops.cpp into lib/mmf_torch.so.
 
 Run as ``python -m matmulfreellm_amd.build``.  hipcc cross-compiles without a GPU.
 """
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 LIBPATH = os.path.join(LIBDIR, "libmmf_hip.so")
+NATIVE_PATH = os.path.join(LIBDIR, "mmf_torch.so")
 SOURCES = ["norm.hip", "quant_pack.hip", "bitlinear_gemv.hip", "bitlinear_mfma.hip", "hgrn.hip", "misc.hip", "decode_layers.hip", "sampling.hip", "loss.hip", "backward.hip", "hgrn_block.hip", "block_forward.hip", "backward_block.hip", "conv.hip"]
 
 # -ffp-contract=off: no multiply-add fusion, so results match a CPU restatement bit for bit.
@@ -47,8 +49,28 @@ def _compile(src, objdir, verbose):
     return obj
 
 
+def build_native(verbose=False):
+    """The calls that take torch tensors: host code over torch's C++ interface and libmmf_hip.so."""
+    import torch
+    root = os.path.dirname(torch.__file__)
+    inc = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"), "/opt/rocm/include",
+           sysconfig.get_paths()["include"]]
+    tmp = NATIVE_PATH + ".tmp"
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-isystem{d}" for d in inc),
+           os.path.join(CSRC, "torch_ops.cpp"), "-o", tmp, "-L", LIBDIR, "-l:" + os.path.basename(LIBPATH), "-L", os.path.join(root, "lib"),
+           "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed on torch_ops.cpp:\n{r.stdout}\n{r.stderr}")
+    os.replace(tmp, NATIVE_PATH)
+    return NATIVE_PATH
+
+
 def build(verbose=False, jobs=None):
-    """Compile every source and link the shared library; returns its path."""
+    """Compile every source and link the shared libraries; returns the HIP library's path."""
     objdir = os.path.join(HERE, "build")
     os.makedirs(objdir, exist_ok=True)
     os.makedirs(LIBDIR, exist_ok=True)
@@ -63,6 +85,7 @@ def build(verbose=False, jobs=None):
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
     os.replace(tmp, LIBPATH)
+    build_native(verbose)
     return LIBPATH
 
 

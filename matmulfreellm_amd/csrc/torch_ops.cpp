@@ -1,0 +1,166 @@
+// Calls on single tensors, where the host is what a user waits for: no Python between the tensor and the launch, and for the scans
+// none in the backward pass either, which autograd runs on a thread of its own (a Python backward waits there for the interpreter
+// lock of the thread that called it).  Measured with kernels of 4.5 and 30 us of device time behind them, per call:
+//   FusedBitLinear 1 x 2048 -> 2048          19.7 us through Python and ctypes, 7.7 here (the launch alone: 3)
+//   fused_recurrent_hgrn, forward + backward  172 us through Python Functions, 71 here
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "../../include/mmf.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+int dtype_of(at::ScalarType t) {
+    return t == at::kFloat ? MMF_F32 : t == at::kBFloat16 ? MMF_BF16 : t == at::kHalf ? MMF_F16 : -1;
+}
+void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
+// the launches go to the current device: this makes it the tensors' for the time of a call
+struct OnDevice {
+    int back = -1;
+    explicit OnDevice(int dev) {
+        const int now = c10::hip::current_device();
+        if (now != dev) { back = now; c10::hip::set_device((c10::DeviceIndex)dev); }
+    }
+    ~OnDevice() { if (back >= 0) c10::hip::set_device((c10::DeviceIndex)back); }
+};
+struct Failed { int rc; const char* what; };
+void check(int rc, const char* what) { if (rc != 0) throw Failed{rc, what}; }
+
+struct NoGil {
+    PyThreadState* state = PyEval_SaveThread();
+    ~NoGil() { PyEval_RestoreThread(state); }
+};
+
+// ------------------------------------------------------------------------------ BitLinear, a few rows
+// (x, norm_weight, packed, wdeq, seg_rows, n, k, eps, most_rows) -> [..., n], or None where an operand is not laid out for the launch or
+// the launch refuses it (the general path then says why)
+PyObject* few_rows(PyObject*, PyObject* const* args, Py_ssize_t count) {
+    HANDLE_TH_ERRORS
+    if (count != 9) { PyErr_SetString(PyExc_TypeError, "bitlinear_few_rows takes 9 arguments"); return nullptr; }
+    for (int i = 0; i < 4; ++i)
+        if (!THPVariable_Check(args[i])) Py_RETURN_NONE;
+    const Tensor &x = THPVariable_Unpack(args[0]), &w = THPVariable_Unpack(args[1]), &packed = THPVariable_Unpack(args[2]),
+                 &wdeq = THPVariable_Unpack(args[3]);
+    const int64_t seg_rows = PyLong_AsLongLong(args[4]), n = PyLong_AsLongLong(args[5]), k = PyLong_AsLongLong(args[6]);
+    const double eps = PyFloat_AsDouble(args[7]);
+    const int64_t most = PyLong_AsLongLong(args[8]);
+    if (PyErr_Occurred()) return nullptr;
+    const int dt = dtype_of(x.scalar_type()), wdt = dtype_of(w.scalar_type());
+    const int64_t total = x.numel();
+    if (dt < 0 || wdt < 0 || x.dim() < 1 || x.size(-1) != k || total == 0 || total > most * k || !x.is_cuda() || !x.is_contiguous() ||
+        !w.is_contiguous() || w.numel() != k || w.device() != x.device() || packed.device() != x.device() || k > mmf_bitlinear_gemv_max_k())
+        Py_RETURN_NONE;
+    Tensor out;
+    int rc;
+    {
+        NoGil nogil;
+        OnDevice on(x.get_device());
+        c10::SmallVector<int64_t, 6> shape(x.sizes().begin(), x.sizes().end());
+        shape.back() = n;
+        out = at::empty(shape, x.options().requires_grad(false));
+        rc = mmf_bitlinear_gemv(x.data_ptr(), w.data_ptr(), packed.data_ptr(), static_cast<const float*>(wdeq.data_ptr()), seg_rows, nullptr,
+                                 nullptr, out.data_ptr(), total / k, k, n, (float)eps, dt, wdt, stream_of(x));
+    }
+    if (rc != 0) Py_RETURN_NONE;
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// ------------------------------------------------------------------------------ scans, differentiable
+float* floats(const Tensor& t) { return t.defined() ? static_cast<float*>(t.data_ptr()) : nullptr; }
+
+// mmfreelm/ops/hgrn/recurrent_fuse.py:136-173 (chunk 0) and chunk.py:223-284
+struct ScanFn : torch::autograd::Function<ScanFn> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& g, const std::optional<Tensor>& h0, bool final_state, int64_t chunk) {
+        OnDevice on(x.get_device());
+        const int64_t b = x.size(0), h = x.size(1), t = x.size(2), d = x.size(3);
+        const int dt = dtype_of(x.scalar_type());
+        const Tensor xc = x.contiguous(), gc = g.contiguous(), state = h0 ? h0->reshape({b * h, d}).to(at::kFloat).contiguous() : Tensor();
+        const auto f32 = x.options().dtype(at::kFloat);
+        Tensor o = at::empty(xc.sizes(), xc.options()), last, ws;
+        if (final_state) last = at::empty({b, h, d}, f32);
+        if (chunk > 0) {
+            if (const int64_t bytes = mmf_hgrn_chunk_workspace_bytes(b * h, t, d, (int)chunk)) ws = at::empty({bytes / 4}, f32);
+            check(mmf_hgrn_chunk(xc.data_ptr(), gc.data_ptr(), floats(state), o.data_ptr(), floats(last), b * h, t, d, (int)chunk, dt, floats(ws),
+                                 stream_of(x)), "mmf_hgrn_chunk");
+        } else {
+            check(mmf_hgrn_recurrent(xc.data_ptr(), gc.data_ptr(), floats(state), o.data_ptr(), floats(last), b * h, t, d, dt, stream_of(x)),
+                  "mmf_hgrn_recurrent");
+        }
+        ctx->save_for_backward({gc, o, state});
+        ctx->saved_data["log_gates"] = chunk > 0;
+        ctx->set_materialize_grads(false);
+        if (!final_state) return {o};
+        ctx->mark_non_differentiable({last});
+        return {o, last};
+    }
+
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        if (!grads[0].defined()) return variable_list(5);
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &g = saved[0], &o = saved[1], &state = saved[2];
+        OnDevice on(g.get_device());
+        const int64_t bh = g.size(0) * g.size(1), t = g.size(2), d = g.size(3);
+        const Tensor dout = grads[0].to(g.scalar_type()).contiguous();
+        Tensor dx = at::empty(g.sizes(), g.options()), dg = at::empty(g.sizes(), g.options()), ws;
+        if (const int64_t bytes = mmf_hgrn_recurrent_bwd_workspace_bytes(bh, t, d)) ws = at::empty({bytes / 4}, g.options().dtype(at::kFloat));
+        const int rc = mmf_hgrn_recurrent_bwd_split(g.data_ptr(), o.data_ptr(), dout.data_ptr(), floats(state), dx.data_ptr(), dg.data_ptr(), bh, t, d,
+                                           ctx->saved_data["log_gates"].toBool() ? 1 : 0, dtype_of(g.scalar_type()), floats(ws),
+                                           stream_of(g));
+        TORCH_CHECK(rc == 0, "mmf_hgrn_recurrent_bwd_split: ", rc < 0 ? "MMF error " : "HIP error ", rc);
+        return {dx, dg, Tensor(), Tensor(), Tensor()};
+    }
+};
+
+// (x, g, initial state or None, final_state, chunk or 0, what raises for a return code) -> (o, final state or None); the caller has
+// checked the operands
+PyObject* scan(PyObject*, PyObject* const* args, Py_ssize_t count) {
+    HANDLE_TH_ERRORS
+    if (count != 6 || !THPVariable_Check(args[0]) || !THPVariable_Check(args[1]) || !(args[2] == Py_None || THPVariable_Check(args[2]))) {
+        PyErr_SetString(PyExc_TypeError, "scan takes (x, g, initial_state, final_state, chunk, check)");
+        return nullptr;
+    }
+    const Tensor &x = THPVariable_Unpack(args[0]), &g = THPVariable_Unpack(args[1]);
+    const std::optional<Tensor> h0 = args[2] == Py_None ? std::nullopt : std::optional<Tensor>(THPVariable_Unpack(args[2]));
+    const bool final_state = PyObject_IsTrue(args[3]) == 1;
+    const int64_t chunk = PyLong_AsLongLong(args[4]);
+    if (PyErr_Occurred()) return nullptr;
+    variable_list out;
+    try {
+        NoGil nogil;
+        out = ScanFn::apply(x, g, h0, final_state, chunk);
+    } catch (const Failed& f) {
+        Py_XDECREF(PyObject_CallFunction(args[5], "is", f.rc, f.what));
+        if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, f.what);
+        return nullptr;
+    }
+    PyObject* o = THPVariable_Wrap(out[0]);
+    PyObject* last = Py_None;
+    if (out.size() > 1) last = THPVariable_Wrap(out[1]);
+    else Py_INCREF(last);
+    PyObject* r = PyTuple_Pack(2, o, last);
+    Py_DECREF(o);
+    Py_DECREF(last);
+    return r;
+    END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef methods[] = {
+    {"bitlinear_few_rows", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(few_rows)), METH_FASTCALL, nullptr},
+    {"scan", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(scan)), METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "mmf_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit_mmf_torch() { return PyModule_Create(&module); }

@@ -419,12 +419,21 @@ def _state32(h0, bh, d, dev):
     return h0.detach().reshape(bh, d).to(device=dev, dtype=torch.float32).contiguous()
 
 
-def hgrn_recurrent(x, g, initial_state=None, output_final_state=False):
-    """x, g [B, H, T, D]; g is the decay itself.  Returns (o, final_state fp32 [B, H, D] or None)."""
-    lib = L.load()
+def check_scan(x, g, initial_state, chunk_size=1):
+    """The operands of a scan: one device, one shape and dtype; returns the device."""
     dev = L.require_gpu(x, g, initial_state)
     if x.shape != g.shape or x.dtype != g.dtype or x.dim() != 4:
         raise ValueError("x and g must be [B, H, T, D] tensors of one dtype")
+    if not 1 <= chunk_size <= 64:
+        raise ValueError("chunk_size must lie in [1, 64]")
+    L.dtype_id(x.dtype)
+    return dev
+
+
+def hgrn_recurrent(x, g, initial_state=None, output_final_state=False):
+    """x, g [B, H, T, D]; g is the decay itself.  Returns (o, final_state fp32 [B, H, D] or None)."""
+    lib = L.load()
+    dev = check_scan(x, g, initial_state)
     b, h, t, d = x.shape
     xc, gc = x.contiguous(), g.contiguous()
     o = torch.empty_like(xc)
@@ -439,16 +448,12 @@ def hgrn_recurrent(x, g, initial_state=None, output_final_state=False):
 def hgrn_chunk(x, g, initial_state=None, output_final_state=False, chunk_size=64):
     """x, g [B, H, T, D]; g is the LOG decay.  Returns (o, final_state fp32 or None)."""
     lib = L.load()
-    dev = L.require_gpu(x, g, initial_state)
-    if x.shape != g.shape or x.dtype != g.dtype or x.dim() != 4:
-        raise ValueError("x and g must be [B, H, T, D] tensors of one dtype")
+    dev = check_scan(x, g, initial_state, chunk_size)
     b, h, t, d = x.shape
     xc, gc = x.contiguous(), g.contiguous()
     o = torch.empty_like(xc)
     h0 = _state32(initial_state, b * h, d, dev)
     ht = torch.empty(b, h, d, dtype=torch.float32, device=dev) if output_final_state else None
-    if not 1 <= chunk_size <= 64:
-        raise ValueError("chunk_size must lie in [1, 64]")
     nws = lib.mmf_hgrn_chunk_workspace_bytes(b * h, t, d, chunk_size)
     ws = torch.empty(nws // 4, dtype=torch.float32, device=dev) if nws else None    # per-segment carries (few KB)
     with L.on(dev):
