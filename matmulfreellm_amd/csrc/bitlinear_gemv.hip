@@ -10,7 +10,7 @@
 // A decode step is a chain of dependent launches whose cost is latency, not bandwidth, so
 // every elementwise op is folded into the GEMV that consumes or produces it.
 //
-// Grid = (groups of 32 - or, for small launches, 8 - output rows, M).  A workgroup of 8 to 16 waves owns R
+// Grid = (groups of 32 - or, for small launches, 8 - output rows, M).  A workgroup of 4 to 16 waves owns R
 // n-blocks (or 8 rows of each) of one row of x.
 //   prologue : every workgroup recomputes the row's input itself (the row is <= 16 KiB and L2
 //              resident) and leaves the int8 codes in LDS:
@@ -458,13 +458,19 @@ int launch_gemv(const GemvArgs& a, int64_t M, bool vec, hipStream_t s) {
     const int64_t nblocks = mmf_ceil_div(a.N / R, 32);
     // few n-blocks (a 2048-row projection has 64): give each workgroup 8 rows, not 32, to reach every CU
     const bool split = vec && nblocks * M <= 64;             // at most 256 workgroups after the split: one per CU
-    // waves per workgroup and passes over the row: the fewest passes, then the fewest waves, that cover K
-    const int nw = a.Kp <= 2048 ? 8 : a.Kp <= 3072 ? 12 : a.Kp <= 4096 ? 16 : a.Kp <= 6144 ? 12 : 16;
+    // waves per workgroup and passes over the row: the fewest passes, then the fewest waves, that cover K (1024 wide, 4 waves instead
+    // of 8 half of which had no element: 5 rows of the 24-layer step 487 -> 453 us).  More workgroups than CUs: a workgroup's cost is
+    // then issue slots, not one stream's latency, and 4 waves of 8 elements spend fewer on the reductions than 8 of 4 (2048 wide, the
+    // step with 5 rows 836 -> 800 us, with 8 905 -> 864; with one workgroup per CU they lose, 515 -> 530)
+    const bool many = nblocks * M > 256;
+    const int nw = a.Kp <= 1024 || (a.Kp <= 2048 && many) ? 4 : a.Kp <= 2048 ? 8 : a.Kp <= 3072 ? 12 : a.Kp <= 4096 ? 16 : a.Kp <= 6144 ? 12 : 16;
     // many more n-blocks than resident workgroups (vocabulary-sized N): a grid of resident workgroups walks them
     const int64_t per_row = gemv_walk_slots(64 * nw) / M;
     const bool walk = vec && EPI == EPI_PLAIN && !a.norm_w2 && per_row >= 32 && nblocks > per_row;
     dim3 grid((unsigned)(walk ? per_row : nblocks * (split ? 4 : 1)), (unsigned)M);
     if (!vec) bitlinear_gemv_kernel<T, TW, 8, 4, PRO, EPI, false, 1, false, NN><<<grid, dim3(512), (size_t)a.Kp * NN, s>>>(a);   // ragged shapes: one generic build
+    else if (a.Kp <= 1024) launch_gemv_shape<T, TW, PRO, EPI, 4, 1, NN>(a, grid, split, walk, s);
+    else if (a.Kp <= 2048 && many) launch_gemv_shape<T, TW, PRO, EPI, 4, 2, NN>(a, grid, split, walk, s);
     else if (a.Kp <= 2048) launch_gemv_shape<T, TW, PRO, EPI, 8, 1, NN>(a, grid, split, walk, s);
     else if (a.Kp <= 3072) launch_gemv_shape<T, TW, PRO, EPI, 12, 1, NN>(a, grid, split, walk, s);
     else if (a.Kp <= 4096) launch_gemv_shape<T, TW, PRO, EPI, 16, 1, NN>(a, grid, split, walk, s);
