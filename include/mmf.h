@@ -328,6 +328,10 @@ int mmf_short_conv_bwd(const void* x, const void* weight, const void* bias, cons
 int64_t mmf_sample_top_p_max_vocab(void);
 int mmf_sample_top_p(const void* logits, int64_t ld, int64_t rows, int64_t V, float temperature, float top_p,
                      int64_t top_k, const float* u, int64_t* out, int dtype, void* stream);
+/* mmf_sample_top_p_recorded: the same draw as a launch that a captured graph can replay with other numbers: params (device memory):
+ *   temperature > 0, top_p in [0, 1] and top_k (as int32 bits); u: fp32 [*, rows], row r draws with u[pos[r] * rows + r]. */
+int mmf_sample_top_p_recorded(const void* logits, int64_t ld, int64_t rows, int64_t V, const float* params, const float* u,
+                              const int* pos, int64_t* out, int dtype, void* stream);
 
 /* ---- one whole batch-1 decode step in one persistent launch ---------------------------------
  * mmf_decode_layers replaces, for one token, the loop over HGRNBitBlock.forward in HGRNBitModel.forward

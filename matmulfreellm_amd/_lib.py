@@ -96,6 +96,7 @@ SIGNATURES = {
     "mmf_block_train_forward": (_i32, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _ptr, _ptr, _ptr, _ptr]),
     "mmf_block_forward": (_i32, [_ptr, _ptr, _ptr, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr]),
     "mmf_sample_top_p_max_vocab": (_i64, []),
+    "mmf_sample_top_p_recorded": (_i32, [_ptr, _i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _i32, _ptr]),
     "mmf_sample_top_p": (_i32, [_ptr, _i64, _i64, _i64, _f32, _f32, _i64, _ptr, _ptr, _i32, _ptr]),
 }
 

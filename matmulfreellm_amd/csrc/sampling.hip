@@ -39,6 +39,8 @@ struct SampleArgs {
     int V;
     float temperature, top_p;
     int top_k;              // 0: no limit
+    const float* params;    // null, or {temperature, top_p, bits of top_k} in device memory instead of the three above
+    const int* pos;         // null, or per row which row of u [*, rows] holds its number
     const float* u;
     int64_t* out;
 };
@@ -137,8 +139,11 @@ __global__ __launch_bounds__(kSampThreads) void sample_top_p_kernel(SampleArgs a
     __shared__ unsigned few_m[64];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int V = a.V;
+    const float temperature = a.params ? a.params[0] : a.temperature, top_p = a.params ? a.params[1] : a.top_p;
+    const int top_k = a.params ? __float_as_int(a.params[2]) : a.top_k;
     const T* row = static_cast<const T*>(a.logits) + (int64_t)blockIdx.x * a.ld;
     const int base = t * NPT;
+    const int64_t u_at = blockIdx.x + (a.pos ? (int64_t)a.pos[blockIdx.x] * gridDim.x : 0);
     const bool vec_ok = (V % 8) == 0 && (a.ld % 8) == 0 && (reinterpret_cast<uintptr_t>(a.logits) & 15u) == 0;
 
     Raw8<T> raw[NPT / 8];
@@ -157,7 +162,7 @@ __global__ __launch_bounds__(kSampThreads) void sample_top_p_kernel(SampleArgs a
         for (int i = 0; i < 8; ++i) {
             const int idx = base + c * 8 + i;
             float x = v[i];
-            x = (idx < V && x == x) ? __fdiv_rn(x, a.temperature) : -INFINITY;
+            x = (idx < V && x == x) ? __fdiv_rn(x, temperature) : -INFINITY;
             l[c * 8 + i] = x;
             mx = fmaxf(mx, x);
         }
@@ -169,7 +174,7 @@ __global__ __launch_bounds__(kSampThreads) void sample_top_p_kernel(SampleArgs a
     for (int w = 0; w < kSampWaves; ++w) mx = fmaxf(mx, wmax[w]);
 
     unsigned m[NPT];
-    if (a.top_k > 0 && a.top_k < V && mx != -INFINITY) {          // a row without a finite logit has no top_k-th largest: it is drawn
+    if (top_k > 0 && top_k < V && mx != -INFINITY) {          // a row without a finite logit has no top_k-th largest: it is drawn
                                                                    // uniformly like without the limit (every mass is 2^31)
         // order-preserving image of the scaled logits: non-negative floats above the negative ones, -inf and the slots
         // past V at 0 (which the descent ignores)
@@ -178,7 +183,7 @@ __global__ __launch_bounds__(kSampThreads) void sample_top_p_kernel(SampleArgs a
             const unsigned b = __float_as_uint(__fadd_rn(l[j], 0.0f));       // -0 counts as +0, as the comparison of floats does
             m[j] = l[j] == -INFINITY ? 0u : (b & 0x80000000u) ? ~b : (b | 0x80000000u);
         }
-        const unsigned kth = samp_descent<true, NPT>(m, (u64)a.top_k, hist, hsum, sel);
+        const unsigned kth = samp_descent<true, NPT>(m, (u64)top_k, hist, hsum, sel);
         // the kept tokens (top_k of them, more on ties) with their masses, in any order, for one wave to finish
         if (t == 0) few_n = 0;
         __syncthreads();
@@ -207,7 +212,7 @@ __global__ __launch_bounds__(kSampThreads) void sample_top_p_kernel(SampleArgs a
 #pragma unroll
                 for (int o = 32; o > 0; o >>= 1) Zf += samp_shfl_down(Zf, o);
                 Zf = ((u64)(unsigned)__builtin_amdgcn_readfirstlane((int)(Zf >> 32)) << 32) | (unsigned)__builtin_amdgcn_readfirstlane((int)Zf);
-                u64 Pf = (u64)((double)a.top_p * (double)Zf);
+                u64 Pf = (u64)((double)top_p * (double)Zf);
                 if (Pf < 1) Pf = 1;
                 u64 heavier = 0;
 #pragma unroll
@@ -220,7 +225,7 @@ __global__ __launch_bounds__(kSampThreads) void sample_top_p_kernel(SampleArgs a
 #pragma unroll
                 for (int o = 32; o > 0; o >>= 1) Sf += samp_shfl_down(Sf, o);
                 Sf = ((u64)(unsigned)__builtin_amdgcn_readfirstlane((int)(Sf >> 32)) << 32) | (unsigned)__builtin_amdgcn_readfirstlane((int)Sf);
-                float uf = a.u[blockIdx.x];
+                float uf = a.u[u_at];
                 uf = uf >= 0.0f ? uf : 0.0f;
                 u64 target = (u64)((double)uf * (double)Sf);
                 if (target >= Sf) target = Sf - 1;
@@ -252,7 +257,7 @@ __global__ __launch_bounds__(kSampThreads) void sample_top_p_kernel(SampleArgs a
     u64 Z = 0;
 #pragma unroll
     for (int w = 0; w < kSampWaves; ++w) Z += wtot[w];
-    u64 P = (u64)((double)a.top_p * (double)Z);
+    u64 P = (u64)((double)top_p * (double)Z);
     if (P < 1) P = 1;
 
     // ---- the nucleus: the smallest kept mass
@@ -277,7 +282,7 @@ __global__ __launch_bounds__(kSampThreads) void sample_top_p_kernel(SampleArgs a
         S += x;
         if (w < wave) before += x;
     }
-    float u = a.u[blockIdx.x];
+    float u = a.u[u_at];
     u = u >= 0.0f ? u : 0.0f;                                     // NaN and negatives draw the first kept token
     u64 target = (u64)((double)u * (double)S);
     if (target >= S) target = S - 1;                              // u >= 1
@@ -328,6 +333,23 @@ int mmf_sample_top_p(const void* logits, int64_t ld, int64_t rows, int64_t V, fl
     a.top_p = top_p < 0.0f ? 0.0f : top_p > 1.0f ? 1.0f : top_p;
     a.top_k = top_k >= V ? 0 : (int)top_k;
     a.u = u; a.out = out;
+    switch (dtype) {
+        case MMF_F32: return launch_sample<float>(a, rows, stream);
+        case MMF_BF16: return launch_sample<bf16_t>(a, rows, stream);
+        case MMF_F16: return launch_sample<f16_t>(a, rows, stream);
+    }
+    return MMF_ERR_ARG;
+}
+
+int mmf_sample_top_p_recorded(const void* logits, int64_t ld, int64_t rows, int64_t V, const float* params, const float* u,
+                              const int* pos, int64_t* out, int dtype, void* stream_) {
+    hipStream_t stream = static_cast<hipStream_t>(stream_);
+    if (rows < 0 || V <= 0 || ld < V || rows > 0x7fffffff) return MMF_ERR_ARG;
+    if (rows == 0) return 0;
+    if (!logits || !params || !u || !pos || !out) return MMF_ERR_ARG;
+    if (V > kSampMaxV) return MMF_ERR_WIDE;
+    SampleArgs a{};
+    a.logits = logits; a.ld = ld; a.V = (int)V; a.params = params; a.u = u; a.pos = pos; a.out = out;
     switch (dtype) {
         case MMF_F32: return launch_sample<float>(a, rows, stream);
         case MMF_BF16: return launch_sample<bf16_t>(a, rows, stream);

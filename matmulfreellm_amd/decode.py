@@ -16,6 +16,7 @@ Every launch is the same C-ABI call with the same arithmetic as the module path,
 produce identical bits (tests/test_gpu_model.py checks that).
 """
 import ctypes
+import struct
 import warnings
 from typing import List, Optional
 
@@ -107,6 +108,9 @@ class DecodeEngine:
         # every step records the token it was fed: row t of the history is step t's, modulo CHUNK, counted per batch row
         self.history = torch.zeros(self.CHUNK, B, dtype=torch.int64, device=dev)
         self.pos = torch.zeros(B, dtype=torch.int32, device=dev)
+        # what a drawing step reads: temperature, top_p and top_k, and the uniform numbers of the steps that leave pos at t in row t
+        self.draw_params = torch.zeros(3, dtype=torch.float32, device=dev)
+        self.draw_u = torch.zeros(self.CHUNK, B, dtype=torch.float32, device=dev)
         self.h = z(B, H)            # residual stream
         self.hn = z(B, H)
         self.ifg = z(B, 3 * D)
@@ -132,7 +136,8 @@ class DecodeEngine:
             raise L.MMFError("DecodeEngine: this model / batch / device does not fit the resident layer chain")
         if self.resident:
             self._build_resident()
-        self.graph = None
+        self.graphs = {}            # recorded steps, by whether they draw their token
+        self.probed = False         # the resident chain's workgroups have been seen to be resident at once
 
     @classmethod
     def _stackable(cls, attn):
@@ -255,8 +260,10 @@ class DecodeEngine:
         torch.cuda.synchronize(self.dev)
         return t.view(256, 128, 12).cpu()
 
-    def _launch_step_resident(self):
+    def _launch_step_resident(self, draw):
         self._launch_layers(True)       # the whole step: final norm, lm_head and argmax are the launch's last two links
+        if draw:
+            self._choose(True)
 
     def resident_ok(self) -> bool:
         """False once a wait inside the resident layer chain ran out of polling rounds (host synchronisation)."""
@@ -288,9 +295,19 @@ class DecodeEngine:
                                               self.history.data_ptr(), self.pos.data_ptr(), self.CHUNK, self.dt_id, L.stream()),
                 "mmf_embedding_record")
 
-    def _launch_step_fused(self, ends=True):
+    def _choose(self, draw):
+        """The step's token from its logits: the largest, or the draw that run() has set up."""
+        if draw:
+            L.check(self.lib.mmf_sample_top_p_recorded(self.logits.data_ptr(), self.V, self.B, self.V, self.draw_params.data_ptr(),
+                                                       self.draw_u.data_ptr(), self.pos.data_ptr(), self.tok.data_ptr(), self.dt_id,
+                                                       L.stream()), "mmf_sample_top_p_recorded")
+        else:
+            L.check(self.lib.mmf_argmax(self.logits.data_ptr(), self.V, self.B, self.V, self.tok.data_ptr(), self.dt_id, L.stream()),
+                    "mmf_argmax")
+
+    def _launch_step_fused(self, ends=True, draw=False):
         """Batch <= GEMV_MAX_M: four launches per layer, every elementwise op folded into a GEMV.
-        ends=False leaves out the embedding gather and the argmax (the 4L+1 GEMV launches only)."""
+        ends=False leaves out the embedding gather and the choice of the token (the 4L+1 GEMV launches only)."""
         lib, s, B, H, D, I = self.lib, L.stream(), self.B, self.H, self.D, self.I
         if ends:
             self._embed()
@@ -316,8 +333,7 @@ class DecodeEngine:
         self._fused(self.NORM, self.E_PLAIN, self.h, H, None, 0, None, self.final_norm, self.eps, self.head, self.logits,
                     None, None, None, self.V, H)
         if ends:
-            L.check(lib.mmf_argmax(self.logits.data_ptr(), self.V, B, self.V, self.tok.data_ptr(), self.dt_id, s),
-                    "mmf_argmax")
+            self._choose(draw)
 
     def fused_step_bytes(self, with_head: bool = True):
         """Algorithmic bytes of the 4L (+1 with head) fused BitLinears of one batch-B step: 2-bit weights once, plus
@@ -342,7 +358,7 @@ class DecodeEngine:
                                             pw.packed.data_ptr(), pw.wdeq.data_ptr(), pw.seg_rows, None, L.ptr(addend),
                                             out.data_ptr(), n, self.B, k, n, self.dt_id, -1, L.stream()), "mmf_bitlinear_mfma")
 
-    def _launch_step_mfma_fused(self):
+    def _launch_step_mfma_fused(self, draw):
         """Batch > GEMV_MAX_M: eight launches per layer -- each BitLinear is a fused prologue+quantiser row kernel
         (norm / recurrence step + gated norm / residual norm / swiglu folded in) and a matrix-core contraction."""
         lib, s, B, H, D, I = self.lib, L.stream(), self.B, self.H, self.D, self.I
@@ -378,7 +394,7 @@ class DecodeEngine:
         self._qfused(1, self.h.data_ptr(), H, None, 0, None, 0, None, self.final_norm, self.eps, self.head[1], self.head[2],
                      None, None, H)
         self._mfma(self.head[0], self.logits, self.V, H)
-        L.check(lib.mmf_argmax(self.logits.data_ptr(), self.V, B, self.V, self.tok.data_ptr(), self.dt_id, s), "mmf_argmax")
+        self._choose(draw)
 
     def _can_fuse_mfma(self):
         same_dt = all(t.dtype == self.final_norm.dtype for e in self.layers
@@ -395,13 +411,13 @@ class DecodeEngine:
         return (self.gemv and same_dt and all(e["ifg"] is not None for e in self.layers)
                 and max(self.H, self.D, self.I) <= kmax and self.D % 32 == 0 and self.I % 32 == 0)
 
-    def _launch_step(self):
+    def _launch_step(self, draw=False):
         if self.resident:
-            return self._launch_step_resident()
+            return self._launch_step_resident(draw)
         if self.fused:
-            return self._launch_step_fused()
+            return self._launch_step_fused(draw=draw)
         if self.fused_mfma:
-            return self._launch_step_mfma_fused()
+            return self._launch_step_mfma_fused(draw)
         lib, s, B, H, D, I = self.lib, L.stream(), self.B, self.H, self.D, self.I
         dt, esz = self.dt_id, self.h.element_size()
         wid = L.dtype_id(self.final_norm.dtype)
@@ -433,16 +449,17 @@ class DecodeEngine:
         L.check(lib.mmf_rmsnorm(self.h.data_ptr(), None, self.final_norm.data_ptr(), self.hn.data_ptr(), None, B, H,
                                 self.eps, dt, dt, wid, s), "mmf_rmsnorm")
         self._bitlinear(self.hn, self.head, self.logits, (self.V, H))
-        L.check(lib.mmf_argmax(self.logits.data_ptr(), self.V, B, self.V, self.tok.data_ptr(), dt, s), "mmf_argmax")
+        self._choose(draw)
 
-    def _capture(self):
-        # warm-up launches on a side stream (module loading, attribute setting), then record
+    def _prepare(self, draw):
+        """Warm-up launches on a side stream (module loading, attribute setting); then the step is recorded, unless it is a single
+        launch (as a graph of one node the resident step takes 399 us for 394)."""
         saved = [e["state"].clone() for e in self.layers]
         tok, pos = self.tok.clone(), self.pos.clone()
         side = torch.cuda.Stream(device=self.dev)
         side.wait_stream(torch.cuda.current_stream(self.dev))
         with torch.cuda.stream(side):
-            self._launch_step()
+            self._launch_step(draw)
         torch.cuda.current_stream(self.dev).wait_stream(side)
         torch.cuda.synchronize(self.dev)
         if self.resident and not self.resident_ok():
@@ -455,18 +472,20 @@ class DecodeEngine:
                 e["state"].copy_(sv)
             self.tok.copy_(tok)
             with torch.cuda.stream(side):
-                self._launch_step()
+                self._launch_step(draw)
             torch.cuda.current_stream(self.dev).wait_stream(side)
             torch.cuda.synchronize(self.dev)
-        g = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(g):
-            self._launch_step()
-        torch.cuda.synchronize(self.dev)
+        self.probed = True
+        if not self.resident:
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g):
+                self._launch_step(draw)
+            torch.cuda.synchronize(self.dev)
+            self.graphs[draw] = g
         for e, sv in zip(self.layers, saved):     # undo the warm-up step's state update
             e["state"].copy_(sv)
         self.tok.copy_(tok)
         self.pos.copy_(pos)
-        self.graph = g
 
     # ------------------------------------------------------------------ public
     def load_state(self, states: Optional[List[torch.Tensor]]):
@@ -481,16 +500,16 @@ class DecodeEngine:
     def export_state(self):
         return [e["state"].clone() for e in self.layers]
 
-    def advance(self):
-        """One decode step from the token buffer; leaves logits in self.logits and the greedy
+    def advance(self, draw: bool = False):
+        """One decode step from the token buffer; leaves logits in self.logits and the greedy (``draw``: the drawn, see run)
         next token in the token buffer (no host synchronisation)."""
         with L.on(self.dev):
-            if not self.use_graph:
-                self._launch_step()
-                return
-            if self.graph is None:
-                self._capture()
-            self.graph.replay()
+            if self.use_graph and not (self.probed if self.resident else draw in self.graphs):
+                self._prepare(draw)
+            if self.use_graph and not self.resident:
+                self.graphs[draw].replay()
+            else:
+                self._launch_step(draw)
 
     def step(self, tokens: torch.Tensor) -> torch.Tensor:
         """Feed `tokens` [B]; returns the logits buffer [B, V] (overwritten by the next step)."""
@@ -498,17 +517,27 @@ class DecodeEngine:
         self.advance()
         return self.logits
 
-    def run(self, n_steps: int, pick=None, seen=None) -> torch.Tensor:
+    def run(self, n_steps: int, pick=None, seen=None, draw=None) -> torch.Tensor:
         """n_steps self-feeding steps from the token buffer; returns the [n_steps + 1, B] tokens: what the buffer held, then what
-        it held after each step.  pick(t), when given, replaces the token step t chose.  seen(tokens [t + 1, B]), when given, is
+        it held after each step.  pick(t), when given, replaces the token step t chose; draw =
+        (uniform numbers [n_steps, B], top_p, temperature, top_k) has the steps draw theirs as functional.sample_top_p does.  seen(tokens [t + 1, B]), when given, is
         asked every CHUNK steps whether to stop there.  No host synchronisation of its own."""
         out = torch.empty(n_steps + 1, self.B, dtype=torch.int64, device=self.dev)
         self.pos.zero_()
+        if draw is not None:
+            u, top_p, temperature, top_k = draw
+            params = struct.pack("=ffi", temperature, min(max(top_p, 0.0), 1.0), top_k if top_k < self.V else 0)
+            self.draw_params.view(torch.uint8).copy_(torch.frombuffer(bytearray(params), dtype=torch.uint8))
         done = 0
         while done < n_steps:
             n = min(self.CHUNK, n_steps - done)
+            if draw is not None:                                # step t of the chunk leaves pos at (t + 1) % CHUNK
+                m = min(n, self.CHUNK - 1)
+                self.draw_u[1:m + 1].copy_(u[done:done + m])
+                if m < n:
+                    self.draw_u[0].copy_(u[done + m])
             for t in range(done, done + n):
-                self.advance()
+                self.advance(draw is not None)
                 if pick is not None:
                     pick(t)
             out[done:done + n].copy_(self.history[:n])

@@ -533,8 +533,12 @@ class HGRNBitForCausalLM(HGRNBitPreTrainedModel, GenerationMixin):
         tok = engine.tok if engine is not None else None         # the engine's own buffer: its first step embeds it
         first = choose(logits, 0, tok) if do_sample else F_.argmax(logits, tok)
         if engine is not None:
-            pick = (lambda step: choose(engine.logits, step + 1, engine.tok)) if do_sample else None
-            new = _self_feeding(engine, max_new_tokens, eos_token_id, pad_token_id, pick=pick)
+            pick = draw = None
+            if do_sample and logits.shape[-1] <= F_.sample_top_p_max_vocab():
+                draw = (uniforms[1:], float(top_p), temperature, top_k)
+            elif do_sample:
+                pick = lambda step: choose(engine.logits, step + 1, engine.tok)
+            new = _self_feeding(engine, max_new_tokens, eos_token_id, pad_token_id, pick=pick, draw=draw)
             engine.check()
             return torch.cat([input_ids, new], dim=1)
         nxt = first
@@ -553,14 +557,14 @@ class HGRNBitForCausalLM(HGRNBitPreTrainedModel, GenerationMixin):
         return torch.cat(tokens, dim=1)
 
 
-def _self_feeding(engine, max_new_tokens, eos_token_id, pad_token_id, pick=None):
+def _self_feeding(engine, max_new_tokens, eos_token_id, pad_token_id, pick=None, draw=None):
     """Decoding from the engine's token buffer without a host round trip per token: every replay of its graph leaves its
-    argmax in the buffer the next replay embeds and records; pick(step), when given, replaces that token by one drawn
-    from the step's logits (sampling).  The end-of-sequence test looks at a whole chunk of steps at a time;
+    choice in the buffer the next replay embeds and records: its argmax, with ``draw`` a token drawn within the step, with pick(step)
+    one drawn from the step's logits behind it (vocabularies the draw kernel does not take).  The end-of-sequence test looks at a whole chunk of steps at a time;
     the steps decoded past the point where every row had finished are cut off, and a finished row's later tokens
     are replaced by the padding id, so the result is the one of the token-by-token loop."""
     seen = (lambda toks: bool((toks == eos_token_id).any(0).all())) if eos_token_id is not None else None
-    seq = engine.run(max_new_tokens - 1, pick, seen).t()                        # [B, produced]
+    seq = engine.run(max_new_tokens - 1, pick, seen, draw).t()                        # [B, produced]
     if eos_token_id is None:
         return seq.contiguous()
     is_eos = seq == eos_token_id
