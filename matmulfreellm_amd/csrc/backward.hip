@@ -149,7 +149,7 @@ __global__ __launch_bounds__(kBT) void rmsnorm_bwd_kernel(NormBwdArgs a) {
                 const int k0 = (v * kBT + (int)threadIdx.x) * 4;
                 float o[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) o[i] = __fmul_rn((float)mmf_code(__fmul_rn(xh[v][i], wv[v][i]), scale), deq);
+                for (int i = 0; i < 4; ++i) o[i] = __fmul_rn(mmf_code_f(__fmul_rn(xh[v][i], wv[v][i]), scale), deq);
                 raw4_store<T, VEC>(y, k0, K, o);
             }
         }

@@ -197,7 +197,7 @@ __global__ __launch_bounds__(KT) void chain_bwd_kernel(ChainArgs a) {
                 float w2[4], o[4];
                 raw4_unpack<TW>(w2r[n][v], w2);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) o[i] = __fmul_rn((float)mmf_code(__fmul_rn(s[v][i], w2[i]), scale[n]), deq[n]);
+                for (int i = 0; i < 4; ++i) o[i] = __fmul_rn(mmf_code_f(__fmul_rn(s[v][i], w2[i]), scale[n]), deq[n]);
                 raw4_store<T, true>(static_cast<T*>(a.y) + ((int64_t)n * a.M + row) * K, k0, K, o);
             }
             float w1[4], o[4];

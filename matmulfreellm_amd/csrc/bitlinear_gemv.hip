@@ -294,14 +294,12 @@ __global__ __launch_bounds__(64 * NW) void bitlinear_gemv_kernel(GemvArgs a) {
             for (int j = 0; j < NN; ++j) {
                 float wv[4];
                 if constexpr (NN > 1) raw4_unpack<TW>(nwraw[j][v], wv);
-                uint32_t packed4 = 0;
+                float y[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float y = NN > 1 ? __fmul_rn(xv[v][i], wv[i]) : xv[v][i];
-                    const int c = (k0 + i < K) ? mmf_code(y, scale[j]) : 0;
-                    qs[j] += c;
-                    packed4 |= (uint32_t)(c & 0xff) << (8 * i);
-                }
+                for (int i = 0; i < 4; ++i) y[i] = NN > 1 && (VEC || k0 + i < K) ? __fmul_rn(xv[v][i], wv[i]) : xv[v][i];   // zeros past K
+                uint32_t packed4 = mmf_code4(y, scale[j]);
+                if (VEC && k0 >= K) packed4 = 0;
+                qs[j] = mmf_code4_sum(packed4, qs[j]);
                 *reinterpret_cast<uint32_t*>(q_lds + j * Kp + k0) = packed4;
             }
         }

@@ -673,10 +673,8 @@ __global__ __launch_bounds__(kNT) void decode_layers_kernel(LayersArgs a) {
 #pragma unroll
             for (int v = 0; v < NPK; ++v) {
                 if (v < g.np) {
-                    uint32_t packed4 = 0;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) packed4 |= (uint32_t)(mmf_code(yv[n][v][i], scale[n]) & 0xff) << (8 * i);
-                    qs = __builtin_amdgcn_sdot4((int)packed4, 0x01010101, qs, false);      // the sum of the four codes
+                    const uint32_t packed4 = mmf_code4(yv[n][v], scale[n]);
+                    qs = mmf_code4_sum(packed4, qs);
                     if (has[v]) *reinterpret_cast<uint32_t*>(qbuf + (NN > 1 ? n * Hh : 0) + k0[v]) = packed4;
                 }
             }

@@ -483,11 +483,22 @@ __device__ __forceinline__ float mmf_rstd(double sumsq, int64_t K, double inv_K,
 }
 
 // int8 code of one normalised value:  clamp(rint(y * scale), -128, 127)
-__device__ __forceinline__ int mmf_code(float y, float scale) {
-    float r = rintf(__fmul_rn(y, scale));
-    r = fminf(fmaxf(r, -128.0f), 127.0f);
-    return (int)r;
+
+// The codes of four neighbouring values in the bytes of a dword, and their sum.  Adding 1.5 * 2^23 to a value of at most 128 rounds it to
+// an integer (nearest, ties to even, as rintf does) whose low byte is the low byte of the sum: three operations a value and
+// three for the dword, where rint, clamp, convert, mask and shift took nine a value.
+__device__ __forceinline__ uint32_t mmf_code4(const float (&y)[4], float scale) {
+    uint32_t b[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        b[i] = __float_as_uint(__fadd_rn(fminf(fmaxf(__fmul_rn(y[i], scale), -128.0f), 127.0f), 12582912.0f));
+    return __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u) | __builtin_amdgcn_perm(b[3], b[2], 0x04000c0cu);
 }
+__device__ __forceinline__ int mmf_code4_sum(uint32_t codes, int sum) {
+    return __builtin_amdgcn_sdot4((int)codes, 0x01010101, sum, false);
+}
+// the code of one value as a float
+__device__ __forceinline__ float mmf_code_f(float y, float scale) { return fminf(fmaxf(rintf(__fmul_rn(y, scale)), -128.0f), 127.0f); }
 
 __host__ __device__ static inline int64_t mmf_ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 __host__ __device__ static inline int64_t mmf_round_up(int64_t a, int64_t b) { return mmf_ceil_div(a, b) * b; }

@@ -7,6 +7,7 @@
 // mmfreelm/modules/fused_norm_gate.py:68-131, mmfreelm/ops/fusedbitnet.py:63-131 and
 // the jiterator kernel at mmfreelm/modules/activations.py:115-119.
 #include "mmf_common.h"
+#include <type_traits>
 #include "../../include/mmf.h"
 
 namespace {
@@ -141,14 +142,11 @@ __global__ __launch_bounds__(kThreads) void row_kernel(RowArgs a) {
     for (int v = 0; v < NV; ++v) {
         const int64_t k0 = ((int64_t)v * kThreads + threadIdx.x) * 8;
         if (k0 < Kp) {
-            uint32_t lo = 0, hi = 0;
+            float y[8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                int c = (k0 + i < K) ? mmf_code(xv[v][i], scale) : 0;   // xv is 0 beyond K
-                qs += c;
-                uint32_t b = (uint32_t)(c & 0xff) << (8 * (i & 3));
-                if (i < 4) lo |= b; else hi |= b;
-            }
+            for (int i = 0; i < 8; ++i) y[i] = k0 + i < K ? xv[v][i] : 0.0f;
+            const uint32_t lo = mmf_code4({y[0], y[1], y[2], y[3]}, scale), hi = mmf_code4({y[4], y[5], y[6], y[7]}, scale);
+            qs = mmf_code4_sum(hi, mmf_code4_sum(lo, qs));
             int64_t off;
             if (a.q_tiled)
                 off = ((row >> 5) * (Kp >> 4) + (k0 >> 4)) * 512 + (row & 31) * 16 + (k0 & 15);
@@ -240,8 +238,11 @@ constexpr int kQWaves = 8, kQThreads = kQWaves * 64;
 // RPW rows per workgroup, 512 / RPW threads per row, NV passes of (512 / RPW) * 4 elements.
 //   RPW = 1 : a decode batch has few rows and each launch is a step of a dependent chain, so all
 //             8 waves share one row (shortest latency);
-//   RPW = 8 : prefill has thousands of rows and the kernel should stream: one wave per row, whose
-//             reductions are DPP folds only - no LDS exchange and no barrier anywhere.
+//   RPW = 2, 4, 8 : prefill has hundreds to thousands of rows and the kernel should stream: few waves per row, whose
+//             reductions cost little, and many elements per thread.
+// Bound by HBM and the vector units about equally (a row of 2048 quantised three times: ~1100 issue slots a wave against 16 KiB of
+// traffic), so what does not depend on the data is kept out: no bounds test in passes known to lie in the row, codes rounded and
+// packed four at a time.  8192 x 2048 bf16, three norms: 37 -> 28 us; residual norm: 33 -> 22.
 // VEC: K, the strides and every pointer allow 4-element accesses.
 // NN = 3: the row is normalised once and quantised under three norm weights (the projections of a trained layer share their
 // input, not their inner norm): one read of the row and one rstd instead of three, the three maxima in one exchange.
@@ -259,8 +260,16 @@ __global__ __launch_bounds__(kQThreads) void row_quant_fused_kernel(FusedQuantAr
     const bool live = row_raw < a.M;                            // rows past M compute on row M-1 and store nothing
     const int64_t row = live ? row_raw : a.M - 1;
     const int K = (int)a.K, Kp = (int)a.Kp;
-    // element k0 + i of the row exists; with vector accesses (K a multiple of 4) a thread's 4 elements stand or fall together
-    auto inb = [&](int k0, int i) { return VEC ? k0 < K : k0 + i < K; };
+    // the first FULL passes lie inside the row whatever K this instance is launched for (the next smaller one would take it otherwise)
+    constexpr int FULL = !VEC ? 0 : NV <= 4 ? NV - 1 : NV == 6 ? 4 : NV == 8 ? 6 : 8;
+    // element k0 + i of pass v of the row exists; with vector accesses (K a multiple of 4) a thread's 4 elements stand or fall together
+    auto inb = [&](int v, int k0, int i) __attribute__((always_inline)) { return v < FULL || (VEC ? k0 < K : k0 + i < K); };
+    // a pass's four elements of a row of E
+    auto ld = [&](auto* p, int v, int k0) __attribute__((always_inline)) {
+        using E = std::remove_const_t<std::remove_pointer_t<decltype(p)>>;
+        if (v < FULL) return Raw4<E>{*reinterpret_cast<const decltype(Raw4<E>::v)*>(p + k0)};
+        return raw4_load<E, VEC>(static_cast<const E*>(p), k0, K);
+    };
     const T* x = static_cast<const T*>(a.x) + row * a.ldx;
     const T* aux = static_cast<const T*>(a.aux) + row * a.ldaux;
     const T* aux2 = static_cast<const T*>(a.aux2) + row * a.ldaux2;
@@ -276,17 +285,17 @@ __global__ __launch_bounds__(kQThreads) void row_quant_fused_kernel(FusedQuantAr
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
         const int k0 = (v * TPR + tr) * 4;
-        xraw[v] = raw4_load<T, VEC>(x, k0, K);
-        if constexpr (HAS_AUX) araw[v] = raw4_load<T, VEC>(aux, k0, K);
+        xraw[v] = ld(x, v, k0);
+        if constexpr (HAS_AUX) araw[v] = ld(aux, v, k0);
         if constexpr (STEP) {
-            graw[v] = raw4_load<T, VEC>(aux2, k0, K);
-            straw[v] = raw4_load<float, VEC>(st, k0, K);
-            if (a.lb) lbraw[v] = raw4_load<float, VEC>(a.lb, k0, K);
+            graw[v] = ld(aux2, v, k0);
+            straw[v] = ld(st, v, k0);
+            if (a.lb) lbraw[v] = ld(a.lb, v, k0);
         }
-        if constexpr (HAS_W1) w1raw[v] = raw4_load<TW, VEC>(w1, k0, K);
+        if constexpr (HAS_W1) w1raw[v] = ld(w1, v, k0);
         if (NN > 1 || nw) {
 #pragma unroll
-            for (int j = 0; j < NN; ++j) nwraw[j][v] = raw4_load<TW, VEC>(nws[j], k0, K);
+            for (int j = 0; j < NN; ++j) nwraw[j][v] = ld(nws[j], v, k0);
         }
     }
     float xv[NV][4], av[HAS_AUX ? NV : 1][4];
@@ -297,14 +306,14 @@ __global__ __launch_bounds__(kQThreads) void row_quant_fused_kernel(FusedQuantAr
         if constexpr (HAS_AUX) raw4_unpack<T>(araw[v], av[v]);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            if (!inb(k0, i)) xv[v][i] = 0.0f;
+            if (!inb(v, k0, i)) xv[v][i] = 0.0f;
     }
     if constexpr (PRO == QPRO_RESNORM) {
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             const int k0 = (v * TPR + tr) * 4;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) xv[v][i] = inb(k0, i) ? __fadd_rn(xv[v][i], av[v][i]) : 0.0f;
+            for (int i = 0; i < 4; ++i) xv[v][i] = inb(v, k0, i) ? __fadd_rn(xv[v][i], av[v][i]) : 0.0f;
             if (a.res_out && live) raw4_store<T, VEC>(static_cast<T*>(a.res_out) + row * K, k0, K, xv[v]);
         }
     }
@@ -327,7 +336,7 @@ __global__ __launch_bounds__(kQThreads) void row_quant_fused_kernel(FusedQuantAr
                 const float h = __fadd_rn(__fmul_rn(go, stv[i]), xo);
                 stv[i] = h;
                 av[v][i] = mmf_round_to<T>(h);          // o, the swish gate of the gated norm
-                xv[v][i] = inb(k0, i) ? gv[i] : 0.0f;   // the gated norm normalises the g projection
+                xv[v][i] = inb(v, k0, i) ? gv[i] : 0.0f;   // the gated norm normalises the g projection
             }
             if (live) raw4_store<float, VEC>(st, k0, K, stv);
         }
@@ -357,7 +366,7 @@ __global__ __launch_bounds__(kQThreads) void row_quant_fused_kernel(FusedQuantAr
             for (int i = 0; i < 4; ++i) {
                 float y = __fmul_rn(__fmul_rn(xv[v][i], rstd1), w1v[i]);
                 if constexpr (STEP || PRO == QPRO_GATEDNORM) y = __fmul_rn(__fmul_rn(y, av[v][i]), sg[i]);
-                xv[v][i] = inb(k0, i) ? mmf_round_to<T>(y) : 0.0f;
+                xv[v][i] = inb(v, k0, i) ? mmf_round_to<T>(y) : 0.0f;
             }
         }
     } else if constexpr (PRO == QPRO_SWIGLU) {
@@ -368,7 +377,7 @@ __global__ __launch_bounds__(kQThreads) void row_quant_fused_kernel(FusedQuantAr
             for (int i = 0; i < 4; ++i) {
                 const float g = xv[v][i];
                 const float z = __fdiv_rn(__fmul_rn(g, av[v][i]), __fadd_rn(1.0f, mmf_exp(-g)));
-                xv[v][i] = inb(k0, i) ? mmf_round_to<T>(z) : 0.0f;
+                xv[v][i] = inb(v, k0, i) ? mmf_round_to<T>(z) : 0.0f;
             }
         }
     }
@@ -431,20 +440,18 @@ __global__ __launch_bounds__(kQThreads) void row_quant_fused_kernel(FusedQuantAr
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
         const int k0 = (v * TPR + tr) * 4;
-        if (k0 < Kp) {
+        if (v < FULL || k0 < Kp) {
             const int64_t off = ((row >> 5) * (Kp >> 4) + (k0 >> 4)) * 512 + (row & 31) * 16 + (k0 & 15);
 #pragma unroll
             for (int j = 0; j < NN; ++j) {
                 float wv[4];
                 if constexpr (NN > 1) raw4_unpack<TW>(nwraw[j][v], wv);
-                uint32_t packed4 = 0;
+                float y[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float y = NN > 1 ? __fmul_rn(xv[v][i], wv[i]) : xv[v][i];
-                    const int c = inb(k0, i) ? mmf_code(y, scale[j]) : 0;
-                    qs[j] += c;
-                    packed4 |= (uint32_t)(c & 0xff) << (8 * i);
-                }
+                for (int i = 0; i < 4; ++i) y[i] = NN > 1 && (VEC || inb(v, k0, i)) ? __fmul_rn(xv[v][i], wv[i]) : xv[v][i];   // zeros past K
+                uint32_t packed4 = mmf_code4(y, scale[j]);
+                if (VEC && !inb(v, k0, 0)) packed4 = 0;
+                qs[j] = mmf_code4_sum(packed4, qs[j]);
                 if (live) *reinterpret_cast<uint32_t*>(a.q + j * a.q_stride + off) = packed4;
             }
         }
@@ -481,11 +488,13 @@ int launch_fused_quant_rpw(const FusedQuantArgs& a, hipStream_t s) {
     else if (nv <= 2) row_quant_fused_kernel<T, TW, 2, PRO, true, RPW, NN><<<grid, block, 0, s>>>(a);
     else if (nv <= 3) row_quant_fused_kernel<T, TW, 3, PRO, true, RPW, NN><<<grid, block, 0, s>>>(a);
     else if (nv <= 4) row_quant_fused_kernel<T, TW, 4, PRO, true, RPW, NN><<<grid, block, 0, s>>>(a);
-    else if (nv <= 6) row_quant_fused_kernel<T, TW, 6, PRO, true, RPW, NN><<<grid, block, 0, s>>>(a);
-    else if (nv <= 8) row_quant_fused_kernel<T, TW, 8, PRO, true, RPW, NN><<<grid, block, 0, s>>>(a);
-    else if constexpr (PRO == QPRO_PLAIN && RPW == 4) {
-        if (nv > 12) return MMF_ERR_WIDE;
-        row_quant_fused_kernel<T, TW, 12, PRO, true, RPW, NN><<<grid, block, 0, s>>>(a);
+    else if constexpr (RPW < 8) {
+        if (nv <= 6) row_quant_fused_kernel<T, TW, 6, PRO, true, RPW, NN><<<grid, block, 0, s>>>(a);
+        else if (nv <= 8) row_quant_fused_kernel<T, TW, 8, PRO, true, RPW, NN><<<grid, block, 0, s>>>(a);
+        else if constexpr (PRO == QPRO_PLAIN && RPW == 4) {
+            if (nv > 12) return MMF_ERR_WIDE;
+            row_quant_fused_kernel<T, TW, 12, PRO, true, RPW, NN><<<grid, block, 0, s>>>(a);
+        } else return MMF_ERR_WIDE;
     } else return MMF_ERR_WIDE;
     MMF_CHECK_LAUNCH();
     return 0;
@@ -499,18 +508,15 @@ int launch_fused_quant(const FusedQuantArgs& a, bool vec, hipStream_t s) {
         MMF_CHECK_LAUNCH();
         return 0;
     }
-    // decode: latency (the recurrence-step prologue only exists there: one token per row)
-    if (a.M <= 256 || PRO == QPRO_STEP_GATE) return launch_fused_quant_rpw<T, TW, PRO, 1, NN>(a, s);
-    // prefill: as many rows per workgroup as 8 passes of 4 elements per thread allow
+    // The recurrence-step prologue exists for decode only: one token per row, latency.
     if constexpr (PRO != QPRO_STEP_GATE) {
-        if (a.Kp <= 64 * 4 * 8) return launch_fused_quant_rpw<T, TW, PRO, 8, NN>(a, s);
-        if (a.Kp <= 128 * 4 * 8) return launch_fused_quant_rpw<T, TW, PRO, 4, NN>(a, s);
-        // the 5632- and 6912-wide rows in front of down_proj (nothing folded in: few registers per element): two waves
-        // per row and 12 passes measured 12 % faster than four waves and 6
-        if constexpr (PRO == QPRO_PLAIN) {
-            if (a.Kp <= 128 * 4 * 12) return launch_fused_quant_rpw<T, TW, PRO, 4, NN>(a, s);
-        }
-        if (a.Kp <= 256 * 4 * 8) return launch_fused_quant_rpw<T, TW, PRO, 2, NN>(a, s);
+        // Thousands of rows: 16 to 24 elements a thread (8192 x 2048: four rows a workgroup 22 to 28 us where eight, with 32 elements
+        // a thread, took 23 to 31; 8192 x 1024: eight 13 to 17, four 14 to 19).  Fewer rows: as few rows a workgroup as reach every
+        // CU about once (320 x 2048: two rows 5.0 to 5.9 us, one 5.5 to 7.0, eight 7.4 to 9.7; 1024 x 2048: four 6.5 to 7.9, one 8.5
+        // to 10.7).  Wide rows with nothing folded in (5632, in front of down_proj) need few registers and take 48 elements.
+        if (a.M > 1280 && a.Kp <= 1024) return launch_fused_quant_rpw<T, TW, PRO, 8, NN>(a, s);
+        if (a.M > 512 && a.Kp <= (PRO == QPRO_PLAIN ? 6144 : 3072)) return launch_fused_quant_rpw<T, TW, PRO, 4, NN>(a, s);
+        if (a.M > 192 && a.Kp <= 8192) return launch_fused_quant_rpw<T, TW, PRO, 2, NN>(a, s);
     }
     return launch_fused_quant_rpw<T, TW, PRO, 1, NN>(a, s);
 }
