@@ -97,19 +97,19 @@ class BitLinear(nn.Linear):
         return F_.bitlinear(x, self.norm.weight, self.packed_weight(), bias=self.bias, eps=self.run_eps(), addend=addend,
                             prologue=prologue, epilogue=epilogue)
 
-    def _few_rows(self, x, eps):
-        """forward() without gradients on a few rows, past everything that is the same on each call; None if it is not that."""
+    def _direct(self, x, eps):
+        """forward() without gradients, past everything that is the same on each call; None where the operands ask for more."""
         own, norm = self._parameters, self.norm._parameters
         weight, norm_weight = own.get("weight"), norm.get("weight")
         if weight is None or norm_weight is None or own.get("bias") is not None or norm.get("bias") is not None:
             return None
         pw = self._pack.get(weight)
-        return L.native().bitlinear_few_rows(x, norm_weight, pw.packed, pw.wdeq, pw.seg_rows, pw.n, pw.k, eps, F_.GEMV_MAX_M)
+        return L.native().bitlinear(x, norm_weight, pw.packed, pw.wdeq, pw.seg_rows, pw.n, pw.k, eps, F_.GEMV_MAX_M)
 
     def forward(self, x):
         eps = self.run_eps()
         if not torch.is_grad_enabled():
-            out = self._few_rows(x, eps)
+            out = self._direct(x, eps)
             if out is not None:
                 return out
         return layer_norm_linear_quant_fn(x, self.norm.weight, self.norm.bias, self.weight, self.bias, eps=eps,

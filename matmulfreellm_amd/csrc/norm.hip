@@ -651,6 +651,10 @@ int mmf_rmsnorm_quant(const void* x, const void* residual, const void* weight, i
     if (!aligned16(q)) return MMF_ERR_ALIGN;
     if (K % 8 == 0 && !(aligned16(x) && aligned16(residual) && aligned16(residual_out) && aligned16(weight)))
         return MMF_ERR_ALIGN;
+    // nothing but the norm in front: the fused kernel's plain form, whose rows per workgroup follow their number
+    if (tiled && !residual && !residual_out && K % 8 == 0 && K <= 16384)
+        return mmf_rmsnorm_quant_fused(QPRO_PLAIN, x, K, nullptr, 0, nullptr, 0, nullptr, nullptr, 0.0f, weight, eps, nullptr, nullptr, q, deq,
+                                       qsum, M, K, x_dtype, weight_dtype, stream_);
     RowArgs a{};
     a.x = x; a.residual = residual; a.weight = weight; a.residual_out = residual_out;
     a.q = q; a.deq = deq; a.qsum = qsum;

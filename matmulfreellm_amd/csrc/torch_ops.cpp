@@ -41,12 +41,13 @@ struct NoGil {
     ~NoGil() { PyEval_RestoreThread(state); }
 };
 
-// ------------------------------------------------------------------------------ BitLinear, a few rows
-// (x, norm_weight, packed, wdeq, seg_rows, n, k, eps, most_rows) -> [..., n], or None where an operand is not laid out for the launch or
-// the launch refuses it (the general path then says why)
-PyObject* few_rows(PyObject*, PyObject* const* args, Py_ssize_t count) {
+// ------------------------------------------------------------------------------ BitLinear
+// (x, norm_weight, packed, wdeq, seg_rows, n, k, eps, most_rows) -> [..., n], or None where an operand is not laid out for the launches or
+// they refuse it (the general path then says why).  Up to most_rows rows run as the one fused launch, more as quantiser + contraction
+// with one allocation for what passes between them.
+PyObject* bitlinear(PyObject*, PyObject* const* args, Py_ssize_t count) {
     HANDLE_TH_ERRORS
-    if (count != 9) { PyErr_SetString(PyExc_TypeError, "bitlinear_few_rows takes 9 arguments"); return nullptr; }
+    if (count != 9) { PyErr_SetString(PyExc_TypeError, "bitlinear takes 9 arguments"); return nullptr; }
     for (int i = 0; i < 4; ++i)
         if (!THPVariable_Check(args[i])) Py_RETURN_NONE;
     const Tensor &x = THPVariable_Unpack(args[0]), &w = THPVariable_Unpack(args[1]), &packed = THPVariable_Unpack(args[2]),
@@ -57,8 +58,8 @@ PyObject* few_rows(PyObject*, PyObject* const* args, Py_ssize_t count) {
     if (PyErr_Occurred()) return nullptr;
     const int dt = dtype_of(x.scalar_type()), wdt = dtype_of(w.scalar_type());
     const int64_t total = x.numel();
-    if (dt < 0 || wdt < 0 || x.dim() < 1 || x.size(-1) != k || total == 0 || total > most * k || !x.is_cuda() || !x.is_contiguous() ||
-        !w.is_contiguous() || w.numel() != k || w.device() != x.device() || packed.device() != x.device() || k > mmf_bitlinear_gemv_max_k())
+    if (dt < 0 || wdt < 0 || x.dim() < 1 || x.size(-1) != k || total == 0 || !x.is_cuda() || !x.is_contiguous() ||
+        !w.is_contiguous() || w.numel() != k || w.device() != x.device() || packed.device() != x.device())
         Py_RETURN_NONE;
     Tensor out;
     int rc;
@@ -68,8 +69,19 @@ PyObject* few_rows(PyObject*, PyObject* const* args, Py_ssize_t count) {
         c10::SmallVector<int64_t, 6> shape(x.sizes().begin(), x.sizes().end());
         shape.back() = n;
         out = at::empty(shape, x.options().requires_grad(false));
-        rc = mmf_bitlinear_gemv(x.data_ptr(), w.data_ptr(), packed.data_ptr(), static_cast<const float*>(wdeq.data_ptr()), seg_rows, nullptr,
-                                 nullptr, out.data_ptr(), total / k, k, n, (float)eps, dt, wdt, stream_of(x));
+        const int64_t rows = total / k;
+        if (rows > most || k > mmf_bitlinear_gemv_max_k()) {
+            const int64_t codes = mmf_codes_bytes(rows, k, 1);          // a multiple of 16 bytes
+            Tensor ws = at::empty({codes + 8 * rows}, x.options().dtype(at::kByte).requires_grad(false));
+            int8_t* q = static_cast<int8_t*>(ws.data_ptr());
+            float* deq = reinterpret_cast<float*>(q + codes);
+            int* qsum = reinterpret_cast<int*>(deq + rows);
+            rc = mmf_rmsnorm_quant(x.data_ptr(), nullptr, w.data_ptr(), q, deq, qsum, nullptr, rows, k, (float)eps, dt, dt, wdt, 1, stream_of(x));
+            if (rc == 0)
+                rc = mmf_bitlinear_mfma(q, deq, qsum, packed.data_ptr(), static_cast<const float*>(wdeq.data_ptr()), seg_rows, nullptr, nullptr,
+                                        out.data_ptr(), n, rows, k, n, dt, -1, stream_of(x));
+        } else rc = mmf_bitlinear_gemv(x.data_ptr(), w.data_ptr(), packed.data_ptr(), static_cast<const float*>(wdeq.data_ptr()), seg_rows, nullptr,
+                                 nullptr, out.data_ptr(), rows, k, n, (float)eps, dt, wdt, stream_of(x));
     }
     if (rc != 0) Py_RETURN_NONE;
     return THPVariable_Wrap(std::move(out));
@@ -156,7 +168,7 @@ PyObject* scan(PyObject*, PyObject* const* args, Py_ssize_t count) {
 }
 
 PyMethodDef methods[] = {
-    {"bitlinear_few_rows", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(few_rows)), METH_FASTCALL, nullptr},
+    {"bitlinear", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(bitlinear)), METH_FASTCALL, nullptr},
     {"scan", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(scan)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "mmf_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
