@@ -204,6 +204,8 @@ int mmf_hgrn_chunk(const void* x, const void* g, const float* h0, void* o, float
 int mmf_hgrn_gate(const void* i_in, int64_t ldi, const void* f_in, int64_t ldf, const float* lower_bound,
                   const uint8_t* mask, void* x_out, void* g_out, int64_t rows, int64_t D, int dtype,
                   void* stream);
+int mmf_hgrn_gate_scan(const void* i_in, int64_t ldi, const void* f_in, int64_t ldf, const float* lower_bound, const uint8_t* mask,
+                       const float* h0, void* o, float* ht, int64_t B, int64_t T, int64_t D, int dtype, void* stream);
 int mmf_hgrn_step(const void* i_in, int64_t ldi, const void* f_in, int64_t ldf, const float* lower_bound,
                   const uint8_t* mask, float* state, void* o, int64_t rows, int64_t D, int dtype,
                   void* stream);

@@ -61,6 +61,7 @@ SIGNATURES = {
     "mmf_hgrn_chunk_workspace_bytes": (_i64, [_i64, _i64, _i64, _i32]),
     "mmf_hgrn_chunk": (_i32, [_ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _i32, _i32, _ptr, _ptr]),
     "mmf_hgrn_gate": (_i32, [_ptr, _i64, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i32, _ptr]),
+    "mmf_hgrn_gate_scan": (_i32, [_ptr, _i64, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _i32, _ptr]),
     "mmf_hgrn_step": (_i32, [_ptr, _i64, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i32, _ptr]),
     "mmf_embedding": (_i32, [_ptr, _ptr, _ptr, _i64, _i64, _i64, _i32, _ptr]),
     "mmf_embedding_record": (_i32, [_ptr, _ptr, _ptr, _i64, _i64, _i64, _ptr, _ptr, _i32, _i32, _ptr]),

@@ -52,7 +52,7 @@ struct Layout {
             ifg = take(M * 3 * p->D * e);
             o = take(M * p->D * e);
             res = take(M * p->H * e);
-            big = take(M * 2 * (p->I > p->D ? p->I : p->D) * e);    // the scan's x and g, later gate/up
+            big = take(M * p->I * e);                            // the MLP's activation
         }
         int64_t codes = 3 * mmf_codes_bytes(M, p->H, 1);
         for (int64_t k : {(int64_t)p->D, (int64_t)p->I})
@@ -143,9 +143,7 @@ int mmf_block_forward(const mmf_block* p, const void* x, void* out, int64_t B, i
     } while (0)
     auto scan = [&]() -> int {                                 // gate math, then the recurrence: o [M, D] contiguous
         if (step) return mmf_hgrn_step(i, 3 * D, f, 3 * D, lower_bound, mask, ht, o, M, D, dt, stream);
-        void *xs = big, *gs = big + M * D * e;
-        if (const int r = mmf_hgrn_gate(i, 3 * D, f, 3 * D, lower_bound, mask, xs, gs, M, D, dt, stream)) return r;
-        return mmf_hgrn_recurrent(xs, gs, h0, o, ht, B, T, D, dt, stream);
+        return mmf_hgrn_gate_scan(i, 3 * D, f, 3 * D, lower_bound, mask, h0, o, ht, B, T, D, dt, stream);
     };
     if (few_rows(p, M)) {
         const int epi = step && !mask ? E_STEP : E_PLAIN;

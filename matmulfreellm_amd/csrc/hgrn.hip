@@ -6,6 +6,7 @@
 //   mmf_hgrn_gate      : sigmoid / lower bound / swiglu / mask of
 //                        mmfreelm/layers/hgrn_bit.py:113-120 as one elementwise pass.
 //   mmf_hgrn_step      : the same gate math fused with one recurrence step (decode, T = 1).
+//   mmf_hgrn_gate_scan : gate math and recurrence of whole sequences in one launch (prompts).
 //
 // Layout: x, g, o are [BH, T, D] contiguous; a lane owns one channel d, a wave 64
 // consecutive channels (128 B per time step in bf16), a workgroup of 8 waves one
@@ -185,6 +186,172 @@ __device__ __forceinline__ void gate_math(float iv, float sf, bool has_lb, float
     xo = mmf_round_to<T>(__fdiv_rn(__fmul_rn(iv, u), __fadd_rn(1.0f, mmf_exp(-iv))));
 }
 
+// -------------------------------------------------------------------------- gate math and recurrence of a prompt in one launch
+// o = scan of the gated (x, g), x and g never leaving the CU.  A workgroup owns CPW channels of one sequence; wave 0 runs the
+// recurrence, the other 15 feed it: they load raw i and f two tiles ahead, do the gate math of the next tile into LDS (float2 per
+// step and channel) and round and store the outputs of the tile before, while wave 0 walks the current tile -- per step one LDS
+// read, multiply, add, LDS write -- at raised priority.  One LDS-only barrier per tile (a full one would wait for the loads ahead).
+// The vector units are the bound: the exact exp, sigmoid and divide are ~85 issue slots an element, which a wave walking time alone
+// would put behind the recurrence; with 16-channel workgroups even one sequence reaches 64 to 128 CUs.  CPW is the narrowest that
+// leaves at most two workgroups per CU (wider blocks have longer rows to load, 32 bytes at 16 channels; the four blocks that share
+// a 128-byte line run on one XCD).  Against gate and scan as two launches, bf16: 1 x 77 x 1024 9.4 -> 5.1 us, 3 x 459 x 2048
+// 26 -> 16, 2 x 1001 x 2048 34 -> 23, 8 x 2048 x 2048 103 -> 81 (twice or half as many workgroups: 93, 96).
+struct GateScanArgs {
+    const void* i; const void* f;       // rows [B * T, D], row strides ldi, ldf
+    const float* lb; const uint8_t* mask;
+    const float* h0; float* ht;         // [B, D]
+    void* o;                            // [B * T, D]
+    int64_t ldi, ldf, D;
+    int T;
+};
+__device__ __forceinline__ void lds_only_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+template <typename T, int CPW, int PASS>
+__global__ __launch_bounds__(1024) void hgrn_gate_scan_kernel(GateScanArgs a) {
+    constexpr int NP = 15, SPW = 64 / CPW, TT = NP * SPW * PASS, U = 10;   // steps of a tile: 120 (60), 60 or 30
+    static_assert(TT % U == 0, "the recurrence walks a full tile in whole groups");
+    __shared__ float2 gx[2][TT * CPW];
+    __shared__ float hb[2][TT * CPW];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    unsigned cb = blockIdx.x;
+    if (CPW == 16 && gridDim.x % 32 == 0) cb = (cb & ~31u) + (cb & 7u) * 4 + ((cb >> 3) & 3u);
+    if (CPW == 32 && gridDim.x % 16 == 0) cb = (cb & ~15u) + (cb & 7u) * 2 + ((cb >> 3) & 1u);
+    const int c = lane & (CPW - 1), sub = lane / CPW;
+    const int64_t d = (int64_t)cb * CPW + c;
+    const bool active = d < a.D;
+    const int64_t dd = active ? d : 0, r0 = (int64_t)blockIdx.y * a.T;
+    const int NT = (a.T + TT - 1) / TT;
+
+    if (wave == 0) {
+        __builtin_amdgcn_s_setprio(3);
+        float h = a.h0 && active ? a.h0[(int64_t)blockIdx.y * a.D + dd] : 0.0f;
+        lds_only_barrier();                                     // tile 0 is there
+        for (int k = 0; k < NT; ++k) {
+            const int n = a.T - k * TT < TT ? a.T - k * TT : TT;
+            const float2* src = gx[k & 1] + c;
+            float* dst = hb[k & 1] + c;
+            float2 cur[U], nxt[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) cur[u] = src[u * CPW];
+            int j = 0;
+            for (; j + U <= n; j += U) {
+                const int jn = j + 2 * U <= TT ? j + U : j;     // the last group re-reads itself
+#pragma unroll
+                for (int u = 0; u < U; ++u) nxt[u] = src[(jn + u) * CPW];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    h = __fadd_rn(__fmul_rn(cur[u].x, h), cur[u].y);
+                    dst[(j + u) * CPW] = h;
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) cur[u] = nxt[u];
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {                       // what is left of the last tile: the group read ahead holds it
+                if (j + u < n) {
+                    h = __fadd_rn(__fmul_rn(cur[u].x, h), cur[u].y);
+                    dst[(j + u) * CPW] = h;
+                }
+            }
+            lds_only_barrier();
+        }
+        if (a.ht && active && lane < CPW) a.ht[(int64_t)blockIdx.y * a.D + d] = h;
+        return;
+    }
+
+    const int p = wave - 1;
+    const T* ip = static_cast<const T*>(a.i);
+    const T* fp = static_cast<const T*>(a.f);
+    T* op = static_cast<T*>(a.o);
+    const bool has_lb = a.lb != nullptr;
+    const float lb = has_lb ? a.lb[dd] : 0.0f;
+    T ir[2][PASS], fr[2][PASS];
+    uint8_t mr[2][PASS];
+    auto at = [&](int q) __attribute__((always_inline)) { return (q * NP + p) * SPW + sub; };   // step of a tile
+    uint32_t oi[PASS], of[PASS];                                // offsets into a tile's rows (the launcher: they fit)
+#pragma unroll
+    for (int q = 0; q < PASS; ++q) {
+        oi[q] = (uint32_t)at(q) * (uint32_t)a.ldi + (uint32_t)dd;
+        of[q] = (uint32_t)at(q) * (uint32_t)a.ldf + (uint32_t)dd;
+    }
+    auto load = [&](int k, auto S) __attribute__((always_inline)) {
+        constexpr int s = decltype(S)::value;
+        const int kk = k < NT ? k : NT - 1, last = a.T - 1 - kk * TT;
+        const int64_t row = r0 + (int64_t)kk * TT;
+        const T* it = ip + row * a.ldi;
+        const T* ft = fp + row * a.ldf;
+        const uint8_t* mt = a.mask ? a.mask + row : nullptr;
+#pragma unroll
+        for (int q = 0; q < PASS; ++q) {
+            if (last >= TT - 1) {
+                ir[s][q] = it[oi[q]];
+                fr[s][q] = ft[of[q]];
+                mr[s][q] = mt ? mt[at(q)] : (uint8_t)1;
+            } else {                                            // steps past the end: the last one once more, never used
+                const uint32_t t = (uint32_t)(at(q) < last ? at(q) : last);
+                ir[s][q] = it[t * (uint32_t)a.ldi + (uint32_t)dd];
+                fr[s][q] = ft[t * (uint32_t)a.ldf + (uint32_t)dd];
+                mr[s][q] = mt ? mt[t] : (uint8_t)1;
+            }
+        }
+    };
+    auto gates = [&](int k, auto S) __attribute__((always_inline)) {
+        constexpr int s = decltype(S)::value;
+        float fv[PASS], sf[PASS];
+#pragma unroll
+        for (int q = 0; q < PASS; ++q) fv[q] = mmf_to_float(fr[s][q]);
+        mmf_sigmoid_n<PASS>(fv, sf);
+#pragma unroll
+        for (int q = 0; q < PASS; ++q) {
+            float xo, go;
+            gate_math<T>(mmf_to_float(ir[s][q]), sf[q], has_lb, lb, xo, go);
+            if (mr[s][q] == 0) xo = 0.0f;
+            gx[k & 1][(q * NP + p) * 64 + lane] = make_float2(go, xo);
+        }
+    };
+    auto put = [&](int k) __attribute__((always_inline)) {
+        T* ot = op + (r0 + (int64_t)k * TT) * a.D;
+        const int n = a.T - k * TT;
+#pragma unroll
+        for (int q = 0; q < PASS; ++q) {
+            const float h = hb[k & 1][(q * NP + p) * 64 + lane];
+            if (at(q) < n && active) ot[(uint32_t)at(q) * (uint32_t)a.D + (uint32_t)d] = mmf_from_float<T>(h);
+        }
+    };
+    load(0, IntC<0>{});
+    load(1, IntC<1>{});
+    gates(0, IntC<0>{});
+    load(2, IntC<0>{});
+    lds_only_barrier();
+    auto turn = [&](int k, auto S) __attribute__((always_inline)) {   // wave 0 walks tile k: store tile k - 1, prepare tile k + 1 (set S)
+        if (k > 0) put(k - 1);
+        if (k + 1 < NT) {
+            gates(k + 1, S);
+            load(k + 3, S);
+        }
+        lds_only_barrier();
+    };
+    for (int k = 0; k < NT; k += 2) {
+        turn(k, IntC<1>{});
+        if (k + 1 < NT) turn(k + 1, IntC<0>{});
+    }
+    put(NT - 1);
+}
+
+template <typename T>
+int launch_gate_scan(const GateScanArgs& a, int64_t B, hipStream_t s) {
+    const int64_t D = a.D;
+    auto grid = [&](int64_t cpw) { return dim3((unsigned)mmf_ceil_div(D, cpw), (unsigned)B); };
+    if (B * mmf_ceil_div(D, (int64_t)16) <= 512) {
+        // short sequences: half the steps a tile, so that the recurrence starts sooner
+        if (a.T <= 512) hgrn_gate_scan_kernel<T, 16, 1><<<grid(16), 1024, 0, s>>>(a);
+        else hgrn_gate_scan_kernel<T, 16, 2><<<grid(16), 1024, 0, s>>>(a);
+    } else if (B * mmf_ceil_div(D, (int64_t)32) <= 512) hgrn_gate_scan_kernel<T, 32, 2><<<grid(32), 1024, 0, s>>>(a);
+    else hgrn_gate_scan_kernel<T, 64, 2><<<grid(64), 1024, 0, s>>>(a);
+    MMF_CHECK_LAUNCH();
+    return 0;
+}
+
 // One kernel for both forms: STEP = false writes (x, g); STEP = true runs one recurrence step on the
 // fp32 state in place and writes o.  grid = (ceil(D / 1024), rows): a thread owns 4 consecutive
 // channels of one row, so there is no index division and the loads are 8- / 16-byte vectors
@@ -309,6 +476,23 @@ int mmf_hgrn_recurrent(const void* x, const void* g, const float* h0, void* o, f
         case MMF_F32: return launch_scan<float>(x, g, h0, o, ht, BH, T, D, stream);
         case MMF_BF16: return launch_scan<bf16_t>(x, g, h0, o, ht, BH, T, D, stream);
         case MMF_F16: return launch_scan<f16_t>(x, g, h0, o, ht, BH, T, D, stream);
+    }
+    return MMF_ERR_ARG;
+}
+
+int mmf_hgrn_gate_scan(const void* i_in, int64_t ldi, const void* f_in, int64_t ldf, const float* lower_bound, const uint8_t* mask,
+                       const float* h0, void* o, float* ht, int64_t B, int64_t T, int64_t D, int dtype, void* stream_) {
+    hipStream_t stream = static_cast<hipStream_t>(stream_);
+    if (B < 0 || T < 0 || D <= 0 || ldi < D || ldf < D || B > 65535) return MMF_ERR_ARG;
+    if (B == 0 || T == 0) return 0;
+    if (!i_in || !f_in || !o) return MMF_ERR_ARG;
+    if (T > (1 << 30) || ldi > (1 << 22) || ldf > (1 << 22)) return MMF_ERR_WIDE;   // a tile of 120 rows within 32-bit offsets
+    GateScanArgs a{};
+    a.i = i_in; a.f = f_in; a.lb = lower_bound; a.mask = mask; a.h0 = h0; a.ht = ht; a.o = o; a.ldi = ldi; a.ldf = ldf; a.D = D; a.T = (int)T;
+    switch (dtype) {
+        case MMF_F32: return launch_gate_scan<float>(a, B, stream);
+        case MMF_BF16: return launch_gate_scan<bf16_t>(a, B, stream);
+        case MMF_F16: return launch_gate_scan<f16_t>(a, B, stream);
     }
     return MMF_ERR_ARG;
 }
