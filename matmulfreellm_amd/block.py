@@ -66,8 +66,8 @@ class _Structure:
         if (D % 32 or I % 32 or H % 8 or max(H, D, I) > 8192 or attn.num_heads * attn.head_dim != D
                 or any(p.run_eps() != projs[0].run_eps() for p in projs[:3])):
             return
-        self.numbers = ([(m, "eps", m.eps) for m in norms + tuple(p.norm for p in projs)]
-                        + [(p, "fused_eps", p.fused_eps) for p in projs])
+        self.numbers = ([(m.__dict__, "eps", m.eps) for m in norms + tuple(p.norm for p in projs)]
+                        + [(p.__dict__, "fused_eps", p.fused_eps) for p in projs])
         self.eps = dict(zip(("attn_eps", "mlp_eps", "g_eps", "ifg_eps", "o_eps", "gate_eps", "down_eps"),
                             [m.eps for m in norms] + [p.run_eps() for p in projs[:1] + projs[3:]]))
         self.attn, self.projs, self.norms = attn, projs, norms
@@ -75,19 +75,7 @@ class _Structure:
         self.fits = True
 
     def current(self):
-        for d in self.dicts:
-            if not _untouched(d):
-                return False
-        for d, k, c in self.children:
-            if d.get(k) is not c:
-                return False
-        for d, k in self.absent:
-            if d.get(k) is not None:
-                return False
-        for m, k, v in self.numbers:
-            if getattr(m, k) != v:
-                return False
-        return True
+        return L.native().structure_holds(self.dicts, self.children, self.absent, self.numbers)
 
     def norm_weights(self):
         """attn_norm, mlp_norm, g_norm, then the inner norms of i, f, g, o, gate, down."""
@@ -161,9 +149,8 @@ class BlockPlan:
     def current(self):
         if not self.structure.current():
             return False
-        for d, k, p, version, address in self.params:
-            if d.get(k) is not p or p._version != version or p.data_ptr() != address:
-                return False
+        if not L.native().parameters_hold(self.params):
+            return False
         for pack, pw in self.packed:
             if pack.pw is not pw:
                 return False
