@@ -284,7 +284,9 @@ class HGRNBitModel(HGRNBitPreTrainedModel):
         x = x.contiguous()
         with L.on(dev):
             stream, ws = L.stream(), native.workspace(plan, B * T)
-            spare, dims = None, plan.dims
+            # `own`: x is a buffer allocated here that only native calls have seen; `spare`: one of those that is read no more.  What a
+            # module was given or has returned may be held by a hook or by the caller: it is never written.
+            spare, own, dims = None, False, plan.dims
             for i, layer in enumerate(self.layers):
                 if output_hidden_states:
                     all_hidden_states += (x,)
@@ -303,6 +305,7 @@ class HGRNBitModel(HGRNBitPreTrainedModel):
                     seen = past_key_values._seen_tokens if use_cache else 0
                     x = layer(x, attention_mask=attention_mask, past_key_values=past_key_values, use_cache=use_cache,
                               output_attentions=False, lower_bound=lb)[0].contiguous()
+                    own = False
                     if use_cache:
                         past_key_values._seen_tokens = seen
                     continue
@@ -310,9 +313,8 @@ class HGRNBitModel(HGRNBitPreTrainedModel):
                 ht = state.data_ptr() if state is not None else None
                 native.forward(plan, x.data_ptr(), out.data_ptr(), B, T, lb.data_ptr() if lb is not None and i > 0 else None,
                                L.ptr(mask), ht if fresh is None else None, ht, ws.data_ptr(), stream)
-                # the input's buffer serves the next block, unless somebody else holds it
-                spare = x if i > 0 and not output_hidden_states else None
-                x = out
+                spare = x if own and not output_hidden_states else None
+                x, own = out, True
         if use_cache:
             past_key_values._seen_tokens += 1
         return x, past_key_values, all_hidden_states

@@ -7,10 +7,10 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-def build(dev, dtype, hidden, trained):
+def build(dev, dtype, hidden, trained, layers=3):
     import matmulfreellm_amd as mm
     torch.manual_seed(3)
-    model = mm.HGRNBitForCausalLM(mm.HGRNBitConfig(vocab_size=500, hidden_size=hidden, num_hidden_layers=3, bos_token_id=None,
+    model = mm.HGRNBitForCausalLM(mm.HGRNBitConfig(vocab_size=500, hidden_size=hidden, num_hidden_layers=layers, bos_token_id=None,
                                                    eos_token_id=None))
     with torch.no_grad():
         for name, p in model.named_parameters():
@@ -46,6 +46,25 @@ def test_native_block_equals_the_module_path(dev, dtype, hidden, trained):
                     h.remove()
             for i, (a, r) in enumerate(zip(got["native"], got["modules"])):
                 assert torch.equal(a, r), (b, t, masked, i)
+
+
+@pytest.mark.parametrize("hooked", [(0,), (1,), (2,), (3,), (4,), (1, 2), (1, 3)])
+def test_what_a_hook_has_kept_is_not_written(dev, hooked):
+    """Forward hooks on some layers keep their inputs and outputs (activation capture): the blocks behind them, native calls that
+    reuse each other's buffers, leave those tensors as the hooks saw them."""
+    model = build(dev, torch.bfloat16, 160, True, layers=6)
+    ids = torch.randint(0, 500, (2, 20), device=dev)
+    with torch.no_grad():
+        want = model(input_ids=ids, output_hidden_states=True).hidden_states
+        kept = []
+        for i in hooked:
+            model.model.layers[i].register_forward_hook(lambda m, args, out, i=i: kept.append((i, args[0], out[0])))
+        logits = model(input_ids=ids).logits
+        again = model(input_ids=ids, output_hidden_states=True)
+    assert [i for i, _, _ in kept] == list(hooked) * 2
+    for i, x, y in kept[:len(hooked)]:
+        assert torch.equal(x, want[i]) and torch.equal(y, want[i + 1]), i
+    assert torch.equal(logits, again.logits)
 
 
 def test_a_written_or_replaced_parameter_is_seen(dev):
