@@ -182,8 +182,9 @@ int mmf_bitlinear_mfma_swiglu(const int8_t* codes_tiled, const float* deq, const
  * mmf_hgrn_chunk replaces chunk_hgrn, mmfreelm/ops/hgrn/chunk.py:287-296 (kernels :49-116):
  *   h = exp(g)*h + x with g the log decay, evaluated in register blocks as the reference's chunked form is per chunk:
  *   a scan from zero with the running product E of the gates, then o_t += E_t * (state at the block's entry).  One pass over
- *   x and g (no fp32 [B,H,T,D] scratch tensors); `chunk` (1 <= chunk <= 64; the reference fixes 128) changes rounding at
- *   most.  A long sequence of few channels is also cut into time segments that run in parallel (a first launch leaves each
+ *   x and g (no fp32 [B,H,T,D] scratch tensors); `chunk` (1 <= chunk <= 64; the reference fixes 128) decides
+ *   from which length on a sequence may be cut (see below) and changes the result by rounding at most.  A long sequence of few
+ *   channels is also cut into time segments that run in parallel (a first launch leaves each
  *   segment's (decay product, end state) pair in `workspace`, mmf_hgrn_chunk_workspace_bytes(BH, T, D, chunk) bytes,
  *   4-byte aligned, may be NULL when that is 0).
  *   exp is the hardware one: results agree with the reference's within rounding, not bit for bit.

@@ -321,6 +321,13 @@ Plan plan(int64_t BH, int64_t Tlen, int64_t D, int blk, bool split) {
     p.NS = (int)mmf_ceil_div(Tlen, p.seg_len);
     return p;
 }
+// The forward cuts time only where few columns meet eight of the blocks that `chunk` makes (whole chunks, at most 8 and at most 64
+// steps): there, and nowhere else, mmf_hgrn_chunk_workspace_bytes asks for a workspace, also where plan() then leaves the sequence whole.
+bool fwd_takes_workspace(int64_t BH, int64_t Tlen, int64_t D, int chunk) {
+    const int64_t block = (64 / chunk > 8 ? 8 : 64 / chunk) * (int64_t)chunk;
+    return BH * mmf_ceil_div(D, 64) < 256 && Tlen >= 8 * block;
+}
+Plan fwd_plan(int64_t BH, int64_t Tlen, int64_t D, int chunk) { return plan(BH, Tlen, D, kFwdBlk, fwd_takes_workspace(BH, Tlen, D, chunk)); }
 int64_t pair_bytes(const Plan& p, int64_t BH, int64_t D) { return p.NS > 1 ? BH * p.NS * 2 * D * (int64_t)sizeof(float) : 0; }
 // The kernels address a block of at most 64 rows with 32-bit offsets and count blocks in an int.
 bool fits(int64_t Tlen, int64_t D, int dtype) {
@@ -344,8 +351,8 @@ int launch_fwd_ls(const Plan& p, const T* x, const T* g, const float* h0, T* o, 
 }
 template <typename T>
 int launch_fwd(const void* x, const void* g, const float* h0, void* o, float* ht, float* agg, int64_t BH, int64_t Tlen, int64_t D,
-               hipStream_t s) {
-    const Plan p = plan(BH, Tlen, D, kFwdBlk, true);
+               int chunk, hipStream_t s) {
+    const Plan p = fwd_plan(BH, Tlen, D, chunk);
     if (p.NS > 1 && !agg) return MMF_ERR_ARG;
     const T* xp = static_cast<const T*>(x);
     const T* gp = static_cast<const T*>(g);
@@ -392,15 +399,12 @@ __global__ __launch_bounds__(256) void state_init_kernel(const float* __restrict
 
 extern "C" {
 
-// chunk: the reference's chunk length.  The result does not depend on it beyond rounding: the register blocks play its part.
-// A workspace is asked for wherever few columns meet eight of the blocks that `chunk` makes (whole chunks, at most 8 and at
-// most 64 steps), which covers every shape that plan() cuts.
+// chunk: the reference's chunk length.  The register blocks play its part: it decides from which length on a sequence may be cut
+// and changes the result by rounding at most.
 int64_t mmf_hgrn_chunk_workspace_bytes(int64_t BH, int64_t T, int64_t D, int chunk) {
     if (BH <= 0 || T <= 0 || D <= 0 || chunk < 1 || chunk > 64) return 0;
-    const int64_t block = (64 / chunk > 8 ? 8 : 64 / chunk) * (int64_t)chunk;
-    if (BH * mmf_ceil_div(D, 64) >= 256 || T < 8 * block) return 0;
-    const Plan p = plan(BH, T, D, kFwdBlk, true);
-    return BH * p.NS * 2 * D * (int64_t)sizeof(float);
+    if (!fwd_takes_workspace(BH, T, D, chunk)) return 0;
+    return BH * fwd_plan(BH, T, D, chunk).NS * 2 * D * (int64_t)sizeof(float);
 }
 
 int mmf_hgrn_chunk(const void* x, const void* g, const float* h0, void* o, float* ht, int64_t BH, int64_t T, int64_t D,
@@ -419,9 +423,9 @@ int mmf_hgrn_chunk(const void* x, const void* g, const float* h0, void* o, float
     if (!fits(T, D, dtype)) return MMF_ERR_WIDE;
     float* agg = static_cast<float*>(workspace);
     switch (dtype) {
-        case MMF_F32: return launch_fwd<float>(x, g, h0, o, ht, agg, BH, T, D, stream);
-        case MMF_BF16: return launch_fwd<bf16_t>(x, g, h0, o, ht, agg, BH, T, D, stream);
-        case MMF_F16: return launch_fwd<f16_t>(x, g, h0, o, ht, agg, BH, T, D, stream);
+        case MMF_F32: return launch_fwd<float>(x, g, h0, o, ht, agg, BH, T, D, chunk, stream);
+        case MMF_BF16: return launch_fwd<bf16_t>(x, g, h0, o, ht, agg, BH, T, D, chunk, stream);
+        case MMF_F16: return launch_fwd<f16_t>(x, g, h0, o, ht, agg, BH, T, D, chunk, stream);
     }
     return MMF_ERR_ARG;
 }

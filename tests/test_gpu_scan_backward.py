@@ -29,3 +29,30 @@ def test_scan_backward_split(dev, bhtd, log):
     for name, a, r in zip(("dx", "dg"), got, want):
         err = ((a.cpu() - r).abs().max() / r.abs().max().clamp_min(1e-30)).item()
         assert err < 2e-5, (name, err)
+
+
+@pytest.mark.parametrize("t", [64, 447, 448, 511, 512, 513])
+@pytest.mark.parametrize("bh,d", [(1, 64), (63, 33), (64, 33)])
+@pytest.mark.parametrize("chunk", [1, 7, 64])
+def test_chunked_scan_where_the_time_axis_begins_to_be_cut(dev, t, bh, d, chunk):
+    """Lengths on both sides of the first cut for every chunk length (448 is where two segments of four blocks fit, 8 blocks of
+    whole chunks where a workspace is asked for) and of the number of columns above which nothing is cut; forward, final state
+    and gradients against the sequential form in double precision.  An fp32 pass adds at most a few roundings per step to values
+    that the gates damp: 2e-5 of the largest value, as the backward's bound above."""
+    import matmulfreellm_amd as mm
+    torch.manual_seed(t + bh)
+    g = torch.nn.functional.logsigmoid(torch.randn(1, bh, t, d) + 2)
+    x, do, h0 = torch.randn(1, bh, t, d), torch.randn(1, bh, t, d), torch.randn(1, bh, d)
+    leaves = [v.double().requires_grad_() for v in (x, g)]
+    h, steps = h0.double(), []
+    for i in range(t):
+        h = leaves[1][:, :, i].exp() * h + leaves[0][:, :, i]
+        steps.append(h)
+    want_o = torch.stack(steps, 2)
+    want = [want_o, h, *torch.autograd.grad(want_o, leaves, do.double())]
+    mine = [v.to(dev).requires_grad_() for v in (x, g)]
+    o, last = mm.chunk_hgrn(*mine, h0.to(dev), output_final_state=True, chunk_size=chunk)
+    got = [o, last, *torch.autograd.grad(o, mine, do.to(dev))]
+    for name, a, r in zip(("o", "state", "dx", "dg"), got, want):
+        err = ((a.detach().cpu().double() - r).abs().max() / r.abs().max()).item()
+        assert err < 2e-5, (name, err)
