@@ -358,10 +358,12 @@ int mmf_sample_top_p_recorded(const void* logits, int64_t ld, int64_t rows, int6
  *     K = H, N = vocabulary size); the launch then also writes the logits [N] (activation dtype), and the greedy token
  *     (lowest index of the largest logit; NaNs never win) to *tok_out, which may be the buffer `tok` points to.
  *     am_words: 256 uint64 scratch words, zero-initialised once.  With head == null the three pointers are ignored.
- *   Requires D == H, H, I multiples of 128, H <= 4096, I <= 8192 (else MMF_ERR_WIDE), 16-bit activations (dtype 1 or 2),
- *   batch 1, norm weights of magnitude below 2^40.  Calls on one device must not overlap (they share the scratch words). */
+ *   Requires D == H, H, I multiples of 128, H <= 4096, I <= 8192 and a table and buffers that fit a CU's LDS (else MMF_ERR_WIDE;
+ *   mmf_decode_layers_fits(norms, n_layers, H, D, I) is 1 where all of that holds), 16-bit activations (dtype 1 or 2), batch 1,
+ *   norm weights of magnitude below 2^40.  Calls on one device must not overlap (they share the scratch words). */
 int mmf_decode_layers_phase_bytes(void);
 int mmf_decode_layers_copies(void);
+int mmf_decode_layers_fits(int norms, int n_layers, int H, int D, int I);
 int64_t mmf_decode_layers_words(int H, int D, int I);
 int mmf_decode_layers(const void* phases, int n_layers, const void* table, const int64_t* tok, int64_t vocab, uint32_t* words,
                       void* h_out, const void* head, void* logits, uint64_t* am_words, int64_t* tok_out, uint32_t* epoch, int* err,

@@ -40,6 +40,7 @@ SIGNATURES = {
                                        _ptr, _i64, _i64, _i32, _i32, _ptr]),
     "mmf_decode_layers_phase_bytes": (_i32, []),
     "mmf_decode_layers_copies": (_i32, []),
+    "mmf_decode_layers_fits": (_i32, [_i32, _i32, _i32, _i32, _i32]),
     "mmf_decode_layers_words": (_i64, [_i32, _i32, _i32]),
     "mmf_decode_layers": (_i32, [_ptr, _i32, _ptr, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr,
                                  _i32, _i32, _i32, _i32, _i32, _ptr]),

@@ -916,10 +916,14 @@ int launch_one(const LayersArgs& a, size_t lds, hipStream_t s) {
     return 0;
 }
 
-template <typename T, bool TRACE, int NORMS>
-int launch_layers(LayersArgs a, hipStream_t s) {
+// Where a launch keeps things in LDS, and how much of it that takes; false where the model does not fit a CU.  Three inner norms behind
+// i, f and g triple the codes of a row and the staged norm weights: 24 layers of 2560 / 6912 take 145 KiB with one norm and 161 with
+// three.  mmf_decode_layers_fits answers with the same rule, so that a caller can decide for the launch chain beforehand.
+constexpr size_t kLdsOfCU = 160 * 1024;
+bool lay_out(LayersArgs& a, int norms, size_t& lds) {
+    if (a.H > 4096 || a.I > 8192 || a.n_layers > kMaxLayers) return false;
     const int kmax = a.H > a.I ? a.H : a.I;
-    a.nqmax = quads_of(kmax) > NORMS * quads_of(a.H) ? quads_of(kmax) : NORMS * quads_of(a.H);
+    a.nqmax = quads_of(kmax) > norms * quads_of(a.H) ? quads_of(kmax) : norms * quads_of(a.H);
     // weight loads (1 KiB each) per wave a link kind needs when all its row-groups are resident: buffer A serves i/f/g
     // and gate/up, buffer B o_proj and down_proj; the lm_head takes what they hold, pass by pass
     const int nqh = quads_of(a.H), nqi = quads_of(a.I);
@@ -927,12 +931,17 @@ int launch_layers(LayersArgs a, hipStream_t s) {
     const int ifg = ngh * 3 * nqh, gate = ngi * 2 * nqh, o = ngh * nqh, down = ngh * nqi;
     a.itemsA = ifg > gate ? ifg : gate;
     a.itemsB = o > down ? o : down;
-    if (a.itemsA > 16 || a.itemsB > 16 || ngh > 2 || ngi * 2 > kItems) return MMF_ERR_WIDE;
+    if (a.itemsA > 16 || a.itemsB > 16 || ngh > 2 || ngi * 2 > kItems) return false;
     const uint32_t tab = (uint32_t)mmf_round_up((4 * a.n_layers + 1) * (int64_t)sizeof(Phase), 16);
     a.off_q = tab;
-    a.off_nrm = a.off_q + (uint32_t)mmf_round_up(kmax > NORMS * a.H ? kmax : NORMS * a.H, 16);
+    a.off_nrm = a.off_q + (uint32_t)mmf_round_up(kmax > norms * a.H ? kmax : norms * a.H, 16);
     a.off_w = a.off_nrm + 2u * kNW * (uint32_t)a.nqmax * 1024u;
-    const size_t lds = a.off_w + (size_t)kNW * (a.itemsA + a.itemsB) * 1024u;
+    lds = a.off_w + (size_t)kNW * (a.itemsA + a.itemsB) * 1024u;
+    return lds + sizeof(Small) <= kLdsOfCU;
+}
+
+template <typename T, bool TRACE, int NORMS>
+int launch_layers(const LayersArgs& a, size_t lds, hipStream_t s) {
     if (a.H == 2048 && a.I == 5632) return launch_one<T, StaticShape<2048, 5632>, TRACE, NORMS>(a, lds, s);
     if (a.H == 1024 && a.I == 2816) return launch_one<T, StaticShape<1024, 2816>, TRACE, NORMS>(a, lds, s);
     if (a.H == 2560 && a.I == 6912) return launch_one<T, StaticShape<2560, 6912>, TRACE, NORMS>(a, lds, s);
@@ -953,29 +962,31 @@ int decode_layers_entry(const void* phases, int n_layers, const void* table, con
     if (head && (!logits || !am_words || !tok_out)) return MMF_ERR_ARG;
     if (H % 128 != 0 || D != H || I % 128 != 0) return MMF_ERR_ARG;      // rows are whole k-blocks: no ragged tail in a link
     if (dtype != MMF_BF16 && dtype != MMF_F16) return MMF_ERR_ARG;        // a tagged word carries a 16-bit value
-    if (H > 4096 || I > 8192 || n_layers > kMaxLayers) return MMF_ERR_WIDE;
+    LayersArgs a{};
+    a.H = H; a.D = D; a.I = I; a.n_layers = n_layers;
+    size_t lds = 0;
+    if (!lay_out(a, norms, lds)) return MMF_ERR_WIDE;
     for (const void* p : {(const void*)words, (const void*)table, (const void*)h_out, phases, head})
         if (reinterpret_cast<uintptr_t>(p) & 15u) return MMF_ERR_ALIGN;
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         return MMF_ERR_ARG;
     if (cus < kWGs) return MMF_ERR_ARG;                                       // the resident grid needs one CU per workgroup
-    LayersArgs a{};
-    a.phases = static_cast<const Phase*>(phases); a.n_layers = n_layers; a.table = table; a.tok = tok; a.vocab = vocab;
+    a.phases = static_cast<const Phase*>(phases); a.table = table; a.tok = tok; a.vocab = vocab;
     a.words = words; a.h_out = h_out; a.head = static_cast<const Phase*>(head); a.logits = logits; a.am_words = am_words;
     a.tok_out = tok_out; a.epoch = epoch; a.err = err; a.trace = reinterpret_cast<long long*>(trace);
-    a.H = H; a.D = D; a.I = I; a.spin = spin;
+    a.spin = spin;
     a.history = history; a.pos = pos; a.cap = cap;
     for (int k = 0; k < 5; ++k) a.delay[k] = delay[k];
     if (trace) {
         switch (dtype) {
-            case MMF_BF16: return launch_layers<bf16_t, true, 1>(a, stream);
-            case MMF_F16: return launch_layers<f16_t, true, 1>(a, stream);
+            case MMF_BF16: return launch_layers<bf16_t, true, 1>(a, lds, stream);
+            case MMF_F16: return launch_layers<f16_t, true, 1>(a, lds, stream);
         }
     } else {
         switch (dtype) {
-            case MMF_BF16: return norms == 3 ? launch_layers<bf16_t, false, 3>(a, stream) : launch_layers<bf16_t, false, 1>(a, stream);
-            case MMF_F16: return norms == 3 ? launch_layers<f16_t, false, 3>(a, stream) : launch_layers<f16_t, false, 1>(a, stream);
+            case MMF_BF16: return norms == 3 ? launch_layers<bf16_t, false, 3>(a, lds, stream) : launch_layers<bf16_t, false, 1>(a, lds, stream);
+            case MMF_F16: return norms == 3 ? launch_layers<f16_t, false, 3>(a, lds, stream) : launch_layers<f16_t, false, 1>(a, lds, stream);
         }
     }
     return MMF_ERR_ARG;
@@ -990,6 +1001,14 @@ int mmf_decode_layers_phase_bytes(void) { return (int)sizeof(Phase); }
 int64_t mmf_decode_layers_words(int H, int D, int I) { return (int64_t)kRep * (3 * (int64_t)H + 2 * (int64_t)D + (int64_t)I); }
 
 int mmf_decode_layers_copies(void) { return kRep; }
+
+int mmf_decode_layers_fits(int norms, int n_layers, int H, int D, int I) {
+    if ((norms != 1 && norms != 3) || n_layers <= 0 || H <= 0 || I <= 0 || D != H || H % 128 != 0 || I % 128 != 0) return 0;
+    LayersArgs a{};
+    a.H = H; a.D = D; a.I = I; a.n_layers = n_layers;
+    size_t lds = 0;
+    return lay_out(a, norms, lds) ? 1 : 0;
+}
 
 int mmf_decode_layers_norms(int norms, const void* phases, int n_layers, const void* table, const int64_t* tok, int64_t vocab, uint32_t* words,
                       void* h_out, const void* head, void* logits, uint64_t* am_words, int64_t* tok_out, uint32_t* epoch, int* err,

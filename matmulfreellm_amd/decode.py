@@ -130,6 +130,8 @@ class DecodeEngine:
         self.gemv = B <= F_.GEMV_MAX_M
         self.fused = fuse and self._can_fuse()
         self.fused_mfma = fuse and self._can_fuse_mfma()
+        # a layer whose i, f and g have inner norms of their own: every layer of the resident launch then has three (equal ones repeated)
+        self.norms = 3 if any(ent["norms"] is not None for ent in self.layers) else 1
         # resident=None: the one-launch layer chain whenever the model fits it; True insists; False never
         self.resident = self.fused and resident is not False and self._can_run_resident()
         if resident and not self.resident:
@@ -193,14 +195,12 @@ class DecodeEngine:
     def _can_run_resident(self):
         props = torch.cuda.get_device_properties(self.dev)
         return (self.B == 1 and self.dtype in (torch.bfloat16, torch.float16) and self.final_norm.dtype == self.dtype
-                and self.D == self.H and self.H % 128 == 0 and self.I % 128 == 0 and self.H <= 4096 and self.I <= 8192
+                and bool(self.lib.mmf_decode_layers_fits(self.norms, self.L, self.H, self.D, self.I))
                 and props.multi_processor_count >= 256)
 
     def _build_resident(self):
         H, D, I = self.H, self.D, self.I
         assert self.lib.mmf_decode_layers_phase_bytes() == ctypes.sizeof(_Phase)
-        # a layer whose i, f and g have inner norms of their own: every layer then runs with three (equal ones repeated)
-        self.norms = 3 if any(ent["norms"] is not None for ent in self.layers) else 1
         table = (_Phase * (4 * self.L + 1))()            # the last record is the final norm + lm_head
 
         def fill(rec, w1, eps1, pw_nw_eps, k, n, lb=None, state=None):

@@ -209,6 +209,17 @@ def test_rejected_shapes_and_pointers_return_their_code_before_any_launch():
                                  None) == -1                      # a head record without its logits buffer
     assert lib.mmf_decode_layers_traced(P, 2, P, P, 1000, P, P, None, None, None, None, P, P, None, 512, 512, 1536, 100, 6, 1,
                                         None) == -1               # the traced form needs its trace buffer
+    # a model whose table and buffers outgrow a CU's LDS is refused, and the engine can ask beforehand: one norm behind i, f and g, or three
+    norms = lambda n, layers, h, i: lib.mmf_decode_layers_norms(n, P, layers, P, P, 1000, P, P, None, None, None, None, P, P + 4, None, None, 0,
+                                                                h, h, i, 100, 1, None)
+    fits = lambda n, layers, h, i, d=None: lib.mmf_decode_layers_fits(n, layers, h, d or h, i)
+    for n, layers, h, i in ((3, 24, 2560, 6912), (3, 32, 2560, 6912), (3, 20, 2560, 6912), (3, 24, 3072, 8192), (3, 6, 4096, 8192),
+                            (1, 97, 1024, 2816), (1, 2, 4224, 4096), (1, 2, 2048, 8320)):
+        assert fits(n, layers, h, i) == 0 and norms(n, layers, h, i) == -2, (n, layers, h, i)
+    for n, layers, h, i in ((1, 32, 2560, 6912), (3, 19, 2560, 6912), (3, 24, 2048, 5632), (3, 24, 1024, 2816), (3, 5, 4096, 8192), (1, 24, 4096, 8192),
+                            (1, 96, 1024, 2816)):
+        assert fits(n, layers, h, i) == 1, (n, layers, h, i)
+    assert fits(2, 2, 512, 1536) == 0 and fits(1, 2, 512, 1536, 256) == 0 and fits(1, 2, 500, 1536) == 0 and fits(1, 0, 512, 1536) == 0
     assert lib.mmf_decode_layers_copies() == 8
     assert lib.mmf_decode_layers_words(512, 512, 1536) == 8 * (5 * 512 + 1536)
     assert lib.mmf_decode_layers_trace_words() == 256 * 128 * 12
