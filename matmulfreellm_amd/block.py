@@ -38,7 +38,18 @@ def _untouched(d):
     return not (d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"] or "forward" in d)
 
 
-class _Structure:
+class NotCopied:
+    """What is laid out once for one module and kept with it: device addresses, the module's own dictionaries, recorded graphs.  A copy
+    of the module (deepcopy, or saved whole and loaded) has none of it and makes its own on its first call."""
+
+    def __deepcopy__(self, memo):
+        return None
+
+    def __reduce__(self):
+        return type(None), ()
+
+
+class _Structure(NotCopied):
     """The modules of a block and the numbers they carry: what a native call takes for granted besides the parameters."""
 
     def __init__(self, block):
@@ -114,7 +125,7 @@ def _structure(block):
     return s
 
 
-class BlockPlan:
+class BlockPlan(NotCopied):
     """The native form of one block for inference: ``None`` from ``of`` where there is none."""
 
     @classmethod

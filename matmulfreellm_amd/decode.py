@@ -24,6 +24,7 @@ import torch
 
 from . import _lib as L
 from . import functional as F_
+from .block import NotCopied
 
 
 class _Phase(ctypes.Structure):
@@ -34,7 +35,7 @@ class _Phase(ctypes.Structure):
                 ("pad", ctypes.c_int)]
 
 
-class DecodeEngine:
+class DecodeEngine(NotCopied):
     CHUNK = 32          # steps whose input tokens the recorded graph keeps before the host has to fetch them
     SPIN = 1 << 15      # polling rounds a resident workgroup waits for its input before it gives up (mmf_decode_layers)
 

@@ -83,3 +83,31 @@ def test_a_written_or_replaced_parameter_is_seen(dev):
         assert torch.equal(logits[-1], model(input_ids=ids).logits)
         hook.remove()
     assert not any(torch.equal(a, b) for a, b in zip(logits, logits[1:]))
+
+
+@pytest.mark.parametrize("after", ["prompt", "training step", "generate"])
+def test_a_model_that_has_run_can_be_copied_and_saved_whole(dev, after):
+    import copy
+    import io
+    model = build(dev, torch.bfloat16, 160, True)
+    ids = torch.randint(0, 500, (2, 20), device=dev)
+    if after == "training step":
+        model.train()(input_ids=ids, labels=ids).loss.backward()
+        model.eval()
+    with torch.no_grad():
+        if after == "generate":
+            model.generate(ids, max_new_tokens=4)
+        want, tokens = model(input_ids=ids).logits, model.generate(ids, max_new_tokens=4) if after == "generate" else None
+        buf = io.BytesIO()
+        torch.save(model, buf)
+        buf.seek(0)
+        for other in (copy.deepcopy(model), torch.load(buf, weights_only=False)):
+            assert torch.equal(other(input_ids=ids).logits, want)
+            if tokens is not None:
+                assert torch.equal(other.generate(ids, max_new_tokens=4), tokens)
+            other.model.layers[1].attn.g_norm.eps = 0.5
+            other.model.layers[1].mlp.down_proj.weight.neg_()
+            changed = other(input_ids=ids).logits
+            other.model.layers[0].attn.g_norm.register_forward_hook(lambda *a: None)
+            assert torch.equal(other(input_ids=ids).logits, changed) and not torch.equal(changed, want)
+        assert torch.equal(model(input_ids=ids).logits, want)

@@ -256,3 +256,24 @@ def test_generation_mixin_wiring():
         model.generate(ids, attention_mask=mask, max_new_tokens=2, num_beams=2, pad_token_id=0)
     with pytest.raises(MMFError):
         model.generate(ids, max_new_tokens=2)
+
+
+def test_a_copied_or_saved_block_leaves_its_plans_behind():
+    """Plans hold device addresses and the dictionaries of the modules they were made for: a copy has none of them and sees its own
+    modules; the original keeps its own."""
+    import copy
+    import io
+    import matmulfreellm_amd as mm
+    from matmulfreellm_amd import block as native
+    layer = mm.HGRNBitModel(mm.HGRNBitConfig(vocab_size=50, hidden_size=32, num_hidden_layers=1)).layers[0].eval()
+    native.BlockPlan.of(layer)
+    plan = layer.__dict__["_native_plan"]
+    plan.native = native._Block()                              # as on a GPU: a struct of pointers, which nothing can pickle
+    buf = io.BytesIO()
+    torch.save(layer, buf)
+    buf.seek(0)
+    for other in (copy.deepcopy(layer), torch.load(buf, weights_only=False)):
+        other.attn.g_norm.eps = 0.5
+        assert native._structure(other).eps["g_eps"] == 0.5
+        assert native._structure(other).attn is other.attn
+    assert layer.__dict__["_native_plan"] is plan and native._structure(layer).eps["g_eps"] == layer.attn.g_norm.eps
