@@ -63,8 +63,10 @@ class _Structure(NotCopied):
         self.children = [(d["_modules"], k, c) for d in self.dicts for k, c in d["_modules"].items()]
         self.absent = [(d["_parameters"], k) for d in self.dicts for k, p in d["_parameters"].items() if p is None]
         self.numbers = []
+        if type(block) is not HGRNBitBlock:
+            return
         attn, mlp = block.attn, block.mlp
-        if (type(block) is not HGRNBitBlock or type(attn) is not HGRNBitAttention or type(mlp) is not HGRNBitMLP
+        if (type(attn) is not HGRNBitAttention or type(mlp) is not HGRNBitMLP
                 or attn.use_short_conv or not all(_untouched(d) for d in self.dicts)):
             return
         projs = (attn.i_proj, attn.f_proj, attn.g_proj, attn.o_proj, mlp.gate_proj, mlp.down_proj)

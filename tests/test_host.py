@@ -277,3 +277,18 @@ def test_a_copied_or_saved_block_leaves_its_plans_behind():
         assert native._structure(other).eps["g_eps"] == 0.5
         assert native._structure(other).attn is other.attn
     assert layer.__dict__["_native_plan"] is plan and native._structure(layer).eps["g_eps"] == layer.attn.g_norm.eps
+
+
+def test_a_layer_of_another_kind_has_no_native_form():
+    """A layer replaced by any other module (no attn, no mlp) is left to the module path, in inference and in training."""
+    import matmulfreellm_amd as mm
+    from matmulfreellm_amd import block as native
+
+    class Skip(torch.nn.Module):
+        def forward(self, hidden_states, **kwargs):
+            return hidden_states, None, kwargs.get("past_key_values")
+
+    model = mm.HGRNBitModel(mm.HGRNBitConfig(vocab_size=50, hidden_size=32, num_hidden_layers=2))
+    for layer in (Skip(), torch.nn.Identity(), torch.nn.Sequential(model.layers[1])):
+        assert native.BlockPlan.of(layer) is None and native.BlockPlan.of(layer) is None
+        assert native.TrainPlan.of(layer, torch.zeros(1, 4, 32)) is None
