@@ -50,7 +50,8 @@ class NotCopied:
 
 
 class _Structure(NotCopied):
-    """The modules of a block and the numbers they carry: what a native call takes for granted besides the parameters."""
+    """The modules of a block and the numbers they carry: what a native call takes for granted besides the parameters.  Nothing here
+    leads back to the block itself or its ``__dict__``, which hold this object: a dropped model is freed at once."""
 
     def __init__(self, block):
         from .attention import HGRNBitAttention
@@ -59,15 +60,10 @@ class _Structure(NotCopied):
         from .layernorm import RMSNorm
         from .modeling_hgrn_bit import HGRNBitBlock, HGRNBitMLP
         self.fits = False
-        self.dicts = [m.__dict__ for m in block.modules()]
-        self.children = [(d["_modules"], k, c) for d in self.dicts for k, c in d["_modules"].items()]
-        self.absent = [(d["_parameters"], k) for d in self.dicts for k, p in d["_parameters"].items() if p is None]
-        self.numbers = []
         if type(block) is not HGRNBitBlock:
             return
         attn, mlp = block.attn, block.mlp
-        if (type(attn) is not HGRNBitAttention or type(mlp) is not HGRNBitMLP
-                or attn.use_short_conv or not all(_untouched(d) for d in self.dicts)):
+        if type(attn) is not HGRNBitAttention or type(mlp) is not HGRNBitMLP or attn.use_short_conv:
             return
         projs = (attn.i_proj, attn.f_proj, attn.g_proj, attn.o_proj, mlp.gate_proj, mlp.down_proj)
         norms = (block.attn_norm, block.mlp_norm, attn.g_norm)
@@ -75,20 +71,29 @@ class _Structure(NotCopied):
                 or any(type(n) is not RMSNorm for n in norms[:2]) or type(norms[2]) is not FusedRMSNormSwishGate
                 or any(n.weight is None for n in norms) or any(p.norm.weight is None for p in projs)):
             return
+        modules = list(block.modules())
+        self.dicts = [m.__dict__ for m in modules[1:]]
+        own = block.__dict__
+        if not all(_untouched(d) for d in [own] + self.dicts):
+            return
         H, D, I = attn.hidden_size, attn.input_dim, mlp.intermediate_size
         if (D % 32 or I % 32 or H % 8 or max(H, D, I) > 8192 or attn.num_heads * attn.head_dim != D
                 or any(p.run_eps() != projs[0].run_eps() for p in projs[:3])):
             return
-        self.numbers = ([(m.__dict__, "eps", m.eps) for m in norms + tuple(p.norm for p in projs)]
-                        + [(p.__dict__, "fused_eps", p.fused_eps) for p in projs])
+        numbers = [(m, "eps") for m in norms + tuple(p.norm for p in projs)] + [(p, "fused_eps") for p in projs]
+        holders = [own["_modules"]] + [d["_modules"] for d in self.dicts]
+        self.parameters = [own["_parameters"]] + [d["_parameters"] for d in self.dicts]
+        self.facts = (own["_modules"], own["_parameters"], self.dicts, [(h, k, c) for h in holders for k, c in h.items()],
+                      [(h, k) for h in self.parameters for k, p in h.items() if p is None],
+                      [(m.__dict__, name, getattr(m, name)) for m, name in numbers])
         self.eps = dict(zip(("attn_eps", "mlp_eps", "g_eps", "ifg_eps", "o_eps", "gate_eps", "down_eps"),
                             [m.eps for m in norms] + [p.run_eps() for p in projs[:1] + projs[3:]]))
         self.attn, self.projs, self.norms = attn, projs, norms
         self.dims, self.heads, self.head_dim, self.mode, self.layer_idx = (H, D, I), attn.num_heads, attn.head_dim, attn.mode, attn.layer_idx
         self.fits = True
 
-    def current(self):
-        return L.native().structure_holds(self.dicts, self.children, self.absent, self.numbers)
+    def current(self, block):
+        return self.fits and L.native().structure_holds(block, self.facts)
 
     def norm_weights(self):
         """attn_norm, mlp_norm, g_norm, then the inner norms of i, f, g, o, gate, down."""
@@ -122,7 +127,7 @@ class _Structure(NotCopied):
 
 def _structure(block):
     s = block.__dict__.get("_native_structure")
-    if s is None or not s.current():
+    if s is None or not s.current(block):
         s = block.__dict__["_native_structure"] = _Structure(block)
     return s
 
@@ -133,19 +138,17 @@ class BlockPlan(NotCopied):
     @classmethod
     def of(cls, block):
         plan = block.__dict__.get("_native_plan")
-        if plan is None or not plan.current():
+        if plan is None or not plan.current(block):
             plan = block.__dict__["_native_plan"] = cls(block)
         return plan if plan.fits else None
 
     def __init__(self, block):
         self.fits = False
         s = self.structure = _structure(block)
-        self.params = [(d["_parameters"], k, p, p._version, p.data_ptr()) for d in s.dicts
-                       for k, p in d["_parameters"].items() if p is not None]
-        self.packed = []
         where = s.fits_tensors() if s.fits else None
         if where is None:
             return
+        self.params = [(h, k, p, p._version, p.data_ptr()) for h in s.parameters for k, p in h.items() if p is not None]
         self.dtype, self.device = where
         nws, pws = s.norm_weights(), [p.packed_weight() for p in s.projs]
         if any(pw.packed.device != self.device for pw in pws):
@@ -159,8 +162,8 @@ class BlockPlan(NotCopied):
         self.H, self.D = s.dims[:2]
         self.fits = True
 
-    def current(self):
-        if not self.structure.current():
+    def current(self, block):
+        if not (self.fits and self.structure.current(block)):
             return False
         if not L.native().parameters_hold(self.params):
             return False

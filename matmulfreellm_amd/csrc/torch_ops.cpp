@@ -168,54 +168,72 @@ PyObject* scan(PyObject*, PyObject* const* args, Py_ssize_t count) {
 }
 
 // ------------------------------------------------------------------------------ what a native block call takes for granted
-// (module dicts, [(dict, key, object)], [(dict, key)], [(dict, key, value)]) -> whether no module has hooks or a forward of its own, the
-// objects are the ones the dicts hold, the keys hold None or nothing, and the values are equal.  Asked for every block of every
-// forward: ~90 dictionary look-ups, 10 us in Python and 2 here.
-PyObject *kHooks[4], *kForward;
+// Whether all of this still holds for a block -- asked for every block of every forward, ~90 look-ups, 10 us in Python and 2 here:
+// (block, (modules dict, parameters dict, [module dict], [(dict, key, object)], [(dict, key)], [(dict, key, value)])):
+//   the block holds those two dicts, and neither it nor a module below it has hooks or a forward of its own;
+//   the dicts hold those objects, nothing or None, and equal values.
+PyObject *kHooks[4], *kForward, *kDict, *kModules, *kParameters;
+// 1 / 0, or -1 with an error set
+int untouched(PyObject* d) {
+    for (PyObject* name : kHooks) {
+        PyObject* hooks = PyDict_GetItemWithError(d, name);
+        if (!hooks) {
+            if (!PyErr_Occurred()) PyErr_SetObject(PyExc_KeyError, name);
+            return -1;
+        }
+        const int any = PyObject_IsTrue(hooks);
+        if (any != 0) return any < 0 ? -1 : 0;
+    }
+    const int own = PyDict_Contains(d, kForward);
+    return own < 0 ? -1 : !own;
+}
+int holds(PyObject* d, PyObject* key, PyObject* object) {
+    PyObject* held = PyDict_GetItemWithError(d, key);
+    return !held && PyErr_Occurred() ? -1 : held == object;
+}
+int structure(PyObject* block, PyObject* facts) {
+    auto fact = [&](int i) { return PyTuple_GET_ITEM(facts, i); };
+    PyObject* d = PyObject_GetAttr(block, kDict);
+    if (!d) return -1;
+    int ok = untouched(d);
+    if (ok == 1) ok = holds(d, kModules, fact(0));
+    if (ok == 1) ok = holds(d, kParameters, fact(1));
+    Py_DECREF(d);
+    if (ok != 1) return ok;
+    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(fact(2)); ++i) {
+        if ((ok = untouched(PyList_GET_ITEM(fact(2), i))) != 1) return ok;
+    }
+    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(fact(3)); ++i) {
+        PyObject* t = PyList_GET_ITEM(fact(3), i);
+        if ((ok = holds(PyTuple_GET_ITEM(t, 0), PyTuple_GET_ITEM(t, 1), PyTuple_GET_ITEM(t, 2))) != 1) return ok;
+    }
+    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(fact(4)); ++i) {
+        PyObject* t = PyList_GET_ITEM(fact(4), i);
+        PyObject* held = PyDict_GetItemWithError(PyTuple_GET_ITEM(t, 0), PyTuple_GET_ITEM(t, 1));
+        if (!held && PyErr_Occurred()) return -1;
+        if (held && held != Py_None) return 0;
+    }
+    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(fact(5)); ++i) {
+        PyObject* t = PyList_GET_ITEM(fact(5), i);
+        PyObject* held = PyDict_GetItemWithError(PyTuple_GET_ITEM(t, 0), PyTuple_GET_ITEM(t, 1));
+        if (!held) return PyErr_Occurred() ? -1 : 0;
+        if (held == PyTuple_GET_ITEM(t, 2)) continue;
+        Py_INCREF(held);                                            // (an __eq__ may be anybody's)
+        ok = PyObject_RichCompareBool(held, PyTuple_GET_ITEM(t, 2), Py_EQ);
+        Py_DECREF(held);
+        if (ok != 1) return ok;
+    }
+    return 1;
+}
 PyObject* structure_holds(PyObject*, PyObject* const* args, Py_ssize_t count) {
-    if (count != 4) { PyErr_SetString(PyExc_TypeError, "structure_holds takes 4 lists"); return nullptr; }
-    for (int i = 0; i < 4; ++i)
-        if (!PyList_Check(args[i])) { PyErr_SetString(PyExc_TypeError, "structure_holds takes 4 lists"); return nullptr; }
-    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(args[0]); ++i) {
-        PyObject* d = PyList_GET_ITEM(args[0], i);
-        for (PyObject* name : kHooks) {
-            PyObject* hooks = PyDict_GetItemWithError(d, name);
-            if (!hooks) {
-                if (!PyErr_Occurred()) PyErr_SetObject(PyExc_KeyError, name);
-                return nullptr;
-            }
-            const int any = PyObject_IsTrue(hooks);
-            if (any < 0) return nullptr;
-            if (any) Py_RETURN_FALSE;
-        }
-        const int own = PyDict_Contains(d, kForward);
-        if (own < 0) return nullptr;
-        if (own) Py_RETURN_FALSE;
+    bool fits = count == 2 && PyTuple_Check(args[1]) && PyTuple_GET_SIZE(args[1]) == 6;
+    for (int i = 2; fits && i < 6; ++i) fits = PyList_Check(PyTuple_GET_ITEM(args[1], i));
+    if (!fits) {
+        PyErr_SetString(PyExc_TypeError, "structure_holds takes (block, (modules, parameters, 4 lists))");
+        return nullptr;
     }
-    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(args[1]); ++i) {
-        PyObject* t = PyList_GET_ITEM(args[1], i);
-        PyObject* held = PyDict_GetItemWithError(PyTuple_GET_ITEM(t, 0), PyTuple_GET_ITEM(t, 1));
-        if (!held && PyErr_Occurred()) return nullptr;
-        if (held != PyTuple_GET_ITEM(t, 2)) Py_RETURN_FALSE;
-    }
-    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(args[2]); ++i) {
-        PyObject* t = PyList_GET_ITEM(args[2], i);
-        PyObject* held = PyDict_GetItemWithError(PyTuple_GET_ITEM(t, 0), PyTuple_GET_ITEM(t, 1));
-        if (!held && PyErr_Occurred()) return nullptr;
-        if (held && held != Py_None) Py_RETURN_FALSE;
-    }
-    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(args[3]); ++i) {
-        PyObject* t = PyList_GET_ITEM(args[3], i);
-        PyObject* held = PyDict_GetItemWithError(PyTuple_GET_ITEM(t, 0), PyTuple_GET_ITEM(t, 1));
-        if (!held) {
-            if (PyErr_Occurred()) return nullptr;
-            Py_RETURN_FALSE;
-        }
-        const int same = held == PyTuple_GET_ITEM(t, 2) ? 1 : PyObject_RichCompareBool(held, PyTuple_GET_ITEM(t, 2), Py_EQ);
-        if (same < 0) return nullptr;
-        if (!same) Py_RETURN_FALSE;
-    }
-    Py_RETURN_TRUE;
+    const int ok = structure(args[0], args[1]);
+    return ok < 0 ? nullptr : PyBool_FromLong(ok);
 }
 
 // [(dict, key, parameter, version, address)] -> whether the dicts hold those parameters, unwritten since
@@ -251,6 +269,8 @@ PyMODINIT_FUNC PyInit_mmf_torch() {
     const char* names[4] = {"_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks"};
     for (int i = 0; i < 4; ++i)
         if (!(kHooks[i] = PyUnicode_InternFromString(names[i]))) return nullptr;
-    if (!(kForward = PyUnicode_InternFromString("forward"))) return nullptr;
+    if (!(kForward = PyUnicode_InternFromString("forward")) || !(kDict = PyUnicode_InternFromString("__dict__")) ||
+        !(kModules = PyUnicode_InternFromString("_modules")) || !(kParameters = PyUnicode_InternFromString("_parameters")))
+        return nullptr;
     return PyModule_Create(&module);
 }

@@ -55,7 +55,6 @@ class DecodeEngine(NotCopied):
             raise NotImplementedError("DecodeEngine has no convolution state: models with use_short_conv decode through "
                                       "the module path (generate() does so by itself)")
         self.lib = L.load()
-        self.model = model
         self.B = B = batch_size
         emb = model.model.embeddings.weight
         self.dev = dev = L.require_gpu(emb)
@@ -66,7 +65,8 @@ class DecodeEngine(NotCopied):
         self.L = len(model.model.layers)
         self.eps = float(cfg.rms_norm_eps)
         self.use_graph = use_graph
-        # what the operands below were taken from: modules, parameters (object, version, address)
+        # what the operands below were taken from: modules, parameters (object, version, address); nothing here leads back to the model,
+        # which holds this engine
         self._children = [(d["_modules"], k, c) for d in (m.__dict__ for m in model.modules()) for k, c in d["_modules"].items()]
         self._parameters = [(d["_parameters"], k, p, p._version, p.data_ptr()) for d in (m.__dict__ for m in model.modules())
                             for k, p in d["_parameters"].items() if p is not None]

@@ -111,3 +111,25 @@ def test_a_model_that_has_run_can_be_copied_and_saved_whole(dev, after):
             other.model.layers[0].attn.g_norm.register_forward_hook(lambda *a: None)
             assert torch.equal(other(input_ids=ids).logits, changed) and not torch.equal(changed, want)
         assert torch.equal(model(input_ids=ids).logits, want)
+
+
+def test_a_dropped_model_gives_its_memory_back(dev):
+    """After prompts, a training step and generation through the captured graphs and the resident launch, with the cycle collector off."""
+    import gc
+    held = []
+    gc.collect()
+    gc.disable()
+    try:
+        for use in (lambda m, ids: m(input_ids=ids), lambda m, ids: m(input_ids=ids, labels=ids).loss.backward(),
+                    lambda m, ids: m.generate(ids, max_new_tokens=3), lambda m, ids: m.generate(ids[:1], max_new_tokens=3)):
+            before = torch.cuda.memory_allocated(dev)
+            model, ids = build(dev, torch.bfloat16, 512, True), torch.randint(0, 500, (2, 20), device=dev)
+            weights = sum(p.numel() * p.element_size() for p in model.parameters())
+            with torch.set_grad_enabled("backward" in use.__code__.co_names):
+                use(model, ids)
+            torch.cuda.synchronize(dev)
+            del model, ids
+            held.append((torch.cuda.memory_allocated(dev) - before) / weights)
+    finally:
+        gc.enable()
+    assert max(held) < 0.2, held

@@ -292,3 +292,30 @@ def test_a_layer_of_another_kind_has_no_native_form():
     for layer in (Skip(), torch.nn.Identity(), torch.nn.Sequential(model.layers[1])):
         assert native.BlockPlan.of(layer) is None and native.BlockPlan.of(layer) is None
         assert native.TrainPlan.of(layer, torch.zeros(1, 4, 32)) is None
+
+
+def test_a_plan_belongs_to_one_block_and_does_not_keep_it():
+    """The weights of a dropped model are given back with its last reference, without a run of the cycle collector; a shallow copy of
+    a block, which takes the plan along, is looked at itself."""
+    import copy
+    import gc
+    import weakref
+    import matmulfreellm_amd as mm
+    from matmulfreellm_amd import block as native
+    layer = mm.HGRNBitModel(mm.HGRNBitConfig(vocab_size=50, hidden_size=32, num_hidden_layers=1)).layers[0]
+    assert native._structure(layer).fits and native.BlockPlan.of(layer) is None      # (no plan without a GPU)
+    other = copy.copy(layer)
+    assert native._structure(other).fits
+    other.forward = lambda *a, **k: None
+    assert not native._structure(other).fits and native._structure(layer).fits
+    replica = copy.copy(layer)                                                       # as torch replicates modules: dicts of its own
+    replica._modules = dict(layer._modules)
+    replica._modules["mlp"] = copy.deepcopy(layer.mlp)
+    assert native._structure(replica).projs[5] is replica.mlp.down_proj
+    kept = weakref.ref(layer.attn.i_proj.weight)
+    gc.disable()
+    try:
+        del layer, other, replica
+        assert kept() is None
+    finally:
+        gc.enable()
