@@ -17,10 +17,12 @@ import torch.nn as nn
 
 from . import functional as F_
 from .autograd import module_needs_grad
+from .block import as_defined
 from .bitlinear import FusedBitLinear as BitLinear
 from .fused_norm_gate import FusedRMSNormSwishGate
 
 
+@as_defined
 class HGRNBitAttention(nn.Module):
 
     def __init__(self, mode: str = "fused_recurrent", hidden_size: int = 1024, num_heads: Optional[int] = None,

@@ -10,6 +10,7 @@ import torch.nn as nn
 from . import _lib as L
 from . import functional as F_
 from .autograd import BitLinearFn, needs_grad
+from .block import as_defined
 from .layernorm import RMSNorm
 
 
@@ -116,6 +117,7 @@ class BitLinear(nn.Linear):
                                           is_rms_norm=True, packed=self.packed_weight())
 
 
+@as_defined
 class FusedBitLinear(BitLinear):
     """mmfreelm/ops/fusedbitnet.py:584-610.  Same math as BitLinear here: both run the fused kernels.
 

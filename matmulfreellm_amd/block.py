@@ -2,9 +2,10 @@
 
 ``BlockPlan.of(block)`` lays the pointers of a block's parameters and packed weights out once, in the struct the native
 side reads, and remembers what they were taken from.  ``current()`` looks, before every call, whether all of that still
-holds: the same modules, parameters neither written nor replaced, the same eps, no hook and no patched ``forward`` anywhere
-inside -- anything else (and every block the native call does not cover) goes through the modules as before.  The
-results are those of the module path bit for bit: the same kernels with the same arguments.
+holds: the same modules of the same classes, parameters neither written nor replaced, the same eps, mode, layer index and sizes,
+no hook and no patched ``forward`` or ``__call__`` anywhere inside, on a module or on its class -- anything else (and every
+block the native call does not cover) goes through the modules as before.  The results are those of the module path bit for bit: the
+same kernels with the same arguments.
 """
 import ctypes
 
@@ -30,8 +31,19 @@ def global_hooks():
                 or nn_module._global_backward_pre_hooks)
 
 
-def hook_free(module):
-    return _untouched(module.__dict__)
+AS_DEFINED = {}
+
+
+def as_defined(cls):
+    """Decorator of the classes whose work native calls do in their place: what their forward and __call__ were at the start."""
+    AS_DEFINED[cls] = (cls.forward, cls.__call__)
+    return cls
+
+
+def plain(module):
+    """Whether a module is one of those classes', unchanged, without a hook or a forward of its own."""
+    c = type(module)
+    return AS_DEFINED.get(c) == (c.forward, c.__call__) and _untouched(module.__dict__)
 
 
 def _untouched(d):
@@ -71,21 +83,21 @@ class _Structure(NotCopied):
                 or any(type(n) is not RMSNorm for n in norms[:2]) or type(norms[2]) is not FusedRMSNormSwishGate
                 or any(n.weight is None for n in norms) or any(p.norm.weight is None for p in projs)):
             return
-        modules = list(block.modules())
-        self.dicts = [m.__dict__ for m in modules[1:]]
-        own = block.__dict__
-        if not all(_untouched(d) for d in [own] + self.dicts):
+        modules = [block, attn, mlp, *norms, *projs, *(p.norm for p in projs)]
+        if not all(plain(m) for m in modules):
             return
         H, D, I = attn.hidden_size, attn.input_dim, mlp.intermediate_size
         if (D % 32 or I % 32 or H % 8 or max(H, D, I) > 8192 or attn.num_heads * attn.head_dim != D
                 or any(p.run_eps() != projs[0].run_eps() for p in projs[:3])):
             return
-        numbers = [(m, "eps") for m in norms + tuple(p.norm for p in projs)] + [(p, "fused_eps") for p in projs]
-        holders = [own["_modules"]] + [d["_modules"] for d in self.dicts]
-        self.parameters = [own["_parameters"]] + [d["_parameters"] for d in self.dicts]
-        self.facts = (own["_modules"], own["_parameters"], self.dicts, [(h, k, c) for h in holders for k, c in h.items()],
+        numbers = [(m, "eps") for m in norms + tuple(p.norm for p in projs)] + [(p, "fused_eps") for p in projs] + [(mlp, "intermediate_size")]
+        numbers += [(attn, name) for name in ("mode", "layer_idx", "hidden_size", "input_dim", "num_heads", "head_dim", "use_short_conv")]
+        self.parameters = [m._parameters for m in modules]
+        self.facts = (type(block), block._modules, block._parameters, [(m, type(m), m.__dict__) for m in modules[1:]],
+                      [(m._modules, k, c) for m in modules for k, c in m._modules.items()],
                       [(h, k) for h in self.parameters for k, p in h.items() if p is None],
-                      [(m.__dict__, name, getattr(m, name)) for m, name in numbers])
+                      [(m.__dict__, name, getattr(m, name)) for m, name in numbers],
+                      [(c, *AS_DEFINED[c]) for c in {type(m) for m in modules}])
         self.eps = dict(zip(("attn_eps", "mlp_eps", "g_eps", "ifg_eps", "o_eps", "gate_eps", "down_eps"),
                             [m.eps for m in norms] + [p.run_eps() for p in projs[:1] + projs[3:]]))
         self.attn, self.projs, self.norms = attn, projs, norms

@@ -3,6 +3,7 @@ import torch
 import torch.nn as nn
 
 from . import functional as F_
+from .block import as_defined
 
 
 def rms_norm_swish_gate_fn(x, o, weight, bias, residual=None, prenorm=False, residual_in_fp32=False, eps=1e-6):
@@ -18,6 +19,7 @@ def rms_norm_swish_gate_fn(x, o, weight, bias, residual=None, prenorm=False, res
                                 residual_in_fp32=residual_in_fp32)
 
 
+@as_defined
 class FusedRMSNormSwishGate(nn.Module):
     """y = RMSNorm(x) * weight * o * sigmoid(o)."""
 

@@ -3,6 +3,7 @@ import torch
 import torch.nn as nn
 
 from . import functional as F_
+from .block import as_defined
 
 
 def rms_norm_fn(x, weight, bias, residual=None, prenorm=False, residual_in_fp32=False, eps=1e-6):
@@ -15,6 +16,7 @@ def rms_norm_fn(x, weight, bias, residual=None, prenorm=False, residual_in_fp32=
     return F_.rmsnorm(x, weight, residual=residual, eps=eps, prenorm=prenorm, residual_in_fp32=residual_in_fp32)
 
 
+@as_defined
 class RMSNorm(nn.Module):
     """mmfreelm/modules/layernorm.py:586-623."""
 

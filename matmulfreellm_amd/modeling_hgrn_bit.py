@@ -47,6 +47,7 @@ def lower_bound_schedule(lower_bounds: torch.Tensor) -> torch.Tensor:
     return lb.to(lower_bounds.device)
 
 
+@native.as_defined
 class HGRNBitMLP(nn.Module):
 
     def __init__(self, hidden_size: int, hidden_ratio: Optional[int] = None, intermediate_size: Optional[int] = None,
@@ -97,6 +98,7 @@ class HGRNBitMLP(nn.Module):
         return self.down_proj.forward_fused(y[..., :inter], ("swiglu", y[..., inter:]), addend=addend)
 
 
+@native.as_defined
 class HGRNBitBlock(nn.Module):
 
     def __init__(self, config: HGRNBitConfig, layer_idx: int):
@@ -152,6 +154,7 @@ class HGRNBitPreTrainedModel(PreTrainedModel):
                         p /= math.sqrt(num_residuals_per_layer * self.config.num_hidden_layers)
 
 
+@native.as_defined
 class HGRNBitModel(HGRNBitPreTrainedModel):
 
     def __init__(self, config: HGRNBitConfig):
@@ -452,7 +455,7 @@ class HGRNBitForCausalLM(HGRNBitPreTrainedModel, GenerationMixin):
         norm, head = self.model.norm, self.lm_head
         return (not output_hidden_states and not getattr(self.config, "output_hidden_states", False)
                 and type(self.model) is HGRNBitModel and type(norm) is RMSNorm and type(head) is BitLinear and type(head.norm) is RMSNorm
-                and not native.global_hooks() and all(native.hook_free(m) for m in (self.model, norm, head, head.norm))
+                and not native.global_hooks() and all(native.plain(m) for m in (self.model, norm, head, head.norm))
                 and norm.weight is not None and head.norm.weight is not None and norm.weight.dtype == head.norm.weight.dtype
                 and head.in_features <= 8192 and (not train or (
                     head.bias is None and not head.weight.is_meta and head.in_features % 8 == 0

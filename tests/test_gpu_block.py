@@ -67,6 +67,36 @@ def test_what_a_hook_has_kept_is_not_written(dev, hooked):
     assert torch.equal(logits, again.logits)
 
 
+def test_changed_modules_are_seen(dev, monkeypatch):
+    """What the module path would refuse or run differently, changed after a first forward: the mode, a module's class, a class's
+    forward."""
+    import matmulfreellm_amd as mm
+    model = build(dev, torch.bfloat16, 160, True)
+    ids = torch.randint(0, 500, (1, 20), device=dev)
+    run = lambda: model(input_ids=ids).logits
+    with torch.no_grad():
+        want = run()
+        attn, mlp = model.model.layers[1].attn, model.model.layers[1].mlp
+        attn.mode = "chunk"
+        with pytest.raises(NotImplementedError):
+            run()
+        attn.mode = "fused_recurrent"
+        assert torch.equal(run(), want)
+
+        class Double(mm.HGRNBitMLP):
+            def forward(self, *args, **kwargs):
+                return super().forward(*args, **kwargs) * 2
+
+        mlp.__class__ = Double
+        assert not torch.equal(run(), want)
+        mlp.__class__ = mm.HGRNBitMLP
+        assert torch.equal(run(), want)
+        with monkeypatch.context() as patch:
+            patch.setattr(mm.HGRNBitMLP, "forward", lambda self, x, residual=None, pre_norm=None: x)
+            assert not torch.equal(run(), want)
+        assert torch.equal(run(), want)
+
+
 def test_a_written_or_replaced_parameter_is_seen(dev):
     model = build(dev, torch.bfloat16, 160, True)
     ids = torch.randint(0, 500, (1, 20), device=dev)

@@ -319,3 +319,41 @@ def test_a_plan_belongs_to_one_block_and_does_not_keep_it():
         assert kept() is None
     finally:
         gc.enable()
+
+
+def test_a_plan_sees_every_change_it_depends_on(monkeypatch):
+    """Attributes, classes, and forward or __call__ replaced on a class, before the first look or after it."""
+    import matmulfreellm_amd as mm
+    from matmulfreellm_amd import block as native
+    layer = mm.HGRNBitModel(mm.HGRNBitConfig(vocab_size=50, hidden_size=32, num_hidden_layers=1)).layers[0]
+    first = native._structure(layer)
+    assert first.fits and native._structure(layer) is first
+    attn, mlp = layer.attn, layer.mlp
+    for module, name, value in ((attn, "mode", "chunk"), (attn, "layer_idx", 3), (attn, "num_heads", 2), (attn, "head_dim", 16),
+                                (attn, "use_short_conv", True), (attn, "input_dim", 64), (attn, "hidden_size", 64), (mlp, "intermediate_size", 96),
+                                (mlp.down_proj.norm, "eps", 0.5), (mlp.down_proj, "fused_eps", 0.5)):
+        before = getattr(module, name)
+        assert native._structure(layer).current(layer)
+        monkeypatch.setattr(module, name, value)
+        assert not layer.__dict__["_native_structure"].current(layer), name
+        monkeypatch.setattr(module, name, before)
+    plain = native._structure(layer)
+    for module in (layer, attn, attn.g_norm, mlp.down_proj, mlp.down_proj.norm, layer.attn_norm):
+        cls = type(module)
+        module.__class__ = type("Other", (cls,), {})
+        assert not plain.current(layer) and not native._structure(layer).fits
+        module.__class__ = cls
+        plain = native._structure(layer)
+        assert plain.fits
+        for name in ("forward", "__call__"):
+            with monkeypatch.context() as patch:
+                patch.setattr(cls, name, lambda self, *a, **k: None)
+                assert not plain.current(layer) and not native._structure(layer).fits and not native.plain(module)
+            plain = native._structure(layer)
+            assert plain.fits and plain.current(layer) and native.plain(module)
+    with monkeypatch.context() as patch:                        # (BitLinear's is the one FusedBitLinear runs)
+        patch.setattr(mm.BitLinear, "forward", lambda self, x: x)
+        assert not plain.current(layer)
+    with monkeypatch.context() as patch:
+        patch.setattr(torch.nn.Module, "__call__", lambda self, *a, **k: None)
+        assert not plain.current(layer)
