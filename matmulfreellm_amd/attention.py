@@ -65,8 +65,8 @@ class HGRNBitAttention(nn.Module):
         self.g_norm = FusedRMSNormSwishGate(self.input_dim, layernorm_eps)
         self.o_proj = BitLinear(self.input_dim, hidden_size, bias=False, fused_eps=bitlinear_eps)
         self.apply(self._initialize_weights)
-        self._ifg_key, self._ifg = None, None
-        self._stack_key, self._stack = None, None
+        self._norms_seen, self._norms_agree = F_.Seen(), False
+        self._stack = None
 
     def _initialize_weights(self, module):
         if getattr(module, "_is_hf_initialized", False):
@@ -81,25 +81,21 @@ class HGRNBitAttention(nn.Module):
     def _stacked_weight(self):
         """PackedWeight of [i; f; g], whatever their inner norms hold."""
         parts = [p.packed_weight() for p in (self.i_proj, self.f_proj, self.g_proj)]
-        key = tuple(id(pw) for pw in parts)
-        if key != self._stack_key:
-            # (the parts stay alive with the projections' pack caches; kept here too, so that an id is not reused)
-            self._stack_key, self._stack = key, (F_.stack_packed(parts), parts)
+        if self._stack is None or any(a is not b for a, b in zip(self._stack[1], parts)):
+            self._stack = (F_.stack_packed(parts), parts)
         return self._stack[0]
 
     def _stacked_ifg(self):
         """PackedWeight of [i; f; g] if the three inner norms are identical, else None."""
         projs = (self.i_proj, self.f_proj, self.g_proj)
-        key = tuple((p.weight.data_ptr(), p.weight._version, p.norm.weight.data_ptr(), p.norm.weight._version,
-                     p.weight.dtype, p.weight.device) for p in projs)
-        if key != self._ifg_key:
-            self._ifg_key = key
-            same = (self.input_dim % 32 == 0 and all(p.bias is None for p in projs)
-                    and all(p.norm.eps == projs[0].norm.eps and p.fused_eps == projs[0].fused_eps for p in projs)
-                    and torch.equal(self.i_proj.norm.weight, self.f_proj.norm.weight)
-                    and torch.equal(self.i_proj.norm.weight, self.g_proj.norm.weight))
-            self._ifg = self._stacked_weight() if same else None
-        return self._ifg
+        if (self.input_dim % 32 or any(p.bias is not None for p in projs)
+                or any(p.norm.eps != projs[0].norm.eps or p.fused_eps != projs[0].fused_eps for p in projs[1:])):
+            return None
+        norms = [p.norm.weight for p in projs]
+        if not self._norms_seen.unchanged(*norms):                   # (the comparison waits for the device)
+            self._norms_agree = torch.equal(norms[0], norms[1]) and torch.equal(norms[0], norms[2])
+            self._norms_seen.take(*norms)
+        return self._stacked_weight() if self._norms_agree else None
 
     def forward(self, hidden_states: torch.Tensor, attention_mask: Optional[torch.Tensor] = None,
                 past_key_values=None, use_cache: Optional[bool] = False, output_attentions: Optional[bool] = False,

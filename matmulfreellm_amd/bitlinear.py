@@ -30,21 +30,20 @@ class _PackCache:
     """Packed codes of one weight tensor, invalidated when the tensor is written or replaced."""
 
     def __init__(self):
-        self.key, self.pw, self.frozen = None, None, False
+        self.seen, self.pw, self.frozen = F_.Seen(), None, False
 
     def freeze(self, pw):
         """Pin codes loaded from a packed checkpoint: there is no latent weight to re-pack from."""
-        self.key, self.pw, self.frozen = None, pw, True
+        self.seen, self.pw, self.frozen = F_.Seen(), pw, True
 
     def get(self, weight):
         if self.frozen:
             if not weight.is_meta:
                 raise RuntimeError("this BitLinear holds packed codes only; assigning a latent weight to it is not supported")
             return self.pw
-        key = (weight.data_ptr(), weight._version, weight.dtype, weight.device, weight.shape)
-        if key != self.key:
+        if not self.seen.unchanged(weight):
             self.pw = F_.ternarize_pack(weight)
-            self.key = key
+            self.seen.take(weight)
         return self.pw
 
 

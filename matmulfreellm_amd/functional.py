@@ -1,4 +1,6 @@
 """Tensor-level wrappers over the C ABI: shape checks, output allocation, one call each."""
+import weakref
+
 import torch
 
 from . import _lib as L
@@ -24,6 +26,29 @@ def _as_2d(x):
 
 
 # ------------------------------------------------------------------------------ weights
+class Seen:
+    """Tensors as they were when something was derived from them: the same objects, unwritten since and at their addresses.  The
+    objects count too, because a tensor that is computed anew on each access (a parametrised weight) may come to lie where the last one
+    did.  They are not kept alive; a copy or a pickle of this has seen nothing."""
+
+    def __init__(self):
+        self.refs, self.facts = (), None
+
+    @staticmethod
+    def _facts(tensors):
+        return [(t.data_ptr(), t._version, t.dtype, t.device, t.shape) for t in tensors]
+
+    def unchanged(self, *tensors):
+        return (len(self.refs) == len(tensors) and all(r() is t for r, t in zip(self.refs, tensors))
+                and self.facts == self._facts(tensors))
+
+    def take(self, *tensors):
+        self.refs, self.facts = [weakref.ref(t) for t in tensors], self._facts(tensors)
+
+    def __reduce__(self):
+        return Seen, ()
+
+
 class PackedWeight:
     """2-bit packed ternary codes of one or more [N_i, K] matrices stacked along N."""
 

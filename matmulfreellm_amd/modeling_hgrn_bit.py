@@ -167,7 +167,7 @@ class HGRNBitModel(HGRNBitPreTrainedModel):
         self.layers = nn.ModuleList([HGRNBitBlock(config, i) for i in range(config.num_hidden_layers)])
         self.norm = RMSNorm(config.hidden_size, eps=config.rms_norm_eps)
         self.gradient_checkpointing = False
-        self._lb_key, self._lb = None, None
+        self._lb_seen, self._lb = F_.Seen(), None
         self.post_init()
 
     def get_input_embeddings(self):
@@ -179,9 +179,9 @@ class HGRNBitModel(HGRNBitPreTrainedModel):
     def lower_bound_rows(self):
         """fp32 [L, H] lower bounds, recomputed only when the parameter changes."""
         p = self.lower_bounds
-        key = (p.data_ptr(), p._version, p.device)
-        if key != self._lb_key:
-            self._lb_key, self._lb = key, lower_bound_schedule(p)
+        if not self._lb_seen.unchanged(p):
+            self._lb = lower_bound_schedule(p)
+            self._lb_seen.take(p)
         return self._lb
 
     def forward(self, input_ids: Optional[torch.LongTensor] = None, attention_mask: Optional[torch.Tensor] = None,

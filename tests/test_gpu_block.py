@@ -97,6 +97,31 @@ def test_changed_modules_are_seen(dev, monkeypatch):
         assert torch.equal(run(), want)
 
 
+def test_a_parametrised_weight_is_packed_anew(dev):
+    """A weight behind a parametrisation is another tensor on each access, often at the same address; its own tensor changes here."""
+    model = build(dev, torch.bfloat16, 160, True)
+    ids = torch.randint(0, 500, (1, 20), device=dev)
+    run = lambda: model(input_ids=ids).logits
+    with torch.no_grad():
+        want, mlp = run(), model.model.layers[1].mlp
+
+        class Scale(torch.nn.Module):
+            def __init__(self):
+                super().__init__()
+                self.s = torch.nn.Parameter(torch.ones((), device=dev, dtype=torch.bfloat16))
+
+            def forward(self, w):
+                return w * self.s
+
+        scale = Scale()
+        torch.nn.utils.parametrize.register_parametrization(mlp.down_proj, "weight", scale)
+        assert torch.equal(run(), want)
+        scale.s.fill_(-1.0)
+        assert not torch.equal(run(), want)
+        mlp.down_proj.parametrizations.weight.original.neg_()
+        assert torch.equal(run(), want)
+
+
 def test_a_written_or_replaced_parameter_is_seen(dev):
     model = build(dev, torch.bfloat16, 160, True)
     ids = torch.randint(0, 500, (1, 20), device=dev)

@@ -357,3 +357,45 @@ def test_a_plan_sees_every_change_it_depends_on(monkeypatch):
     with monkeypatch.context() as patch:
         patch.setattr(torch.nn.Module, "__call__", lambda self, *a, **k: None)
         assert not plain.current(layer)
+
+
+def test_codes_are_packed_anew_for_another_tensor_at_the_same_place(monkeypatch):
+    """A weight that is computed on each access (a parametrisation) may lie where the last one did, version 0 again: the codes
+    kept from the last one are not its codes.  Nor does a stacked weight outlive its parts."""
+    import copy
+    import pickle
+    import matmulfreellm_amd as mm
+    from matmulfreellm_amd import functional as F_
+    monkeypatch.setattr(F_, "ternarize_pack", lambda w: F_.PackedWeight(w.clone(), None, *w.shape, w.shape[0]))
+    monkeypatch.setattr(F_, "stack_packed", lambda parts: torch.cat([p.packed for p in parts]))
+    memory = bytearray(4 * 64)
+    at = lambda: torch.frombuffer(memory, dtype=torch.float32).view(8, 8)
+    layer = mm.FusedBitLinear(8, 8)
+    first = at()
+    kept = layer._pack.get(first)
+    assert layer._pack.get(first) is kept
+    memory[:] = bytes(range(64)) * 4
+    second = at()
+    assert second.data_ptr() == first.data_ptr() and second._version == first._version
+    assert torch.equal(layer._pack.get(second).packed, second)
+    again = layer._pack.get(second)
+    second.add_(1.0)
+    assert layer._pack.get(second) is not again
+    seen = F_.Seen()
+    seen.take(first, second)
+    assert seen.unchanged(first, second) and not seen.unchanged(second, first) and not seen.unchanged(first)
+    assert not any(c.unchanged(first, second) for c in (copy.deepcopy(seen), copy.copy(seen), pickle.loads(pickle.dumps(seen))))
+    del first, second
+    assert not seen.unchanged(at(), at())
+
+    attn = mm.HGRNBitAttention(hidden_size=32)
+    stacked = attn._stacked_weight()
+    assert attn._stacked_weight() is stacked and attn._stacked_ifg() is stacked
+    with torch.no_grad():
+        attn.f_proj.weight.mul_(-1.0)
+    assert torch.equal(attn._stacked_weight()[32:64], attn.f_proj.weight) and attn._stacked_ifg() is attn._stacked_weight()
+    attn.g_proj.fused_eps = 0.5
+    assert attn._stacked_ifg() is None
+    attn.g_proj.fused_eps = attn.i_proj.fused_eps
+    attn.g_proj.norm.weight = torch.nn.Parameter(torch.full((32,), 2.0))
+    assert attn._stacked_ifg() is None and attn._stacked_weight() is not None
