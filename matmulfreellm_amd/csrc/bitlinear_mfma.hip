@@ -886,13 +886,18 @@ int launch_mfma(MfmaArgs a, hipStream_t s) {
     return 0;
 }
 
-// Which kernel is the fastest, from its measured time on MI355X (us, N from 1024 to 11264, K from 1024 to 5632, M from 77 to 8192):
+// Which kernel is the fastest, from its measured time on MI355X (us; N from 1024 to 11264, K from 1024 to 9216, M from 77 to 11500):
 //   weight stream  3 + 0.7 ns per output block + 0.18 ns per output block and k-block, as long as the row fits its LDS;
 //   split tiles    (64 x 256, two groups of waves on every second k-block) one round of at most one tile per CU: a chain of
-//                  0.29 us per k-block, and what a fuller chip adds.  Beyond one round they only add traffic: 2048 over
-//                  6144 columns at M 777 (312 tiles) 17.0 us against 15.3 -- except where two rounds of whole tiles would leave
-//                  the second one more than half empty: the same columns at M 1377 (528 against 264 tiles) 26.1 against 27.5;
+//                  0.29 us per k-block, and what a fuller chip adds.  Beyond one round, 3.4 + 0.345 us per k-block for each;
 //   tiles          (64 x 512) 4 + 0.6 us per k-block and round.
+// A whole tile is worth two split ones, so against an even number of split rounds whole tiles win or tie (by 0 to 50 %, least on the longest
+// rows).  Where two rounds of whole tiles would leave the second less than half full, three split rounds do instead of four.  Split against
+// whole at 513 to 768 split tiles: 8 k-blocks (1024 -> 5632, 2099 rows) 21.2 / 19.3, (1024 -> 1024, 8448) 18.2 / 17.9; 12 (1536 -> 3072,
+// 2995) 23.7 / 23.0; 14, where the line lies, 0.96 to 1.05; 16 (2048 -> 6144, 1395) 26.3 / 27.7, (2048 -> 2048, 5107) 26.5 / 28.2,
+// (2048 -> 11264, 960) 27.3 / 28.1; 20 (2560 -> 7680, 1203) 30.7 / 32.6; 22 (2816 -> 1024, 9600) 33.0 / 35.3; 44 (5632 -> 2048, 4467)
+// 55.7 / 61.2.  Five split rounds for three of whole tiles: 42.3 / 42.5 at 16 k-blocks, 94 / 100 at 44 (left to whole tiles), 148 / 159 at
+// 72 (taken).
 // 2002 x 5632 -> 2048: stream 37 us, split 23, tiles 31; 1377 x 2048 -> 2048: 12.2 / 10.5 / 14.3.
 enum class MfmaPick { kStream, kSplit, kTiles };
 inline MfmaPick mfma_pick(const MfmaArgs& a) {
@@ -902,8 +907,8 @@ inline MfmaPick mfma_pick(const MfmaArgs& a) {
     const double t_stream = 3.0 + blocks * (0.0007 + 0.00018 * (double)((KB + 7) / 8 * 8));
     const double t_tiles = (double)mmf_ceil_div(full, 256) * (4.0 + 0.6 * kb);
     double t_split = 1e30;
-    if (KB % 2 == 0 && half <= 256) t_split = 4.4 + 0.29 * kb + (double)half / 256.0 * (1.0 + 0.1 * kb);
-    if (KB % 2 == 0 && KB >= 16 && half > 512 && half <= 768) t_split = 0.95 * t_tiles;
+    if (KB % 2 == 0)
+        t_split = half <= 256 ? 4.4 + 0.29 * kb + (double)half / 256.0 * (1.0 + 0.1 * kb) : (double)mmf_ceil_div(half, 256) * (3.4 + 0.345 * kb);
     if (a.Kp <= 8192 && a.M <= 65535 * 32 && (a.M <= 64 || (t_stream <= t_split && t_stream <= t_tiles))) return MfmaPick::kStream;
     return t_split < t_tiles ? MfmaPick::kSplit : MfmaPick::kTiles;
 }

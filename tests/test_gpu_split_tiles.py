@@ -45,3 +45,13 @@ def test_segments_contract_their_own_codes(dev, seg):
     for s in range(3):
         alone = F.bitlinear_mfma(q[s], deq[s], qsum[s], pw, m, torch.bfloat16, config=5)
         assert torch.equal(out[:, s * seg:(s + 1) * seg], alone[:, s * seg:(s + 1) * seg]), s
+
+
+@pytest.mark.parametrize("m,k,n", [(3968, 2048, 2048), (4147, 2048, 2048), (6387, 2048, 2048), (1216, 1792, 7168), (1216, 1536, 7168),
+                                   (8256, 8704, 2048)])
+def test_the_kernel_picked_beyond_one_round_of_split_tiles_gives_the_same_bits(dev, m, k, n):
+    """496, 520 and 800 split tiles (two, three and four rounds of 256), 14 and 12 k-blocks at three rounds, five rounds of long rows."""
+    F, lib, pw, q, codes, deq, qsum = operands(dev, m, k, n, seed=4)
+    picked = F.bitlinear_mfma(q[0], deq[0], qsum[0], pw, m, torch.bfloat16)
+    for config in (16, 17, 18):
+        assert torch.equal(picked, F.bitlinear_mfma(q[0], deq[0], qsum[0], pw, m, torch.bfloat16, config=config)), config
