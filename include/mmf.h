@@ -416,10 +416,10 @@ typedef struct {
 int64_t mmf_block_struct_bytes(void);
 int64_t mmf_block_workspace_bytes(const mmf_block* p, int64_t rows);
 /* mmf_block_train_forward: the same block with what its backward needs kept apart: ifg [M, 3D] (raw projections), xg [2, M, D] (the
- * scan's input and gate), o [M, D], res [M, H] (attention output + x), y [M, 2I] (gate and up); no state.  workspace:
+ * scan's input and gate), o [M, D], attn [M, H] (attention output), y [M, 2I] (gate and up); no state.  workspace:
  * mmf_block_train_workspace_bytes(p, M) bytes. */
 int64_t mmf_block_train_workspace_bytes(const mmf_block* p, int64_t rows);
-int mmf_block_train_forward(const mmf_block* p, const void* x, void* out, void* ifg, void* xg, void* o, void* res, void* y, int64_t B,
+int mmf_block_train_forward(const mmf_block* p, const void* x, void* out, void* ifg, void* xg, void* o, void* attn, void* y, int64_t B,
                             int64_t T, const float* lower_bound, const uint8_t* mask, void* workspace, void* stream);
 int mmf_block_forward(const mmf_block* p, const void* x, void* out, int64_t B, int64_t T, const float* lower_bound,
                       const uint8_t* mask, const float* h0, float* ht, void* workspace, void* stream);
@@ -427,10 +427,11 @@ int mmf_block_forward(const mmf_block* p, const void* x, void* out, int64_t B, i
 /* ---- backward of a block between its dense products (csrc/backward_block.hip)
  * mmf_chain_bwd: the gradient through one BitLinear norm (or three that share their input) and the op in front of it, in one
  *   pass over the rows.  kind 0: norm(x; w1, eps1), with dres (null, or [M, K]) added to dx; kind 1: norm(x; w1, eps1) * aux *
- *   sigmoid(aux); kind 2: swiglu(x, aux).  w2 / dy: HOST arrays of `norms` device pointers: norm weights and the gradients dout @ W_q
+ *   sigmoid(aux); kind 2: swiglu(x, aux); kind 3: norm(x + aux; w1, eps1), the sum unrounded, with dres as kind 0 and dx the gradient
+ *   of the sum (daux ignored).  w2 / dy: HOST arrays of `norms` device pointers: norm weights and the gradients dout @ W_q
  *   of the quantised inputs (row stride lddy).  Writes dx, daux, y [norms, M, K] (the de-quantised codes the weight gradients
- *   contract with, the forward's bit for bit) and dweights [(kind < 2) + norms, K] (w1 first) in the weights' type; part:
- *   mmf_chain_bwd_groups(M) * ((kind < 2) + norms) * K floats of scratch.  K a multiple of 4, at most 8192 (4096 with three norms).
+ *   contract with, the forward's bit for bit) and dweights [(kind != 2) + norms, K] (w1 first) in the weights' type; part:
+ *   mmf_chain_bwd_groups(M) * ((kind != 2) + norms) * K floats of scratch.  K a multiple of 4, at most 8192 (4096 with three norms).
  * mmf_unpack_dequant: out [N, K] = ternary code * wdeq[row / seg_rows], in `dtype`. */
 int mmf_chain_bwd_groups(int64_t rows);
 int mmf_chain_bwd(int kind, const void* x, int64_t ldx, const void* aux, int64_t ldaux, const void* w1, float eps1, int norms,

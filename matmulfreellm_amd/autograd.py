@@ -222,7 +222,7 @@ def _scan_bwd(g, o, do, h0, log_gates):
     return dx, dg
 
 
-CHAIN_NORM, CHAIN_GATED, CHAIN_SWIGLU = 0, 1, 2
+CHAIN_NORM, CHAIN_GATED, CHAIN_SWIGLU, CHAIN_RESNORM = 0, 1, 2, 3
 
 
 def _chain_bwd(kind, x, aux, w1, eps1, w2, eps2, dy, dres=None, dx=None, daux=None):
@@ -271,20 +271,20 @@ class BlockFn(torch.autograd.Function):
         dev, dt = x.device, x.dtype
         with L.on(dev):
             empty = lambda *shape: torch.empty(*shape, dtype=dt, device=dev)
-            out, ifg, xg, o, res, y = torch.empty_like(x), empty(m, 3 * D), empty(2, m, D), empty(m, D), empty(m, H), empty(m, 2 * I)
+            out, ifg, xg, o, attn, y = torch.empty_like(x), empty(m, 3 * D), empty(2, m, D), empty(m, D), empty(m, H), empty(m, 2 * I)
             lb = lower_bound.detach().float().contiguous() if lower_bound is not None else None
             mk = F_._mask_rows(mask, m, dev)
             ws = torch.empty(lib.mmf_block_train_workspace_bytes(plan.ref, m), dtype=torch.uint8, device=dev)
             L.check(lib.mmf_block_train_forward(plan.ref, x.data_ptr(), out.data_ptr(), ifg.data_ptr(), xg.data_ptr(), o.data_ptr(),
-                                                res.data_ptr(), y.data_ptr(), b, t, L.ptr(lb), L.ptr(mk), ws.data_ptr(), L.stream()),
+                                                attn.data_ptr(), y.data_ptr(), b, t, L.ptr(lb), L.ptr(mk), ws.data_ptr(), L.stream()),
                     "mmf_block_train_forward")
-        ctx.save_for_backward(x, lb, mk, ifg, xg, o, res, y, *params[:9])
+        ctx.save_for_backward(x, lb, mk, ifg, xg, o, attn, y, *params[:9])
         ctx.plan, ctx.lb_dtype = plan, lower_bound.dtype if lower_bound is not None else None
         return out
 
     @staticmethod
     def backward(ctx, dout):
-        x, lb, mk, ifg, xg, o, res, y, *nw = ctx.saved_tensors
+        x, lb, mk, ifg, xg, o, attn, y, *nw = ctx.saved_tensors
         attn_norm, mlp_norm, g_norm, i_n, f_n, gp_n, o_n, gate_n, down_n = nw
         plan, need = ctx.plan, ctx.needs_input_grad[4:]
         H, D, I = plan.dims
@@ -303,7 +303,8 @@ class BlockFn(torch.autograd.Function):
             d_down = d2.t() @ yq[0] if need[14] else None
             # gate_proj behind mlp_norm, the residual's gradient joining
             dh = dy @ _dequantised(gate_pw, dt)
-            dres, _, yq, dw_gate = _chain_bwd(CHAIN_NORM, res, None, mlp_norm, eps["mlp_eps"], [gate_n], eps["gate_eps"], [dh], dres=d2)
+            dres, _, yq, dw_gate = _chain_bwd(CHAIN_RESNORM, attn, x.view(m, H), mlp_norm, eps["mlp_eps"], [gate_n], eps["gate_eps"], [dh],
+                                               dres=d2)
             d_gate = dy.t() @ yq[0] if need[13] else None
             # o_proj behind the gated norm: the g columns of the stacked projection's gradient, and the scan's output
             do2 = dres @ _dequantised(o_pw, dt)

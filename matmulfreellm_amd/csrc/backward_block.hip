@@ -1,7 +1,8 @@
 // Backward of an HGRNBit block between its dense products: the row kernels that carry a gradient through a BitLinear's norm
 // AND the elementwise op in front of it in one pass, and the ternary weights as a dense matrix.
 //
-//   mmf_chain_bwd        CHAIN_NORM    norm(x; w1) -> 1 or 3 BitLinears' norms (block norm in front of i/f/g, of gate/up, of the head)
+//   mmf_chain_bwd        CHAIN_NORM    norm(x; w1) -> 1 or 3 BitLinears' norms (block norm in front of i/f/g, norm in front of the head)
+//                        CHAIN_RESNORM norm(x + a; w1) -> a BitLinear's norm (residual and mlp_norm in front of gate/up)
 //                        CHAIN_GATED   norm(x; w1) * a * sigmoid(a) -> a BitLinear's norm (g_norm in front of o_proj)
 //                        CHAIN_SWIGLU  swiglu(x, a) -> a BitLinear's norm (the MLP activation in front of down_proj)
 //     i.e. mmfreelm/ops/fusedbitnet.py:209-317 followed by mmfreelm/modules/layernorm.py:245-330,
@@ -16,14 +17,14 @@
 
 namespace {
 
-enum Chain : int { CHAIN_NORM = 0, CHAIN_GATED = 1, CHAIN_SWIGLU = 2 };
+enum Chain : int { CHAIN_NORM = 0, CHAIN_GATED = 1, CHAIN_SWIGLU = 2, CHAIN_RESNORM = 3 };
 
 struct ChainArgs {
     const void* x; const void* aux;     // the op's inputs, row strides ldx, ldaux
-    const void* w1;                     // NORM, GATED: weight of the norm in front
+    const void* w1;                     // all but SWIGLU: weight of the norm in front
     const void* w2[3];                  // the BitLinears' norm weights
     const void* dy[3];                  // gradients of their normalised inputs (dout @ W_q), row stride lddy
-    const void* dres;                   // NORM: null, or a gradient that joins dx (the residual branch), row stride K
+    const void* dres;                   // NORM, RESNORM: null, or a gradient that joins dx (the residual branch), row stride K
     void* dx; void* daux;               // gradients of x and aux, row strides lddx, lddaux
     void* y;                            // [NN][M, K]: the de-quantised codes of the BitLinears' inputs
     float* part;                        // [gridDim.x][W1 + NN][K]: sums for w1, then for the w2
@@ -42,7 +43,10 @@ struct ChainArgs {
 // one to two on a SIMD, 159 us.
 template <typename T, typename TW, int KT, int NV, int ST, int NN>
 __global__ __launch_bounds__(KT) void chain_bwd_kernel(ChainArgs a) {
-    constexpr bool W1 = ST != CHAIN_SWIGLU, AUX = ST != CHAIN_NORM, RES = ST == CHAIN_NORM;
+    // RESNORM adds its operands again instead of reading their rounded sum: the forward normalised the unrounded one, and from the rounded
+    // one 4.5 % of the bf16 codes come out as others (8192 x 2048), which put gate_proj's weight gradient 8.7e-3 from the exact one
+    // where it is 3.3e-3 now.  The second operand's load hides: 54 us with either (column sums included).
+    constexpr bool W1 = ST != CHAIN_SWIGLU, AUX = ST != CHAIN_NORM, ADD = ST == CHAIN_RESNORM, RES = ST == CHAIN_NORM || ADD;
     constexpr int kW = KT / 64;
     __shared__ double s_sum1[kW], s_sum2[kW];
     __shared__ float s_max[NN][kW], s_dot2[kW], s_dot1[kW];
@@ -104,6 +108,7 @@ __global__ __launch_bounds__(KT) void chain_bwd_kernel(ChainArgs a) {
             const bool in = in_row(v);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
+                if constexpr (ADD) x[v][i] = __fadd_rn(x[v][i], av[v][i]);
                 x[v][i] = in ? x[v][i] : 0.0f;
                 if constexpr (AUX) av[v][i] = in ? av[v][i] : 0.0f;
 #pragma unroll
@@ -222,7 +227,7 @@ __global__ __launch_bounds__(KT) void chain_bwd_kernel(ChainArgs a) {
                     dot1 += xh * wd[v][i];
                 }
             }
-            if constexpr (AUX) raw4_store<T, true>(static_cast<T*>(a.daux) + row * a.lddaux, k0, K, o);
+            if constexpr (AUX && !ADD) raw4_store<T, true>(static_cast<T*>(a.daux) + row * a.lddaux, k0, K, o);
             if constexpr (ST == CHAIN_SWIGLU) raw4_store<T, true>(static_cast<T*>(a.dx) + row * a.lddx, k0, K, x[v]);
         }
         if constexpr (W1) {
@@ -302,6 +307,7 @@ template <typename T, typename TW>
 int dispatch_chain(const ChainArgs& a, int kind, int n, int groups, void* dw, hipStream_t s) {
     switch (kind) {
         case CHAIN_NORM: return n == 3 ? launch_chain<T, TW, CHAIN_NORM, 3>(a, groups, dw, s) : launch_chain<T, TW, CHAIN_NORM, 1>(a, groups, dw, s);
+        case CHAIN_RESNORM: return launch_chain<T, TW, CHAIN_RESNORM, 1>(a, groups, dw, s);
         case CHAIN_GATED: return launch_chain<T, TW, CHAIN_GATED, 1>(a, groups, dw, s);
         case CHAIN_SWIGLU: return launch_chain<T, TW, CHAIN_SWIGLU, 1>(a, groups, dw, s);
     }
@@ -354,11 +360,13 @@ int mmf_chain_bwd(int kind, const void* x, int64_t ldx, const void* aux, int64_t
                   void* daux, int64_t lddaux, void* y, float* part, void* dweights, int64_t M, int64_t K, int x_dtype, int weight_dtype,
                   void* stream_) {
     hipStream_t stream = static_cast<hipStream_t>(stream_);
-    if (kind < CHAIN_NORM || kind > CHAIN_SWIGLU || M < 0 || K <= 0 || ldx < K || lddy < K || lddx < K) return MMF_ERR_ARG;
+    if (kind < CHAIN_NORM || kind > CHAIN_RESNORM || M < 0 || K <= 0 || ldx < K || lddy < K || lddx < K) return MMF_ERR_ARG;
     if (M == 0) return 0;
     if (!(norms == 1 || (norms == 3 && kind == CHAIN_NORM)) || !x || !w2 || !dy || !dx || !y || !part || !dweights) return MMF_ERR_ARG;
     if (kind != CHAIN_SWIGLU && !w1) return MMF_ERR_ARG;
-    if (kind != CHAIN_NORM && (!aux || !daux || ldaux < K || lddaux < K || dres)) return MMF_ERR_ARG;
+    if (kind != CHAIN_NORM && (!aux || ldaux < K)) return MMF_ERR_ARG;
+    const bool two = kind == CHAIN_GATED || kind == CHAIN_SWIGLU;             // gradients of both operands
+    if (two && (!daux || lddaux < K || dres)) return MMF_ERR_ARG;
     if (K % 4 != 0 || K > 8192) return MMF_ERR_WIDE;
     ChainArgs a{};
     a.x = x; a.aux = aux; a.w1 = w1; a.dres = dres; a.dx = dx; a.daux = daux; a.y = y; a.part = part;
@@ -371,7 +379,7 @@ int mmf_chain_bwd(int kind, const void* x, int64_t ldx, const void* aux, int64_t
     a.eps1 = eps1; a.eps2 = eps2; a.inv_K = 1.0 / (double)K;
     const uintptr_t xm = 4 * (x_dtype == MMF_F32 ? 4 : 2) - 1, wm = 4 * (weight_dtype == MMF_F32 ? 4 : 2) - 1;
     auto off = [](const void* p, uintptr_t m) { return (reinterpret_cast<uintptr_t>(p) & m) != 0; };
-    for (int64_t ld : {ldx, kind != CHAIN_NORM ? ldaux : 0, lddy, lddx, kind != CHAIN_NORM ? lddaux : 0})
+    for (int64_t ld : {ldx, kind != CHAIN_NORM ? ldaux : 0, lddy, lddx, two ? lddaux : 0})
         if (ld % 4 != 0) return MMF_ERR_ALIGN;
     for (const void* p : {x, aux, dres, (const void*)dx, (const void*)daux, (const void*)y, a.dy[0], a.dy[1], a.dy[2]})
         if (off(p, xm)) return MMF_ERR_ALIGN;

@@ -39,7 +39,7 @@ int project_ifg(const mmf_block* p, const void* x, int64_t M, int8_t* q, float* 
 
 // Offsets of the intermediates in the workspace (each 256-byte aligned).
 struct Layout {
-    int64_t ifg = 0, o = 0, attn, res = 0, big = 0, q, deq, qsum, bytes = 0;
+    int64_t ifg = 0, o = 0, attn = 0, res, big = 0, q, deq, qsum, bytes = 0;
     Layout(const mmf_block* p, int64_t M, bool train) {
         const int64_t e = esize(p);
         auto take = [&](int64_t n) {
@@ -47,11 +47,11 @@ struct Layout {
             bytes += mmf_round_up(n, 256);
             return at;
         };
-        attn = take(M * p->H * e);
+        res = take(M * p->H * e);
         if (!train) {                                            // training keeps these in tensors of the caller's
+            attn = take(M * p->H * e);
             ifg = take(M * 3 * p->D * e);
             o = take(M * p->D * e);
-            res = take(M * p->H * e);
             big = take(M * p->I * e);                            // the MLP's activation
         }
         int64_t codes = 3 * mmf_codes_bytes(M, p->H, 1);
@@ -79,16 +79,16 @@ int64_t mmf_block_train_workspace_bytes(const mmf_block* p, int64_t rows) {
     return Layout(p, rows, true).bytes;
 }
 
-int mmf_block_train_forward(const mmf_block* p, const void* x, void* out, void* ifg, void* xg, void* o, void* res, void* y, int64_t B,
+int mmf_block_train_forward(const mmf_block* p, const void* x, void* out, void* ifg, void* xg, void* o, void* attn, void* y, int64_t B,
                             int64_t T, const float* lower_bound, const uint8_t* mask, void* workspace, void* stream) {
     if (!p || B < 0 || T < 0 || p->H <= 0 || p->D <= 0 || p->I <= 0 || p->D % 32 || p->I % 32) return MMF_ERR_ARG;
     const int64_t M = B * T, H = p->H, D = p->D, I = p->I, e = esize(p);
     if (M == 0) return 0;
-    if (!x || !out || !ifg || !xg || !o || !res || !y || !workspace) return MMF_ERR_ARG;
+    if (!x || !out || !ifg || !xg || !o || !attn || !y || !workspace) return MMF_ERR_ARG;
     if (reinterpret_cast<uintptr_t>(workspace) & 255u) return MMF_ERR_ALIGN;
     const Layout L(p, M, true);
     char* w = static_cast<char*>(workspace);
-    void* attn = w + L.attn;
+    void* res = w + L.res;
     int8_t* q = reinterpret_cast<int8_t*>(w + L.q);
     float* deq = reinterpret_cast<float*>(w + L.deq);
     int* qsum = reinterpret_cast<int*>(w + L.qsum);
