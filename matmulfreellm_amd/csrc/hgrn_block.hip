@@ -60,8 +60,9 @@ __device__ __forceinline__ unsigned column_block() {
 __device__ __forceinline__ void wait_turn(int& turn, int n) {
     while (__hip_atomic_load(&turn, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) != n) __builtin_amdgcn_s_sleep(1);
 }
-// What the carry c makes of a run of steps with the product P and the own contribution l.
-__device__ __forceinline__ float fold(float l, float P, float c) { return fmaf(P, c, l); }
+// What the carry c makes of a run of steps with the product P and the own contribution l.  (A zero carry stays zero also where
+// a product of gates beyond one has overflowed.)
+__device__ __forceinline__ float fold(float l, float P, float c) { return c == 0.0f ? l : fmaf(P, c, l); }
 // The parts of a wave's block in the order the scan takes them, k = 0 .. LS - 1 in lanes part(k): (lin, Pin) composes the parts
 // in front of this lane's, (lb, Pb) all of them.
 template <int LS, bool REVERSE>

@@ -84,3 +84,25 @@ def test_scans_round_once_per_step(dev, bhtd, log):
     assert rel(dx, torch.stack(dhs[::-1], 2)) < (5e-8 if log else 4.2e-8)
     assert rel(o, torch.stack(hs, 2)) < 5e-8
     assert rel(last, h) < 6e-8                       # as few as 128 values (their mean scatters by 5 %): one unit roundoff
+
+
+@pytest.mark.parametrize("log", [False, True])
+def test_a_zero_carry_survives_a_product_of_gates_that_overflows(dev, log):
+    """40 gates of 1e4 (not a decay, but taken): their product is infinite, and what enters or leaves them is zero."""
+    import matmulfreellm_amd as mm
+    t = 200
+    a = torch.full((1, 1, t, 64), 0.5)
+    a[:, :, 60:100] = 1e4
+    x, do = torch.zeros(1, 1, t, 64), torch.zeros(1, 1, t, 64)
+    do[:, :, :50] = 1.0
+    if not log:
+        x[:, :, 150:] = 1.0
+    g = a.log() if log else a
+    mine = [v.to(dev).requires_grad_() for v in (x, g)]
+    o, _ = (mm.chunk_hgrn if log else mm.fused_recurrent_hgrn)(*mine)
+    dx, dg = torch.autograd.grad(o, mine, do.to(dev))
+    want = torch.zeros(t)
+    for k in reversed(range(50)):
+        want[k] = 1.0 + 0.5 * want[k + 1]
+    assert torch.isfinite(o).all() and torch.isfinite(dg).all()
+    assert torch.allclose(dx[0, 0, :, 0].cpu(), want, rtol=1e-6, atol=0)
