@@ -14,6 +14,7 @@
 // quantised activations that the weight gradient contracts with are recomputed in the forward's arithmetic, bit for bit;
 // gradients are fp32 between the stages.
 #include "mmf_common.h"
+#include "column_sum.h"
 
 namespace {
 
@@ -256,35 +257,6 @@ __global__ __launch_bounds__(KT) void chain_bwd_kernel(ChainArgs a) {
     }
 }
 
-// out[k] = T(sum_g part[g, k]).  A workgroup owns 32 columns; its 32 lanes per column each add every 32nd group in index order and
-// the 32 lane sums are then added in lane order, so the result depends on the shape only.
-constexpr int kCols = 32, kLanes = 32;
-template <typename T>
-__global__ __launch_bounds__(kCols * kLanes) void colsum_rows_kernel(const float* __restrict__ part, int groups, int K, T* __restrict__ out) {
-    __shared__ float lane_sum[kLanes][kCols + 1];
-    const int c = (int)threadIdx.x % kCols, l = (int)threadIdx.x / kCols;
-    const int k = (int)blockIdx.x * kCols + c;
-    float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
-    if (k < K) {
-        int g = l;
-        for (; g + 3 * kLanes < groups; g += 4 * kLanes) {
-            s0 += part[(int64_t)g * K + k];
-            s1 += part[(int64_t)(g + kLanes) * K + k];
-            s2 += part[(int64_t)(g + 2 * kLanes) * K + k];
-            s3 += part[(int64_t)(g + 3 * kLanes) * K + k];
-        }
-        for (; g < groups; g += kLanes) s0 += part[(int64_t)g * K + k];
-    }
-    lane_sum[l][c] = (s0 + s1) + (s2 + s3);
-    __syncthreads();
-    if (l == 0 && k < K) {
-        float s = 0.0f;
-#pragma unroll
-        for (int i = 0; i < kLanes; ++i) s += lane_sum[i][c];
-        out[k] = mmf_from_float<T>(s);
-    }
-}
-
 template <typename T, typename TW, int ST, int NN>
 int launch_chain(const ChainArgs& a, int groups, void* dw, hipStream_t s) {
     if (a.K <= 1024) chain_bwd_kernel<T, TW, 256, 1, ST, NN><<<groups, 256, 0, s>>>(a);
@@ -299,7 +271,7 @@ int launch_chain(const ChainArgs& a, int groups, void* dw, hipStream_t s) {
     } else return MMF_ERR_WIDE;
     MMF_CHECK_LAUNCH();
     const int cols = ((ST != CHAIN_SWIGLU ? 1 : 0) + NN) * a.K;
-    colsum_rows_kernel<TW><<<(unsigned)mmf_ceil_div(cols, kCols), kCols * kLanes, 0, s>>>(a.part, groups, cols, static_cast<TW*>(dw));
+    launch_colsum(a.part, groups, cols, static_cast<TW*>(dw), s);
     MMF_CHECK_LAUNCH();
     return 0;
 }

@@ -482,8 +482,6 @@ __device__ __forceinline__ float mmf_rstd(double sumsq, int64_t K, double inv_K,
     return mmf_rcp_pos(mmf_sqrt_pos(__fadd_rn(var, eps)));   // == 1 / sqrtf(var + eps), both correctly rounded
 }
 
-// int8 code of one normalised value:  clamp(rint(y * scale), -128, 127)
-
 // The codes of four neighbouring values in the bytes of a dword, and their sum.  Adding 1.5 * 2^23 to a value of at most 128 rounds it to
 // an integer (nearest, ties to even, as rintf does) whose low byte is the low byte of the sum: three operations a value and
 // three for the dword, where rint, clamp, convert, mask and shift took nine a value.
@@ -497,7 +495,7 @@ __device__ __forceinline__ uint32_t mmf_code4(const float (&y)[4], float scale) 
 __device__ __forceinline__ int mmf_code4_sum(uint32_t codes, int sum) {
     return __builtin_amdgcn_sdot4((int)codes, 0x01010101, sum, false);
 }
-// the code of one value as a float
+// int8 code of one normalised value, as a float: clamp(rint(y * scale), -128, 127)
 __device__ __forceinline__ float mmf_code_f(float y, float scale) { return fminf(fmaxf(rintf(__fmul_rn(y, scale)), -128.0f), 127.0f); }
 
 __host__ __device__ static inline int64_t mmf_ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
