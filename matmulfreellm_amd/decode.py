@@ -67,9 +67,12 @@ class DecodeEngine(NotCopied):
         self.use_graph = use_graph
         # what the operands below were taken from: modules, parameters (object, version, address); nothing here leads back to the model,
         # which holds this engine
-        self._children = [(d["_modules"], k, c) for d in (m.__dict__ for m in model.modules()) for k, c in d["_modules"].items()]
-        self._parameters = [(d["_parameters"], k, p, p._version, p.data_ptr()) for d in (m.__dict__ for m in model.modules())
+        dicts = [m.__dict__ for m in model.modules()]
+        self._children = [(d["_modules"], k, c) for d in dicts for k, c in d["_modules"].items()]
+        self._parameters = [(d["_parameters"], k, p, p._version, p.data_ptr()) for d in dicts
                             for k, p in d["_parameters"].items() if p is not None]
+        self._absent = [(d["_parameters"], k) for d in dicts for k, p in d["_parameters"].items() if p is None]
+        self._sizes = [(d[name], len(d[name])) for d in dicts for name in ("_modules", "_parameters")]
 
         attn0 = model.model.layers[0].attn
         self.D = D = attn0.input_dim
@@ -153,14 +156,14 @@ class DecodeEngine(NotCopied):
         return float(p.norm.eps if getattr(p, "fused_eps", None) is None else p.fused_eps)
 
     def stale(self):
-        """Whether a module or parameter the engine was built on has been replaced or written since."""
+        """Whether a module or parameter the engine was built on has been replaced or written since, or one has come or gone."""
         for d, k, p, version, address in self._parameters:
             if d.get(k) is not p or p._version != version or p.data_ptr() != address:
                 return True
         for d, k, c in self._children:
             if d.get(k) is not c:
                 return True
-        return False
+        return any(len(d) != n for d, n in self._sizes) or any(d.get(k) is not None for d, k in self._absent)
 
     # ------------------------------------------------------------------ launches
     def _bitlinear(self, x, pw_nw_eps, out, n_k, addend=None):

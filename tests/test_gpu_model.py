@@ -680,3 +680,28 @@ def test_wide_vocabulary_sampling_fallback(dev, tiny_bf16, monkeypatch):
     assert outs[0].shape == (3, 18) and torch.equal(outs[0], outs[1])
     cpu_gen = model.generate(ids, generator=torch.Generator().manual_seed(5), **kw)      # a CPU generator is accepted too
     assert cpu_gen.shape == (3, 18)
+
+
+def test_generate_sees_a_layer_or_a_bias_added_after_the_engine_was_built(dev):
+    """The engine kept from an earlier call is not one for a model with a layer more, or with a bias where there was none."""
+    import copy
+    import matmulfreellm_amd as mm
+    torch.manual_seed(4)
+    model = mm.HGRNBitForCausalLM(mm.HGRNBitConfig(vocab_size=500, hidden_size=256, num_hidden_layers=3, eos_token_id=None,
+                                                   use_lower_bound=False)).to(dev, torch.bfloat16).eval()
+    ids = torch.randint(0, 500, (1, 9), device=dev)
+    run = lambda graph: model.generate(ids, max_new_tokens=12, use_graph=graph)
+    extra = copy.deepcopy(model.model.layers[2])
+    extra.attn.layer_idx = 3
+    with torch.no_grad():
+        extra.mlp.down_proj.weight.neg_()
+    first = run(True)
+    assert torch.equal(first, run(False))
+    model.model.layers.append(extra)
+    longer = run(True)
+    assert torch.equal(longer, run(False)) and not torch.equal(longer, first)
+    del model.model.layers[3]
+    assert torch.equal(run(True), first)
+    model.model.layers[1].mlp.down_proj.bias = torch.nn.Parameter(torch.ones(256, device=dev, dtype=torch.bfloat16))
+    with pytest.raises(NotImplementedError):
+        run(True)
