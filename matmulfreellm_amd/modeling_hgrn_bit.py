@@ -418,7 +418,12 @@ class HGRNBitForCausalLM(HGRNBitPreTrainedModel, GenerationMixin):
         fold = self._folds_final_norm(output_hidden_states, train)
         args = dict(input_ids=input_ids, attention_mask=attention_mask, inputs_embeds=inputs_embeds, past_key_values=past_key_values,
                     use_cache=use_cache, output_attentions=output_attentions, output_hidden_states=output_hidden_states, return_dict=True)
-        outputs = self.model._forward(train, **args, final_norm=False) if fold else self.model(**args)
+        if fold:                                         # as HGRNBitModel.forward: a frozen body runs as in inference below a trained head
+            body = module_needs_grad(self.model, inputs_embeds)
+            with torch.enable_grad() if body else torch.no_grad():
+                outputs = self.model._forward(body, **args, final_norm=False)
+        else:
+            outputs = self.model(**args)
         hidden_states = outputs.last_hidden_state
         if logits_to_keep:
             hidden_states = hidden_states[:, -logits_to_keep:, :]

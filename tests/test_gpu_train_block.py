@@ -49,6 +49,39 @@ def test_block_step_equals_the_composition(dev, dtype, hidden, b, t, masked, lb)
         assert err < (2e-5 if dtype == torch.float32 else 2e-2), (name, err)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_a_trained_head_on_a_frozen_body_keeps_the_cache(dev, dtype):
+    """Gradients enabled, only the head's parameters ask for one: the body runs as in inference, takes and returns a cache; the
+    head's gradients are those of the modules one by one."""
+    import matmulfreellm_amd as mm
+    torch.manual_seed(29)
+    model = mm.HGRNBitForCausalLM(mm.HGRNBitConfig(vocab_size=200, hidden_size=96, num_hidden_layers=2)).to(dev, dtype)
+    model.model.requires_grad_(False)
+    ids, more = (torch.randint(0, 200, (2, n), device=dev) for n in (7, 1))
+    with torch.no_grad():
+        want = model(input_ids=ids, use_cache=True)
+        want_next = model(input_ids=more, past_key_values=want.past_key_values, use_cache=True)
+    out = model(input_ids=ids, use_cache=True)
+    assert torch.equal(out.logits, want.logits) and out.logits.requires_grad
+    step = model(input_ids=more, past_key_values=out.past_key_values, use_cache=True)
+    assert torch.equal(step.logits, want_next.logits)
+    _, got = step_of(model, ids)
+    hook = model.model.norm.register_forward_hook(lambda *a: None)
+    _, ref = step_of(model, ids)
+    hook.remove()
+    assert set(got) == {"lm_head.weight", "lm_head.norm.weight"}
+    for name in got:
+        err = ((got[name].double() - ref[name].double()).norm() / ref[name].double().norm()).item()
+        assert err < (1e-6 if dtype == torch.float32 else 1e-2), (name, err)
+
+
+def step_of(model, ids):
+    model.zero_grad(set_to_none=True)
+    loss = model(input_ids=ids, labels=ids).loss
+    loss.backward()
+    return loss.detach(), {n: p.grad for n, p in model.named_parameters() if p.grad is not None}
+
+
 def in_64_bits(layer, x, lb, mask, dout):
     """The layer in double precision; every tensor that the kernels materialise takes the value they gave it (straight-through), codes too."""
     import matmulfreellm_amd.functional as F_
