@@ -65,7 +65,7 @@ class HGRNBitAttention(nn.Module):
         self.g_norm = FusedRMSNormSwishGate(self.input_dim, layernorm_eps)
         self.o_proj = BitLinear(self.input_dim, hidden_size, bias=False, fused_eps=bitlinear_eps)
         self.apply(self._initialize_weights)
-        self._norms_seen, self._norms_agree = F_.Seen(), False
+        self._norms_seen, self._norms_agree = [F_.Seen() for _ in range(3)], False
         self._stack = None
 
     def _initialize_weights(self, module):
@@ -92,9 +92,10 @@ class HGRNBitAttention(nn.Module):
                 or any(p.norm.eps != projs[0].norm.eps or p.fused_eps != projs[0].fused_eps for p in projs[1:])):
             return None
         norms = [p.norm.weight for p in projs]
-        if not self._norms_seen.unchanged(*norms):                   # (the comparison waits for the device)
+        if not all(seen.unchanged(w) for seen, w in zip(self._norms_seen, norms)):           # (the comparison waits for the device)
             self._norms_agree = torch.equal(norms[0], norms[1]) and torch.equal(norms[0], norms[2])
-            self._norms_seen.take(*norms)
+            for seen, w in zip(self._norms_seen, norms):
+                seen.take(w)
         return self._stacked_weight() if self._norms_agree else None
 
     def forward(self, hidden_states: torch.Tensor, attention_mask: Optional[torch.Tensor] = None,

@@ -168,13 +168,13 @@ PyObject* scan(PyObject*, PyObject* const* args, Py_ssize_t count) {
 }
 
 // ------------------------------------------------------------------------------ what a native block call takes for granted
-// Whether all of this still holds for a block -- asked for every block of every forward, ~120 look-ups, 13 us in Python and 2.5 here:
+// Whether all of this still holds for a block -- asked for every block of every forward, ~130 look-ups in 1.6 us:
 // (block, (class, modules dict, parameters dict, [(module, class, dict)], [(dict, key, object)], [(dict, key)], [(dict, key, value)],
 // [(class, forward, __call__)])):
 //   the block is of that class and holds those two dicts; the modules below it are of theirs;
 //   none of them has hooks or a forward of its own;
 //   the dicts hold those objects, nothing or None, and equal values; the classes' forward and __call__ are the ones they were.
-PyObject *kHooks[4], *kForward, *kCall, *kDict, *kModules, *kParameters;
+PyObject *kHooks[4], *kForward, *kCall, *kModules, *kParameters;
 // 1 / 0, or -1 with an error set
 int untouched(PyObject* d) {
     for (PyObject* name : kHooks) {
@@ -193,16 +193,14 @@ int holds(PyObject* d, PyObject* key, PyObject* object) {
     PyObject* held = PyDict_GetItemWithError(d, key);
     return !held && PyErr_Occurred() ? -1 : held == object;
 }
-int attribute_is(PyObject* of, PyObject* name, PyObject* object) {
-    PyObject* now = PyObject_GetAttr(of, name);
-    if (!now) return -1;
-    Py_DECREF(now);
-    return now == object;
+// (the type's method cache: a tenth of what a general attribute look-up of a class costs)
+bool method_is(PyObject* cls, PyObject* name, PyObject* function) {
+    return _PyType_Lookup(reinterpret_cast<PyTypeObject*>(cls), name) == function;
 }
 int structure(PyObject* block, PyObject* facts) {
     auto fact = [&](int i) { return PyTuple_GET_ITEM(facts, i); };
     if (reinterpret_cast<PyObject*>(Py_TYPE(block)) != fact(0)) return 0;
-    PyObject* d = PyObject_GetAttr(block, kDict);
+    PyObject* d = PyObject_GenericGetDict(block, nullptr);
     if (!d) return -1;
     int ok = untouched(d);
     if (ok == 1) ok = holds(d, kModules, fact(1));
@@ -236,8 +234,8 @@ int structure(PyObject* block, PyObject* facts) {
     }
     for (Py_ssize_t i = 0; i < PyList_GET_SIZE(fact(7)); ++i) {
         PyObject* t = PyList_GET_ITEM(fact(7), i);
-        if ((ok = attribute_is(PyTuple_GET_ITEM(t, 0), kForward, PyTuple_GET_ITEM(t, 1))) != 1) return ok;
-        if ((ok = attribute_is(PyTuple_GET_ITEM(t, 0), kCall, PyTuple_GET_ITEM(t, 2))) != 1) return ok;
+        if (!method_is(PyTuple_GET_ITEM(t, 0), kForward, PyTuple_GET_ITEM(t, 1)) || !method_is(PyTuple_GET_ITEM(t, 0), kCall, PyTuple_GET_ITEM(t, 2)))
+            return 0;
     }
     return 1;
 }
@@ -286,8 +284,7 @@ PyMODINIT_FUNC PyInit_mmf_torch() {
     for (int i = 0; i < 4; ++i)
         if (!(kHooks[i] = PyUnicode_InternFromString(names[i]))) return nullptr;
     if (!(kForward = PyUnicode_InternFromString("forward")) || !(kCall = PyUnicode_InternFromString("__call__")) ||
-        !(kDict = PyUnicode_InternFromString("__dict__")) || !(kModules = PyUnicode_InternFromString("_modules")) ||
-        !(kParameters = PyUnicode_InternFromString("_parameters")))
+        !(kModules = PyUnicode_InternFromString("_modules")) || !(kParameters = PyUnicode_InternFromString("_parameters")))
         return nullptr;
     return PyModule_Create(&module);
 }

@@ -72,7 +72,7 @@ class DecodeEngine(NotCopied):
         self._parameters = [(d["_parameters"], k, p, p._version, p.data_ptr()) for d in dicts
                             for k, p in d["_parameters"].items() if p is not None]
         self._absent = [(d["_parameters"], k) for d in dicts for k, p in d["_parameters"].items() if p is None]
-        self._sizes = [(d[name], len(d[name])) for d in dicts for name in ("_modules", "_parameters")]
+        self._blocks = model.model.layers._modules
 
         attn0 = model.model.layers[0].attn
         self.D = D = attn0.input_dim
@@ -156,14 +156,15 @@ class DecodeEngine(NotCopied):
         return float(p.norm.eps if getattr(p, "fused_eps", None) is None else p.fused_eps)
 
     def stale(self):
-        """Whether a module or parameter the engine was built on has been replaced or written since, or one has come or gone."""
+        """Whether a module or parameter the engine was built on has been replaced or written since, or a layer or an absent parameter
+        has come."""
         for d, k, p, version, address in self._parameters:
             if d.get(k) is not p or p._version != version or p.data_ptr() != address:
                 return True
         for d, k, c in self._children:
             if d.get(k) is not c:
                 return True
-        return any(len(d) != n for d, n in self._sizes) or any(d.get(k) is not None for d, k in self._absent)
+        return len(self._blocks) != self.L or any(d.get(k) is not None for d, k in self._absent)
 
     # ------------------------------------------------------------------ launches
     def _bitlinear(self, x, pw_nw_eps, out, n_k, addend=None):

@@ -27,23 +27,18 @@ def _as_2d(x):
 
 # ------------------------------------------------------------------------------ weights
 class Seen:
-    """Tensors as they were when something was derived from them: the same objects, unwritten since and at their addresses.  The
-    objects count too, because a tensor that is computed anew on each access (a parametrised weight) may come to lie where the last one
-    did.  They are not kept alive; a copy or a pickle of this has seen nothing."""
+    """A tensor as it was when something was derived from it: the same object, unwritten since and at its address.  The object
+    counts too, because a tensor that is computed anew on each access (a parametrised weight) may come to lie where the last one
+    did.  It is not kept alive; a copy or a pickle of this has seen nothing."""
 
     def __init__(self):
-        self.refs, self.facts = (), None
+        self.ref, self.facts = None, None
 
-    @staticmethod
-    def _facts(tensors):
-        return [(t.data_ptr(), t._version, t.dtype, t.device, t.shape) for t in tensors]
+    def unchanged(self, t):
+        return self.ref is not None and self.ref() is t and self.facts == (t.data_ptr(), t._version, t.dtype, t.device, t.shape)
 
-    def unchanged(self, *tensors):
-        return (len(self.refs) == len(tensors) and all(r() is t for r, t in zip(self.refs, tensors))
-                and self.facts == self._facts(tensors))
-
-    def take(self, *tensors):
-        self.refs, self.facts = [weakref.ref(t) for t in tensors], self._facts(tensors)
+    def take(self, t):
+        self.ref, self.facts = weakref.ref(t), (t.data_ptr(), t._version, t.dtype, t.device, t.shape)
 
     def __reduce__(self):
         return Seen, ()
