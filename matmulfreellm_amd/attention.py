@@ -7,8 +7,9 @@ Interface of mmfreelm/layers/hgrn_bit.py:22-162.  Data flow of forward (:83-142)
     o, state = recurrence(i, f, state)                   h_t = f_t * h_{t-1} + i_t
     o = g_norm(g, o)                                     RMSNorm(g) * o * sigmoid(o)
     o = o_proj(o)
-The three input projections run as one contraction over the stacked packed weights when
-their inner norm weights are equal (they then share the int8 codes of h).
+As a module, the three input projections run as one contraction over the stacked packed weights when
+their inner norm weights are equal (they then share the int8 codes of h); the native block call (block.py) and the
+decode engine stack them in either case.
 """
 from typing import Optional, Tuple
 

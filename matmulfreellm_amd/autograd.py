@@ -9,7 +9,8 @@ Each Function mirrors one of the reference's autograd Functions:
   HGRNGateFn               the elementwise ops of mmfreelm/layers/hgrn_bit.py:113-120, differentiated as one op
   CrossEntropyFn           CrossEntropyLossFunction      mmfreelm/modules/fused_cross_entropy.py:163-310
 
-The forward values are those of the inference kernels (same launches); the backward kernels live in csrc/backward.hip.
+The forward values are those of the inference kernels (same launches); the backward kernels live in csrc/backward.hip,
+csrc/backward_block.hip (a block's row kernels) and csrc/hgrn_block.hip (the scans).
 The two dense products of a BitLinear's backward (dout @ W_q and dout^T @ y_q, fusedbitnet.py:474, :498) are plain
 library GEMMs (torch.matmul).  Modules pick these Functions when gradients are enabled and an input or parameter
 requires one (`needs_grad`); otherwise they keep the fused inference launches.  The scans differentiate in native code

@@ -4,7 +4,7 @@
 side reads, and remembers what they were taken from.  ``current()`` looks, before every call, whether all of that still
 holds: the same modules of the same classes, parameters neither written nor replaced, the same eps, mode, layer index and sizes,
 no hook and no patched ``forward`` or ``__call__`` anywhere inside, on a module or on its class -- anything else (and every
-block the native call does not cover) goes through the modules as before.  The results are those of the module path bit for bit: the
+block the native call does not cover) goes through the modules.  The results are those of the module path bit for bit: the
 same kernels with the same arguments.
 """
 import ctypes

@@ -1,16 +1,17 @@
-"""Whole-model single-token decode step as one HIP graph.
+"""Whole-model single-token decode step as one launch or one HIP graph.
 
-At batch 1 the 4L fused BitLinears of the layers run as ONE persistent launch (mmf_decode_layers: resident
-workgroups hand activations to each other as tagged words), followed by the lm_head launch and the argmax.
+At batch 1 the whole step -- embedding row, the 4L fused BitLinears of the layers, final norm and lm_head, argmax -- is ONE
+persistent launch (mmf_decode_layers_norms: resident workgroups hand activations to each other as tagged words), launched
+directly, where the model fits it; a step that samples is followed by the launch of its draw.
 
 The module path (HGRNBitForCausalLM.forward with T = 1) issues the same kernels through
 nn.Module calls and fresh output tensors; at batch 1 that host work dwarfs the ~40 us the
-weights take to stream.  DecodeEngine lays the step out once over static buffers, records it
-into a graph (torch.cuda.CUDAGraph = hipGraph) and replays it per token: embedding gather ->
+weights take to stream.  DecodeEngine lays the step out once over static buffers; beyond batch 1 (or that
+launch's limits) it records it into a graph (torch.cuda.CUDAGraph = hipGraph) and replays it per token: embedding gather ->
 L x [RMSNorm, i/f/g BitLinear, gate + recurrence step, gated norm, o_proj BitLinear,
 residual RMSNorm, gate_proj BitLinear, swiglu, down_proj BitLinear (+residual)] -> final
-norm -> lm_head BitLinear -> argmax.  The argmax writes the token buffer the next replay's
-embedding reads, so consecutive steps need no host round trip.
+norm -> lm_head BitLinear -> argmax or draw.  The last writes the token buffer the next step's
+embedding reads, so consecutive steps need no host round trip; the tokens fed are recorded by the step itself.
 
 Every launch is the same C-ABI call with the same arithmetic as the module path, so the two
 produce identical bits (tests/test_gpu_model.py checks that).

@@ -11,7 +11,8 @@ Differences, all on the host side:
     PreTrainedModel a generate());
   * ``logits_to_keep`` lets a caller ask for the last positions' logits only (the
     reference projects all T positions through the 32000-wide head);
-  * ``labels`` gives the evaluation loss (forward only, fp32): there is no backward.
+  * ``labels`` gives the loss: with gradients the fused one (autograd.FusedCrossEntropyLoss), without them the evaluation
+    loss, forward only and in fp32.
 """
 from __future__ import annotations
 
@@ -190,9 +191,10 @@ class HGRNBitModel(HGRNBitPreTrainedModel):
                 output_hidden_states: Optional[bool] = None, return_dict: Optional[bool] = None
                 ) -> Union[Tuple, BaseModelOutputWithPast]:
         """With gradients enabled and a parameter or the input embeddings requiring one -- in train or eval mode, as the
-        reference -- the forward runs the reference's op-by-op composition through the autograd Functions
-        (matmulfreellm_amd/autograd.py); everything else (torch.no_grad(), generate()) runs the fused inference launches
-        without a graph."""
+        reference -- every block is one autograd op (BlockFn); one that the native calls do not cover (a hook, a replaced or
+        subclassed module, mixed dtypes, short convolutions) runs the reference's op-by-op composition through
+        the autograd Functions (matmulfreellm_amd/autograd.py).  Everything else (torch.no_grad(), generate()) runs without a
+        graph: a block as one native call (block.py), or its modules with their fused launches."""
         train = module_needs_grad(self, inputs_embeds)
         with torch.enable_grad() if train else torch.no_grad():
             return self._forward(train, input_ids, attention_mask, inputs_embeds, past_key_values, use_cache,
@@ -478,17 +480,18 @@ class HGRNBitForCausalLM(HGRNBitPreTrainedModel, GenerationMixin):
                  generator: Optional[torch.Generator] = None, **kwargs) -> torch.LongTensor:
         """Greedy (default) or top-p sampling; returns [B, T + new] token ids like HF's generate.
 
-        With the arguments above (what the reference's generate.py passes), prefill runs the module path with
-        last-position logits only and decode runs the captured whole-step HIP graph of DecodeEngine when
-        use_graph is set.  Sampling draws every token with one launch of the top-p kernel (functional.sample_top_p)
-        on the step's logits and feeds it back without a host round trip; the uniform numbers of the whole run are
-        drawn up front from `generator` (torch.rand), and the logits are bit-identical to the module path's, so a
+        With the arguments above (what the reference's generate.py passes), prefill is the model's forward with
+        last-position logits only and decode runs the whole steps of DecodeEngine when use_graph is set: one resident
+        launch a token at batch 1, else a replayed HIP graph.  Sampling draws every token within the step (the top-p
+        kernel is the recorded step's last launch, and follows the resident one; vocabularies beyond its limit are drawn by
+        library calls behind the step) and feeds it back without a host round trip; the uniform numbers of the whole run
+        are drawn up front from `generator` (torch.rand), and the logits are bit-identical to the module path's, so a
         seeded generator gives the same tokens either way (not the tokens torch.multinomial would draw from the
         same seed).  top_k, when not given, is the generation config's, else transformers' default of 50 (what the
         reference's call, which passes none, samples with); top_k=0 switches the limit off.  Rows that
         have produced eos_token_id (default: the generation config's) are filled with pad_token_id (eos_token_id
         when not given); generation ends early once every row has.  At batch 1 the whole decode step is one resident
-        launch when the model fits it; resident=False keeps one launch per fused BitLinear.
+        launch when the model fits it (mmf_decode_layers_fits); resident=False keeps one launch per fused BitLinear.
 
         Any further keyword (num_beams, repetition_penalty, logits_processor, stopping_criteria, streamer,
         generation_config, return_dict_in_generate, ...) sends the whole call to
