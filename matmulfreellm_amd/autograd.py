@@ -197,7 +197,7 @@ class HGRNGateFn(torch.autograd.Function):
         gg2 = _2d(gg).to(i.dtype).contiguous() if gg is not None else torch.zeros(rows, d, dtype=i.dtype, device=dev)
         di = torch.empty(rows, d, dtype=i.dtype, device=dev)
         df = torch.empty(rows, d, dtype=i.dtype, device=dev)
-        lbf = lb.detach().float().contiguous() if lb is not None else None
+        lbf = F_.lower_bound_row(lb, d)
         dlb = torch.empty(d, dtype=torch.float32, device=dev) if lb is not None else None
         part = torch.empty(lib.mmf_backward_groups(rows), d, dtype=torch.float32, device=dev) if lb is not None else None
         mk = F_._mask_rows(mask, rows, dev) if mask is not None else None
@@ -273,7 +273,7 @@ class BlockFn(torch.autograd.Function):
         with L.on(dev):
             empty = lambda *shape: torch.empty(*shape, dtype=dt, device=dev)
             out, ifg, xg, o, attn, y = torch.empty_like(x), empty(m, 3 * D), empty(2, m, D), empty(m, D), empty(m, H), empty(m, 2 * I)
-            lb = lower_bound.detach().float().contiguous() if lower_bound is not None else None
+            lb = F_.lower_bound_row(lower_bound, D)
             mk = F_._mask_rows(mask, m, dev)
             ws = torch.empty(lib.mmf_block_train_workspace_bytes(plan.ref, m), dtype=torch.uint8, device=dev)
             L.check(lib.mmf_block_train_forward(plan.ref, x.data_ptr(), out.data_ptr(), ifg.data_ptr(), xg.data_ptr(), o.data_ptr(),

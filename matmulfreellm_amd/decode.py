@@ -97,7 +97,7 @@ class DecodeEngine(NotCopied):
                 "o": (a.o_proj.packed_weight(), a.o_proj.norm.weight.detach(), self._eps_of(a.o_proj)),
                 "gate": (m.gate_proj.packed_weight(), m.gate_proj.norm.weight.detach(), self._eps_of(m.gate_proj)),
                 "down": (m.down_proj.packed_weight(), m.down_proj.norm.weight.detach(), self._eps_of(m.down_proj)),
-                "lb": lbs[li].contiguous() if (lbs is not None and li > 0) else None,
+                "lb": F_.lower_bound_row(lbs[li], D) if lbs is not None and li > 0 else None,
                 "state": z(B, D, dtype=torch.float32),
             }
             for p in (a.i_proj, a.f_proj, a.g_proj, a.o_proj, m.gate_proj, m.down_proj):

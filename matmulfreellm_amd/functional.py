@@ -504,6 +504,16 @@ def _mask_rows(mask, rows, dev):
     return m
 
 
+def lower_bound_row(lower_bound, d):
+    """The lower bounds of a gate of ``d`` channels in fp32: one for each channel, or the kernels would read past them."""
+    if lower_bound is None:
+        return None
+    if lower_bound.numel() != d:
+        raise ValueError(f"{lower_bound.numel()} lower bounds for {d} gate channels (HGRNBitModel has one row of hidden_size per layer: "
+                         "expand_ratio other than 1 needs use_lower_bound=False)")
+    return lower_bound.detach().to(torch.float32).contiguous()
+
+
 def hgrn_gate(i, f, lower_bound=None, attention_mask=None):
     """Fused sigmoid / lower bound / swiglu / mask.  i, f [..., D] -> (x, g) contiguous [..., D]."""
     lib = L.load()
@@ -511,7 +521,7 @@ def hgrn_gate(i, f, lower_bound=None, attention_mask=None):
     d = i.shape[-1]
     i2, rows, ldi = _rows_ld(i, d)
     f2, _, ldf = _rows_ld(f, d)
-    lb = lower_bound.detach().to(torch.float32).contiguous() if lower_bound is not None else None
+    lb = lower_bound_row(lower_bound, d)
     mk = _mask_rows(attention_mask, rows, dev)
     xo = torch.empty(i.shape, dtype=i.dtype, device=dev)
     go = torch.empty(i.shape, dtype=i.dtype, device=dev)
@@ -530,7 +540,7 @@ def hgrn_step(i, f, state, lower_bound=None, attention_mask=None):
     f2, _, ldf = _rows_ld(f, d)
     if state.dtype != torch.float32 or not state.is_contiguous() or state.numel() != rows * d:
         raise ValueError("state must be a contiguous fp32 tensor of rows*D elements")
-    lb = lower_bound.detach().to(torch.float32).contiguous() if lower_bound is not None else None
+    lb = lower_bound_row(lower_bound, d)
     mk = _mask_rows(attention_mask, rows, dev)
     o = torch.empty(i.shape, dtype=i.dtype, device=dev)
     with L.on(dev):

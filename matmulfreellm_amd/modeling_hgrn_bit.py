@@ -304,6 +304,8 @@ class HGRNBitModel(HGRNBitPreTrainedModel):
                     fits = (state.dtype == torch.float32 and state.device == dev and state.is_contiguous()
                             and state.numel() == B * plan.D)
                 lb = lbs[i] if lbs is not None else None
+                if lb is not None and i > 0 and fits:
+                    F_.lower_bound_row(lb, plan.D)
                 if not fits:
                     if fresh is not None:
                         state.zero_()

@@ -705,3 +705,39 @@ def test_generate_sees_a_layer_or_a_bias_added_after_the_engine_was_built(dev):
     model.model.layers[1].mlp.down_proj.bias = torch.nn.Parameter(torch.ones(256, device=dev, dtype=torch.bfloat16))
     with pytest.raises(NotImplementedError):
         run(True)
+
+
+def test_lower_bounds_of_another_width_than_the_gates_are_refused(dev):
+    """A model has one row of hidden_size lower bounds a layer; with expand_ratio 2 the gates are twice as wide.  From the second layer
+    on, where they apply, every path refuses them (as the reference's broadcast does); without them the widths are free."""
+    import matmulfreellm_amd as mm
+    import matmulfreellm_amd.functional as F_
+    torch.manual_seed(6)
+    for layers, use, fails in ((2, True, True), (1, True, False), (2, False, False)):
+        model = mm.HGRNBitForCausalLM(mm.HGRNBitConfig(vocab_size=100, hidden_size=64, num_hidden_layers=layers, expand_ratio=2,
+                                                       use_lower_bound=use, eos_token_id=None)).to(dev, torch.bfloat16).eval()
+        hook = lambda *a: None
+
+        def train():
+            with torch.enable_grad():
+                model(input_ids=ids, labels=ids).loss.backward()
+
+        for b, t in ((1, 1), (2, 9), (3, 40)):
+            ids = torch.randint(0, 100, (b, t), device=dev)
+            calls = [lambda: model.generate(ids, max_new_tokens=3), train, lambda: mm.DecodeEngine(model, b)]
+            for hooked in (False, True):
+                handle = model.model.layers[-1].attn.g_norm.register_forward_hook(hook) if hooked else None
+                for call in calls:
+                    if fails:
+                        with pytest.raises(ValueError, match="lower bounds"):
+                            call()
+                    else:
+                        call()
+                if hooked:
+                    handle.remove()
+    i = torch.zeros(2, 8, device=dev)
+    for lb in (torch.zeros(4, device=dev), torch.zeros(16, device=dev)):
+        with pytest.raises(ValueError, match="lower bounds"):
+            F_.hgrn_gate(i, i, lb)
+        with pytest.raises(ValueError, match="lower bounds"):
+            F_.hgrn_step(i, i, torch.zeros(2, 8, device=dev), lb)
