@@ -59,7 +59,7 @@ def _norm_bwd(mode, xs, gate, weight, dy, dres, eps, want_y=False):
     dx = torch.empty(m, k, dtype=x2.dtype, device=dev)
     dgate = torch.empty(m, k, dtype=x2.dtype, device=dev) if mode == 1 else None
     yq = torch.empty(m, k, dtype=x2.dtype, device=dev) if want_y else None
-    w = weight.detach() if weight is not None else None
+    w = F_.vector(weight, k, "norm weight")
     if w is not None and w.dtype not in (torch.float32, x2.dtype):
         w = w.float()
     dw = torch.empty_like(w) if w is not None else None

@@ -83,20 +83,32 @@ class DecodeEngine(NotCopied):
         def z(*shape, dtype=dt):
             return torch.zeros(*shape, dtype=dtype, device=dev)
 
+        w = lambda norm, n: F_.vector(norm.weight, n, "norm weight")
+
+        def codes(proj, n, k):
+            """A projection's packed weight: the launches take every layer's sizes from the first one's, the vocabulary's from the configuration."""
+            pw = proj.packed_weight()
+            if (pw.n, pw.k) != (n, k):
+                raise NotImplementedError(f"DecodeEngine: a projection {pw.k} -> {pw.n} where the model's are {k} -> {n}; "
+                                          "generate(use_graph=False) decodes layers of different widths")
+            return pw
+
+        if tuple(emb.shape) != (self.V, H):
+            raise NotImplementedError(f"DecodeEngine: an embedding {tuple(emb.shape)} in a model of {self.V} x {H}; generate(use_graph=False) takes it")
+
         # ---- per-layer operands (references keep the packed weights alive)
         self.layers = []
         for li, blk in enumerate(model.model.layers):
             a, m = blk.attn, blk.mlp
             ent = {
-                "attn_norm": blk.attn_norm.weight.detach(), "mlp_norm": blk.mlp_norm.weight.detach(),
-                "g_norm": a.g_norm.weight.detach(), "g_eps": float(a.g_norm.eps),
+                "attn_norm": w(blk.attn_norm, H), "mlp_norm": w(blk.mlp_norm, H), "g_norm": w(a.g_norm, D), "g_eps": float(a.g_norm.eps),
                 "ifg": a._stacked_weight() if self._stackable(a) else None,
                 # None where the three inner norms agree (one row of codes serves i, f and g), else the three weights
-                "norms": None if a._stacked_ifg() is not None else [p.norm.weight.detach() for p in (a.i_proj, a.f_proj, a.g_proj)],
-                "projs": [(p.packed_weight(), p.norm.weight.detach(), self._eps_of(p)) for p in (a.i_proj, a.f_proj, a.g_proj)],
-                "o": (a.o_proj.packed_weight(), a.o_proj.norm.weight.detach(), self._eps_of(a.o_proj)),
-                "gate": (m.gate_proj.packed_weight(), m.gate_proj.norm.weight.detach(), self._eps_of(m.gate_proj)),
-                "down": (m.down_proj.packed_weight(), m.down_proj.norm.weight.detach(), self._eps_of(m.down_proj)),
+                "norms": None if a._stacked_ifg() is not None else [w(p.norm, H) for p in (a.i_proj, a.f_proj, a.g_proj)],
+                "projs": [(codes(p, D, H), w(p.norm, H), self._eps_of(p)) for p in (a.i_proj, a.f_proj, a.g_proj)],
+                "o": (codes(a.o_proj, H, D), w(a.o_proj.norm, D), self._eps_of(a.o_proj)),
+                "gate": (codes(m.gate_proj, 2 * I, H), w(m.gate_proj.norm, H), self._eps_of(m.gate_proj)),
+                "down": (codes(m.down_proj, H, I), w(m.down_proj.norm, I), self._eps_of(m.down_proj)),
                 "lb": F_.lower_bound_row(lbs[li], D) if lbs is not None and li > 0 else None,
                 "state": z(B, D, dtype=torch.float32),
             }
@@ -104,9 +116,9 @@ class DecodeEngine(NotCopied):
                 if p.bias is not None:
                     raise NotImplementedError("DecodeEngine: BitLinear bias is not on the model path")
             self.layers.append(ent)
-        self.final_norm = model.model.norm.weight.detach()
-        self.head = (model.lm_head.packed_weight(), model.lm_head.norm.weight.detach(), self._eps_of(model.lm_head))
-        self.table = emb.detach()
+        self.final_norm = w(model.model.norm, H)
+        self.head = (codes(model.lm_head, self.V, H), w(model.lm_head.norm, H), self._eps_of(model.lm_head))
+        self.table = emb.detach().contiguous()
 
         # ---- static activation buffers
         self.tok = torch.zeros(B, dtype=torch.int64, device=dev)

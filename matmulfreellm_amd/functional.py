@@ -86,6 +86,15 @@ def unpack_ternary(pw):
     return codes
 
 
+def vector(v, n, what):
+    """A per-column operand of rows of n values, contiguous: the kernels read n of it."""
+    if v is None:
+        return None
+    if v.numel() != n:
+        raise ValueError(f"{what} of {v.numel()} elements for rows of {n}")
+    return v.detach().contiguous()
+
+
 # ------------------------------------------------------------------------------ norms
 def _norm_common(x, residual, weight, prenorm, residual_in_fp32, keep_strided=False):
     dev = L.require_gpu(x, residual, weight)
@@ -102,8 +111,7 @@ def _norm_common(x, residual, weight, prenorm, residual_in_fp32, keep_strided=Fa
     need_res_out = r2 is not None or res_dtype != x2.dtype
     # the summed residual stream is only materialised when the caller asks for it back (prenorm)
     res_out = torch.empty(tuple(x2.shape), dtype=res_dtype, device=dev) if (need_res_out and prenorm) else None
-    w = weight.detach().contiguous() if weight is not None else None
-    return dev, shp, x2, r2, res_dtype, res_out, w
+    return dev, shp, x2, r2, res_dtype, res_out, vector(weight, shp[-1], "norm weight")
 
 
 def rmsnorm(x, weight, residual=None, eps=1e-6, prenorm=False, residual_in_fp32=False):
@@ -261,7 +269,7 @@ def bitlinear_mfma(q_tiled, deq, qsum, pw, m, out_dtype, bias=None, config=-1, o
         out = torch.empty(m, pw.n, dtype=out_dtype, device=dev)
     ldo = out.stride(0) if m > 1 else max(out.shape[-1], pw.n)
     if bias is not None:
-        bias = bias.detach().to(out_dtype).contiguous()
+        bias = vector(bias, pw.n, "bias").to(out_dtype)
     if addend is not None:
         addend = addend.reshape(m, pw.n)
         if addend.dtype != out_dtype or not addend.is_contiguous() or ldo != pw.n:
@@ -297,10 +305,12 @@ def bitlinear_gemv(x2, norm_weight, pw, eps, bias=None, addend=None):
     lib = L.load()
     dev = L.require_gpu(x2, norm_weight, pw.packed, bias)
     m, k = x2.shape
+    if k != pw.k:
+        raise ValueError(f"input features {k} != weight in_features {pw.k}")
     out = torch.empty(m, pw.n, dtype=x2.dtype, device=dev)
-    nw = norm_weight.detach().contiguous() if norm_weight is not None else None
+    nw = vector(norm_weight, k, "norm weight")
     if bias is not None:
-        bias = bias.detach().to(x2.dtype).contiguous()
+        bias = vector(bias, pw.n, "bias").to(x2.dtype)
     if addend is not None:
         addend = addend.reshape(m, pw.n)
         if addend.dtype != x2.dtype or not addend.is_contiguous():
@@ -342,8 +352,7 @@ def _bitlinear_prologue(x, norm_weight, pw, bias, eps, addend, prologue, epilogu
     m = x2.shape[0]
     if a2 is not None and (a2.shape != x2.shape or a2.dtype != x2.dtype):
         raise ValueError("the prologue operand must match x in shape and dtype")
-    nw = norm_weight.detach().contiguous() if norm_weight is not None else None
-    w1c = w1.detach().contiguous() if w1 is not None else None
+    nw, w1c = vector(norm_weight, k, "norm weight"), vector(w1, k, "norm weight")
     wdt = nw.dtype if nw is not None else (w1c.dtype if w1c is not None else torch.float32)
     if w1c is not None and nw is not None and w1c.dtype != nw.dtype:
         raise ValueError("the two norm weights must share a dtype")
@@ -352,7 +361,7 @@ def _bitlinear_prologue(x, norm_weight, pw, bias, eps, addend, prologue, epilogu
         _check_swiglu_epilogue(epilogue, m, pw, x2.dtype, bias, addend)
     out = torch.empty(m, pw.n, dtype=x2.dtype, device=dev) if epilogue is None else None
     if bias is not None:
-        bias = bias.detach().to(x2.dtype).contiguous()
+        bias = vector(bias, pw.n, "bias").to(x2.dtype)
     if addend is not None:
         addend = addend.reshape(m, pw.n)
         if addend.dtype != x2.dtype or not addend.is_contiguous():
@@ -518,6 +527,8 @@ def hgrn_gate(i, f, lower_bound=None, attention_mask=None):
     """Fused sigmoid / lower bound / swiglu / mask.  i, f [..., D] -> (x, g) contiguous [..., D]."""
     lib = L.load()
     dev = L.require_gpu(i, f, lower_bound)
+    if f.shape != i.shape or f.dtype != i.dtype:
+        raise ValueError("i and f must match in shape and dtype")
     d = i.shape[-1]
     i2, rows, ldi = _rows_ld(i, d)
     f2, _, ldf = _rows_ld(f, d)
@@ -535,6 +546,8 @@ def hgrn_step(i, f, state, lower_bound=None, attention_mask=None):
     """One decode step: gate math + h = g*h + x.  state fp32 [rows, D] is updated in place; returns o."""
     lib = L.load()
     dev = L.require_gpu(i, f, state, lower_bound)
+    if f.shape != i.shape or f.dtype != i.dtype:
+        raise ValueError("i and f must match in shape and dtype")
     d = i.shape[-1]
     i2, rows, ldi = _rows_ld(i, d)
     f2, _, ldf = _rows_ld(f, d)
@@ -639,7 +652,7 @@ def _conv_args(x, weight, bias):
     w2 = weight.detach().reshape(weight.shape[0], -1).to(x.dtype).contiguous()       # nn.Conv1d keeps [D, 1, W]
     if w2.shape[0] != d:
         raise ValueError(f"convolution has {w2.shape[0]} channels, the input {d}")
-    b1 = bias.detach().to(x.dtype).contiguous() if bias is not None else None
+    b1 = vector(bias, d, "bias").to(x.dtype) if bias is not None else None
     return dev, w2, b1
 
 

@@ -61,3 +61,45 @@ def test_native_scans_differentiate_like_autograd_of_the_recurrence(dev, scan, s
         scan(x, g[:, :, :-1])
     with pytest.raises(L.MMFError):
         scan(x.detach().cpu().requires_grad_(), g)
+
+
+def test_operands_of_another_size_are_refused(dev):
+    """Per-column operands that are shorter or longer than the rows, gates of other sizes, layers of other widths: an error from the
+    host, in every path, instead of a kernel that reads what is not there."""
+    def refused(call, error=ValueError):
+        with pytest.raises(error):
+            call()
+
+    w = lambda n, dtype=torch.float32: torch.ones(n, device=dev, dtype=dtype)
+    for n in (32, 128):
+        for x in (torch.randn(2, 64, device=dev), torch.randn(300, 64, device=dev)):
+            layer = mm.FusedBitLinear(64, 40).to(dev)
+            pw = layer.packed_weight()
+            for grad in (False, True):
+                with torch.set_grad_enabled(grad):
+                    refused(lambda: mm.RMSNorm(n).to(dev)(x))
+                    refused(lambda: mm.FusedRMSNormSwishGate(n).to(dev)(x, x))
+                    other = mm.FusedBitLinear(64, 40).to(dev)
+                    other.norm = mm.RMSNorm(n).to(dev)
+                    refused(lambda: other(x))
+                    biased = mm.FusedBitLinear(64, 40, bias=True).to(dev)
+                    biased.bias = torch.nn.Parameter(w(n))
+                    refused(lambda: biased(x))
+            refused(lambda: F.bitlinear(x, w(64), pw, prologue=("norm", w(n), 1e-6)))
+            refused(lambda: F.bitlinear(x, w(n), pw, prologue=("swiglu", x)))
+            refused(lambda: F.rmsnorm_quant(x, w(n)))
+    i = torch.zeros(3, 16, device=dev)
+    for f in (torch.zeros(3, 8, device=dev), torch.zeros(2, 16, device=dev), torch.zeros(3, 16, device=dev, dtype=torch.bfloat16)):
+        refused(lambda: F.hgrn_gate(i, f))
+        refused(lambda: F.hgrn_step(i, f, torch.zeros(3, 16, device=dev)))
+    refused(lambda: F.short_conv(torch.zeros(1, 5, 16, device=dev), torch.zeros(16, 1, 4, device=dev), w(8)))
+
+    config = dict(vocab_size=100, hidden_size=64, num_hidden_layers=2, eos_token_id=None, bos_token_id=None)
+    ids = torch.randint(0, 100, (1, 5), device=dev)
+    for change in (lambda m: setattr(m.model.layers[1], "mlp", mm.HGRNBitMLP(64, intermediate_size=96).to(dev)),
+                   lambda m: setattr(m, "lm_head", mm.FusedBitLinear(64, 80).to(dev)),
+                   lambda m: setattr(m.model, "embeddings", torch.nn.Embedding(120, 64).to(dev))):
+        model = mm.HGRNBitForCausalLM(mm.HGRNBitConfig(**config)).to(dev).eval()
+        change(model)
+        refused(lambda: model.generate(ids, max_new_tokens=3), NotImplementedError)
+        assert model.generate(ids, max_new_tokens=3, use_graph=False).shape == (1, 8)
