@@ -284,6 +284,8 @@ class HGRNBitModel(HGRNBitPreTrainedModel):
         elif use_cache and not isinstance(past_key_values, RecurrentCache):
             past_key_values = RecurrentCache.from_legacy_cache(past_key_values)
         lbs = self.lower_bound_rows() if self.config.use_lower_bound else None
+        if lbs is not None and len(self.layers) > 1:
+            F_.lower_bound_row(lbs[1], plan.D)                   # (every block below that runs natively has this one's sizes)
         mask = F_._mask_rows(attention_mask, B * T, dev)
         all_hidden_states = () if output_hidden_states else None
         x = x.contiguous()
@@ -304,8 +306,6 @@ class HGRNBitModel(HGRNBitPreTrainedModel):
                     fits = (state.dtype == torch.float32 and state.device == dev and state.is_contiguous()
                             and state.numel() == B * plan.D)
                 lb = lbs[i] if lbs is not None else None
-                if lb is not None and i > 0 and fits:
-                    F_.lower_bound_row(lb, plan.D)
                 if not fits:
                     if fresh is not None:
                         state.zero_()
