@@ -247,11 +247,11 @@ def _chain_bwd(kind, x, aux, w1, eps1, w2, eps2, dy, dres=None, dx=None, daux=No
 
 
 def _dequantised(pw, dtype):
-    """t * wdeq of a packed weight as a dense [N, K] matrix (fusedbitnet.py:456-458)."""
-    w = torch.empty(pw.n, pw.k, dtype=dtype, device=pw.packed.device)
-    L.check(L.load().mmf_unpack_dequant(pw.packed.data_ptr(), pw.wdeq.data_ptr(), pw.seg_rows, pw.n, pw.k, w.data_ptr(), L.dtype_id(dtype),
-                                        L.stream()), "mmf_unpack_dequant")
-    return w
+    """t * wdeq of a packed weight as a dense [N, K] matrix (fusedbitnet.py:456-458), contiguous along N: dout @ W_q contracts there."""
+    w = torch.empty(pw.k, pw.n, dtype=dtype, device=pw.packed.device)
+    L.check(L.load().mmf_unpack_dequant_t(pw.packed.data_ptr(), pw.wdeq.data_ptr(), pw.seg_rows, pw.n, pw.k, w.data_ptr(), L.dtype_id(dtype),
+                                          L.stream()), "mmf_unpack_dequant_t")
+    return w.t()
 
 
 class BlockFn(torch.autograd.Function):

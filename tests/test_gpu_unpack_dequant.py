@@ -33,3 +33,21 @@ def test_chained_norm_backward_equals_autograd(dev, rows, k, norms):
     ref = torch.autograd.grad([norm(s, w) for w in leaf[2:]], leaf, [d.double() for d in dy])
     for got, want in zip((dx - dres, *dw), ref):
         assert (got.double() - want).norm() <= 2e-6 * want.norm()
+
+
+@pytest.mark.parametrize("n,k,seg", [(1, 1, 1), (9, 17, 4), (31, 129, 31), (256 * 8 + 8, 144, 1024), (72, 260, 24)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_both_layouts_of_the_dense_weights_hold_the_same_values(dev, n, k, seg, dtype):
+    """[N, K] and [K, N], at the edges of the row vectors, the workgroups' columns, the 16-input pieces and the segments."""
+    import matmulfreellm_amd._lib as L
+    import matmulfreellm_amd.functional as F
+    from matmulfreellm_amd.autograd import _dequantised
+    torch.manual_seed(n * k)
+    pw = F.ternarize_pack(torch.randn(n, k, device=dev))
+    pw.wdeq, pw.seg_rows = torch.rand(-(-n // seg), device=dev) + 0.5, seg
+    rows = torch.full((n, k), float("nan"), dtype=dtype, device=dev)
+    with L.on(dev):
+        L.check(L.load().mmf_unpack_dequant(pw.packed.data_ptr(), pw.wdeq.data_ptr(), seg, n, k, rows.data_ptr(), L.dtype_id(dtype),
+                                            L.stream()), "mmf_unpack_dequant")
+        columns = _dequantised(pw, dtype)
+    assert columns.t().is_contiguous() and torch.equal(rows, columns)
