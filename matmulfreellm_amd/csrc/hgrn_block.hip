@@ -21,10 +21,10 @@
 // LS = 2: a workgroup owns 32 channels and the halves of a wave two consecutive runs of steps, for twice the workgroups.
 // When there are still too few, a first launch (AGG) runs steps 1-3 only and leaves per time segment the pair (P, l); the
 // second enters segment s with the fold carry = l_j + P_j * carry over the segments before (backward: behind) it.
-// Measured, bf16, backward: 8 x 1024 x 2048 145 -> 40 us (4.1 TB/s), 64 x 16384 x 128 with log gates 2290 -> 369 us
-// (3.6 TB/s), against a kernel that loaded under a branch per step, so one load after the other, and read g and do twice.
+// Measured, bf16, backward: 8 x 1024 x 2048 145 -> 40 us (4.1 TB/s), 64 x 16384 x 128 with log gates 2290 -> 262 us
+// (5.1 TB/s), against a kernel that loaded under a branch per step, so one load after the other, and read g and do twice.
 // 16 to 28 steps a block and 8 or 16 waves a workgroup lie within 10 % of each other.  Forward, bf16:
-// 64 x 16384 x 128 317 -> 214 us (3.8 TB/s), 4 x 2048 x 2048 61 -> 28 us, against 64-step blocks that took a second exp per step
+// 64 x 16384 x 128 317 -> 160 us (5.0 TB/s), 4 x 2048 x 2048 61 -> 28 us, against 64-step blocks that took a second exp per step
 // for P_t and cut these shapes in time, two launches over x and g.
 #include <type_traits>
 #include "mmf_common.h"
@@ -33,15 +33,16 @@ namespace {
 
 constexpr int kMaxWaves = 8, kFwdBlk = 28, kBwdBlk = 24;
 
-template <typename T>
+// NT: streamed past the caches (each value is read or written once).
+template <typename T, bool NT>
 __device__ __forceinline__ uint32_t buf_bits(__amdgpu_buffer_rsrc_t r, uint32_t vo, uint32_t so) {   // a register per value: no packing of pairs
-    if constexpr (sizeof(T) == 2) return (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r, vo, so, 0);
-    else return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, vo, so, 0);
+    if constexpr (sizeof(T) == 2) return (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r, vo, so, NT ? 2 : 0);
+    else return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, vo, so, NT ? 2 : 0);
 }
-template <typename T>
+template <typename T, bool NT>
 __device__ __forceinline__ void buf_put(__amdgpu_buffer_rsrc_t r, uint32_t vo, uint32_t so, float v) {
-    if constexpr (sizeof(T) == 2) __builtin_amdgcn_raw_buffer_store_b16(mmf_bits16(mmf_from_float<T>(v)), r, vo, so, 0);
-    else __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, vo, so, 0);
+    if constexpr (sizeof(T) == 2) __builtin_amdgcn_raw_buffer_store_b16(mmf_bits16(mmf_from_float<T>(v)), r, vo, so, NT ? 2 : 0);
+    else __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, vo, so, NT ? 2 : 0);
 }
 template <typename T>
 __device__ __forceinline__ float bits_val(uint32_t v) {
@@ -57,12 +58,81 @@ template <int LS>
 __device__ __forceinline__ unsigned column_block() {
     return LS == 2 && gridDim.x % 16 == 0 ? (blockIdx.x & ~15u) + (blockIdx.x & 7u) * 2 + ((blockIdx.x >> 3) & 1u) : blockIdx.x;
 }
-__device__ __forceinline__ void wait_turn(int& turn, int n) {
-    while (__hip_atomic_load(&turn, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) != n) __builtin_amdgcn_s_sleep(1);
+// The carry of a channel that enters block n, as one LDS word with the block's number beside the value: a poll that finds the
+// number has the value, and passing it on is one write.  (A turn counter with the carries behind it cost two more trips through
+// LDS a turn: 350 ns, 205 of the 208 us of 64 x 16384 x 128, whose 585 blocks follow one another.)
+__device__ __forceinline__ void pass_carry(uint64_t& word, float c, int n) {
+    __hip_atomic_store(&word, (uint64_t)(uint32_t)n << 32 | __float_as_uint(c), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ float take_carry(uint64_t& word, int n) {
+    uint64_t w = __hip_atomic_load(&word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    while ((int)(w >> 32) != n) {                               // all lanes see the same number
+        if ((int)(w >> 32) < n - 1) __builtin_amdgcn_s_sleep(1);   // not the next one in line: leave LDS to the others
+        w = __hip_atomic_load(&word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    return __uint_as_float((uint32_t)w);
+}
+// The local pass ends here.  Left to itself the compiler moves it behind the wait, next to the first use of its results, and the
+// turns that were to be a handful of instructions each take the loads' latency and all the arithmetic of a block: 570 ns a turn
+// (64 x 16384 x 128 on 128 workgroups: 333 us forward, 218 with this line).
+__device__ __forceinline__ void done_before_the_turn(float& l, float& P, float& lin, float& Pin, float& lb, float& Pb) {
+    asm volatile("" : "+v"(l), "+v"(P), "+v"(lin), "+v"(Pin), "+v"(lb), "+v"(Pb)::"memory");
+}
+// JOINT: G workgroups share a column and take its superblocks (a block for each wave) in turn; what enters superblock n travels in a
+// word of memory per channel, number beside value as in LDS.  A member composes its waves' blocks before the carry arrives, so
+// between taking it and passing it on lies one multiply-add.  Who waits, waits for a member that was dispatched before it or next to it (the
+// members of a column follow one another on one XCD); a wait that gives up all the same goes on with NaN, which the results show.
+struct Joint {
+    uint64_t* words;      // [BH][D, rounded up to 64], zeroed in front of the launch
+    int G;                // members of a column
+    int64_t BH;
+};
+constexpr int kJointPolls = 1 << 22;                                    // seconds
+__device__ __forceinline__ void pass_joint(uint64_t* word, float c, int n) {
+    __hip_atomic_store(word, (uint64_t)(uint32_t)n << 32 | __float_as_uint(c), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float take_joint(uint64_t* word, int n) {
+    uint64_t w = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int i = 0; __builtin_amdgcn_ballot_w64((int)(w >> 32) != n) != 0 && i < kJointPolls; ++i) {
+        __builtin_amdgcn_s_sleep(2);
+        w = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    return (int)(w >> 32) == n ? __uint_as_float((uint32_t)w) : __builtin_nanf("");
 }
 // What the carry c makes of a run of steps with the product P and the own contribution l.  (A zero carry stays zero also where
 // a product of gates beyond one has overflowed.)
 __device__ __forceinline__ float fold(float l, float P, float c) { return c == 0.0f ? l : fmaf(P, c, l); }
+// The carry that enters this wave's block (l, P) of superblock n, whose `nw` waves all come here.  last: no superblock follows.
+__device__ __forceinline__ float joint_carry(float l, float P, int n, bool last, int wave, int nw, float2 (*pair)[64], uint64_t* carry,
+                                             uint64_t* word, float first) {
+    const int lane = (int)threadIdx.x & 63;
+    pair[wave][lane] = make_float2(l, P);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");     // LDS only: loads and stores stay in flight
+    float lin = 0.0f, Pin = 1.0f;
+    for (int w = 0; w < wave; ++w) {
+        const float2 q = pair[w][lane];
+        lin = fold(q.x, q.y, lin);
+        Pin *= q.y;
+    }
+    float c;
+    if (wave == nw - 1) {
+        const float lt = fold(l, P, lin), Pt = P * Pin;
+        c = n == 0 ? first : take_joint(word, n);
+        if (!last) pass_joint(word, fold(lt, Pt, c), n + 1);
+        pass_carry(carry[lane], c, n);
+    } else {
+        c = take_carry(carry[lane], n);
+    }
+    return fold(lin, Pin, c);
+}
+// Which column and member a workgroup of a joint launch is: the G members of a column follow one another on one XCD.
+__device__ __forceinline__ bool joint_place(const Joint& jt, int64_t D, int64_t& bh, unsigned& cb, int& member) {
+    const unsigned G = (unsigned)jt.G, nd = (unsigned)((D + 63) / 64), col = blockIdx.x / (8u * G) * 8u + blockIdx.x % 8u;
+    member = (int)(blockIdx.x / 8u % G);
+    bh = col / nd;
+    cb = col % nd;
+    return bh < jt.BH;                                                  // columns are padded to eights
+}
 // The parts of a wave's block in the order the scan takes them, k = 0 .. LS - 1 in lanes part(k): (lin, Pin) composes the parts
 // in front of this lane's, (lb, Pb) all of them.
 template <int LS, bool REVERSE>
@@ -83,19 +153,25 @@ __device__ __forceinline__ void compose_parts(float l, float P, int u, int ch, f
 }
 
 // -------------------------------------------------------------------------- forward, log gates
-template <typename T, bool AGG, int LS>
-__global__ __launch_bounds__(64 * kMaxWaves) void hgrn_scan_fwd_kernel(const T* __restrict__ x, const T* __restrict__ g,
+template <typename T, bool AGG, int LS, bool NT, bool JOINT>
+__global__ __launch_bounds__(64 * kMaxWaves, 4) void hgrn_scan_fwd_kernel(const T* __restrict__ x, const T* __restrict__ g,
                                                                        const float* __restrict__ h0, T* __restrict__ o,
                                                                        float* __restrict__ ht, float* __restrict__ agg,
-                                                                       int64_t Tlen, int64_t D, int64_t seg_len, int NS) {
+                                                                       int64_t Tlen, int64_t D, int64_t seg_len, int NS, Joint jt) {
     constexpr int CH = 64 / LS, kBlk = kFwdBlk, kStep = LS * kBlk;      // channels of a workgroup, steps of a wave's block
-    __shared__ float carry_h[CH], carry_p[CH];
-    __shared__ int turn;
+    __shared__ uint64_t carry[CH];
+    __shared__ float prod[AGG ? kMaxWaves : 1][64];
+    __shared__ float2 pairs[JOINT ? 2 : 1][JOINT ? kMaxWaves : 1][64];
     const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), nw = (int)blockDim.x >> 6;
     const int ch = lane % CH, u = lane / CH;                            // channel, and which kBlk steps of the wave's block
-    const int64_t bh = blockIdx.y;
-    const int seg = (int)blockIdx.z;                                    // AGG: nobody folds the pair of the last segment
-    const int64_t d = (int64_t)column_block<LS>() * CH + ch;
+    int64_t bh = blockIdx.y;
+    const int seg = JOINT ? 0 : (int)blockIdx.z;                        // AGG: nobody folds the pair of the last segment
+    unsigned cb = JOINT ? 0u : column_block<LS>();
+    int member = 0;
+    if constexpr (JOINT) {
+        if (!joint_place(jt, D, bh, cb, member)) return;
+    }
+    const int64_t d = (int64_t)cb * CH + ch;
     const bool active = d < D;
     const int64_t dl = active ? d : D - 1;
     const uint32_t rowb = (uint32_t)D * (uint32_t)sizeof(T);
@@ -103,7 +179,11 @@ __global__ __launch_bounds__(64 * kMaxWaves) void hgrn_scan_fwd_kernel(const T* 
     const uint32_t voff = cho + (uint32_t)(u * kBlk) * rowb;
     const int64_t t0 = (int64_t)seg * seg_len, t1 = t0 + seg_len < Tlen ? t0 + seg_len : Tlen;
     const int nblk = (int)((t1 - t0 + kStep - 1) / kStep);
-    if (wave == 0) {
+    const float first = JOINT && h0 ? h0[bh * D + dl] : 0.0f;
+    uint64_t* const word = JOINT ? jt.words + (bh * ((D + 63) / 64) + cb) * 64 + lane : nullptr;   // (lanes past D: words of their own)
+    int super = member;                                                 // JOINT: the superblock
+    if (JOINT && wave == 0) pass_carry(carry[ch], 0.0f, -1);
+    if (!JOINT && wave == 0) {
         float c = h0 && (!AGG || seg == 0) ? h0[bh * D + dl] : 0.0f;    // h0 enters the fold through segment 0's pair
         if constexpr (!AGG) {
             if (seg > 0) c = 0.0f;
@@ -112,10 +192,9 @@ __global__ __launch_bounds__(64 * kMaxWaves) void hgrn_scan_fwd_kernel(const T* 
                 c = fold(ag[D], ag[0], c);
             }
         }
-        carry_h[ch] = c;
-        carry_p[ch] = 1.0f;
-        if (lane == 0) turn = 0;
+        pass_carry(carry[ch], c, 0);
     }
+    float own = 1.0f;                                                   // AGG: product of this wave's gates
     __syncthreads();
     // One block; FULL: it has all its steps (no tests), otherwise the tail of the segment.
     auto block = [&](int n, int64_t tb, int rem, auto full) __attribute__((always_inline)) {
@@ -127,12 +206,12 @@ __global__ __launch_bounds__(64 * kMaxWaves) void hgrn_scan_fwd_kernel(const T* 
 #pragma unroll
         for (int t = 0; t < kBlk; ++t) {
             if constexpr (FULL) {
-                gr[t] = buf_bits<T>(rg, voff, (uint32_t)t * rowb);
-                xr[t] = buf_bits<T>(rx, voff, (uint32_t)t * rowb);
+                gr[t] = buf_bits<T, NT>(rg, voff, (uint32_t)t * rowb);
+                xr[t] = buf_bits<T, NT>(rx, voff, (uint32_t)t * rowb);
             } else {                                                     // rows past the end re-read the last one
                 const int row = u * kBlk + t < rem ? u * kBlk + t : rem - 1;
-                gr[t] = buf_bits<T>(rg, cho + (uint32_t)row * rowb, 0);
-                xr[t] = buf_bits<T>(rx, cho + (uint32_t)row * rowb, 0);
+                gr[t] = buf_bits<T, NT>(rg, cho + (uint32_t)row * rowb, 0);
+                xr[t] = buf_bits<T, NT>(rx, cho + (uint32_t)row * rowb, 0);
             }
         }
         float l = 0.0f, P = 1.0f;
@@ -152,56 +231,75 @@ __global__ __launch_bounds__(64 * kMaxWaves) void hgrn_scan_fwd_kernel(const T* 
         }
         float lin, Pin, lb, Pb;
         compose_parts<LS, false>(l, P, u, ch, lin, Pin, lb, Pb);
-        wait_turn(turn, n);
-        const float cb = carry_h[ch];
-        carry_h[ch] = fold(lb, Pb, cb);                                 // (the parts of a channel write the same value)
-        if constexpr (AGG) carry_p[ch] *= Pb;
-        __hip_atomic_store(&turn, n + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+        done_before_the_turn(l, P, lin, Pin, lb, Pb);
+        float cb;
+        if constexpr (JOINT) {
+            cb = joint_carry(lb, Pb, super, (super + 1) * nw >= nblk, wave, nw, pairs[super / jt.G & 1], carry, word, first);
+        } else {
+            cb = take_carry(carry[ch], n);
+            pass_carry(carry[ch], fold(lb, Pb, cb), n + 1);             // (the parts of a channel write the same value)
+            if constexpr (AGG) own *= Pb;
+        }
         if constexpr (!AGG) {
             const __amdgpu_buffer_rsrc_t ro = rsrc(o + row0);
             float h = fold(lin, Pin, cb);
 #pragma unroll
             for (int t = 0; t < kBlk; ++t) {
                 h = fmaf(h, __uint_as_float(gr[t]), __uint_as_float(xr[t]));
-                if (FULL || t < remu) buf_put<T>(ro, voff, (uint32_t)t * rowb, h);
+                if (FULL || t < remu) buf_put<T, NT>(ro, voff, (uint32_t)t * rowb, h);
             }
             // (steps past the end have left h alone; the part that holds the last step knows the state)
             if (ht && seg == NS - 1 && n == nblk - 1 && active && u == (rem - 1) / kBlk) ht[bh * D + d] = h;
         }
     };
-    for (int n = wave; n < nblk; n += nw) {
+    auto run = [&](int n) __attribute__((always_inline)) {
         const int64_t tb = t0 + (int64_t)n * kStep;
         const int rem = __builtin_amdgcn_readfirstlane((int)((t1 - tb) < (int64_t)kStep ? (t1 - tb) : (int64_t)kStep));
         if (rem == kStep) block(n, tb, rem, std::true_type{});
         else block(n, tb, rem, std::false_type{});
+    };
+    if constexpr (JOINT) {
+        for (; super * nw < nblk; super += jt.G) {
+            if (super * nw + wave < nblk) run(super * nw + wave);
+            else joint_carry(0.0f, 1.0f, super, true, wave, nw, pairs[super / jt.G & 1], carry, word, first);   // no block left for this wave
+        }
+    } else {
+        for (int n = wave; n < nblk; n += nw) run(n);
     }
     if constexpr (AGG) {
-        if (wave == 0) {
-            wait_turn(turn, nblk);
-            if (active) {
-                float* ag = agg + (bh * NS + seg) * 2 * D;
-                ag[d] = carry_p[ch];
-                ag[D + d] = carry_h[ch];
-            }
+        prod[wave][lane] = own;
+        __syncthreads();
+        if (wave == 0 && active) {
+            float P = 1.0f;
+            for (int w = 0; w < nw; ++w) P *= prod[w][lane];
+            float* ag = agg + (bh * NS + seg) * 2 * D;
+            ag[d] = P;
+            ag[D + d] = take_carry(carry[ch], nblk);
         }
     }
 }
 
 // -------------------------------------------------------------------------- backward
-template <typename T, bool LOG, bool AGG, int LS>
-__global__ __launch_bounds__(64 * kMaxWaves) void hgrn_scan_bwd_kernel(const T* __restrict__ g, const T* __restrict__ o,
+template <typename T, bool LOG, bool AGG, int LS, bool NT, bool JOINT>
+__global__ __launch_bounds__(64 * kMaxWaves, 4) void hgrn_scan_bwd_kernel(const T* __restrict__ g, const T* __restrict__ o,
                                                                        const T* __restrict__ dout, const float* __restrict__ h0,
                                                                        T* __restrict__ dx, T* __restrict__ dg,
                                                                        float* __restrict__ agg, int64_t Tlen, int64_t D,
-                                                                       int64_t seg_len, int NS) {
+                                                                       int64_t seg_len, int NS, Joint jt) {
     constexpr int CH = 64 / LS, kBlk = kBwdBlk, kStep = LS * kBlk;                      // channels of a workgroup, steps of a wave's block
-    __shared__ float carry_l[CH], carry_p[CH];
-    __shared__ int turn;
+    __shared__ uint64_t carry[CH];
+    __shared__ float prod[AGG ? kMaxWaves : 1][64];
+    __shared__ float2 pairs[JOINT ? 2 : 1][JOINT ? kMaxWaves : 1][64];
     const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), nw = (int)blockDim.x >> 6;
     const int ch = lane % CH, u = lane / CH;                            // channel, and which kBlk steps of the wave's block
-    const int64_t bh = blockIdx.y;
-    const int seg = AGG ? (int)blockIdx.z + 1 : (int)blockIdx.z;       // nobody folds the pair of segment 0
-    const int64_t d = (int64_t)column_block<LS>() * CH + ch;
+    int64_t bh = blockIdx.y;
+    const int seg = JOINT ? 0 : AGG ? (int)blockIdx.z + 1 : (int)blockIdx.z;   // nobody folds the pair of segment 0
+    unsigned cb = JOINT ? 0u : column_block<LS>();
+    int member = 0;
+    if constexpr (JOINT) {
+        if (!joint_place(jt, D, bh, cb, member)) return;
+    }
+    const int64_t d = (int64_t)cb * CH + ch;
     const bool active = d < D;
     const int64_t dl = active ? d : D - 1;
     const uint32_t rowb = (uint32_t)D * (uint32_t)sizeof(T);
@@ -210,7 +308,10 @@ __global__ __launch_bounds__(64 * kMaxWaves) void hgrn_scan_bwd_kernel(const T* 
     const int64_t t0 = (int64_t)seg * seg_len, t1 = t0 + seg_len < Tlen ? t0 + seg_len : Tlen;
     const int nblk = (int)((t1 - t0 + kStep - 1) / kStep);
     const float hinit = !AGG && h0 ? h0[bh * D + dl] : 0.0f;
-    if (wave == 0) {
+    uint64_t* const word = JOINT ? jt.words + (bh * ((D + 63) / 64) + cb) * 64 + lane : nullptr;   // (lanes past D: words of their own)
+    int super = member;                                                 // JOINT: the superblock
+    if (JOINT && wave == 0) pass_carry(carry[ch], 0.0f, -1);
+    if (!JOINT && wave == 0) {
         float c = 0.0f;
         if constexpr (!AGG) {
             for (int j = NS - 1; j > seg; --j) {
@@ -218,10 +319,9 @@ __global__ __launch_bounds__(64 * kMaxWaves) void hgrn_scan_bwd_kernel(const T* 
                 c = fold(ag[D], ag[0], c);
             }
         }
-        carry_l[ch] = c;
-        carry_p[ch] = 1.0f;
-        if (lane == 0) turn = 0;
+        pass_carry(carry[ch], c, 0);
     }
+    float own = 1.0f;                                                   // AGG: product of this wave's gates
     __syncthreads();
     // One block; FULL: it has all its steps (no tests), otherwise the tail of the segment.
     auto block = [&](int n, int64_t tb, int rem, auto full) __attribute__((always_inline)) {
@@ -236,17 +336,17 @@ __global__ __launch_bounds__(64 * kMaxWaves) void hgrn_scan_bwd_kernel(const T* 
 #pragma unroll
         for (int t = kBlk - 1; t >= 0; --t) {
             if constexpr (FULL) {
-                gr[t] = buf_bits<T>(rg, voff, (uint32_t)t * rowb);
-                dr[t] = buf_bits<T>(rd, voff, (uint32_t)t * rowb);
+                gr[t] = buf_bits<T, NT>(rg, voff, (uint32_t)t * rowb);
+                dr[t] = buf_bits<T, NT>(rd, voff, (uint32_t)t * rowb);
                 if constexpr (!AGG) {
-                    if (t > 0) hr[t] = buf_bits<T>(ro, voff, (uint32_t)(t - 1) * rowb + first);
-                    else hr[t] = buf_bits<T>(ro, back || u == 0 ? voff : voff - rowb, 0);
+                    if (t > 0) hr[t] = buf_bits<T, NT>(ro, voff, (uint32_t)(t - 1) * rowb + first);
+                    else hr[t] = buf_bits<T, NT>(ro, back || u == 0 ? voff : voff - rowb, 0);
                 }
             } else {                                                     // rows past the end re-read the last one
                 const int row = u * kBlk + t < rem ? u * kBlk + t : rem - 1, prev = row - 1 + back;
-                gr[t] = buf_bits<T>(rg, cho + (uint32_t)row * rowb, 0);
-                dr[t] = buf_bits<T>(rd, cho + (uint32_t)row * rowb, 0);
-                if constexpr (!AGG) hr[t] = buf_bits<T>(ro, cho + (uint32_t)(prev > 0 ? prev : 0) * rowb, 0);
+                gr[t] = buf_bits<T, NT>(rg, cho + (uint32_t)row * rowb, 0);
+                dr[t] = buf_bits<T, NT>(rd, cho + (uint32_t)row * rowb, 0);
+                if constexpr (!AGG) hr[t] = buf_bits<T, NT>(ro, cho + (uint32_t)(prev > 0 ? prev : 0) * rowb, 0);
             }
         }
         float last = 0.0f, glast = 1.0f, P = 1.0f;                      // the step after t: its dh from zero, its gate
@@ -270,14 +370,18 @@ __global__ __launch_bounds__(64 * kMaxWaves) void hgrn_scan_bwd_kernel(const T* 
             glast = gl;
             P *= gl;
         }
-        const float l = last * glast;
+        float l = last * glast;
         float lin, Pin, lb, Pb;
         compose_parts<LS, true>(l, P, u, ch, lin, Pin, lb, Pb);
-        wait_turn(turn, n);
-        const float cb = carry_l[ch];
-        carry_l[ch] = fold(lb, Pb, cb);                                 // (the parts of a channel write the same value)
-        if constexpr (AGG) carry_p[ch] *= Pb;
-        __hip_atomic_store(&turn, n + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+        done_before_the_turn(l, P, lin, Pin, lb, Pb);
+        float cb;
+        if constexpr (JOINT) {
+            cb = joint_carry(lb, Pb, super, (super + 1) * nw >= nblk, wave, nw, pairs[super / jt.G & 1], carry, word, 0.0f);
+        } else {
+            cb = take_carry(carry[ch], n);
+            pass_carry(carry[ch], fold(lb, Pb, cb), n + 1);             // (the parts of a channel write the same value)
+            if constexpr (AGG) own *= Pb;
+        }
         if constexpr (!AGG) {
             const __amdgpu_buffer_rsrc_t rx = rsrc(dx + row0), ry = rsrc(dg + row0);
             float dh = fold(lin, Pin, cb), gate = 1.0f;                 // of the step behind
@@ -286,43 +390,64 @@ __global__ __launch_bounds__(64 * kMaxWaves) void hgrn_scan_bwd_kernel(const T* 
                 dh = fmaf(dh, gate, __uint_as_float(dr[t]));
                 gate = __uint_as_float(gr[t]);
                 if (FULL || t < remu) {
-                    buf_put<T>(rx, voff, (uint32_t)t * rowb, dh);
-                    buf_put<T>(ry, voff, (uint32_t)t * rowb, dh * __uint_as_float(hr[t]));
+                    buf_put<T, NT>(rx, voff, (uint32_t)t * rowb, dh);
+                    buf_put<T, NT>(ry, voff, (uint32_t)t * rowb, dh * __uint_as_float(hr[t]));
                 }
             }
         }
     };
-    for (int n = wave; n < nblk; n += nw) {
+    auto run = [&](int n) __attribute__((always_inline)) {
         const int64_t tb = t0 + (int64_t)(nblk - 1 - n) * kStep;        // blocks from the latest to the earliest
         const int rem = __builtin_amdgcn_readfirstlane((int)((t1 - tb) < (int64_t)kStep ? (t1 - tb) : (int64_t)kStep));
         if (rem == kStep) block(n, tb, rem, std::true_type{});
         else block(n, tb, rem, std::false_type{});
+    };
+    if constexpr (JOINT) {
+        for (; super * nw < nblk; super += jt.G) {
+            if (super * nw + wave < nblk) run(super * nw + wave);
+            else joint_carry(0.0f, 1.0f, super, true, wave, nw, pairs[super / jt.G & 1], carry, word, 0.0f);   // no block left for this wave
+        }
+    } else {
+        for (int n = wave; n < nblk; n += nw) run(n);
     }
     if constexpr (AGG) {
-        if (wave == 0) {
-            wait_turn(turn, nblk);
-            if (active) {
-                float* ag = agg + (bh * NS + seg) * 2 * D;
-                ag[d] = carry_p[ch];
-                ag[D + d] = carry_l[ch];
-            }
+        prod[wave][lane] = own;
+        __syncthreads();
+        if (wave == 0 && active) {
+            float P = 1.0f;
+            for (int w = 0; w < nw; ++w) P *= prod[w][lane];
+            float* ag = agg + (bh * NS + seg) * 2 * D;
+            ag[d] = P;
+            ag[D + d] = take_carry(carry[ch], nblk);
         }
     }
 }
 
-// wgs = workgroups that columns of 64 channels give.  From 256 on nothing is split.  From 128 on a column is halved (LS = 2:
-// 55 -> 48 us for 4 x 2048 x 2048 bf16) rather than cut in time, whose pair launch reads two of the five streams again (68 us).
-// Below, short sequences are halved too (8.5 -> 6 us for 2 x 333 x 1024 fp32); from 2048 steps on whole 128-byte rows
-// (LS = 1: 113 against 126 us for 1 x 16384 x 2048) in time segments for about two workgroups per CU.  A segment is at
-// least four blocks long.
+// wgs = workgroups that columns of 64 channels give.  A CU keeps about 60 KB of loads in flight, whole 128-byte lines, so fewer workgroups
+// than CUs leave bandwidth unused: 128 of them reach 3.7 TB/s where 256 reach 5.2.  From 171 on nothing is split.
+//   32 to 170, long sequences: G workgroups share a column's superblocks (JOINT), about 256 workgroups up to 64 columns and 512 (two a CU)
+//      beyond.  bf16, forward + backward against the plans below: 64 x 16384 x 128 220 + 374 -> 160 + 262 us, 6 x 16384 x 1024 189 + 277 ->
+//      136 + 220, 16 x 16384 x 128 64 + 84 -> 50 + 71, 9 x 5000 x 1024 74 + 124 -> 69 + 109.  Below 3072 steps the hand-overs between
+//      workgroups show (64 x 2048 x 64 18 + 22 against 18 + 24, 7 x 1024 x 1024 11 + 16 against 17 + 22), below 32 columns the cut in time is as
+//      good (24 x 16384 x 64 48 + 63 / 48 + 64, 8 x 16384 x 64 28 + 31 / 45 + 60).
+//   up to 128, short sequences (and 128 columns at any length): a column is halved (LS = 2; 8.5 -> 6 us for 2 x 333 x 1024 fp32), at half
+//      a line a row and so half the bytes in flight; with more columns than that whole ones win (12 x 2048 x 1024 35 + 58 against 50 + 79).
+//   fewer columns, 2048 steps and more: whole 128-byte rows in time segments for about two workgroups per CU, a segment at least four
+//      blocks long; a first launch reads x and g (g and do) of all but one segment once more.
 struct Plan {
     int64_t seg_len;
-    int NS, LS;
+    int NS, LS, G;
 };
 Plan plan(int64_t BH, int64_t Tlen, int64_t D, int blk, bool split) {
     Plan p;
     const int64_t wgs = BH * mmf_ceil_div(D, 64);
-    p.LS = wgs < 256 && (wgs >= 128 || Tlen < 2048) ? 2 : 1;
+    p.G = split && wgs >= 32 && wgs <= 170 && Tlen >= 3072 ? (int)((wgs <= 64 ? 256 : 512) / wgs) : 1;
+    if (p.G > 1) {
+        p.LS = p.NS = 1;
+        p.seg_len = mmf_round_up(Tlen, blk);
+        return p;
+    }
+    p.LS = wgs <= 128 && (wgs == 128 || Tlen < 2048) ? 2 : 1;
     const int64_t now = BH * mmf_ceil_div(D, 64 / p.LS), step = p.LS * blk;
     int64_t ns = 1;
     if (split && now < 128) {
@@ -341,65 +466,104 @@ bool fwd_takes_workspace(int64_t BH, int64_t Tlen, int64_t D, int chunk) {
     return BH * mmf_ceil_div(D, 64) < 256 && Tlen >= 8 * block;
 }
 Plan fwd_plan(int64_t BH, int64_t Tlen, int64_t D, int chunk) { return plan(BH, Tlen, D, kFwdBlk, fwd_takes_workspace(BH, Tlen, D, chunk)); }
-int64_t pair_bytes(const Plan& p, int64_t BH, int64_t D) { return p.NS > 1 ? BH * p.NS * 2 * D * (int64_t)sizeof(float) : 0; }
+int64_t joint_bytes(int64_t BH, int64_t D) { return BH * mmf_round_up(D, 64) * 8; }
+int64_t pair_bytes(const Plan& p, int64_t BH, int64_t D) {
+    return p.G > 1 ? joint_bytes(BH, D) : p.NS > 1 ? BH * p.NS * 2 * D * (int64_t)sizeof(float) : 0;
+}
 // The kernels address a block of at most 64 rows with 32-bit offsets and count blocks in an int.
 bool fits(int64_t Tlen, int64_t D, int dtype) {
     return Tlen / kBwdBlk < (1ll << 30) && 64 * D * (int64_t)(dtype == MMF_F32 ? 4 : 2) < (1ll << 31);
 }
 
-template <typename T, int LS>
+__global__ __launch_bounds__(256) void joint_words_kernel(uint64_t* __restrict__ words, int64_t n) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) words[i] = 0;
+}
+bool holds_words(const float* workspace) { return workspace && (reinterpret_cast<uintptr_t>(workspace) & 7u) == 0; }
+int64_t joint_grid(const Plan& p, int64_t BH, int64_t D) { return mmf_round_up(BH * mmf_ceil_div(D, 64), 8) * p.G; }
+Joint joint_begin(const Plan& p, float* workspace, int64_t BH, int64_t D, hipStream_t s) {
+    uint64_t* words = reinterpret_cast<uint64_t*>(workspace);
+    const int64_t n = joint_bytes(BH, D) / 8;
+    joint_words_kernel<<<(unsigned)mmf_ceil_div(n, 256), 256, 0, s>>>(words, n);
+    return Joint{words, p.G, BH};
+}
+// Whether loads and stores are streamed past the caches.  Large tensors gain (40 x 2048 x 1024 bf16 118 + 198 -> 111 + 188 us, 128 x
+// 8192 x 128 156 + 259 -> 138 + 241, 5.8 TB/s), smaller ones that a consumer finds in the 256 MB last-level cache lose (16 x 777 x 1024
+// 14.5 + 27 against 18 + 29; even at 64 MB a tensor); in the second launch over time segments from 24 MB on (6000 x 64 columns 46 + 69 -> 45 + 62).
+bool streams(const Plan& p, int64_t bytes) { return bytes >= (p.NS > 1 ? 24ll << 20 : 64ll << 20); }
+template <typename T, int LS, bool NT>
 int launch_fwd_ls(const Plan& p, const T* x, const T* g, const float* h0, T* o, float* ht, float* agg, int64_t BH, int64_t Tlen,
                   int64_t D, hipStream_t s) {
     const int64_t nblk = p.seg_len / (LS * kFwdBlk);
     const unsigned threads = 64u * (unsigned)(nblk < kMaxWaves ? nblk : kMaxWaves), gx = (unsigned)mmf_ceil_div(D, 64 / LS);
     if (p.NS > 1) {
-        hgrn_scan_fwd_kernel<T, true, LS><<<dim3(gx, (unsigned)BH, (unsigned)(p.NS - 1)), threads, 0, s>>>(x, g, h0, o, ht, agg, Tlen, D,
-                                                                                                  p.seg_len, p.NS);
+        hgrn_scan_fwd_kernel<T, true, LS, false, false><<<dim3(gx, (unsigned)BH, (unsigned)(p.NS - 1)), threads, 0, s>>>(
+            x, g, h0, o, ht, agg, Tlen, D, p.seg_len, p.NS, Joint{});
         MMF_CHECK_LAUNCH();
     }
-    hgrn_scan_fwd_kernel<T, false, LS><<<dim3(gx, (unsigned)BH, (unsigned)p.NS), threads, 0, s>>>(x, g, h0, o, ht, agg, Tlen, D,
-                                                                                         p.seg_len, p.NS);
+    hgrn_scan_fwd_kernel<T, false, LS, NT, false><<<dim3(gx, (unsigned)BH, (unsigned)p.NS), threads, 0, s>>>(
+        x, g, h0, o, ht, agg, Tlen, D, p.seg_len, p.NS, Joint{});
     MMF_CHECK_LAUNCH();
     return 0;
 }
 template <typename T>
 int launch_fwd(const void* x, const void* g, const float* h0, void* o, float* ht, float* agg, int64_t BH, int64_t Tlen, int64_t D,
                int chunk, hipStream_t s) {
-    const Plan p = fwd_plan(BH, Tlen, D, chunk);
+    Plan p = fwd_plan(BH, Tlen, D, chunk);
+    if (p.G > 1 && !holds_words(agg)) p = plan(BH, Tlen, D, kFwdBlk, false);
     if (p.NS > 1 && !agg) return MMF_ERR_ARG;
     const T* xp = static_cast<const T*>(x);
     const T* gp = static_cast<const T*>(g);
     T* op = static_cast<T*>(o);
-    return p.LS == 2 ? launch_fwd_ls<T, 2>(p, xp, gp, h0, op, ht, agg, BH, Tlen, D, s)
-                     : launch_fwd_ls<T, 1>(p, xp, gp, h0, op, ht, agg, BH, Tlen, D, s);
+    if (p.G > 1) {
+        const Joint jt = joint_begin(p, agg, BH, D, s);
+        MMF_CHECK_LAUNCH();
+        hgrn_scan_fwd_kernel<T, false, 1, true, true><<<(unsigned)joint_grid(p, BH, D), 64 * kMaxWaves, 0, s>>>(
+            xp, gp, h0, op, ht, nullptr, Tlen, D, p.seg_len, 1, jt);
+        MMF_CHECK_LAUNCH();
+        return 0;
+    }
+    return p.LS == 2 ? launch_fwd_ls<T, 2, false>(p, xp, gp, h0, op, ht, agg, BH, Tlen, D, s)
+           : streams(p, BH * Tlen * D * (int64_t)sizeof(T)) ? launch_fwd_ls<T, 1, true>(p, xp, gp, h0, op, ht, agg, BH, Tlen, D, s)
+                                                        : launch_fwd_ls<T, 1, false>(p, xp, gp, h0, op, ht, agg, BH, Tlen, D, s);
 }
 
-template <typename T, bool LOG, int LS>
+template <typename T, bool LOG, int LS, bool NT>
 int launch_bwd_ls(const Plan& p, const T* g, const T* o, const T* dout, const float* h0, T* dx, T* dg, float* agg, int64_t BH,
                   int64_t Tlen, int64_t D, hipStream_t s) {
     const int64_t nblk = p.seg_len / (LS * kBwdBlk);
     const unsigned threads = 64u * (unsigned)(nblk < kMaxWaves ? nblk : kMaxWaves), gx = (unsigned)mmf_ceil_div(D, 64 / LS);
     if (p.NS > 1) {
-        hgrn_scan_bwd_kernel<T, LOG, true, LS><<<dim3(gx, (unsigned)BH, (unsigned)(p.NS - 1)), threads, 0, s>>>(
-            g, o, dout, h0, dx, dg, agg, Tlen, D, p.seg_len, p.NS);
+        hgrn_scan_bwd_kernel<T, LOG, true, LS, false, false><<<dim3(gx, (unsigned)BH, (unsigned)(p.NS - 1)), threads, 0, s>>>(
+            g, o, dout, h0, dx, dg, agg, Tlen, D, p.seg_len, p.NS, Joint{});
         MMF_CHECK_LAUNCH();
     }
-    hgrn_scan_bwd_kernel<T, LOG, false, LS><<<dim3(gx, (unsigned)BH, (unsigned)p.NS), threads, 0, s>>>(g, o, dout, h0, dx, dg, agg, Tlen,
-                                                                                              D, p.seg_len, p.NS);
+    hgrn_scan_bwd_kernel<T, LOG, false, LS, NT, false><<<dim3(gx, (unsigned)BH, (unsigned)p.NS), threads, 0, s>>>(
+        g, o, dout, h0, dx, dg, agg, Tlen, D, p.seg_len, p.NS, Joint{});
     MMF_CHECK_LAUNCH();
     return 0;
 }
 template <typename T, bool LOG>
 int launch_bwd(const void* g, const void* o, const void* dout, const float* h0, void* dx, void* dg, float* agg, int64_t BH,
                int64_t Tlen, int64_t D, hipStream_t s) {
-    const Plan p = plan(BH, Tlen, D, kBwdBlk, agg != nullptr);
+    Plan p = plan(BH, Tlen, D, kBwdBlk, agg != nullptr);
+    if (p.G > 1 && !holds_words(agg)) p = plan(BH, Tlen, D, kBwdBlk, false);
     const T* gp = static_cast<const T*>(g);
     const T* op = static_cast<const T*>(o);
     const T* dp = static_cast<const T*>(dout);
     T* xp = static_cast<T*>(dx);
     T* yp = static_cast<T*>(dg);
-    return p.LS == 2 ? launch_bwd_ls<T, LOG, 2>(p, gp, op, dp, h0, xp, yp, agg, BH, Tlen, D, s)
-                     : launch_bwd_ls<T, LOG, 1>(p, gp, op, dp, h0, xp, yp, agg, BH, Tlen, D, s);
+    if (p.G > 1) {
+        const Joint jt = joint_begin(p, agg, BH, D, s);
+        MMF_CHECK_LAUNCH();
+        hgrn_scan_bwd_kernel<T, LOG, false, 1, true, true><<<(unsigned)joint_grid(p, BH, D), 64 * kMaxWaves, 0, s>>>(
+            gp, op, dp, h0, xp, yp, nullptr, Tlen, D, p.seg_len, 1, jt);
+        MMF_CHECK_LAUNCH();
+        return 0;
+    }
+    return p.LS == 2 ? launch_bwd_ls<T, LOG, 2, false>(p, gp, op, dp, h0, xp, yp, agg, BH, Tlen, D, s)
+           : streams(p, BH * Tlen * D * (int64_t)sizeof(T)) ? launch_bwd_ls<T, LOG, 1, true>(p, gp, op, dp, h0, xp, yp, agg, BH, Tlen, D, s)
+                                                        : launch_bwd_ls<T, LOG, 1, false>(p, gp, op, dp, h0, xp, yp, agg, BH, Tlen, D, s);
 }
 
 // ht = h0 (or zeros) for an empty sequence; a kernel, not a memset, so it can be graph captured.
@@ -417,7 +581,8 @@ extern "C" {
 int64_t mmf_hgrn_chunk_workspace_bytes(int64_t BH, int64_t T, int64_t D, int chunk) {
     if (BH <= 0 || T <= 0 || D <= 0 || chunk < 1 || chunk > 64) return 0;
     if (!fwd_takes_workspace(BH, T, D, chunk)) return 0;
-    return BH * fwd_plan(BH, T, D, chunk).NS * 2 * D * (int64_t)sizeof(float);
+    const Plan p = fwd_plan(BH, T, D, chunk);
+    return p.G > 1 ? joint_bytes(BH, D) : BH * p.NS * 2 * D * (int64_t)sizeof(float);
 }
 
 int mmf_hgrn_chunk(const void* x, const void* g, const float* h0, void* o, float* ht, int64_t BH, int64_t T, int64_t D,

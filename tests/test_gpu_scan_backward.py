@@ -106,3 +106,35 @@ def test_a_zero_carry_survives_a_product_of_gates_that_overflows(dev, log):
         want[k] = 1.0 + 0.5 * want[k + 1]
     assert torch.isfinite(o).all() and torch.isfinite(dg).all()
     assert torch.allclose(dx[0, 0, :, 0].cpu(), want, rtol=1e-6, atol=0)
+
+
+@pytest.mark.parametrize("bh,d,t", [(32, 64, 3072), (11, 130, 3101), (31, 64, 3072), (64, 64, 3100), (65, 33, 3073), (128, 64, 3361), (170, 40, 3080),
+                                    (171, 40, 3080)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_scans_whose_columns_are_shared_by_workgroups(dev, bh, d, t, dtype):
+    """Long sequences around the numbers of columns (32, 64, 170) and the length from which 8 to 3 workgroups take turns on one column:
+    ragged columns, last rounds with fewer blocks than waves, an initial state; twice, on the same buffers.  The bound is that of the
+    cut sequences above; a 16-bit result is rounded once more (2^-8 of the value) and its gradients see a rounded o."""
+    import matmulfreellm_amd as mm
+    torch.manual_seed(bh + t)
+    g = torch.nn.functional.logsigmoid(torch.randn(1, bh, t, d, device=dev) + 2).to(dtype)
+    x, do, h0 = torch.randn(1, bh, t, d, device=dev).to(dtype), torch.randn(1, bh, t, d, device=dev).to(dtype), torch.randn(1, bh, d, device=dev)
+    a, xd, dd = g[0].double().exp(), x[0].double(), do[0].double()
+    h, dh, hs, dhs = h0[0].double(), 0.0, [], []
+    for i in range(t):
+        h = a[:, i] * h + xd[:, i]
+        hs.append(h)
+    for i in reversed(range(t)):
+        dh = dd[:, i] + dh
+        dhs.append(dh)
+        dh = dh * a[:, i]
+    o = torch.stack(hs, 1)
+    dx = torch.stack(dhs[::-1], 1)
+    want = [o, h, dx, dx * torch.cat([h0[0].double()[:, None], o[:, :-1]], 1) * a]
+    mine = [v.clone().requires_grad_() for v in (x, g)]
+    for _ in range(2):
+        got_o, last = mm.chunk_hgrn(*mine, h0, output_final_state=True)
+        got = [got_o[0], last[0], *(v[0] for v in torch.autograd.grad(got_o, mine, do))]
+        for name, p, r in zip(("o", "state", "dx", "dg"), got, want):
+            err = ((p.detach().double() - r).abs().max() / r.abs().max()).item()
+            assert err < (2e-5 if dtype == torch.float32 or name == "state" else 8e-3), (name, err)
