@@ -45,6 +45,13 @@ int mmf_decode_layers_traced(const void* phases, int n_layers, const void* table
  *   on whole vectors of such arguments differs.  All but [5] must be 0 (tests/test_gpu_ops.py). */
 int mmf_diag_check_exact_forms(unsigned long long* counts, void* stream);
 
+/* mmf_diag_check_near_forms: activations whose result is rounded to 16 bits are evaluated with hardware exp2 and rcp where both ends of
+ *   the interval that leaves round alike, and by their definition elsewhere.  counts = 9 zeroed uint64 on the device: [0] floats
+ *   x >= -87 (all of them are run) whose near sigmoid lies outside its stated bound; [1..4] results of swiglu, of the norm's swish
+ *   gate and of the gate math (g, x) that differ from the definition in bf16, [5..8] in fp16, each 16-bit argument with `partners`
+ *   (1..65536) values of the other operands.  All must be 0. */
+int mmf_diag_check_near_forms(int partners, unsigned long long* counts, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

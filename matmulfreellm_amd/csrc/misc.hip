@@ -106,6 +106,48 @@ __global__ __launch_bounds__(256) void exact_forms_kernel(unsigned long long* co
     if (bad_mid) atomicAdd(&counts[6], bad_mid);
 }
 
+// counts[0]: floats x >= -87 where mmf_sigmoid_near(x) is further from 1 / (1 + exp(-x)) than mmf_near_slack allows it.
+__global__ __launch_bounds__(256) void near_sigmoid_kernel(unsigned long long* counts) {
+    unsigned long long bad = 0;
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < (1ull << 32); i += stride) {
+        const float x = __uint_as_float((uint32_t)i);
+        if (!mmf_near_ok(x)) continue;
+        const double d = (double)__fadd_rn(1.0f, mmf_exp(-x));
+        if (x < 1e30f && fabs((double)mmf_sigmoid_near(x) * d - 1.0) > (3.0 + 1.25 * fabs((double)x)) * 0x1p-24) ++bad;
+        if (x >= 1e30f && mmf_sigmoid_near(x) != 1.0f) ++bad;
+    }
+    if (bad) atomicAdd(&counts[0], bad);
+}
+// Each of the 65536 values of T as the argument of the activations, against `partners` values for the other operands: results whose
+// bits differ from the definitions' (two NaNs count as equal).  counts[1..4]: swiglu, swish gate, gate math's g and x.
+template <typename T>
+__global__ __launch_bounds__(256) void near_forms_kernel(int partners, unsigned long long* counts) {
+    unsigned long long bad[4] = {0, 0, 0, 0};
+    const float a = mmf_to_float(mmf_from_bits16<T>((uint16_t)(blockIdx.x * 256 + threadIdx.x)));
+    auto same = [](float p, float q) { return (p != p && q != q) || __float_as_uint(p) == __float_as_uint(q); };
+    auto mix = [](uint32_t x) { x ^= x >> 16; x *= 0x7feb352du; x ^= x >> 15; x *= 0x846ca68bu; x ^= x >> 16; return x; };
+    for (int j = blockIdx.y; j < partners; j += gridDim.y) {
+        const uint32_t h = mix(blockIdx.x * 256 + threadIdx.x + 65536u * (uint32_t)j), h2 = mix(h + 0x9e3779b9u);
+        // operands of every magnitude for a quarter of the partners, of an activation's for the rest
+        const float wild = mmf_to_float(mmf_from_bits16<T>((uint16_t)h)), tame = ((float)(int)h2) * 0x1p-29f;
+        const float u[1] = {mmf_round_to<T>((j & 3) == 0 ? wild : tame)}, y[1] = {(j & 3) == 0 ? __uint_as_float(h) : tame}, av[1] = {a};
+        const float lb[1] = {(j & 1) == 0 ? 0.0f : (j & 7) == 1 ? wild : (float)(h2 >> 8) * 0x1p-24f};
+        float o[1], x[1], g[1];
+        mmf_swiglu_n<T, 1>(av, u, o);
+        bad[0] += !same(o[0], mmf_round_to<T>(mmf_swiglu_definition(a, u[0])));
+        mmf_swish_gate_n<T, 1>(y, av, o);
+        bad[1] += !same(o[0], mmf_round_to<T>(__fmul_rn(__fmul_rn(y[0], a), mmf_sigmoid_definition(a))));
+        mmf_gate_n<T, 1>(u, av, lb, x, g);
+        const float gd = mmf_round_to<T>(mmf_gate_definition(mmf_sigmoid_definition(a), lb[0]));
+        bad[2] += !same(g[0], gd);
+        bad[3] += !same(x[0], mmf_round_to<T>(mmf_swiglu_definition(u[0], __fsub_rn(1.0f, gd))));
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        if (bad[j]) atomicAdd(&counts[1 + j], bad[j]);
+}
+
 }  // namespace
 
 extern "C" {
@@ -152,6 +194,18 @@ int mmf_diag_check_exact_forms(unsigned long long* counts, void* stream_) {
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     if (!counts) return MMF_ERR_ARG;
     exact_forms_kernel<<<4096, 256, 0, stream>>>(counts);
+    MMF_CHECK_LAUNCH();
+    return 0;
+}
+
+int mmf_diag_check_near_forms(int partners, unsigned long long* counts, void* stream_) {
+    hipStream_t stream = static_cast<hipStream_t>(stream_);
+    if (!counts || partners < 1 || partners > (1 << 16)) return MMF_ERR_ARG;
+    near_sigmoid_kernel<<<4096, 256, 0, stream>>>(counts);
+    MMF_CHECK_LAUNCH();
+    near_forms_kernel<bf16_t><<<dim3(256, 16), 256, 0, stream>>>(partners, counts);
+    MMF_CHECK_LAUNCH();
+    near_forms_kernel<f16_t><<<dim3(256, 16), 256, 0, stream>>>(partners, counts + 4);   // its results go to [5..8]
     MMF_CHECK_LAUNCH();
     return 0;
 }

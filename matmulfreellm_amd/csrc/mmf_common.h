@@ -12,6 +12,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 // Keep every multiply and add separately rounded in all code that includes this header,
 // whatever -ffp-contract the translation unit is built with.
@@ -314,6 +315,125 @@ __device__ __forceinline__ void mmf_sigmoid_n(const float (&x)[N], float (&s)[N]
 #pragma unroll
         for (int i = 0; i < N; ++i) s[i] = mmf_sigmoid(x[i]);
     }
+}
+
+// Activations whose result is rounded to 16 bits.  The exact exp, reciprocal and divide of the definitions take 40 to 50 issue
+// slots an element, and 16 of the 24 result bits are thrown away.  mmf_sigmoid_near takes 10 (hardware exp2 and rcp); what is rounded
+// is then known to lie within v * (1 +- slack), and when both ends round to the same T, so does the defining sequence's value.
+// Otherwise (about 2 elements in 10^4 for bf16, 2 in 10^3 for fp16, and arguments or products outside the middle range) the
+// element takes the defining sequence.  Same bits either way.
+// mmf_sigmoid_near(x) is within (3 + 1.25 |x|) * 2^-24 of 1 / d, d = 1 + mmf_exp(-x) as rounded, for every float x >= -87
+// (mmf_diag_check_near_forms runs them all: the rounding of the exponent and of log2 e grows with |x|, 2.8 is left); each rounding
+// on top, of either side, is one unit more, and one is for the ends' own.
+__device__ __forceinline__ float mmf_sigmoid_near(float x) {
+    return __builtin_amdgcn_rcpf(__fadd_rn(1.0f, __builtin_amdgcn_exp2f(__fmul_rn(x, -1.44269504088896341f))));
+}
+__device__ __forceinline__ bool mmf_near_ok(float x) { return x >= -87.0f; }          // (false for NaN)
+template <int ROUNDINGS>
+__device__ __forceinline__ float mmf_near_slack(float x) {
+    return __builtin_fmaf(fabsf(x), 1.25f * 0x1p-24f, (4.0f + ROUNDINGS) * 0x1p-24f);
+}
+// T(v), brought back; `redo` is set when a value within v * (1 +- slack) rounds to another T.  Where v is subnormal a relative
+// bound says nothing: SMALL says that it can be.
+template <typename T, bool SMALL>
+__device__ __forceinline__ float mmf_round_if_sure(float v, float slack, bool& redo) {
+    const float hi = __builtin_fmaf(v, slack, v), lo = __builtin_fmaf(v, -slack, v);
+    if constexpr (SMALL) redo = redo | (bool)__builtin_amdgcn_classf(v, 0x90);
+    if constexpr (std::is_same<T, bf16_t>::value) {              // both ends in one convert
+        typedef float f2 __attribute__((ext_vector_type(2)));
+        typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+        const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2{lo, hi}), b2));
+        redo = redo | ((uint16_t)w != (uint16_t)(w >> 16));
+        return __uint_as_float(w & 0xffff0000u);
+    } else {
+        const T th = mmf_from_float<T>(hi), tl = mmf_from_float<T>(lo);
+        redo = redo | (mmf_bits16(th) != mmf_bits16(tl));
+        return mmf_to_float(th);
+    }
+}
+// What it costs: a wave in which one lane of one element falls back runs the definition's code once more, 1 to 2 % of the waves per
+// element in bf16 and 8 to 12 % in fp16.  Where waves wait for each other the slowest one counts, so kernels whose time is a
+// dependent chain keep the definitions (NEAR = false): the o_proj GEMV of five rows 3.8 us with them, 4.3 with the near form.
+// o = T((g * u) / (1 + exp(-g))); T = float: the definition, nothing to round.
+__device__ __forceinline__ float mmf_swiglu_definition(float g, float u) {
+    return __fdiv_rn(__fmul_rn(g, u), __fadd_rn(1.0f, mmf_exp(-g)));
+}
+template <typename T, int N, bool NEAR = true>
+__device__ __forceinline__ void mmf_swiglu_n(const float (&g)[N], const float (&u)[N], float (&o)[N]) {
+    if constexpr (sizeof(T) == 4 || !NEAR) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) o[i] = mmf_round_to<T>(mmf_swiglu_definition(g[i], u[i]));
+    } else {
+        bool redo[N], any = false;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            redo[i] = !mmf_near_ok(g[i]);
+            o[i] = mmf_round_if_sure<T, true>(__fmul_rn(__fmul_rn(g[i], u[i]), mmf_sigmoid_near(g[i])), mmf_near_slack<2>(g[i]), redo[i]);
+            any = any | redo[i];
+        }
+        if (__builtin_expect(any, 0)) {
+#pragma unroll
+            for (int i = 0; i < N; ++i)
+                if (redo[i]) o[i] = mmf_round_to<T>(mmf_swiglu_definition(g[i], u[i]));
+        }
+    }
+}
+// o = T((y * a) * sigmoid(a)), the swish gate behind a norm
+template <typename T, int N, bool NEAR = true>
+__device__ __forceinline__ void mmf_swish_gate_n(const float (&y)[N], const float (&a)[N], float (&o)[N]) {
+    float p[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) p[i] = __fmul_rn(y[i], a[i]);
+    if constexpr (sizeof(T) == 4 || !NEAR) {
+        float s[N];
+        mmf_sigmoid_n<N>(a, s);
+#pragma unroll
+        for (int i = 0; i < N; ++i) o[i] = mmf_round_to<T>(__fmul_rn(p[i], s[i]));
+    } else {
+        bool redo[N], any = false;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            redo[i] = !mmf_near_ok(a[i]);
+            o[i] = mmf_round_if_sure<T, true>(__fmul_rn(p[i], mmf_sigmoid_near(a[i])), mmf_near_slack<3>(a[i]), redo[i]);
+            any = any | redo[i];
+        }
+        if (__builtin_expect(any, 0)) {
+#pragma unroll
+            for (int i = 0; i < N; ++i)
+                if (redo[i]) o[i] = mmf_round_to<T>(__fmul_rn(p[i], mmf_sigmoid(a[i])));
+        }
+    }
+}
+// The gate math of mmfreelm/layers/hgrn_bit.py:113-120:
+//   go = T(lb + (1 - lb) * sigmoid(f))
+//   xo = T((i * (1 - go)) / (1 + exp(-i)))
+// without lower bounds lb = 0, which leaves sigmoid(f) bit for bit.  The bound on go needs both terms of the sum positive, as lower
+// bounds are: in [0, 1].
+__device__ __forceinline__ float mmf_gate_definition(float s, float lb) { return __fadd_rn(lb, __fmul_rn(__fsub_rn(1.0f, lb), s)); }
+template <typename T, int N, bool NEAR = true>
+__device__ __forceinline__ void mmf_gate_n(const float (&iv)[N], const float (&fv)[N], const float (&lb)[N], float (&xo)[N], float (&go)[N]) {
+    float u[N];
+    if constexpr (sizeof(T) == 4 || !NEAR) {
+        mmf_sigmoid_n<N>(fv, go);
+#pragma unroll
+        for (int i = 0; i < N; ++i) go[i] = mmf_round_to<T>(mmf_gate_definition(go[i], lb[i]));
+    } else {
+        bool redo[N], any = false;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            redo[i] = !mmf_near_ok(fv[i]) | !((lb[i] >= 0.0f) & (lb[i] <= 1.0f));
+            go[i] = mmf_round_if_sure<T, false>(mmf_gate_definition(mmf_sigmoid_near(fv[i]), lb[i]), mmf_near_slack<5>(fv[i]), redo[i]);
+            any = any | redo[i];
+        }
+        if (__builtin_expect(any, 0)) {
+#pragma unroll
+            for (int i = 0; i < N; ++i)
+                if (redo[i]) go[i] = mmf_round_to<T>(mmf_gate_definition(mmf_sigmoid(fv[i]), lb[i]));
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) u[i] = __fsub_rn(1.0f, go[i]);
+    mmf_swiglu_n<T, N, NEAR>(iv, u, xo);
 }
 
 // ---------------------------------------------------------------- reductions (wave64)

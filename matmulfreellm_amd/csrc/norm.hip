@@ -122,10 +122,10 @@ __global__ __launch_bounds__(kThreads) void row_kernel(RowArgs a) {
                 amax = fmaxf(amax, fabsf(y));
             }
             if constexpr (MODE == ROW_GATE) {
-                float sg[8];
-                mmf_sigmoid_n<8>(ov[v], sg);
+                float y[8];
 #pragma unroll
-                for (int i = 0; i < 8; ++i) xv[v][i] = __fmul_rn(__fmul_rn(xv[v][i], ov[v][i]), sg[i]);
+                for (int i = 0; i < 8; ++i) y[i] = xv[v][i];
+                mmf_swish_gate_n<T, 8>(y, ov[v], xv[v]);
             }
             if constexpr (MODE != ROW_QUANT)
                 mmf_store8<T>(static_cast<T*>(a.y) + row * K, k0, K, vec_ok, xv[v]);
@@ -242,7 +242,9 @@ constexpr int kQWaves = 8, kQThreads = kQWaves * 64;
 //             reductions cost little, and many elements per thread.
 // Bound by HBM and the vector units about equally (a row of 2048 quantised three times: ~1100 issue slots a wave against 16 KiB of
 // traffic), so what does not depend on the data is kept out: no bounds test in passes known to lie in the row, codes rounded and
-// packed four at a time.  8192 x 2048 bf16, three norms: 37 -> 28 us; residual norm: 33 -> 22.
+// packed four at a time.  8192 x 2048 bf16, three norms: 37 -> 28 us; residual norm: 33 -> 22.  The gated form takes its sigmoids near
+// (16384 x 2048: 56 -> 52 us, 2002 x 2048 10.6 -> 9.8), and so does the step form (64 x 2048: 5.5 -> 4.9); with a row a workgroup the
+// gated form keeps the exact ones (64 x 2048: 4.1 against 4.3).
 // VEC: K, the strides and every pointer allow 4-element accesses.
 // NN = 3: the row is normalised once and quantised under three norm weights (the projections of a trained layer share their
 // input, not their inner norm): one read of the row and one rstd instead of three, the three maxima in one exchange.
@@ -322,18 +324,14 @@ __global__ __launch_bounds__(kQThreads) void row_quant_fused_kernel(FusedQuantAr
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             const int k0 = (v * TPR + tr) * 4;
-            float gv[4], stv[4], lbv[4];
+            float gv[4], stv[4], lbv[4] = {0.0f, 0.0f, 0.0f, 0.0f}, xo[4], go[4];
             raw4_unpack<T>(graw[v], gv);
             raw4_unpack<float>(straw[v], stv);
             if (a.lb) raw4_unpack<float>(lbraw[v], lbv);
+            mmf_gate_n<T, 4>(xv[v], av[v], lbv, xo, go);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const float iv = xv[v][i], fv = av[v][i];
-                float s = mmf_sigmoid(fv);
-                if (a.lb) s = __fadd_rn(lbv[i], __fmul_rn(__fsub_rn(1.0f, lbv[i]), s));
-                const float go = mmf_round_to<T>(s);
-                const float xo = mmf_round_to<T>(__fdiv_rn(__fmul_rn(iv, __fsub_rn(1.0f, go)), __fadd_rn(1.0f, mmf_exp(-iv))));
-                const float h = __fadd_rn(__fmul_rn(go, stv[i]), xo);
+                const float h = __fadd_rn(__fmul_rn(go[i], stv[i]), xo[i]);
                 stv[i] = h;
                 av[v][i] = mmf_round_to<T>(h);          // o, the swish gate of the gated norm
                 xv[v][i] = inb(v, k0, i) ? gv[i] : 0.0f;   // the gated norm normalises the g projection
@@ -359,26 +357,25 @@ __global__ __launch_bounds__(kQThreads) void row_quant_fused_kernel(FusedQuantAr
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             const int k0 = (v * TPR + tr) * 4;
-            float w1v[4], sg[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            float w1v[4], y[4];
             raw4_unpack<TW>(w1raw[v], w1v);
-            if constexpr (STEP || PRO == QPRO_GATEDNORM) mmf_sigmoid_n<4>(av[v], sg);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) y[i] = __fmul_rn(__fmul_rn(xv[v][i], rstd1), w1v[i]);
+            if constexpr (STEP || PRO == QPRO_GATEDNORM) mmf_swish_gate_n<T, 4, STEP || (RPW > 1)>(y, av[v], xv[v]);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                float y = __fmul_rn(__fmul_rn(xv[v][i], rstd1), w1v[i]);
-                if constexpr (STEP || PRO == QPRO_GATEDNORM) y = __fmul_rn(__fmul_rn(y, av[v][i]), sg[i]);
-                xv[v][i] = inb(v, k0, i) ? mmf_round_to<T>(y) : 0.0f;
+                if constexpr (!(STEP || PRO == QPRO_GATEDNORM)) xv[v][i] = mmf_round_to<T>(y[i]);
+                if (!inb(v, k0, i)) xv[v][i] = 0.0f;
             }
         }
     } else if constexpr (PRO == QPRO_SWIGLU) {
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             const int k0 = (v * TPR + tr) * 4;
+            float z[4];
+            mmf_swiglu_n<T, 4>(xv[v], av[v], z);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float g = xv[v][i];
-                const float z = __fdiv_rn(__fmul_rn(g, av[v][i]), __fadd_rn(1.0f, mmf_exp(-g)));
-                xv[v][i] = inb(v, k0, i) ? mmf_round_to<T>(z) : 0.0f;
-            }
+            for (int i = 0; i < 4; ++i) xv[v][i] = inb(v, k0, i) ? z[i] : 0.0f;
         }
     }
     // BitLinear's own norm + absmax codes
@@ -566,13 +563,11 @@ __global__ __launch_bounds__(256) void swiglu_kernel(const T* __restrict__ x, in
     const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= rows * vpr) return;
     const int64_t r = idx / vpr, c0 = (idx % vpr) * 8;
-    float xv[8], yv[8];
+    float xv[8], yv[8], z[8];
     mmf_load8<T>(x + r * ldx, c0, cols, true, xv);
     mmf_load8<T>(y + r * ldy, c0, cols, true, yv);
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-        xv[i] = __fdiv_rn(__fmul_rn(xv[i], yv[i]), __fadd_rn(1.0f, mmf_exp(-xv[i])));
-    mmf_store8<T>(out + r * cols, c0, cols, true, xv);
+    mmf_swiglu_n<T, 8>(xv, yv, z);
+    mmf_store8<T>(out + r * cols, c0, cols, true, z);
 }
 
 template <typename T>
@@ -582,7 +577,7 @@ __global__ __launch_bounds__(256) void swiglu_scalar_kernel(const T* __restrict_
     if (idx >= rows * cols) return;
     const int64_t r = idx / cols, c = idx % cols;
     const float xv = mmf_to_float(x[r * ldx + c]), yv = mmf_to_float(y[r * ldy + c]);
-    out[r * cols + c] = mmf_from_float<T>(__fdiv_rn(__fmul_rn(xv, yv), __fadd_rn(1.0f, mmf_exp(-xv))));
+    out[r * cols + c] = mmf_from_float<T>(mmf_swiglu_definition(xv, yv));
 }
 
 template <typename T>
