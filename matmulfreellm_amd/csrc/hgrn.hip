@@ -174,28 +174,22 @@ __global__ __launch_bounds__(64 * NW) void hgrn_recurrent_pipelined_kernel(const
 }
 
 // -------------------------------------------------------------------------- gate math
-// g_out = T( lb + (1 - lb) * sigmoid(f) )   (lb == null: T(sigmoid(f)))
-// x_out = T( (i * (1 - g_out)) / (1 + exp(-i)) ), zeroed where mask == 0
-// sf = sigmoid(f), taken by the caller for all its elements at once (mmf_sigmoid_n)
-template <typename T>
-__device__ __forceinline__ void gate_math(float iv, float sf, bool has_lb, float lb, float& xo, float& go) {
-    float s = sf;
-    if (has_lb) s = __fadd_rn(lb, __fmul_rn(__fsub_rn(1.0f, lb), s));
-    go = mmf_round_to<T>(s);
-    const float u = __fsub_rn(1.0f, go);
-    xo = mmf_round_to<T>(__fdiv_rn(__fmul_rn(iv, u), __fadd_rn(1.0f, mmf_exp(-iv))));
-}
+// mmf_gate_n gives g_out and x_out, x_out zeroed where mask == 0.
 
 // -------------------------------------------------------------------------- gate math and recurrence of a prompt in one launch
 // o = scan of the gated (x, g), x and g never leaving the CU.  A workgroup owns CPW channels of one sequence; wave 0 runs the
 // recurrence, the other 15 feed it: they load raw i and f two tiles ahead, do the gate math of the next tile into LDS (float2 per
 // step and channel) and round and store the outputs of the tile before, while wave 0 walks the current tile -- per step one LDS
 // read, multiply, add, LDS write -- at raised priority.  One LDS-only barrier per tile (a full one would wait for the loads ahead).
-// The vector units are the bound: the exact exp, sigmoid and divide are ~85 issue slots an element, which a wave walking time alone
-// would put behind the recurrence; with 16-channel workgroups even one sequence reaches 64 to 128 CUs.  CPW is the narrowest that
+// HBM and the vector units bound it about equally (the gate math is ~55 issue slots an element, which a wave walking time alone
+// would put behind the recurrence); with 16-channel workgroups even one sequence reaches 64 to 128 CUs.  CPW is the narrowest that
 // leaves at most two workgroups per CU (wider blocks have longer rows to load, 32 bytes at 16 channels; the four blocks that share
-// a 128-byte line run on one XCD).  Against gate and scan as two launches, bf16: 1 x 77 x 1024 9.4 -> 5.1 us, 3 x 459 x 2048
-// 26 -> 16, 2 x 1001 x 2048 34 -> 23, 8 x 2048 x 2048 103 -> 81 (twice or half as many workgroups: 93, 96).
+// a 128-byte line run on one XCD).  A turn requests and stores the same number of vectors whatever the tile, past the sequence's
+// ends through resources without records: the compiler then waits for one set of loads by count, where a store or load under a
+// branch made it wait for everything in flight, a trip to memory in every turn.  Wave 0 reads its steps a group ahead into two
+// sets of registers in turn, without copies between them.  bf16 in us, against branches, copies and the exact gate math: 8 x 2048 x 2048
+// 95 -> 63 (201 MB: 3.2 TB/s), 16 x 900 x 1024 42 -> 28, 2 x 1001 x 2048 24 -> 18, 3 x 459 x 2048 16 -> 12, 64 x 32 x 2048 23 -> 18, 4 x 300 x 1024
+// 9.5 -> 7.2, 1 x 77 x 1024 5.1 -> 4.9.
 struct GateScanArgs {
     const void* i; const void* f;       // rows [B * T, D], row strides ldi, ldf
     const float* lb; const uint8_t* mask;
@@ -206,10 +200,10 @@ struct GateScanArgs {
 };
 __device__ __forceinline__ void lds_only_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-template <typename T, int CPW, int PASS>
+template <typename T, int CPW, int PASS, bool MASK>
 __global__ __launch_bounds__(1024) void hgrn_gate_scan_kernel(GateScanArgs a) {
-    constexpr int NP = 15, SPW = 64 / CPW, TT = NP * SPW * PASS, U = 10;   // steps of a tile: 120 (60), 60 or 30
-    static_assert(TT % U == 0, "the recurrence walks a full tile in whole groups");
+    constexpr int NP = 15, SPW = 64 / CPW, TT = NP * SPW * PASS, U = TT >= 60 ? 10 : 5;   // steps of a tile: 120 (60), 60 or 30
+    static_assert(TT % (2 * U) == 0, "the recurrence walks a full tile in pairs of groups");
     __shared__ float2 gx[2][TT * CPW];
     __shared__ float hb[2][TT * CPW];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -220,37 +214,53 @@ __global__ __launch_bounds__(1024) void hgrn_gate_scan_kernel(GateScanArgs a) {
     const int64_t d = (int64_t)cb * CPW + c;
     const bool active = d < a.D;
     const int64_t dd = active ? d : 0, r0 = (int64_t)blockIdx.y * a.T;
-    const int NT = (a.T + TT - 1) / TT;
+    const int NT = (a.T + TT - 1) / TT, turns = NT + NT % 2;
 
     if (wave == 0) {
         __builtin_amdgcn_s_setprio(3);
         float h = a.h0 && active ? a.h0[(int64_t)blockIdx.y * a.D + dd] : 0.0f;
         lds_only_barrier();                                     // tile 0 is there
-        for (int k = 0; k < NT; ++k) {
-            const int n = a.T - k * TT < TT ? a.T - k * TT : TT;
+        for (int k = 0; k < turns; ++k) {
+            const int n = a.T - k * TT < TT ? a.T - k * TT : TT;   // (<= 0 in the turn that evens their number)
             const float2* src = gx[k & 1] + c;
             float* dst = hb[k & 1] + c;
-            float2 cur[U], nxt[U];
+            float2 va[U], vb[U];                                // groups of steps, read one ahead
+            auto read = [&](float2 (&v)[U], int j) __attribute__((always_inline)) {
+                const float2* p = src + (j <= TT - U ? j : TT - U) * CPW;
 #pragma unroll
-            for (int u = 0; u < U; ++u) cur[u] = src[u * CPW];
-            int j = 0;
-            for (; j + U <= n; j += U) {
-                const int jn = j + 2 * U <= TT ? j + U : j;     // the last group re-reads itself
-#pragma unroll
-                for (int u = 0; u < U; ++u) nxt[u] = src[(jn + u) * CPW];
+                for (int u = 0; u < U; ++u) v[u] = p[u * CPW];
+            };
+            auto walk = [&](const float2 (&v)[U], int j) __attribute__((always_inline)) {
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    h = __fadd_rn(__fmul_rn(cur[u].x, h), cur[u].y);
+                    h = __fadd_rn(__fmul_rn(v[u].x, h), v[u].y);
                     dst[(j + u) * CPW] = h;
                 }
+            };
+            auto walk_tail = [&](const float2 (&v)[U], int j) __attribute__((always_inline)) {
 #pragma unroll
-                for (int u = 0; u < U; ++u) cur[u] = nxt[u];
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {                       // what is left of the last tile: the group read ahead holds it
-                if (j + u < n) {
-                    h = __fadd_rn(__fmul_rn(cur[u].x, h), cur[u].y);
-                    dst[(j + u) * CPW] = h;
+                for (int u = 0; u < U; ++u) {
+                    if (j + u < n) {
+                        h = __fadd_rn(__fmul_rn(v[u].x, h), v[u].y);
+                        dst[(j + u) * CPW] = h;
+                    }
+                }
+            };
+            if (lane < CPW) {
+                read(va, 0);
+                int j = 0;
+                for (; j + 2 * U <= n; j += 2 * U) {
+                    read(vb, j + U);
+                    walk(va, j);
+                    read(va, j + 2 * U);
+                    walk(vb, j + U);
+                }
+                if (j + U <= n) {                               // what is left of the last tile
+                    read(vb, j + U);
+                    walk(va, j);
+                    walk_tail(vb, j + U);
+                } else if (j < n) {
+                    walk_tail(va, j);
                 }
             }
             lds_only_barrier();
@@ -259,97 +269,123 @@ __global__ __launch_bounds__(1024) void hgrn_gate_scan_kernel(GateScanArgs a) {
         return;
     }
 
+    using R = typename std::conditional<sizeof(T) == 4, float, uint16_t>::type;
+    constexpr int e = (int)sizeof(T), kRsrcFlags = 0x00020000;
     const int p = wave - 1;
-    const T* ip = static_cast<const T*>(a.i);
-    const T* fp = static_cast<const T*>(a.f);
-    T* op = static_cast<T*>(a.o);
-    const bool has_lb = a.lb != nullptr;
-    const float lb = has_lb ? a.lb[dd] : 0.0f;
-    T ir[2][PASS], fr[2][PASS];
+    const float lb = a.lb ? a.lb[dd] : 0.0f;
+    R ir[2][PASS], fr[2][PASS];
     uint8_t mr[2][PASS];
     auto at = [&](int q) __attribute__((always_inline)) { return (q * NP + p) * SPW + sub; };   // step of a tile
-    uint32_t oi[PASS], of[PASS];                                // offsets into a tile's rows (the launcher: they fit)
+    const int ldi = (int)a.ldi * e, ldf = (int)a.ldf * e, ldo = (int)a.D * e;   // bytes; the launcher: a tile of rows fits 31 bits
+    uint32_t oi[PASS], of[PASS], oo[PASS];                      // byte offsets into a tile's rows
 #pragma unroll
     for (int q = 0; q < PASS; ++q) {
-        oi[q] = (uint32_t)at(q) * (uint32_t)a.ldi + (uint32_t)dd;
-        of[q] = (uint32_t)at(q) * (uint32_t)a.ldf + (uint32_t)dd;
+        oi[q] = (uint32_t)at(q) * (uint32_t)ldi + (uint32_t)dd * e;
+        of[q] = (uint32_t)at(q) * (uint32_t)ldf + (uint32_t)dd * e;
+        oo[q] = active ? (uint32_t)at(q) * (uint32_t)ldo + (uint32_t)dd * e : 0x80000000u;   // lanes past D store nothing
     }
-    auto load = [&](int k, auto S) __attribute__((always_inline)) {
+    // the tile to load next and the tile to store next: bases, and the sequence's rows from there on (loads past them give zeros,
+    // stores are dropped: a resource of no records)
+    const char* ip = static_cast<const char*>(a.i) + r0 * ldi;
+    const char* fp = static_cast<const char*>(a.f) + r0 * ldf;
+    const uint8_t* mp = MASK ? a.mask + r0 : nullptr;
+    char* op = static_cast<char*>(a.o) + r0 * ldo;
+    int rows_in = a.T, rows_out = a.T;
+    auto rsrc = [&](const void* base, int rows, int ld) __attribute__((always_inline)) {
+        // (uniform values, which the compiler has to be told of pointers carried round the loop: it looped over lanes otherwise)
+        const uint64_t b = (uint64_t)base;
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((int)b), hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+        return __builtin_amdgcn_make_buffer_rsrc((void*)((uint64_t)hi << 32 | lo), 0,
+                                                 __builtin_amdgcn_readfirstlane((rows < 0 ? 0 : rows < TT ? rows : TT) * ld), kRsrcFlags);
+    };
+    auto load = [&](auto S) __attribute__((always_inline)) {
         constexpr int s = decltype(S)::value;
-        const int kk = k < NT ? k : NT - 1, last = a.T - 1 - kk * TT;
-        const int64_t row = r0 + (int64_t)kk * TT;
-        const T* it = ip + row * a.ldi;
-        const T* ft = fp + row * a.ldf;
-        const uint8_t* mt = a.mask ? a.mask + row : nullptr;
+        const __amdgpu_buffer_rsrc_t ti = rsrc(ip, rows_in, ldi), tf = rsrc(fp, rows_in, ldf);
 #pragma unroll
         for (int q = 0; q < PASS; ++q) {
-            if (last >= TT - 1) {
-                ir[s][q] = it[oi[q]];
-                fr[s][q] = ft[of[q]];
-                mr[s][q] = mt ? mt[at(q)] : (uint8_t)1;
-            } else {                                            // steps past the end: the last one once more, never used
-                const uint32_t t = (uint32_t)(at(q) < last ? at(q) : last);
-                ir[s][q] = it[t * (uint32_t)a.ldi + (uint32_t)dd];
-                fr[s][q] = ft[t * (uint32_t)a.ldf + (uint32_t)dd];
-                mr[s][q] = mt ? mt[t] : (uint8_t)1;
-            }
+            ir[s][q] = buf_load<R>(ti, oi[q], 0);
+            fr[s][q] = buf_load<R>(tf, of[q], 0);
         }
+        if constexpr (MASK) {
+            const __amdgpu_buffer_rsrc_t tm = rsrc(mp, rows_in, 1);
+#pragma unroll
+            for (int q = 0; q < PASS; ++q) mr[s][q] = (uint8_t)__builtin_amdgcn_raw_buffer_load_b8(tm, (uint32_t)at(q), 0, 0);
+            mp += TT;
+        }
+        ip += (int64_t)TT * ldi;
+        fp += (int64_t)TT * ldf;
+        rows_in -= TT;
     };
     auto gates = [&](int k, auto S) __attribute__((always_inline)) {
         constexpr int s = decltype(S)::value;
-        float fv[PASS], sf[PASS];
-#pragma unroll
-        for (int q = 0; q < PASS; ++q) fv[q] = mmf_to_float(fr[s][q]);
-        mmf_sigmoid_n<PASS>(fv, sf);
+        float iv[PASS], fv[PASS], lbv[PASS], xo[PASS], go[PASS];
 #pragma unroll
         for (int q = 0; q < PASS; ++q) {
-            float xo, go;
-            gate_math<T>(mmf_to_float(ir[s][q]), sf[q], has_lb, lb, xo, go);
-            if (mr[s][q] == 0) xo = 0.0f;
-            gx[k & 1][(q * NP + p) * 64 + lane] = make_float2(go, xo);
+            iv[q] = raw_get<T, R>(ir[s][q]);
+            fv[q] = raw_get<T, R>(fr[s][q]);
+            lbv[q] = lb;
         }
-    };
-    auto put = [&](int k) __attribute__((always_inline)) {
-        T* ot = op + (r0 + (int64_t)k * TT) * a.D;
-        const int n = a.T - k * TT;
+        mmf_gate_n<T, PASS>(iv, fv, lbv, xo, go);
 #pragma unroll
         for (int q = 0; q < PASS; ++q) {
-            const float h = hb[k & 1][(q * NP + p) * 64 + lane];
-            if (at(q) < n && active) ot[(uint32_t)at(q) * (uint32_t)a.D + (uint32_t)d] = mmf_from_float<T>(h);
+            if constexpr (MASK) xo[q] = mr[s][q] == 0 ? 0.0f : xo[q];
+            gx[k & 1][(q * NP + p) * 64 + lane] = make_float2(go[q], xo[q]);
         }
     };
-    load(0, IntC<0>{});
-    load(1, IntC<1>{});
+    float hv[PASS];                                             // outputs on their way from LDS to memory
+    auto fetch = [&](int k) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < PASS; ++q) hv[q] = hb[k & 1][(q * NP + p) * 64 + lane];
+    };
+    auto put = [&](int rows) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t to = rsrc(op, rows, ldo);
+#pragma unroll
+        for (int q = 0; q < PASS; ++q) buf_store<T>(hv[q], to, oo[q], 0);
+    };
+    fetch(0);
+    load(IntC<0>{});
+    load(IntC<1>{});
+    put(0);                                                     // nothing: the count of a turn
     gates(0, IntC<0>{});
-    load(2, IntC<0>{});
+    load(IntC<0>{});
+    put(0);
     lds_only_barrier();
-    auto turn = [&](int k, auto S) __attribute__((always_inline)) {   // wave 0 walks tile k: store tile k - 1, prepare tile k + 1 (set S)
-        if (k > 0) put(k - 1);
-        if (k + 1 < NT) {
-            gates(k + 1, S);
-            load(k + 3, S);
-        }
+    // wave 0 walks tile k: store tile k - 1, whose outputs are read first and arrive under the arithmetic; prepare tile k + 1 (set S)
+    auto turn = [&](int k, auto S) __attribute__((always_inline)) {
+        fetch(k - 1);
+        if (k + 1 < NT) gates(k + 1, S);
+        load(S);
+        put(k > 0 ? rows_out : 0);
+        op += k > 0 ? (int64_t)TT * ldo : 0;
+        rows_out -= k > 0 ? TT : 0;
         lds_only_barrier();
     };
-    for (int k = 0; k < NT; k += 2) {
+    for (int k = 0; k < NT; k += 2) {                           // (an odd number of tiles: one more turn, of nothing but the last store)
         turn(k, IntC<1>{});
-        if (k + 1 < NT) turn(k + 1, IntC<0>{});
+        turn(k + 1, IntC<0>{});
     }
-    put(NT - 1);
+    if (NT % 2 == 0) {
+        fetch(NT - 1);
+        put(rows_out);
+    }
 }
 
-template <typename T>
-int launch_gate_scan(const GateScanArgs& a, int64_t B, hipStream_t s) {
+template <typename T, bool MASK>
+int launch_gate_scan_masked(const GateScanArgs& a, int64_t B, hipStream_t s) {
     const int64_t D = a.D;
     auto grid = [&](int64_t cpw) { return dim3((unsigned)mmf_ceil_div(D, cpw), (unsigned)B); };
     if (B * mmf_ceil_div(D, (int64_t)16) <= 512) {
         // short sequences: half the steps a tile, so that the recurrence starts sooner
-        if (a.T <= 512) hgrn_gate_scan_kernel<T, 16, 1><<<grid(16), 1024, 0, s>>>(a);
-        else hgrn_gate_scan_kernel<T, 16, 2><<<grid(16), 1024, 0, s>>>(a);
-    } else if (B * mmf_ceil_div(D, (int64_t)32) <= 512) hgrn_gate_scan_kernel<T, 32, 2><<<grid(32), 1024, 0, s>>>(a);
-    else hgrn_gate_scan_kernel<T, 64, 2><<<grid(64), 1024, 0, s>>>(a);
+        if (a.T <= 512) hgrn_gate_scan_kernel<T, 16, 1, MASK><<<grid(16), 1024, 0, s>>>(a);
+        else hgrn_gate_scan_kernel<T, 16, 2, MASK><<<grid(16), 1024, 0, s>>>(a);
+    } else if (B * mmf_ceil_div(D, (int64_t)32) <= 512) hgrn_gate_scan_kernel<T, 32, 2, MASK><<<grid(32), 1024, 0, s>>>(a);
+    else hgrn_gate_scan_kernel<T, 64, 2, MASK><<<grid(64), 1024, 0, s>>>(a);
     MMF_CHECK_LAUNCH();
     return 0;
+}
+template <typename T>
+int launch_gate_scan(const GateScanArgs& a, int64_t B, hipStream_t s) {
+    return a.mask ? launch_gate_scan_masked<T, true>(a, B, s) : launch_gate_scan_masked<T, false>(a, B, s);
 }
 
 // One kernel for both forms: STEP = false writes (x, g); STEP = true runs one recurrence step on the
@@ -375,11 +411,9 @@ __global__ __launch_bounds__(256) void hgrn_gate_kernel(const T* __restrict__ i_
     raw4_unpack<T>(fraw, fv);
     if (lb) raw4_unpack<float>(lbraw, lbv);
     if constexpr (STEP) raw4_unpack<float>(straw, stv);
-    float sf[4];
-    mmf_sigmoid_n<4>(fv, sf);
+    mmf_gate_n<T, 4>(iv, fv, lbv, xo, go);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        gate_math<T>(iv[e], sf[e], lb != nullptr, lbv[e], xo[e], go[e]);
         if (!keep) xo[e] = 0.0f;
         if constexpr (STEP) {
             stv[e] = __fadd_rn(__fmul_rn(go[e], stv[e]), xo[e]);
