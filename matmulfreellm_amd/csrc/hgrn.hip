@@ -188,8 +188,9 @@ __global__ __launch_bounds__(64 * NW) void hgrn_recurrent_pipelined_kernel(const
 // ends through resources without records: the compiler then waits for one set of loads by count, where a store or load under a
 // branch made it wait for everything in flight, a trip to memory in every turn.  Wave 0 reads its steps a group ahead into two
 // sets of registers in turn, without copies between them.  bf16 in us, against branches, copies and the exact gate math: 8 x 2048 x 2048
-// 95 -> 63 (201 MB: 3.2 TB/s), 16 x 900 x 1024 42 -> 28, 2 x 1001 x 2048 24 -> 18, 3 x 459 x 2048 16 -> 12, 64 x 32 x 2048 23 -> 18, 4 x 300 x 1024
-// 9.5 -> 7.2, 1 x 77 x 1024 5.1 -> 4.9.
+// 95 -> 63 (201 MB: 3.2 TB/s), 16 x 900 x 1024 42 -> 28, 2 x 1001 x 2048 24 -> 17, 3 x 459 x 2048 16 -> 12, 64 x 32 x 2048 23 -> 17, 4 x 300 x 1024
+// 9.5 -> 7.1, 1 x 77 x 1024 5.1 -> 4.7.  With few columns time is wave 0's own, 12 ns a step (1 x 2048 x 1024 40 -> 28; half as many channels a
+// workgroup: 28).
 struct GateScanArgs {
     const void* i; const void* f;       // rows [B * T, D], row strides ldi, ldf
     const float* lb; const uint8_t* mask;
@@ -229,6 +230,7 @@ __global__ __launch_bounds__(1024) void hgrn_gate_scan_kernel(GateScanArgs a) {
                 const float2* p = src + (j <= TT - U ? j : TT - U) * CPW;
 #pragma unroll
                 for (int u = 0; u < U; ++u) v[u] = p[u * CPW];
+                __builtin_amdgcn_sched_barrier(0);              // in front of the group walked meanwhile, not behind it (2 x 1001: 17.7 -> 16.8 us)
             };
             auto walk = [&](const float2 (&v)[U], int j) __attribute__((always_inline)) {
 #pragma unroll
@@ -252,8 +254,10 @@ __global__ __launch_bounds__(1024) void hgrn_gate_scan_kernel(GateScanArgs a) {
                 for (; j + 2 * U <= n; j += 2 * U) {
                     read(vb, j + U);
                     walk(va, j);
+                    __builtin_amdgcn_sched_barrier(0);
                     read(va, j + 2 * U);
                     walk(vb, j + U);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
                 if (j + U <= n) {                               // what is left of the last tile
                     read(vb, j + U);
