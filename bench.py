@@ -254,9 +254,9 @@ def mfma_bench(dev, m=4096, k=2048, n=11264, iters=20):
         F_.L.check(lib.mmf_bitlinear_mfma_clock_sink(None, 0), "mmf_bitlinear_mfma_clock_sink")
     c = clocks.double().cpu()
     ghz = float((c[:, 0] / c[:, 1].clamp(min=1)).median()) * 0.1
-    # a SIMD holds 2 waves of a workgroup, each issuing (k / 32) steps of 4 MFMAs of 32 pipe cycles per tile; two
+    # a SIMD holds 2 waves of a workgroup, each issuing (k / 64) steps of 16 MFMAs of 16 pipe cycles per tile; two
     # workgroups share a CU when the launch has more than 256 of them
-    busy = (k // 32) * 4 * 32 * 2 * (2 if wgs > 256 else 1) / float(c[:, 0].median())
+    busy = (k // 64) * 16 * 16 * 2 * (2 if wgs > 256 else 1) / float(c[:, 0].median())
     return {"shape": [m, k, n], "contract_ms": round(ms_mm, 4), "quant_prologue_ms": round(ms_q, 4),
             "int8_TOPs": round(tops, 1), "frac_of_5POPs": round(tops / INT8_PEAK_TOPS, 4),
             "shader_clock_GHz_in_kernel": round(ghz, 3), "workgroup_cycles_median": int(c[:, 0].median()),
@@ -264,7 +264,7 @@ def mfma_bench(dev, m=4096, k=2048, n=11264, iters=20):
 
 
 def mfma_pipe_bench(dev, random_operands, steps=512, per_cu=2):
-    """The matrix pipe alone: the tiled kernel's four independent MFMAs per step on register operands, nothing else.
+    """The matrix pipe alone: four independent 32x32x32 MFMAs per step on register operands, nothing else.
     With constant operands the pipe switches little and draws little power; random int8 codes and ternary weights
     are what a contraction feeds it."""
     import matmulfreellm_amd.functional as F_

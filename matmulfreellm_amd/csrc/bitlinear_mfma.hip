@@ -1,4 +1,4 @@
-// Ternary-weight contraction on the int8 matrix cores (v_mfma_i32_32x32x32_i8, gfx950).
+// Ternary-weight contraction on the int8 matrix cores (v_mfma_i32_16x16x64_i8 and v_mfma_i32_32x32x32_i8, gfx950).
 //
 //   out[m, n] = T( fp32( sum_k q[m,k] * t[n,k] ) * deq[m] * wdeq[seg(n)] (+ bias[n]) )
 //
@@ -17,7 +17,7 @@
 //
 // Three kernels, chosen by a measured cost model (dispatch_mfma):
 //   large problems : a workgroup of WGM x WGN waves computes a (WGM*WM*32) x (WGN*WN*32) tile; each
-//                    wave owns WM x WN accumulators of 32x32 (16 VGPRs each); A is staged through
+//                    wave owns WM x WN accumulators of 32x32 (16 VGPRs each, four 16x16x64 blocks); A is staged through
 //                    LDS by DMA in k-blocks of 128, three buffers, one barrier per k-block
 //                    (bitlinear_mfma_dma3_kernel);
 //   small problems : one 32x32 output block per workgroup, 8 waves split K, operands straight
@@ -70,34 +70,53 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
     return (uint32_t)mmf_bits16(ta) | ((uint32_t)mmf_bits16(tb) << 16);
 }
 
-// Epilogue of the tiled kernels.  The MFMAs are issued with the weights as the first operand,
-// so an accumulator holds the TRANSPOSED 32x32 block: register r of lane l is output column
-// n = 8*(r/4) + 4*(l/32) + r%4 and output row m = l%32.  A lane therefore needs one (deq, qsum)
-// pair per block and holds four consecutive columns in registers 4g..4g+3, which pack into one
-// 8-byte piece with no cross-lane traffic.  The wave stages its 32 x (WN*32) outputs in a
+// Where the four groups of four accumulators that a lane holds of a 32 x 32 block lie.  The MFMAs are issued with the weights as
+// the first operand, so a group is four consecutive output COLUMNS of one row, and packs into one 8-byte piece with no
+// cross-lane traffic.
+//   Lay32  one v_mfma_i32_32x32x32_i8 block: group g is column 8 g + 4 (l / 32), row l % 32
+//   Lay16  four v_mfma_i32_16x16x64_i8 blocks, g = 2 * (row half) + (column half): column 16 (g % 2) + 4 (l / 16), row 16 (g / 2) + l % 16
+struct Lay32 {
+    static constexpr int RH = 1;                                 // rows of a lane
+    static __device__ __forceinline__ int row(int lane, int) { return lane & 31; }
+    static __device__ __forceinline__ int col(int lane, int g) { return 8 * g + 4 * (lane >> 5); }
+    static __device__ __forceinline__ constexpr int half(int) { return 0; }
+};
+struct Lay16 {
+    static constexpr int RH = 2;
+    static __device__ __forceinline__ int row(int lane, int g) { return 16 * (g >> 1) + (lane & 15); }
+    static __device__ __forceinline__ int col(int lane, int g) { return 16 * (g & 1) + 4 * (lane >> 4); }
+    static __device__ __forceinline__ constexpr int half(int g) { return g >> 1; }
+};
+struct Acc16 { v4i g[4]; };                                      // a 32 x 32 block in Lay16
+__device__ __forceinline__ int acc_at(const v16i& a, int g, int t) { return a[4 * g + t]; }
+__device__ __forceinline__ int acc_at(const Acc16& a, int g, int t) { return a.g[g][t]; }
+
+// Epilogue of the tiled kernels.  The wave stages its 32 x (WN*32) outputs in a
 // private LDS region and writes them out as aligned 16-byte vectors (128-byte row segments).
 // Per-lane row scales and per-block weight scales of the epilogue, fetched at kernel start so
 // their latency hides behind the whole K loop.
-template <int WM, int WN>
-struct EpiScales { float dq[WM]; int qs[WM]; float wdq[WN]; };
+template <class L, int WM, int WN>
+struct EpiScales { float dq[WM][L::RH]; int qs[WM][L::RH]; float wdq[WN]; };
 
-template <int WM, int WN>
-__device__ __forceinline__ void mfma_prefetch_scales(const MfmaArgs& p, EpiScales<WM, WN>& sc, int lane, int wm,
+template <class L, int WM, int WN>
+__device__ __forceinline__ void mfma_prefetch_scales(const MfmaArgs& p, EpiScales<L, WM, WN>& sc, int lane, int wm,
                                                      int64_t mb0, int64_t nb0) {
     const int64_t NB = (p.N + 31) >> 5;
 #pragma unroll
-    for (int i = 0; i < WM; ++i) {
-        const int64_t m = (mb0 + wm * WM + i) * 32 + (lane & 31);
-        sc.dq[i] = m < p.M ? p.deq[m] : 0.0f;
-        sc.qs[i] = m < p.M ? p.qsum[m] : 0;
-    }
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int h = 0; h < L::RH; ++h) {
+            const int64_t m = (mb0 + wm * WM + i) * 32 + L::row(lane, 2 * h);
+            sc.dq[i][h] = m < p.M ? p.deq[m] : 0.0f;
+            sc.qs[i][h] = m < p.M ? p.qsum[m] : 0;
+        }
 #pragma unroll
     for (int j = 0; j < WN; ++j)   // seg_rows is a multiple of 32: one weight scale per n-block
         sc.wdq[j] = (nb0 + j < NB) ? p.wdeq[(uint32_t)((nb0 + j) * 32) / (uint32_t)p.seg_rows] : 0.0f;
 }
 
-template <typename T, int WM, int WN>
-__device__ __forceinline__ void mfma_epilogue(const MfmaArgs& p, v16i (&acc)[WM][WN], const EpiScales<WM, WN>& sc,
+template <typename T, class L, class A, int WM, int WN>
+__device__ __forceinline__ void mfma_epilogue(const MfmaArgs& p, A (&acc)[WM][WN], const EpiScales<L, WM, WN>& sc,
                                               unsigned char* smem, int lane, int wave, int wm, int64_t mb0, int64_t nb0) {
     const T* bias = static_cast<const T*>(p.bias);
     const T* addend = static_cast<const T*>(p.addend);
@@ -107,22 +126,21 @@ __device__ __forceinline__ void mfma_epilogue(const MfmaArgs& p, v16i (&acc)[WM]
     constexpr int RS = WN * 32 * E + 16;          // LDS row stride of a wave's 32 x (WN*32) staging tile
     constexpr int CPR = WN * 32 * E / 16;         // 16-byte chunks per row
     unsigned char* stage = smem + wave * (32 * RS);
-    const int half = lane >> 5, mloc = lane & 31;
 #pragma unroll
     for (int i = 0; i < WM; ++i) {
         const int64_t mblk = (mb0 + wm * WM + i) * 32;
-        const int64_t m = mblk + mloc;
-        const float dq = sc.dq[i];
-        const int qs = sc.qs[i];
 #pragma unroll
         for (int j = 0; j < WN; ++j)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                const int ncol = j * 32 + 8 * g + 4 * half;          // first of 4 consecutive columns, tile-relative
+                const float dq = sc.dq[i][L::half(g)];
+                const int qs = sc.qs[i][L::half(g)], mloc = L::row(lane, g);
+                const int64_t m = mblk + mloc;
+                const int ncol = j * 32 + L::col(lane, g);           // first of 4 consecutive columns, tile-relative
                 float o[4];
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
-                    o[t] = __fmul_rn(__fmul_rn((float)(acc[i][j][4 * g + t] - qs), dq), wdq[j]);
+                    o[t] = __fmul_rn(__fmul_rn((float)(acc_at(acc[i][j], g, t) - qs), dq), wdq[j]);
                     if (bias) {
                         const int64_t n = nb0 * 32 + ncol + t;
                         o[t] = __fadd_rn(o[t], n < p.N ? mmf_to_float(bias[n]) : 0.0f);
@@ -179,7 +197,7 @@ __device__ __forceinline__ void mfma_epilogue(const MfmaArgs& p, v16i (&acc)[WM]
 // started at -qsum[m], so a value costs one convert and two multiplies; lane-constant parts of the
 // store addresses are computed once; interior tiles skip the bounds tests.
 template <typename T, int WM, int WN>
-__device__ __forceinline__ void mfma_epilogue_fast(const MfmaArgs& p, v16i (&acc)[WM][WN], const EpiScales<WM, WN>& sc,
+__device__ __forceinline__ void mfma_epilogue_fast(const MfmaArgs& p, Acc16 (&acc)[WM][WN], const EpiScales<Lay16, WM, WN>& sc,
                                                    unsigned char* smem, int lane, int wave, int wm, int64_t mb0, int64_t nb0) {
     const T* addend = static_cast<const T*>(p.addend);
     T* out = static_cast<T*>(p.out);
@@ -188,25 +206,24 @@ __device__ __forceinline__ void mfma_epilogue_fast(const MfmaArgs& p, v16i (&acc
     constexpr int CPR = WN * 32 * E / 16;         // 16-byte chunks per row (divides 64)
     constexpr int RPI = 64 / CPR;                 // rows covered by one 64-lane store
     unsigned char* stage = smem + wave * (32 * RS);
-    const int half = lane >> 5, mloc = lane & 31;
     const int cc = lane % CPR, rsub = lane / CPR;
     const int64_t m_first = (mb0 + wm * WM) * 32, n_first = nb0 * 32;
     const bool interior = m_first + WM * 32 <= p.M && n_first + WN * 32 <= p.N;
     const int64_t n = n_first + cc * (16 / E);
     const int64_t lane_off = (m_first + rsub) * p.ldo + n;         // element offset of this lane's first chunk
-    unsigned char* wr = stage + mloc * RS + 4 * half * E;
+    unsigned char* wr = stage + (lane & 15) * RS + 4 * (lane >> 4) * E;
     const unsigned char* rd = stage + rsub * RS + cc * 16;
 #pragma unroll
     for (int i = 0; i < WM; ++i) {
-        const float dq = sc.dq[i];
 #pragma unroll
         for (int j = 0; j < WN; ++j)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
+                const float dq = sc.dq[i][g >> 1];
                 float o[4];
 #pragma unroll
-                for (int t = 0; t < 4; ++t) o[t] = __fmul_rn(__fmul_rn((float)acc[i][j][4 * g + t], dq), sc.wdq[j]);
-                unsigned char* w = wr + (j * 32 + 8 * g) * E;
+                for (int t = 0; t < 4; ++t) o[t] = __fmul_rn(__fmul_rn((float)acc_at(acc[i][j], g, t), dq), sc.wdq[j]);
+                unsigned char* w = wr + (g >> 1) * 16 * RS + (j * 32 + 16 * (g & 1)) * E;
                 if constexpr (E == 2) *reinterpret_cast<uint2*>(w) = make_uint2(pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3]));
                 else *reinterpret_cast<float4*>(w) = make_float4(o[0], o[1], o[2], o[3]);
             }
@@ -243,7 +260,7 @@ __device__ __forceinline__ void mfma_epilogue_fast(const MfmaArgs& p, v16i (&acc
 // launch took beyond the plain one: 16384 x 2048 -> 11264 in bf16 356 us with the exact exp and divide, 322 with mmf_swiglu_n (the plain
 // contraction of as many columns about 300); 2002 rows 57 and 54; fp16, whose elements fall back eight times as often, 1377 rows 36.8 and 36.3.
 template <typename T, int WM>
-__device__ __forceinline__ void mfma_epilogue_swiglu(const MfmaArgs& p, v16i (&acc)[WM][2], const EpiScales<WM, 2>& sc,
+__device__ __forceinline__ void mfma_epilogue_swiglu(const MfmaArgs& p, Acc16 (&acc)[WM][2], const EpiScales<Lay16, WM, 2>& sc,
                                                      unsigned char* smem, int lane, int wave, int wm, int64_t mb0, int64_t nbg) {
     T* out = static_cast<T*>(p.out);
     constexpr int E = sizeof(T);
@@ -251,28 +268,27 @@ __device__ __forceinline__ void mfma_epilogue_swiglu(const MfmaArgs& p, v16i (&a
     constexpr int CPR = 32 * E / 16;              // 16-byte chunks per row
     constexpr int RPI = 64 / CPR;                 // rows covered by one 64-lane store
     unsigned char* stage = smem + wave * (32 * RS);
-    const int half = lane >> 5, mloc = lane & 31;
     const int cc = lane % CPR, rsub = lane / CPR;
     const int64_t nseg = p.N >> 1;
     const int64_t m_first = (mb0 + wm * WM) * 32, n_first = nbg * 32;
     const bool interior = m_first + WM * 32 <= p.M && n_first + 32 <= nseg;
     const int64_t n = n_first + cc * (16 / E);
     const int64_t lane_off = (m_first + rsub) * p.ldo + n;
-    unsigned char* wr = stage + mloc * RS + 4 * half * E;
+    unsigned char* wr = stage + (lane & 15) * RS + 4 * (lane >> 4) * E;
     const unsigned char* rd = stage + rsub * RS + cc * 16;
 #pragma unroll
     for (int i = 0; i < WM; ++i) {
-        const float dq = sc.dq[i];
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
+            const float dq = sc.dq[i][g >> 1];
             float gv[4], uv[4], o[4];
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                gv[t] = mmf_round_to<T>(__fmul_rn(__fmul_rn((float)acc[i][0][4 * g + t], dq), sc.wdq[0]));
-                uv[t] = mmf_round_to<T>(__fmul_rn(__fmul_rn((float)acc[i][1][4 * g + t], dq), sc.wdq[1]));
+                gv[t] = mmf_round_to<T>(__fmul_rn(__fmul_rn((float)acc_at(acc[i][0], g, t), dq), sc.wdq[0]));
+                uv[t] = mmf_round_to<T>(__fmul_rn(__fmul_rn((float)acc_at(acc[i][1], g, t), dq), sc.wdq[1]));
             }
             mmf_swiglu_n<T, 4>(gv, uv, o);
-            unsigned char* w = wr + (8 * g) * E;
+            unsigned char* w = wr + (g >> 1) * 16 * RS + 16 * (g & 1) * E;
             if constexpr (E == 2) *reinterpret_cast<uint2*>(w) = make_uint2(pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3]));
             else *reinterpret_cast<float4*>(w) = make_float4(o[0], o[1], o[2], o[3]);
         }
@@ -314,8 +330,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) void bitlinear_mfma_kernel(MfmaArgs
     const int64_t MB = (p.M + 31) >> 5, NB = (p.N + 31) >> 5;
     const int64_t KB = p.Kp >> 7, KG = p.Kp >> 4;
     const int64_t mb0 = tile_m * BMB, nb0 = tile_n * BNB + wn * WN;
-    EpiScales<WM, WN> sc;
-    mfma_prefetch_scales<WM, WN>(p, sc, lane, wm, mb0, nb0);
+    EpiScales<Lay32, WM, WN> sc;
+    mfma_prefetch_scales<Lay32, WM, WN>(p, sc, lane, wm, mb0, nb0);
 
     v16i acc[WM][WN];
 #pragma unroll
@@ -406,11 +422,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) void bitlinear_mfma_kernel(MfmaArgs
         __syncthreads();
     }
 
-    mfma_epilogue<T, WM, WN>(p, acc, sc, smem, lane, wave, wm, mb0, nb0);
+    mfma_epilogue<T, Lay32>(p, acc, sc, smem, lane, wave, wm, mb0, nb0);
 }
-
-typedef __attribute__((address_space(3))) void* mmf_lds_ptr;
-typedef __attribute__((address_space(1))) const void* mmf_glb_ptr;
 
 // One 1 KiB wave-load global -> LDS (16 bytes per lane; lane l lands at lds + 16 l) from `base` (wave-uniform) + 16 l.
 // Written in assembly so that the compiler does not know of an LDS write in flight: it answers the builtin with waits
@@ -422,6 +435,21 @@ __device__ __forceinline__ void mfma_dma_1k(const void* base, uint32_t lane16, c
     const uint64_t b = (uint64_t)base;
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(l), "v"(lane16), "s"(b) : "memory");
 }
+// acc += b x a on a 16 x 16 block over 64 inputs, in place.  (From the builtin the compiler gives every product a destination of its own
+// and the 16 four-register accumulators wander through the registers until some are spilled.)  What the compiler would see to for
+// the builtin: the two wait states behind the vector operations that wrote b (FRESH: its first use); before anything else reads the
+// accumulators, mfma_done().
+template <bool FRESH>
+__device__ __forceinline__ void mfma_16x16x64(v4i& acc, const v4i& b, const v4i& a) {
+    if constexpr (FRESH) asm volatile("s_nop 1\n\tv_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+v"(acc) : "v"(b), "v"(a));
+    else asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+v"(acc) : "v"(b), "v"(a));
+}
+template <int WM, int WN>
+__device__ __forceinline__ void mfma_done(Acc16 (&acc)[WM][WN]) {
+    asm volatile("s_nop 15\n\ts_nop 15");
+#pragma unroll
+    for (int t = 0; t < WM * WN * 4; ++t) asm volatile("" : "+v"(acc[t / (WN * 4)][t / 4 % WN].g[t & 3]));   // no reader moves in front of the wait
+}
 // Workgroup barrier behind an explicit wait: at most `VM` vector-memory operations may stay in flight, LDS traffic done.
 // Only VM = 0 says anything about a transfer into LDS: such transfers and ordinary loads complete in no fixed order.
 template <int VM>
@@ -430,12 +458,21 @@ __device__ __forceinline__ void mfma_barrier_vm() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(VM) : "memory");
 }
 
+// LDS of the large-M kernel: three activation buffers, the exchange of partial sums or the epilogue's staging area, whichever is largest; behind
+// them the rows' scales and code sums (registers held through the k-loop otherwise).
+template <typename T, int WGM, int WGN, int WM, int WN, int KS, bool SWI>
+constexpr int dma3_work_bytes() {
+    constexpr int waves = WGM * WGN * KS, a = 3 * WGM * WM * 4096 * KS, e = waves * 32 * ((SWI ? 1 : WN) * 32 * (int)sizeof(T) + 16),
+                  x = KS > 1 ? waves * (KS - 1) * WN * 4096 : 0;
+    return a > e ? (a > x ? a : x) : (e > x ? e : x);
+}
+
 // ------------------------------------------------------------------------------------------
 // The large-M kernel.  Same tiling, but A goes global -> LDS by DMA (global_load_lds_dwordx4:
 // lane l's 16 bytes land at the wave-uniform LDS base + 16*l, which is exactly the
 // fragment-tiled layout), so no VGPRs stage it and no ds_write sits in the instruction stream.
 // Three A buffers of one 128-wide k-block each and ONE barrier per k-block,
-// placed after the second of its four k-steps.  At that barrier every wave has left the previous
+// placed between its two k-steps of 64.  At that barrier every wave has left the previous
 // k-block, so its buffer is free for the DMA of k-block s+2, and k-block s+1 (issued one k-block
 // earlier, waited for by each wave just before the barrier, together with the packed weights
 // requested with it) is complete for everybody.  K-block
@@ -447,6 +484,12 @@ __device__ __forceinline__ void mfma_barrier_vm() {
 // KS > 1: the workgroup's waves form KS groups that take every KS-th k-block of the same (KS times narrower) tile: a mid-sized
 // problem then has KS times as many tiles at the same work per wave, and each wave's chain is KS times shorter.  The groups
 // exchange partial sums through LDS at the end (integers: exact), each finishing its share of the wave tile.
+// What bounds it: on many tiles the power that the matrix cores draw on real codes.  On register operands v_mfma_i32_32x32x32_i8 reaches
+// 3.6 P op/s before the clock gives way, v_mfma_i32_16x16x64_i8 4.8, which is why the products are of the second form although there are twice as
+// many of them.  Measured with 32x32x32, then with
+// 16x16x64, us: 16384 x 2048 -> 6144 204 and 172-180 (2.4 P op/s), x 5632 -> 2048 147 and 126-130 (3.0), x 2048 -> 11264 with swiglu 363-369 and
+// 316-325; 4096 x 2048 -> 11264 83 and 73, 2002 rows 44 and 40.  On at most one tile per CU what counts is each wave's chain of instructions: there both
+// forms take the same time within 5 % (5632 -> 2048 split: 2002 rows 24 and 23.4, 1377 rows 21.4 and 21.8).
 template <typename T, int WGM, int WGN, int WM, int WN, int KS, bool FAST, bool SWI = false>
 __global__ __launch_bounds__(64 * WGM * WGN * KS, (WM * WN <= 4 ? 4 : 1))   // small wave tiles: 4 waves per SIMD = two workgroups per CU
 void bitlinear_mfma_dma3_kernel(MfmaArgs p) {
@@ -469,19 +512,19 @@ void bitlinear_mfma_dma3_kernel(MfmaArgs p) {
     // XCD x owns rows [x * RB, (x + 1) * RB) and walks the columns with the rows running fastest: the RB workgroups that
     // share a weight tile run together, and the RB activation panels (sized by the host to stay in that XCD's L2) are
     // re-read from L2 for every column.  Bands follow one another.
-    int64_t wg = blockIdx.x;
-    const int64_t total = (int64_t)p.tiles_m * p.tiles_n;
+    uint32_t wg = blockIdx.x;                                     // 32 bits: a 64-bit division is 200 scalar instructions in front of the first load
+    const uint32_t total = gridDim.x, tiles_n = (uint32_t)p.tiles_n;
     int64_t tile_m, tile_n;
     if (p.rows_per_xcd > 0) {
-        const int RB = p.rows_per_xcd, x = (int)(wg & 7);
-        const int64_t l = wg >> 3, per_band = (int64_t)RB * p.tiles_n;
-        const int64_t band = l / per_band, l2 = l % per_band;
+        const uint32_t RB = (uint32_t)p.rows_per_xcd, x = wg & 7;
+        const uint32_t l = wg >> 3, per_band = RB * tiles_n;
+        const uint32_t band = l / per_band, l2 = l % per_band;
         tile_m = band * 8 * RB + x * RB + l2 % RB;
         tile_n = l2 / RB;
     } else {
         if (total % 8 == 0) wg = (wg % 8) * (total / 8) + wg / 8;
-        tile_m = wg / p.tiles_n;
-        tile_n = wg % p.tiles_n;
+        tile_m = wg / tiles_n;
+        tile_n = wg % tiles_n;
     }
     const int64_t MB = (p.M + 31) >> 5, NB = (p.N + 31) >> 5;
     const int KB = (int)(p.Kp >> 7), KBs = KB / KS;               // k-blocks of the row, steps (the launcher: KB % KS == 0)
@@ -495,12 +538,19 @@ void bitlinear_mfma_dma3_kernel(MfmaArgs p) {
         else return nb0 + j < NB ? nb0 + j : NB - 1;
     };
     if constexpr (!SWI) mfma_select_segment(p, tile_n * BNB);
-    EpiScales<WM, WN> sc;
-    mfma_prefetch_scales<WM, WN>(p, sc, lane, wm, mb0, nb0);
-    if constexpr (SWI) {
-#pragma unroll
-        for (int j = 0; j < WN; ++j) sc.wdq[j] = p.wdeq[(uint32_t)(nblock(j) * 32) / (uint32_t)p.seg_rows];
+    float* const row_dq = reinterpret_cast<float*>(smem + dma3_work_bytes<T, WGM, WGN, WM, WN, KS, SWI>());
+    int* const row_qs = reinterpret_cast<int*>(row_dq + BMB * 32);
+    static_assert(BMB * 32 <= 64 * NW, "a row's scale and code sum per thread");
+    float my_dq = 0.0f;                            // on their way while the first transfers are requested; into LDS behind the first wait
+    int my_qs = 0;
+    if (const int64_t m = mb0 * 32 + threadIdx.x; threadIdx.x < BMB * 32 && m < p.M) {
+        my_dq = p.deq[m];
+        my_qs = p.qsum[m];
     }
+    EpiScales<Lay16, WM, WN> sc;
+#pragma unroll
+    for (int j = 0; j < WN; ++j)   // seg_rows is a multiple of 32: one weight scale per n-block
+        sc.wdq[j] = p.wdeq[(uint32_t)(nblock(j) * 32) / (uint32_t)p.seg_rows];
 
     auto dma_block = [&](int kb, int boff) {                      // k-block kb -> buffer at byte offset boff
 #pragma unroll
@@ -514,6 +564,7 @@ void bitlinear_mfma_dma3_kernel(MfmaArgs p) {
             mfma_dma_1k(g, (uint32_t)lane * 16u, smem + boff + w * 1024);
         }
     };
+    const uint32_t boff = (uint32_t)(((lane >> 4) & 1) * 32 + (lane >> 5) * 16 + (lane & 15)) * 16u;
     auto load_b = [&](int kb, uint4 (&dst)[WN]) {                 // unconditional: the barrier's vmcnt counts on WN loads
 #pragma unroll
         for (int j = 0; j < WN; ++j) {
@@ -522,18 +573,27 @@ void bitlinear_mfma_dma3_kernel(MfmaArgs p) {
             // wave-uniform block address + a 32-bit lane offset: the load then takes its base from scalar registers and
             // no 64-bit per-lane address is kept alive
             const unsigned char* blk = reinterpret_cast<const unsigned char*>(p.b + (nb * KB + kbc) * 64);
-            dst[j] = *reinterpret_cast<const uint4*>(blk + (uint32_t)(lane * 16));
+            dst[j] = *reinterpret_cast<const uint4*>(blk + boff);
         }
     };
-    auto expand_b = [&](const uint4 (&src)[WN], int ks, v4i (&bf)[WN]) {
+    // A loaded set as operands.  Lane l loaded the dwords of weight row 16 (l / 32) + l % 16, k-half (l / 16) % 2; exchanging the upper half of the
+    // lanes of the first dword with the lower half of the second leaves rows 0-15 in x and rows 16-31 in y, the lanes' fourths on
+    // inputs 0-15, 16-31, 32-47, 48-63 of the k-block; z and w the same of its second half.
+    auto arrange_b = [&](uint4 (&s)[WN]) {
 #pragma unroll
         for (int j = 0; j < WN; ++j) {
-            const uint32_t w = ks == 0 ? src[j].x : ks == 1 ? src[j].y : ks == 2 ? src[j].z : src[j].w;
-            bf[j][0] = (int)(w & 0x03030303u);
-            bf[j][1] = (int)((w >> 2) & 0x03030303u);
-            bf[j][2] = (int)((w >> 4) & 0x03030303u);
-            bf[j][3] = (int)((w >> 6) & 0x03030303u);
+            const auto lo = __builtin_amdgcn_permlane32_swap(s[j].x, s[j].y, false, false);
+            const auto hi = __builtin_amdgcn_permlane32_swap(s[j].z, s[j].w, false, false);
+            s[j] = make_uint4(lo[0], lo[1], hi[0], hi[1]);
         }
+    };
+    auto expand = [](uint32_t w) {
+        v4i b;
+        b[0] = (int)(w & 0x03030303u);
+        b[1] = (int)((w >> 2) & 0x03030303u);
+        b[2] = (int)((w >> 4) & 0x03030303u);
+        b[3] = (int)((w >> 6) & 0x03030303u);
+        return b;
     };
 
     // B is requested a k-block and a half before its first use, into a ring of three register sets.  The ring is walked
@@ -546,86 +606,108 @@ void bitlinear_mfma_dma3_kernel(MfmaArgs p) {
     load_b(0, bset0);
     load_b(1, bset1);
     __builtin_amdgcn_s_waitcnt(0x0F70);            // vmcnt(0): this wave's pieces of k-blocks 0 and 1 have landed
+    if (threadIdx.x < BMB * 32) {
+        row_dq[threadIdx.x] = my_dq;
+        row_qs[threadIdx.x] = my_qs;
+    }
     __syncthreads();
 
-    // a lane's 16 accumulator registers of one tile all belong to output row (lane % 32)
-    v16i acc[WM][WN];
-#pragma unroll
-    for (int i = 0; i < WM; ++i) {
-        const int init = FAST && wk == 0 ? -sc.qs[i] : 0;
-#pragma unroll
-        for (int j = 0; j < WN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = init;
-    }
-    const int aoff = (wk * BMB + wm * WM) * CH + lane * 16;
-    int cur = 0, nxt = BUF, fre = 2 * BUF;         // byte offsets of the buffers of k-blocks s, s+1, s+2
-    v4i af[2][WM];
-#pragma unroll
-    for (int i = 0; i < WM; ++i) af[0][i] = *reinterpret_cast<const v4i*>(smem + cur + aoff + i * CH);
+    arrange_b(bset0);
 
-    // one k-block: contracts with the set `bcur`, requests k-block kb + 2 into `bfar`; the expansion of the NEXT step's
-    // weights (the first step of `bnxt` at the end) is interleaved with this step's MFMAs
-    v4i bf[WN];
-    expand_b(bset0, 0, bf);
-    auto kblock = [&](int kb, const uint4 (&bcur)[WN], const uint4 (&bnxt)[WN], uint4 (&bfar)[WN]) {
+    // FAST: a lane's accumulators start at -qsum of their row (read for every group and masked: as a choice the compiler branches around
+    // a read of its own for each of the accumulators, 2 us of a launch)
+    Acc16 acc[WM][WN];
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            if (ks == 2) {
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int init = FAST ? -row_qs[(wm * WM + i) * 32 + Lay16::row(lane, g)] & (KS == 1 || wk == 0 ? -1 : 0) : 0;
+#pragma unroll
+            for (int j = 0; j < WN; ++j)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) acc[i][j].g[g][t] = init;
+        }
+    // A 16 x 64 fragment: lane l reads input group l / 16 of row l % 16
+    const int aoff = (wk * BMB + wm * WM) * CH + (lane >> 4) * 512 + (lane & 15) * 16;
+    int cur = 0, nxt = BUF, fre = 2 * BUF;         // byte offsets of the buffers of k-blocks s, s+1, s+2
+    constexpr int MF = 2 * WM, NF = 2 * WN;        // 16-row and 16-column fragments of the wave tile
+    auto read_a = [&](int off, int f) { return *reinterpret_cast<const v4i*>(smem + off + aoff + (f >> 1) * CH + (f & 1) * 256); };
+    // word of the arranged set for step q of its k-block, column fragment c
+    auto word = [](const uint4 (&s)[WN], int q, int c) {
+        const uint4 w = s[c >> 1];
+        return q == 0 ? ((c & 1) == 0 ? w.x : w.y) : (c & 1) == 0 ? w.z : w.w;
+    };
+    v4i af[2], bf[NF];
+    af[0] = read_a(cur, 0);
+#pragma unroll
+    for (int c = 0; c < NF; ++c) bf[c] = expand(word(bset0, 0, c));
+
+    // One k-block in two steps of 64: contracts with the set `bcur`, requests k-block kb + 2 into `bfar`.  Activation rows outermost, the next
+    // row's fragment on its way from LDS under this row's MFMAs; under the last row every weight fragment is replaced by the next step's
+    // as soon as its MFMA has been issued.  (A step's weights and two row fragments: 24 registers, which is what 64 accumulators, three
+    // sets in flight and addresses leave of 128.  Columns outermost, two more weight fragments expanded a row earlier, or four and eight row fragments
+    // ahead, where one workgroup per CU leaves the registers, all measured the same or slower.)
+    auto kblock = [&](int kb, const uint4 (&bcur)[WN], uint4 (&bnxt)[WN], uint4 (&bfar)[WN]) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            if (q == 1) {
                 // Everything requested one k-block ago -- this wave's pieces of A k-block kb+1 and the weights of kb+1 --
                 // has to be here now.  The wait is for ALL vector-memory traffic: a transfer into LDS and an ordinary load
                 // do not complete in the order they were issued (a count that leaves the younger weight loads in flight let
-                // warm weight loads overtake a cold A transfer and gave wrong sums), so the next requests go out right
-                // behind the barrier and have a whole k-block to land.
+                // warm weight loads overtake a cold A transfer and gave wrong sums), so the next requests go out after
+                // the barrier, between the rows' MFMAs (ahead of them all waves' address arithmetic left the matrix pipe idle: 0.64 us a k-block
+                // with one workgroup per CU, 0.61 so), and have the rest of the k-block and half the next to land.  The weights that have
+                // come in are arranged ahead of them: the compiler waits for them by a count that does not know of the transfer, which behind it
+                // would be a wait for the transfer.
                 mfma_barrier_vm<0>();
-                dma_block(kb + 2, fre);
-                load_b(kb + 2, bfar);
             }
-            const unsigned char* nsrc = ks < 3 ? smem + cur + aoff + (ks + 1) * 1024 : smem + nxt + aoff;
-#pragma unroll
-            for (int i = 0; i < WM; ++i) af[(ks + 1) & 1][i] = *reinterpret_cast<const v4i*>(nsrc + i * CH);
-            // weight columns outermost: once the MFMAs of column j are issued, the next step's expansion of column j can
-            // reuse its registers and runs in the shadow of the matrix pipe
-            v4i bn[WN];
-#pragma unroll
-            for (int j = 0; j < WN; ++j) {
-#pragma unroll
-                for (int i = 0; i < WM; ++i)
-                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf[j], af[ks & 1][i], acc[i][j], 0, 0, 0);
-                const uint32_t w = ks == 0 ? bcur[j].y : ks == 1 ? bcur[j].z : ks == 2 ? bcur[j].w : bnxt[j].x;
-                bn[j][0] = (int)(w & 0x03030303u);
-                bn[j][1] = (int)((w >> 2) & 0x03030303u);
-                bn[j][2] = (int)((w >> 4) & 0x03030303u);
-                bn[j][3] = (int)((w >> 6) & 0x03030303u);
-            }
-            __builtin_amdgcn_sched_group_barrier(0x100, WM, 0);
-#pragma unroll
-            for (int j = 0; j < WN; ++j) {
-                __builtin_amdgcn_sched_group_barrier(0x008, WM, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);
-            }
-#pragma unroll
-            for (int j = 0; j < WN; ++j) bf[j] = bn[j];
             __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int f = 0; f < MF; ++f) {
+                const int t = q * MF + f + 1;                      // of the 2 MF fragments of this k-block, then the next one's first
+                af[t & 1] = t < 2 * MF ? read_a(cur + t / MF * 2048, t % MF) : read_a(nxt, 0);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int c = 0; c < NF; ++c) {
+                    v4i& d = acc[f >> 1][c >> 1].g[2 * (f & 1) + (c & 1)];
+                    if (f == 0 && c == 0) mfma_16x16x64<true>(d, bf[c], af[f & 1]);
+                    else mfma_16x16x64<false>(d, bf[c], af[f & 1]);
+                    if (f == MF - 1) bf[c] = expand(q == 0 ? word(bcur, 1, c) : word(bnxt, 0, c));
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (q == 1) {
+                    if (f == 0) arrange_b(bnxt);
+                    if (f == 1 || MF == 1) dma_block(kb + 2, fre);
+                    if (f == (MF > 2 ? 2 : MF - 1)) load_b(kb + 2, bfar);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
         }
         const int t = cur; cur = nxt; nxt = fre; fre = t;
     };
     int kb = 0;
-    for (; kb + 3 <= KBs; kb += 3) {
+    for (;;) {                                     // left in the middle: no copy of a k-block for the remainder, whose code a launch would fetch cold
         kblock(kb, bset0, bset1, bset2);
-        kblock(kb + 1, bset1, bset2, bset0);
-        kblock(kb + 2, bset2, bset0, bset1);
+        if (++kb >= KBs) break;
+        kblock(kb, bset1, bset2, bset0);
+        if (++kb >= KBs) break;
+        kblock(kb, bset2, bset0, bset1);
+        if (++kb >= KBs) break;
     }
-    if (kb < KBs) {
-        kblock(kb, bset0, bset1, bset2);
-        if (kb + 1 < KBs) kblock(kb + 1, bset1, bset2, bset0);
-    }
+    mfma_done(acc);
     __builtin_amdgcn_s_waitcnt(0x0F70);            // the trailing DMA must not land in the epilogue's staging area
     __syncthreads();
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            sc.dq[i][h] = row_dq[(wm * WM + i) * 32 + Lay16::row(lane, 2 * h)];
+            sc.qs[i][h] = FAST ? 0 : row_qs[(wm * WM + i) * 32 + Lay16::row(lane, 2 * h)];
+        }
     if constexpr (KS == 1) {
         if constexpr (SWI) mfma_epilogue_swiglu<T, WM>(p, acc, sc, smem, lane, wave, wm, mb0, nb0);
         else if constexpr (FAST) mfma_epilogue_fast<T, WM, WN>(p, acc, sc, smem, lane, wave, wm, mb0, nb0);
-        else mfma_epilogue<T, WM, WN>(p, acc, sc, smem, lane, wave, wm, mb0, nb0);
+        else mfma_epilogue<T, Lay16>(p, acc, sc, smem, lane, wave, wm, mb0, nb0);
     } else {
         // group g finishes row block g of the wave tile: it takes the other groups' partial sums of that block
         static_assert(KS == WM, "a row block of the wave tile per group");
@@ -638,17 +720,20 @@ void bitlinear_mfma_dma3_kernel(MfmaArgs p) {
 #pragma unroll
                 for (int j = 0; j < WN; ++j)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) dst[(j * 16 + r) * 64] = acc[i][j][r];
+                    for (int r = 0; r < 16; ++r) dst[(j * 16 + r) * 64] = acc[i][j].g[r >> 2][r & 3];
             }
         }
         __syncthreads();
-        v16i mine[1][WN];
-        EpiScales<1, WN> sc1;
+        Acc16 mine[1][WN];
+        EpiScales<Lay16, 1, WN> sc1;
 #pragma unroll
         for (int i = 0; i < WM; ++i) {
             if (i == wk) {
-                sc1.dq[0] = sc.dq[i];
-                sc1.qs[0] = sc.qs[i];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    sc1.dq[0][h] = sc.dq[i][h];
+                    sc1.qs[0][h] = sc.qs[i][h];
+                }
 #pragma unroll
                 for (int j = 0; j < WN; ++j) mine[0][j] = acc[i][j];
             }
@@ -662,14 +747,14 @@ void bitlinear_mfma_dma3_kernel(MfmaArgs p) {
 #pragma unroll
                 for (int j = 0; j < WN; ++j)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) mine[0][j][r] += src[(j * 16 + r) * 64];
+                    for (int r = 0; r < 16; ++r) mine[0][j].g[r >> 2][r & 3] += src[(j * 16 + r) * 64];
             }
         }
         __syncthreads();                                         // the exchange area becomes the epilogue's staging area
         const int wm1 = wm * WM + wk;
         if constexpr (SWI) mfma_epilogue_swiglu<T, 1>(p, mine, sc1, smem, lane, wave, wm1, mb0, nb0);
         else if constexpr (FAST) mfma_epilogue_fast<T, 1, WN>(p, mine, sc1, smem, lane, wave, wm1, mb0, nb0);
-        else mfma_epilogue<T, 1, WN>(p, mine, sc1, smem, lane, wave, wm1, mb0, nb0);
+        else mfma_epilogue<T, Lay16>(p, mine, sc1, smem, lane, wave, wm1, mb0, nb0);
     }
     if (p.clocks && threadIdx.x == 0 && (int64_t)blockIdx.x < p.clock_cap) {
         p.clocks[2 * blockIdx.x] = __builtin_amdgcn_s_memtime() - clk0;
@@ -700,12 +785,8 @@ int launch_mfma_dma3(MfmaArgs a, hipStream_t s) {
     a.tiles_m = (int)mmf_ceil_div(a.M, BM);
     a.tiles_n = SWI ? (int)mmf_ceil_div(a.N / 2, BN / 2) : (int)mmf_ceil_div(a.N, BN);
     a.rows_per_xcd = mfma_rows_per_xcd(a.tiles_m, BM, a.Kp);
-    size_t lds = 3u * (WGM * WM) * 4096u * KS;
     constexpr int waves = WGM * WGN * KS;
-    const size_t lds_epi = (size_t)waves * 32u * ((SWI ? 1 : WN) * 32u * sizeof(T) + 16u);
-    const size_t lds_ex = KS > 1 ? (size_t)waves * (KS - 1) * WN * 4096u : 0;
-    if (lds_epi > lds) lds = lds_epi;
-    if (lds_ex > lds) lds = lds_ex;
+    constexpr size_t lds = dma3_work_bytes<T, WGM, WGN, WM, WN, KS, SWI>() + BM * 8;
     const int per_vec = 16 / (int)sizeof(T);
     a.vec_store = SWI || ((a.N % per_vec == 0) && (a.ldo % per_vec == 0) && ((reinterpret_cast<uintptr_t>(a.out) & 15u) == 0) &&
                           ((reinterpret_cast<uintptr_t>(a.addend) & 15u) == 0));
@@ -890,29 +971,30 @@ int launch_mfma(MfmaArgs a, hipStream_t s) {
     return 0;
 }
 
-// Which kernel is the fastest, from its measured time on MI355X (us; N from 1024 to 11264, K from 1024 to 9216, M from 77 to 11500):
+// Which kernel is the fastest, from its measured time on MI355X (us; N from 1024 to 11264, K from 1024 to 9216, M from 77 to 9600):
 //   weight stream  3 + 0.7 ns per output block + 0.18 ns per output block and k-block, as long as the row fits its LDS;
-//   split tiles    (64 x 256, two groups of waves on every second k-block) one round of at most one tile per CU: a chain of
-//                  0.29 us per k-block, and what a fuller chip adds.  Beyond one round, 3.4 + 0.345 us per k-block for each;
-//   tiles          (64 x 512) 4 + 0.6 us per k-block and round.
-// A whole tile is worth two split ones, so against an even number of split rounds whole tiles win or tie (by 0 to 50 %, least on the longest
-// rows).  Where two rounds of whole tiles would leave the second less than half full, three split rounds do instead of four.  Split against
-// whole at 513 to 768 split tiles: 8 k-blocks (1024 -> 5632, 2099 rows) 21.2 / 19.3, (1024 -> 1024, 8448) 18.2 / 17.9; 12 (1536 -> 3072,
-// 2995) 23.7 / 23.0; 14, where the line lies, 0.96 to 1.05; 16 (2048 -> 6144, 1395) 26.3 / 27.7, (2048 -> 2048, 5107) 26.5 / 28.2,
-// (2048 -> 11264, 960) 27.3 / 28.1; 20 (2560 -> 7680, 1203) 30.7 / 32.6; 22 (2816 -> 1024, 9600) 33.0 / 35.3; 44 (5632 -> 2048, 4467)
-// 55.7 / 61.2.  Five split rounds for three of whole tiles: 42.3 / 42.5 at 16 k-blocks, 94 / 100 at 44 (left to whole tiles), 148 / 159 at
-// 72 (taken).
-// 2002 x 5632 -> 2048: stream 37 us, split 23, tiles 31; 1377 x 2048 -> 2048: 12.2 / 10.5 / 14.3.
+//   split tiles    (64 x 256, two groups of waves on every second k-block) at most one tile per CU: a chain of 0.31 us per k-block, and
+//                  what a fuller chip adds.  At most two per CU run side by side and share it: one time, whatever their number.  Beyond
+//                  that, 3.9 + 0.295 us per k-block for every 256;
+//   tiles          (64 x 512) at most one per CU: 4.4 + 0.58 us per k-block and what a fuller chip adds; beyond, 4.4 + 0.62 per 256.
+// A whole tile is worth two split ones, so against an even number of split rounds whole tiles win or tie, but for two rounds of long rows,
+// and where the last round of whole tiles would be less than half full, an odd number of split rounds does instead.  Split against whole:
+// 5632 -> 2048 (44 k-blocks), 2002 rows (256 split tiles) 23.4 / 33.8, 3600 (456) 34.6 / 38.8, 9600 82.1 / 87.2; 6912 -> 2560 (54), 2300 rows
+// 39.7 / 43.3, 6500 86.5 / 77.4; 2048 -> 2048 (16), 2002 rows 12.2 / 15.1, 3600 18.0 / 18.5; 2048 -> 6144, 2002 rows (768) 27.1 / 26.4.  Stream against split:
+// 1024 -> 5632, 300 rows 6.0 / 8.4, 700 9.9 / 9.4; 2048 -> 2048, 1203 rows 10.9 / 11.4, 1395 12.1 / 11.3.
+// Over the 240 shapes of that sweep the choice costs 0.2 % against the best of the three on average, 19 % at most (460 x 1024 -> 5632: 1.4 us).
 enum class MfmaPick { kStream, kSplit, kTiles };
 inline MfmaPick mfma_pick(const MfmaArgs& a) {
     const int64_t KB = a.Kp >> 7;
     const double kb = (double)KB, blocks = (double)mmf_ceil_div(a.M, 32) * (double)mmf_ceil_div(a.N, 32);
     const int64_t half = mmf_ceil_div(a.M, 64) * mmf_ceil_div(a.N, 256), full = mmf_ceil_div(a.M, 64) * mmf_ceil_div(a.N, 512);
     const double t_stream = 3.0 + blocks * (0.0007 + 0.00018 * (double)((KB + 7) / 8 * 8));
-    const double t_tiles = (double)mmf_ceil_div(full, 256) * (4.0 + 0.6 * kb);
+    const double t_tiles = full <= 256 ? 4.4 + 0.58 * kb + (double)full / 256.0 * (1.0 + 0.18 * kb) : (double)mmf_ceil_div(full, 256) * (4.4 + 0.62 * kb);
     double t_split = 1e30;
     if (KB % 2 == 0)
-        t_split = half <= 256 ? 4.4 + 0.29 * kb + (double)half / 256.0 * (1.0 + 0.1 * kb) : (double)mmf_ceil_div(half, 256) * (3.4 + 0.345 * kb);
+        t_split = half <= 256   ? 5.2 + 0.31 * kb + (double)half / 256.0 * (0.75 + 0.107 * kb)
+                  : half <= 512 ? 8.5 + 0.59 * kb
+                                : (double)mmf_ceil_div(half, 256) * (3.9 + 0.295 * kb);
     if (a.Kp <= 8192 && a.M <= 65535 * 32 && (a.M <= 64 || (t_stream <= t_split && t_stream <= t_tiles))) return MfmaPick::kStream;
     return t_split < t_tiles ? MfmaPick::kSplit : MfmaPick::kTiles;
 }
@@ -975,7 +1057,7 @@ int dispatch_mfma_swiglu(const MfmaArgs& a, hipStream_t s) {
     return MMF_ERR_ARG;
 }
 
-// The matrix pipe with nothing else to do: every wave issues the tiled kernel's four independent 32x32x32 int8 MFMAs per
+// The matrix pipe with nothing else to do: every wave issues four independent 32x32x32 int8 MFMAs per
 // step on operands that never leave its registers (8 waves per workgroup, 4 waves per SIMD with two workgroups per CU).
 // random_operands: int8 codes and ternary weights drawn per lane (the switching activity of real operands) instead of the
 // constant 1s, on which the pipe draws far less power.

@@ -20,6 +20,17 @@ def test_split_tiles_are_exact(dev, m, k, n, dtype):
                            F.bitlinear_mfma(q[0], deq[0], qsum[0], pw, m, dtype, config=16, **kw)), tuple(kw)
 
 
+@pytest.mark.parametrize("blocks", range(1, 9))
+def test_every_end_of_the_k_loop_is_exact(dev, blocks):
+    """One to eight k-blocks, so that the loop of three ends at each of them in each of its first rounds; rows that end inside, at and behind a
+    16-row fragment, columns inside one; the lean epilogue (n = 264) and the general one (n = 257)."""
+    for m, n in ((15, 264), (112, 257), (145, 264)):
+        F, lib, pw, q, codes, deq, qsum = operands(dev, m, 128 * blocks - 3, n, seed=blocks)
+        want = exact(F, pw, codes[0], deq[0], torch.bfloat16)
+        for config in (15, 16, 17) + ((18,) if blocks % 2 == 0 else ()):
+            assert torch.equal(F.bitlinear_mfma(q[0], deq[0], qsum[0], pw, m, torch.bfloat16, config=config).cpu(), want), (m, n, config)
+
+
 def test_odd_number_of_k_blocks_is_refused(dev):
     F, lib, pw, q, codes, deq, qsum = operands(dev, 70, 384, 256)
     with pytest.raises(RuntimeError):
