@@ -245,7 +245,12 @@ constexpr int kQWaves = 8, kQThreads = kQWaves * 64;
 // packed four at a time.  8192 x 2048 bf16, three norms: 37 -> 28 us; residual norm: 33 -> 22.  The gated form takes its sigmoids near
 // (16384 x 2048: 56 -> 52 us, 2002 x 2048 10.6 -> 9.8), and so does the step form (64 x 2048: 5.5 -> 4.9); with a row a workgroup the
 // gated form keeps the exact ones (64 x 2048: 4.1 against 4.3).
-// VEC: K, the strides and every pointer allow 4-element accesses.
+// With several rows a workgroup the codes go out through LDS: a thread's four are 4 bytes of a 16-byte piece, pieces of a row lie 512 bytes apart,
+// and written as they come every store touched 16 lines for 256 bytes; the caches' write requests, not the bytes, set the pace.  From LDS a
+// store writes 16 pieces of all the workgroup's rows (64 bytes for four), and neighbouring workgroups share an XCD, so that whole lines leave its L2.
+// 16384 rows bf16: 5632 wide 73.5 -> 53.3 us (5.2 TB/s; 57.6 without the sharing, 64.8 with it alone), residual norm of 2048 60.4 -> 46.9, gated
+// norm 53.3 -> 44.0, norm 30.0 -> 29.8 (bound by the vector units); 2002 rows the same to 6 % faster.
+// VEC: K, the strides and every pointer allow 4-element accesses (the entry points ask for codes at 16 bytes).
 // NN = 3: the row is normalised once and quantised under three norm weights (the projections of a trained layer share their
 // input, not their inner norm): one read of the row and one rstd instead of three, the three maxima in one exchange.
 template <typename T, typename TW, int NV, int PRO, bool VEC, int RPW, int NN = 1>
@@ -254,11 +259,16 @@ __global__ __launch_bounds__(kQThreads) void row_quant_fused_kernel(FusedQuantAr
     __shared__ double red_a[kQWaves], red_b[kQWaves];
     __shared__ float red_f[NN][kQWaves];
     __shared__ int red_i[NN][kQWaves];
+    constexpr bool STAGED = VEC && RPW > 1;                     // the codes go out through LDS, as [group of 16 inputs][row][16 bytes]
+    __shared__ __align__(16) uint32_t stage[STAGED ? NN : 1][STAGED ? NV * kQThreads : 1];
     constexpr bool HAS_AUX = PRO >= QPRO_RESNORM, STEP = PRO == QPRO_STEP_GATE, HAS_W1 = PRO != QPRO_SWIGLU && PRO != QPRO_PLAIN;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int w0 = (wave / WPR) * WPR;                          // first wave of this row
     const int tr = (int)threadIdx.x % TPR;                      // thread within the row
-    const int64_t row_raw = (int64_t)blockIdx.x * RPW + (int)threadIdx.x / TPR;
+    // XCD: workgroups are dealt round-robin to the 8 XCDs; of every 64 in turn each takes 8 neighbours, so the rows of a 32-row code block meet in
+    // one L2 and leave it as whole lines
+    const uint32_t in64 = blockIdx.x & 63, wg = RPW > 1 && (blockIdx.x | 63) < gridDim.x ? blockIdx.x - in64 + (in64 & 7) * 8 + (in64 >> 3) : blockIdx.x;
+    const int64_t row0 = (int64_t)wg * RPW, row_raw = row0 + (int)threadIdx.x / TPR;
     const bool live = row_raw < a.M;                            // rows past M compute on row M-1 and store nothing
     const int64_t row = live ? row_raw : a.M - 1;
     const int K = (int)a.K, Kp = (int)a.Kp;
@@ -449,7 +459,8 @@ __global__ __launch_bounds__(kQThreads) void row_quant_fused_kernel(FusedQuantAr
                 uint32_t packed4 = mmf_code4(y, scale[j]);
                 if (VEC && !inb(v, k0, 0)) packed4 = 0;
                 qs[j] = mmf_code4_sum(packed4, qs[j]);
-                if (live) *reinterpret_cast<uint32_t*>(a.q + j * a.q_stride + off) = packed4;
+                if constexpr (STAGED) stage[j][((k0 >> 4) * RPW + (int)threadIdx.x / TPR) * 4 + ((k0 & 15) >> 2)] = packed4;
+                else if (live) *reinterpret_cast<uint32_t*>(a.q + j * a.q_stride + off) = packed4;
             }
         }
     }
@@ -459,12 +470,28 @@ __global__ __launch_bounds__(kQThreads) void row_quant_fused_kernel(FusedQuantAr
 #pragma unroll
         for (int j = 0; j < NN; ++j)
             if ((threadIdx.x & 63) == 0) red_i[j][wave] = qs[j];
-        __syncthreads();
+    }
+    if constexpr (WPR > 1 || STAGED) __syncthreads();
+    if constexpr (WPR > 1) {
 #pragma unroll
         for (int j = 0; j < NN; ++j) {
             qs[j] = 0;
 #pragma unroll
             for (int w = 0; w < WPR; ++w) qs[j] += red_i[j][w0 + w];
+        }
+    }
+    if constexpr (STAGED) {
+        // the workgroup's rows lie in one 32-row block (RPW divides 32): RPW * 16 contiguous bytes per group
+        const int chunks = (Kp >> 4) * RPW;
+        const int64_t base = (row0 >> 5) * (Kp >> 4) * 512 + (row0 & 31) * 16;
+#pragma unroll
+        for (int v = 0; v < mmf_ceil_div(NV, 4); ++v) {
+            const int c = v * kQThreads + (int)threadIdx.x, r = c % RPW;
+            if (c < chunks && row0 + r < a.M) {
+#pragma unroll
+                for (int j = 0; j < NN; ++j)
+                    *reinterpret_cast<uint4*>(a.q + j * a.q_stride + base + (int64_t)(c / RPW) * 512 + r * 16) = *reinterpret_cast<const uint4*>(&stage[j][c * 4]);
+            }
         }
     }
     if (tr == 0 && live) {
