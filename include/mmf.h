@@ -433,7 +433,8 @@ int mmf_block_forward(const mmf_block* p, const void* x, void* out, int64_t B, i
  *   contract with, the forward's bit for bit) and dweights [(kind != 2) + norms, K] (w1 first) in the weights' type; part:
  *   mmf_chain_bwd_groups(M) * ((kind != 2) + norms) * K floats of scratch.  K a multiple of 4, at most 8192 (4096 with three norms).
  * mmf_unpack_dequant: out [N, K] = ternary code * wdeq[row / seg_rows], in `dtype`; mmf_unpack_dequant_t: the same matrix stored
- *   [K, N] (K up to 1048448). */
+ *   [K, N] (K up to 1048448).
+ * mmf_transpose16: out [cols, rows] = x [rows, cols], 16-bit elements (rows up to 4194240). */
 int mmf_chain_bwd_groups(int64_t rows);
 int mmf_chain_bwd(int kind, const void* x, int64_t ldx, const void* aux, int64_t ldaux, const void* w1, float eps1, int norms,
                   const void* const* w2, float eps2, const void* const* dy, int64_t lddy, const void* dres, void* dx, int64_t lddx,
@@ -443,6 +444,7 @@ int mmf_unpack_dequant(const void* packed, const float* wdeq, int64_t seg_rows, 
                        void* stream);
 int mmf_unpack_dequant_t(const void* packed, const float* wdeq, int64_t seg_rows, int64_t N, int64_t K, void* out, int dtype,
                          void* stream);
+int mmf_transpose16(const void* x, int64_t rows, int64_t cols, void* out, void* stream);
 
 #ifdef __cplusplus
 }

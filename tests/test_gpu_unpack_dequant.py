@@ -51,3 +51,25 @@ def test_both_layouts_of_the_dense_weights_hold_the_same_values(dev, n, k, seg, 
                                             L.stream()), "mmf_unpack_dequant")
         columns = _dequantised(pw, dtype)
     assert columns.t().is_contiguous() and torch.equal(rows, columns)
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (7, 65), (64, 64), (72, 8), (130, 264), (1031, 33), (1024, 2048)])
+def test_transpose_of_16_bit_elements(dev, rows, cols):
+    """Whole and partial tiles, both widths of access, and a matrix that begins off a 16-byte boundary; nothing written past the end."""
+    import matmulfreellm_amd._lib as L
+    for off in (0, 1):
+        x = torch.randint(-32768, 32767, (rows * cols + off,), dtype=torch.int16, device=dev)[off:].view(rows, cols)
+        out = torch.full((rows * cols + 8,), 77, dtype=torch.int16, device=dev)
+        L.check(L.load().mmf_transpose16(x.data_ptr(), rows, cols, out.data_ptr(), L.stream()), "mmf_transpose16")
+        assert torch.equal(out[:rows * cols].view(cols, rows), x.t()) and bool((out[rows * cols:] == 77).all())
+
+
+@pytest.mark.parametrize("m,n,k", [(1023, 16384, 64), (1024, 16384, 64), (1025, 16390, 70)])
+def test_weight_gradient_of_a_vocabulary_is_the_product(dev, m, n, k):
+    """Both sides of the line where the inputs are transposed first; bf16 products summed in fp32: half an ulp of the result and m roundings of the sum."""
+    from matmulfreellm_amd.autograd import _weight_grad
+    torch.manual_seed(m)
+    d, y = torch.randn(m, n, device=dev).bfloat16(), torch.randn(m, k, device=dev).bfloat16()
+    want = d.t().double() @ y.double()
+    bound = want.abs() * 2 ** -8 + (d.t().double().abs() @ y.double().abs()) * m * 2 ** -24
+    assert bool(((_weight_grad(d, y).double() - want).abs() <= bound).all())
