@@ -196,7 +196,7 @@ __device__ __forceinline__ void mfma_epilogue(const MfmaArgs& p, A (&acc)[WM][WN
 // Lean epilogue of the common case (16-byte stores possible, no bias): the accumulators were
 // started at -qsum[m], so a value costs one convert and two multiplies; lane-constant parts of the
 // store addresses are computed once; interior tiles skip the bounds tests.
-template <typename T, int WM, int WN>
+template <bool STREAM, typename T, int WM, int WN>
 __device__ __forceinline__ void mfma_epilogue_fast(const MfmaArgs& p, Acc16 (&acc)[WM][WN], const EpiScales<Lay16, WM, WN>& sc,
                                                    unsigned char* smem, int lane, int wave, int wm, int64_t mb0, int64_t nb0) {
     const T* addend = static_cast<const T*>(p.addend);
@@ -244,7 +244,8 @@ __device__ __forceinline__ void mfma_epilogue_fast(const MfmaArgs& p, Acc16 (&ac
                     for (int e = 0; e < 16 / E; ++e) oe[e] = mmf_from_float<T>(__fadd_rn(mmf_to_float(pe[e]), mmf_to_float(ae[e])));
                     __builtin_memcpy(&v, oe, 16);
                 }
-                *reinterpret_cast<uint4*>(out + off) = v;
+                if constexpr (STREAM) __builtin_nontemporal_store(*reinterpret_cast<const v4i*>(&v), reinterpret_cast<v4i*>(out + off));
+                else *reinterpret_cast<uint4*>(out + off) = v;
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -478,7 +479,7 @@ constexpr int dma3_work_bytes() {
 // requested with it) is complete for everybody.  K-block
 // boundaries therefore carry no synchronisation: the A fragments of the next k-block's first
 // step are read while the current one's last MFMAs run, and the matrix pipe never drains.
-// FAST (chosen by the launcher): 16-byte stores possible and no bias -> lean epilogue, accumulators start at -qsum.
+// FAST (chosen by the launcher): 16-byte stores possible and no bias -> lean epilogue, accumulators start at -qsum.  2: stores past the caches.
 // SWI: the weight is the stacked [gate; up] projection (N = 2 * I): a wave's two n-blocks are the gate and the up rows
 // of the same 32 channels, a workgroup tile covers WGN such channel blocks, and the epilogue writes swiglu(gate, up).
 // KS > 1: the workgroup's waves form KS groups that take every KS-th k-block of the same (KS times narrower) tile: a mid-sized
@@ -490,7 +491,7 @@ constexpr int dma3_work_bytes() {
 // 16x16x64, us: 16384 x 2048 -> 6144 204 and 172-180 (2.4 P op/s), x 5632 -> 2048 147 and 126-130 (3.0), x 2048 -> 11264 with swiglu 363-369 and
 // 316-325; 4096 x 2048 -> 11264 83 and 73, 2002 rows 44 and 40.  On at most one tile per CU what counts is each wave's chain of instructions: there both
 // forms take the same time within 5 % (5632 -> 2048 split: 2002 rows 24 and 23.4, 1377 rows 21.4 and 21.8).
-template <typename T, int WGM, int WGN, int WM, int WN, int KS, bool FAST, bool SWI = false>
+template <typename T, int WGM, int WGN, int WM, int WN, int KS, int FAST, bool SWI = false>
 __global__ __launch_bounds__(64 * WGM * WGN * KS, (WM * WN <= 4 ? 4 : 1))   // small wave tiles: 4 waves per SIMD = two workgroups per CU
 void bitlinear_mfma_dma3_kernel(MfmaArgs p) {
     constexpr int NT = WGM * WGN;                  // waves that cover the tile once
@@ -706,7 +707,7 @@ void bitlinear_mfma_dma3_kernel(MfmaArgs p) {
         }
     if constexpr (KS == 1) {
         if constexpr (SWI) mfma_epilogue_swiglu<T, WM>(p, acc, sc, smem, lane, wave, wm, mb0, nb0);
-        else if constexpr (FAST) mfma_epilogue_fast<T, WM, WN>(p, acc, sc, smem, lane, wave, wm, mb0, nb0);
+        else if constexpr (FAST) mfma_epilogue_fast<FAST == 2, T, WM, WN>(p, acc, sc, smem, lane, wave, wm, mb0, nb0);
         else mfma_epilogue<T, Lay16>(p, acc, sc, smem, lane, wave, wm, mb0, nb0);
     } else {
         // group g finishes row block g of the wave tile: it takes the other groups' partial sums of that block
@@ -753,7 +754,7 @@ void bitlinear_mfma_dma3_kernel(MfmaArgs p) {
         __syncthreads();                                         // the exchange area becomes the epilogue's staging area
         const int wm1 = wm * WM + wk;
         if constexpr (SWI) mfma_epilogue_swiglu<T, 1>(p, mine, sc1, smem, lane, wave, wm1, mb0, nb0);
-        else if constexpr (FAST) mfma_epilogue_fast<T, 1, WN>(p, mine, sc1, smem, lane, wave, wm1, mb0, nb0);
+        else if constexpr (FAST) mfma_epilogue_fast<FAST == 2, T, 1, WN>(p, mine, sc1, smem, lane, wave, wm1, mb0, nb0);
         else mfma_epilogue<T, Lay16>(p, mine, sc1, smem, lane, wave, wm1, mb0, nb0);
     }
     if (p.clocks && threadIdx.x == 0 && (int64_t)blockIdx.x < p.clock_cap) {
@@ -790,9 +791,16 @@ int launch_mfma_dma3(MfmaArgs a, hipStream_t s) {
     const int per_vec = 16 / (int)sizeof(T);
     a.vec_store = SWI || ((a.N % per_vec == 0) && (a.ldo % per_vec == 0) && ((reinterpret_cast<uintptr_t>(a.out) & 15u) == 0) &&
                           ((reinterpret_cast<uintptr_t>(a.addend) & 15u) == 0));
-    auto kern = bitlinear_mfma_dma3_kernel<T, WGM, WGN, WM, WN, KS, true, SWI>;
+    // 16-bit outputs of 20 MB and more leave the caches to the activations and weights.  bf16, the launch and what reads its output next, us: 16384 x 2048 ->
+    // 6144 (201 MB) 148 and 70 (gate and scan), streamed 147 and 62; -> 2048 and 5632 -> 2048 (67 MB) 98.5 on average and 46.9 (residual norm), 94.6
+    // and 44.6; 2002 x 2048 -> 6144 (25 MB) 31.7 and 16.4, 29.5 and 17.0.  1377 rows (17 MB): 26.3 and 12.5, 25.1 and 13.2, no gain.  Not the swiglu form, whose
+    // output is half as large for its time: 293 and 54 (quantiser), 297 and 65; nor fp32: 666 x 1024 -> 32000 (85 MB) 36.6 and 18.9 (loss), 34.7 and 30.0.
+    auto kern = bitlinear_mfma_dma3_kernel<T, WGM, WGN, WM, WN, KS, 1, SWI>;
     if constexpr (!SWI) {
-        if (!a.vec_store || a.bias) kern = bitlinear_mfma_dma3_kernel<T, WGM, WGN, WM, WN, KS, false, false>;
+        if (!a.vec_store || a.bias) kern = bitlinear_mfma_dma3_kernel<T, WGM, WGN, WM, WN, KS, 0, false>;
+        else if constexpr (sizeof(T) == 2) {
+            if (a.M * a.N * 2 >= (20 << 20)) kern = bitlinear_mfma_dma3_kernel<T, WGM, WGN, WM, WN, KS, 2, false>;
+        }
     }
     if (lds > 48 * 1024) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
