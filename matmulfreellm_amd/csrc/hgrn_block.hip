@@ -490,7 +490,12 @@ Joint joint_begin(const Plan& p, float* workspace, int64_t BH, int64_t D, hipStr
 // Whether loads and stores are streamed past the caches.  Large tensors gain (40 x 2048 x 1024 bf16 118 + 198 -> 111 + 188 us, 128 x
 // 8192 x 128 156 + 259 -> 138 + 241, 5.8 TB/s), smaller ones that a consumer finds in the 256 MB last-level cache lose (16 x 777 x 1024
 // 14.5 + 27 against 18 + 29; even at 64 MB a tensor); in the second launch over time segments from 24 MB on (6000 x 64 columns 46 + 69 -> 45 + 62).
-bool streams(const Plan& p, int64_t bytes) { return bytes >= (p.NS > 1 ? 24ll << 20 : 64ll << 20); }
+// Only whole lines: where a row is no multiple of 128 bytes neighbouring columns share lines, which streamed are fetched twice (9 x 3068 x 1808
+// bf16, forward and backward, 312 us, streamed 418; columns shared by workgroups: 30 x 12073 x 144 288 and 406, 8 x 4049 x 720 148 and 169).
+bool whole_lines(int64_t row_bytes) { return row_bytes % 128 == 0; }
+bool streams(const Plan& p, int64_t row_bytes, int64_t rows) {
+    return whole_lines(row_bytes) && rows * row_bytes >= (p.NS > 1 ? 24ll << 20 : 64ll << 20);
+}
 template <typename T, int LS, bool NT>
 int launch_fwd_ls(const Plan& p, const T* x, const T* g, const float* h0, T* o, float* ht, float* agg, int64_t BH, int64_t Tlen,
                   int64_t D, hipStream_t s) {
@@ -518,13 +523,14 @@ int launch_fwd(const void* x, const void* g, const float* h0, void* o, float* ht
     if (p.G > 1) {
         const Joint jt = joint_begin(p, agg, BH, D, s);
         MMF_CHECK_LAUNCH();
-        hgrn_scan_fwd_kernel<T, false, 1, true, true><<<(unsigned)joint_grid(p, BH, D), 64 * kMaxWaves, 0, s>>>(
+        auto kern = whole_lines(D * (int64_t)sizeof(T)) ? hgrn_scan_fwd_kernel<T, false, 1, true, true> : hgrn_scan_fwd_kernel<T, false, 1, false, true>;
+        kern<<<(unsigned)joint_grid(p, BH, D), 64 * kMaxWaves, 0, s>>>(
             xp, gp, h0, op, ht, nullptr, Tlen, D, p.seg_len, 1, jt);
         MMF_CHECK_LAUNCH();
         return 0;
     }
     return p.LS == 2 ? launch_fwd_ls<T, 2, false>(p, xp, gp, h0, op, ht, agg, BH, Tlen, D, s)
-           : streams(p, BH * Tlen * D * (int64_t)sizeof(T)) ? launch_fwd_ls<T, 1, true>(p, xp, gp, h0, op, ht, agg, BH, Tlen, D, s)
+           : streams(p, D * (int64_t)sizeof(T), BH * Tlen) ? launch_fwd_ls<T, 1, true>(p, xp, gp, h0, op, ht, agg, BH, Tlen, D, s)
                                                         : launch_fwd_ls<T, 1, false>(p, xp, gp, h0, op, ht, agg, BH, Tlen, D, s);
 }
 
@@ -556,13 +562,14 @@ int launch_bwd(const void* g, const void* o, const void* dout, const float* h0, 
     if (p.G > 1) {
         const Joint jt = joint_begin(p, agg, BH, D, s);
         MMF_CHECK_LAUNCH();
-        hgrn_scan_bwd_kernel<T, LOG, false, 1, true, true><<<(unsigned)joint_grid(p, BH, D), 64 * kMaxWaves, 0, s>>>(
+        auto kern = whole_lines(D * (int64_t)sizeof(T)) ? hgrn_scan_bwd_kernel<T, LOG, false, 1, true, true> : hgrn_scan_bwd_kernel<T, LOG, false, 1, false, true>;
+        kern<<<(unsigned)joint_grid(p, BH, D), 64 * kMaxWaves, 0, s>>>(
             gp, op, dp, h0, xp, yp, nullptr, Tlen, D, p.seg_len, 1, jt);
         MMF_CHECK_LAUNCH();
         return 0;
     }
     return p.LS == 2 ? launch_bwd_ls<T, LOG, 2, false>(p, gp, op, dp, h0, xp, yp, agg, BH, Tlen, D, s)
-           : streams(p, BH * Tlen * D * (int64_t)sizeof(T)) ? launch_bwd_ls<T, LOG, 1, true>(p, gp, op, dp, h0, xp, yp, agg, BH, Tlen, D, s)
+           : streams(p, D * (int64_t)sizeof(T), BH * Tlen) ? launch_bwd_ls<T, LOG, 1, true>(p, gp, op, dp, h0, xp, yp, agg, BH, Tlen, D, s)
                                                         : launch_bwd_ls<T, LOG, 1, false>(p, gp, op, dp, h0, xp, yp, agg, BH, Tlen, D, s);
 }
 
