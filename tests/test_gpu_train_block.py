@@ -174,3 +174,41 @@ def test_block_gradients_are_no_further_from_64_bits_than_the_compositions(dev, 
         block, composition = (((v.double() - r).norm() / r.norm()).item() for v in (a, c))
         assert block <= 1.1 * composition, (name, block, composition)
         assert dtype == torch.float32 or block < 4 * torch.finfo(dtype).eps / 2, (name, block)
+
+
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("k", [2048, 2052, 5632])
+def test_gradients_take_the_sigmoid_of_the_definition(dev, gated, k):
+    """bf16 rows whose gate arguments lie in [-30, -16], where a sigmoid from hardware exp2 alone is up to 30 units of 2^-24 off.  A stored
+    gradient misses the exact one by half a spacing of bf16 and at most 14 units: 3 in the sigmoid, 1 in each root, 4 in the gradient
+    through the norm, 5 in the products behind it (3.1 measured; with hardware exp2 alone 22 to 27)."""
+    import matmulfreellm_amd.functional as F
+    from matmulfreellm_amd.autograd import CHAIN_GATED, CHAIN_SWIGLU, _chain_bwd
+    torch.manual_seed(k)
+    rows = 1024
+    gate = (-16 - 14 * torch.rand(rows, k, device=dev)).bfloat16()
+    other, dy = torch.randn(rows, k, device=dev).bfloat16(), torch.randn(rows, k, device=dev).bfloat16()
+    w1, w2 = ((0.5 + torch.rand(k, device=dev)).bfloat16() for _ in range(2))
+    a, v, d64 = gate.double(), other.double(), dy.double()
+    sg = torch.sigmoid(a)
+    other_grad = torch.empty_like(gate)
+    if gated:
+        s = F.rmsnorm_swishgate(other, gate, w1, eps=1e-6).double()
+        x, aux, kind = other, gate, CHAIN_GATED
+        xh = v * torch.rsqrt(v.square().mean(-1, keepdim=True) + 1e-6)
+    else:
+        s = F.swiglu(gate, other).double()
+        x, aux, kind = gate, other, CHAIN_SWIGLU
+    rstd = torch.rsqrt(s.square().mean(-1, keepdim=True) + 1e-6)
+    wd = w2.double() * d64
+    d = (wd - s * rstd * (s * rstd * wd).mean(-1, keepdim=True)) * rstd
+    got, daux, _, _ = _chain_bwd(kind, x, aux, w1 if gated else None, 1e-6, [w2], 1e-6, [dy], daux=other_grad)
+    if gated:
+        pairs = [(daux, d * xh * w1.double() * sg * (1 + a * (1 - sg)))]
+    else:
+        pairs = [(daux, d * a * sg), (got, sg * (1 + a * (1 - sg)) * d * v)]
+    for value, want in pairs:
+        spacing = torch.exp2(torch.floor(torch.log2(want.abs())) - 7)
+        beyond = ((value.double() - want).abs() - spacing / 2) / want.abs()
+        beyond = beyond[(wd.abs() > 0.05) & (want != 0)]                 # (the subtraction in d has cancelled nothing there)
+        assert beyond.max().item() <= 14 * 2 ** -24
