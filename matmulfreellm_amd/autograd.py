@@ -254,6 +254,19 @@ def _dequantised(pw, dtype):
     return w.t()
 
 
+def _dense_weight(pw, dtype):
+    """The dense ternary weights for dout @ W_q, stored as that product and their unpacking take least time together.
+
+    16-bit products run faster with the contraction contiguous (_dequantised).  Single-precision ones take the same time either way, and
+    rows are written faster than columns: a 1024-wide step's 13 unpackings 126 us stored [K, N], 103 us stored [N, K]."""
+    if dtype != torch.float32:
+        return _dequantised(pw, dtype)
+    w = torch.empty(pw.n, pw.k, dtype=dtype, device=pw.packed.device)
+    L.check(L.load().mmf_unpack_dequant(pw.packed.data_ptr(), pw.wdeq.data_ptr(), pw.seg_rows, pw.n, pw.k, w.data_ptr(), L.dtype_id(dtype),
+                                        L.stream()), "mmf_unpack_dequant")
+    return w
+
+
 def _weight_grad(dout, y):
     """dout^T @ y_q of [M, N] gradients and [M, K] de-quantised inputs.
 
@@ -262,7 +275,7 @@ def _weight_grad(dout, y):
     1097 / 816, 16384 x 1024 1154 / 824, 4096 x 2048 493 / 410, 1024 x 2048 152 / 131; the transposition moves 4 bytes an element, 1.6 % of the
     product.  For fewer outputs it costs more of the product (11264: 4 %) than it gives there (-5 to 12 %)."""
     m, k = y.shape
-    if y.element_size() == 2 and dout.shape[1] >= 16384 and m >= 1024 and y.is_contiguous():
+    if y.element_size() == 2 and dout.shape[1] >= 16384 and 1024 <= m <= 4194240 and y.is_contiguous():
         yt = torch.empty(k, m, dtype=y.dtype, device=y.device)
         L.check(L.load().mmf_transpose16(y.data_ptr(), m, k, yt.data_ptr(), L.stream()), "mmf_transpose16")
         y = yt.t()
@@ -312,18 +325,18 @@ class BlockFn(torch.autograd.Function):
             d2 = dout.to(dt).reshape(m, H).contiguous()
             o_pw, gate_pw, down_pw = plan.pws[3:]
             # down_proj behind the swiglu: the gradients of gate and up land side by side
-            dz = d2 @ _dequantised(down_pw, dt)
+            dz = d2 @ _dense_weight(down_pw, dt)
             dy = torch.empty_like(y)
             _, _, yq, dw_down = _chain_bwd(CHAIN_SWIGLU, y[:, :I], y[:, I:], None, 0.0, [down_n], eps["down_eps"], [dz], dx=dy[:, :I],
                                            daux=dy[:, I:])
             d_down = d2.t() @ yq[0] if need[14] else None
             # gate_proj behind mlp_norm, the residual's gradient joining
-            dh = dy @ _dequantised(gate_pw, dt)
+            dh = dy @ _dense_weight(gate_pw, dt)
             dres, _, yq, dw_gate = _chain_bwd(CHAIN_RESNORM, attn, x.view(m, H), mlp_norm, eps["mlp_eps"], [gate_n], eps["gate_eps"], [dh],
                                                dres=d2)
             d_gate = dy.t() @ yq[0] if need[13] else None
             # o_proj behind the gated norm: the g columns of the stacked projection's gradient, and the scan's output
-            do2 = dres @ _dequantised(o_pw, dt)
+            do2 = dres @ _dense_weight(o_pw, dt)
             difg, do = torch.empty_like(ifg), torch.empty_like(o)
             _, _, yq, dw_o = _chain_bwd(CHAIN_GATED, ifg[:, 2 * D:], o, g_norm, eps["g_eps"], [o_n], eps["o_eps"], [do2],
                                         dx=difg[:, 2 * D:], daux=do)
@@ -337,7 +350,7 @@ class BlockFn(torch.autograd.Function):
                                           dgs.data_ptr(), difg.data_ptr(), 3 * D, difg.data_ptr() + D * e, 3 * D, L.ptr(part), L.ptr(dlb),
                                           m, D, L.dtype_id(dt), L.stream()), "mmf_hgrn_gate_bwd")
             # i, f, g behind attn_norm: three products, one pass over the rows, the residual's gradient joining
-            w3, dh3 = _dequantised(plan.stacked, dt), torch.empty(3, m, H, dtype=dt, device=dev)
+            w3, dh3 = _dense_weight(plan.stacked, dt), torch.empty(3, m, H, dtype=dt, device=dev)
             cols = [difg[:, j * D:(j + 1) * D] for j in range(3)]
             for j in range(3):
                 torch.mm(cols[j], w3[j * D:(j + 1) * D], out=dh3[j])
@@ -366,7 +379,7 @@ class NormHeadFn(torch.autograd.Function):
         x, norm_weight, head_norm_weight = ctx.saved_tensors
         with L.on(x.device):
             x2, d2 = _2d(x).contiguous(), _2d(dout).to(x.dtype).contiguous()
-            dh = d2 @ _dequantised(ctx.pw, x.dtype)
+            dh = d2 @ _dense_weight(ctx.pw, x.dtype)
             dx, _, yq, dw = _chain_bwd(CHAIN_NORM, x2, None, norm_weight, ctx.eps1, [head_norm_weight], ctx.eps2, [dh])
             d_weight = _weight_grad(d2, yq[0]) if ctx.needs_input_grad[3] else None
         return dx.view(x.shape), dw[0], dw[1], d_weight, None, None, None

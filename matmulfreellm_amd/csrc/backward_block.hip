@@ -329,8 +329,8 @@ __global__ __launch_bounds__(256) void unpack_dequant_kernel(const uint32_t* __r
 // The same matrix stored [K, N]: the product dout @ W_q contracts over N, and the library's kernels run fastest where both
 // operands are contiguous along the contraction.  8192 rows in bf16 on random data, [N, K] against [K, N]: 32000 x 2048 798 / 657 us,
 // 11264 x 2048 300 / 242, 2048 x 5632 158 / 161; inside a training step of three layers the 19 products take 2797 / 2501 us (the step 10739 /
-// 10544).  fp32 products take either in the same time.  A thread owns one dword of codes
-// (16 inputs) of VE neighbouring output rows, so a wave's store is 1 KiB of one input's row.
+// 10544).  fp32 products take either in the same time (666 and 2002 rows, 1024 to 32000 outputs), so fp32
+// weights are stored [N, K], 23 against 27 us at 32000 x 1024.  A thread owns one dword of codes (16 inputs) of VE neighbouring output rows, so a wave's store is 1 KiB of one input's row.
 template <typename T>
 __global__ __launch_bounds__(256) void unpack_dequant_t_kernel(const uint32_t* __restrict__ packed, const float* __restrict__ wdeq,
                                                                uint32_t seg_rows, int N, int K, int KB, bool whole, T* __restrict__ out) {

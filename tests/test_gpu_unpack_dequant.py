@@ -73,3 +73,18 @@ def test_weight_gradient_of_a_vocabulary_is_the_product(dev, m, n, k):
     want = d.t().double() @ y.double()
     bound = want.abs() * 2 ** -8 + (d.t().double().abs() @ y.double().abs()) * m * 2 ** -24
     assert bool(((_weight_grad(d, y).double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("n,k,seg", [(1, 4, 1), (33, 132, 33), (96, 1024, 32)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_dense_weights_are_stored_as_their_product_takes_least_time(dev, n, k, seg, dtype):
+    """The training products' weights: contraction (N) contiguous in 16 bits, rows as the packed ones in single precision; same values."""
+    import matmulfreellm_amd.functional as F
+    from matmulfreellm_amd.autograd import _dense_weight
+    torch.manual_seed(n + k)
+    pw = F.ternarize_pack(torch.randn(n, k, device=dev))
+    codes = F.unpack_ternary(pw).float()
+    pw.wdeq, pw.seg_rows = torch.rand(-(-n // seg), device=dev) + 0.5, seg
+    w = _dense_weight(pw, dtype)
+    assert (w if dtype == torch.float32 else w.t()).is_contiguous()
+    assert torch.equal(w, (codes * pw.wdeq.repeat_interleave(seg)[:n].view(n, 1)).to(dtype))
