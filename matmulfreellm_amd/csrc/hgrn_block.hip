@@ -78,14 +78,20 @@ __device__ __forceinline__ float take_carry(uint64_t& word, int n) {
 __device__ __forceinline__ void done_before_the_turn(float& l, float& P, float& lin, float& Pin, float& lb, float& Pb) {
     asm volatile("" : "+v"(l), "+v"(P), "+v"(lin), "+v"(Pin), "+v"(lb), "+v"(Pb)::"memory");
 }
-// JOINT: G workgroups share a column and take its superblocks (a block for each wave) in turn; what enters superblock n travels in a
-// word of memory per channel, number beside value as in LDS.  A member composes its waves' blocks before the carry arrives, so
-// between taking it and passing it on lies one multiply-add.  Who waits, waits for a member that was dispatched before it or next to it (the
-// members of a column follow one another on one XCD); a wait that gives up all the same goes on with NaN, which the results show.
+// JOINT: G workgroups share a column; each claims the column's next superblock (a block for each wave) from a counter.  What enters superblock
+// n travels in a word of memory per channel, number beside value as in LDS.  A member composes its waves' blocks before the carry
+// arrives, so between taking it and passing it on lies one multiply-add.
+// Every wait ends, however few members run at once and whatever else the GPU runs: a member works on what it has claimed, claims are in order,
+// and so everything that it waits for is in the hands of a running member, whose own wait is for something earlier still.  (With every
+// G-th superblock assigned to a member, members that run could wait for one that found no room beside other kernels.)  The polls are bounded
+// all the same; one that gave up would go on with NaN, which the results show.
+// A claim is made when the carry is there, in the order in which the carry passes: the members keep taking turns, and the claim travels while the block
+// is stored.  Made earlier, the claims came in no particular order and the chain waited for loads (64 x 16384 x 128 bf16 forward: every G-th
+// 156 us, claimed so 156, in front of a superblock's loads 171 to 174, behind them 178).
 struct Joint {
-    uint64_t* words;      // [BH][D, rounded up to 64], zeroed in front of the launch
+    uint64_t* words;      // per column: 64 carries, and behind all of them a counter each; zeroed in front of the launch
     int G;                // members of a column
-    int64_t BH;
+    int64_t BH, columns;
 };
 constexpr int kJointPolls = 1 << 22;                                    // seconds
 __device__ __forceinline__ void pass_joint(uint64_t* word, float c, int n) {
@@ -102,10 +108,28 @@ __device__ __forceinline__ float take_joint(uint64_t* word, int n) {
 // What the carry c makes of a run of steps with the product P and the own contribution l.  (A zero carry stays zero also where
 // a product of gates beyond one has overflowed.)
 __device__ __forceinline__ float fold(float l, float P, float c) { return c == 0.0f ? l : fmaf(P, c, l); }
-// The carry that enters this wave's block (l, P) of superblock n, whose `nw` waves all come here.  last: no superblock follows.
-__device__ __forceinline__ float joint_carry(float l, float P, int n, bool last, int wave, int nw, float2 (*pair)[64], uint64_t* carry,
-                                             uint64_t* word, float first) {
-    const int lane = (int)threadIdx.x & 63;
+// A workgroup's work on a column: the superblock it holds, the one it has claimed to follow (thread 0), how many it has taken.
+struct Turns {
+    uint64_t* word;       // this lane's carry
+    uint64_t* counter;
+    uint64_t next;
+    int n, taken;
+};
+struct JointLds {
+    float2 pair[2][kMaxWaves][64];
+    uint64_t next[2];                                                   // how many were taken | the next one
+};
+__device__ __forceinline__ uint64_t claim(uint64_t* counter) {
+    uint32_t at = 0;                                                    // an offset of the lane's own: for a uniform address the compiler waits on the spot
+    asm volatile("" : "+v"(at));
+    uint64_t n = 0;
+    if (threadIdx.x == 0) n = __hip_atomic_fetch_add(counter + at, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return n;
+}
+// The carry that enters this wave's block (l, P) of superblock t.n, whose `nw` waves all come here.  last: no superblock follows.
+__device__ __forceinline__ float joint_carry(float l, float P, Turns& t, bool last, int wave, int nw, JointLds& lds, uint64_t* carry, float first) {
+    const int lane = (int)threadIdx.x & 63, n = t.n;
+    float2 (*pair)[64] = lds.pair[t.taken & 1];
     pair[wave][lane] = make_float2(l, P);
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");     // LDS only: loads and stores stay in flight
     float lin = 0.0f, Pin = 1.0f;
@@ -117,21 +141,37 @@ __device__ __forceinline__ float joint_carry(float l, float P, int n, bool last,
     float c;
     if (wave == nw - 1) {
         const float lt = fold(l, P, lin), Pt = P * Pin;
-        c = n == 0 ? first : take_joint(word, n);
-        if (!last) pass_joint(word, fold(lt, Pt, c), n + 1);
+        c = n == 0 ? first : take_joint(t.word, n);
+        if (!last) pass_joint(t.word, fold(lt, Pt, c), n + 1);
         pass_carry(carry[lane], c, n);
     } else {
         c = take_carry(carry[lane], n);
     }
+    t.next = claim(t.counter);
     return fold(lin, Pin, c);
 }
-// Which column and member a workgroup of a joint launch is: the G members of a column follow one another on one XCD.
-__device__ __forceinline__ bool joint_place(const Joint& jt, int64_t D, int64_t& bh, unsigned& cb, int& member) {
+// Which column a workgroup of a joint launch works on: the G members of a column follow one another on one XCD.
+__device__ __forceinline__ bool joint_place(const Joint& jt, int64_t D, int64_t& bh, unsigned& cb, Turns& t) {
     const unsigned G = (unsigned)jt.G, nd = (unsigned)((D + 63) / 64), col = blockIdx.x / (8u * G) * 8u + blockIdx.x % 8u;
-    member = (int)(blockIdx.x / 8u % G);
     bh = col / nd;
     cb = col % nd;
+    t = Turns{jt.words + (int64_t)col * 64 + (threadIdx.x & 63), jt.words + jt.columns * 64 + col, 0, 0, 0};   // (lanes past D: words of their own)
     return bh < jt.BH;                                                  // columns are padded to eights
+}
+// run(n): the block n of a wave, through joint_carry; idle(): its part in that where the superblock has no block left for it.
+template <typename Run, typename Idle>
+__device__ __forceinline__ void joint_turns(Turns& t, JointLds& lds, int nblk, int wave, int nw, Run&& run, Idle&& idle) {
+    while (t.n * nw < nblk) {
+        if (t.n * nw + wave < nblk) run(t.n * nw + wave);
+        else idle();
+        uint64_t* const slot = &lds.next[t.taken & 1];                  // (written again two superblocks on, a barrier behind everyone's read)
+        if (threadIdx.x == 0) __hip_atomic_store(slot, (uint64_t)(uint32_t)(t.taken + 1) << 32 | (uint32_t)t.next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        ++t.taken;
+        uint64_t w;
+        do w = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        while ((int)(w >> 32) != t.taken);
+        t.n = __builtin_amdgcn_readfirstlane((int)w);
+    }
 }
 // The parts of a wave's block in the order the scan takes them, k = 0 .. LS - 1 in lanes part(k): (lin, Pin) composes the parts
 // in front of this lane's, (lb, Pb) all of them.
@@ -161,15 +201,15 @@ __global__ __launch_bounds__(64 * kMaxWaves, 4) void hgrn_scan_fwd_kernel(const 
     constexpr int CH = 64 / LS, kBlk = kFwdBlk, kStep = LS * kBlk;      // channels of a workgroup, steps of a wave's block
     __shared__ uint64_t carry[CH];
     __shared__ float prod[AGG ? kMaxWaves : 1][64];
-    __shared__ float2 pairs[JOINT ? 2 : 1][JOINT ? kMaxWaves : 1][64];
+    __shared__ typename std::conditional<JOINT, JointLds, int>::type joint_lds;
     const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), nw = (int)blockDim.x >> 6;
     const int ch = lane % CH, u = lane / CH;                            // channel, and which kBlk steps of the wave's block
     int64_t bh = blockIdx.y;
     const int seg = JOINT ? 0 : (int)blockIdx.z;                        // AGG: nobody folds the pair of the last segment
     unsigned cb = JOINT ? 0u : column_block<LS>();
-    int member = 0;
+    Turns turns{};
     if constexpr (JOINT) {
-        if (!joint_place(jt, D, bh, cb, member)) return;
+        if (!joint_place(jt, D, bh, cb, turns)) return;
     }
     const int64_t d = (int64_t)cb * CH + ch;
     const bool active = d < D;
@@ -180,9 +220,14 @@ __global__ __launch_bounds__(64 * kMaxWaves, 4) void hgrn_scan_fwd_kernel(const 
     const int64_t t0 = (int64_t)seg * seg_len, t1 = t0 + seg_len < Tlen ? t0 + seg_len : Tlen;
     const int nblk = (int)((t1 - t0 + kStep - 1) / kStep);
     const float first = JOINT && h0 ? h0[bh * D + dl] : 0.0f;
-    uint64_t* const word = JOINT ? jt.words + (bh * ((D + 63) / 64) + cb) * 64 + lane : nullptr;   // (lanes past D: words of their own)
-    int super = member;                                                 // JOINT: the superblock
-    if (JOINT && wave == 0) pass_carry(carry[ch], 0.0f, -1);
+    if constexpr (JOINT) {
+        if (wave == 0) pass_carry(carry[ch], 0.0f, -1);
+        const uint64_t n = claim(turns.counter);
+        if (threadIdx.x == 0) {
+            joint_lds.next[0] = 0;
+            joint_lds.next[1] = (uint32_t)n;
+        }
+    }
     if (!JOINT && wave == 0) {
         float c = h0 && (!AGG || seg == 0) ? h0[bh * D + dl] : 0.0f;    // h0 enters the fold through segment 0's pair
         if constexpr (!AGG) {
@@ -196,6 +241,7 @@ __global__ __launch_bounds__(64 * kMaxWaves, 4) void hgrn_scan_fwd_kernel(const 
     }
     float own = 1.0f;                                                   // AGG: product of this wave's gates
     __syncthreads();
+    if constexpr (JOINT) turns.n = __builtin_amdgcn_readfirstlane((int)joint_lds.next[1]);
     // One block; FULL: it has all its steps (no tests), otherwise the tail of the segment.
     auto block = [&](int n, int64_t tb, int rem, auto full) __attribute__((always_inline)) {
         constexpr bool FULL = decltype(full)::value;
@@ -234,7 +280,7 @@ __global__ __launch_bounds__(64 * kMaxWaves, 4) void hgrn_scan_fwd_kernel(const 
         done_before_the_turn(l, P, lin, Pin, lb, Pb);
         float cb;
         if constexpr (JOINT) {
-            cb = joint_carry(lb, Pb, super, (super + 1) * nw >= nblk, wave, nw, pairs[super / jt.G & 1], carry, word, first);
+            cb = joint_carry(lb, Pb, turns, (turns.n + 1) * nw >= nblk, wave, nw, joint_lds, carry, first);
         } else {
             cb = take_carry(carry[ch], n);
             pass_carry(carry[ch], fold(lb, Pb, cb), n + 1);             // (the parts of a channel write the same value)
@@ -259,10 +305,7 @@ __global__ __launch_bounds__(64 * kMaxWaves, 4) void hgrn_scan_fwd_kernel(const 
         else block(n, tb, rem, std::false_type{});
     };
     if constexpr (JOINT) {
-        for (; super * nw < nblk; super += jt.G) {
-            if (super * nw + wave < nblk) run(super * nw + wave);
-            else joint_carry(0.0f, 1.0f, super, true, wave, nw, pairs[super / jt.G & 1], carry, word, first);   // no block left for this wave
-        }
+        joint_turns(turns, joint_lds, nblk, wave, nw, run, [&] { joint_carry(0.0f, 1.0f, turns, true, wave, nw, joint_lds, carry, first); });
     } else {
         for (int n = wave; n < nblk; n += nw) run(n);
     }
@@ -289,15 +332,15 @@ __global__ __launch_bounds__(64 * kMaxWaves, 4) void hgrn_scan_bwd_kernel(const 
     constexpr int CH = 64 / LS, kBlk = kBwdBlk, kStep = LS * kBlk;                      // channels of a workgroup, steps of a wave's block
     __shared__ uint64_t carry[CH];
     __shared__ float prod[AGG ? kMaxWaves : 1][64];
-    __shared__ float2 pairs[JOINT ? 2 : 1][JOINT ? kMaxWaves : 1][64];
+    __shared__ typename std::conditional<JOINT, JointLds, int>::type joint_lds;
     const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), nw = (int)blockDim.x >> 6;
     const int ch = lane % CH, u = lane / CH;                            // channel, and which kBlk steps of the wave's block
     int64_t bh = blockIdx.y;
     const int seg = JOINT ? 0 : AGG ? (int)blockIdx.z + 1 : (int)blockIdx.z;   // nobody folds the pair of segment 0
     unsigned cb = JOINT ? 0u : column_block<LS>();
-    int member = 0;
+    Turns turns{};
     if constexpr (JOINT) {
-        if (!joint_place(jt, D, bh, cb, member)) return;
+        if (!joint_place(jt, D, bh, cb, turns)) return;
     }
     const int64_t d = (int64_t)cb * CH + ch;
     const bool active = d < D;
@@ -308,9 +351,14 @@ __global__ __launch_bounds__(64 * kMaxWaves, 4) void hgrn_scan_bwd_kernel(const 
     const int64_t t0 = (int64_t)seg * seg_len, t1 = t0 + seg_len < Tlen ? t0 + seg_len : Tlen;
     const int nblk = (int)((t1 - t0 + kStep - 1) / kStep);
     const float hinit = !AGG && h0 ? h0[bh * D + dl] : 0.0f;
-    uint64_t* const word = JOINT ? jt.words + (bh * ((D + 63) / 64) + cb) * 64 + lane : nullptr;   // (lanes past D: words of their own)
-    int super = member;                                                 // JOINT: the superblock
-    if (JOINT && wave == 0) pass_carry(carry[ch], 0.0f, -1);
+    if constexpr (JOINT) {
+        if (wave == 0) pass_carry(carry[ch], 0.0f, -1);
+        const uint64_t n = claim(turns.counter);
+        if (threadIdx.x == 0) {
+            joint_lds.next[0] = 0;
+            joint_lds.next[1] = (uint32_t)n;
+        }
+    }
     if (!JOINT && wave == 0) {
         float c = 0.0f;
         if constexpr (!AGG) {
@@ -323,6 +371,7 @@ __global__ __launch_bounds__(64 * kMaxWaves, 4) void hgrn_scan_bwd_kernel(const 
     }
     float own = 1.0f;                                                   // AGG: product of this wave's gates
     __syncthreads();
+    if constexpr (JOINT) turns.n = __builtin_amdgcn_readfirstlane((int)joint_lds.next[1]);
     // One block; FULL: it has all its steps (no tests), otherwise the tail of the segment.
     auto block = [&](int n, int64_t tb, int rem, auto full) __attribute__((always_inline)) {
         constexpr bool FULL = decltype(full)::value;
@@ -376,7 +425,7 @@ __global__ __launch_bounds__(64 * kMaxWaves, 4) void hgrn_scan_bwd_kernel(const 
         done_before_the_turn(l, P, lin, Pin, lb, Pb);
         float cb;
         if constexpr (JOINT) {
-            cb = joint_carry(lb, Pb, super, (super + 1) * nw >= nblk, wave, nw, pairs[super / jt.G & 1], carry, word, 0.0f);
+            cb = joint_carry(lb, Pb, turns, (turns.n + 1) * nw >= nblk, wave, nw, joint_lds, carry, 0.0f);
         } else {
             cb = take_carry(carry[ch], n);
             pass_carry(carry[ch], fold(lb, Pb, cb), n + 1);             // (the parts of a channel write the same value)
@@ -403,10 +452,7 @@ __global__ __launch_bounds__(64 * kMaxWaves, 4) void hgrn_scan_bwd_kernel(const 
         else block(n, tb, rem, std::false_type{});
     };
     if constexpr (JOINT) {
-        for (; super * nw < nblk; super += jt.G) {
-            if (super * nw + wave < nblk) run(super * nw + wave);
-            else joint_carry(0.0f, 1.0f, super, true, wave, nw, pairs[super / jt.G & 1], carry, word, 0.0f);   // no block left for this wave
-        }
+        joint_turns(turns, joint_lds, nblk, wave, nw, run, [&] { joint_carry(0.0f, 1.0f, turns, true, wave, nw, joint_lds, carry, 0.0f); });
     } else {
         for (int n = wave; n < nblk; n += nw) run(n);
     }
@@ -466,7 +512,8 @@ bool fwd_takes_workspace(int64_t BH, int64_t Tlen, int64_t D, int chunk) {
     return BH * mmf_ceil_div(D, 64) < 256 && Tlen >= 8 * block;
 }
 Plan fwd_plan(int64_t BH, int64_t Tlen, int64_t D, int chunk) { return plan(BH, Tlen, D, kFwdBlk, fwd_takes_workspace(BH, Tlen, D, chunk)); }
-int64_t joint_bytes(int64_t BH, int64_t D) { return BH * mmf_round_up(D, 64) * 8; }
+int64_t joint_columns(int64_t BH, int64_t D) { return BH * mmf_ceil_div(D, 64); }
+int64_t joint_bytes(int64_t BH, int64_t D) { return joint_columns(BH, D) * 65 * 8; }
 int64_t pair_bytes(const Plan& p, int64_t BH, int64_t D) {
     return p.G > 1 ? joint_bytes(BH, D) : p.NS > 1 ? BH * p.NS * 2 * D * (int64_t)sizeof(float) : 0;
 }
@@ -480,12 +527,12 @@ __global__ __launch_bounds__(256) void joint_words_kernel(uint64_t* __restrict__
     if (i < n) words[i] = 0;
 }
 bool holds_words(const float* workspace) { return workspace && (reinterpret_cast<uintptr_t>(workspace) & 7u) == 0; }
-int64_t joint_grid(const Plan& p, int64_t BH, int64_t D) { return mmf_round_up(BH * mmf_ceil_div(D, 64), 8) * p.G; }
+int64_t joint_grid(const Plan& p, int64_t BH, int64_t D) { return mmf_round_up(joint_columns(BH, D), 8) * p.G; }
 Joint joint_begin(const Plan& p, float* workspace, int64_t BH, int64_t D, hipStream_t s) {
     uint64_t* words = reinterpret_cast<uint64_t*>(workspace);
     const int64_t n = joint_bytes(BH, D) / 8;
     joint_words_kernel<<<(unsigned)mmf_ceil_div(n, 256), 256, 0, s>>>(words, n);
-    return Joint{words, p.G, BH};
+    return Joint{words, p.G, BH, joint_columns(BH, D)};
 }
 // Whether loads and stores are streamed past the caches.  Large tensors gain (40 x 2048 x 1024 bf16 118 + 198 -> 111 + 188 us, 128 x
 // 8192 x 128 156 + 259 -> 138 + 241, 5.8 TB/s), smaller ones that a consumer finds in the 256 MB last-level cache lose (16 x 777 x 1024

@@ -138,3 +138,31 @@ def test_scans_whose_columns_are_shared_by_workgroups(dev, bh, d, t, dtype):
         for name, p, r in zip(("o", "state", "dx", "dg"), got, want):
             err = ((p.detach().double() - r).abs().max() / r.abs().max()).item()
             assert err < (2e-5 if dtype == torch.float32 or name == "state" else 8e-3), (name, err)
+
+
+def test_shared_columns_beside_other_streams(dev):
+    """Three streams whose workgroups together are several times what the GPU holds, so that members of a column run without the others:
+    every result is what the same call gives by itself, bit for bit (the carries are folded in one order, whoever does it)."""
+    import matmulfreellm_amd as mm
+    torch.manual_seed(5)
+    calls = []
+    for bh, t, d, dtype, log in ((128, 6000, 64, torch.bfloat16, True), (64, 9000, 64, torch.float32, False), (10, 5000, 1024, torch.float16, True)):
+        z = torch.randn(1, bh, t, d, device=dev) + 1
+        g = (torch.nn.functional.logsigmoid if log else torch.sigmoid)(z).to(dtype).requires_grad_()
+        x, do = torch.randn(1, bh, t, d, device=dev).to(dtype).requires_grad_(), torch.randn(1, bh, t, d, device=dev).to(dtype)
+        calls.append((mm.chunk_hgrn if log else mm.fused_recurrent_hgrn, x, g, do))
+    def run(scan, x, g, do):
+        o, last = scan(x, g, output_final_state=True)
+        return [o.detach(), last, *torch.autograd.grad(o, (x, g), do)]
+    alone = [run(*c) for c in calls]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in calls]
+    together = [[] for _ in calls]
+    for _ in range(4):
+        for s, c, out in zip(streams, calls, together):
+            with torch.cuda.stream(s):
+                out.append(run(*c))
+    torch.cuda.synchronize()
+    for outs, want in zip(together, alone):
+        for got in outs:
+            assert all(torch.equal(a, b) for a, b in zip(got, want))
