@@ -72,6 +72,17 @@ __device__ __forceinline__ float take_carry(uint64_t& word, int n) {
     }
     return __uint_as_float((uint32_t)w);
 }
+// AGG: the product of the gates in front of block n travels in a word of its own, so that it is taken in the blocks' order (grouped by wave, a product
+// that stays in range can meet an infinite partial one, and NaN where another is zero).  Both words are read in one trip.
+__device__ __forceinline__ float take_pair(uint64_t& word, uint64_t& word_p, int n, float& p) {
+    uint64_t c, q;
+    do {
+        c = __hip_atomic_load(&word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        q = __hip_atomic_load(&word_p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    } while ((int)(c >> 32) != n || (int)(q >> 32) != n);
+    p = __uint_as_float((uint32_t)q);
+    return __uint_as_float((uint32_t)c);
+}
 // The local pass ends here.  Left to itself the compiler moves it behind the wait, next to the first use of its results, and the
 // turns that were to be a handful of instructions each take the loads' latency and all the arithmetic of a block: 570 ns a turn
 // (64 x 16384 x 128 on 128 workgroups: 333 us forward, 218 with this line).
@@ -127,28 +138,44 @@ __device__ __forceinline__ uint64_t claim(uint64_t* counter) {
     return n;
 }
 // The carry that enters this wave's block (l, P) of superblock t.n, whose `nw` waves all come here.  last: no superblock follows.
+// Composed only while every block's product is at most one (and NaN nowhere): beyond, the product of eight overflows where a step for each block
+// stays in range, and an infinite one that meets a zero gives NaN.  There the blocks are folded in one by one, as without members.
 __device__ __forceinline__ float joint_carry(float l, float P, Turns& t, bool last, int wave, int nw, JointLds& lds, uint64_t* carry, float first) {
     const int lane = (int)threadIdx.x & 63, n = t.n;
     float2 (*pair)[64] = lds.pair[t.taken & 1];
     pair[wave][lane] = make_float2(l, P);
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");     // LDS only: loads and stores stay in flight
-    float lin = 0.0f, Pin = 1.0f;
+    float lin = 0.0f, Pin = 1.0f, most = fabsf(P), least = most;
     for (int w = 0; w < wave; ++w) {
         const float2 q = pair[w][lane];
         lin = fold(q.x, q.y, lin);
         Pin *= q.y;
+        most = fmaxf(most, fabsf(q.y));
+        least = fminf(least, fabsf(q.y));
     }
+    float Pt = P * Pin;
+    const bool composed = __builtin_amdgcn_ballot_w64(!(most <= 1.0f) || Pt != Pt) == 0;
+    // only a zero gate makes a product zero: an infinite carry stays infinite as it does block by block
+    if (least > 0.0f) {
+        Pin = Pin == 0.0f ? copysignf(0x1p-149f, Pin) : Pin;
+        Pt = Pt == 0.0f ? copysignf(0x1p-149f, Pt) : Pt;
+    }
+    auto enter = [&](float c) __attribute__((always_inline)) {           // what the carry c of the superblock is in front of this wave's block
+        if (composed) return fold(lin, Pin, c);
+        for (int w = 0; w < wave; ++w) c = fold(pair[w][lane].x, pair[w][lane].y, c);
+        return c;
+    };
     float c;
     if (wave == nw - 1) {
-        const float lt = fold(l, P, lin), Pt = P * Pin;
+        const float lt = fold(l, P, lin);
         c = n == 0 ? first : take_joint(t.word, n);
-        if (!last) pass_joint(t.word, fold(lt, Pt, c), n + 1);
+        if (!last) pass_joint(t.word, composed ? fold(lt, Pt, c) : fold(l, P, enter(c)), n + 1);
         pass_carry(carry[lane], c, n);
     } else {
         c = take_carry(carry[lane], n);
     }
     t.next = claim(t.counter);
-    return fold(lin, Pin, c);
+    return enter(c);
 }
 // Which column a workgroup of a joint launch works on: the G members of a column follow one another on one XCD.
 __device__ __forceinline__ bool joint_place(const Joint& jt, int64_t D, int64_t& bh, unsigned& cb, Turns& t) {
@@ -200,7 +227,7 @@ __global__ __launch_bounds__(64 * kMaxWaves, 4) void hgrn_scan_fwd_kernel(const 
                                                                        int64_t Tlen, int64_t D, int64_t seg_len, int NS, Joint jt) {
     constexpr int CH = 64 / LS, kBlk = kFwdBlk, kStep = LS * kBlk;      // channels of a workgroup, steps of a wave's block
     __shared__ uint64_t carry[CH];
-    __shared__ float prod[AGG ? kMaxWaves : 1][64];
+    __shared__ uint64_t carry_p[AGG ? CH : 1];
     __shared__ typename std::conditional<JOINT, JointLds, int>::type joint_lds;
     const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), nw = (int)blockDim.x >> 6;
     const int ch = lane % CH, u = lane / CH;                            // channel, and which kBlk steps of the wave's block
@@ -238,8 +265,8 @@ __global__ __launch_bounds__(64 * kMaxWaves, 4) void hgrn_scan_fwd_kernel(const 
             }
         }
         pass_carry(carry[ch], c, 0);
+        if constexpr (AGG) pass_carry(carry_p[ch], 1.0f, 0);
     }
-    float own = 1.0f;                                                   // AGG: product of this wave's gates
     __syncthreads();
     if constexpr (JOINT) turns.n = __builtin_amdgcn_readfirstlane((int)joint_lds.next[1]);
     // One block; FULL: it has all its steps (no tests), otherwise the tail of the segment.
@@ -282,9 +309,11 @@ __global__ __launch_bounds__(64 * kMaxWaves, 4) void hgrn_scan_fwd_kernel(const 
         if constexpr (JOINT) {
             cb = joint_carry(lb, Pb, turns, (turns.n + 1) * nw >= nblk, wave, nw, joint_lds, carry, first);
         } else {
-            cb = take_carry(carry[ch], n);
+            float p = 1.0f;
+            if constexpr (AGG) cb = take_pair(carry[ch], carry_p[ch], n, p);
+            else cb = take_carry(carry[ch], n);
             pass_carry(carry[ch], fold(lb, Pb, cb), n + 1);             // (the parts of a channel write the same value)
-            if constexpr (AGG) own *= Pb;
+            if constexpr (AGG) pass_carry(carry_p[ch], p * Pb, n + 1);
         }
         if constexpr (!AGG) {
             const __amdgpu_buffer_rsrc_t ro = rsrc(o + row0);
@@ -310,14 +339,14 @@ __global__ __launch_bounds__(64 * kMaxWaves, 4) void hgrn_scan_fwd_kernel(const 
         for (int n = wave; n < nblk; n += nw) run(n);
     }
     if constexpr (AGG) {
-        prod[wave][lane] = own;
-        __syncthreads();
-        if (wave == 0 && active) {
-            float P = 1.0f;
-            for (int w = 0; w < nw; ++w) P *= prod[w][lane];
-            float* ag = agg + (bh * NS + seg) * 2 * D;
-            ag[d] = P;
-            ag[D + d] = take_carry(carry[ch], nblk);
+        if (wave == 0) {
+            float p;
+            const float c = take_pair(carry[ch], carry_p[ch], nblk, p);
+            if (active) {
+                float* ag = agg + (bh * NS + seg) * 2 * D;
+                ag[d] = p;
+                ag[D + d] = c;
+            }
         }
     }
 }
@@ -331,7 +360,7 @@ __global__ __launch_bounds__(64 * kMaxWaves, 4) void hgrn_scan_bwd_kernel(const 
                                                                        int64_t seg_len, int NS, Joint jt) {
     constexpr int CH = 64 / LS, kBlk = kBwdBlk, kStep = LS * kBlk;                      // channels of a workgroup, steps of a wave's block
     __shared__ uint64_t carry[CH];
-    __shared__ float prod[AGG ? kMaxWaves : 1][64];
+    __shared__ uint64_t carry_p[AGG ? CH : 1];
     __shared__ typename std::conditional<JOINT, JointLds, int>::type joint_lds;
     const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), nw = (int)blockDim.x >> 6;
     const int ch = lane % CH, u = lane / CH;                            // channel, and which kBlk steps of the wave's block
@@ -368,8 +397,8 @@ __global__ __launch_bounds__(64 * kMaxWaves, 4) void hgrn_scan_bwd_kernel(const 
             }
         }
         pass_carry(carry[ch], c, 0);
+        if constexpr (AGG) pass_carry(carry_p[ch], 1.0f, 0);
     }
-    float own = 1.0f;                                                   // AGG: product of this wave's gates
     __syncthreads();
     if constexpr (JOINT) turns.n = __builtin_amdgcn_readfirstlane((int)joint_lds.next[1]);
     // One block; FULL: it has all its steps (no tests), otherwise the tail of the segment.
@@ -427,9 +456,11 @@ __global__ __launch_bounds__(64 * kMaxWaves, 4) void hgrn_scan_bwd_kernel(const 
         if constexpr (JOINT) {
             cb = joint_carry(lb, Pb, turns, (turns.n + 1) * nw >= nblk, wave, nw, joint_lds, carry, 0.0f);
         } else {
-            cb = take_carry(carry[ch], n);
+            float p = 1.0f;
+            if constexpr (AGG) cb = take_pair(carry[ch], carry_p[ch], n, p);
+            else cb = take_carry(carry[ch], n);
             pass_carry(carry[ch], fold(lb, Pb, cb), n + 1);             // (the parts of a channel write the same value)
-            if constexpr (AGG) own *= Pb;
+            if constexpr (AGG) pass_carry(carry_p[ch], p * Pb, n + 1);
         }
         if constexpr (!AGG) {
             const __amdgpu_buffer_rsrc_t rx = rsrc(dx + row0), ry = rsrc(dg + row0);
@@ -457,14 +488,14 @@ __global__ __launch_bounds__(64 * kMaxWaves, 4) void hgrn_scan_bwd_kernel(const 
         for (int n = wave; n < nblk; n += nw) run(n);
     }
     if constexpr (AGG) {
-        prod[wave][lane] = own;
-        __syncthreads();
-        if (wave == 0 && active) {
-            float P = 1.0f;
-            for (int w = 0; w < nw; ++w) P *= prod[w][lane];
-            float* ag = agg + (bh * NS + seg) * 2 * D;
-            ag[d] = P;
-            ag[D + d] = take_carry(carry[ch], nblk);
+        if (wave == 0) {
+            float p;
+            const float c = take_pair(carry[ch], carry_p[ch], nblk, p);
+            if (active) {
+                float* ag = agg + (bh * NS + seg) * 2 * D;
+                ag[d] = p;
+                ag[D + d] = c;
+            }
         }
     }
 }

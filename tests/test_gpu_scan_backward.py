@@ -166,3 +166,53 @@ def test_shared_columns_beside_other_streams(dev):
     for outs, want in zip(together, alone):
         for got in outs:
             assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def _by_blocks(t, block, products, reverse, per_segment=None):
+    """Gates of [t] steps whose products over the kernels' blocks (of 28 steps, backwards 24 from the last one on, counted anew in every
+    `per_segment` of them) are `products` in turn, and 0.5 a step beyond."""
+    a = torch.full((t,), 0.5, dtype=torch.double)
+    per_segment = per_segment or -(-t // block)
+    for s in range(0, t, per_segment * block):
+        e = min(t, s + per_segment * block)
+        blocks = [(i, min(e, i + block)) for i in range(s, e, block)]
+        for (i, j), p in zip(blocks[::-1] if reverse else blocks, products):
+            a[i:j] = p ** (1.0 / block)
+    return a
+
+
+@pytest.mark.parametrize("bh,per_segment,reverse,kind", [(32, None, r, k) for r in (False, True) for k in ("grows", "vanishes", "infinite")] +
+                         [(1, 10, False, "grows"), (1, 11, True, "grows")])
+def test_products_of_gates_keep_the_range_of_a_block(dev, bh, per_segment, reverse, kind):
+    """Gates that are no decays, by blocks: columns shared by workgroups (32 of 3100 steps) and cut in time (one of 16384, 10 or 11 blocks a
+    segment).  grows: a carry of 1e-25 passes blocks of 1e30, 1e30, 1e-30, 1e-30, whose product from the left overflows where the carry does not.
+    vanishes: one of 1e-50 in front of 1e50: nothing is left of the carry, and no NaN.  infinite: an infinite carry stays infinite while
+    each block's product is above zero."""
+    import matmulfreellm_amd as mm
+    t, block = 16384 if per_segment else 3100, 24 if reverse else 28
+    products = {"grows": [1.0] * 2 + [1e30, 1e30, 1e-30, 1e-30] + [1.0] * 4, "vanishes": [1.0, 1e-50, 1e50] + [1.0] * 7, "infinite": []}[kind]
+    if per_segment and kind == "grows":                # by waves: two blocks of 1e25 in one's hands, two of 1e-25 in another's
+        products = [1e25, 1e-25] + [1.0] * 6 + [1e25, 1e-25, 1.0]
+    a = _by_blocks(t, block, products, reverse, per_segment)
+    g = a.float()[None, None, :, None].expand(1, bh, t, 64).contiguous()
+    x, do, h0 = torch.zeros(1, bh, t, 64), torch.zeros(1, bh, t, 64), torch.zeros(1, bh, 64)
+    start = {"grows": 1e-25, "vanishes": 1.0, "infinite": float("inf")}[kind]
+    if reverse:
+        do[:, :, -1] = start
+    else:
+        h0[:] = start
+    mine = [v.to(dev).requires_grad_() for v in (x, g.double().log().float() if not reverse else g)]
+    o, last = (mm.fused_recurrent_hgrn if reverse else mm.chunk_hgrn)(*mine, h0.to(dev), output_final_state=True)
+    got = torch.autograd.grad(o, mine, do.to(dev))[0] if reverse else o.detach()
+    gd = g[0, 0, :, 0].double()
+    if reverse:
+        want = start * torch.cat([gd.flip(0).cumprod(0).flip(0)[1:], torch.ones(1, dtype=torch.double)])
+    else:
+        want = start * gd.cumprod(0)
+    got = got[0, :, :, ::9].double().cpu()
+    if kind == "infinite":
+        assert torch.isinf(got).all()
+    elif kind == "vanishes":
+        assert torch.isfinite(got).all()
+    else:                                               # 28 roundings of a log gate of 2.5 a block, exp's own, and denormal ends
+        assert ((got - want[None, :, None]).abs() <= 1e-4 * want[None, :, None] + 1e-37).all()
