@@ -181,12 +181,15 @@ int mmf_bitlinear_mfma_swiglu(const int8_t* codes_tiled, const float* deq, const
  *   176-185 (kernel :32-68): h = g*h + x with g the decay itself.
  * mmf_hgrn_chunk replaces chunk_hgrn, mmfreelm/ops/hgrn/chunk.py:287-296 (kernels :49-116):
  *   h = exp(g)*h + x with g the log decay, evaluated in register blocks as the reference's chunked form is per chunk:
- *   a scan from zero with the running product E of the gates, then o_t += E_t * (state at the block's entry).  One pass over
+ *   a scan from zero with the product of the gates, then the recurrence once more from the state at the block's entry.  One pass over
  *   x and g (no fp32 [B,H,T,D] scratch tensors); `chunk` (1 <= chunk <= 64; the reference fixes 128) decides
  *   from which length on a sequence may be cut (see below) and changes the result by rounding at most.  A long sequence of few
  *   channels is also cut into time segments that run in parallel (a first launch leaves each
- *   segment's (decay product, end state) pair in `workspace`, mmf_hgrn_chunk_workspace_bytes(BH, T, D, chunk) bytes,
- *   4-byte aligned, may be NULL when that is 0).
+ *   segment's (decay product, end state) pair in `workspace`), or several workgroups take turns on 64 channels (32 to 170 times 64 of them, 3072
+ *   steps and more) and hand the state on in 64-bit words there.  workspace: mmf_hgrn_chunk_workspace_bytes(BH, T, D, chunk)
+ *   bytes, 4-byte aligned, any contents; NULL where that is 0, and accepted where the sequence can go uncut (from 128 times 64 channels on), else
+ *   MMF_ERR_ARG.  The turns need no more than one of their workgroups on the GPU at a time; a hand-over that did not come within
+ *   seconds would leave NaN in everything behind it.
  *   exp is the hardware one: results agree with the reference's within rounding, not bit for bit.
  * The final state is fp32 in both (the reference rounds the recurrent one to x's dtype).
  * MMF_ERR_WIDE when 64 rows of D elements reach 2 GiB. */
@@ -267,8 +270,9 @@ int mmf_hgrn_gate_bwd(const void* i_in, int64_t ldi, const void* f_in, int64_t l
  *   exp(g_t) and dg_t = dh h_{t-1} exp(g_t).  As in the reference the gradient of the final state is not propagated. */
 int mmf_hgrn_recurrent_bwd(const void* g, const void* o, const void* grad_o, const float* h0, void* dx, void* dg, int64_t BH,
                            int64_t T, int64_t D, int log_gates, int dtype, void* stream);
-/* The same with a workspace of mmf_hgrn_recurrent_bwd_workspace_bytes(BH, T, D) bytes (fp32, 0 bytes: may be NULL): a long
- *   sequence of few channels is then cut into time segments that run in parallel. */
+/* The same with a workspace of mmf_hgrn_recurrent_bwd_workspace_bytes(BH, T, D) bytes, 4-byte aligned, any contents; NULL leaves every sequence
+ *   whole.  A long sequence of few channels is then cut into time segments that run in parallel, or its channels are shared by workgroups that
+ *   hand the gradient on, as in mmf_hgrn_chunk. */
 int64_t mmf_hgrn_recurrent_bwd_workspace_bytes(int64_t BH, int64_t T, int64_t D);
 int mmf_hgrn_recurrent_bwd_split(const void* g, const void* o, const void* grad_o, const float* h0, void* dx, void* dg, int64_t BH,
                                  int64_t T, int64_t D, int log_gates, int dtype, void* workspace, void* stream);

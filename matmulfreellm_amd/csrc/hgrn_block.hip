@@ -515,10 +515,10 @@ struct Plan {
     int64_t seg_len;
     int NS, LS, G;
 };
-Plan plan(int64_t BH, int64_t Tlen, int64_t D, int blk, bool split) {
+Plan plan(int64_t BH, int64_t Tlen, int64_t D, int blk, bool split, bool joint) {
     Plan p;
     const int64_t wgs = BH * mmf_ceil_div(D, 64);
-    p.G = split && wgs >= 32 && wgs <= 170 && Tlen >= 3072 ? (int)((wgs <= 64 ? 256 : 512) / wgs) : 1;
+    p.G = joint && wgs >= 32 && wgs <= 170 && Tlen >= 3072 ? (int)((wgs <= 64 ? 256 : 512) / wgs) : 1;
     if (p.G > 1) {
         p.LS = p.NS = 1;
         p.seg_len = mmf_round_up(Tlen, blk);
@@ -542,9 +542,12 @@ bool fwd_takes_workspace(int64_t BH, int64_t Tlen, int64_t D, int chunk) {
     const int64_t block = (64 / chunk > 8 ? 8 : 64 / chunk) * (int64_t)chunk;
     return BH * mmf_ceil_div(D, 64) < 256 && Tlen >= 8 * block;
 }
-Plan fwd_plan(int64_t BH, int64_t Tlen, int64_t D, int chunk) { return plan(BH, Tlen, D, kFwdBlk, fwd_takes_workspace(BH, Tlen, D, chunk)); }
+Plan fwd_plan(int64_t BH, int64_t Tlen, int64_t D, int chunk, bool joint) {
+    const bool split = fwd_takes_workspace(BH, Tlen, D, chunk);
+    return plan(BH, Tlen, D, kFwdBlk, split, split && joint);
+}
 int64_t joint_columns(int64_t BH, int64_t D) { return BH * mmf_ceil_div(D, 64); }
-int64_t joint_bytes(int64_t BH, int64_t D) { return joint_columns(BH, D) * 65 * 8; }
+int64_t joint_bytes(int64_t BH, int64_t D) { return joint_columns(BH, D) * 65 * 8 + 8; }   // (8 over: the words begin at the workspace's first multiple of 8)
 int64_t pair_bytes(const Plan& p, int64_t BH, int64_t D) {
     return p.G > 1 ? joint_bytes(BH, D) : p.NS > 1 ? BH * p.NS * 2 * D * (int64_t)sizeof(float) : 0;
 }
@@ -557,11 +560,10 @@ __global__ __launch_bounds__(256) void joint_words_kernel(uint64_t* __restrict__
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i < n) words[i] = 0;
 }
-bool holds_words(const float* workspace) { return workspace && (reinterpret_cast<uintptr_t>(workspace) & 7u) == 0; }
 int64_t joint_grid(const Plan& p, int64_t BH, int64_t D) { return mmf_round_up(joint_columns(BH, D), 8) * p.G; }
 Joint joint_begin(const Plan& p, float* workspace, int64_t BH, int64_t D, hipStream_t s) {
-    uint64_t* words = reinterpret_cast<uint64_t*>(workspace);
-    const int64_t n = joint_bytes(BH, D) / 8;
+    uint64_t* words = reinterpret_cast<uint64_t*>((reinterpret_cast<uintptr_t>(workspace) + 7) & ~(uintptr_t)7);
+    const int64_t n = joint_columns(BH, D) * 65;
     joint_words_kernel<<<(unsigned)mmf_ceil_div(n, 256), 256, 0, s>>>(words, n);
     return Joint{words, p.G, BH, joint_columns(BH, D)};
 }
@@ -592,8 +594,7 @@ int launch_fwd_ls(const Plan& p, const T* x, const T* g, const float* h0, T* o, 
 template <typename T>
 int launch_fwd(const void* x, const void* g, const float* h0, void* o, float* ht, float* agg, int64_t BH, int64_t Tlen, int64_t D,
                int chunk, hipStream_t s) {
-    Plan p = fwd_plan(BH, Tlen, D, chunk);
-    if (p.G > 1 && !holds_words(agg)) p = plan(BH, Tlen, D, kFwdBlk, false);
+    const Plan p = fwd_plan(BH, Tlen, D, chunk, agg != nullptr);
     if (p.NS > 1 && !agg) return MMF_ERR_ARG;
     const T* xp = static_cast<const T*>(x);
     const T* gp = static_cast<const T*>(g);
@@ -630,8 +631,7 @@ int launch_bwd_ls(const Plan& p, const T* g, const T* o, const T* dout, const fl
 template <typename T, bool LOG>
 int launch_bwd(const void* g, const void* o, const void* dout, const float* h0, void* dx, void* dg, float* agg, int64_t BH,
                int64_t Tlen, int64_t D, hipStream_t s) {
-    Plan p = plan(BH, Tlen, D, kBwdBlk, agg != nullptr);
-    if (p.G > 1 && !holds_words(agg)) p = plan(BH, Tlen, D, kBwdBlk, false);
+    const Plan p = plan(BH, Tlen, D, kBwdBlk, agg != nullptr, agg != nullptr);
     const T* gp = static_cast<const T*>(g);
     const T* op = static_cast<const T*>(o);
     const T* dp = static_cast<const T*>(dout);
@@ -666,7 +666,7 @@ extern "C" {
 int64_t mmf_hgrn_chunk_workspace_bytes(int64_t BH, int64_t T, int64_t D, int chunk) {
     if (BH <= 0 || T <= 0 || D <= 0 || chunk < 1 || chunk > 64) return 0;
     if (!fwd_takes_workspace(BH, T, D, chunk)) return 0;
-    const Plan p = fwd_plan(BH, T, D, chunk);
+    const Plan p = fwd_plan(BH, T, D, chunk, true);
     return p.G > 1 ? joint_bytes(BH, D) : BH * p.NS * 2 * D * (int64_t)sizeof(float);
 }
 
@@ -695,7 +695,7 @@ int mmf_hgrn_chunk(const void* x, const void* g, const float* h0, void* o, float
 
 int64_t mmf_hgrn_recurrent_bwd_workspace_bytes(int64_t BH, int64_t T, int64_t D) {
     if (BH <= 0 || T <= 0 || D <= 0) return 0;
-    return pair_bytes(plan(BH, T, D, kBwdBlk, true), BH, D);
+    return pair_bytes(plan(BH, T, D, kBwdBlk, true, true), BH, D);
 }
 
 int mmf_hgrn_recurrent_bwd_split(const void* g, const void* o, const void* grad_o, const float* h0, void* dx, void* dg, int64_t BH,

@@ -216,3 +216,32 @@ def test_products_of_gates_keep_the_range_of_a_block(dev, bh, per_segment, rever
         assert torch.isfinite(got).all()
     else:                                               # 28 roundings of a log gate of 2.5 a block, exp's own, and denormal ends
         assert ((got - want[None, :, None]).abs() <= 1e-4 * want[None, :, None] + 1e-37).all()
+
+
+def test_workspace_of_shared_columns(dev):
+    """The C entries: a workspace at any multiple of 4 bytes serves the same plan (same bits); none is an error where the sequence has to be cut, as
+    for fewer than 128 columns it always had, and leaves it whole from there on."""
+    from matmulfreellm_amd import _lib as L
+    lib = L.load()
+    torch.manual_seed(2)
+    for bh, refused in ((32, True), (127, True), (128, False), (170, False)):
+        t, d = 3100, 64
+        x, do, z = (torch.randn(bh, t, d, device=dev) for _ in range(3))
+        g = torch.nn.functional.logsigmoid(z + 1)
+        nbytes = max(lib.mmf_hgrn_chunk_workspace_bytes(bh, t, d, 64), lib.mmf_hgrn_recurrent_bwd_workspace_bytes(bh, t, d))
+        ws = torch.full((nbytes // 4 + 4,), float("nan"), device=dev)
+        results = []
+        for at in (0, 4):
+            o, dx, dg = (torch.zeros_like(x) for _ in range(3))
+            p = ws.data_ptr() + at
+            L.check(lib.mmf_hgrn_chunk(x.data_ptr(), g.data_ptr(), None, o.data_ptr(), None, bh, t, d, 64, L.dtype_id(x.dtype), p, L.stream()), "fwd")
+            L.check(lib.mmf_hgrn_recurrent_bwd_split(g.data_ptr(), o.data_ptr(), do.data_ptr(), None, dx.data_ptr(), dg.data_ptr(), bh, t, d, 1,
+                                                     L.dtype_id(x.dtype), p, L.stream()), "bwd")
+            results.append((o, dx, dg))
+        assert all(torch.equal(a, b) for a, b in zip(*results))
+        assert all(torch.isfinite(a).all() for a in results[0])
+        o = torch.zeros_like(x)
+        rc = lib.mmf_hgrn_chunk(x.data_ptr(), g.data_ptr(), None, o.data_ptr(), None, bh, t, d, 64, L.dtype_id(x.dtype), None, L.stream())
+        assert (rc != 0) == refused
+        if not refused:
+            assert torch.allclose(o, results[0][0], rtol=1e-4, atol=1e-5)
