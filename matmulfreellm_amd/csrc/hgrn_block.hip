@@ -570,6 +570,8 @@ Joint joint_begin(const Plan& p, float* workspace, int64_t BH, int64_t D, hipStr
 // Whether loads and stores are streamed past the caches.  Large tensors gain (40 x 2048 x 1024 bf16 118 + 198 -> 111 + 188 us, 128 x
 // 8192 x 128 156 + 259 -> 138 + 241, 5.8 TB/s), smaller ones that a consumer finds in the 256 MB last-level cache lose (16 x 777 x 1024
 // 14.5 + 27 against 18 + 29; even at 64 MB a tensor); in the second launch over time segments from 24 MB on (6000 x 64 columns 46 + 69 -> 45 + 62).
+// Shared columns the same, with what reads their results next (streamed / not, us): 64 x 5000 x 64 bf16 (39 MB) forward and a reader 51 / 47, backward
+// and a reader 71 / 65, forward and backward 86 / 77; 59 MB 72 / 67, 108 / 109, 133 / 131; 94 MB 113 / 118, 166 / 171, 200 / 204.
 // Only whole lines: where a row is no multiple of 128 bytes neighbouring columns share lines, which streamed are fetched twice (9 x 3068 x 1808
 // bf16, forward and backward, 312 us, streamed 418; columns shared by workgroups: 30 x 12073 x 144 288 and 406, 8 x 4049 x 720 148 and 169).
 bool whole_lines(int64_t row_bytes) { return row_bytes % 128 == 0; }
@@ -602,7 +604,7 @@ int launch_fwd(const void* x, const void* g, const float* h0, void* o, float* ht
     if (p.G > 1) {
         const Joint jt = joint_begin(p, agg, BH, D, s);
         MMF_CHECK_LAUNCH();
-        auto kern = whole_lines(D * (int64_t)sizeof(T)) ? hgrn_scan_fwd_kernel<T, false, 1, true, true> : hgrn_scan_fwd_kernel<T, false, 1, false, true>;
+        auto kern = streams(p, D * (int64_t)sizeof(T), BH * Tlen) ? hgrn_scan_fwd_kernel<T, false, 1, true, true> : hgrn_scan_fwd_kernel<T, false, 1, false, true>;
         kern<<<(unsigned)joint_grid(p, BH, D), 64 * kMaxWaves, 0, s>>>(
             xp, gp, h0, op, ht, nullptr, Tlen, D, p.seg_len, 1, jt);
         MMF_CHECK_LAUNCH();
@@ -640,7 +642,7 @@ int launch_bwd(const void* g, const void* o, const void* dout, const float* h0, 
     if (p.G > 1) {
         const Joint jt = joint_begin(p, agg, BH, D, s);
         MMF_CHECK_LAUNCH();
-        auto kern = whole_lines(D * (int64_t)sizeof(T)) ? hgrn_scan_bwd_kernel<T, LOG, false, 1, true, true> : hgrn_scan_bwd_kernel<T, LOG, false, 1, false, true>;
+        auto kern = streams(p, D * (int64_t)sizeof(T), BH * Tlen) ? hgrn_scan_bwd_kernel<T, LOG, false, 1, true, true> : hgrn_scan_bwd_kernel<T, LOG, false, 1, false, true>;
         kern<<<(unsigned)joint_grid(p, BH, D), 64 * kMaxWaves, 0, s>>>(
             gp, op, dp, h0, xp, yp, nullptr, Tlen, D, p.seg_len, 1, jt);
         MMF_CHECK_LAUNCH();
