@@ -507,10 +507,14 @@ __global__ __launch_bounds__(64 * kMaxWaves, 4) void hgrn_scan_bwd_kernel(const 
 //      136 + 220, 16 x 16384 x 128 64 + 84 -> 50 + 71, 9 x 5000 x 1024 74 + 124 -> 69 + 109.  Below 3072 steps the hand-overs between
 //      workgroups show (64 x 2048 x 64 18 + 22 against 18 + 24, 7 x 1024 x 1024 11 + 16 against 17 + 22), below 32 columns the cut in time is as
 //      good (24 x 16384 x 64 48 + 63 / 48 + 64, 8 x 16384 x 64 28 + 31 / 45 + 60).
-//   up to 128, short sequences (and 128 columns at any length): a column is halved (LS = 2; 8.5 -> 6 us for 2 x 333 x 1024 fp32), at half
-//      a line a row and so half the bytes in flight; with more columns than that whole ones win (12 x 2048 x 1024 35 + 58 against 50 + 79).
-//   fewer columns, 2048 steps and more: whole 128-byte rows in time segments for about two workgroups per CU, a segment at least four
-//      blocks long; a first launch reads x and g (g and do) of all but one segment once more.
+//   up to 128, where they are not shared: a column is halved (LS = 2; 8.5 -> 6 us for 2 x 333 x 1024 fp32), at half a line a row and so half the
+//      bytes in flight; with more columns than that whole ones win at every length (12 x 2048 x 1024 35 + 58 against 50 + 79; halved against whole,
+//      forward + backward: 132 columns of 150 to 2500 steps 6.0 + 7.8 / 5.7 + 7.3 to 46 + 71 / 33 + 50, 192 of 300 9.2 + 13.1 / 8.0 + 11.2; 128 of 300
+//      6.6 + 9.6 / 7.6 + 10.8).
+//   64 columns and fewer, 2048 steps and more: whole 128-byte rows in time segments for about two workgroups per CU, a segment at least four
+//      blocks long; a first launch reads x and g (g and do) of all but one segment once more.  Halved against cut, forward + backward, 2500 steps, bf16 and
+//      fp32: 56 columns 49 / 48 and 53 / 73, 66 columns 52 / 52 and 59 / 87, 80 (of 1024-wide rows) 52 / 66 and 78 / 104, 96 54 / 76 and 99 / 123, 112 57 / 88
+//      and 116 / 143; 127 (of 64-wide rows, whose halves no neighbour shares) 87 / 90 and 122 / 155.
 struct Plan {
     int64_t seg_len;
     int NS, LS, G;
@@ -524,7 +528,7 @@ Plan plan(int64_t BH, int64_t Tlen, int64_t D, int blk, bool split, bool joint) 
         p.seg_len = mmf_round_up(Tlen, blk);
         return p;
     }
-    p.LS = wgs <= 128 && (wgs == 128 || Tlen < 2048) ? 2 : 1;
+    p.LS = wgs <= 128 && (wgs > 64 || Tlen < 2048) ? 2 : 1;
     const int64_t now = BH * mmf_ceil_div(D, 64 / p.LS), step = p.LS * blk;
     int64_t ns = 1;
     if (split && now < 128) {
@@ -597,7 +601,7 @@ template <typename T>
 int launch_fwd(const void* x, const void* g, const float* h0, void* o, float* ht, float* agg, int64_t BH, int64_t Tlen, int64_t D,
                int chunk, hipStream_t s) {
     const Plan p = fwd_plan(BH, Tlen, D, chunk, agg != nullptr);
-    if (p.NS > 1 && !agg) return MMF_ERR_ARG;
+    if (!agg && (p.NS > 1 || (fwd_takes_workspace(BH, Tlen, D, chunk) && BH * mmf_ceil_div(D, 64) < 128 && Tlen >= 2048))) return MMF_ERR_ARG;
     const T* xp = static_cast<const T*>(x);
     const T* gp = static_cast<const T*>(g);
     T* op = static_cast<T*>(o);

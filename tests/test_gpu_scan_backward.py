@@ -109,17 +109,19 @@ def test_a_zero_carry_survives_a_product_of_gates_that_overflows(dev, log):
 
 
 @pytest.mark.parametrize("bh,d,t", [(32, 64, 3072), (11, 130, 3101), (31, 64, 3072), (64, 64, 3100), (65, 33, 3073), (128, 64, 3361), (170, 40, 3080),
-                                    (171, 40, 3080)])
-@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-def test_scans_whose_columns_are_shared_by_workgroups(dev, bh, d, t, dtype):
-    """Long sequences around the numbers of columns (32, 64, 170) and the length from which 8 to 3 workgroups take turns on one column:
-    ragged columns, last rounds with fewer blocks than waves, an initial state; twice, on the same buffers.  The bound is that of the
-    cut sequences above; a 16-bit result is rounded once more (2^-8 of the value) and its gradients see a rounded o."""
+                                    (171, 40, 3080), (64, 64, 2050), (65, 64, 2050), (127, 33, 3071)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("log", [True, False])
+def test_scans_whose_columns_are_shared_by_workgroups(dev, bh, d, t, dtype, log):
+    """Long sequences around the numbers of columns (32, 64, 128, 170) and the lengths from which 8 to 3 workgroups take turns on one column or
+    columns are halved: ragged columns, last rounds with fewer blocks than waves, an initial state; log gates and linear ones; twice, on the same
+    buffers.  The bound is that of the cut sequences above; a 16-bit result is rounded once more (2^-8 of the value) and its gradients see a rounded o."""
     import matmulfreellm_amd as mm
     torch.manual_seed(bh + t)
-    g = torch.nn.functional.logsigmoid(torch.randn(1, bh, t, d, device=dev) + 2).to(dtype)
+    z = torch.randn(1, bh, t, d, device=dev) + 2
+    g = (torch.nn.functional.logsigmoid if log else torch.sigmoid)(z).to(dtype)
     x, do, h0 = torch.randn(1, bh, t, d, device=dev).to(dtype), torch.randn(1, bh, t, d, device=dev).to(dtype), torch.randn(1, bh, d, device=dev)
-    a, xd, dd = g[0].double().exp(), x[0].double(), do[0].double()
+    a, xd, dd = g[0].double().exp() if log else g[0].double(), x[0].double(), do[0].double()
     h, dh, hs, dhs = h0[0].double(), 0.0, [], []
     for i in range(t):
         h = a[:, i] * h + xd[:, i]
@@ -130,10 +132,11 @@ def test_scans_whose_columns_are_shared_by_workgroups(dev, bh, d, t, dtype):
         dh = dh * a[:, i]
     o = torch.stack(hs, 1)
     dx = torch.stack(dhs[::-1], 1)
-    want = [o, h, dx, dx * torch.cat([h0[0].double()[:, None], o[:, :-1]], 1) * a]
+    dg = dx * torch.cat([h0[0].double()[:, None], o[:, :-1]], 1)
+    want = [o, h, dx, dg * a if log else dg]
     mine = [v.clone().requires_grad_() for v in (x, g)]
     for _ in range(2):
-        got_o, last = mm.chunk_hgrn(*mine, h0, output_final_state=True)
+        got_o, last = (mm.chunk_hgrn if log else mm.fused_recurrent_hgrn)(*mine, h0, output_final_state=True)
         got = [got_o[0], last[0], *(v[0] for v in torch.autograd.grad(got_o, mine, do))]
         for name, p, r in zip(("o", "state", "dx", "dg"), got, want):
             err = ((p.detach().double() - r).abs().max() / r.abs().max()).item()
