@@ -219,9 +219,11 @@ __device__ __forceinline__ void compose_parts(float l, float P, int u, int ch, f
     }
 }
 
+// Registers: halved columns (LS = 2) have at most one workgroup a CU and use what they need; held to 128 for two of them, their 16-bit backward took 7.4
+// for 6.8 us (8 x 333 x 1024, linear gates), 9.5 for 8.8 (8 x 500 x 1024 fp16), 6.2 for 5.6 (2 x 333 x 1024).
 // -------------------------------------------------------------------------- forward, log gates
 template <typename T, bool AGG, int LS, bool NT, bool JOINT>
-__global__ __launch_bounds__(64 * kMaxWaves, 4) void hgrn_scan_fwd_kernel(const T* __restrict__ x, const T* __restrict__ g,
+__global__ __launch_bounds__(64 * kMaxWaves, LS == 2 ? 2 : 4) void hgrn_scan_fwd_kernel(const T* __restrict__ x, const T* __restrict__ g,
                                                                        const float* __restrict__ h0, T* __restrict__ o,
                                                                        float* __restrict__ ht, float* __restrict__ agg,
                                                                        int64_t Tlen, int64_t D, int64_t seg_len, int NS, Joint jt) {
@@ -353,7 +355,7 @@ __global__ __launch_bounds__(64 * kMaxWaves, 4) void hgrn_scan_fwd_kernel(const 
 
 // -------------------------------------------------------------------------- backward
 template <typename T, bool LOG, bool AGG, int LS, bool NT, bool JOINT>
-__global__ __launch_bounds__(64 * kMaxWaves, 4) void hgrn_scan_bwd_kernel(const T* __restrict__ g, const T* __restrict__ o,
+__global__ __launch_bounds__(64 * kMaxWaves, LS == 2 ? 2 : 4) void hgrn_scan_bwd_kernel(const T* __restrict__ g, const T* __restrict__ o,
                                                                        const T* __restrict__ dout, const float* __restrict__ h0,
                                                                        T* __restrict__ dx, T* __restrict__ dg,
                                                                        float* __restrict__ agg, int64_t Tlen, int64_t D,
