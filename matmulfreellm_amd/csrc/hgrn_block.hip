@@ -219,11 +219,11 @@ __device__ __forceinline__ void compose_parts(float l, float P, int u, int ch, f
     }
 }
 
-// Registers: halved columns (LS = 2) have at most one workgroup a CU and use what they need; held to 128 for two of them, their 16-bit backward took 7.4
-// for 6.8 us (8 x 333 x 1024, linear gates), 9.5 for 8.8 (8 x 500 x 1024 fp16), 6.2 for 5.6 (2 x 333 x 1024).
-// -------------------------------------------------------------------------- forward, log gates
-template <typename T, bool AGG, int LS, bool NT, bool JOINT>
-__global__ __launch_bounds__(64 * kMaxWaves, LS == 2 ? 2 : 4) void hgrn_scan_fwd_kernel(const T* __restrict__ x, const T* __restrict__ g,
+// ONE: halved columns that are not cut have at most one workgroup a CU and use the registers they need; held to 128 for two of them, their 16-bit backward
+// took 7.4 for 6.8 us (8 x 333 x 1024, linear gates), 9.5 for 8.8 (8 x 500 x 1024 fp16), 6.2 for 5.6 (2 x 333 x 1024).  (Cut ones have two, and took 11.4
+// for 10.2 us without the limit: 2 x 1000 x 1024.)
+template <typename T, bool AGG, int LS, bool NT, bool JOINT, bool ONE = false>
+__global__ __launch_bounds__(64 * kMaxWaves, ONE ? 2 : 4) void hgrn_scan_fwd_kernel(const T* __restrict__ x, const T* __restrict__ g,
                                                                        const float* __restrict__ h0, T* __restrict__ o,
                                                                        float* __restrict__ ht, float* __restrict__ agg,
                                                                        int64_t Tlen, int64_t D, int64_t seg_len, int NS, Joint jt) {
@@ -354,8 +354,8 @@ __global__ __launch_bounds__(64 * kMaxWaves, LS == 2 ? 2 : 4) void hgrn_scan_fwd
 }
 
 // -------------------------------------------------------------------------- backward
-template <typename T, bool LOG, bool AGG, int LS, bool NT, bool JOINT>
-__global__ __launch_bounds__(64 * kMaxWaves, LS == 2 ? 2 : 4) void hgrn_scan_bwd_kernel(const T* __restrict__ g, const T* __restrict__ o,
+template <typename T, bool LOG, bool AGG, int LS, bool NT, bool JOINT, bool ONE = false>
+__global__ __launch_bounds__(64 * kMaxWaves, ONE ? 2 : 4) void hgrn_scan_bwd_kernel(const T* __restrict__ g, const T* __restrict__ o,
                                                                        const T* __restrict__ dout, const float* __restrict__ h0,
                                                                        T* __restrict__ dx, T* __restrict__ dg,
                                                                        float* __restrict__ agg, int64_t Tlen, int64_t D,
@@ -594,7 +594,8 @@ int launch_fwd_ls(const Plan& p, const T* x, const T* g, const float* h0, T* o, 
             x, g, h0, o, ht, agg, Tlen, D, p.seg_len, p.NS, Joint{});
         MMF_CHECK_LAUNCH();
     }
-    hgrn_scan_fwd_kernel<T, false, LS, NT, false><<<dim3(gx, (unsigned)BH, (unsigned)p.NS), threads, 0, s>>>(
+    auto kern = LS == 2 && p.NS == 1 ? hgrn_scan_fwd_kernel<T, false, LS, NT, false, LS == 2> : hgrn_scan_fwd_kernel<T, false, LS, NT, false>;
+    kern<<<dim3(gx, (unsigned)BH, (unsigned)p.NS), threads, 0, s>>>(
         x, g, h0, o, ht, agg, Tlen, D, p.seg_len, p.NS, Joint{});
     MMF_CHECK_LAUNCH();
     return 0;
@@ -631,7 +632,8 @@ int launch_bwd_ls(const Plan& p, const T* g, const T* o, const T* dout, const fl
             g, o, dout, h0, dx, dg, agg, Tlen, D, p.seg_len, p.NS, Joint{});
         MMF_CHECK_LAUNCH();
     }
-    hgrn_scan_bwd_kernel<T, LOG, false, LS, NT, false><<<dim3(gx, (unsigned)BH, (unsigned)p.NS), threads, 0, s>>>(
+    auto kern = LS == 2 && p.NS == 1 ? hgrn_scan_bwd_kernel<T, LOG, false, LS, NT, false, LS == 2> : hgrn_scan_bwd_kernel<T, LOG, false, LS, NT, false>;
+    kern<<<dim3(gx, (unsigned)BH, (unsigned)p.NS), threads, 0, s>>>(
         g, o, dout, h0, dx, dg, agg, Tlen, D, p.seg_len, p.NS, Joint{});
     MMF_CHECK_LAUNCH();
     return 0;
