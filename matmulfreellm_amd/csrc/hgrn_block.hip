@@ -574,15 +574,17 @@ Joint joint_begin(const Plan& p, float* workspace, int64_t BH, int64_t D, hipStr
     return Joint{words, p.G, BH, joint_columns(BH, D)};
 }
 // Whether loads and stores are streamed past the caches.  Large tensors gain (40 x 2048 x 1024 bf16 118 + 198 -> 111 + 188 us, 128 x
-// 8192 x 128 156 + 259 -> 138 + 241, 5.8 TB/s), smaller ones that a consumer finds in the 256 MB last-level cache lose (16 x 777 x 1024
-// 14.5 + 27 against 18 + 29; even at 64 MB a tensor); in the second launch over time segments from 24 MB on (6000 x 64 columns 46 + 69 -> 45 + 62).
-// Shared columns the same, with what reads their results next (streamed / not, us): 64 x 5000 x 64 bf16 (39 MB) forward and a reader 51 / 47, backward
-// and a reader 71 / 65, forward and backward 86 / 77; 59 MB 72 / 67, 108 / 109, 133 / 131; 94 MB 113 / 118, 166 / 171, 200 / 204.
+// 8192 x 128 156 + 259 -> 138 + 241, 5.8 TB/s), smaller ones are found in the 256 MB last-level cache, by the scan or by what reads its results.  With
+// x and g (do) written just before and the results read next, 16 x T x 1024 bf16, forward, streamed / not: 40 MB a tensor 65 / 62 us, 64 116 / 116, 85
+// 157 / 151, 100 175 / 169, 130 222 / 223; backward 80 / 78, 123 / 126, 176 / 171, 198 / 198, 253 / 258; by itself on the same buffers the forward turns
+// at 85 MB (64 MB 40 / 36, 100 MB 63 / 67), the backward at 60 (64 MB 67 / 71).  In the second launch over time segments from 24 MB on (6000 x 64 columns
+// 46 + 69 -> 45 + 62).  Shared columns as whole ones (6 x 16384 x 1024 110 + 118 for 114 + 126; 4 x 5000 x 1024, 39 MB, forward and backward 86 / 77).
 // Only whole lines: where a row is no multiple of 128 bytes neighbouring columns share lines, which streamed are fetched twice (9 x 3068 x 1808
 // bf16, forward and backward, 312 us, streamed 418; columns shared by workgroups: 30 x 12073 x 144 288 and 406, 8 x 4049 x 720 148 and 169).
+constexpr int64_t kFwdStream = 90ll << 20, kBwdStream = 64ll << 20;      // bytes of a tensor
 bool whole_lines(int64_t row_bytes) { return row_bytes % 128 == 0; }
-bool streams(const Plan& p, int64_t row_bytes, int64_t rows) {
-    return whole_lines(row_bytes) && rows * row_bytes >= (p.NS > 1 ? 24ll << 20 : 64ll << 20);
+bool streams(const Plan& p, int64_t row_bytes, int64_t rows, int64_t from) {
+    return whole_lines(row_bytes) && rows * row_bytes >= (p.NS > 1 ? 24ll << 20 : from);
 }
 template <typename T, int LS, bool NT>
 int launch_fwd_ls(const Plan& p, const T* x, const T* g, const float* h0, T* o, float* ht, float* agg, int64_t BH, int64_t Tlen,
@@ -611,14 +613,14 @@ int launch_fwd(const void* x, const void* g, const float* h0, void* o, float* ht
     if (p.G > 1) {
         const Joint jt = joint_begin(p, agg, BH, D, s);
         MMF_CHECK_LAUNCH();
-        auto kern = streams(p, D * (int64_t)sizeof(T), BH * Tlen) ? hgrn_scan_fwd_kernel<T, false, 1, true, true> : hgrn_scan_fwd_kernel<T, false, 1, false, true>;
+        auto kern = streams(p, D * (int64_t)sizeof(T), BH * Tlen, kFwdStream) ? hgrn_scan_fwd_kernel<T, false, 1, true, true> : hgrn_scan_fwd_kernel<T, false, 1, false, true>;
         kern<<<(unsigned)joint_grid(p, BH, D), 64 * kMaxWaves, 0, s>>>(
             xp, gp, h0, op, ht, nullptr, Tlen, D, p.seg_len, 1, jt);
         MMF_CHECK_LAUNCH();
         return 0;
     }
     return p.LS == 2 ? launch_fwd_ls<T, 2, false>(p, xp, gp, h0, op, ht, agg, BH, Tlen, D, s)
-           : streams(p, D * (int64_t)sizeof(T), BH * Tlen) ? launch_fwd_ls<T, 1, true>(p, xp, gp, h0, op, ht, agg, BH, Tlen, D, s)
+           : streams(p, D * (int64_t)sizeof(T), BH * Tlen, kFwdStream) ? launch_fwd_ls<T, 1, true>(p, xp, gp, h0, op, ht, agg, BH, Tlen, D, s)
                                                         : launch_fwd_ls<T, 1, false>(p, xp, gp, h0, op, ht, agg, BH, Tlen, D, s);
 }
 
@@ -650,14 +652,14 @@ int launch_bwd(const void* g, const void* o, const void* dout, const float* h0, 
     if (p.G > 1) {
         const Joint jt = joint_begin(p, agg, BH, D, s);
         MMF_CHECK_LAUNCH();
-        auto kern = streams(p, D * (int64_t)sizeof(T), BH * Tlen) ? hgrn_scan_bwd_kernel<T, LOG, false, 1, true, true> : hgrn_scan_bwd_kernel<T, LOG, false, 1, false, true>;
+        auto kern = streams(p, D * (int64_t)sizeof(T), BH * Tlen, kBwdStream) ? hgrn_scan_bwd_kernel<T, LOG, false, 1, true, true> : hgrn_scan_bwd_kernel<T, LOG, false, 1, false, true>;
         kern<<<(unsigned)joint_grid(p, BH, D), 64 * kMaxWaves, 0, s>>>(
             gp, op, dp, h0, xp, yp, nullptr, Tlen, D, p.seg_len, 1, jt);
         MMF_CHECK_LAUNCH();
         return 0;
     }
     return p.LS == 2 ? launch_bwd_ls<T, LOG, 2, false>(p, gp, op, dp, h0, xp, yp, agg, BH, Tlen, D, s)
-           : streams(p, D * (int64_t)sizeof(T), BH * Tlen) ? launch_bwd_ls<T, LOG, 1, true>(p, gp, op, dp, h0, xp, yp, agg, BH, Tlen, D, s)
+           : streams(p, D * (int64_t)sizeof(T), BH * Tlen, kBwdStream) ? launch_bwd_ls<T, LOG, 1, true>(p, gp, op, dp, h0, xp, yp, agg, BH, Tlen, D, s)
                                                         : launch_bwd_ls<T, LOG, 1, false>(p, gp, op, dp, h0, xp, yp, agg, BH, Tlen, D, s);
 }
 
