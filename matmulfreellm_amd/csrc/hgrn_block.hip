@@ -557,6 +557,15 @@ int64_t joint_bytes(int64_t BH, int64_t D) { return joint_columns(BH, D) * 65 * 
 int64_t pair_bytes(const Plan& p, int64_t BH, int64_t D) {
     return p.G > 1 ? joint_bytes(BH, D) : p.NS > 1 ? BH * p.NS * 2 * D * (int64_t)sizeof(float) : 0;
 }
+// A forward of 65 to 128 columns up to 5120 steps whose three tensors fit the 256 MB last-level cache, or nearly, is faster halved than shared, as long as the halves'
+// half lines come together: rows of 512 channels and more (column_block), or of fp32, where a half is a line.  Halved / shared, us: 8 x 3072 x 1024 bf16
+// 29 / 35, 8 x 5000 x 1024 50 / 58, 5 x 5000 x 1024 37 / 37, 8 x 6500 x 1024 87 / 74; fp32 112 x 3072 x 64 49 / 55, 68 x 4000 x 64 39 / 45, 96 x 4000 x 64 (94 MB)
+// 56 / 58, 128 x 3072 x 64 (96 MB) 59 / 62, 112 x 4000 x 64 (109 MB) 69 / 68; bf16 128 x 4000 x 64, whose halves are apart, 53 / 42.  The backward's five tensors fit it up to half that
+// length: 8 x 3072 x 1024 44 / 49, 8 x 4000 x 1024 90 / 79, and with its forward just before 106 / 99.
+bool fwd_halves(int64_t BH, int64_t Tlen, int64_t D, int64_t elem) {
+    const int64_t columns = BH * mmf_ceil_div(D, 64);
+    return columns > 64 && columns <= 128 && Tlen <= 5120 && BH * Tlen * D * elem <= (96ll << 20) && (D % 512 == 0 || (elem == 4 && D % 32 == 0));
+}
 // The kernels address a block of at most 64 rows with 32-bit offsets and count blocks in an int.
 bool fits(int64_t Tlen, int64_t D, int dtype) {
     return Tlen / kBwdBlk < (1ll << 30) && 64 * D * (int64_t)(dtype == MMF_F32 ? 4 : 2) < (1ll << 31);
@@ -605,7 +614,7 @@ int launch_fwd_ls(const Plan& p, const T* x, const T* g, const float* h0, T* o, 
 template <typename T>
 int launch_fwd(const void* x, const void* g, const float* h0, void* o, float* ht, float* agg, int64_t BH, int64_t Tlen, int64_t D,
                int chunk, hipStream_t s) {
-    const Plan p = fwd_plan(BH, Tlen, D, chunk, agg != nullptr);
+    const Plan p = fwd_plan(BH, Tlen, D, chunk, agg && !fwd_halves(BH, Tlen, D, sizeof(T)));
     if (!agg && (p.NS > 1 || (fwd_takes_workspace(BH, Tlen, D, chunk) && BH * mmf_ceil_div(D, 64) < 128 && Tlen >= 2048))) return MMF_ERR_ARG;
     const T* xp = static_cast<const T*>(x);
     const T* gp = static_cast<const T*>(g);
