@@ -90,6 +90,8 @@ struct Lay16 {
 struct Acc16 { v4i g[4]; };                                      // a 32 x 32 block in Lay16
 __device__ __forceinline__ int acc_at(const v16i& a, int g, int t) { return a[4 * g + t]; }
 __device__ __forceinline__ int acc_at(const Acc16& a, int g, int t) { return a.g[g][t]; }
+__device__ __forceinline__ void acc_set(v16i& a, int g, int t, int v) { a[4 * g + t] = v; }
+__device__ __forceinline__ void acc_set(Acc16& a, int g, int t, int v) { a.g[g][t] = v; }
 
 // Epilogue of the tiled kernels.  The wave stages its 32 x (WN*32) outputs in a
 // private LDS region and writes them out as aligned 16-byte vectors (128-byte row segments).
@@ -196,8 +198,8 @@ __device__ __forceinline__ void mfma_epilogue(const MfmaArgs& p, A (&acc)[WM][WN
 // Lean epilogue of the common case (16-byte stores possible, no bias): the accumulators were
 // started at -qsum[m], so a value costs one convert and two multiplies; lane-constant parts of the
 // store addresses are computed once; interior tiles skip the bounds tests.
-template <bool STREAM, typename T, int WM, int WN>
-__device__ __forceinline__ void mfma_epilogue_fast(const MfmaArgs& p, Acc16 (&acc)[WM][WN], const EpiScales<Lay16, WM, WN>& sc,
+template <bool STREAM, typename T, class L, class A, int WM, int WN>
+__device__ __forceinline__ void mfma_epilogue_fast(const MfmaArgs& p, A (&acc)[WM][WN], const EpiScales<L, WM, WN>& sc,
                                                    unsigned char* smem, int lane, int wave, int wm, int64_t mb0, int64_t nb0) {
     const T* addend = static_cast<const T*>(p.addend);
     T* out = static_cast<T*>(p.out);
@@ -211,7 +213,7 @@ __device__ __forceinline__ void mfma_epilogue_fast(const MfmaArgs& p, Acc16 (&ac
     const bool interior = m_first + WM * 32 <= p.M && n_first + WN * 32 <= p.N;
     const int64_t n = n_first + cc * (16 / E);
     const int64_t lane_off = (m_first + rsub) * p.ldo + n;         // element offset of this lane's first chunk
-    unsigned char* wr = stage + (lane & 15) * RS + 4 * (lane >> 4) * E;
+    unsigned char* wr = stage + L::row(lane, 0) * RS + L::col(lane, 0) * E;
     const unsigned char* rd = stage + rsub * RS + cc * 16;
 #pragma unroll
     for (int i = 0; i < WM; ++i) {
@@ -219,11 +221,11 @@ __device__ __forceinline__ void mfma_epilogue_fast(const MfmaArgs& p, Acc16 (&ac
         for (int j = 0; j < WN; ++j)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                const float dq = sc.dq[i][g >> 1];
+                const float dq = sc.dq[i][L::half(g)];
                 float o[4];
 #pragma unroll
                 for (int t = 0; t < 4; ++t) o[t] = __fmul_rn(__fmul_rn((float)acc_at(acc[i][j], g, t), dq), sc.wdq[j]);
-                unsigned char* w = wr + (g >> 1) * 16 * RS + (j * 32 + 16 * (g & 1)) * E;
+                unsigned char* w = wr + L::row(0, g) * RS + (j * 32 + L::col(0, g)) * E;
                 if constexpr (E == 2) *reinterpret_cast<uint2*>(w) = make_uint2(pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3]));
                 else *reinterpret_cast<float4*>(w) = make_float4(o[0], o[1], o[2], o[3]);
             }
@@ -260,8 +262,8 @@ __device__ __forceinline__ void mfma_epilogue_fast(const MfmaArgs& p, Acc16 (&ac
 // Same conditions as the lean epilogue (accumulators started at -qsum, 16-byte stores).  The activation was most of what this
 // launch took beyond the plain one: 16384 x 2048 -> 11264 in bf16 356 us with the exact exp and divide, 322 with mmf_swiglu_n (the plain
 // contraction of as many columns about 300); 2002 rows 57 and 54; fp16, whose elements fall back eight times as often, 1377 rows 36.8 and 36.3.
-template <typename T, int WM>
-__device__ __forceinline__ void mfma_epilogue_swiglu(const MfmaArgs& p, Acc16 (&acc)[WM][2], const EpiScales<Lay16, WM, 2>& sc,
+template <typename T, class L, class A, int WM>
+__device__ __forceinline__ void mfma_epilogue_swiglu(const MfmaArgs& p, A (&acc)[WM][2], const EpiScales<L, WM, 2>& sc,
                                                      unsigned char* smem, int lane, int wave, int wm, int64_t mb0, int64_t nbg) {
     T* out = static_cast<T*>(p.out);
     constexpr int E = sizeof(T);
@@ -275,13 +277,13 @@ __device__ __forceinline__ void mfma_epilogue_swiglu(const MfmaArgs& p, Acc16 (&
     const bool interior = m_first + WM * 32 <= p.M && n_first + 32 <= nseg;
     const int64_t n = n_first + cc * (16 / E);
     const int64_t lane_off = (m_first + rsub) * p.ldo + n;
-    unsigned char* wr = stage + (lane & 15) * RS + 4 * (lane >> 4) * E;
+    unsigned char* wr = stage + L::row(lane, 0) * RS + L::col(lane, 0) * E;
     const unsigned char* rd = stage + rsub * RS + cc * 16;
 #pragma unroll
     for (int i = 0; i < WM; ++i) {
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            const float dq = sc.dq[i][g >> 1];
+            const float dq = sc.dq[i][L::half(g)];
             float gv[4], uv[4], o[4];
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
@@ -289,7 +291,7 @@ __device__ __forceinline__ void mfma_epilogue_swiglu(const MfmaArgs& p, Acc16 (&
                 uv[t] = mmf_round_to<T>(__fmul_rn(__fmul_rn((float)acc_at(acc[i][1], g, t), dq), sc.wdq[1]));
             }
             mmf_swiglu_n<T, 4>(gv, uv, o);
-            unsigned char* w = wr + (g >> 1) * 16 * RS + 16 * (g & 1) * E;
+            unsigned char* w = wr + L::row(0, g) * RS + L::col(0, g) * E;
             if constexpr (E == 2) *reinterpret_cast<uint2*>(w) = make_uint2(pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3]));
             else *reinterpret_cast<float4*>(w) = make_float4(o[0], o[1], o[2], o[3]);
         }
@@ -489,11 +491,16 @@ constexpr int dma3_work_bytes() {
 // 3.6 P op/s before the clock gives way, v_mfma_i32_16x16x64_i8 4.8, which is why the products are of the second form although there are twice as
 // many of them.  Measured with 32x32x32, then with
 // 16x16x64, us: 16384 x 2048 -> 6144 204 and 172-180 (2.4 P op/s), x 5632 -> 2048 147 and 126-130 (3.0), x 2048 -> 11264 with swiglu 363-369 and
-// 316-325; 4096 x 2048 -> 11264 83 and 73, 2002 rows 44 and 40.  On at most one tile per CU what counts is each wave's chain of instructions: there both
-// forms take the same time within 5 % (5632 -> 2048 split: 2002 rows 24 and 23.4, 1377 rows 21.4 and 21.8).
-template <typename T, int WGM, int WGN, int WM, int WN, int KS, int FAST, bool SWI = false>
+// 316-325; 4096 x 2048 -> 11264 83 and 73, 2002 rows 44 and 40.
+// W32: the first form, for at most one split tile per CU: what counts there is each wave's chain of instructions, which has half as many products and no
+// exchange of half-waves, and in front of it no rows' scales to pass through LDS.  us, 32x32x32 and 16x16x64: 5632 -> 2048, 1377 rows 21.6 and 23.1, 700 rows
+// 19.8 and 21.3, 2002 rows (a tile for every CU) 24.3 and 24.1, 2500 (on some two) 35.4 and 33.3; 2048 -> 6144, 460 rows 11.8 and 12.4; 1024 -> 1024, 128
+// to 4096 rows 7.4 to 9.2 and 8.0 to 9.7.  Whole tiles, one per CU, differ by 2 % either way.
+template <typename T, int WGM, int WGN, int WM, int WN, int KS, int FAST, bool SWI = false, bool W32 = false>
 __global__ __launch_bounds__(64 * WGM * WGN * KS, (WM * WN <= 4 ? 4 : 1))   // small wave tiles: 4 waves per SIMD = two workgroups per CU
 void bitlinear_mfma_dma3_kernel(MfmaArgs p) {
+    using L = typename std::conditional<W32, Lay32, Lay16>::type;
+    using Acc = typename std::conditional<W32, v16i, Acc16>::type;
     constexpr int NT = WGM * WGN;                  // waves that cover the tile once
     constexpr int NW = NT * KS;
     constexpr int BMB = WGM * WM;
@@ -544,11 +551,12 @@ void bitlinear_mfma_dma3_kernel(MfmaArgs p) {
     static_assert(BMB * 32 <= 64 * NW, "a row's scale and code sum per thread");
     float my_dq = 0.0f;                            // on their way while the first transfers are requested; into LDS behind the first wait
     int my_qs = 0;
-    if (const int64_t m = mb0 * 32 + threadIdx.x; threadIdx.x < BMB * 32 && m < p.M) {
+    EpiScales<L, WM, WN> sc;
+    if constexpr (W32) mfma_prefetch_scales<L, WM, WN>(p, sc, lane, wm, mb0, nb0);   // one row a lane: into registers
+    else if (const int64_t m = mb0 * 32 + threadIdx.x; threadIdx.x < BMB * 32 && m < p.M) {
         my_dq = p.deq[m];
         my_qs = p.qsum[m];
     }
-    EpiScales<Lay16, WM, WN> sc;
 #pragma unroll
     for (int j = 0; j < WN; ++j)   // seg_rows is a multiple of 32: one weight scale per n-block
         sc.wdq[j] = p.wdeq[(uint32_t)(nblock(j) * 32) / (uint32_t)p.seg_rows];
@@ -565,7 +573,7 @@ void bitlinear_mfma_dma3_kernel(MfmaArgs p) {
             mfma_dma_1k(g, (uint32_t)lane * 16u, smem + boff + w * 1024);
         }
     };
-    const uint32_t boff = (uint32_t)(((lane >> 4) & 1) * 32 + (lane >> 5) * 16 + (lane & 15)) * 16u;
+    const uint32_t boff = W32 ? (uint32_t)lane * 16u : (uint32_t)(((lane >> 4) & 1) * 32 + (lane >> 5) * 16 + (lane & 15)) * 16u;
     auto load_b = [&](int kb, uint4 (&dst)[WN]) {                 // unconditional: the barrier's vmcnt counts on WN loads
 #pragma unroll
         for (int j = 0; j < WN; ++j) {
@@ -607,108 +615,155 @@ void bitlinear_mfma_dma3_kernel(MfmaArgs p) {
     load_b(0, bset0);
     load_b(1, bset1);
     __builtin_amdgcn_s_waitcnt(0x0F70);            // vmcnt(0): this wave's pieces of k-blocks 0 and 1 have landed
-    if (threadIdx.x < BMB * 32) {
+    if (!W32 && threadIdx.x < BMB * 32) {
         row_dq[threadIdx.x] = my_dq;
         row_qs[threadIdx.x] = my_qs;
     }
     __syncthreads();
 
-    arrange_b(bset0);
+    if constexpr (!W32) arrange_b(bset0);
 
     // FAST: a lane's accumulators start at -qsum of their row (read for every group and masked: as a choice the compiler branches around
     // a read of its own for each of the accumulators, 2 us of a launch)
-    Acc16 acc[WM][WN];
+    Acc acc[WM][WN];
 #pragma unroll
     for (int i = 0; i < WM; ++i)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            const int init = FAST ? -row_qs[(wm * WM + i) * 32 + Lay16::row(lane, g)] & (KS == 1 || wk == 0 ? -1 : 0) : 0;
+            const int qs = W32 ? sc.qs[i][0] : FAST ? row_qs[(wm * WM + i) * 32 + L::row(lane, g)] : 0;
+            const int init = FAST ? -qs & (KS == 1 || wk == 0 ? -1 : 0) : 0;
 #pragma unroll
             for (int j = 0; j < WN; ++j)
 #pragma unroll
-                for (int t = 0; t < 4; ++t) acc[i][j].g[g][t] = init;
+                for (int t = 0; t < 4; ++t) acc_set(acc[i][j], g, t, init);
         }
-    // A 16 x 64 fragment: lane l reads input group l / 16 of row l % 16
-    const int aoff = (wk * BMB + wm * WM) * CH + (lane >> 4) * 512 + (lane & 15) * 16;
     int cur = 0, nxt = BUF, fre = 2 * BUF;         // byte offsets of the buffers of k-blocks s, s+1, s+2
-    constexpr int MF = 2 * WM, NF = 2 * WN;        // 16-row and 16-column fragments of the wave tile
-    auto read_a = [&](int off, int f) { return *reinterpret_cast<const v4i*>(smem + off + aoff + (f >> 1) * CH + (f & 1) * 256); };
-    // word of the arranged set for step q of its k-block, column fragment c
-    auto word = [](const uint4 (&s)[WN], int q, int c) {
-        const uint4 w = s[c >> 1];
-        return q == 0 ? ((c & 1) == 0 ? w.x : w.y) : (c & 1) == 0 ? w.z : w.w;
+    auto k_loop = [&](auto&& kblock) __attribute__((always_inline)) {
+        int kb = 0;
+        for (;;) {                                 // left in the middle: no copy of a k-block for the remainder, whose code a launch would fetch cold
+            kblock(kb, bset0, bset1, bset2);
+            if (++kb >= KBs) break;
+            kblock(kb, bset1, bset2, bset0);
+            if (++kb >= KBs) break;
+            kblock(kb, bset2, bset0, bset1);
+            if (++kb >= KBs) break;
+        }
     };
-    v4i af[2], bf[NF];
-    af[0] = read_a(cur, 0);
+    if constexpr (W32) {
+        // One k-block in four steps of 32; the requests go out right behind the barrier, and a step's weights are expanded under the MFMAs of the
+        // step before, columns outermost: once the MFMAs of a column are issued, its registers take the next step's.
+        const int aoff = (wk * BMB + wm * WM) * CH + lane * 16;
+        v4i af[2][WM], bf[WN];
 #pragma unroll
-    for (int c = 0; c < NF; ++c) bf[c] = expand(word(bset0, 0, c));
-
-    // One k-block in two steps of 64: contracts with the set `bcur`, requests k-block kb + 2 into `bfar`.  Activation rows outermost, the next
-    // row's fragment on its way from LDS under this row's MFMAs; under the last row every weight fragment is replaced by the next step's
-    // as soon as its MFMA has been issued.  (A step's weights and two row fragments: 24 registers, which is what 64 accumulators, three
-    // sets in flight and addresses leave of 128.  Columns outermost, two more weight fragments expanded a row earlier, or four and eight row fragments
-    // ahead, where one workgroup per CU leaves the registers, all measured the same or slower.)
-    auto kblock = [&](int kb, const uint4 (&bcur)[WN], uint4 (&bnxt)[WN], uint4 (&bfar)[WN]) {
+        for (int i = 0; i < WM; ++i) af[0][i] = *reinterpret_cast<const v4i*>(smem + cur + aoff + i * CH);
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            if (q == 1) {
-                // Everything requested one k-block ago -- this wave's pieces of A k-block kb+1 and the weights of kb+1 --
-                // has to be here now.  The wait is for ALL vector-memory traffic: a transfer into LDS and an ordinary load
-                // do not complete in the order they were issued (a count that leaves the younger weight loads in flight let
-                // warm weight loads overtake a cold A transfer and gave wrong sums), so the next requests go out after
-                // the barrier, between the rows' MFMAs (ahead of them all waves' address arithmetic left the matrix pipe idle: 0.64 us a k-block
-                // with one workgroup per CU, 0.61 so), and have the rest of the k-block and half the next to land.  The weights that have
-                // come in are arranged ahead of them: the compiler waits for them by a count that does not know of the transfer, which behind it
-                // would be a wait for the transfer.
-                mfma_barrier_vm<0>();
+        for (int j = 0; j < WN; ++j) bf[j] = expand(bset0[j].x);
+        k_loop([&](int kb, const uint4 (&bcur)[WN], const uint4 (&bnxt)[WN], uint4 (&bfar)[WN]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) {
+                if (ks == 2) {                                     // (the wait of the other form below)
+                    mfma_barrier_vm<0>();
+                    dma_block(kb + 2, fre);
+                    load_b(kb + 2, bfar);
+                }
+                const unsigned char* nsrc = ks < 3 ? smem + cur + aoff + (ks + 1) * 1024 : smem + nxt + aoff;
+#pragma unroll
+                for (int i = 0; i < WM; ++i) af[(ks + 1) & 1][i] = *reinterpret_cast<const v4i*>(nsrc + i * CH);
+                v4i bn[WN];
+#pragma unroll
+                for (int j = 0; j < WN; ++j) {
+#pragma unroll
+                    for (int i = 0; i < WM; ++i) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf[j], af[ks & 1][i], acc[i][j], 0, 0, 0);
+                    bn[j] = expand(ks == 0 ? bcur[j].y : ks == 1 ? bcur[j].z : ks == 2 ? bcur[j].w : bnxt[j].x);
+                }
+                __builtin_amdgcn_sched_group_barrier(0x100, WM, 0);
+#pragma unroll
+                for (int j = 0; j < WN; ++j) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, WM, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);
+                }
+#pragma unroll
+                for (int j = 0; j < WN; ++j) bf[j] = bn[j];
+                __builtin_amdgcn_sched_barrier(0);
             }
-            __builtin_amdgcn_sched_barrier(0);
+            const int t = cur; cur = nxt; nxt = fre; fre = t;
+        });
+    } else {
+        // A 16 x 64 fragment: lane l reads input group l / 16 of row l % 16
+        const int aoff = (wk * BMB + wm * WM) * CH + (lane >> 4) * 512 + (lane & 15) * 16;
+        constexpr int MF = 2 * WM, NF = 2 * WN;        // 16-row and 16-column fragments of the wave tile
+        auto read_a = [&](int off, int f) { return *reinterpret_cast<const v4i*>(smem + off + aoff + (f >> 1) * CH + (f & 1) * 256); };
+        // word of the arranged set for step q of its k-block, column fragment c
+        auto word = [](const uint4 (&s)[WN], int q, int c) {
+            const uint4 w = s[c >> 1];
+            return q == 0 ? ((c & 1) == 0 ? w.x : w.y) : (c & 1) == 0 ? w.z : w.w;
+        };
+        v4i af[2], bf[NF];
+        af[0] = read_a(cur, 0);
 #pragma unroll
-            for (int f = 0; f < MF; ++f) {
-                const int t = q * MF + f + 1;                      // of the 2 MF fragments of this k-block, then the next one's first
-                af[t & 1] = t < 2 * MF ? read_a(cur + t / MF * 2048, t % MF) : read_a(nxt, 0);
+        for (int c = 0; c < NF; ++c) bf[c] = expand(word(bset0, 0, c));
+
+        // One k-block in two steps of 64: contracts with the set `bcur`, requests k-block kb + 2 into `bfar`.  Activation rows outermost, the next
+        // row's fragment on its way from LDS under this row's MFMAs; under the last row every weight fragment is replaced by the next step's
+        // as soon as its MFMA has been issued.  (A step's weights and two row fragments: 24 registers, which is what 64 accumulators, three
+        // sets in flight and addresses leave of 128.  Columns outermost, two more weight fragments expanded a row earlier, or four and eight row fragments
+        // ahead, where one workgroup per CU leaves the registers, all measured the same or slower.)
+        auto kblock = [&](int kb, const uint4 (&bcur)[WN], uint4 (&bnxt)[WN], uint4 (&bfar)[WN]) {
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                if (q == 1) {
+                    // Everything requested one k-block ago -- this wave's pieces of A k-block kb+1 and the weights of kb+1 --
+                    // has to be here now.  The wait is for ALL vector-memory traffic: a transfer into LDS and an ordinary load
+                    // do not complete in the order they were issued (a count that leaves the younger weight loads in flight let
+                    // warm weight loads overtake a cold A transfer and gave wrong sums), so the next requests go out after
+                    // the barrier, between the rows' MFMAs (ahead of them all waves' address arithmetic left the matrix pipe idle: 0.64 us a k-block
+                    // with one workgroup per CU, 0.61 so), and have the rest of the k-block and half the next to land.  The weights that have
+                    // come in are arranged ahead of them: the compiler waits for them by a count that does not know of the transfer, which behind it
+                    // would be a wait for the transfer.
+                    mfma_barrier_vm<0>();
+                }
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int c = 0; c < NF; ++c) {
-                    v4i& d = acc[f >> 1][c >> 1].g[2 * (f & 1) + (c & 1)];
-                    if (f == 0 && c == 0) mfma_16x16x64<true>(d, bf[c], af[f & 1]);
-                    else mfma_16x16x64<false>(d, bf[c], af[f & 1]);
-                    if (f == MF - 1) bf[c] = expand(q == 0 ? word(bcur, 1, c) : word(bnxt, 0, c));
+                for (int f = 0; f < MF; ++f) {
+                    const int t = q * MF + f + 1;                      // of the 2 MF fragments of this k-block, then the next one's first
+                    af[t & 1] = t < 2 * MF ? read_a(cur + t / MF * 2048, t % MF) : read_a(nxt, 0);
                     __builtin_amdgcn_sched_barrier(0);
-                }
-                if (q == 1) {
-                    if (f == 0) arrange_b(bnxt);
-                    if (f == 1 || MF == 1) dma_block(kb + 2, fre);
-                    if (f == (MF > 2 ? 2 : MF - 1)) load_b(kb + 2, bfar);
-                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int c = 0; c < NF; ++c) {
+                        v4i& d = acc[f >> 1][c >> 1].g[2 * (f & 1) + (c & 1)];
+                        if (f == 0 && c == 0) mfma_16x16x64<true>(d, bf[c], af[f & 1]);
+                        else mfma_16x16x64<false>(d, bf[c], af[f & 1]);
+                        if (f == MF - 1) bf[c] = expand(q == 0 ? word(bcur, 1, c) : word(bnxt, 0, c));
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    if (q == 1) {
+                        if (f == 0) arrange_b(bnxt);
+                        if (f == 1 || MF == 1) dma_block(kb + 2, fre);
+                        if (f == (MF > 2 ? 2 : MF - 1)) load_b(kb + 2, bfar);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
                 }
             }
-        }
-        const int t = cur; cur = nxt; nxt = fre; fre = t;
-    };
-    int kb = 0;
-    for (;;) {                                     // left in the middle: no copy of a k-block for the remainder, whose code a launch would fetch cold
-        kblock(kb, bset0, bset1, bset2);
-        if (++kb >= KBs) break;
-        kblock(kb, bset1, bset2, bset0);
-        if (++kb >= KBs) break;
-        kblock(kb, bset2, bset0, bset1);
-        if (++kb >= KBs) break;
+            const int t = cur; cur = nxt; nxt = fre; fre = t;
+        };
+        k_loop(kblock);
+        mfma_done(acc);
     }
-    mfma_done(acc);
     __builtin_amdgcn_s_waitcnt(0x0F70);            // the trailing DMA must not land in the epilogue's staging area
     __syncthreads();
+    if constexpr (!W32) {
 #pragma unroll
-    for (int i = 0; i < WM; ++i)
+        for (int i = 0; i < WM; ++i)
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            sc.dq[i][h] = row_dq[(wm * WM + i) * 32 + Lay16::row(lane, 2 * h)];
-            sc.qs[i][h] = FAST ? 0 : row_qs[(wm * WM + i) * 32 + Lay16::row(lane, 2 * h)];
-        }
+            for (int h = 0; h < 2; ++h) {
+                sc.dq[i][h] = row_dq[(wm * WM + i) * 32 + L::row(lane, 2 * h)];
+                sc.qs[i][h] = FAST ? 0 : row_qs[(wm * WM + i) * 32 + L::row(lane, 2 * h)];
+            }
+    }
     if constexpr (KS == 1) {
-        if constexpr (SWI) mfma_epilogue_swiglu<T, WM>(p, acc, sc, smem, lane, wave, wm, mb0, nb0);
-        else if constexpr (FAST) mfma_epilogue_fast<FAST == 2, T, WM, WN>(p, acc, sc, smem, lane, wave, wm, mb0, nb0);
-        else mfma_epilogue<T, Lay16>(p, acc, sc, smem, lane, wave, wm, mb0, nb0);
+        if constexpr (SWI) mfma_epilogue_swiglu<T, L>(p, acc, sc, smem, lane, wave, wm, mb0, nb0);
+        else if constexpr (FAST) mfma_epilogue_fast<FAST == 2, T, L>(p, acc, sc, smem, lane, wave, wm, mb0, nb0);
+        else mfma_epilogue<T, L>(p, acc, sc, smem, lane, wave, wm, mb0, nb0);
     } else {
         // group g finishes row block g of the wave tile: it takes the other groups' partial sums of that block
         static_assert(KS == WM, "a row block of the wave tile per group");
@@ -721,17 +776,17 @@ void bitlinear_mfma_dma3_kernel(MfmaArgs p) {
 #pragma unroll
                 for (int j = 0; j < WN; ++j)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) dst[(j * 16 + r) * 64] = acc[i][j].g[r >> 2][r & 3];
+                    for (int r = 0; r < 16; ++r) dst[(j * 16 + r) * 64] = acc_at(acc[i][j], r >> 2, r & 3);
             }
         }
         __syncthreads();
-        Acc16 mine[1][WN];
-        EpiScales<Lay16, 1, WN> sc1;
+        Acc mine[1][WN];
+        EpiScales<L, 1, WN> sc1;
 #pragma unroll
         for (int i = 0; i < WM; ++i) {
             if (i == wk) {
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
+                for (int h = 0; h < L::RH; ++h) {
                     sc1.dq[0][h] = sc.dq[i][h];
                     sc1.qs[0][h] = sc.qs[i][h];
                 }
@@ -748,14 +803,14 @@ void bitlinear_mfma_dma3_kernel(MfmaArgs p) {
 #pragma unroll
                 for (int j = 0; j < WN; ++j)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) mine[0][j].g[r >> 2][r & 3] += src[(j * 16 + r) * 64];
+                    for (int r = 0; r < 16; ++r) acc_set(mine[0][j], r >> 2, r & 3, acc_at(mine[0][j], r >> 2, r & 3) + src[(j * 16 + r) * 64]);
             }
         }
         __syncthreads();                                         // the exchange area becomes the epilogue's staging area
         const int wm1 = wm * WM + wk;
-        if constexpr (SWI) mfma_epilogue_swiglu<T, 1>(p, mine, sc1, smem, lane, wave, wm1, mb0, nb0);
-        else if constexpr (FAST) mfma_epilogue_fast<FAST == 2, T, 1, WN>(p, mine, sc1, smem, lane, wave, wm1, mb0, nb0);
-        else mfma_epilogue<T, Lay16>(p, mine, sc1, smem, lane, wave, wm1, mb0, nb0);
+        if constexpr (SWI) mfma_epilogue_swiglu<T, L>(p, mine, sc1, smem, lane, wave, wm1, mb0, nb0);
+        else if constexpr (FAST) mfma_epilogue_fast<FAST == 2, T, L>(p, mine, sc1, smem, lane, wave, wm1, mb0, nb0);
+        else mfma_epilogue<T, L>(p, mine, sc1, smem, lane, wave, wm1, mb0, nb0);
     }
     if (p.clocks && threadIdx.x == 0 && (int64_t)blockIdx.x < p.clock_cap) {
         p.clocks[2 * blockIdx.x] = __builtin_amdgcn_s_memtime() - clk0;
@@ -800,6 +855,14 @@ int launch_mfma_dma3(MfmaArgs a, hipStream_t s) {
         if (!a.vec_store || a.bias) kern = bitlinear_mfma_dma3_kernel<T, WGM, WGN, WM, WN, KS, 0, false>;
         else if constexpr (sizeof(T) == 2) {
             if (a.M * a.N * 2 >= (20 << 20)) kern = bitlinear_mfma_dma3_kernel<T, WGM, WGN, WM, WN, KS, 2, false>;
+        }
+    }
+    if constexpr (KS > 1) {
+        if ((int64_t)a.tiles_m * a.tiles_n <= 256) {             // (too small an output to be streamed)
+            kern = bitlinear_mfma_dma3_kernel<T, WGM, WGN, WM, WN, KS, 1, SWI, true>;
+            if constexpr (!SWI) {
+                if (!a.vec_store || a.bias) kern = bitlinear_mfma_dma3_kernel<T, WGM, WGN, WM, WN, KS, 0, false, true>;
+            }
         }
     }
     if (lds > 48 * 1024) {
@@ -981,7 +1044,7 @@ int launch_mfma(MfmaArgs a, hipStream_t s) {
 
 // Which kernel is the fastest, from its measured time on MI355X (us; N from 1024 to 11264, K from 1024 to 9216, M from 77 to 9600):
 //   weight stream  3 + 0.7 ns per output block + 0.18 ns per output block and k-block, as long as the row fits its LDS;
-//   split tiles    (64 x 256, two groups of waves on every second k-block) at most one tile per CU: a chain of 0.31 us per k-block, and
+//   split tiles    (64 x 256, two groups of waves on every second k-block) at most one tile per CU: a chain of 0.29 us per k-block, and
 //                  what a fuller chip adds.  At most two per CU run side by side and share it: one time, whatever their number.  Beyond
 //                  that, 3.9 + 0.295 us per k-block for every 256;
 //   tiles          (64 x 512) at most one per CU: 4.4 + 0.58 us per k-block and what a fuller chip adds; beyond, 4.4 + 0.62 per 256.
@@ -1000,7 +1063,7 @@ inline MfmaPick mfma_pick(const MfmaArgs& a) {
     const double t_tiles = full <= 256 ? 4.4 + 0.58 * kb + (double)full / 256.0 * (1.0 + 0.18 * kb) : (double)mmf_ceil_div(full, 256) * (4.4 + 0.62 * kb);
     double t_split = 1e30;
     if (KB % 2 == 0)
-        t_split = half <= 256   ? 5.2 + 0.31 * kb + (double)half / 256.0 * (0.75 + 0.107 * kb)
+        t_split = half <= 256   ? 4.4 + 0.29 * kb + (double)half / 256.0 * (1.0 + 0.1 * kb)
                   : half <= 512 ? 8.5 + 0.59 * kb
                                 : (double)mmf_ceil_div(half, 256) * (3.9 + 0.295 * kb);
     if (a.Kp <= 8192 && a.M <= 65535 * 32 && (a.M <= 64 || (t_stream <= t_split && t_stream <= t_tiles))) return MfmaPick::kStream;

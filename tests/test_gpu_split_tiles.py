@@ -31,6 +31,21 @@ def test_every_end_of_the_k_loop_is_exact(dev, blocks):
             assert torch.equal(F.bitlinear_mfma(q[0], deq[0], qsum[0], pw, m, torch.bfloat16, config=config).cpu(), want), (m, n, config)
 
 
+@pytest.mark.parametrize("k", [256, 512, 765, 1021, 2048])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_split_tiles_on_both_sides_of_one_per_cu(dev, k, dtype):
+    """256 and 272 split tiles (the two forms of the product), 2 to 16 k-blocks, the lean and the general epilogue, an addend, the swiglu form."""
+    for m, n in ((1009, 4096), (1009, 4093), (1025, 4096), (1025, 4093)):
+        F, lib, pw, q, codes, deq, qsum = operands(dev, m, k, n, seed=k)
+        want = F.bitlinear_mfma(q[0], deq[0], qsum[0], pw, m, dtype, config=16)
+        assert torch.equal(F.bitlinear_mfma(q[0], deq[0], qsum[0], pw, m, dtype, config=18), want), (m, n)
+        if n % 32 == 0:
+            add = torch.randn(m, n, device=dev).to(dtype)
+            assert torch.equal(F.bitlinear_mfma(q[0], deq[0], qsum[0], pw, m, dtype, config=18, addend=add),
+                               F.bitlinear_mfma(q[0], deq[0], qsum[0], pw, m, dtype, config=16, addend=add)), (m, n)
+            assert torch.equal(F.bitlinear_mfma_swiglu(q[0], deq[0], qsum[0], pw, m, dtype), F.swiglu(want[:, :n // 2], want[:, n // 2:])), (m, n)
+
+
 def test_odd_number_of_k_blocks_is_refused(dev):
     F, lib, pw, q, codes, deq, qsum = operands(dev, 70, 384, 256)
     with pytest.raises(RuntimeError):
