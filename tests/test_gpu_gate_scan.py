@@ -1,5 +1,7 @@
 """Gate math and recurrence in one launch against the two launches it stands for (bit for bit): around the lengths of its tiles for each
 width of a workgroup's columns, ragged columns, masks, lower bounds, states, strided operands."""
+import itertools
+
 import pytest
 import torch
 
@@ -8,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("b,d", [(1, 16), (2, 40), (3, 1024), (3, 4096), (5, 2080), (9, 4096)])
 @pytest.mark.parametrize("t", [1, 9, 10, 29, 30, 31, 60, 61, 119, 120, 121, 240, 367, 512, 513])
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_gate_scan_equals_gate_then_scan(dev, b, d, t, dtype):
     import matmulfreellm_amd.functional as F
     torch.manual_seed(t)
@@ -16,7 +18,7 @@ def test_gate_scan_equals_gate_then_scan(dev, b, d, t, dtype):
     i, f = ifg[:, :d], ifg[:, d:2 * d]
     lb, h0 = torch.rand(d, device=dev) * 0.5, torch.randn(b, 1, d, device=dev)
     mask = (torch.rand(b * t, device=dev) > 0.2).to(torch.uint8)
-    for use_lb, use_mask, use_h0 in ((True, True, True), (False, False, False)):
+    for use_lb, use_mask, use_h0 in itertools.product((True, False), repeat=3):
         x, g = F.hgrn_gate(i, f, lb if use_lb else None, mask if use_mask else None)
         want, last = F.hgrn_recurrent(x.view(b, 1, t, d), g.view(b, 1, t, d), h0 if use_h0 else None, True)
         o, ht = torch.empty(b * t, d, dtype=dtype, device=dev), torch.empty(b, d, device=dev)
