@@ -352,8 +352,9 @@ __device__ __forceinline__ float mmf_round_if_sure(float v, float slack, bool& r
     }
 }
 // What it costs: a wave in which one lane of one element falls back runs the definition's code once more, 1 to 2 % of the waves per
-// element in bf16 and 8 to 12 % in fp16.  Where waves wait for each other the slowest one counts, so kernels whose time is a
-// dependent chain keep the definitions (NEAR = false): the o_proj GEMV of five rows 3.8 us with them, 4.3 with the near form.
+// element in bf16 and 8 to 12 % in fp16.  Where waves wait for each other, or a launch has no more workgroups than there are CUs, the slowest one
+// counts: such kernels keep the definitions (the decode kernels call them directly, the row kernels choose with NEAR by their rows): the
+// o_proj GEMV of five rows 3.8 us with them, 4.3 with the near form.
 // o = T((g * u) / (1 + exp(-g))); T = float: the definition, nothing to round.
 __device__ __forceinline__ float mmf_swiglu_definition(float g, float u) {
     return __fdiv_rn(__fmul_rn(g, u), __fadd_rn(1.0f, mmf_exp(-g)));

@@ -125,7 +125,10 @@ __global__ __launch_bounds__(kThreads) void row_kernel(RowArgs a) {
                 float y[8];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) y[i] = xv[v][i];
-                mmf_swish_gate_n<T, 8>(y, ov[v], xv[v]);
+                // fp16 falls back in most waves of 512 elements: rows of one vector a thread keep the definition (64 x 2048 3.8 us, near 5.4; 16384 x 2048
+                // 51 and 63), longer ones where there are more rows than CUs (2002 x 2560 12.1 near, 13.2 exact; 64 x 2560 4.4 and 4.2)
+                if (!std::is_same<T, f16_t>::value || (NV > 1 && gridDim.x > 256)) mmf_swish_gate_n<T, 8, !std::is_same<T, f16_t>::value || (NV > 1)>(y, ov[v], xv[v]);
+                else mmf_swish_gate_n<T, 8, false>(y, ov[v], xv[v]);
             }
             if constexpr (MODE != ROW_QUANT)
                 mmf_store8<T>(static_cast<T*>(a.y) + row * K, k0, K, vec_ok, xv[v]);
@@ -243,8 +246,8 @@ constexpr int kQWaves = 8, kQThreads = kQWaves * 64;
 // Bound by HBM and the vector units about equally (a row of 2048 quantised three times: ~1100 issue slots a wave against 16 KiB of
 // traffic), so what does not depend on the data is kept out: no bounds test in passes known to lie in the row, codes rounded and
 // packed four at a time.  8192 x 2048 bf16, three norms: 37 -> 28 us; residual norm: 33 -> 22.  The gated form takes its sigmoids near
-// (16384 x 2048: 56 -> 52 us, 2002 x 2048 10.6 -> 9.8), and so does the step form (64 x 2048: 5.5 -> 4.9); with a row a workgroup the
-// gated form keeps the exact ones (64 x 2048: 4.1 against 4.3).
+// (16384 x 2048: 56 -> 52 us, 2002 x 2048 10.6 -> 9.8), and so does the step form (64 x 2048: 5.5 -> 4.9); with a row a workgroup, or one
+// vector a thread, the gated form keeps the exact ones (64 x 2048: 4.1 against 4.3; 320 x 1024 fp16 4.7 against 5.1).
 // With several rows a workgroup the codes go out through LDS: a thread's four are 4 bytes of a 16-byte piece, pieces of a row lie 512 bytes apart,
 // and written as they come every store touched 16 lines for 256 bytes; the caches' write requests, not the bytes, set the pace.  From LDS a
 // store writes 16 pieces of all the workgroup's rows (64 bytes for four), and neighbouring workgroups share an XCD, so that whole lines leave its L2.
@@ -371,7 +374,7 @@ __global__ __launch_bounds__(kQThreads) void row_quant_fused_kernel(FusedQuantAr
             raw4_unpack<TW>(w1raw[v], w1v);
 #pragma unroll
             for (int i = 0; i < 4; ++i) y[i] = __fmul_rn(__fmul_rn(xv[v][i], rstd1), w1v[i]);
-            if constexpr (STEP || PRO == QPRO_GATEDNORM) mmf_swish_gate_n<T, 4, STEP || (RPW > 1)>(y, av[v], xv[v]);
+            if constexpr (STEP || PRO == QPRO_GATEDNORM) mmf_swish_gate_n<T, 4, STEP || (RPW > 1 && NV > 1)>(y, av[v], xv[v]);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 if constexpr (!(STEP || PRO == QPRO_GATEDNORM)) xv[v][i] = mmf_round_to<T>(y[i]);
@@ -593,7 +596,9 @@ __global__ __launch_bounds__(256) void swiglu_kernel(const T* __restrict__ x, in
     float xv[8], yv[8], z[8];
     mmf_load8<T>(x + r * ldx, c0, cols, true, xv);
     mmf_load8<T>(y + r * ldy, c0, cols, true, yv);
-    mmf_swiglu_n<T, 8>(xv, yv, z);
+    // fp16 near only with more workgroups than CUs: fewer run as long as their slowest wave (64 x 2048 3.2 us, near 3.4)
+    if (!std::is_same<T, f16_t>::value || gridDim.x > 256) mmf_swiglu_n<T, 8>(xv, yv, z);
+    else mmf_swiglu_n<T, 8, false>(xv, yv, z);
     mmf_store8<T>(out + r * cols, c0, cols, true, z);
 }
 
