@@ -441,7 +441,8 @@ __device__ __forceinline__ void mfma_dma_1k(const void* base, uint32_t lane16, c
 // acc += b x a on a 16 x 16 block over 64 inputs, in place.  (From the builtin the compiler gives every product a destination of its own
 // and the 16 four-register accumulators wander through the registers until some are spilled.)  What the compiler would see to for
 // the builtin: the two wait states behind the vector operations that wrote b (FRESH: its first use); before anything else reads the
-// accumulators, mfma_done().
+// accumulators, mfma_done().  That no copy of an accumulator and no other write falls between is this compiler's choice of registers:
+// tests/test_product_hazards.py reads the assembly for it.
 template <bool FRESH>
 __device__ __forceinline__ void mfma_16x16x64(v4i& acc, const v4i& b, const v4i& a) {
     if constexpr (FRESH) asm volatile("s_nop 1\n\tv_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+v"(acc) : "v"(b), "v"(a));
