@@ -849,13 +849,16 @@ int launch_mfma_dma3(MfmaArgs a, hipStream_t s) {
                           ((reinterpret_cast<uintptr_t>(a.addend) & 15u) == 0));
     // 16-bit outputs of 20 MB and more leave the caches to the activations and weights.  bf16, the launch and what reads its output next, us: 16384 x 2048 ->
     // 6144 (201 MB) 148 and 70 (gate and scan), streamed 147 and 62; -> 2048 and 5632 -> 2048 (67 MB) 98.5 on average and 46.9 (residual norm), 94.6
-    // and 44.6; 2002 x 2048 -> 6144 (25 MB) 31.7 and 16.4, 29.5 and 17.0.  1377 rows (17 MB): 26.3 and 12.5, 25.1 and 13.2, no gain.  Not the swiglu form, whose
-    // output is half as large for its time: 293 and 54 (quantiser), 297 and 65; nor fp32: 666 x 1024 -> 32000 (85 MB) 36.6 and 18.9 (loss), 34.7 and 30.0.
+    // and 44.6; 2002 x 2048 -> 6144 (25 MB) 31.7 and 16.4, 29.5 and 17.0.  1377 rows (17 MB): 26.3 and 12.5, 25.1 and 13.2, no gain.  Whole forwards: 16384
+    // tokens 21.01 ms, streamed 20.77, 2002 tokens with logits and loss 4.45 and 4.41.  By itself the launch is 2 to 4 % shorter over outputs of 1024 to 11264
+    // columns and 20 to 160 MB, with a copy behind it as long.  Only whole lines: rows that share theirs are written twice, alone and with a copy behind
+    // it 40 MB of 1000 columns 25.9 and 40.6, streamed 27.6 and 43.7, of 1960 39.0 and 52.9, 40.4 and 53.8, of 4104 37.3 and 52.1, 39.9 and 54.8.  Not the swiglu
+    // form, whose output is half as large for its time: 293 and 54 (quantiser), 297 and 65; nor fp32: 666 x 1024 -> 32000 (85 MB) 36.6 and 18.9 (loss), 34.7 and 30.0.
     auto kern = bitlinear_mfma_dma3_kernel<T, WGM, WGN, WM, WN, KS, 1, SWI>;
     if constexpr (!SWI) {
         if (!a.vec_store || a.bias) kern = bitlinear_mfma_dma3_kernel<T, WGM, WGN, WM, WN, KS, 0, false>;
         else if constexpr (sizeof(T) == 2) {
-            if (a.M * a.N * 2 >= (20 << 20)) kern = bitlinear_mfma_dma3_kernel<T, WGM, WGN, WM, WN, KS, 2, false>;
+            if (a.M * a.N * 2 >= (20 << 20) && a.ldo % 64 == 0 && (reinterpret_cast<uintptr_t>(a.out) & 127u) == 0) kern = bitlinear_mfma_dma3_kernel<T, WGM, WGN, WM, WN, KS, 2, false>;
         }
     }
     if constexpr (KS > 1) {

@@ -83,11 +83,11 @@ def test_the_kernel_picked_beyond_one_round_of_split_tiles_gives_the_same_bits(d
         assert torch.equal(picked, F.bitlinear_mfma(q[0], deq[0], qsum[0], pw, m, torch.bfloat16, config=config)), config
 
 
-@pytest.mark.parametrize("n", [4104, 4101])
+@pytest.mark.parametrize("n", [4160, 4104, 4101])
 @pytest.mark.parametrize("config", [15, 16, 17, 18])
 def test_outputs_written_past_the_caches_are_the_same(dev, n, config):
-    """2600 rows of bf16 outputs (21 MB) against their first 1312 alone (11 MB, the ordinary stores), ragged rows and columns, with an addend; a width
-    that takes the general epilogue either way."""
+    """2600 rows of bf16 outputs (21 MB) against their first 1312 alone (11 MB, the ordinary stores), ragged rows and columns, with an addend; one
+    whose rows share lines, and a width that takes the general epilogue either way."""
     m, part, k = 2600, 1312, 256
     F, lib, pw, q, codes, deq, qsum = operands(dev, m, k, n, seed=5)
     add = torch.randn(m, n, device=dev).bfloat16()
