@@ -270,12 +270,14 @@ def _dense_weight(pw, dtype):
 def _weight_grad(dout, y):
     """dout^T @ y_q of [M, N] gradients and [M, K] de-quantised inputs.
 
-    For as many outputs as a vocabulary the inputs are stored [K, M] first, contiguous along the contraction: the library's kernels run at a
-    higher rate then, 1024 to 16384 rows in bf16 and fp16, 32000 outputs (us, as they are / transposed): 8192 x 1024 488 / 428, 8192 x 2048
-    1097 / 816, 16384 x 1024 1154 / 824, 4096 x 2048 493 / 410, 1024 x 2048 152 / 131; the transposition moves 4 bytes an element, 1.6 % of the
-    product.  For fewer outputs it costs more of the product (11264: 4 %) than it gives there (-5 to 12 %)."""
+    For as many outputs as a vocabulary the inputs are stored [K, M] first, contiguous along the contraction, where the library's kernels
+    run at a higher rate then: rows a multiple of 64, from 3000 on of 8.  bf16, us, as they are / transposed: 8192 x 1024 -> 32000 488 / 428,
+    8192 x 2048 1097 / 816, 3072 x 2048 10 % less, 1024 x 2048 152 / 131, 5000 rows 7 % less; 1056 rows 20 % more, 2016 5 % more, 2002 and 3001, which
+    are no multiple of 8 (the transposition moves single elements), 0 to 7 % more; the same for 16384 to 50304 outputs and in fp16.  For fewer outputs the
+    transposition, 4 bytes an element, costs more of the product (11264: 4 %) than it gives there (-5 to 12 %)."""
     m, k = y.shape
-    if y.element_size() == 2 and dout.shape[1] >= 16384 and 1024 <= m <= 4194240 and y.is_contiguous():
+    whole = m % 64 == 0 if m < 3000 else m % 8 == 0
+    if y.element_size() == 2 and dout.shape[1] >= 16384 and 1024 <= m <= 4194240 and whole and y.is_contiguous():
         yt = torch.empty(k, m, dtype=y.dtype, device=y.device)
         L.check(L.load().mmf_transpose16(y.data_ptr(), m, k, yt.data_ptr(), L.stream()), "mmf_transpose16")
         y = yt.t()

@@ -64,9 +64,9 @@ def test_transpose_of_16_bit_elements(dev, rows, cols):
         assert torch.equal(out[:rows * cols].view(cols, rows), x.t()) and bool((out[rows * cols:] == 77).all())
 
 
-@pytest.mark.parametrize("m,n,k", [(1023, 16384, 64), (1024, 16384, 64), (1025, 16390, 70)])
+@pytest.mark.parametrize("m,n,k", [(1023, 16384, 64), (1024, 16384, 64), (1025, 16390, 70), (1088, 16390, 70), (3000, 16384, 64), (3004, 16384, 64)])
 def test_weight_gradient_of_a_vocabulary_is_the_product(dev, m, n, k):
-    """Both sides of the line where the inputs are transposed first; bf16 products summed in fp32: half an ulp of the result and m roundings of the sum."""
+    """Both sides of the lines where the inputs are transposed first; bf16 products summed in fp32: half an ulp of the result and m roundings of the sum."""
     from matmulfreellm_amd.autograd import _weight_grad
     torch.manual_seed(m)
     d, y = torch.randn(m, n, device=dev).bfloat16(), torch.randn(m, k, device=dev).bfloat16()
