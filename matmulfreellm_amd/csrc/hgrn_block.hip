@@ -513,15 +513,16 @@ __global__ __launch_bounds__(64 * kMaxWaves, ONE ? 2 : 4) void hgrn_scan_bwd_ker
 //      bytes in flight; with more columns than that whole ones win at every length (12 x 2048 x 1024 35 + 58 against 50 + 79; halved against whole,
 //      forward + backward: 132 columns of 150 to 2500 steps 6.0 + 7.8 / 5.7 + 7.3 to 46 + 71 / 33 + 50, 192 of 300 9.2 + 13.1 / 8.0 + 11.2; 128 of 300
 //      6.6 + 9.6 / 7.6 + 10.8).
-//   64 columns and fewer, 2048 steps and more: whole 128-byte rows in time segments for about two workgroups per CU, a segment at least four
+//   64 columns and fewer, in fp32 40 (half a column's row is a whole line there), 2048 steps and more: whole 128-byte rows in time segments for about two workgroups per CU, a segment at least four
 //      blocks long; a first launch reads x and g (g and do) of all but one segment once more.  Halved against cut, forward + backward, 2500 steps, bf16 and
 //      fp32: 56 columns 49 / 48 and 53 / 73, 66 columns 52 / 52 and 59 / 87, 80 (of 1024-wide rows) 52 / 66 and 78 / 104, 96 54 / 76 and 99 / 123, 112 57 / 88
-//      and 116 / 143; 127 (of 64-wide rows, whose halves no neighbour shares) 87 / 90 and 122 / 155.
+//      and 116 / 143; 127 (of 64-wide rows, whose halves no neighbour shares) 87 / 90 and 122 / 155.  fp32 alone: 32 columns 47 to 53 / 44, 40 47 to 54 / 55,
+//      44 48 / 61, 64 58 to 63 / 80 to 84.
 struct Plan {
     int64_t seg_len;
     int NS, LS, G;
 };
-Plan plan(int64_t BH, int64_t Tlen, int64_t D, int blk, bool split, bool joint) {
+Plan plan(int64_t BH, int64_t Tlen, int64_t D, int blk, bool split, bool joint, int elem) {
     Plan p;
     const int64_t wgs = BH * mmf_ceil_div(D, 64);
     p.G = joint && wgs >= 32 && wgs <= 170 && Tlen >= 3072 ? (int)((wgs <= 64 ? 256 : 512) / wgs) : 1;
@@ -530,7 +531,7 @@ Plan plan(int64_t BH, int64_t Tlen, int64_t D, int blk, bool split, bool joint) 
         p.seg_len = mmf_round_up(Tlen, blk);
         return p;
     }
-    p.LS = wgs <= 128 && (wgs > 64 || Tlen < 2048) ? 2 : 1;
+    p.LS = wgs <= 128 && (wgs > (elem == 4 ? 40 : 64) || Tlen < 2048) ? 2 : 1;
     const int64_t now = BH * mmf_ceil_div(D, 64 / p.LS), step = p.LS * blk;
     int64_t ns = 1;
     if (split && now < 128) {
@@ -548,9 +549,9 @@ bool fwd_takes_workspace(int64_t BH, int64_t Tlen, int64_t D, int chunk) {
     const int64_t block = (64 / chunk > 8 ? 8 : 64 / chunk) * (int64_t)chunk;
     return BH * mmf_ceil_div(D, 64) < 256 && Tlen >= 8 * block;
 }
-Plan fwd_plan(int64_t BH, int64_t Tlen, int64_t D, int chunk, bool joint) {
+Plan fwd_plan(int64_t BH, int64_t Tlen, int64_t D, int chunk, bool joint, int elem) {
     const bool split = fwd_takes_workspace(BH, Tlen, D, chunk);
-    return plan(BH, Tlen, D, kFwdBlk, split, split && joint);
+    return plan(BH, Tlen, D, kFwdBlk, split, split && joint, elem);
 }
 int64_t joint_columns(int64_t BH, int64_t D) { return BH * mmf_ceil_div(D, 64); }
 int64_t joint_bytes(int64_t BH, int64_t D) { return joint_columns(BH, D) * 65 * 8 + 8; }   // (8 over: the words begin at the workspace's first multiple of 8)
@@ -614,7 +615,7 @@ int launch_fwd_ls(const Plan& p, const T* x, const T* g, const float* h0, T* o, 
 template <typename T>
 int launch_fwd(const void* x, const void* g, const float* h0, void* o, float* ht, float* agg, int64_t BH, int64_t Tlen, int64_t D,
                int chunk, hipStream_t s) {
-    const Plan p = fwd_plan(BH, Tlen, D, chunk, agg && !fwd_halves(BH, Tlen, D, sizeof(T)));
+    const Plan p = fwd_plan(BH, Tlen, D, chunk, agg && !fwd_halves(BH, Tlen, D, sizeof(T)), sizeof(T));
     if (!agg && (p.NS > 1 || (fwd_takes_workspace(BH, Tlen, D, chunk) && BH * mmf_ceil_div(D, 64) < 128 && Tlen >= 2048))) return MMF_ERR_ARG;
     const T* xp = static_cast<const T*>(x);
     const T* gp = static_cast<const T*>(g);
@@ -652,7 +653,7 @@ int launch_bwd_ls(const Plan& p, const T* g, const T* o, const T* dout, const fl
 template <typename T, bool LOG>
 int launch_bwd(const void* g, const void* o, const void* dout, const float* h0, void* dx, void* dg, float* agg, int64_t BH,
                int64_t Tlen, int64_t D, hipStream_t s) {
-    const Plan p = plan(BH, Tlen, D, kBwdBlk, agg != nullptr, agg != nullptr);
+    const Plan p = plan(BH, Tlen, D, kBwdBlk, agg != nullptr, agg != nullptr, sizeof(T));
     const T* gp = static_cast<const T*>(g);
     const T* op = static_cast<const T*>(o);
     const T* dp = static_cast<const T*>(dout);
@@ -687,7 +688,7 @@ extern "C" {
 int64_t mmf_hgrn_chunk_workspace_bytes(int64_t BH, int64_t T, int64_t D, int chunk) {
     if (BH <= 0 || T <= 0 || D <= 0 || chunk < 1 || chunk > 64) return 0;
     if (!fwd_takes_workspace(BH, T, D, chunk)) return 0;
-    const Plan p = fwd_plan(BH, T, D, chunk, true);
+    const Plan p = fwd_plan(BH, T, D, chunk, true, 2);   // (fp32 is cut in no more places)
     return p.G > 1 ? joint_bytes(BH, D) : BH * p.NS * 2 * D * (int64_t)sizeof(float);
 }
 
@@ -716,7 +717,7 @@ int mmf_hgrn_chunk(const void* x, const void* g, const float* h0, void* o, float
 
 int64_t mmf_hgrn_recurrent_bwd_workspace_bytes(int64_t BH, int64_t T, int64_t D) {
     if (BH <= 0 || T <= 0 || D <= 0) return 0;
-    return pair_bytes(plan(BH, T, D, kBwdBlk, true, true), BH, D);
+    return pair_bytes(plan(BH, T, D, kBwdBlk, true, true, 2), BH, D);
 }
 
 int mmf_hgrn_recurrent_bwd_split(const void* g, const void* o, const void* grad_o, const float* h0, void* dx, void* dg, int64_t BH,

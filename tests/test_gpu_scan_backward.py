@@ -109,7 +109,7 @@ def test_a_zero_carry_survives_a_product_of_gates_that_overflows(dev, log):
 
 
 @pytest.mark.parametrize("bh,d,t", [(32, 64, 3072), (11, 130, 3101), (31, 64, 3072), (64, 64, 3100), (65, 33, 3073), (128, 64, 3361), (170, 40, 3080),
-                                    (171, 40, 3080), (64, 64, 2050), (65, 64, 2050), (127, 33, 3071), (9, 512, 3072), (9, 512, 5121), (128, 32, 5120)])
+                                    (171, 40, 3080), (40, 64, 2050), (41, 64, 2050), (64, 64, 2050), (65, 64, 2050), (127, 33, 3071), (9, 512, 3072), (9, 512, 5121), (128, 32, 5120)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("log", [True, False])
 def test_scans_whose_columns_are_shared_by_workgroups(dev, bh, d, t, dtype, log):
