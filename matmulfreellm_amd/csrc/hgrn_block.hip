@@ -21,10 +21,10 @@
 // LS = 2: a workgroup owns 32 channels and the halves of a wave two consecutive runs of steps, for twice the workgroups.
 // When there are still too few, a first launch (AGG) runs steps 1-3 only and leaves per time segment the pair (P, l); the
 // second enters segment s with the fold carry = l_j + P_j * carry over the segments before (backward: behind) it.
-// Measured, bf16, backward: 8 x 1024 x 2048 145 -> 40 us (4.1 TB/s), 64 x 16384 x 128 with log gates 2290 -> 262 us
-// (5.1 TB/s), against a kernel that loaded under a branch per step, so one load after the other, and read g and do twice.
+// Measured, bf16, backward: 8 x 1024 x 2048 145 -> 36 us in a training step (4.7 TB/s), 64 x 16384 x 128 with log gates 2290 -> 254 us
+// (5.3 TB/s), against a kernel that loaded under a branch per step, so one load after the other, and read g and do twice.
 // 16 to 28 steps a block and 8 or 16 waves a workgroup lie within 10 % of each other.  Forward, bf16:
-// 64 x 16384 x 128 317 -> 160 us (5.0 TB/s), 4 x 2048 x 2048 61 -> 28 us, against 64-step blocks that took a second exp per step
+// 64 x 16384 x 128 317 -> 160 us (5.0 TB/s), 4 x 2048 x 2048 61 -> 28 us (20 with the tensors in the last-level cache), against 64-step blocks that took a second exp per step
 // for P_t and cut these shapes in time, two launches over x and g.
 #include <type_traits>
 #include "mmf_common.h"
