@@ -1058,18 +1058,27 @@ int launch_mfma(MfmaArgs a, hipStream_t s) {
 // 39.7 / 43.3, 6500 86.5 / 77.4; 2048 -> 2048 (16), 2002 rows 12.2 / 15.1, 3600 18.0 / 18.5; 2048 -> 6144, 2002 rows (768) 27.1 / 26.4.  Stream against split:
 // 1024 -> 5632, 300 rows 6.0 / 8.4, 700 9.9 / 9.4; 2048 -> 2048, 1203 rows 10.9 / 11.4, 1395 12.1 / 11.3.
 // Over 389 shapes, 66 to 8000 rows, the choice costs 0.01 % against the best of the three on average, 15 % at most (377 x 1536 -> 4608: 1.2 us).
+// With the swiglu epilogue (M from 66 to 6300, K from 512 to 4096, N from 2048 to 22016) the stream's workgroups each own two blocks, of gate and of up, and
+// take 1.3 + 0.1 ns per k-block a block; a tile's epilogue, which nothing hides where a CU has one, is 3 to 5 us.  Over 461 shapes beside the 357 fitted the choice costs 0.25 %
+// on average, 8 % at most; with the plain products' times it cost 4 %, and 58 % at most (106 x 2560 -> 13824, stream / split 9.7 / 15.3 us; 410 x 1024 -> 5632
+// 9.1 / 12.1 in a model).
 enum class MfmaPick { kStream, kSplit, kTiles };
-inline MfmaPick mfma_pick(const MfmaArgs& a) {
+inline MfmaPick mfma_pick(const MfmaArgs& a, bool swiglu) {
     const int64_t KB = a.Kp >> 7;
     const double kb = (double)KB, blocks = (double)mmf_ceil_div(a.M, 32) * (double)mmf_ceil_div(a.N, 32);
     const int64_t half = mmf_ceil_div(a.M, 64) * mmf_ceil_div(a.N, 256), full = mmf_ceil_div(a.M, 64) * mmf_ceil_div(a.N, 512);
-    const double t_stream = 3.0 + blocks * (0.0007 + 0.00018 * (double)((KB + 7) / 8 * 8));
-    const double t_tiles = full <= 256 ? 4.4 + 0.58 * kb + (double)full / 256.0 * (1.0 + 0.18 * kb) : (double)mmf_ceil_div(full, 256) * (4.4 + 0.62 * kb);
-    double t_split = 1e30;
-    if (KB % 2 == 0)
-        t_split = half <= 256   ? 4.4 + 0.29 * kb + (double)half / 256.0 * (1.0 + 0.1 * kb)
-                  : half <= 512 ? 8.5 + 0.59 * kb
-                                : (double)mmf_ceil_div(half, 256) * (3.9 + 0.295 * kb);
+    const double halves = (double)half / 256.0, wholes = (double)full / 256.0, half_rounds = (double)mmf_ceil_div(half, 256), rounds = (double)mmf_ceil_div(full, 256);
+    double t_stream, t_tiles, t_split;
+    if (swiglu) {
+        t_stream = 3.5 + blocks * (0.0013 + 0.0001 * kb);
+        t_tiles = full <= 256 ? 9.2 + 0.585 * kb + wholes * (0.19 * kb - 1.0) : 6.5 + rounds * (3.5 + 0.54 * kb);
+        t_split = half <= 256 ? 8.0 + 0.285 * kb + halves * 0.1 * kb : half <= 512 ? 10.5 + 0.595 * kb : 5.8 + half_rounds * (2.4 + 0.297 * kb);
+    } else {
+        t_stream = 3.0 + blocks * (0.0007 + 0.00018 * (double)((KB + 7) / 8 * 8));
+        t_tiles = full <= 256 ? 4.4 + 0.58 * kb + wholes * (1.0 + 0.18 * kb) : rounds * (4.4 + 0.62 * kb);
+        t_split = half <= 256 ? 4.4 + 0.29 * kb + halves * (1.0 + 0.1 * kb) : half <= 512 ? 8.5 + 0.59 * kb : half_rounds * (3.9 + 0.295 * kb);
+    }
+    if (KB % 2 != 0) t_split = 1e30;
     if (a.Kp <= 8192 && a.M <= 65535 * 32 && (a.M <= 64 || (t_stream <= t_split && t_stream <= t_tiles))) return MfmaPick::kStream;
     return t_split < t_tiles ? MfmaPick::kSplit : MfmaPick::kTiles;
 }
@@ -1083,7 +1092,7 @@ int dispatch_mfma(const MfmaArgs& a, int config, hipStream_t s) {
     //   15 / 16 / 17  256x256 / 128x256 / 64x512 tiles, A staged by DMA (17: every wave reads the whole activation
     //            tile from LDS and owns its own weight columns, so no weight block is fetched twice)
     if (config < 0) {
-        const MfmaPick pick = mfma_pick(a);
+        const MfmaPick pick = mfma_pick(a, false);
         if (pick == MfmaPick::kStream) config = 5;
         else if (a.M <= 32) config = 0;
         else if (a.M <= 64) config = 1;
@@ -1124,7 +1133,7 @@ int dispatch_mfma(const MfmaArgs& a, int config, hipStream_t s) {
 
 template <typename T>
 int dispatch_mfma_swiglu(const MfmaArgs& a, hipStream_t s) {
-    switch (mfma_pick(a)) {
+    switch (mfma_pick(a, true)) {
         case MfmaPick::kStream: return launch_skinny_swiglu<T>(a, s);
         case MfmaPick::kSplit: return launch_mfma_dma3<T, 1, 4, 2, 2, 2, true>(a, s);
         case MfmaPick::kTiles: return launch_mfma_dma3<T, 1, 8, 2, 2, 1, true>(a, s);

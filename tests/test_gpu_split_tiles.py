@@ -46,6 +46,15 @@ def test_split_tiles_on_both_sides_of_one_per_cu(dev, k, dtype):
             assert torch.equal(F.bitlinear_mfma_swiglu(q[0], deq[0], qsum[0], pw, m, dtype), F.swiglu(want[:, :n // 2], want[:, n // 2:])), (m, n)
 
 
+# the stream (410 rows) | split tiles: one per CU, two, three rounds | whole tiles: one per CU (15 k-blocks), four rounds; ragged rows and columns
+@pytest.mark.parametrize("m,k,inter", [(410, 1024, 2816), (1009, 2048, 2016), (3833, 2048, 992), (2050, 1024, 2816), (2033, 1920, 2016), (5001, 1024, 2816)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_the_kernel_picked_for_the_swiglu_gives_the_same_bits(dev, m, k, inter, dtype):
+    F, lib, pw, q, codes, deq, qsum = operands(dev, m, k, 2 * inter, seed=3)
+    y = F.bitlinear_mfma(q[0], deq[0], qsum[0], pw, m, dtype, config=16)
+    assert torch.equal(F.bitlinear_mfma_swiglu(q[0], deq[0], qsum[0], pw, m, dtype), F.swiglu(y[:, :inter], y[:, inter:]))
+
+
 def test_odd_number_of_k_blocks_is_refused(dev):
     F, lib, pw, q, codes, deq, qsum = operands(dev, 70, 384, 256)
     with pytest.raises(RuntimeError):
