@@ -123,7 +123,6 @@ int mmf_rmsnorm_quant_fused(int prologue, const void* x, int64_t ldx, const void
                             int64_t ldaux2, void* res_out, const void* w1, float eps1, const void* norm_weight, float eps,
                             const float* lower_bound, float* state, int8_t* q, float* deq, int* qsum, int64_t M, int64_t K,
                             int x_dtype, int weight_dtype, void* stream);
-
 /* ---- BitLinear contraction ------------------------------------------------------------
  * Both replace F.linear(y, weight_quant(W)) at mmfreelm/ops/fusedbitnet.py:456-458 (class
  * FusedBitLinear :584-610, layer_norm_linear_quant_fn :513-536):
@@ -396,6 +395,17 @@ int mmf_bitlinear_gemv_multi(int epilogue, const void* x, int64_t ldx, const voi
                              const void* norm_weight1, const void* norm_weight2, float eps, const void* packed, const float* wdeq,
                              int64_t seg_rows, void* out, void* g_out, const float* lower_bound, float* state, int64_t M, int64_t K,
                              int64_t N, int x_dtype, int weight_dtype, void* stream);
+
+/* ---- quantisers that know which weights come behind them.  As the calls without _ahead; `ahead_bytes` bytes at `ahead` (device memory, 16-byte
+ * aligned; null or 0: nothing) are brought into the last-level cache meanwhile: the packed weights that the next launch contracts.  No
+ * result depends on them.  At most as many lines of 128 bytes as the launch has threads, and none where a row has a workgroup of its own. */
+int mmf_rmsnorm_quant_fused_ahead(int prologue, const void* x, int64_t ldx, const void* aux, int64_t ldaux, const void* aux2,
+                                  int64_t ldaux2, void* res_out, const void* w1, float eps1, const void* norm_weight, float eps,
+                                  const float* lower_bound, float* state, int8_t* q, float* deq, int* qsum, int64_t M, int64_t K,
+                                  const void* ahead, int64_t ahead_bytes, int x_dtype, int weight_dtype, void* stream);
+int mmf_rmsnorm_quant_multi_ahead(const void* x, int64_t ldx, const void* w1, float eps1, const void* norm_weight0,
+                                  const void* norm_weight1, const void* norm_weight2, float eps, int8_t* q, float* deq, int* qsum, int64_t M,
+                                  int64_t K, const void* ahead, int64_t ahead_bytes, int x_dtype, int weight_dtype, void* stream);
 
 /* ---- a whole block (mmfreelm/models/hgrn_bit/modeling_hgrn_bit.py:97-111) as one host call: the launches above in the order
  * of the model, bit for bit what they give one by one.  out [B, T, H] = block(x [B, T, H]); mask: null or [B, T] bytes;

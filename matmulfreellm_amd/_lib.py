@@ -38,6 +38,8 @@ SIGNATURES = {
     "mmf_layernorm_quant": (_i32, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _f32, _i32, _i32, _i32, _i32, _ptr]),
     "mmf_rmsnorm_quant_fused": (_i32, [_i32, _ptr, _i64, _ptr, _i64, _ptr, _i64, _ptr, _ptr, _f32, _ptr, _f32, _ptr, _ptr, _ptr, _ptr,
                                        _ptr, _i64, _i64, _i32, _i32, _ptr]),
+    "mmf_rmsnorm_quant_fused_ahead": (_i32, [_i32, _ptr, _i64, _ptr, _i64, _ptr, _i64, _ptr, _ptr, _f32, _ptr, _f32, _ptr, _ptr, _ptr,
+                                             _ptr, _ptr, _i64, _i64, _ptr, _i64, _i32, _i32, _ptr]),
     "mmf_decode_layers_phase_bytes": (_i32, []),
     "mmf_decode_layers_copies": (_i32, []),
     "mmf_decode_layers_fits": (_i32, [_i32, _i32, _i32, _i32, _i32]),
@@ -86,6 +88,8 @@ SIGNATURES = {
     "mmf_short_conv_bwd_groups": (_i32, [_i64]),
     "mmf_short_conv_bwd": (_i32, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _i32, _i32, _i32, _ptr]),
     "mmf_rmsnorm_quant_multi": (_i32, [_ptr, _i64, _ptr, _f32, _ptr, _ptr, _ptr, _f32, _ptr, _ptr, _ptr, _i64, _i64, _i32, _i32, _ptr]),
+    "mmf_rmsnorm_quant_multi_ahead": (_i32, [_ptr, _i64, _ptr, _f32, _ptr, _ptr, _ptr, _f32, _ptr, _ptr, _ptr, _i64, _i64, _ptr, _i64, _i32,
+                                             _i32, _ptr]),
     "mmf_bitlinear_mfma_multi": (_i32, [_ptr, _i64, _ptr, _ptr, _ptr, _ptr, _i64, _ptr, _i64, _i64, _i64, _i64, _i32, _i32, _ptr]),
     "mmf_bitlinear_gemv_multi": (_i32, [_i32, _ptr, _i64, _ptr, _f32, _ptr, _ptr, _ptr, _f32, _ptr, _ptr, _i64, _ptr, _ptr, _ptr, _ptr,
                                         _i64, _i64, _i64, _i32, _i32, _ptr]),

@@ -20,19 +20,33 @@ bool few_rows(const mmf_block* p, int64_t M) {
     return M <= kGemvRows && (k > p->D ? k : p->D) <= mmf_bitlinear_gemv_max_k();
 }
 
+// The quantisers of middle-sized prompts bring the weights behind them (the packed bytes of [n, k], n a multiple of 32) into the last-level
+// cache: a contraction that finds them in memory waits for each of its first k-blocks.  us a launch at the 1.3B shape, weights in memory and in the
+// cache: 459 rows, i/f/g 13.4 and 12.4, o 7.0 and 6.2, gate/up 19.9 and 18.5, down 13.0 and 11.9; 1377 rows 25.8 / 25.0, 13.2 / 11.7, 33.4 / 32.8,
+// 23.6 / 20.5.  The quantiser, 9 to 12 us of 1377 rows, takes 0.3 us more.  Forwards: 3 x 459 tokens 3630 -> 3530 us, 2 x 1001 with logits 4406 -> 4285,
+// 270 tokens 1603 -> 1576, 2 x 2000 6398 -> 6320; 370M shape, 4 x 700 2781 -> 2754.  With fewer rows the quantiser is as short as memory's answer (a
+// decode step of 64 rows 0.5 to 5 % longer, however the touches were spread over its launches); with 8192 and 16384, rounds of tiles hide
+// the start and the touches only delay the rows (1 to 2 % of a forward).
+constexpr int64_t kAheadMinRows = 256, kAheadMaxRows = 5120;
+struct Ahead { const void* p; int64_t bytes; };
+Ahead ahead(const void* packed, int64_t n, int64_t k, int64_t M) {
+    return M > kAheadMinRows && M <= kAheadMaxRows ? Ahead{packed, n * mmf_round_up(k, 128) / 4} : Ahead{nullptr, 0};
+}
+
 // What the i/f/g projections contract: codes of x under the block norm and their inner norm(s), q [1 or 3], deq, qsum.
 int project_ifg(const mmf_block* p, const void* x, int64_t M, int8_t* q, float* deq, int* qsum, void* ifg, void* stream) {
     const int64_t H = p->H, D = p->D;
     const int dt = p->dtype, wt = p->weight_dtype;
+    const Ahead w = ahead(p->ifg_packed, 3 * D, H, M);
     if (p->f_norm) {
-        if (const int rc = mmf_rmsnorm_quant_multi(x, H, p->attn_norm, p->attn_eps, p->i_norm, p->f_norm, p->g_proj_norm, p->ifg_eps, q, deq,
-                                                   qsum, M, H, dt, wt, stream))
+        if (const int rc = mmf_rmsnorm_quant_multi_ahead(x, H, p->attn_norm, p->attn_eps, p->i_norm, p->f_norm, p->g_proj_norm, p->ifg_eps, q,
+                                                         deq, qsum, M, H, w.p, w.bytes, dt, wt, stream))
             return rc;
         return mmf_bitlinear_mfma_multi(q, mmf_codes_bytes(M, H, 1), deq, qsum, p->ifg_packed, p->ifg_wdeq, D, ifg, 3 * D, M, H, 3 * D, dt,
                                         -1, stream);
     }
-    if (const int rc = mmf_rmsnorm_quant_fused(Q_NORM, x, H, nullptr, 0, nullptr, 0, nullptr, p->attn_norm, p->attn_eps, p->i_norm, p->ifg_eps,
-                                               nullptr, nullptr, q, deq, qsum, M, H, dt, wt, stream))
+    if (const int rc = mmf_rmsnorm_quant_fused_ahead(Q_NORM, x, H, nullptr, 0, nullptr, 0, nullptr, p->attn_norm, p->attn_eps, p->i_norm,
+                                                     p->ifg_eps, nullptr, nullptr, q, deq, qsum, M, H, w.p, w.bytes, dt, wt, stream))
         return rc;
     return mmf_bitlinear_mfma(q, deq, qsum, p->ifg_packed, p->ifg_wdeq, D, nullptr, nullptr, ifg, 3 * D, M, H, 3 * D, dt, -1, stream);
 }
@@ -95,6 +109,7 @@ int mmf_block_train_forward(const mmf_block* p, const void* x, void* out, void* 
     char *i = static_cast<char*>(ifg), *f = i + D * e, *g = i + 2 * D * e, *gs = static_cast<char*>(xg) + M * D * e;
     char* up = static_cast<char*>(y) + I * e;
     const int dt = p->dtype, wt = p->weight_dtype;
+    const Ahead o_w = ahead(p->o_packed, H, D, M), gate_w = ahead(p->gate_packed, 2 * I, H, M), down_w = ahead(p->down_packed, H, I, M);
     int rc = 0;
 #define MMF_DO(call)                \
     do {                            \
@@ -103,15 +118,15 @@ int mmf_block_train_forward(const mmf_block* p, const void* x, void* out, void* 
     MMF_DO(project_ifg(p, x, M, q, deq, qsum, ifg, stream));
     MMF_DO(mmf_hgrn_gate(i, 3 * D, f, 3 * D, lower_bound, mask, xg, gs, M, D, dt, stream));
     MMF_DO(mmf_hgrn_recurrent(xg, gs, nullptr, o, nullptr, B, T, D, dt, stream));
-    MMF_DO(mmf_rmsnorm_quant_fused(Q_GATEDNORM, g, 3 * D, o, D, nullptr, 0, nullptr, p->g_norm, p->g_eps, p->o_norm, p->o_eps, nullptr,
-                                   nullptr, q, deq, qsum, M, D, dt, wt, stream));
+    MMF_DO(mmf_rmsnorm_quant_fused_ahead(Q_GATEDNORM, g, 3 * D, o, D, nullptr, 0, nullptr, p->g_norm, p->g_eps, p->o_norm, p->o_eps, nullptr,
+                                         nullptr, q, deq, qsum, M, D, o_w.p, o_w.bytes, dt, wt, stream));
     MMF_DO(mmf_bitlinear_mfma(q, deq, qsum, p->o_packed, p->o_wdeq, p->o_seg_rows, nullptr, nullptr, attn, H, M, D, H, dt, -1, stream));
-    MMF_DO(mmf_rmsnorm_quant_fused(Q_RESNORM, attn, H, x, H, nullptr, 0, res, p->mlp_norm, p->mlp_eps, p->gate_norm, p->gate_eps, nullptr,
-                                   nullptr, q, deq, qsum, M, H, dt, wt, stream));
+    MMF_DO(mmf_rmsnorm_quant_fused_ahead(Q_RESNORM, attn, H, x, H, nullptr, 0, res, p->mlp_norm, p->mlp_eps, p->gate_norm, p->gate_eps, nullptr,
+                                         nullptr, q, deq, qsum, M, H, gate_w.p, gate_w.bytes, dt, wt, stream));
     MMF_DO(mmf_bitlinear_mfma(q, deq, qsum, p->gate_packed, p->gate_wdeq, p->gate_seg_rows, nullptr, nullptr, y, 2 * I, M, H, 2 * I, dt, -1,
                               stream));
-    MMF_DO(mmf_rmsnorm_quant_fused(Q_SWIGLU, y, 2 * I, up, 2 * I, nullptr, 0, nullptr, nullptr, 0.0f, p->down_norm, p->down_eps, nullptr,
-                                   nullptr, q, deq, qsum, M, I, dt, wt, stream));
+    MMF_DO(mmf_rmsnorm_quant_fused_ahead(Q_SWIGLU, y, 2 * I, up, 2 * I, nullptr, 0, nullptr, nullptr, 0.0f, p->down_norm, p->down_eps, nullptr,
+                                         nullptr, q, deq, qsum, M, I, down_w.p, down_w.bytes, dt, wt, stream));
     MMF_DO(mmf_bitlinear_mfma(q, deq, qsum, p->down_packed, p->down_wdeq, p->down_seg_rows, nullptr, res, out, H, M, I, H, dt, -1, stream));
 #undef MMF_DO
     return 0;
@@ -136,6 +151,7 @@ int mmf_block_forward(const mmf_block* p, const void* x, void* out, int64_t B, i
     const int dt = p->dtype, wt = p->weight_dtype;
     const bool multi = p->f_norm != nullptr;                   // i, f and g have inner norms of their own
     const bool step = T == 1 && h0 && h0 == ht;                // one token on a kept state: gate math + recurrence step in one kernel
+    const Ahead o_w = ahead(p->o_packed, H, D, M), gate_w = ahead(p->gate_packed, 2 * I, H, M), down_w = ahead(p->down_packed, H, I, M);
     int rc = 0;
 #define MMF_DO(call)                \
     do {                            \
@@ -175,15 +191,15 @@ int mmf_block_forward(const mmf_block* p, const void* x, void* out, int64_t B, i
                                        lower_bound, ht, q, deq, qsum, M, D, dt, wt, stream));
     } else {
         MMF_DO(scan());
-        MMF_DO(mmf_rmsnorm_quant_fused(Q_GATEDNORM, g, 3 * D, o, D, nullptr, 0, nullptr, p->g_norm, p->g_eps, p->o_norm, p->o_eps,
-                                       nullptr, nullptr, q, deq, qsum, M, D, dt, wt, stream));
+        MMF_DO(mmf_rmsnorm_quant_fused_ahead(Q_GATEDNORM, g, 3 * D, o, D, nullptr, 0, nullptr, p->g_norm, p->g_eps, p->o_norm, p->o_eps,
+                                             nullptr, nullptr, q, deq, qsum, M, D, o_w.p, o_w.bytes, dt, wt, stream));
     }
     MMF_DO(mmf_bitlinear_mfma(q, deq, qsum, p->o_packed, p->o_wdeq, p->o_seg_rows, nullptr, nullptr, attn, H, M, D, H, dt, -1, stream));
-    MMF_DO(mmf_rmsnorm_quant_fused(Q_RESNORM, attn, H, x, H, nullptr, 0, res, p->mlp_norm, p->mlp_eps, p->gate_norm, p->gate_eps, nullptr,
-                                   nullptr, q, deq, qsum, M, H, dt, wt, stream));
+    MMF_DO(mmf_rmsnorm_quant_fused_ahead(Q_RESNORM, attn, H, x, H, nullptr, 0, res, p->mlp_norm, p->mlp_eps, p->gate_norm, p->gate_eps, nullptr,
+                                         nullptr, q, deq, qsum, M, H, gate_w.p, gate_w.bytes, dt, wt, stream));
     MMF_DO(mmf_bitlinear_mfma_swiglu(q, deq, qsum, p->gate_packed, p->gate_wdeq, p->gate_seg_rows, big, I, M, H, 2 * I, dt, stream));
-    MMF_DO(mmf_rmsnorm_quant_fused(Q_PLAIN, big, I, nullptr, 0, nullptr, 0, nullptr, nullptr, 0.0f, p->down_norm, p->down_eps, nullptr,
-                                   nullptr, q, deq, qsum, M, I, dt, wt, stream));
+    MMF_DO(mmf_rmsnorm_quant_fused_ahead(Q_PLAIN, big, I, nullptr, 0, nullptr, 0, nullptr, nullptr, 0.0f, p->down_norm, p->down_eps, nullptr,
+                                         nullptr, q, deq, qsum, M, I, down_w.p, down_w.bytes, dt, wt, stream));
     MMF_DO(mmf_bitlinear_mfma(q, deq, qsum, p->down_packed, p->down_wdeq, p->down_seg_rows, nullptr, res, out, H, M, I, H, dt, -1, stream));
 #undef MMF_DO
     return 0;

@@ -580,6 +580,25 @@ __device__ __forceinline__ float mmf_block_max_once(float v, float* slot) {
     return s;
 }
 
+// What a launch behind this one reads first, its packed weights, is brought into the last-level cache meanwhile: a wave touches a dword of each of
+// 64 lines of 128 bytes and waits for none of them.  `slot` numbers the waves of the grid.  The touch stands behind the kernel's own
+// loads, which return in order, and its value is kept (mmf_touched, at the end) only so that the load is.
+struct MmfAhead { const unsigned char* p; uint32_t lines; };
+__device__ __forceinline__ uint32_t mmf_touch(const MmfAhead& a, uint32_t slot) {
+    const uint32_t line = slot * 64 + (threadIdx.x & 63);
+    uint32_t v = 0;
+    if (line < a.lines) v = *reinterpret_cast<const uint32_t*>(a.p + (uint64_t)line * 128);
+    return v;
+}
+__device__ __forceinline__ void mmf_touched(uint32_t v) { asm volatile("" ::"v"(v)); }
+static inline int mmf_set_ahead(MmfAhead& a, const void* p, int64_t bytes) {
+    if (bytes < 0) return MMF_ERR_ARG;
+    if (reinterpret_cast<uintptr_t>(p) & 15u) return MMF_ERR_ALIGN;
+    a.p = static_cast<const unsigned char*>(p);
+    a.lines = p ? (uint32_t)(bytes / 128 < (1 << 24) ? bytes / 128 : 1 << 24) : 0;   // (2 GiB)
+    return 0;
+}
+
 // rstd = 1 / sqrt( fp32(sumsq / K) + eps ).
 // sumsq / K is the correctly rounded fp64 quotient without the division sequence: with
 // inv_K = RN(1 / K) from the host, q0 = sumsq * inv_K is within two ulps, one residual step

@@ -234,6 +234,7 @@ struct FusedQuantArgs {
     int64_t M, K, Kp;
     double inv_K;            // RN(1 / K)
     float eps1, eps;
+    MmfAhead ahead;          // the packed weights that the next launch contracts
 };
 
 constexpr int kQWaves = 8, kQThreads = kQWaves * 64;
@@ -313,6 +314,8 @@ __global__ __launch_bounds__(kQThreads) void row_quant_fused_kernel(FusedQuantAr
             for (int j = 0; j < NN; ++j) nwraw[j][v] = ld(nws[j], v, k0);
         }
     }
+    uint32_t touched = 0;
+    if constexpr (RPW > 1) touched = mmf_touch(a.ahead, (uint32_t)wave * (((uint32_t)a.M + RPW - 1) / RPW) + blockIdx.x);   // (a row a workgroup: decode, no longer than the touch would take)
     float xv[NV][4], av[HAS_AUX ? NV : 1][4];
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
@@ -504,6 +507,7 @@ __global__ __launch_bounds__(kQThreads) void row_quant_fused_kernel(FusedQuantAr
             a.qsum[j * a.M + row] = qs[j];
         }
     }
+    if constexpr (RPW > 1) mmf_touched(touched);
 }
 
 template <typename T, typename TW, int PRO, int RPW, int NN>
@@ -709,6 +713,14 @@ int mmf_rmsnorm_quant_fused(int prologue, const void* x, int64_t ldx, const void
                             int64_t ldaux2, void* res_out, const void* w1, float eps1, const void* norm_weight, float eps,
                             const float* lower_bound, float* state, int8_t* q, float* deq, int* qsum, int64_t M, int64_t K,
                             int x_dtype, int weight_dtype, void* stream_) {
+    return mmf_rmsnorm_quant_fused_ahead(prologue, x, ldx, aux, ldaux, aux2, ldaux2, res_out, w1, eps1, norm_weight, eps, lower_bound, state, q,
+                                         deq, qsum, M, K, nullptr, 0, x_dtype, weight_dtype, stream_);
+}
+
+int mmf_rmsnorm_quant_fused_ahead(int prologue, const void* x, int64_t ldx, const void* aux, int64_t ldaux, const void* aux2,
+                                  int64_t ldaux2, void* res_out, const void* w1, float eps1, const void* norm_weight, float eps,
+                                  const float* lower_bound, float* state, int8_t* q, float* deq, int* qsum, int64_t M, int64_t K,
+                                  const void* ahead, int64_t ahead_bytes, int x_dtype, int weight_dtype, void* stream_) {
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     if (M < 0 || K <= 0 || ldx < K) return MMF_ERR_ARG;
     if (M == 0) return 0;
@@ -721,6 +733,7 @@ int mmf_rmsnorm_quant_fused(int prologue, const void* x, int64_t ldx, const void
     a.x = x; a.aux = aux ? aux : x; a.aux2 = aux2 ? aux2 : x; a.ldx = ldx; a.ldaux = aux ? ldaux : ldx;
     a.ldaux2 = aux2 ? ldaux2 : ldx; a.res_out = res_out; a.w1 = w1; a.norm_w = norm_weight; a.lb = lower_bound; a.state = state;
     a.q = q; a.deq = deq; a.qsum = qsum; a.M = M; a.K = K; a.inv_K = 1.0 / (double)K; a.Kp = mmf_round_up(K, 128); a.eps1 = eps1; a.eps = eps;
+    if (const int rc = mmf_set_ahead(a.ahead, ahead, ahead_bytes)) return rc;
     if (!aligned16(q)) return MMF_ERR_ALIGN;
     if (!norm_weight && !w1) weight_dtype = MMF_F32;
     return run_fused_quant(a, prologue, x_dtype, weight_dtype, stream);
@@ -729,6 +742,13 @@ int mmf_rmsnorm_quant_fused(int prologue, const void* x, int64_t ldx, const void
 int mmf_rmsnorm_quant_multi(const void* x, int64_t ldx, const void* w1, float eps1, const void* norm_weight0, const void* norm_weight1,
                             const void* norm_weight2, float eps, int8_t* q, float* deq, int* qsum, int64_t M, int64_t K, int x_dtype,
                             int weight_dtype, void* stream_) {
+    return mmf_rmsnorm_quant_multi_ahead(x, ldx, w1, eps1, norm_weight0, norm_weight1, norm_weight2, eps, q, deq, qsum, M, K, nullptr, 0, x_dtype,
+                                         weight_dtype, stream_);
+}
+
+int mmf_rmsnorm_quant_multi_ahead(const void* x, int64_t ldx, const void* w1, float eps1, const void* norm_weight0,
+                                  const void* norm_weight1, const void* norm_weight2, float eps, int8_t* q, float* deq, int* qsum, int64_t M,
+                                  int64_t K, const void* ahead, int64_t ahead_bytes, int x_dtype, int weight_dtype, void* stream_) {
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     if (M < 0 || K <= 0 || ldx < K) return MMF_ERR_ARG;
     if (M == 0) return 0;
@@ -738,6 +758,7 @@ int mmf_rmsnorm_quant_multi(const void* x, int64_t ldx, const void* w1, float ep
     a.x = a.aux = a.aux2 = x; a.ldx = a.ldaux = a.ldaux2 = ldx; a.w1 = w1; a.norm_w = norm_weight0; a.norm_w2 = norm_weight1;
     a.norm_w3 = norm_weight2; a.q_stride = mmf_codes_bytes(M, K, 1); a.q = q; a.deq = deq; a.qsum = qsum; a.M = M; a.K = K;
     a.inv_K = 1.0 / (double)K; a.Kp = mmf_round_up(K, 128); a.eps1 = eps1; a.eps = eps;
+    if (const int rc = mmf_set_ahead(a.ahead, ahead, ahead_bytes)) return rc;
     return run_fused_quant(a, QPRO_NORM, x_dtype, weight_dtype, stream);
 }
 
