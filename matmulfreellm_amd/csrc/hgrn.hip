@@ -190,7 +190,7 @@ __global__ __launch_bounds__(64 * NW) void hgrn_recurrent_pipelined_kernel(const
 // sets of registers in turn, without copies between them.  bf16 in us, against branches, copies and the exact gate math: 8 x 2048 x 2048
 // 95 -> 63 (201 MB: 3.2 TB/s), 16 x 900 x 1024 42 -> 28, 2 x 1001 x 2048 24 -> 17, 3 x 459 x 2048 16 -> 12, 64 x 32 x 2048 23 -> 17, 4 x 300 x 1024
 // 9.5 -> 7.1, 1 x 77 x 1024 5.1 -> 4.7.  With few columns time is wave 0's own, 12 ns a step (1 x 2048 x 1024 40 -> 28; half as many channels a
-// workgroup: 28).
+// workgroup: 28).  hgrn_gate_scan_kernel takes single channels (odd widths and strides, rows beyond 256 KiB), the kernel behind it pairs.
 struct GateScanArgs {
     const void* i; const void* f;       // rows [B * T, D], row strides ldi, ldf
     const float* lb; const uint8_t* mask;
@@ -198,13 +198,73 @@ struct GateScanArgs {
     void* o;                            // [B * T, D]
     int64_t ldi, ldf, D;
     int T;
+    int span;                           // pairs: tiles between two shifts of the bases
 };
 __device__ __forceinline__ void lds_only_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// Wave 0: time, tile after tile.  gx, hb: two tiles of (gate, input) and of states.
+template <int CPW, int TT, int U>
+__device__ __forceinline__ void walk_time(const GateScanArgs& a, const float2* gx, float* hb, int64_t d, bool active, int turns) {
+    static_assert(TT % (2 * U) == 0, "the recurrence walks a full tile in pairs of groups");
+    const int lane = threadIdx.x & 63, c = lane & (CPW - 1);
+    const int64_t dd = active ? d : 0;
+    __builtin_amdgcn_s_setprio(3);
+    float h = a.h0 && active ? a.h0[(int64_t)blockIdx.y * a.D + dd] : 0.0f;
+    lds_only_barrier();                                     // tile 0 is there
+    for (int k = 0; k < turns; ++k) {
+        const int n = a.T - k * TT < TT ? a.T - k * TT : TT;   // (<= 0 in the turn that evens their number)
+        const float2* src = gx + (k & 1) * (TT * CPW) + c;
+        float* dst = hb + (k & 1) * (TT * CPW) + c;
+        float2 va[U], vb[U];                                // groups of steps, read one ahead
+        auto read = [&](float2 (&v)[U], int j) __attribute__((always_inline)) {
+            const float2* p = src + (j <= TT - U ? j : TT - U) * CPW;
+#pragma unroll
+            for (int u = 0; u < U; ++u) v[u] = p[u * CPW];
+            __builtin_amdgcn_sched_barrier(0);              // in front of the group walked meanwhile, not behind it (2 x 1001: 17.7 -> 16.8 us)
+        };
+        auto walk = [&](const float2 (&v)[U], int j) __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                h = __fadd_rn(__fmul_rn(v[u].x, h), v[u].y);
+                dst[(j + u) * CPW] = h;
+            }
+        };
+        auto walk_tail = [&](const float2 (&v)[U], int j) __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (j + u < n) {
+                    h = __fadd_rn(__fmul_rn(v[u].x, h), v[u].y);
+                    dst[(j + u) * CPW] = h;
+                }
+            }
+        };
+        if (lane < CPW) {
+            read(va, 0);
+            int j = 0;
+            for (; j + 2 * U <= n; j += 2 * U) {
+                read(vb, j + U);
+                walk(va, j);
+                __builtin_amdgcn_sched_barrier(0);
+                read(va, j + 2 * U);
+                walk(vb, j + U);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (j + U <= n) {                               // what is left of the last tile
+                read(vb, j + U);
+                walk(va, j);
+                walk_tail(vb, j + U);
+            } else if (j < n) {
+                walk_tail(va, j);
+            }
+        }
+        lds_only_barrier();
+    }
+    if (a.ht && active && lane < CPW) a.ht[(int64_t)blockIdx.y * a.D + d] = h;
+}
 
 template <typename T, int CPW, int PASS, bool MASK>
 __global__ __launch_bounds__(1024) void hgrn_gate_scan_kernel(GateScanArgs a) {
     constexpr int NP = 15, SPW = 64 / CPW, TT = NP * SPW * PASS, U = TT >= 60 ? 10 : 5;   // steps of a tile: 120 (60), 60 or 30
-    static_assert(TT % (2 * U) == 0, "the recurrence walks a full tile in pairs of groups");
     __shared__ float2 gx[2][TT * CPW];
     __shared__ float hb[2][TT * CPW];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -218,58 +278,7 @@ __global__ __launch_bounds__(1024) void hgrn_gate_scan_kernel(GateScanArgs a) {
     const int NT = (a.T + TT - 1) / TT, turns = NT + NT % 2;
 
     if (wave == 0) {
-        __builtin_amdgcn_s_setprio(3);
-        float h = a.h0 && active ? a.h0[(int64_t)blockIdx.y * a.D + dd] : 0.0f;
-        lds_only_barrier();                                     // tile 0 is there
-        for (int k = 0; k < turns; ++k) {
-            const int n = a.T - k * TT < TT ? a.T - k * TT : TT;   // (<= 0 in the turn that evens their number)
-            const float2* src = gx[k & 1] + c;
-            float* dst = hb[k & 1] + c;
-            float2 va[U], vb[U];                                // groups of steps, read one ahead
-            auto read = [&](float2 (&v)[U], int j) __attribute__((always_inline)) {
-                const float2* p = src + (j <= TT - U ? j : TT - U) * CPW;
-#pragma unroll
-                for (int u = 0; u < U; ++u) v[u] = p[u * CPW];
-                __builtin_amdgcn_sched_barrier(0);              // in front of the group walked meanwhile, not behind it (2 x 1001: 17.7 -> 16.8 us)
-            };
-            auto walk = [&](const float2 (&v)[U], int j) __attribute__((always_inline)) {
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    h = __fadd_rn(__fmul_rn(v[u].x, h), v[u].y);
-                    dst[(j + u) * CPW] = h;
-                }
-            };
-            auto walk_tail = [&](const float2 (&v)[U], int j) __attribute__((always_inline)) {
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    if (j + u < n) {
-                        h = __fadd_rn(__fmul_rn(v[u].x, h), v[u].y);
-                        dst[(j + u) * CPW] = h;
-                    }
-                }
-            };
-            if (lane < CPW) {
-                read(va, 0);
-                int j = 0;
-                for (; j + 2 * U <= n; j += 2 * U) {
-                    read(vb, j + U);
-                    walk(va, j);
-                    __builtin_amdgcn_sched_barrier(0);
-                    read(va, j + 2 * U);
-                    walk(vb, j + U);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                if (j + U <= n) {                               // what is left of the last tile
-                    read(vb, j + U);
-                    walk(va, j);
-                    walk_tail(vb, j + U);
-                } else if (j < n) {
-                    walk_tail(va, j);
-                }
-            }
-            lds_only_barrier();
-        }
-        if (a.ht && active && lane < CPW) a.ht[(int64_t)blockIdx.y * a.D + d] = h;
+        walk_time<CPW, TT, U>(a, &gx[0][0], &hb[0][0], d, active, turns);
         return;
     }
 
@@ -374,10 +383,156 @@ __global__ __launch_bounds__(1024) void hgrn_gate_scan_kernel(GateScanArgs a) {
     }
 }
 
+// The same where rows and pointers allow two channels at once: a lane takes a pair of channels of one step, so a turn is one request each for i, f
+// and the store, and one LDS vector each way, instead of two, and the resources stand for the whole sequence: offsets advance by a vector add where the
+// bases of every tile took some 70 scalar operations a turn.  NP waves feed the one that walks: 15, or 8 for up to 512 steps, whose tiles of 64
+// are sooner ready.  us, single channels and pairs: 8 x 2048 x 2048 bf16 73.9 and 67.8 (2.97 TB/s), 8 x 512 x 2048 22.8 and 19.3, 16 x 1000 x 1024 38.1 and
+// 32.1, 64 x 32 x 2048 17.3 and 15.9, 3 x 459 x 2048 fp16 13.3 and 12.4, 1 x 77 x 1024 4.6 and 4.5; 1 x 2000 x 1024 28.3 and 28.1, the walk itself: 12.5 ns a step, two
+// dependent operations and one LDS access.  Where there are many columns the vector units bound it: with neither the test of the near forms nor
+// their fall-back 8 x 2048 x 2048 takes 42 us, without gate math 38.
+template <typename T, int CPW, int NP, bool MASK>
+__global__ __launch_bounds__(64 * (NP + 1)) void hgrn_gate_scan_pair_kernel(GateScanArgs a) {
+    constexpr int CP = CPW / 2, SPW = 64 / CP, TT = NP * SPW, U = TT % 20 == 0 ? 10 : TT % 16 == 0 ? 8 : 5, e = (int)sizeof(T), kRsrcFlags = 0x00020000;
+    __shared__ __align__(16) float2 gx[2][TT * CPW];
+    __shared__ __align__(16) float hb[2][TT * CPW];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const unsigned cbs = ((unsigned)a.D + CPW - 1) / CPW;       // workgroups of a sequence
+    unsigned cb = blockIdx.x;
+    if (CPW == 16 && cbs % 32 == 0) cb = (cb & ~31u) + (cb & 7u) * 4 + ((cb >> 3) & 3u);
+    if (CPW == 32 && cbs % 16 == 0) cb = (cb & ~15u) + (cb & 7u) * 2 + ((cb >> 3) & 1u);
+    const int64_t r0 = (int64_t)blockIdx.y * a.T;
+    const int NT = (a.T + TT - 1) / TT, turns = NT + NT % 2;
+    if (wave == 0) {
+        const int64_t d = (int64_t)cb * CPW + (lane & (CPW - 1));
+        walk_time<CPW, TT, U>(a, &gx[0][0], &hb[0][0], d, d < a.D, turns);
+        return;
+    }
+    using V = typename std::conditional<sizeof(T) == 4, uint2, uint32_t>::type;   // a pair as loaded
+    const int p = wave - 1, D = (int)a.D;
+    const int d = (int)cb * CPW + 2 * (lane % CP), dd = d < D ? d : 0;            // (D is even)
+    const int step = p * SPW + lane / CP;
+    const float lb0 = a.lb ? a.lb[dd] : 0.0f, lb1 = a.lb ? a.lb[dd + 1] : 0.0f;
+    const int ldi = (int)a.ldi * e, ldf = (int)a.ldf * e, ldo = D * e;            // bytes
+    const int tile_i = TT * ldi, tile_f = TT * ldf, tile_o = TT * ldo;
+    const char* ip = static_cast<const char*>(a.i) + r0 * ldi;
+    const char* fp = static_cast<const char*>(a.f) + r0 * ldf;
+    const uint8_t* mp = MASK ? a.mask + r0 : nullptr;
+    char* op = static_cast<char*>(a.o) + r0 * ldo;
+    // Steps past the sequence load zeros and store nothing: their offsets lie past the resource's records.  So do those of the three stores in
+    // front of the first tile's (unsigned, they wrap) and, by 2^31, those of lanes past D.
+    uint32_t oi = (uint32_t)(step * ldi + dd * e), of = (uint32_t)(step * ldf + dd * e), om = (uint32_t)step;
+    uint32_t oo = (d < D ? (uint32_t)(step * ldo + d * e) : 0x80000000u) - 3u * (uint32_t)tile_o;
+    int rows = a.T, base = 0;                                   // of the sequence, from tile `base` on, where the bases stand
+    auto records = [&](int ld) { return (rows < (a.span + 8) * TT ? rows : (a.span + 8) * TT) * ld; };
+    auto rsrc = [&](const void* ptr, int ld) __attribute__((always_inline)) {
+        const uint64_t b = (uint64_t)ptr;
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((int)b), hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+        return __builtin_amdgcn_make_buffer_rsrc((void*)((uint64_t)hi << 32 | lo), 0, __builtin_amdgcn_readfirstlane(records(ld)), kRsrcFlags);
+    };
+    __amdgpu_buffer_rsrc_t ti = rsrc(ip, ldi), tf = rsrc(fp, ldf), to = rsrc(op, ldo), tm = rsrc(MASK ? (const void*)mp : ip, 1);
+    V ir[2], fr[2];
+    uint8_t mr[2];
+    auto ld2 = [](__amdgpu_buffer_rsrc_t r, uint32_t off) __attribute__((always_inline)) {
+        if constexpr (sizeof(T) == 4) {
+            const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
+            return make_uint2(v[0], v[1]);
+        } else return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);
+    };
+    auto load = [&](auto S) __attribute__((always_inline)) {
+        constexpr int s = decltype(S)::value;
+        ir[s] = ld2(ti, oi);
+        fr[s] = ld2(tf, of);
+        if constexpr (MASK) mr[s] = (uint8_t)__builtin_amdgcn_raw_buffer_load_b8(tm, om, 0, 0);
+        oi += (uint32_t)tile_i;
+        of += (uint32_t)tile_f;
+        om += TT;
+    };
+    auto floats_of = [](V v, float (&f)[2]) __attribute__((always_inline)) {
+        if constexpr (sizeof(T) == 4) { f[0] = __uint_as_float(v.x); f[1] = __uint_as_float(v.y); }
+        else { f[0] = mmf_to_float(mmf_from_bits16<T>((uint16_t)v)); f[1] = mmf_to_float(mmf_from_bits16<T>((uint16_t)(v >> 16))); }
+    };
+    auto gates = [&](int k, auto S) __attribute__((always_inline)) {
+        constexpr int s = decltype(S)::value;
+        float iv[2], fv[2], xo[2], go[2];
+        const float lbv[2] = {lb0, lb1};
+        floats_of(ir[s], iv);
+        floats_of(fr[s], fv);
+        mmf_gate_n<T, 2>(iv, fv, lbv, xo, go);
+        if constexpr (MASK) {
+            xo[0] = mr[s] == 0 ? 0.0f : xo[0];
+            xo[1] = mr[s] == 0 ? 0.0f : xo[1];
+        }
+        *reinterpret_cast<float4*>(&gx[k & 1][(p * 64 + lane) * 2]) = make_float4(go[0], xo[0], go[1], xo[1]);
+    };
+    float2 hv;                                                  // outputs on their way from LDS to memory
+    auto fetch = [&](int k) __attribute__((always_inline)) { hv = *reinterpret_cast<const float2*>(&hb[k & 1][(p * 64 + lane) * 2]); };
+    auto put = [&]() __attribute__((always_inline)) {
+        if constexpr (sizeof(T) == 4) {
+            typedef unsigned u2 __attribute__((ext_vector_type(2)));
+            __builtin_amdgcn_raw_buffer_store_b64(u2{__float_as_uint(hv.x), __float_as_uint(hv.y)}, to, oo, 0, 0);
+        } else {
+            const uint32_t w = (uint32_t)mmf_bits16(mmf_from_float<T>(hv.x)) | (uint32_t)mmf_bits16(mmf_from_float<T>(hv.y)) << 16;
+            __builtin_amdgcn_raw_buffer_store_b32(w, to, oo, 0, 0);
+        }
+        oo += (uint32_t)tile_o;
+    };
+    fetch(0);
+    load(IntC<0>{});
+    load(IntC<1>{});
+    put();                                                      // nothing: the count of a turn
+    gates(0, IntC<0>{});
+    load(IntC<0>{});
+    put();
+    lds_only_barrier();
+    // wave 0 walks tile k: store tile k - 1, whose outputs are read first and arrive under the arithmetic; prepare tile k + 1 (set S)
+    auto turn = [&](int k, auto S) __attribute__((always_inline)) {
+        if (k - base > a.span) {                                // offsets stay below 2^30: the bases move to tile k - 1
+            const int n = k - 1 - base;
+            base += n;
+            rows -= n * TT;
+            ip += (int64_t)n * tile_i; fp += (int64_t)n * tile_f; op += (int64_t)n * tile_o;
+            oi -= (uint32_t)n * (uint32_t)tile_i; of -= (uint32_t)n * (uint32_t)tile_f; oo -= (uint32_t)n * (uint32_t)tile_o;
+            ti = rsrc(ip, ldi); tf = rsrc(fp, ldf); to = rsrc(op, ldo);
+            if constexpr (MASK) {
+                mp += n * TT;
+                om -= (uint32_t)(n * TT);
+                tm = rsrc(mp, 1);
+            }
+        }
+        fetch(k - 1);
+        if (k + 1 < NT) gates(k + 1, S);
+        load(S);
+        put();
+        lds_only_barrier();
+    };
+    for (int k = 0; k < NT; k += 2) {                           // (an odd number of tiles: one more turn, of nothing but the last store)
+        turn(k, IntC<1>{});
+        turn(k + 1, IntC<0>{});
+    }
+    if (NT % 2 == 0) {
+        fetch(NT - 1);
+        put();
+    }
+}
+
 template <typename T, bool MASK>
-int launch_gate_scan_masked(const GateScanArgs& a, int64_t B, hipStream_t s) {
+int launch_gate_scan_masked(GateScanArgs a, int64_t B, hipStream_t s) {
     const int64_t D = a.D;
     auto grid = [&](int64_t cpw) { return dim3((unsigned)mmf_ceil_div(D, cpw), (unsigned)B); };
+    auto even = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % (2 * sizeof(T)) == 0; };
+    const int64_t row = (a.ldi > a.ldf ? a.ldi : a.ldf) * (int64_t)sizeof(T);   // (the outputs' rows, D, are no longer)
+    // pairs of channels: faster at every size (hgrn_gate_scan_pair_kernel has the times); 2^18 bytes a row keep 16 tiles within 2^29
+    if (D % 2 == 0 && a.ldi % 2 == 0 && a.ldf % 2 == 0 && even(a.i) && even(a.f) && even(a.o) && row <= (1 << 18)) {
+        a.span = (int)((1 << 29) / (128 * row));                // at least 16; offsets reach (span + 8) tiles
+        if (a.span > (1 << 20)) a.span = 1 << 20;
+        if (B * mmf_ceil_div(D, (int64_t)16) <= 512) {
+            if (a.T <= 512) hgrn_gate_scan_pair_kernel<T, 16, 8, MASK><<<grid(16), 64 * (8 + 1), 0, s>>>(a);
+            else hgrn_gate_scan_pair_kernel<T, 16, 15, MASK><<<grid(16), 1024, 0, s>>>(a);
+        } else if (B * mmf_ceil_div(D, (int64_t)32) <= 512) hgrn_gate_scan_pair_kernel<T, 32, 15, MASK><<<grid(32), 1024, 0, s>>>(a);
+        else hgrn_gate_scan_pair_kernel<T, 64, 15, MASK><<<grid(64), 1024, 0, s>>>(a);
+        MMF_CHECK_LAUNCH();
+        return 0;
+    }
     if (B * mmf_ceil_div(D, (int64_t)16) <= 512) {
         // short sequences: half the steps a tile, so that the recurrence starts sooner
         if (a.T <= 512) hgrn_gate_scan_kernel<T, 16, 1, MASK><<<grid(16), 1024, 0, s>>>(a);

@@ -26,3 +26,23 @@ def test_gate_scan_equals_gate_then_scan(dev, b, d, t, dtype):
                                                 F.L.ptr(mask) if use_mask else None, F.L.ptr(h0) if use_h0 else None, o.data_ptr(),
                                                 ht.data_ptr(), b, t, d, F.L.dtype_id(dtype), F.L.stream()), "gate_scan")
         assert torch.equal(o.view(b, t, d), want.view(b, t, d)) and torch.equal(ht, last.view(b, d))
+
+
+# single channels (odd widths and strides) and pairs; rows of 256 KiB, whose bases move every 16 tiles (of 120 steps), and more
+@pytest.mark.parametrize("b,t,d,ld", [(2, 130, 41, 123), (1, 65, 40, 121), (3, 700, 34, 102), (1, 4100, 16, 131072), (2, 2161, 18, 131072), (1, 300, 32, 131072),
+                                      (1, 130, 32, 140000), (9, 2100, 128, 32768)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_single_channels_and_pairs(dev, b, t, d, ld, dtype):
+    import matmulfreellm_amd.functional as F
+    torch.manual_seed(t)
+    if dtype == torch.float32 and ld > 100000:
+        ld //= 2
+    wide = torch.randn(b * t, ld, device=dev).to(dtype)
+    i, f = wide[:, :d], wide[:, ld - d - ld % 2:ld - ld % 2]
+    lb, mask = torch.rand(d, device=dev), (torch.rand(b * t, device=dev) > 0.2).to(torch.uint8)
+    x, g = F.hgrn_gate(i.contiguous(), f.contiguous(), lb, mask)
+    want, last = F.hgrn_recurrent(x.view(b, 1, t, d), g.view(b, 1, t, d), None, True)
+    o, ht = torch.empty(b * t, d, dtype=dtype, device=dev), torch.empty(b, d, device=dev)
+    F.L.check(F.L.load().mmf_hgrn_gate_scan(i.data_ptr(), ld, f.data_ptr(), ld, F.L.ptr(lb), F.L.ptr(mask), None, o.data_ptr(), ht.data_ptr(), b, t, d,
+                                            F.L.dtype_id(dtype), F.L.stream()), "gate_scan")
+    assert torch.equal(o.view(b, t, d), want.view(b, t, d)) and torch.equal(ht, last.view(b, d))
