@@ -24,7 +24,7 @@
 // neighbouring lanes hit different banks; a thread merges runs of equal bins before it touches LDS), a suffix scan of
 // the bins by one wave, and the digit whose bin straddles P.  The top_k-th largest scaled logit comes from the same
 // descent on token counts over an order-preserving integer image of the floats, BEFORE the exp: only the kept tokens
-// (some 50 of 32000) then pay for it.
+// (some 50 of 32000) then pay for it.  Limits of at most 64 take no descent at all where they can (samp_pick_few).
 #include "mmf_common.h"
 
 namespace {
@@ -127,6 +127,161 @@ __device__ __forceinline__ unsigned samp_descent(const unsigned (&m)[NPT], u64 l
     return prefix;
 }
 
+// One wave, n <= 64 kept tokens with their masses in any order: the nucleus and the draw by direct comparison (64 x 64), same rule as below.
+__device__ __forceinline__ void samp_finish_few(const unsigned* few_m, const int* few_i, int n, float top_p, float u, int64_t* out) {
+    const int lane = threadIdx.x & 63;
+    const unsigned mi = lane < n ? few_m[lane] : 0u;
+    const int ii = lane < n ? few_i[lane] : 0x7fffffff;
+    u64 Zf = mi;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) Zf += samp_shfl_down(Zf, o);
+    Zf = ((u64)(unsigned)__builtin_amdgcn_readfirstlane((int)(Zf >> 32)) << 32) | (unsigned)__builtin_amdgcn_readfirstlane((int)Zf);
+    u64 Pf = (u64)((double)top_p * (double)Zf);
+    if (Pf < 1) Pf = 1;
+    u64 heavier = 0;
+#pragma unroll
+    for (int j = 0; j < 64; ++j) {
+        const unsigned mj = (unsigned)__builtin_amdgcn_readlane((int)mi, j);
+        heavier += mj > mi ? mj : 0u;
+    }
+    const unsigned kept = (mi != 0u && heavier < Pf) ? mi : 0u;
+    u64 Sf = kept;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) Sf += samp_shfl_down(Sf, o);
+    Sf = ((u64)(unsigned)__builtin_amdgcn_readfirstlane((int)(Sf >> 32)) << 32) | (unsigned)__builtin_amdgcn_readfirstlane((int)Sf);
+    float uf = u;
+    uf = uf >= 0.0f ? uf : 0.0f;
+    u64 target = (u64)((double)uf * (double)Sf);
+    if (target >= Sf) target = Sf - 1;
+    u64 before = 0;                                   // kept mass at lower vocabulary indices
+#pragma unroll
+    for (int j = 0; j < 64; ++j) {
+        const unsigned kj = (unsigned)__builtin_amdgcn_readlane((int)kept, j);
+        const int ij = __builtin_amdgcn_readlane(ii, j);
+        before += ij < ii ? kj : 0u;
+    }
+    if (kept != 0u && before <= target && target < before + kept) *out = ii;
+}
+
+// The tokens of a limit of at most 64, without a histogram: a bound below the top_k-th largest logit first, then exact ranks among the few
+// logits that reach it.  Scaling does not change the order, so only those are divided.  The bound: every wave's fourth largest (or third, ..: 16 waves have top_k
+// between them) of its threads' maxima, the least of them; a thread's logits come from all over the vocabulary, so that no wave has only rare
+// tokens.  200 to 300 of 32000 normal logits reach it.  Two unequal logits can scale to equal ones: what lies less than 2^-21 below the
+// bound is ranked too, and a bound whose scaled value is not in the middle range, where that covers such pairs, decides nothing.
+// Returns the number of kept tokens (more than top_k on ties), their masses and places in ps.mass, ps.at; -1, for the whole workgroup, when the
+// caller has to go the general way.
+// Bound by latency: a row has one CU, whose waves wait for each other four times.  32000 logits, limit 50, 1 to 64 rows, us, descent and ranks: bf16 23.0 to
+// 24.9 and 10.2 to 11.7, fp16 22.8 to 24.7 and 9.0 to 12.3, fp32 33 and 21 to 24 (128 KB through one CU); limit 64 with ties at it 39.5 to 41.6 and 10.8 to
+// 12.7, limit 1 22 and 8.  What goes the general way after all pays 7 us for the attempt.
+constexpr int kPickMax = 1024;
+struct PickShared { float l[kPickMax], top[kSampWaves], low[kSampWaves]; int idx[kPickMax], at[kPickMax]; unsigned mass[kPickMax], kept[kPickMax]; int n, few; };
+template <typename T, int NPT>
+__device__ __forceinline__ int samp_pick_few(const T* row, int V, bool vec_ok, int top_k, float temperature, PickShared& ps) {
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    Raw8<T> raw[NPT / 8];
+#pragma unroll
+    for (int c = 0; c < NPT / 8; ++c) raw[c] = mmf_load8_raw<T>(row, ((int64_t)c * kSampThreads + t) * 8, V, vec_ok);
+    if (t == 0) { ps.n = 0; ps.few = 0; }
+    float x[NPT], most = -INFINITY;
+#pragma unroll
+    for (int c = 0; c < NPT / 8; ++c) {
+        float v[8];
+        mmf_unpack8<T>(raw[c], v);
+        const int at = (c * kSampThreads + t) * 8;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            x[c * 8 + i] = at + i < V ? v[i] : -INFINITY;
+            most = fmaxf(most, x[c * 8 + i]);                     // (NaN counts as -inf, here and in the comparisons below)
+        }
+    }
+    const int q = (top_k + kSampWaves - 1) / kSampWaves;
+    float rest = most, first = 0.0f, low = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (i < q) {
+            low = mmf_wave_max(rest);
+            if (i == 0) first = low;
+            const u64 at = __builtin_amdgcn_ballot_w64(rest == low);
+            if (at != 0 && lane == (int)__builtin_ctzll(at)) rest = -INFINITY;
+        }
+    }
+    if (lane == 0) { ps.top[wave] = first; ps.low[wave] = low; }
+    __syncthreads();
+    float mx = -INFINITY;
+    low = INFINITY;
+#pragma unroll
+    for (int w = 0; w < kSampWaves; ++w) {
+        mx = fmaxf(mx, ps.top[w]);
+        low = fminf(low, ps.low[w]);
+    }
+    const float scaled = fabsf(__fdiv_rn(low, temperature));
+    if (!(fabsf(low) >= 0x1p-100f && fabsf(low) <= 0x1p100f && scaled >= 0x1p-100f && scaled <= 0x1p100f)) return -1;
+    const float cut = __fsub_rn(low, __fmul_rn(fabsf(low), 0x1p-21f));
+    if (most >= cut) {
+#pragma unroll
+        for (int j = 0; j < NPT; ++j) {
+            if (x[j] >= cut) {
+                const int pos = atomicAdd(&ps.n, 1);
+                if (pos < kPickMax) { ps.l[pos] = __fdiv_rn(x[j], temperature); ps.idx[pos] = ((j >> 3) * kSampThreads + t) * 8 + (j & 7); }
+            }
+        }
+    }
+    __syncthreads();
+    const int n = ps.n;
+    if (n > kPickMax) return -1;
+    mx = __fdiv_rn(mx, temperature);
+    if (wave * 64 < n) {
+        const float mine = t < n ? ps.l[t] : -INFINITY;
+        int larger = 0;
+        int j = 0;
+        for (; j + 8 <= n; j += 8) {
+            const float4 a = *reinterpret_cast<const float4*>(&ps.l[j]), b = *reinterpret_cast<const float4*>(&ps.l[j + 4]);
+            larger += (a.x > mine) + (a.y > mine) + (a.z > mine) + (a.w > mine) + (b.x > mine) + (b.y > mine) + (b.z > mine) + (b.w > mine);
+        }
+        for (; j < n; ++j) larger += ps.l[j] > mine;
+        if (t < n && larger < top_k) {                            // = no less than the top_k-th largest
+            const float p = mine == mx ? 1.0f : mmf_exp(__fsub_rn(mine, mx));
+            const int pos = atomicAdd(&ps.few, 1);
+            ps.mass[pos] = (unsigned)__fmul_rn(p, 2147483648.0f);
+            ps.at[pos] = ps.idx[t];
+        }
+    }
+    __syncthreads();
+    return ps.few;
+}
+
+// The nucleus and the draw among up to kPickMax kept tokens (more than 64: ties at the limit), a thread each over all of them.
+__device__ __forceinline__ void samp_finish_listed(PickShared& ps, int n, float top_p, float u, int64_t* out) {
+    const int t = threadIdx.x;
+    const unsigned mine = t < n ? ps.mass[t] : 0u;
+    const int at = t < n ? ps.at[t] : 0;
+    if ((t & ~63) < n) {
+        u64 Z = 0, heavier = 0;
+        for (int j = 0; j < n; ++j) {
+            const unsigned m = ps.mass[j];
+            Z += m;
+            heavier += m > mine ? m : 0u;
+        }
+        u64 P = (u64)((double)top_p * (double)Z);
+        if (P < 1) P = 1;
+        if (t < n) ps.kept[t] = mine != 0u && heavier < P ? mine : 0u;
+    }
+    __syncthreads();
+    if ((t & ~63) < n) {
+        u64 S = 0, before = 0;
+        for (int j = 0; j < n; ++j) {
+            const unsigned m = ps.kept[j];
+            S += m;
+            before += ps.at[j] < at ? m : 0u;
+        }
+        u = u >= 0.0f ? u : 0.0f;
+        u64 target = (u64)((double)u * (double)S);
+        if (target >= S) target = S - 1;
+        const unsigned kept = t < n ? ps.kept[t] : 0u;
+        if (kept != 0u && before <= target && target < before + kept) *out = at;
+    }
+}
+
 template <typename T, int NPT>
 __global__ __launch_bounds__(kSampThreads) void sample_top_p_kernel(SampleArgs a) {
     __shared__ u64 hist[kSampBins * kSampCopies];                // 32 KiB
@@ -146,6 +301,16 @@ __global__ __launch_bounds__(kSampThreads) void sample_top_p_kernel(SampleArgs a
     const int64_t u_at = blockIdx.x + (a.pos ? (int64_t)a.pos[blockIdx.x] * gridDim.x : 0);
     const bool vec_ok = (V % 8) == 0 && (a.ld % 8) == 0 && (reinterpret_cast<uintptr_t>(a.logits) & 15u) == 0;
 
+    if (top_k > 0 && top_k <= 64 && top_k < V) {                  // four of each wave's 64 maxima bound 64 tokens; more maxima a wave cost what they save
+        __shared__ __align__(16) PickShared ps;
+        const int n = samp_pick_few<T, NPT>(row, V, vec_ok, top_k, temperature, ps);
+        if (n >= 0) {
+            if (n > 64) samp_finish_listed(ps, n, top_p, a.u[u_at], a.out + blockIdx.x);
+            else if (wave == 0) samp_finish_few(ps.mass, ps.at, n, top_p, a.u[u_at], a.out + blockIdx.x);
+            return;
+        }
+        // a clustered or tiny vocabulary, a thousand ties, logits out of range: the general way
+    }
     Raw8<T> raw[NPT / 8];
 #pragma unroll
     for (int c = 0; c < NPT / 8; ++c) raw[c] = mmf_load8_raw<T>(row, (int64_t)base + c * 8, V, vec_ok);
@@ -204,40 +369,8 @@ __global__ __launch_bounds__(kSampThreads) void sample_top_p_kernel(SampleArgs a
         __syncthreads();
         const int n = few_n;
         if (n <= 64) {
-            // Few enough for one lane each: the nucleus and the draw by direct comparison (64 x 64), same rule as below.
-            if (wave == 0) {
-                const unsigned mi = lane < n ? few_m[lane] : 0u;
-                const int ii = lane < n ? few_i[lane] : 0x7fffffff;
-                u64 Zf = mi;
-#pragma unroll
-                for (int o = 32; o > 0; o >>= 1) Zf += samp_shfl_down(Zf, o);
-                Zf = ((u64)(unsigned)__builtin_amdgcn_readfirstlane((int)(Zf >> 32)) << 32) | (unsigned)__builtin_amdgcn_readfirstlane((int)Zf);
-                u64 Pf = (u64)((double)top_p * (double)Zf);
-                if (Pf < 1) Pf = 1;
-                u64 heavier = 0;
-#pragma unroll
-                for (int j = 0; j < 64; ++j) {
-                    const unsigned mj = (unsigned)__builtin_amdgcn_readlane((int)mi, j);
-                    heavier += mj > mi ? mj : 0u;
-                }
-                const unsigned kept = (mi != 0u && heavier < Pf) ? mi : 0u;
-                u64 Sf = kept;
-#pragma unroll
-                for (int o = 32; o > 0; o >>= 1) Sf += samp_shfl_down(Sf, o);
-                Sf = ((u64)(unsigned)__builtin_amdgcn_readfirstlane((int)(Sf >> 32)) << 32) | (unsigned)__builtin_amdgcn_readfirstlane((int)Sf);
-                float uf = a.u[u_at];
-                uf = uf >= 0.0f ? uf : 0.0f;
-                u64 target = (u64)((double)uf * (double)Sf);
-                if (target >= Sf) target = Sf - 1;
-                u64 before = 0;                                   // kept mass at lower vocabulary indices
-#pragma unroll
-                for (int j = 0; j < 64; ++j) {
-                    const unsigned kj = (unsigned)__builtin_amdgcn_readlane((int)kept, j);
-                    const int ij = __builtin_amdgcn_readlane(ii, j);
-                    before += ij < ii ? kj : 0u;
-                }
-                if (kept != 0u && before <= target && target < before + kept) a.out[blockIdx.x] = ii;
-            }
+            // few enough for one lane each
+            if (wave == 0) samp_finish_few(few_m, few_i, n, top_p, a.u[u_at], a.out + blockIdx.x);
             return;
         }
     } else {

@@ -141,3 +141,27 @@ def test_rejected_arguments(dev):
         F().sample_top_p(logits, 0.5, 1.0, u.double())
     with pytest.raises(MMFError):
         F().sample_top_p(logits.cpu(), 0.5, 1.0, u)
+
+
+@pytest.mark.parametrize("v", [4096, 32000, 65536])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_ranked_tokens_of_a_small_limit(dev, v, dtype):
+    """Limits on both sides of what is ranked (64) and of a wave's share (16), on rows that reach its ends: logits that only scaling makes
+    equal, ties at the limit (65 to 1024 kept, and more), the largest logits next to each other, NaN and infinities among the largest, values
+    near the ends of the float range, rows with fewer finite logits than the limit."""
+    g = torch.Generator().manual_seed(41)
+    rows = 10
+    logits = torch.randn(rows, v, generator=g) * 3
+    logits[1] = 1.0 + torch.randint(0, 64, (v,), generator=g) * 2.0 ** -23            # unequal in single precision, equal once divided
+    logits[2, torch.randperm(v, generator=g)[:300]] = 20.0                            # 300 tie at the limit
+    logits[3, torch.randperm(v, generator=g)[:2000]] = 20.0                           # 2000: not ranked
+    logits[4] = logits[4].sort(descending=True).values                                # the largest in one thread's places
+    logits[5, ::97], logits[5, 5], logits[5, 6] = float("nan"), float("inf"), float("inf")
+    logits[6] *= 1e37                                                                 # out of the middle range: some overflow when scaled
+    logits[7] = (logits[7] * 1e-38)
+    logits[8, 40:] = float("-inf")
+    logits[9] -= 1000.0
+    logits = logits.to(dtype)
+    u = torch.rand(rows, generator=g)
+    for top_k, temperature, top_p in ((1, 0.6, 0.4), (16, 0.7, 1.0), (17, 3.0, 0.9), (50, 0.6, 0.4), (63, 1.0, 0.97), (64, 0.3, 0.8), (65, 0.6, 0.6)):
+        _check_rows(dev, logits, temperature, top_p, u, f"V={v} {dtype} top_k={top_k}", top_k=top_k)
