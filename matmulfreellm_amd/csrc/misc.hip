@@ -34,49 +34,69 @@ __global__ __launch_bounds__(256) void embedding_kernel(const T* __restrict__ ta
     }
 }
 
-// One workgroup of 512 threads per row; 8 elements (16 B for 16-bit types) per thread per pass.  The loads of 8 passes
-// (32768 elements, a whole 32000-wide row) are issued raw before the first compare, so the row costs one memory round
-// trip instead of one per pass.  Lowest index wins ties; NaNs never win.
+// One workgroup of 1024 threads per row, four vectors of 8 elements a thread requested before the first is looked at, so that a 32000-wide row costs one
+// memory round trip.  First the largest value (one operation an element), then the lowest index that holds it, which only the
+// threads whose own maximum it is look for: with an index carried beside every comparison a row took 8.5 us.  us, then and now: bf16 1 row 8.0 and 4.1, 64 rows 8.4
+// and 4.6, 64 rows of 128000 22.6 and 8.7; fp32 64 rows 19.3 and 16.9.
+// NaNs never win; a row of nothing else gives 0.
 template <typename T>
-__global__ __launch_bounds__(512) void argmax_kernel(const T* __restrict__ logits, int64_t ld, int64_t V,
-                                                     int64_t* __restrict__ out) {
-    constexpr int PASSES = 8;
-    __shared__ float best_v[8];
-    __shared__ int64_t best_i[8];
-    const int64_t r = blockIdx.x;
-    const T* row = logits + r * ld;
+__global__ __launch_bounds__(1024) void argmax_kernel(const T* __restrict__ logits, int64_t ld, int64_t V, int64_t* __restrict__ out) {
+    constexpr int VECS = 4;
+    __shared__ float top[16];
+    __shared__ unsigned long long lowest;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const T* row = logits + (int64_t)blockIdx.x * ld;
     const bool vec_ok = (V % 8) == 0 && (ld % 8) == 0 && (reinterpret_cast<uintptr_t>(logits) & 15u) == 0;
-    float bv = -INFINITY;
-    int64_t bi = V;   // larger than any valid index: "nothing yet"
-    for (int64_t base = (int64_t)threadIdx.x * 8; base < V; base += (int64_t)PASSES * 512 * 8) {
-        Raw8<T> raw[PASSES];
+    constexpr int64_t kPass = VECS * 1024 * 8;
+    Raw8<T> raw[VECS];
+    auto load = [&](int64_t at) __attribute__((always_inline)) {
 #pragma unroll
-        for (int p = 0; p < PASSES; ++p) raw[p] = mmf_load8_raw<T>(row, base + (int64_t)p * 512 * 8, V, vec_ok);
+        for (int c = 0; c < VECS; ++c) raw[c] = mmf_load8_raw<T>(row, at + (c * 1024 + t) * 8, V, vec_ok);
+    };
+    float best = __builtin_nanf("");                            // NaN: nothing yet (fmaxf takes the other)
+    int64_t where = 0, last = 0;                                // the pass this thread's maximum was first seen in, the pass in its registers
+    for (int64_t at = 0; at < V; at += kPass) {
+        load(at);
+        last = at;
+        float most = __builtin_nanf("");
 #pragma unroll
-        for (int p = 0; p < PASSES; ++p) {
-            const int64_t c0 = base + (int64_t)p * 512 * 8;
+        for (int c = 0; c < VECS; ++c) {
             float v[8];
-            mmf_unpack8<T>(raw[p], v);
+            mmf_unpack8<T>(raw[c], v);
+            const int64_t c0 = at + (c * 1024 + t) * 8;
+            if (c0 + 8 <= V) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int64_t c = c0 + i;
-                if (c < V && (v[i] > bv || (bi == V && v[i] == v[i]))) { bv = v[i]; bi = c; }   // ascending c: first max kept
+                for (int i = 0; i < 8; ++i) most = fmaxf(most, v[i]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) most = c0 + i < V ? fmaxf(most, v[i]) : most;
             }
         }
+        if (most > best || (best != best && most == most)) { best = most; where = at; }
     }
-    for (int o = 32; o > 0; o >>= 1) {
-        const float ov = __shfl_xor(bv, o, 64);
-        const int64_t oi = __shfl_xor(bi, o, 64);
-        if (oi < V && (bi == V || ov > bv || (ov == bv && oi < bi))) { bv = ov; bi = oi; }
-    }
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) { best_v[w] = bv; best_i[w] = bi; }
+    const float mine = mmf_wave_max(best);
+    if (lane == 0) top[wave] = mine;
+    if (t == 0) lowest = (unsigned long long)V;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int i = 1; i < 8; ++i)
-            if (best_i[i] < V && (bi == V || best_v[i] > bv || (best_v[i] == bv && best_i[i] < bi))) { bv = best_v[i]; bi = best_i[i]; }
-        out[r] = bi < V ? bi : 0;
+    float mx = top[0];
+#pragma unroll
+    for (int w = 1; w < 16; ++w) mx = fmaxf(mx, top[w]);
+    if (best == mx) {
+        if (where != last) load(where);
+        unsigned long long idx = (unsigned long long)V;
+#pragma unroll
+        for (int c = VECS - 1; c >= 0; --c) {
+            float v[8];
+            mmf_unpack8<T>(raw[c], v);
+            const int64_t c0 = where + (c * 1024 + t) * 8;
+#pragma unroll
+            for (int i = 7; i >= 0; --i)
+                if (c0 + i < V && v[i] == mx) idx = (unsigned long long)(c0 + i);
+        }
+        atomicMin(&lowest, idx);
     }
+    __syncthreads();
+    if (t == 0) out[blockIdx.x] = lowest < (unsigned long long)V ? (int64_t)lowest : 0;
 }
 
 
@@ -181,9 +201,9 @@ int mmf_argmax(const void* logits, int64_t ld, int64_t rows, int64_t V, int64_t*
     if (rows == 0) return 0;
     if (!logits || !out) return MMF_ERR_ARG;
     switch (dtype) {
-        case MMF_F32: argmax_kernel<float><<<(unsigned)rows, 512, 0, stream>>>(static_cast<const float*>(logits), ld, V, out); break;
-        case MMF_BF16: argmax_kernel<bf16_t><<<(unsigned)rows, 512, 0, stream>>>(static_cast<const bf16_t*>(logits), ld, V, out); break;
-        case MMF_F16: argmax_kernel<f16_t><<<(unsigned)rows, 512, 0, stream>>>(static_cast<const f16_t*>(logits), ld, V, out); break;
+        case MMF_F32: argmax_kernel<float><<<(unsigned)rows, 1024, 0, stream>>>(static_cast<const float*>(logits), ld, V, out); break;
+        case MMF_BF16: argmax_kernel<bf16_t><<<(unsigned)rows, 1024, 0, stream>>>(static_cast<const bf16_t*>(logits), ld, V, out); break;
+        case MMF_F16: argmax_kernel<f16_t><<<(unsigned)rows, 1024, 0, stream>>>(static_cast<const f16_t*>(logits), ld, V, out); break;
         default: return MMF_ERR_ARG;
     }
     MMF_CHECK_LAUNCH();
