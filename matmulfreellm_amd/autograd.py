@@ -267,6 +267,41 @@ def _dense_weight(pw, dtype):
     return w
 
 
+def _turns(dout, y):
+    """Whether mmf_weight_grad takes a product: 16-bit rows of whole, aligned 16-byte pieces."""
+    return y.element_size() == 2 and dout.dtype == y.dtype and len(dout) > 0 and all(
+        t.stride(1) == 1 and t.shape[1] > 0 and t.shape[1] % 8 == 0 and t.stride(0) % 8 == 0 and t.shape[1] <= t.stride(0) <= 1 << 25
+        and t.data_ptr() % 16 == 0 for t in (dout, y))
+
+
+def _turned_products(pairs):
+    """[dout^T @ y] of [M, N] gradients and [M, K] inputs over the same M rows, at most eight, in one launch."""
+    lib, n, m = L.load(), len(pairs), pairs[0][0].shape[0]
+    ptrs, ints = ctypes.c_void_p * n, ctypes.c_int64 * n
+    ns, ks = ints(*[d.shape[1] for d, _ in pairs]), ints(*[y.shape[1] for _, y in pairs])
+    out = [torch.empty(d.shape[1], y.shape[1], dtype=y.dtype, device=y.device) for d, y in pairs]
+    size = lib.mmf_weight_grad_workspace_bytes(n, ns, ks, m)
+    ws = torch.empty(size, dtype=torch.uint8, device=out[0].device) if size else None
+    L.check(lib.mmf_weight_grad(n, ptrs(*[d.data_ptr() for d, _ in pairs]), ints(*[d.stride(0) for d, _ in pairs]),
+                                ptrs(*[y.data_ptr() for _, y in pairs]), ints(*[y.stride(0) for _, y in pairs]),
+                                ptrs(*[o.data_ptr() for o in out]), ns, ks, m, L.dtype_id(out[0].dtype), L.ptr(ws), L.stream()), "mmf_weight_grad")
+    return out
+
+
+def _weight_grads(pairs):
+    """dout^T @ y_q of a block's BitLinears, [M, N] gradients and [M, K] de-quantised inputs; None where the gradients are None.
+
+    In 16 bits two or more go in one launch: each by itself leaves much of the chip idle, or its launch takes longer than it does.  The six of
+    a block, one library product each / together, us: 2048 wide 64 rows 114 / 41, 1024 186 / 123, 8192 916 / 716; 1024 wide 112 / 34 and
+    456 / 206 (1024, 8192 rows).  One alone (2048 x 2048: 1024 rows 21 / 29, 8192 86 / 81) stays with the library."""
+    take = [i for i, p in enumerate(pairs) if p[0] is not None and _turns(*p)]
+    out = [None] * len(pairs)
+    if len(take) >= 2:
+        for i, o in zip(take, _turned_products([pairs[i] for i in take])):
+            out[i] = o
+    return [d.t() @ y if o is None and d is not None else o for o, (d, y) in zip(out, pairs)]
+
+
 def _weight_grad(dout, y):
     """dout^T @ y_q of [M, N] gradients and [M, K] de-quantised inputs.
 
@@ -274,13 +309,17 @@ def _weight_grad(dout, y):
     run at a higher rate then: rows a multiple of 64, from 3000 on of 8.  bf16, us, as they are / transposed: 8192 x 1024 -> 32000 488 / 428,
     8192 x 2048 1097 / 816, 3072 x 2048 10 % less, 1024 x 2048 152 / 131, 5000 rows 7 % less; 1056 rows 20 % more, 2016 5 % more, 2002 and 3001, which
     are no multiple of 8 (the transposition moves single elements), 0 to 7 % more; the same for 16384 to 50304 outputs and in fp16.  For fewer outputs the
-    transposition, 4 bytes an element, costs more of the product (11264: 4 %) than it gives there (-5 to 12 %)."""
+    transposition, 4 bytes an element, costs more of the product (11264: 4 %) than it gives there (-5 to 12 %).
+    Other rows, from 600 on, take mmf_weight_grad: 2048 -> 32000 666 rows 128 us by the library, 105 by it, 2002 rows 266 and 237 (1024 wide 69 and 54, 138 and
+    121); 512 rows 88 and 89.  Where the transposition pays it is 4 to 8 % behind (8192 rows 878 us)."""
     m, k = y.shape
-    whole = m % 64 == 0 if m < 3000 else m % 8 == 0
-    if y.element_size() == 2 and dout.shape[1] >= 16384 and 1024 <= m <= 4194240 and whole and y.is_contiguous():
-        yt = torch.empty(k, m, dtype=y.dtype, device=y.device)
-        L.check(L.load().mmf_transpose16(y.data_ptr(), m, k, yt.data_ptr(), L.stream()), "mmf_transpose16")
-        y = yt.t()
+    if y.element_size() == 2 and dout.shape[1] >= 16384 and y.is_contiguous():
+        if 1024 <= m <= 4194240 and (m % 64 == 0 if m < 3000 else m % 8 == 0):
+            yt = torch.empty(k, m, dtype=y.dtype, device=y.device)
+            L.check(L.load().mmf_transpose16(y.data_ptr(), m, k, yt.data_ptr(), L.stream()), "mmf_transpose16")
+            y = yt.t()
+        elif 600 <= m <= 0x7fffffff and _turns(dout, y):
+            return _turned_products([(dout, y)])[0]
     return dout.t() @ y
 
 
@@ -331,18 +370,18 @@ class BlockFn(torch.autograd.Function):
             dy = torch.empty_like(y)
             _, _, yq, dw_down = _chain_bwd(CHAIN_SWIGLU, y[:, :I], y[:, I:], None, 0.0, [down_n], eps["down_eps"], [dz], dx=dy[:, :I],
                                            daux=dy[:, I:])
-            d_down = d2.t() @ yq[0] if need[14] else None
+            down = (d2 if need[14] else None, yq[0])
             # gate_proj behind mlp_norm, the residual's gradient joining
             dh = dy @ _dense_weight(gate_pw, dt)
             dres, _, yq, dw_gate = _chain_bwd(CHAIN_RESNORM, attn, x.view(m, H), mlp_norm, eps["mlp_eps"], [gate_n], eps["gate_eps"], [dh],
                                                dres=d2)
-            d_gate = dy.t() @ yq[0] if need[13] else None
+            gate = (dy if need[13] else None, yq[0])
             # o_proj behind the gated norm: the g columns of the stacked projection's gradient, and the scan's output
             do2 = dres @ _dense_weight(o_pw, dt)
             difg, do = torch.empty_like(ifg), torch.empty_like(o)
             _, _, yq, dw_o = _chain_bwd(CHAIN_GATED, ifg[:, 2 * D:], o, g_norm, eps["g_eps"], [o_n], eps["o_eps"], [do2],
                                         dx=difg[:, 2 * D:], daux=do)
-            d_o = dres.t() @ yq[0] if need[12] else None
+            o_ = (dres if need[12] else None, yq[0])
             # scan and gate math
             dxs, dgs = _scan_bwd(xg[1].view(b, 1, t, D), o.view(b, 1, t, D), do.view(b, 1, t, D), None, False)
             dlb = torch.empty(D, dtype=torch.float32, device=dev) if lb is not None else None
@@ -358,11 +397,11 @@ class BlockFn(torch.autograd.Function):
                 torch.mm(cols[j], w3[j * D:(j + 1) * D], out=dh3[j])
             dx, _, yq, dw_ifg = _chain_bwd(CHAIN_NORM, x.view(m, H), None, attn_norm, eps["attn_eps"], [i_n, f_n, gp_n], eps["ifg_eps"],
                                            dh3, dres=dres)
-            d_ifg = [cols[j].t() @ yq[j] if need[9 + j] else None for j in range(3)]
+            d_weights = _weight_grads([*[(cols[j] if need[9 + j] else None, yq[j]) for j in range(3)], o_, gate, down])
         grads = [dw_ifg[0], dw_gate[0], dw_o[0], dw_ifg[1], dw_ifg[2], dw_ifg[3], dw_o[1], dw_gate[1], dw_down[0]]
         if dlb is not None:
             dlb = dlb.to(ctx.lb_dtype)
-        return (None, dx.view(x.shape), dlb, None, *grads, *d_ifg, d_o, d_gate, d_down)
+        return (None, dx.view(x.shape), dlb, None, *grads, *d_weights)
 
 
 class NormHeadFn(torch.autograd.Function):

@@ -13,7 +13,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 LIBPATH = os.path.join(LIBDIR, "libmmf_hip.so")
 NATIVE_PATH = os.path.join(LIBDIR, "mmf_torch.so")
-SOURCES = ["norm.hip", "quant_pack.hip", "bitlinear_gemv.hip", "bitlinear_mfma.hip", "hgrn.hip", "misc.hip", "decode_layers.hip", "sampling.hip", "loss.hip", "backward.hip", "hgrn_block.hip", "block_forward.hip", "backward_block.hip", "conv.hip"]
+SOURCES = ["norm.hip", "quant_pack.hip", "bitlinear_gemv.hip", "bitlinear_mfma.hip", "hgrn.hip", "misc.hip", "decode_layers.hip", "sampling.hip", "loss.hip", "backward.hip", "hgrn_block.hip", "block_forward.hip", "backward_block.hip", "conv.hip", "weight_grad.hip"]
 
 # -ffp-contract=off: no multiply-add fusion, so results match a CPU restatement bit for bit.
 # packed-fp32-ops disabled: keep the compiler from forming v_pk_*_f32.
