@@ -99,7 +99,7 @@ SIGNATURES = {
     "mmf_unpack_dequant": (_i32, [_ptr, _ptr, _i64, _i64, _i64, _ptr, _i32, _ptr]),
     "mmf_unpack_dequant_t": (_i32, [_ptr, _ptr, _i64, _i64, _i64, _ptr, _i32, _ptr]),
     "mmf_transpose16": (_i32, [_ptr, _i64, _i64, _ptr, _ptr]),
-    "mmf_weight_grad_workspace_bytes": (_i64, [_i32, _ptr, _ptr, _i64]),
+    "mmf_weight_grad_workspace_bytes": (_i64, [_i32, _ptr, _ptr, _i64, _i32]),
     "mmf_weight_grad": (_i32, [_i32, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i32, _ptr, _ptr]),
     "mmf_block_struct_bytes": (_i64, []),
     "mmf_block_workspace_bytes": (_i64, [_ptr, _i64]),

@@ -268,9 +268,10 @@ def _dense_weight(pw, dtype):
 
 
 def _turns(dout, y):
-    """Whether mmf_weight_grad takes a product: 16-bit rows of whole, aligned 16-byte pieces."""
-    return y.element_size() == 2 and dout.dtype == y.dtype and len(dout) > 0 and all(
-        t.stride(1) == 1 and t.shape[1] > 0 and t.shape[1] % 8 == 0 and t.stride(0) % 8 == 0 and t.shape[1] <= t.stride(0) <= 1 << 25
+    """Whether mmf_weight_grad takes a product: rows of whole, aligned 16-byte pieces."""
+    whole = 16 // y.element_size()
+    return y.dtype in (torch.float32, torch.bfloat16, torch.float16) and dout.dtype == y.dtype and 0 < len(dout) <= 0x7fffffff and all(
+        t.stride(1) == 1 and t.shape[1] > 0 and t.shape[1] % whole == 0 and t.stride(0) % whole == 0 and t.shape[1] <= t.stride(0) <= 1 << 24
         and t.data_ptr() % 16 == 0 for t in (dout, y))
 
 
@@ -280,7 +281,7 @@ def _turned_products(pairs):
     ptrs, ints = ctypes.c_void_p * n, ctypes.c_int64 * n
     ns, ks = ints(*[d.shape[1] for d, _ in pairs]), ints(*[y.shape[1] for _, y in pairs])
     out = [torch.empty(d.shape[1], y.shape[1], dtype=y.dtype, device=y.device) for d, y in pairs]
-    size = lib.mmf_weight_grad_workspace_bytes(n, ns, ks, m)
+    size = lib.mmf_weight_grad_workspace_bytes(n, ns, ks, m, L.dtype_id(out[0].dtype))
     ws = torch.empty(size, dtype=torch.uint8, device=out[0].device) if size else None
     L.check(lib.mmf_weight_grad(n, ptrs(*[d.data_ptr() for d, _ in pairs]), ints(*[d.stride(0) for d, _ in pairs]),
                                 ptrs(*[y.data_ptr() for _, y in pairs]), ints(*[y.stride(0) for _, y in pairs]),
@@ -291,10 +292,15 @@ def _turned_products(pairs):
 def _weight_grads(pairs):
     """dout^T @ y_q of a block's BitLinears, [M, N] gradients and [M, K] de-quantised inputs; None where the gradients are None.
 
-    In 16 bits two or more go in one launch: each by itself leaves much of the chip idle, or its launch takes longer than it does.  The six of
-    a block, one library product each / together, us: 2048 wide 64 rows 114 / 41, 1024 186 / 123, 8192 916 / 716; 1024 wide 112 / 34 and
-    456 / 206 (1024, 8192 rows).  One alone (2048 x 2048: 1024 rows 21 / 29, 8192 86 / 81) stays with the library."""
+    Two or more go in one launch: each by itself leaves much of the chip idle, or its launch takes longer than it does.  The six of a
+    block, one library product each / together, us: bf16, 2048 wide 64 rows 114 / 41, 1024 186 / 123, 8192 916 / 716; 1024 wide 112 / 34 and
+    456 / 206 (1024, 8192 rows); fp32, 1024 wide 666 rows 220 / 143, 2048 wide 591 / 514 and 1522 / 1487 (666, 2002 rows).  One alone
+    (2048 x 2048, bf16: 1024 rows 21 / 29, 8192 86 / 81) stays with the library, and so do many rows of wide blocks in fp32, where each
+    product fills the chip (2048 wide, 4096 rows 2859 / 2999; 1536 wide 1659 / 1671; 1024 wide 801 / 783)."""
     take = [i for i, p in enumerate(pairs) if p[0] is not None and _turns(*p)]
+    if take and pairs[take[0]][1].dtype == torch.float32 and len(pairs[take[0]][1]) > 2048 and sum(
+            pairs[i][0].shape[1] * pairs[i][1].shape[1] for i in take) > 1 << 24:
+        take = []
     out = [None] * len(pairs)
     if len(take) >= 2:
         for i, o in zip(take, _turned_products([pairs[i] for i in take])):
@@ -318,7 +324,7 @@ def _weight_grad(dout, y):
             yt = torch.empty(k, m, dtype=y.dtype, device=y.device)
             L.check(L.load().mmf_transpose16(y.data_ptr(), m, k, yt.data_ptr(), L.stream()), "mmf_transpose16")
             y = yt.t()
-        elif 600 <= m <= 0x7fffffff and _turns(dout, y):
+        elif m >= 600 and _turns(dout, y):
             return _turned_products([(dout, y)])[0]
     return dout.t() @ y
 

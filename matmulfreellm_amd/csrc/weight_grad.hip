@@ -1,4 +1,4 @@
-// The weight gradients of a training step's BitLinears in 16 bits: dw[N, K] = dout[M, N]^T @ y[M, K], several products over the same
+// The weight gradients of a training step's BitLinears: dw[N, K] = dout[M, N]^T @ y[M, K], several products over the same
 // M rows in one launch (the six of an HGRNBitBlock), fp32 sums, one rounding (mmfreelm/ops/fusedbitnet.py:498).
 #include "mmf_common.h"
 
@@ -18,14 +18,15 @@ namespace {
 // products and their transfers in pairs behind them 231; a fifth buffer changes nothing.
 // The six gradients of a 2048-wide block over 8192 rows: 686 us (1.23 PFLOP/s), as a library product each 892; 2048 rows 207 and
 // 270, 1024 rows 118 and 190: by themselves 64 or 352 tiles leave much of the chip idle, 784 together do not.
-constexpr int kSide = 256, kRows = 32, kOperand = kRows * kSide * 2, kBuffer = 2 * kOperand, kBuffers = 4, kCUs = 256, kMaxProducts = 8;
+constexpr int kSide = 256, kSide32 = 128, kRows = 32, kOperand = kRows * kSide * 2, kBuffer = 2 * kOperand, kBuffers = 4, kCUs = 256, kMaxProducts = 8;
+constexpr int kRows32 = 16, kOperand32 = kRows32 * kSide32 * 4, kBuffer32 = 2 * kOperand32, kFlight32 = kBuffer32 / 1024 / 4;
 constexpr int kFlight = kBuffer / 1024 / 4;                         // transfers of 1 KiB that a wave issues per buffer
 constexpr int kMaxSplit = 16;
 
 struct Product {
-    const uint16_t* p;      // dout, row stride ldp
-    const uint16_t* q;      // y, row stride ldq
-    uint16_t* out;          // [N, K]
+    const void* p;          // dout, row stride ldp
+    const void* q;          // y, row stride ldq
+    void* out;              // [N, K]
     int64_t ldp, ldq;
     int N, K, tiles_k, tile0;
 };
@@ -33,7 +34,7 @@ struct GradArgs {
     Product pr[kMaxProducts];
     int n, full, rest, split;       // `full` tiles over all rows, then `rest` tiles in `split` slices of the rows each
     int64_t M;
-    float* part;                    // [split][rest][256 * 256] in the order of waves, accumulators and lanes
+    float* part;                    // [split][rest][side * side] in the order of waves, accumulators and lanes
 };
 
 typedef short v4s __attribute__((ext_vector_type(4)));
@@ -75,14 +76,15 @@ __device__ __forceinline__ uint2 grad_round(float a, float b, float c, float d) 
 // The product that a tile belongs to and its first output: panels of four tiles along K, so that the 32 tiles that an XCD holds at a time
 // share eight strips of dout and four of y.
 struct GradTile { int w, n0, k0; };
+template <int SIDE>
 __device__ __forceinline__ GradTile grad_tile(const GradArgs& a, int tile) {
     GradTile t{0, 0, 0};
     while (t.w + 1 < a.n && tile >= a.pr[t.w + 1].tile0) ++t.w;
     const Product& pr = a.pr[t.w];
-    const int i = tile - pr.tile0, tn = (pr.N + kSide - 1) / kSide, panel = i / (4 * tn), r = i - panel * 4 * tn;
+    const int i = tile - pr.tile0, tn = (pr.N + SIDE - 1) / SIDE, panel = i / (4 * tn), r = i - panel * 4 * tn;
     const int left = pr.tiles_k - panel * 4, width = left < 4 ? left : 4;
-    t.n0 = r / width * kSide;
-    t.k0 = (panel * 4 + r % width) * kSide;
+    t.n0 = r / width * SIDE;
+    t.k0 = (panel * 4 + r % width) * SIDE;
     return t;
 }
 // Workgroup b of `total` runs on XCD b % 8: each XCD walks a stretch of its own.
@@ -102,7 +104,7 @@ __global__ __launch_bounds__(256, 1) void weight_grad_kernel(GradArgs a) {
         slice = piece / a.rest;
         tile = a.full + piece % a.rest;
     }
-    const GradTile t = grad_tile(a, tile);
+    const GradTile t = grad_tile<kSide>(a, tile);
     const Product& pr = a.pr[t.w];
     const int N = pr.N, K = pr.K, n0 = t.n0, k0 = t.k0;
     const int64_t stages = (a.M + kRows - 1) / kRows;
@@ -124,8 +126,8 @@ __global__ __launch_bounds__(256, 1) void weight_grad_kernel(GradArgs a) {
     };
     offsets(count == 1 ? valid : kRows);
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
-    const uint16_t* gp = pr.p + n0 + s0 * kRows * pr.ldp;
-    const uint16_t* gq = pr.q + k0 + s0 * kRows * pr.ldq;
+    const uint16_t* gp = static_cast<const uint16_t*>(pr.p) + n0 + s0 * kRows * pr.ldp;
+    const uint16_t* gq = static_cast<const uint16_t*>(pr.q) + k0 + s0 * kRows * pr.ldq;
     const int64_t stepp = kRows * pr.ldp, stepq = kRows * pr.ldq;
     auto dma = [&](int q, int side, uint32_t into) __attribute__((always_inline)) {
         if (side == 0) grad_dma(gp, offp[q], lds0 + into + (wave * 4 + q) * 1024);
@@ -245,41 +247,169 @@ __global__ __launch_bounds__(256, 1) void weight_grad_kernel(GradArgs a) {
         for (int h = 0; h < 8; ++h) {
             const int row = h * 4 + (lane >> 4), col = (lane & 15) * 8, n = nw + j * 32 + row;
             const uint4 v = *reinterpret_cast<const uint4*>(st + row * kPitch + col * 2);
-            if (n < N && kw + col < K) *reinterpret_cast<uint4*>(pr.out + (int64_t)n * K + kw + col) = v;
+            if (n < N && kw + col < K) *reinterpret_cast<uint4*>(static_cast<uint16_t*>(pr.out) + (int64_t)n * K + kw + col) = v;
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_wave_barrier();
     }
 }
 
-// The slices of the split tiles added up in their order: 64 workgroups of 1024 outputs a tile.
-template <typename T>
-__global__ __launch_bounds__(256) void weight_grad_sum_kernel(GradArgs a) {
-    const int r = (int)blockIdx.x >> 6, sub = (int)blockIdx.x & 63;
-    const GradTile t = grad_tile(a, a.full + r);
+// In single precision the matrix cores are the bound by far (157 TFLOP/s dense): 16 rows of 128 x 128 outputs take 2048 cycles and 16 KiB.  A
+// row of 128 floats is as long as one of 256 16-bit elements and travels as above; a fragment of two rows is read as it lies.  Two
+// workgroups on a CU cover each other's barriers, starts and ends: the six gradients of a 1024-wide block over 666 rows 143 us, one
+// workgroup with buffers of 32 rows 163, and 172 where its transfers left together and no read crossed a stage's end; one library
+// product each 220.  Tiles of 128 leave a smaller rest than tiles of 256.
+__global__ __launch_bounds__(256, 2) void weight_grad32_kernel(GradArgs a) {
+    extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+    const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), wp = wave & 1, wq = wave >> 1;
+    int tile, slice = 0, piece = -1;
+    if ((int)blockIdx.x < a.full) tile = grad_stretch((int)blockIdx.x, a.full);
+    else {
+        piece = grad_stretch((int)blockIdx.x - a.full, a.rest * a.split);
+        slice = piece / a.rest;
+        tile = a.full + piece % a.rest;
+    }
+    const GradTile t = grad_tile<kSide32>(a, tile);
     const Product& pr = a.pr[t.w];
-    const float* o = a.part + (int64_t)r * kSide * kSide + sub * 1024 + (int)threadIdx.x * 4;
+    const int N = pr.N, K = pr.K, n0 = t.n0, k0 = t.k0;
+    const int64_t stages = (a.M + kRows32 - 1) / kRows32;
+    const int64_t s0 = stages * slice / a.split, s1 = piece < 0 ? stages : stages * (slice + 1) / a.split;
+    const int count = (int)(s1 - s0);
+    const int valid = s1 == stages && a.M % kRows32 ? (int)(a.M % kRows32) : kRows32;
+
+    uint32_t offp[2], offq[2];
+    auto offsets = [&](int rows) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int r = wave * 4 + 2 * q + (lane >> 5), src = r < rows ? r : rows - 1, col = (lane & 31) * 4;
+            offp[q] = (uint32_t)(src * (int)pr.ldp + (n0 + col < N ? col : 0)) * 4;
+            offq[q] = (uint32_t)(src * (int)pr.ldq + (k0 + col < K ? col : 0)) * 4;
+        }
+    };
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
+    const float* gp = static_cast<const float*>(pr.p) + n0 + s0 * kRows32 * pr.ldp;
+    const float* gq = static_cast<const float*>(pr.q) + k0 + s0 * kRows32 * pr.ldq;
+    auto dma = [&](int q, int side, uint32_t into) __attribute__((always_inline)) {
+        if (side == 0) grad_dma(gp, offp[q], lds0 + into + (wave * 2 + q) * 1024);
+        else grad_dma(gq, offq[q], lds0 + into + kOperand32 + (wave * 2 + q) * 1024);
+    };
+    v16f acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+    auto clear = [&](uint32_t into) __attribute__((always_inline)) {
+        for (int i = (int)threadIdx.x; i < 2 * (kRows32 - valid) * 32; i += 256) {
+            const int side = i >= (kRows32 - valid) * 32, j = i - side * (kRows32 - valid) * 32;
+            *reinterpret_cast<uint4*>(smem + into + side * kOperand32 + valid * 512 + j * 16) = uint4{0, 0, 0, 0};
+        }
+        grad_barrier<0>();
+    };
+    offsets(count == 1 ? valid : kRows32);
+#pragma unroll
+    for (int b = 0; b < kBuffers - 1; ++b)
+        if (b < count) {
+            if (b > 0 && b == count - 1) offsets(valid);
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                dma(q, 0, b * kBuffer32);
+                dma(q, 1, b * kBuffer32);
+            }
+            gp += kRows32 * pr.ldp;
+            gq += kRows32 * pr.ldq;
+        }
+    if (count >= kBuffers - 1) grad_barrier<(kBuffers - 2) * kFlight32>();
+    else grad_barrier<0>();
+    if (count == 1 && valid < kRows32) clear(0);
+    const unsigned char* atp = smem + (lane >> 5) * 512 + wp * 256 + (lane & 31) * 4;
+    const unsigned char* atq = smem + kOperand32 + (lane >> 5) * 512 + wq * 256 + (lane & 31) * 4;
+    float pf[2][2], qf[2][2];
+    auto read = [&](int set, uint32_t b, int k) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            pf[set][i] = *reinterpret_cast<const float*>(atp + b + k * 1024 + i * 128);
+            qf[set][i] = *reinterpret_cast<const float*>(atq + b + k * 1024 + i * 128);
+        }
+    };
+    read(0, 0, 0);
+    uint32_t buf = 0;
+    for (int s = 0; s < count; ++s) {
+        const uint32_t next = (buf + kBuffer32) & (kBuffers * kBuffer32 - 1), last = (buf - kBuffer32) & (kBuffers * kBuffer32 - 1);
+        const bool more = s + kBuffers - 1 < count;
+        if (s + kBuffers == count && valid < kRows32) offsets(valid);
+#pragma unroll
+        for (int k = 0; k < kRows32 / 2; ++k) {                        // the next two rows arrive under four products
+            if (k + 1 < kRows32 / 2) read((k + 1) & 1, buf, k + 1);
+            else {
+                // Every wave has read this stage's buffer out; of the three stages in flight the next has to be there.
+                if (more) grad_barrier<(kBuffers - 2) * kFlight32>();
+                else grad_barrier<0>();
+                if (s + 2 == count && valid < kRows32) clear(next);
+                read(0, next, 0);                                    // (behind the last stage: what nothing uses)
+            }
+            __builtin_amdgcn_sched_barrier(0);                       // the reads leave first: four products cover them, one would not
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(qf[k & 1][i], pf[k & 1][j], acc[i][j], 0, 0, 0);
+            if (more && k < 4) dma(k >> 1, k & 1, last);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        gp += kRows32 * pr.ldp;
+        gq += kRows32 * pr.ldq;
+        buf = next;
+    }
+    float* o = piece < 0 ? nullptr : a.part + (int64_t)piece * kSide32 * kSide32 + wave * 4096 + lane * 4;
+    float* out = static_cast<float*>(pr.out);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const v4f v = v4f{acc[i][j][4 * e], acc[i][j][4 * e + 1], acc[i][j][4 * e + 2], acc[i][j][4 * e + 3]};
+                const int n = n0 + wp * 64 + j * 32 + (lane & 31), k = k0 + wq * 64 + i * 32 + e * 8 + (lane >> 5) * 4;
+                if (o) *reinterpret_cast<v4f*>(o + ((i * 2 + j) * 4 + e) * 256) = v;
+                else if (n < N && k < K) *reinterpret_cast<v4f*>(out + (int64_t)n * K + k) = v;
+            }
+}
+
+// The slices of the split tiles added up in their order, 1024 outputs a workgroup.
+template <typename T, int SIDE>
+__global__ __launch_bounds__(256) void weight_grad_sum_kernel(GradArgs a) {
+    constexpr int kSubs = SIDE * SIDE / 1024, F = SIDE / 64;          // a wave's tile: F x F fragments, one a workgroup
+    const int r = (int)blockIdx.x / kSubs, sub = (int)blockIdx.x % kSubs;
+    const GradTile t = grad_tile<SIDE>(a, a.full + r);
+    const Product& pr = a.pr[t.w];
+    const float* o = a.part + (int64_t)r * SIDE * SIDE + sub * 1024 + (int)threadIdx.x * 4;
     v4f v = *reinterpret_cast<const v4f*>(o);
     for (int s = 1; s < a.split; ++s) {
-        const v4f w = *reinterpret_cast<const v4f*>(o + (int64_t)s * a.rest * kSide * kSide);
+        const v4f w = *reinterpret_cast<const v4f*>(o + (int64_t)s * a.rest * SIDE * SIDE);
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[i] = __fadd_rn(v[i], w[i]);
     }
-    const int wave = sub >> 4, i = sub >> 2 & 3, j = sub & 3, e = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
-    const int n = t.n0 + (wave & 1) * 128 + j * 32 + (lane & 31), k = t.k0 + (wave >> 1) * 128 + i * 32 + e * 8 + (lane >> 5) * 4;
-    if (n < pr.N && k < pr.K) *reinterpret_cast<uint2*>(pr.out + (int64_t)n * pr.K + k) = grad_round<T>(v[0], v[1], v[2], v[3]);
+    const int wave = sub / (F * F), i = sub / F % F, j = sub % F, e = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
+    const int n = t.n0 + (wave & 1) * (SIDE / 2) + j * 32 + (lane & 31), k = t.k0 + (wave >> 1) * (SIDE / 2) + i * 32 + e * 8 + (lane >> 5) * 4;
+    if (n >= pr.N || k >= pr.K) return;
+    T* out = static_cast<T*>(pr.out) + (int64_t)n * pr.K + k;
+    if constexpr (std::is_same_v<T, float>) *reinterpret_cast<v4f*>(out) = v;
+    else *reinterpret_cast<uint2*>(out) = grad_round<T>(v[0], v[1], v[2], v[3]);
 }
 
 // The tiles behind the last whole round of the chip, cut into slices of the rows where that is estimated to end sooner: microseconds from a stage's
 // 0.85, a workgroup's start and end 5, the second launch 4 and 0.1 per slice written and read.  8192 rows, as they are / cut: one product of
 // 2048 x 2048 (64 tiles, 4 slices) 167 / 80 us, 11264 x 2048 (96 of 352 tiles, 2 slices) 360 / 313, 2048 x 5632 (176 tiles) 179 whole, 228 in 4.
+// Single precision: 0.95 a stage, 0.025 a slice.
 struct GradPlan { int full, rest, split; };
-GradPlan grad_plan(int64_t tiles, int64_t M) {
-    const int64_t stages = mmf_ceil_div(M, kRows), rest = tiles % kCUs;
+GradPlan grad_plan(int64_t tiles, int64_t M, bool f32) {
+    const int64_t stages = mmf_ceil_div(M, f32 ? kRows32 : kRows), rest = tiles % kCUs;
+    const double stage = f32 ? 0.95 : 0.85, slice = f32 ? 0.025 : 0.1;
     int best = 1;
     double least = 0.0;
-    for (int s = 1; s <= kMaxSplit && stages / s >= 4; ++s) {
-        const double us = (double)mmf_ceil_div(rest * s, kCUs) * ((double)mmf_ceil_div(stages, s) * 0.85 + 5.0) + (s > 1 ? 4.0 + 0.1 * (double)(rest * s) : 0.0);
+    for (int s = 1; s <= kMaxSplit && stages / s >= (f32 ? 2 : 4); ++s) {
+        const double us = (double)mmf_ceil_div(rest * s, kCUs) * ((double)mmf_ceil_div(stages, s) * stage + 5.0) + (s > 1 ? 4.0 + slice * (double)(rest * s) : 0.0);
         if (s == 1 || us < least) {
             best = s;
             least = us;
@@ -288,21 +418,26 @@ GradPlan grad_plan(int64_t tiles, int64_t M) {
     if (rest == 0 || best == 1) return GradPlan{(int)tiles, 0, 1};
     return GradPlan{(int)(tiles - rest), (int)rest, best};
 }
-int64_t grad_tiles(int n, const int64_t* N, const int64_t* K) {
+int64_t grad_tiles(int n, const int64_t* N, const int64_t* K, int side) {
     int64_t t = 0;
-    for (int i = 0; i < n; ++i) t += mmf_ceil_div(N[i], kSide) * mmf_ceil_div(K[i], kSide);
+    for (int i = 0; i < n; ++i) t += mmf_ceil_div(N[i], side) * mmf_ceil_div(K[i], side);
     return t;
 }
 
 template <typename T>
 int launch_grad(const GradArgs& a, hipStream_t s) {
-    auto kern = weight_grad_kernel<T>;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kBuffers * kBuffer);
+    constexpr bool f32 = std::is_same_v<T, float>;
+    constexpr int side = f32 ? kSide32 : kSide;
+    void (*kern)(GradArgs);
+    if constexpr (f32) kern = weight_grad32_kernel;
+    else kern = weight_grad_kernel<T>;
+    constexpr int lds = kBuffers * (f32 ? kBuffer32 : kBuffer);
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e != hipSuccess) return (int)e;
-    kern<<<(unsigned)(a.full + a.rest * a.split), 256, kBuffers * kBuffer, s>>>(a);
+    kern<<<(unsigned)(a.full + a.rest * a.split), 256, lds, s>>>(a);
     MMF_CHECK_LAUNCH();
     if (a.rest) {
-        weight_grad_sum_kernel<T><<<(unsigned)a.rest * 64u, 256, 0, s>>>(a);
+        weight_grad_sum_kernel<T, side><<<(unsigned)(a.rest * (side * side / 1024)), 256, 0, s>>>(a);
         MMF_CHECK_LAUNCH();
     }
     return 0;
@@ -312,36 +447,46 @@ int launch_grad(const GradArgs& a, hipStream_t s) {
 
 extern "C" {
 
-int64_t mmf_weight_grad_workspace_bytes(int products, const int64_t* N, const int64_t* K, int64_t M) {
+int64_t mmf_weight_grad_workspace_bytes(int products, const int64_t* N, const int64_t* K, int64_t M, int dtype) {
     if (products < 1 || products > kMaxProducts || !N || !K || M < 1) return 0;
     for (int i = 0; i < products; ++i)
         if (N[i] < 1 || K[i] < 1 || N[i] > 0x7fffff00 || K[i] > 0x7fffff00) return 0;
-    const GradPlan plan = grad_plan(grad_tiles(products, N, K), M);
-    return (int64_t)plan.rest * (plan.split > 1 ? plan.split : 0) * kSide * kSide * 4;
+    const bool f32 = dtype == MMF_F32;
+    const int side = f32 ? kSide32 : kSide;
+    const GradPlan plan = grad_plan(grad_tiles(products, N, K, side), M, f32);
+    return (int64_t)plan.rest * (plan.split > 1 ? plan.split : 0) * side * side * 4;
 }
 
 int mmf_weight_grad(int products, const void* const* dout, const int64_t* lddout, const void* const* y, const int64_t* ldy, void* const* dw,
                     const int64_t* N, const int64_t* K, int64_t M, int dtype, void* workspace, void* stream_) {
+    hipStream_t stream = static_cast<hipStream_t>(stream_);
     if (products < 1 || products > kMaxProducts || !dout || !lddout || !y || !ldy || !dw || !N || !K || M < 1) return MMF_ERR_ARG;
-    if (dtype != MMF_BF16 && dtype != MMF_F16) return MMF_ERR_ARG;
+    if (dtype != MMF_BF16 && dtype != MMF_F16 && dtype != MMF_F32) return MMF_ERR_ARG;
     if (M > 0x7fffffff) return MMF_ERR_WIDE;
+    const bool f32 = dtype == MMF_F32;
+    const int side = f32 ? kSide32 : kSide, whole = f32 ? 4 : 8;                               // elements of 16 bytes
     GradArgs a{};
     int64_t tiles = 0;
     auto off = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) != 0; };
     for (int i = 0; i < products; ++i) {
         if (N[i] < 1 || K[i] < 1 || lddout[i] < N[i] || ldy[i] < K[i] || !dout[i] || !y[i] || !dw[i]) return MMF_ERR_ARG;
-        if (N[i] % 8 || K[i] % 8 || lddout[i] % 8 || ldy[i] % 8 || off(dout[i]) || off(y[i]) || off(dw[i])) return MMF_ERR_ALIGN;
-        if (lddout[i] > 1 << 25 || ldy[i] > 1 << 25) return MMF_ERR_WIDE;                      // 32 rows in 32-bit byte offsets
-        const int64_t tk = mmf_ceil_div(K[i], kSide);
-        a.pr[i] = Product{static_cast<const uint16_t*>(dout[i]), static_cast<const uint16_t*>(y[i]), static_cast<uint16_t*>(dw[i]), lddout[i], ldy[i],
-                          (int)N[i], (int)K[i], (int)tk, (int)tiles};
-        tiles += tk * mmf_ceil_div(N[i], kSide);
+        if (N[i] % whole || K[i] % whole || lddout[i] % whole || ldy[i] % whole || off(dout[i]) || off(y[i]) || off(dw[i])) return MMF_ERR_ALIGN;
+        if (lddout[i] > 1 << 24 || ldy[i] > 1 << 24) return MMF_ERR_WIDE;                      // 32 rows in 32-bit byte offsets
+        const int64_t tk = mmf_ceil_div(K[i], side);
+        a.pr[i] = Product{dout[i], y[i], dw[i], lddout[i], ldy[i], (int)N[i], (int)K[i], (int)tk, (int)tiles};
+        tiles += tk * mmf_ceil_div(N[i], side);
         if (tiles > 0x3fffffff) return MMF_ERR_WIDE;
     }
-    const GradPlan plan = grad_plan(tiles, M);
-    if (plan.rest && (!workspace || off(workspace))) return workspace ? MMF_ERR_ALIGN : MMF_ERR_ARG;
+    const GradPlan plan = grad_plan(tiles, M, f32);
+    if (plan.rest && !workspace) return MMF_ERR_ARG;
+    if (plan.rest && off(workspace)) return MMF_ERR_ALIGN;
     a.n = products; a.full = plan.full; a.rest = plan.rest; a.split = plan.split; a.M = M; a.part = static_cast<float*>(workspace);
-    return dtype == MMF_BF16 ? launch_grad<bf16_t>(a, static_cast<hipStream_t>(stream_)) : launch_grad<f16_t>(a, static_cast<hipStream_t>(stream_));
+    switch (dtype) {
+        case MMF_F32: return launch_grad<float>(a, stream);
+        case MMF_BF16: return launch_grad<bf16_t>(a, stream);
+        case MMF_F16: return launch_grad<f16_t>(a, stream);
+    }
+    return MMF_ERR_ARG;
 }
 
 }  // extern "C"
