@@ -208,21 +208,6 @@ class HGRNGateFn(torch.autograd.Function):
         return di.reshape(i.shape), df.reshape(f.shape), (dlb.to(lb.dtype) if lb is not None else None), None
 
 
-def _scan_bwd(g, o, do, h0, log_gates):
-    lib = L.load()
-    b, h, t, d = g.shape
-    gc, oc, dc = g.contiguous(), o.contiguous(), do.to(g.dtype).contiguous()
-    dx, dg = torch.empty_like(gc), torch.empty_like(gc)
-    h0f = h0.detach().reshape(b * h, d).float().contiguous() if h0 is not None else None
-    nws = lib.mmf_hgrn_recurrent_bwd_workspace_bytes(b * h, t, d)
-    ws = torch.empty(nws // 4, dtype=torch.float32, device=g.device) if nws else None    # per-segment carries (few KB)
-    with L.on(g.device):
-        L.check(lib.mmf_hgrn_recurrent_bwd_split(gc.data_ptr(), oc.data_ptr(), dc.data_ptr(), L.ptr(h0f), dx.data_ptr(),
-                                                 dg.data_ptr(), b * h, t, d, 1 if log_gates else 0, L.dtype_id(g.dtype),
-                                                 L.ptr(ws), L.stream()), "mmf_hgrn_recurrent_bwd_split")
-    return dx, dg
-
-
 CHAIN_NORM, CHAIN_GATED, CHAIN_SWIGLU, CHAIN_RESNORM = 0, 1, 2, 3
 
 
@@ -289,25 +274,6 @@ def _turned_products(pairs):
     return out
 
 
-def _weight_grads(pairs):
-    """dout^T @ y_q of a block's BitLinears, [M, N] gradients and [M, K] de-quantised inputs; None where the gradients are None.
-
-    Two or more go in one launch: each by itself leaves much of the chip idle, or its launch takes longer than it does.  The six of a
-    block, one library product each / together, us: bf16, 2048 wide 64 rows 114 / 41, 1024 186 / 123, 8192 916 / 716; 1024 wide 112 / 34 and
-    456 / 206 (1024, 8192 rows); fp32, 1024 wide 666 rows 220 / 143, 2048 wide 591 / 514 and 1522 / 1487 (666, 2002 rows).  One alone
-    (2048 x 2048, bf16: 1024 rows 21 / 29, 8192 86 / 81) stays with the library, and so do many rows of wide blocks in fp32, where each
-    product fills the chip (2048 wide, 4096 rows 2859 / 2999; 1536 wide 1659 / 1671; 1024 wide 801 / 783)."""
-    take = [i for i, p in enumerate(pairs) if p[0] is not None and _turns(*p)]
-    if take and pairs[take[0]][1].dtype == torch.float32 and len(pairs[take[0]][1]) > 2048 and sum(
-            pairs[i][0].shape[1] * pairs[i][1].shape[1] for i in take) > 1 << 24:
-        take = []
-    out = [None] * len(pairs)
-    if len(take) >= 2:
-        for i, o in zip(take, _turned_products([pairs[i] for i in take])):
-            out[i] = o
-    return [d.t() @ y if o is None and d is not None else o for o, (d, y) in zip(out, pairs)]
-
-
 def _weight_grad(dout, y):
     """dout^T @ y_q of [M, N] gradients and [M, K] de-quantised inputs.
 
@@ -334,7 +300,7 @@ class BlockFn(torch.autograd.Function):
 
     The forward is one native call that gives the bits of the op-by-op composition.  The backward runs the same dense
     products as that composition's (dout @ W_q and dout^T @ y_q per BitLinear) and one row kernel between them where the
-    composition had a norm behind a norm, three norms added up, or sliced tensors to put together.
+    composition had a norm behind a norm, three norms added up, or sliced tensors to put together; it is native too.
     ``params``: the nine norm weights (block.py's order), then the six BitLinear weights i, f, g, o, gate, down."""
 
     @staticmethod
@@ -361,53 +327,17 @@ class BlockFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dout):
         x, lb, mk, ifg, xg, o, attn, y, *nw = ctx.saved_tensors
-        attn_norm, mlp_norm, g_norm, i_n, f_n, gp_n, o_n, gate_n, down_n = nw
-        plan, need = ctx.plan, ctx.needs_input_grad[4:]
-        H, D, I = plan.dims
-        eps, dt, dev = plan.eps, x.dtype, x.device
-        lib = L.load()
-        b, t, _ = x.shape
-        m = b * t
-        with L.on(dev):
-            d2 = dout.to(dt).reshape(m, H).contiguous()
-            o_pw, gate_pw, down_pw = plan.pws[3:]
-            # down_proj behind the swiglu: the gradients of gate and up land side by side
-            dz = d2 @ _dense_weight(down_pw, dt)
-            dy = torch.empty_like(y)
-            _, _, yq, dw_down = _chain_bwd(CHAIN_SWIGLU, y[:, :I], y[:, I:], None, 0.0, [down_n], eps["down_eps"], [dz], dx=dy[:, :I],
-                                           daux=dy[:, I:])
-            down = (d2 if need[14] else None, yq[0])
-            # gate_proj behind mlp_norm, the residual's gradient joining
-            dh = dy @ _dense_weight(gate_pw, dt)
-            dres, _, yq, dw_gate = _chain_bwd(CHAIN_RESNORM, attn, x.view(m, H), mlp_norm, eps["mlp_eps"], [gate_n], eps["gate_eps"], [dh],
-                                               dres=d2)
-            gate = (dy if need[13] else None, yq[0])
-            # o_proj behind the gated norm: the g columns of the stacked projection's gradient, and the scan's output
-            do2 = dres @ _dense_weight(o_pw, dt)
-            difg, do = torch.empty_like(ifg), torch.empty_like(o)
-            _, _, yq, dw_o = _chain_bwd(CHAIN_GATED, ifg[:, 2 * D:], o, g_norm, eps["g_eps"], [o_n], eps["o_eps"], [do2],
-                                        dx=difg[:, 2 * D:], daux=do)
-            o_ = (dres if need[12] else None, yq[0])
-            # scan and gate math
-            dxs, dgs = _scan_bwd(xg[1].view(b, 1, t, D), o.view(b, 1, t, D), do.view(b, 1, t, D), None, False)
-            dlb = torch.empty(D, dtype=torch.float32, device=dev) if lb is not None else None
-            part = torch.empty(lib.mmf_backward_groups(m), D, dtype=torch.float32, device=dev) if lb is not None else None
-            e = x.element_size()
-            L.check(lib.mmf_hgrn_gate_bwd(ifg.data_ptr(), 3 * D, ifg.data_ptr() + D * e, 3 * D, L.ptr(lb), L.ptr(mk), dxs.data_ptr(),
-                                          dgs.data_ptr(), difg.data_ptr(), 3 * D, difg.data_ptr() + D * e, 3 * D, L.ptr(part), L.ptr(dlb),
-                                          m, D, L.dtype_id(dt), L.stream()), "mmf_hgrn_gate_bwd")
-            # i, f, g behind attn_norm: three products, one pass over the rows, the residual's gradient joining
-            w3, dh3 = _dense_weight(plan.stacked, dt), torch.empty(3, m, H, dtype=dt, device=dev)
-            cols = [difg[:, j * D:(j + 1) * D] for j in range(3)]
-            for j in range(3):
-                torch.mm(cols[j], w3[j * D:(j + 1) * D], out=dh3[j])
-            dx, _, yq, dw_ifg = _chain_bwd(CHAIN_NORM, x.view(m, H), None, attn_norm, eps["attn_eps"], [i_n, f_n, gp_n], eps["ifg_eps"],
-                                           dh3, dres=dres)
-            d_weights = _weight_grads([*[(cols[j] if need[9 + j] else None, yq[j]) for j in range(3)], o_, gate, down])
-        grads = [dw_ifg[0], dw_gate[0], dw_o[0], dw_ifg[1], dw_ifg[2], dw_ifg[3], dw_o[1], dw_gate[1], dw_down[0]]
+        plan, eps = ctx.plan, ctx.plan.eps
+        b, t, H = x.shape
+        d2 = dout.to(x.dtype).reshape(b * t, H).contiguous()
+        packed = tuple((pw.packed, pw.wdeq, pw.seg_rows, pw.n, pw.k) for pw in (plan.stacked, *plan.pws[3:]))
+        dx, dlb, ifg_n, o_n, gate_n, down_n, *d_weights = L.native().block_backward(
+            d2, (b, t), plan.dims, (x, lb, mk, ifg, xg, o, attn, y, *nw), packed,
+            tuple(float(eps[k]) for k in ("attn_eps", "ifg_eps", "g_eps", "o_eps", "mlp_eps", "gate_eps", "down_eps")), ctx.needs_input_grad[13:19], L.check)
+        grads = [ifg_n[0], gate_n[0], o_n[0], ifg_n[1], ifg_n[2], ifg_n[3], o_n[1], gate_n[1], down_n[0]]
         if dlb is not None:
             dlb = dlb.to(ctx.lb_dtype)
-        return (None, dx.view(x.shape), dlb, None, *grads, *d_weights)
+        return (None, dx, dlb, None, *grads, *d_weights)
 
 
 class NormHeadFn(torch.autograd.Function):

@@ -3,6 +3,7 @@
 // lock of the thread that called it).  Measured with kernels of 4.5 and 30 us of device time behind them, per call:
 //   FusedBitLinear 1 x 2048 -> 2048          19.7 us through Python and ctypes, 7.7 here (the launch alone: 3)
 //   fused_recurrent_hgrn, forward + backward  172 us through Python Functions, 71 here
+//   the backward of a block, ~30 launches      359 us through Python and ctypes, 239 here
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -167,6 +168,194 @@ PyObject* scan(PyObject*, PyObject* const* args, Py_ssize_t count) {
     END_HANDLE_TH_ERRORS
 }
 
+// ------------------------------------------------------------------------------ backward of a block
+enum Chain : int { CHAIN_NORM = 0, CHAIN_GATED = 1, CHAIN_SWIGLU = 2, CHAIN_RESNORM = 3 };
+void* address(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+
+struct Chained { Tensor dx, y, dw; };
+// mmf_chain_bwd over [M, K] operands (column slices keep their row stride; dy: one [M, K] a norm); dx is allocated unless given
+Chained chain(int kind, const Tensor& x, const Tensor& aux, const Tensor& w1, double eps1, at::ArrayRef<Tensor> w2, double eps2, at::ArrayRef<Tensor> dy,
+              const Tensor& dres, Tensor dx, const Tensor& daux) {
+    const int64_t m = x.size(0), k = x.size(1), n = (int64_t)w2.size(), rows = n + (kind != CHAIN_SWIGLU);
+    if (!dx.defined()) dx = at::empty({m, k}, x.options());
+    Tensor y = at::empty({n, m, k}, x.options()), dw = at::empty({rows, k}, w2[0].options());
+    Tensor part = at::empty({mmf_chain_bwd_groups(m) * rows * k}, x.options().dtype(at::kFloat));
+    const void *w2p[3] = {}, *dyp[3] = {};
+    for (int64_t i = 0; i < n; ++i) {
+        w2p[i] = w2[i].data_ptr();
+        dyp[i] = dy[i].data_ptr();
+    }
+    check(mmf_chain_bwd(kind, x.data_ptr(), x.stride(0), address(aux), aux.defined() ? aux.stride(0) : 0, address(w1), (float)eps1, (int)n, w2p,
+                        (float)eps2, dyp, k, address(dres), dx.data_ptr(), dx.stride(0), address(daux), daux.defined() ? daux.stride(0) : 0, y.data_ptr(),
+                        floats(part), dw.data_ptr(), m, k, dtype_of(x.scalar_type()), dtype_of(dw.scalar_type()), stream_of(x)),
+          "mmf_chain_bwd");
+    return {dx, y, dw};
+}
+
+struct Packed { Tensor codes, wdeq; int64_t seg_rows, n, k; };
+// t * wdeq as a dense [N, K] matrix for dout @ W_q (autograd.py's _dense_weight): 16-bit types contiguous along N
+Tensor dense(const Packed& p, const at::TensorOptions& like) {
+    const auto type = c10::typeMetaToScalarType(like.dtype());
+    const bool rows = type == at::kFloat;
+    Tensor w = rows ? at::empty({p.n, p.k}, like) : at::empty({p.k, p.n}, like);
+    check((rows ? mmf_unpack_dequant : mmf_unpack_dequant_t)(p.codes.data_ptr(), floats(p.wdeq), p.seg_rows, p.n, p.k, w.data_ptr(), dtype_of(type),
+                                                             stream_of(w)),
+          rows ? "mmf_unpack_dequant" : "mmf_unpack_dequant_t");
+    return rows ? w : w.t();
+}
+
+// dout^T @ y of a block's BitLinears, [M, N] gradients and [M, K] de-quantised inputs; undefined where a gradient is.
+// Two or more go in one launch: each by itself leaves much of the chip idle, or its launch takes longer than it does.  The six of a
+// block, one library product each / together, us: bf16, 2048 wide 64 rows 114 / 41, 1024 186 / 123, 8192 916 / 716; 1024 wide 112 / 34
+// and 456 / 206 (1024, 8192 rows); fp32, 1024 wide 666 rows 220 / 143, 2048 wide 591 / 514 and 1522 / 1487 (666, 2002 rows).  One alone
+// (2048 x 2048, bf16: 1024 rows 21 / 29, 8192 86 / 81) stays with the library, and so do many rows of wide blocks in fp32, where each
+// product fills the chip (2048 wide, 4096 rows 2859 / 2999; 1536 wide 1659 / 1671; 1024 wide 801 / 783).
+std::vector<Tensor> weight_grads(at::ArrayRef<std::pair<Tensor, Tensor>> pairs) {
+    std::vector<Tensor> out(pairs.size());
+    const void *p[8], *q[8];
+    void* o[8];
+    int64_t ldp[8], ldq[8], n[8], k[8], outputs = 0;
+    int count = 0, which[8];
+    for (size_t i = 0; i < pairs.size(); ++i) {
+        const Tensor &d = pairs[i].first, &y = pairs[i].second;
+        if (!d.defined() || dtype_of(y.scalar_type()) < 0 || d.scalar_type() != y.scalar_type() || d.size(0) < 1 || d.size(0) > 0x7fffffff) continue;
+        const int64_t whole = 16 / (int64_t)y.element_size();
+        auto turns = [&](const Tensor& t) {
+            return t.stride(1) == 1 && t.size(1) > 0 && t.size(1) % whole == 0 && t.stride(0) % whole == 0 && t.size(1) <= t.stride(0) &&
+                   t.stride(0) <= 1 << 24 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+        };
+        if (!turns(d) || !turns(y)) continue;
+        p[count] = d.data_ptr();
+        q[count] = y.data_ptr();
+        ldp[count] = d.stride(0);
+        ldq[count] = y.stride(0);
+        n[count] = d.size(1);
+        k[count] = y.size(1);
+        outputs += d.size(1) * y.size(1);
+        which[count++] = (int)i;
+    }
+    if (count >= 2) {
+        const Tensor& y = pairs[which[0]].second;
+        const int64_t m = y.size(0);
+        const int dt = dtype_of(y.scalar_type());
+        if (dt != MMF_F32 || m <= 2048 || outputs <= 1 << 24) {
+            for (int i = 0; i < count; ++i) o[i] = (out[which[i]] = at::empty({n[i], k[i]}, y.options())).data_ptr();
+            Tensor ws;
+            if (const int64_t bytes = mmf_weight_grad_workspace_bytes(count, n, k, m, dt)) ws = at::empty({bytes}, y.options().dtype(at::kByte));
+            check(mmf_weight_grad(count, p, ldp, q, ldq, o, n, k, m, dt, address(ws), stream_of(y)), "mmf_weight_grad");
+        }
+    }
+    for (size_t i = 0; i < pairs.size(); ++i)
+        if (!out[i].defined() && pairs[i].first.defined()) out[i] = at::mm(pairs[i].first.t(), pairs[i].second);
+    return out;
+}
+
+// (dout [M, H], (B, T), (H, D, I), (x, lower_bound or None, mask or None, ifg, xg, o, attn, y, the nine norm weights), 4 packed weights (codes,
+// wdeq, seg_rows, n, k) of the stacked projection, o, gate, down, 7 eps (attn, ifg, g, o, mlp, gate, down), the six weights' needs, what raises
+// for a return code) -> (dx, d lower_bound, dw of ifg's / o's / gate's / down's chains, the six weight gradients)
+PyObject* block_backward(PyObject*, PyObject* const* args, Py_ssize_t count) {
+    HANDLE_TH_ERRORS
+    bool fits = count == 8 && THPVariable_Check(args[0]);
+    for (int i = 1; fits && i < 7; ++i) fits = PyTuple_Check(args[i]);
+    if (fits) fits = PyTuple_GET_SIZE(args[1]) == 2 && PyTuple_GET_SIZE(args[2]) == 3 && PyTuple_GET_SIZE(args[3]) == 17 && PyTuple_GET_SIZE(args[4]) == 4 &&
+                     PyTuple_GET_SIZE(args[5]) == 7 && PyTuple_GET_SIZE(args[6]) == 6;
+    Tensor s[17];
+    for (int i = 0; fits && i < 17; ++i) {
+        PyObject* t = PyTuple_GET_ITEM(args[3], i);
+        if (THPVariable_Check(t)) s[i] = THPVariable_Unpack(t);
+        else fits = t == Py_None && (i == 1 || i == 2);
+    }
+    Packed pw[4];
+    for (int i = 0; fits && i < 4; ++i) {
+        PyObject* t = PyTuple_GET_ITEM(args[4], i);
+        if (!(fits = PyTuple_Check(t) && PyTuple_GET_SIZE(t) == 5 && THPVariable_Check(PyTuple_GET_ITEM(t, 0)) && THPVariable_Check(PyTuple_GET_ITEM(t, 1)))) break;
+        pw[i] = Packed{THPVariable_Unpack(PyTuple_GET_ITEM(t, 0)), THPVariable_Unpack(PyTuple_GET_ITEM(t, 1)), PyLong_AsLongLong(PyTuple_GET_ITEM(t, 2)),
+                       PyLong_AsLongLong(PyTuple_GET_ITEM(t, 3)), PyLong_AsLongLong(PyTuple_GET_ITEM(t, 4))};
+    }
+    if (!fits) {
+        PyErr_SetString(PyExc_TypeError, "block_backward takes (dout, (B, T), (H, D, I), 17 saved, 4 packed weights, 7 eps, 6 needs, check)");
+        return nullptr;
+    }
+    auto whole = [&](int a, int i) { return (int64_t)PyLong_AsLongLong(PyTuple_GET_ITEM(args[a], i)); };
+    const int64_t b = whole(1, 0), t = whole(1, 1), H = whole(2, 0), D = whole(2, 1), I = whole(2, 2), m = b * t;
+    double eps[7];
+    int need[6];
+    for (int i = 0; i < 7; ++i) eps[i] = PyFloat_AsDouble(PyTuple_GET_ITEM(args[5], i));
+    for (int i = 0; i < 6; ++i) need[i] = PyObject_IsTrue(PyTuple_GET_ITEM(args[6], i));
+    if (PyErr_Occurred()) return nullptr;
+    const Tensor &x = s[0], &lb = s[1], &mask = s[2], &ifg = s[3], &xg = s[4], &o = s[5], &attn = s[6], &y = s[7], *nw = s + 8;
+    const Tensor& d2 = THPVariable_Unpack(args[0]);
+    Tensor grads[12];
+    try {
+        NoGil nogil;
+        OnDevice on(x.get_device());
+        const auto like = x.options().requires_grad(false);
+        const int dt = dtype_of(x.scalar_type());
+        const Tensor none, x2 = x.view({m, H});
+        std::pair<Tensor, Tensor> products[6];
+        auto product = [&](int i, const Tensor& d, const Tensor& yq) { products[i] = {need[i] ? d : none, yq}; };
+        // down_proj behind the swiglu: the gradients of gate and up land side by side
+        const Tensor dz = at::mm(d2, dense(pw[3], like)), dy = at::empty(y.sizes(), like);
+        Chained down = chain(CHAIN_SWIGLU, y.narrow(1, 0, I), y.narrow(1, I, I), none, 0.0, {nw[8]}, eps[6], {dz}, none, dy.narrow(1, 0, I), dy.narrow(1, I, I));
+        product(5, d2, down.y[0]);
+        // gate_proj behind mlp_norm, the residual's gradient joining
+        const Tensor dh = at::mm(dy, dense(pw[2], like));
+        Chained gate = chain(CHAIN_RESNORM, attn, x2, nw[1], eps[4], {nw[7]}, eps[5], {dh}, d2, none, none);
+        product(4, dy, gate.y[0]);
+        // o_proj behind the gated norm: the g columns of the stacked projection's gradient, and the scan's output
+        const Tensor &dres = gate.dx, do2 = at::mm(dres, dense(pw[1], like)), difg = at::empty(ifg.sizes(), like), dout = at::empty(o.sizes(), like);
+        Chained oc = chain(CHAIN_GATED, ifg.narrow(1, 2 * D, D), o, nw[2], eps[2], {nw[6]}, eps[3], {do2}, none, difg.narrow(1, 2 * D, D), dout);
+        product(3, dres, oc.y[0]);
+        // scan and gate math
+        const auto f32 = like.dtype(at::kFloat);
+        const Tensor gates = xg[1].contiguous(), out = o.contiguous();
+        Tensor dxs = at::empty({m, D}, like), dgs = at::empty({m, D}, like), ws, dlb, part;
+        if (const int64_t bytes = mmf_hgrn_recurrent_bwd_workspace_bytes(b, t, D)) ws = at::empty({bytes / 4}, f32);
+        check(mmf_hgrn_recurrent_bwd_split(gates.data_ptr(), out.data_ptr(), dout.data_ptr(), nullptr, dxs.data_ptr(), dgs.data_ptr(), b, t, D, 0, dt, floats(ws),
+                                           stream_of(x)),
+              "mmf_hgrn_recurrent_bwd_split");
+        if (lb.defined()) {
+            dlb = at::empty({D}, f32);
+            part = at::empty({mmf_backward_groups(m), D}, f32);
+        }
+        auto column = [&](const Tensor& a, int64_t j) { return a.narrow(1, j * D, D); };
+        const Tensor ii = column(ifg, 0), ff = column(ifg, 1), di = column(difg, 0), df = column(difg, 1);
+        check(mmf_hgrn_gate_bwd(ii.data_ptr(), 3 * D, ff.data_ptr(), 3 * D, floats(lb), static_cast<const uint8_t*>(address(mask)), dxs.data_ptr(), dgs.data_ptr(),
+                                di.data_ptr(), 3 * D, df.data_ptr(), 3 * D, floats(part), floats(dlb), m, D, dt, stream_of(x)),
+              "mmf_hgrn_gate_bwd");
+        // i, f, g behind attn_norm: three products, one pass over the rows, the residual's gradient joining
+        const Tensor w3 = dense(pw[0], like), dh3 = at::empty({3, m, H}, like), dhs[3] = {dh3[0], dh3[1], dh3[2]};
+        for (int j = 0; j < 3; ++j) {
+            Tensor to = dhs[j];
+            at::mm_out(to, column(difg, j), w3.narrow(0, j * D, D));
+        }
+        Chained in = chain(CHAIN_NORM, x2, none, nw[0], eps[0], {nw[3], nw[4], nw[5]}, eps[1], dhs, dres, none, none);
+        for (int j = 0; j < 3; ++j) product(j, column(difg, j), in.y[j]);
+        const std::vector<Tensor> dw = weight_grads(products);
+        grads[0] = in.dx.view(x.sizes());
+        grads[1] = dlb;
+        grads[2] = in.dw;
+        grads[3] = oc.dw;
+        grads[4] = gate.dw;
+        grads[5] = down.dw;
+        for (int i = 0; i < 6; ++i) grads[6 + i] = dw[i];
+    } catch (const Failed& f) {
+        Py_XDECREF(PyObject_CallFunction(args[7], "is", f.rc, f.what));
+        if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, f.what);
+        return nullptr;
+    }
+    PyObject* r = PyTuple_New(12);
+    for (int i = 0; r && i < 12; ++i) {
+        PyObject* g = Py_None;
+        if (grads[i].defined()) g = THPVariable_Wrap(grads[i]);
+        else Py_INCREF(g);
+        if (!g) { Py_DECREF(r); return nullptr; }
+        PyTuple_SET_ITEM(r, i, g);
+    }
+    return r;
+    END_HANDLE_TH_ERRORS
+}
+
 // ------------------------------------------------------------------------------ what a native block call takes for granted
 // Whether all of this still holds for a block -- asked for every block of every forward, ~130 look-ups in 1.6 us:
 // (block, (class, modules dict, parameters dict, [(module, class, dict)], [(dict, key, object)], [(dict, key)], [(dict, key, value)],
@@ -273,6 +462,7 @@ PyMethodDef methods[] = {
     {"structure_holds", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(structure_holds)), METH_FASTCALL, nullptr},
     {"parameters_hold", parameters_hold, METH_O, nullptr},
     {"bitlinear", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(bitlinear)), METH_FASTCALL, nullptr},
+    {"block_backward", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(block_backward)), METH_FASTCALL, nullptr},
     {"scan", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(scan)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "mmf_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
