@@ -123,6 +123,7 @@ int mmf_rmsnorm_quant_fused(int prologue, const void* x, int64_t ldx, const void
                             int64_t ldaux2, void* res_out, const void* w1, float eps1, const void* norm_weight, float eps,
                             const float* lower_bound, float* state, int8_t* q, float* deq, int* qsum, int64_t M, int64_t K,
                             int x_dtype, int weight_dtype, void* stream);
+
 /* ---- BitLinear contraction ------------------------------------------------------------
  * Both replace F.linear(y, weight_quant(W)) at mmfreelm/ops/fusedbitnet.py:456-458 (class
  * FusedBitLinear :584-610, layer_norm_linear_quant_fn :513-536):
@@ -135,7 +136,8 @@ int mmf_rmsnorm_quant_fused(int prologue, const void* x, int64_t ldx, const void
  * mmf_bitlinear_gemv: decode-sized M; norm + quantiser + contraction in one launch, x is
  *   the un-normalised input [M, K] (K <= mmf_bitlinear_gemv_max_k()).
  * mmf_bitlinear_mfma: int8 matrix-core contraction on codes from mmf_rmsnorm_quant
- *   (tiled = 1); out has leading dimension ldo; config < 0 picks the tile shape from M. */
+ *   (tiled = 1); out has leading dimension ldo; config < 0 picks the tile shapes from M, N
+ *   and K (the rows behind the last whole round of tiles may take a second launch). */
 int64_t mmf_bitlinear_gemv_max_k(void);
 /* mmf_bitlinear_gemv_fused: the same launch with the elementwise ops the model runs around a
  * BitLinear folded in (a decode step is latency bound: one launch per BitLinear, none between).

@@ -41,7 +41,7 @@ struct MfmaArgs {
     const void* addend;   // [M, N] (leading dimension ldo) or null: out = T(T(o) + addend)
     void* out;            // [M, N]
     int64_t M, N, Kp, seg_rows, ldo;
-    int64_t a_seg;        // 0, or the bytes from one weight segment's codes to the next's (deq, qsum: M entries): stacked
+    int64_t a_seg, m_seg; // 0, or the bytes from one weight segment's codes to the next's, and the entries between their deq and qsum: stacked
                           // projections whose inner norms differ contract each its own codes of the same rows
     int tiles_m, tiles_n;
     int rows_per_xcd;     // tile rows an XCD keeps in its L2 while it walks the columns (0: row-major tile order)
@@ -59,8 +59,8 @@ __device__ __forceinline__ void mfma_select_segment(MfmaArgs& p, int64_t nb0) {
     if (p.a_seg == 0) return;
     const int64_t seg = (int64_t)((uint32_t)(nb0 * 32) / (uint32_t)p.seg_rows);
     p.a += seg * p.a_seg;
-    p.deq += seg * p.M;
-    p.qsum += seg * p.M;
+    p.deq += seg * p.m_seg;
+    p.qsum += seg * p.m_seg;
 }
 
 // Pack rounded outputs: two floats -> one dword of bf16/f16 (round to nearest even).
@@ -1063,10 +1063,11 @@ int launch_mfma(MfmaArgs a, hipStream_t s) {
 // on average, 8 % at most; with the plain products' times it cost 4 %, and 58 % at most (106 x 2560 -> 13824, stream / split 9.7 / 15.3 us; 410 x 1024 -> 5632
 // 9.1 / 12.1 in a model).
 enum class MfmaPick { kStream, kSplit, kTiles };
-inline MfmaPick mfma_pick(const MfmaArgs& a, bool swiglu) {
-    const int64_t KB = a.Kp >> 7;
-    const double kb = (double)KB, blocks = (double)mmf_ceil_div(a.M, 32) * (double)mmf_ceil_div(a.N, 32);
-    const int64_t half = mmf_ceil_div(a.M, 64) * mmf_ceil_div(a.N, 256), full = mmf_ceil_div(a.M, 64) * mmf_ceil_div(a.N, 512);
+struct MfmaChoice { MfmaPick pick; double us; };
+inline MfmaChoice mfma_choice(int64_t M, int64_t N, int64_t Kp, bool swiglu) {
+    const int64_t KB = Kp >> 7;
+    const double kb = (double)KB, blocks = (double)mmf_ceil_div(M, 32) * (double)mmf_ceil_div(N, 32);
+    const int64_t half = mmf_ceil_div(M, 64) * mmf_ceil_div(N, 256), full = mmf_ceil_div(M, 64) * mmf_ceil_div(N, 512);
     const double halves = (double)half / 256.0, wholes = (double)full / 256.0, half_rounds = (double)mmf_ceil_div(half, 256), rounds = (double)mmf_ceil_div(full, 256);
     double t_stream, t_tiles, t_split;
     if (swiglu) {
@@ -1079,20 +1080,64 @@ inline MfmaPick mfma_pick(const MfmaArgs& a, bool swiglu) {
         t_split = half <= 256 ? 4.4 + 0.29 * kb + halves * (1.0 + 0.1 * kb) : half <= 512 ? 8.5 + 0.59 * kb : half_rounds * (3.9 + 0.295 * kb);
     }
     if (KB % 2 != 0) t_split = 1e30;
-    if (a.Kp <= 8192 && a.M <= 65535 * 32 && (a.M <= 64 || (t_stream <= t_split && t_stream <= t_tiles))) return MfmaPick::kStream;
-    return t_split < t_tiles ? MfmaPick::kSplit : MfmaPick::kTiles;
+    if (Kp <= 8192 && M <= 65535 * 32 && (M <= 64 || (t_stream <= t_split && t_stream <= t_tiles))) return {MfmaPick::kStream, t_stream};
+    if (t_split < t_tiles) return {MfmaPick::kSplit, t_split};
+    return {MfmaPick::kTiles, t_tiles};
+}
+
+// The rows of the first of two launches, or all of them: where the tiles' last round holds a few of them, its rows go in a launch of their own, most
+// often the stream's.  us, one launch / two (rows of the second): 2048 -> 6144, 1377 rows (528 split tiles; 33) 27.2 / 23.3, 2693 (5) 36.6 / 29.0, 5549 (109)
+// 59.6 / 54.5; gate and up to 5632 with swiglu, 3066 (122) 80.6 / 73.7, 715 (11) 26.3 / 25.2; 5632 -> 2048, 2096 (48) 32.6 / 27.7; 1536 -> 4608, 3586 (2)
+// 30.9 / 23.7; 6912 -> 2560, 3357 (93) 61.2 / 49.2.  Over 87 shapes with at most 320 rows in the second, 65 to 16384 in all, that were estimated to gain 3 %: 5 % less
+// on average, 15 % more at most.  Where the estimate has to promise 7 % (10 % from 129 rows on; 3 % with swiglu, whose rounds take longer than
+// estimated) none took longer.  With 340 to 600 rows in the second two launches took between 12 % less and 12 % more (2048 -> 6144, 4843 (747)
+// 47.7 / 53.5; 6912 -> 2560, 5431 (567) 70.6 / 79.2).  The sums are integers and a row's do not depend on the others: the same bits.
+constexpr int64_t kCutRows = 320;
+inline int64_t mfma_first_rows(int64_t M, int64_t N, int64_t Kp, bool swiglu) {
+    const double whole = mfma_choice(M, N, Kp, swiglu).us;
+    double least = whole;
+    int64_t first = M;
+    for (const int64_t cols : {256, 512}) {
+        const int64_t across = mmf_ceil_div(N, cols), rounds = mmf_ceil_div(mmf_ceil_div(M, 64) * across, 256);
+        for (int64_t r = rounds - 1; r >= 1 && r >= rounds - 2; --r) {
+            const int64_t m = 256 * r / across * 64;
+            if (m < 64 || m >= M || M - m > kCutRows) continue;
+            const double us = mfma_choice(m, N, Kp, swiglu).us + mfma_choice(M - m, N, Kp, swiglu).us;
+            if (us < least && us < (swiglu ? 0.97 : M - m <= 128 ? 0.93 : 0.90) * whole) {
+                least = us;
+                first = m;
+            }
+        }
+    }
+    return first;
+}
+// rows m0 to m0 + m of a contraction (m0 a multiple of 32)
+template <typename T>
+MfmaArgs mfma_rows(MfmaArgs a, int64_t m0, int64_t m) {
+    a.a += m0 * a.Kp;
+    a.deq += m0;
+    a.qsum += m0;
+    if (a.addend) a.addend = static_cast<const T*>(a.addend) + m0 * a.ldo;
+    a.out = static_cast<T*>(a.out) + m0 * a.ldo;
+    a.M = m;
+    return a;
 }
 
 template <typename T>
-int dispatch_mfma(const MfmaArgs& a, int config, hipStream_t s) {
-    // config < 0: pick by shape.
+int dispatch_mfma(const MfmaArgs& a, int config, hipStream_t s, bool cut = true) {
+    // config < 0: pick by shape, the rows in two launches where that is estimated to be faster (cut).
     //   5        weight-stream kernel: one 32x32 output block per workgroup, 8 waves split K (needs Kp <= 8192)
     //   0 / 1    32x256 / 64x256 tiles, A staged through registers (small M with Kp > 8192)
     //   18       64x256 tiles, two groups of waves on every second k-block (needs an even number of k-blocks)
     //   15 / 16 / 17  256x256 / 128x256 / 64x512 tiles, A staged by DMA (17: every wave reads the whole activation
     //            tile from LDS and owns its own weight columns, so no weight block is fetched twice)
     if (config < 0) {
-        const MfmaPick pick = mfma_pick(a, false);
+        const int64_t first = cut ? mfma_first_rows(a.M, a.N, a.Kp, false) : a.M;
+        if (first < a.M) {
+            if (const int rc = dispatch_mfma<T>(mfma_rows<T>(a, 0, first), -1, s, false)) return rc;
+            return dispatch_mfma<T>(mfma_rows<T>(a, first, a.M - first), -1, s, false);
+        }
+        const MfmaPick pick = mfma_choice(a.M, a.N, a.Kp, false).pick;
         if (pick == MfmaPick::kStream) config = 5;
         else if (a.M <= 32) config = 0;
         else if (a.M <= 64) config = 1;
@@ -1108,8 +1153,8 @@ int dispatch_mfma(const MfmaArgs& a, int config, hipStream_t s) {
             const int64_t seg = n0 / a.seg_rows;
             MfmaArgs b = a;
             b.a += seg * a.a_seg;
-            b.deq += seg * a.M;
-            b.qsum += seg * a.M;
+            b.deq += seg * a.m_seg;
+            b.qsum += seg * a.m_seg;
             b.a_seg = 0;
             b.b += (n0 >> 5) * (a.Kp >> 7) * 64;
             b.wdeq += seg;
@@ -1132,8 +1177,13 @@ int dispatch_mfma(const MfmaArgs& a, int config, hipStream_t s) {
 }
 
 template <typename T>
-int dispatch_mfma_swiglu(const MfmaArgs& a, hipStream_t s) {
-    switch (mfma_pick(a, true)) {
+int dispatch_mfma_swiglu(const MfmaArgs& a, hipStream_t s, bool cut = true) {
+    const int64_t first = cut ? mfma_first_rows(a.M, a.N, a.Kp, true) : a.M;
+    if (first < a.M) {
+        if (const int rc = dispatch_mfma_swiglu<T>(mfma_rows<T>(a, 0, first), s, false)) return rc;
+        return dispatch_mfma_swiglu<T>(mfma_rows<T>(a, first, a.M - first), s, false);
+    }
+    switch (mfma_choice(a.M, a.N, a.Kp, true).pick) {
         case MfmaPick::kStream: return launch_skinny_swiglu<T>(a, s);
         case MfmaPick::kSplit: return launch_mfma_dma3<T, 1, 4, 2, 2, 2, true>(a, s);
         case MfmaPick::kTiles: return launch_mfma_dma3<T, 1, 8, 2, 2, 1, true>(a, s);
@@ -1228,7 +1278,7 @@ int mmf_bitlinear_mfma_multi(const int8_t* codes_tiled, int64_t codes_stride, co
     if ((reinterpret_cast<uintptr_t>(codes_tiled) & 15u) || (codes_stride & 15) || (reinterpret_cast<uintptr_t>(packed) & 15u))
         return MMF_ERR_ALIGN;
     MfmaArgs a{};
-    a.a = codes_tiled; a.a_seg = codes_stride; a.b = static_cast<const uint4*>(packed); a.deq = deq; a.qsum = qsum; a.wdeq = wdeq;
+    a.a = codes_tiled; a.a_seg = codes_stride; a.m_seg = M; a.b = static_cast<const uint4*>(packed); a.deq = deq; a.qsum = qsum; a.wdeq = wdeq;
     a.out = out; a.M = M; a.N = N; a.Kp = mmf_round_up(K, 128); a.seg_rows = seg_rows; a.ldo = ldo;
     switch (out_dtype) {
         case MMF_F32: return dispatch_mfma<float>(a, config, stream);
