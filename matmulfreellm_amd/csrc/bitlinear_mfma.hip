@@ -1058,18 +1058,26 @@ int launch_mfma(MfmaArgs a, hipStream_t s) {
 // 39.7 / 43.3, 6500 86.5 / 77.4; 2048 -> 2048 (16), 2002 rows 12.2 / 15.1, 3600 18.0 / 18.5; 2048 -> 6144, 2002 rows (768) 27.1 / 26.4.  Stream against split:
 // 1024 -> 5632, 300 rows 6.0 / 8.4, 700 9.9 / 9.4; 2048 -> 2048, 1203 rows 10.9 / 11.4, 1395 12.1 / 11.3.
 // Over 389 shapes, 66 to 8000 rows, the choice costs 0.01 % against the best of the three on average, 15 % at most (377 x 1536 -> 4608: 1.2 us).
+//   narrow tiles   (64 x 128, split like the others) where they give every CU at most one, or three in all; with rows of 2560 and more also instead of a
+//                  split one on nearly every CU.  us, best of the others / narrow: 5632 -> 2048, 700 rows 15.6 / 12.8, 1001 (256 narrow tiles) 19.0 / 13.9, 1377 (352)
+//                  20.1 / 20.5, 2002 (512) 24.5 / 23.2, 2400 (608) 32.9 / 29.2; 2048 -> 2048, 830 rows 8.3 / 7.4, 1001 9.2 / 7.8, 1200 (304) 10.4 / 10.8, 2002
+//                  11.7 / 11.8; 2816 -> 1024, 1600 rows 11.9 / 8.4, 4022 (504) 16.4 / 14.5, 4100 (520) 19.7 / 17.4; 2560 -> 2560, 711 rows 11.3 / 8.4, 1491 (480) 13.0 / 13.2,
+//                  1966 (620) 20.3 / 18.4; 2048 -> 6144, 320 rows 9.3 / 7.6.  Weights that an XCD's L2 does not hold cost it more (6912 -> 2560, 580 rows 18.9 / 19.2,
+//                  700 21.3 / 19.6).  Against the stream, whose time is overestimated where it is short, with a margin (670 rows of 1536 -> 1536 stream 5.4, narrow 6.3).
+//                  Over 110 shapes, 163 to 6000 rows, the choice with it takes 5.5 % less, at best 35.  Two groups of two waves, 64 columns each: 3 to 12 % slower
+//                  than of four with 32.
 // With the swiglu epilogue (M from 66 to 6300, K from 512 to 4096, N from 2048 to 22016) the stream's workgroups each own two blocks, of gate and of up, and
 // take 1.3 + 0.1 ns per k-block a block; a tile's epilogue, which nothing hides where a CU has one, is 3 to 5 us.  Over 461 shapes beside the 357 fitted the choice costs 0.25 %
 // on average, 8 % at most; with the plain products' times it cost 4 %, and 58 % at most (106 x 2560 -> 13824, stream / split 9.7 / 15.3 us; 410 x 1024 -> 5632
 // 9.1 / 12.1 in a model).
-enum class MfmaPick { kStream, kSplit, kTiles };
+enum class MfmaPick { kStream, kSplit, kNarrow, kTiles };
 struct MfmaChoice { MfmaPick pick; double us; };
 inline MfmaChoice mfma_choice(int64_t M, int64_t N, int64_t Kp, bool swiglu) {
     const int64_t KB = Kp >> 7;
     const double kb = (double)KB, blocks = (double)mmf_ceil_div(M, 32) * (double)mmf_ceil_div(N, 32);
     const int64_t half = mmf_ceil_div(M, 64) * mmf_ceil_div(N, 256), full = mmf_ceil_div(M, 64) * mmf_ceil_div(N, 512);
     const double halves = (double)half / 256.0, wholes = (double)full / 256.0, half_rounds = (double)mmf_ceil_div(half, 256), rounds = (double)mmf_ceil_div(full, 256);
-    double t_stream, t_tiles, t_split;
+    double t_stream, t_tiles, t_split, t_narrow = 1e30;
     if (swiglu) {
         t_stream = 3.5 + blocks * (0.0013 + 0.0001 * kb);
         t_tiles = full <= 256 ? 9.2 + 0.585 * kb + wholes * (0.19 * kb - 1.0) : 6.5 + rounds * (3.5 + 0.54 * kb);
@@ -1079,8 +1087,15 @@ inline MfmaChoice mfma_choice(int64_t M, int64_t N, int64_t Kp, bool swiglu) {
         t_tiles = full <= 256 ? 4.4 + 0.58 * kb + wholes * (1.0 + 0.18 * kb) : rounds * (4.4 + 0.62 * kb);
         t_split = half <= 256 ? 4.4 + 0.29 * kb + halves * (1.0 + 0.1 * kb) : half <= 512 ? 8.5 + 0.59 * kb : half_rounds * (3.9 + 0.295 * kb);
     }
-    if (KB % 2 != 0) t_split = 1e30;
-    if (Kp <= 8192 && M <= 65535 * 32 && (M <= 64 || (t_stream <= t_split && t_stream <= t_tiles))) return {MfmaPick::kStream, t_stream};
+    if (!swiglu) {
+        const int64_t narrow = mmf_ceil_div(M, 64) * mmf_ceil_div(N, 128);
+        if (narrow <= 256) t_narrow = 3.9 + 0.17 * kb + (double)narrow / 256.0 * (0.3 + 0.045 * kb) + (N * Kp > 16 << 20 ? 0.1 * kb : 0.0);
+        else if (narrow > 480 && half <= 256 && KB >= 20) t_narrow = t_split - 0.1;
+        else if (narrow > 512 && narrow <= 768) t_narrow = 7.0 + 0.54 * kb;
+    }
+    if (KB % 2 != 0) t_split = t_narrow = 1e30;
+    if (Kp <= 8192 && M <= 65535 * 32 && (M <= 64 || (t_stream <= t_split && t_stream <= t_tiles && t_stream * (KB < 20 ? 0.85 : 0.95) <= t_narrow))) return {MfmaPick::kStream, t_stream};
+    if (t_narrow < t_split && t_narrow < t_tiles) return {MfmaPick::kNarrow, t_narrow};
     if (t_split < t_tiles) return {MfmaPick::kSplit, t_split};
     return {MfmaPick::kTiles, t_tiles};
 }
@@ -1128,7 +1143,7 @@ int dispatch_mfma(const MfmaArgs& a, int config, hipStream_t s, bool cut = true)
     // config < 0: pick by shape, the rows in two launches where that is estimated to be faster (cut).
     //   5        weight-stream kernel: one 32x32 output block per workgroup, 8 waves split K (needs Kp <= 8192)
     //   0 / 1    32x256 / 64x256 tiles, A staged through registers (small M with Kp > 8192)
-    //   18       64x256 tiles, two groups of waves on every second k-block (needs an even number of k-blocks)
+    //   18 / 19  64x256 / 64x128 tiles, two groups of waves on every second k-block (need an even number of k-blocks)
     //   15 / 16 / 17  256x256 / 128x256 / 64x512 tiles, A staged by DMA (17: every wave reads the whole activation
     //            tile from LDS and owns its own weight columns, so no weight block is fetched twice)
     if (config < 0) {
@@ -1142,11 +1157,12 @@ int dispatch_mfma(const MfmaArgs& a, int config, hipStream_t s, bool cut = true)
         else if (a.M <= 32) config = 0;
         else if (a.M <= 64) config = 1;
         else if (pick == MfmaPick::kSplit) config = 18;
+        else if (pick == MfmaPick::kNarrow) config = 19;
         else config = a.N >= 512 ? 17 : 16;
     }
-    if (config == 18 && (a.Kp >> 7) % 2 != 0) return MMF_ERR_ARG;
+    if ((config == 18 || config == 19) && (a.Kp >> 7) % 2 != 0) return MMF_ERR_ARG;
     if (config == 5 && (a.Kp > 8192 || a.M > 65535 * 32)) return MMF_ERR_ARG;
-    const int64_t tile_cols = config == 5 ? 32 : config == 16 || config == 18 ? 256 : config == 17 ? 512 : 0;
+    const int64_t tile_cols = config == 5 ? 32 : config == 19 ? 128 : config == 16 || config == 18 ? 256 : config == 17 ? 512 : 0;
     if (a.a_seg != 0 && a.N > a.seg_rows && (tile_cols == 0 || a.seg_rows % tile_cols != 0)) {
         // tiles that would straddle two segments (or tiles of the kernels that take one set of codes): a launch per segment
         for (int64_t n0 = 0; n0 < a.N; n0 += a.seg_rows) {
@@ -1172,6 +1188,7 @@ int dispatch_mfma(const MfmaArgs& a, int config, hipStream_t s, bool cut = true)
         case 16: return launch_mfma_dma3<T, 2, 4, 2, 2, 1, false>(a, s);
         case 17: return launch_mfma_dma3<T, 1, 8, 2, 2, 1, false>(a, s);
         case 18: return launch_mfma_dma3<T, 1, 4, 2, 2, 2, false>(a, s);
+        case 19: return launch_mfma_dma3<T, 1, 4, 2, 1, 2, false>(a, s);
     }
     return MMF_ERR_ARG;
 }
@@ -1186,6 +1203,7 @@ int dispatch_mfma_swiglu(const MfmaArgs& a, hipStream_t s, bool cut = true) {
     switch (mfma_choice(a.M, a.N, a.Kp, true).pick) {
         case MfmaPick::kStream: return launch_skinny_swiglu<T>(a, s);
         case MfmaPick::kSplit: return launch_mfma_dma3<T, 1, 4, 2, 2, 2, true>(a, s);
+        case MfmaPick::kNarrow:
         case MfmaPick::kTiles: return launch_mfma_dma3<T, 1, 8, 2, 2, 1, true>(a, s);
     }
     return MMF_ERR_ARG;
