@@ -544,9 +544,13 @@ int launch_fused_quant(const FusedQuantArgs& a, bool vec, hipStream_t s) {
         // Thousands of rows: 16 to 24 elements a thread (8192 x 2048: four rows a workgroup 22 to 28 us where eight, with 32 elements
         // a thread, took 23 to 31; 8192 x 1024: eight 13 to 17, four 14 to 19).  Fewer rows: as few rows a workgroup as reach every
         // CU about once (320 x 2048: two rows 5.0 to 5.9 us, one 5.5 to 7.0, eight 7.4 to 9.7; 1024 x 2048: four 6.5 to 7.9, one 8.5
-        // to 10.7).  Wide rows with nothing folded in (5632, in front of down_proj) need few registers and take 48 elements.
-        if (a.M > 1280 && a.Kp <= 1024) return launch_fused_quant_rpw<T, TW, PRO, 8, NN>(a, s);
-        if (a.M > 512 && a.Kp <= (PRO == QPRO_PLAIN ? 6144 : 3072)) return launch_fused_quant_rpw<T, TW, PRO, 4, NN>(a, s);
+        // to 10.7).  Wide rows with nothing folded in (5632, in front of down_proj) need few registers and take 48 elements.  Just past a workgroup a CU (four rows: 1024)
+        // the few CUs with a second one set the time: 1025 to 1536 rows take two a workgroup, at most three a CU (1377 rows, four / two: 2048 wide, three norms
+        // 9.6 / 9.3 us, residual norm 8.2 / 7.7, gated 8.8 / 8.1, 5632 plain 9.2 / 8.5, 2560 wide three norms 11.7 / 10.8; 1700 rows 10.0 / 10.9, 8.7 / 9.1, 8.8 / 9.4,
+        // 9.5 / 9.9, 12.3 / 12.7), narrow rows eight (1200 x 1024: 6.8 / 6.3, 5.9 / 5.5; 1001 5.4 / 6.2, 5.0 / 5.5).
+        if (a.M > 1024 && a.Kp <= 1024) return launch_fused_quant_rpw<T, TW, PRO, 8, NN>(a, s);
+        const bool second = a.M > 1024 && a.M <= 1536;
+        if (a.M > 512 && !second && a.Kp <= (PRO == QPRO_PLAIN ? 6144 : 3072)) return launch_fused_quant_rpw<T, TW, PRO, 4, NN>(a, s);
         if (a.M > 192 && a.Kp <= 8192) return launch_fused_quant_rpw<T, TW, PRO, 2, NN>(a, s);
     }
     return launch_fused_quant_rpw<T, TW, PRO, 1, NN>(a, s);
