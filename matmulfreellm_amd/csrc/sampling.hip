@@ -163,20 +163,39 @@ __device__ __forceinline__ void samp_finish_few(const unsigned* few_m, const int
     if (kept != 0u && before <= target && target < before + kept) *out = ii;
 }
 
-// The tokens of a limit of at most 64, without a histogram: a bound below the top_k-th largest logit first, then exact ranks among the few
+// The lowest float above -inf that scales to no less than `low` does.
+__device__ __forceinline__ float samp_lowest_reaching(float low, float temperature) {
+    constexpr unsigned kBottom = 0x007fffffu;                     // -inf in the order of the floats
+    auto order = [](float f) { const unsigned b = __float_as_uint(f); return b & 0x80000000u ? ~b : b | 0x80000000u; };
+    auto value = [](unsigned k) { return __uint_as_float(k & 0x80000000u ? k & 0x7fffffffu : ~k); };
+    const float reach = __fdiv_rn(low, temperature);
+    unsigned no = kBottom, yes = order(low) > kBottom ? order(low) : kBottom + 1;
+    while (yes - no > 1) {
+        const unsigned mid = no + (yes - no) / 2;
+        if (__fdiv_rn(value(mid), temperature) >= reach) yes = mid; else no = mid;
+    }
+    return value(yes);
+}
+
+// The tokens of a limit of at most 64, without a histogram: a bound no higher than the top_k-th largest logit first, then exact ranks among the few
 // logits that reach it.  Scaling does not change the order, so only those are divided.  The bound: every wave's fourth largest (or third, ..: 16 waves have top_k
-// between them) of its threads' maxima, the least of them; a thread's logits come from all over the vocabulary, so that no wave has only rare
-// tokens.  200 to 300 of 32000 normal logits reach it.  Two unequal logits can scale to equal ones: what lies less than 2^-21 below the
-// bound is ranked too, and a bound whose scaled value is not in the middle range, where that covers such pairs, decides nothing.
+// between them) of its threads' maxima, the least of them; or, where the large logits lie close together, the least maximum of some wave's 64 threads.  A thread's
+// logits come from all over the vocabulary, so that no wave has only rare tokens.  200 to 300 of 32000 normal logits reach it, 505 of sorted ones.  Two unequal
+// logits can scale to equal ones: what lies less than 2^-21 below the bound is ranked too; where the bound or its scaled value is not in the
+// middle range, where that covers such pairs, the lowest float that reaches it is searched for (all finite logits, where there are few).
 // Returns the number of kept tokens (more than top_k on ties), their masses and places in ps.mass, ps.at; -1, for the whole workgroup, when the
 // caller has to go the general way.
 // Bound by latency: a row has one CU, whose waves wait for each other four times.  32000 logits, limit 50, 1 to 64 rows, us, descent and ranks: bf16 23.0 to
-// 24.9 and 10.2 to 11.7, fp16 22.8 to 24.7 and 9.0 to 12.3, fp32 33 and 21 to 24 (128 KB through one CU); limit 64 with ties at it 39.5 to 41.6 and 10.8 to
-// 12.7, limit 1 22 and 8.  What goes the general way after all pays 7 us for the attempt.
+// 24.9 and 9.4 to 11.8, fp16 22.8 to 24.7 and 9.0 to 12.3, fp32 33 and 19 to 21 (128 KB through one CU); limit 64 with ties at it 39.5 to 41.6 and 10.8 to
+// 12.7, limit 1 22 and 8; sorted logits bf16 25.6 and 13.7, fp32 35.4 and 22.4; all but 20 masked 19.9 and 7.6, 29.9 and 16.5; out of the middle range 23.6 and
+// 13.4, 33.0 and 22.1.  What goes the general way after all has spent 5 us (fp32 15, its second read) and gets 10 back if a thousand ties at the bound are why:
+// equal logits bf16 46.5 and 41.2, fp32 56.2 and 59.6.
 constexpr int kPickMax = 1024;
-struct PickShared { float l[kPickMax], top[kSampWaves], low[kSampWaves]; int idx[kPickMax], at[kPickMax]; unsigned mass[kPickMax], kept[kPickMax]; int n, few; };
+// Four of each wave's 64 maxima bound 64 tokens (more maxima a wave cost what they save), where every thread has logits.
+__host__ __device__ __forceinline__ bool samp_picks(int top_k, int V) { return top_k > 0 && top_k <= 64 && V >= 8 * kSampThreads; }
+struct PickShared { float l[kPickMax], top[kSampWaves], low[kSampWaves], least[kSampWaves]; int idx[kPickMax], at[kPickMax]; unsigned mass[kPickMax], kept[kPickMax]; int n, few; };
 template <typename T, int NPT>
-__device__ __forceinline__ int samp_pick_few(const T* row, int V, bool vec_ok, int top_k, float temperature, PickShared& ps) {
+__device__ __forceinline__ int samp_pick_few(const T* row, int V, bool vec_ok, int top_k, float temperature, float& reach, PickShared& ps) {
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     Raw8<T> raw[NPT / 8];
 #pragma unroll
@@ -205,18 +224,23 @@ __device__ __forceinline__ int samp_pick_few(const T* row, int V, bool vec_ok, i
             if (at != 0 && lane == (int)__builtin_ctzll(at)) rest = -INFINITY;
         }
     }
-    if (lane == 0) { ps.top[wave] = first; ps.low[wave] = low; }
+    const float least = -mmf_wave_max(-most);
+    if (lane == 0) { ps.top[wave] = first; ps.low[wave] = low; ps.least[wave] = least; }
     __syncthreads();
-    float mx = -INFINITY;
+    float mx = -INFINITY, close = -INFINITY;
     low = INFINITY;
 #pragma unroll
     for (int w = 0; w < kSampWaves; ++w) {
         mx = fmaxf(mx, ps.top[w]);
         low = fminf(low, ps.low[w]);
+        close = fmaxf(close, ps.least[w]);
     }
-    const float scaled = fabsf(__fdiv_rn(low, temperature));
-    if (!(fabsf(low) >= 0x1p-100f && fabsf(low) <= 0x1p100f && scaled >= 0x1p-100f && scaled <= 0x1p100f)) return -1;
-    const float cut = __fsub_rn(low, __fmul_rn(fabsf(low), 0x1p-21f));
+    low = fmaxf(low, close);
+    reach = __fdiv_rn(low, temperature);
+    if (mx == -INFINITY) return -1;
+    float cut = __fsub_rn(low, __fmul_rn(fabsf(low), 0x1p-21f));
+    if (!(fabsf(low) >= 0x1p-100f && fabsf(low) <= 0x1p100f && fabsf(reach) >= 0x1p-100f && fabsf(reach) <= 0x1p100f))
+        cut = samp_lowest_reaching(low, temperature);
     if (most >= cut) {
 #pragma unroll
         for (int j = 0; j < NPT; ++j) {
@@ -282,7 +306,11 @@ __device__ __forceinline__ void samp_finish_listed(PickShared& ps, int n, float 
     }
 }
 
-template <typename T, int NPT>
+// Beyond 32768 tokens an instance for each kind of limit that the host knows: the registers that a thread's 64 logits leave do not hold all ways.  50257 tokens, one row,
+// all in one instance / one each, us: bf16 no limit 115 / 108, 1000 152 / 149, 65 137 / 132; fp32 113 / 112, 146 / 143, 134 / 131.  32 logits a thread take the
+// same time either way (32000 tokens, no limit: 27.8 and 27.9).
+enum Limit : int { kNoLimit, kLargeLimit, kAnyLimit };
+template <typename T, int NPT, int LIMIT>
 __global__ __launch_bounds__(kSampThreads) void sample_top_p_kernel(SampleArgs a) {
     __shared__ u64 hist[kSampBins * kSampCopies];                // 32 KiB
     __shared__ u64 hsum[kSampBins];
@@ -301,15 +329,18 @@ __global__ __launch_bounds__(kSampThreads) void sample_top_p_kernel(SampleArgs a
     const int64_t u_at = blockIdx.x + (a.pos ? (int64_t)a.pos[blockIdx.x] * gridDim.x : 0);
     const bool vec_ok = (V % 8) == 0 && (a.ld % 8) == 0 && (reinterpret_cast<uintptr_t>(a.logits) & 15u) == 0;
 
-    if (top_k > 0 && top_k <= 64 && top_k < V) {                  // four of each wave's 64 maxima bound 64 tokens; more maxima a wave cost what they save
-        __shared__ __align__(16) PickShared ps;
-        const int n = samp_pick_few<T, NPT>(row, V, vec_ok, top_k, temperature, ps);
-        if (n >= 0) {
-            if (n > 64) samp_finish_listed(ps, n, top_p, a.u[u_at], a.out + blockIdx.x);
-            else if (wave == 0) samp_finish_few(ps.mass, ps.at, n, top_p, a.u[u_at], a.out + blockIdx.x);
-            return;
-        }
-        // a clustered or tiny vocabulary, a thousand ties, logits out of range: the general way
+    const bool pick = LIMIT == kAnyLimit && samp_picks(top_k, V) && temperature > 0.0f;
+    float reach = 0.0f;                                           // no more than the top_k-th largest scaled logit
+    __shared__ __align__(16) PickShared ps;
+    if constexpr (LIMIT == kAnyLimit) {
+        if (pick) {
+            const int n = samp_pick_few<T, NPT>(row, V, vec_ok, top_k, temperature, reach, ps);
+            if (n >= 0) {
+                if (n > 64) samp_finish_listed(ps, n, top_p, a.u[u_at], a.out + blockIdx.x);
+                else if (wave == 0) samp_finish_few(ps.mass, ps.at, n, top_p, a.u[u_at], a.out + blockIdx.x);
+                return;
+            }
+        }   // a thousand ties, clusters in several places, no finite logit: the general way
     }
     Raw8<T> raw[NPT / 8];
 #pragma unroll
@@ -333,13 +364,21 @@ __global__ __launch_bounds__(kSampThreads) void sample_top_p_kernel(SampleArgs a
         }
     }
     mx = mmf_wave_max(mx);
+    constexpr bool TIES = LIMIT == kAnyLimit && NPT <= 32;                      // (more logits a thread leave no registers for it)
+    if (TIES && pick) {                                           // ties at the bound: it is the top_k-th largest
+        int larger = 0;
+#pragma unroll
+        for (int j = 0; j < NPT; ++j) larger += l[j] > reach;
+        larger = mmf_wave_sum(larger);
+        if (lane == 0) atomicAdd(&ps.few, larger);
+    }
     if (lane == 0) wmax[wave] = mx;
     __syncthreads();                                              // also publishes the zeroed histogram
 #pragma unroll
     for (int w = 0; w < kSampWaves; ++w) mx = fmaxf(mx, wmax[w]);
 
     unsigned m[NPT];
-    if (top_k > 0 && top_k < V && mx != -INFINITY) {          // a row without a finite logit has no top_k-th largest: it is drawn
+    if (LIMIT != kNoLimit && top_k > 0 && top_k < V && mx != -INFINITY) {          // a row without a finite logit has no top_k-th largest: it is drawn
                                                                    // uniformly like without the limit (every mass is 2^31)
         // order-preserving image of the scaled logits: non-negative floats above the negative ones, -inf and the slots
         // past V at 0 (which the descent ignores)
@@ -348,7 +387,11 @@ __global__ __launch_bounds__(kSampThreads) void sample_top_p_kernel(SampleArgs a
             const unsigned b = __float_as_uint(__fadd_rn(l[j], 0.0f));       // -0 counts as +0, as the comparison of floats does
             m[j] = l[j] == -INFINITY ? 0u : (b & 0x80000000u) ? ~b : (b | 0x80000000u);
         }
-        const unsigned kth = samp_descent<true, NPT>(m, (u64)top_k, hist, hsum, sel);
+        unsigned kth;
+        if (TIES && pick && ps.few < top_k) {
+            const unsigned b = __float_as_uint(__fadd_rn(reach, 0.0f));
+            kth = (b & 0x80000000u) ? ~b : (b | 0x80000000u);
+        } else kth = samp_descent<true, NPT>(m, (u64)top_k, hist, hsum, sel);
         // the kept tokens (top_k of them, more on ties) with their masses, in any order, for one wave to finish
         if (t == 0) few_n = 0;
         __syncthreads();
@@ -441,8 +484,11 @@ __global__ __launch_bounds__(kSampThreads) void sample_top_p_kernel(SampleArgs a
 
 template <typename T>
 int launch_sample(const SampleArgs& a, int64_t rows, hipStream_t s) {
-    if (a.V <= 32 * kSampThreads) sample_top_p_kernel<T, 32><<<(unsigned)rows, kSampThreads, 0, s>>>(a);
-    else sample_top_p_kernel<T, 64><<<(unsigned)rows, kSampThreads, 0, s>>>(a);
+    auto launch = [&](auto* kernel) { kernel<<<(unsigned)rows, kSampThreads, 0, s>>>(a); };
+    if (a.V <= 32 * kSampThreads) launch(sample_top_p_kernel<T, 32, kAnyLimit>);
+    else if (a.params || samp_picks(a.top_k, a.V)) launch(sample_top_p_kernel<T, 64, kAnyLimit>);
+    else if (a.top_k > 0) launch(sample_top_p_kernel<T, 64, kLargeLimit>);
+    else launch(sample_top_p_kernel<T, 64, kNoLimit>);
     MMF_CHECK_LAUNCH();
     return 0;
 }

@@ -165,3 +165,45 @@ def test_ranked_tokens_of_a_small_limit(dev, v, dtype):
     u = torch.rand(rows, generator=g)
     for top_k, temperature, top_p in ((1, 0.6, 0.4), (16, 0.7, 1.0), (17, 3.0, 0.9), (50, 0.6, 0.4), (63, 1.0, 0.97), (64, 0.3, 0.8), (65, 0.6, 0.6)):
         _check_rows(dev, logits, temperature, top_p, u, f"V={v} {dtype} top_k={top_k}", top_k=top_k)
+
+
+@pytest.mark.parametrize("v", [8191, 8192, 32768, 32769])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_small_limits_where_the_bound_is_out_of_the_ordinary(dev, v, dtype):
+    """Vocabularies around the smallest that are ranked and the most a thread holds in one half; bounds at zero, at subnormals, at the largest floats and
+    below every finite logit; thousands of ties at, above and below the limit; the large logits in one wave's places and in several waves'."""
+    g = torch.Generator().manual_seed(43)
+    rows = 12
+    logits = torch.randn(rows, v, generator=g) * 3
+    logits[1] = (logits[1] - 9).clamp(min=0)                                          # a few above zero, thousands of zeros
+    logits[2] = -(logits[2] - 9).clamp(min=0)                                         # and below it
+    logits[3] = torch.where(torch.rand(v, generator=g) < 0.5, -0.0, 0.0)
+    logits[4, 7:] = float("-inf")
+    logits[5, 300:] = float("-inf")
+    logits[6] = torch.randint(-3, 4, (v,), generator=g) * 1e-44
+    logits[7] = torch.randint(1, 4, (v,), generator=g) * 1e38
+    logits[8] = -logits[7]
+    logits[9, 512:1024] += 30.0                                                       # one wave's
+    logits[10, 4096:6144] += 30.0                                                     # four waves'
+    logits[11] = 1.0
+    logits[11, torch.randperm(v, generator=g)[:49]] = 2.0
+    logits = logits.to(dtype)
+    u = torch.rand(rows, generator=g)
+    for top_k, temperature, top_p in ((1, 0.6, 1.0), (49, 0.6, 0.9), (50, 0.6, 0.9), (64, 3.0, 1.0)):
+        _check_rows(dev, logits, temperature, top_p, u, f"V={v} {dtype} top_k={top_k}", top_k=top_k)
+
+
+def test_recorded_draws_with_a_temperature_that_turns_the_order_round(dev):
+    """The parameters of a recorded draw are read on the device, where nothing refuses them: scaled logits decide, as without a limit."""
+    from matmulfreellm_amd import _lib as L
+    g = torch.Generator().manual_seed(44)
+    logits = (torch.randn(4, 32000, generator=g) * 3).bfloat16()
+    u = torch.rand(4, generator=g)
+    x, un, out, pos = logits.to(dev), u.to(dev), torch.full((4,), -1, dtype=torch.int64, device=dev), torch.zeros(4, dtype=torch.int32, device=dev)
+    params = torch.tensor([-0.6, 0.9, 0.0])
+    params[2:].view(torch.int32).fill_(50)
+    params = params.to(dev)
+    L.check(L.load().mmf_sample_top_p_recorded(x.data_ptr(), 32000, 4, 32000, params.data_ptr(), un.data_ptr(), pos.data_ptr(), out.data_ptr(),
+                                               L.dtype_id(x.dtype), L.stream()), "mmf_sample_top_p_recorded")
+    want = [S.sample_top_p_spec(logits[r].float().numpy(), -0.6, 0.9, float(u[r]), top_k=50)[0] for r in range(4)]
+    assert out.tolist() == want
