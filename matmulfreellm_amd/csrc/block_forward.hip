@@ -23,7 +23,7 @@ bool few_rows(const mmf_block* p, int64_t M) {
 // The quantisers of middle-sized prompts bring the weights behind them (the packed bytes of [n, k], n a multiple of 32) into the last-level
 // cache: a contraction that finds them in memory waits for each of its first k-blocks.  us a launch at the 1.3B shape, weights in memory and in the
 // cache: 459 rows, i/f/g 13.4 and 12.4, o 7.0 and 6.2, gate/up 19.9 and 18.5, down 13.0 and 11.9; 1377 rows 25.8 / 25.0, 13.2 / 11.7, 33.4 / 32.8,
-// 23.6 / 20.5.  The quantiser, 9 to 12 us of 1377 rows, takes 0.3 us more.  Forwards: 3 x 459 tokens 3630 -> 3530 us, 2 x 1001 with logits 4406 -> 4285,
+// 23.6 / 20.5.  The quantiser, 8 to 9 us of 1377 rows, takes 0.1 to 0.5 us more, memory's time for the weights.  Forwards: 3 x 459 tokens 3630 -> 3530 us, 2 x 1001 with logits 4406 -> 4285,
 // 270 tokens 1603 -> 1576, 2 x 2000 6398 -> 6320; 370M shape, 4 x 700 2781 -> 2754.  With fewer rows the quantiser is as short as memory's answer (a
 // decode step of 64 rows 0.5 to 5 % longer, however the touches were spread over its launches); with 8192 and 16384, rounds of tiles hide
 // the start and the touches only delay the rows (1 to 2 % of a forward).

@@ -581,21 +581,25 @@ __device__ __forceinline__ float mmf_block_max_once(float v, float* slot) {
 }
 
 // What a launch behind this one reads first, its packed weights, is brought into the last-level cache meanwhile: a wave touches a dword of each of
-// 64 lines of 128 bytes and waits for none of them.  `slot` numbers the waves of the grid.  The touch stands behind the kernel's own
-// loads, which return in order, and its value is kept (mmf_touched, at the end) only so that the load is.
+// 64 lines of 128 bytes.  `slot` numbers the waves of the grid.  The touch stands behind the kernel's own loads, and loads return in order, so that no wait
+// for those is one for it.  That takes a load that no branch goes around (behind a branch's end the compiler waits for all that may be in flight):
+// what lies past the last line, or everything where there is nothing to read, is past the descriptor's records and asks memory for nothing.
+// mmf_touched, at the kernel's end, keeps the value so that the load is kept, and waits for it.
+// Quantisers of 300 to 5000 rows take the same time to 0.2 us as with a wait in the middle of the row; forwards of 3 x 459, 2 x 1001 and 2 x 2000 tokens
+// (1.3B) went from 3292 to 3277, 4310 to 4285 and 6556 to 6530 us.
 struct MmfAhead { const unsigned char* p; uint32_t lines; };
 __device__ __forceinline__ uint32_t mmf_touch(const MmfAhead& a, uint32_t slot) {
-    const uint32_t line = slot * 64 + (threadIdx.x & 63);
-    uint32_t v = 0;
-    if (line < a.lines) v = *reinterpret_cast<const uint32_t*>(a.p + (uint64_t)line * 128);
-    return v;
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)a.p, 0, (int)(a.lines * 128), 0x00020000);
+    __builtin_amdgcn_sched_barrier(0x38f);                                       // no memory load moves behind the touch
+    const uint32_t last = 1 << 18;                                               // (no wave behind 2 GiB starts over)
+    return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, ((slot < last ? slot : last) * 64 + (threadIdx.x & 63)) * 128, 0, 0);
 }
 __device__ __forceinline__ void mmf_touched(uint32_t v) { asm volatile("" ::"v"(v)); }
 static inline int mmf_set_ahead(MmfAhead& a, const void* p, int64_t bytes) {
     if (bytes < 0) return MMF_ERR_ARG;
     if (reinterpret_cast<uintptr_t>(p) & 15u) return MMF_ERR_ALIGN;
     a.p = static_cast<const unsigned char*>(p);
-    a.lines = p ? (uint32_t)(bytes / 128 < (1 << 24) ? bytes / 128 : 1 << 24) : 0;   // (2 GiB)
+    a.lines = p ? (uint32_t)(bytes / 128 < (1 << 24) - 1 ? bytes / 128 : (1 << 24) - 1) : 0;   // (2 GiB)
     return 0;
 }
 
