@@ -466,7 +466,7 @@ int mmf_transpose16(const void* x, int64_t rows, int64_t cols, void* out, void* 
  * mmf_weight_grad: dw[i] [N[i], K[i]] = dout[i] [M, N[i]]^T @ y[i] [M, K[i]] for 1 to 8 products over the same M >= 1 rows, fp32 sums, one
  *   rounding.  dout, lddout, y, ldy, dw, N, K: HOST arrays (device pointers in the first, third and fifth; row strides in elements, up to
  *   2^24).  N, K and the row strides multiples of 8 (fp32: 4), pointers 16-byte aligned (else MMF_ERR_ALIGN).  workspace:
- *   mmf_weight_grad_workspace_bytes of the same products, M and dtype (0: may be null), at most 1 GiB. */
+ *   mmf_weight_grad_workspace_bytes of the same products, M and dtype (0: may be null), at most 192 MiB. */
 int64_t mmf_weight_grad_workspace_bytes(int products, const int64_t* N, const int64_t* K, int64_t M, int dtype);
 int mmf_weight_grad(int products, const void* const* dout, const int64_t* lddout, const void* const* y, const int64_t* ldy, void* const* dw,
                     const int64_t* N, const int64_t* K, int64_t M, int dtype, void* workspace, void* stream);

@@ -293,19 +293,30 @@ PyObject* block_backward(PyObject*, PyObject* const* args, Py_ssize_t count) {
         const int dt = dtype_of(x.scalar_type());
         const Tensor none, x2 = x.view({m, H});
         std::pair<Tensor, Tensor> products[6];
-        auto product = [&](int i, const Tensor& d, const Tensor& yq) { products[i] = {need[i] ? d : none, yq}; };
+        auto product = [&](int i, const Tensor& d, const Tensor& yq) { if (need[i]) products[i] = {d, yq}; };
+        // The weights' products wait for each other with their operands, 7.75 rows of H an input row at I = 2.75 H.  What nothing reads any more is given
+        // back as soon as its last reader is launched, some 10 rows of H, so that a step takes no more memory than with a product at a time.
         // down_proj behind the swiglu: the gradients of gate and up land side by side
-        const Tensor dz = at::mm(d2, dense(pw[3], like)), dy = at::empty(y.sizes(), like);
+        Tensor dz = at::mm(d2, dense(pw[3], like)), dy = at::empty(y.sizes(), like);
         Chained down = chain(CHAIN_SWIGLU, y.narrow(1, 0, I), y.narrow(1, I, I), none, 0.0, {nw[8]}, eps[6], {dz}, none, dy.narrow(1, 0, I), dy.narrow(1, I, I));
+        dz.reset();
         product(5, d2, down.y[0]);
+        down.y.reset();
         // gate_proj behind mlp_norm, the residual's gradient joining
-        const Tensor dh = at::mm(dy, dense(pw[2], like));
+        Tensor dh = at::mm(dy, dense(pw[2], like));
         Chained gate = chain(CHAIN_RESNORM, attn, x2, nw[1], eps[4], {nw[7]}, eps[5], {dh}, d2, none, none);
+        dh.reset();
         product(4, dy, gate.y[0]);
+        gate.y.reset();
+        dy.reset();
+        down.dx.reset();
         // o_proj behind the gated norm: the g columns of the stacked projection's gradient, and the scan's output
-        const Tensor &dres = gate.dx, do2 = at::mm(dres, dense(pw[1], like)), difg = at::empty(ifg.sizes(), like), dout = at::empty(o.sizes(), like);
+        const Tensor& dres = gate.dx;
+        Tensor do2 = at::mm(dres, dense(pw[1], like)), difg = at::empty(ifg.sizes(), like), dout = at::empty(o.sizes(), like);
         Chained oc = chain(CHAIN_GATED, ifg.narrow(1, 2 * D, D), o, nw[2], eps[2], {nw[6]}, eps[3], {do2}, none, difg.narrow(1, 2 * D, D), dout);
+        do2.reset();
         product(3, dres, oc.y[0]);
+        oc.y.reset();
         // scan and gate math
         const auto f32 = like.dtype(at::kFloat);
         const Tensor gates = xg[1].contiguous(), out = o.contiguous();
@@ -314,6 +325,8 @@ PyObject* block_backward(PyObject*, PyObject* const* args, Py_ssize_t count) {
         check(mmf_hgrn_recurrent_bwd_split(gates.data_ptr(), out.data_ptr(), dout.data_ptr(), nullptr, dxs.data_ptr(), dgs.data_ptr(), b, t, D, 0, dt, floats(ws),
                                            stream_of(x)),
               "mmf_hgrn_recurrent_bwd_split");
+        dout.reset();
+        ws.reset();
         if (lb.defined()) {
             dlb = at::empty({D}, f32);
             part = at::empty({mmf_backward_groups(m), D}, f32);
@@ -323,13 +336,18 @@ PyObject* block_backward(PyObject*, PyObject* const* args, Py_ssize_t count) {
         check(mmf_hgrn_gate_bwd(ii.data_ptr(), 3 * D, ff.data_ptr(), 3 * D, floats(lb), static_cast<const uint8_t*>(address(mask)), dxs.data_ptr(), dgs.data_ptr(),
                                 di.data_ptr(), 3 * D, df.data_ptr(), 3 * D, floats(part), floats(dlb), m, D, dt, stream_of(x)),
               "mmf_hgrn_gate_bwd");
+        dxs.reset();
+        dgs.reset();
         // i, f, g behind attn_norm: three products, one pass over the rows, the residual's gradient joining
-        const Tensor w3 = dense(pw[0], like), dh3 = at::empty({3, m, H}, like), dhs[3] = {dh3[0], dh3[1], dh3[2]};
-        for (int j = 0; j < 3; ++j) {
-            Tensor to = dhs[j];
-            at::mm_out(to, column(difg, j), w3.narrow(0, j * D, D));
+        Chained in;
+        {
+            const Tensor w3 = dense(pw[0], like), dh3 = at::empty({3, m, H}, like), dhs[3] = {dh3[0], dh3[1], dh3[2]};
+            for (int j = 0; j < 3; ++j) {
+                Tensor to = dhs[j];
+                at::mm_out(to, column(difg, j), w3.narrow(0, j * D, D));
+            }
+            in = chain(CHAIN_NORM, x2, none, nw[0], eps[0], {nw[3], nw[4], nw[5]}, eps[1], dhs, dres, none, none);
         }
-        Chained in = chain(CHAIN_NORM, x2, none, nw[0], eps[0], {nw[3], nw[4], nw[5]}, eps[1], dhs, dres, none, none);
         for (int j = 0; j < 3; ++j) product(j, column(difg, j), in.y[j]);
         const std::vector<Tensor> dw = weight_grads(products);
         grads[0] = in.dx.view(x.sizes());

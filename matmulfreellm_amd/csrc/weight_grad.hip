@@ -21,7 +21,7 @@ namespace {
 constexpr int kSide = 256, kSide32 = 128, kRows = 32, kOperand = kRows * kSide * 2, kBuffer = 2 * kOperand, kBuffers = 4, kCUs = 256, kMaxProducts = 8;
 constexpr int kRows32 = 16, kOperand32 = kRows32 * kSide32 * 4, kBuffer32 = 2 * kOperand32, kFlight32 = kBuffer32 / 1024 / 4;
 constexpr int kFlight = kBuffer / 1024 / 4;                         // transfers of 1 KiB that a wave issues per buffer
-constexpr int kMaxSplit = 16;
+constexpr int kMaxSplit = 16, kMaxSlices = 768, kMaxSlices32 = 3072;  // 192 MiB
 
 struct Product {
     const void* p;          // dout, row stride ldp
@@ -402,14 +402,15 @@ __global__ __launch_bounds__(256) void weight_grad_sum_kernel(GradArgs a) {
 // The tiles behind the last whole round of the chip, cut into slices of the rows where that is estimated to end sooner: microseconds from a stage's
 // 0.85, a workgroup's start and end 5, the second launch 4 and 0.1 per slice written and read.  8192 rows, as they are / cut: one product of
 // 2048 x 2048 (64 tiles, 4 slices) 167 / 80 us, 11264 x 2048 (96 of 352 tiles, 2 slices) 360 / 313, 2048 x 5632 (176 tiles) 179 whole, 228 in 4.
-// Single precision: 0.95 a stage, 0.025 a slice.
+// Single precision: 0.95 a stage, 0.025 a slice.  The slices of a launch are held to 192 MiB of workspace: for blocks of widths 256 to 4096 the estimate is that
+// without a bound up to 16384 rows, and 0 to 7 % above it at 32768, 0 to 15 % at 65536 (1024 wide).
 struct GradPlan { int full, rest, split; };
 GradPlan grad_plan(int64_t tiles, int64_t M, bool f32) {
     const int64_t stages = mmf_ceil_div(M, f32 ? kRows32 : kRows), rest = tiles % kCUs;
     const double stage = f32 ? 0.95 : 0.85, slice = f32 ? 0.025 : 0.1;
     int best = 1;
     double least = 0.0;
-    for (int s = 1; s <= kMaxSplit && stages / s >= (f32 ? 2 : 4); ++s) {
+    for (int s = 1; s <= kMaxSplit && (s == 1 || rest * s <= (f32 ? kMaxSlices32 : kMaxSlices)) && stages / s >= (f32 ? 2 : 4); ++s) {
         const double us = (double)mmf_ceil_div(rest * s, kCUs) * ((double)mmf_ceil_div(stages, s) * stage + 5.0) + (s > 1 ? 4.0 + slice * (double)(rest * s) : 0.0);
         if (s == 1 || us < least) {
             best = s;
