@@ -356,7 +356,7 @@ class NormHeadFn(torch.autograd.Function):
         x, norm_weight, head_norm_weight = ctx.saved_tensors
         with L.on(x.device):
             x2, d2 = _2d(x).contiguous(), _2d(dout).to(x.dtype).contiguous()
-            dh = d2 @ _dense_weight(ctx.pw, x.dtype)
+            dh = (d2 @ _dense_weight(ctx.pw, x.dtype)).to(x.dtype)    # (another type under autocast)
             dx, _, yq, dw = _chain_bwd(CHAIN_NORM, x2, None, norm_weight, ctx.eps1, [head_norm_weight], ctx.eps2, [dh])
             d_weight = _weight_grad(d2, yq[0]) if ctx.needs_input_grad[3] else None
         return dx.view(x.shape), dw[0], dw[1], d_weight, None, None, None

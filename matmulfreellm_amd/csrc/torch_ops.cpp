@@ -289,6 +289,8 @@ PyObject* block_backward(PyObject*, PyObject* const* args, Py_ssize_t count) {
     try {
         NoGil nogil;
         OnDevice on(x.get_device());
+        // backward() may be called under autocast, which would give the row kernels products of another type than they read
+        c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
         const auto like = x.options().requires_grad(false);
         const int dt = dtype_of(x.scalar_type());
         const Tensor none, x2 = x.view({m, H});

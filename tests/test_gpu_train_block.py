@@ -238,3 +238,21 @@ def test_the_backward_of_a_block_takes_no_more_memory_than_with_a_product_at_a_t
         peak = torch.cuda.max_memory_allocated() - base - sum(g.numel() * g.element_size() for g in grads[2:])
         del out, grads
     assert peak <= 23 * x.numel() * x.element_size(), peak / (x.numel() * x.element_size())
+
+
+def test_backward_under_autocast(dev):
+    """loss.backward() inside a region of autocast, the forward outside: the row kernels read their operands' own type.  The blocks' gradients see autocast
+    only through the head's products (bf16: 2^-8 an operand)."""
+    import matmulfreellm_amd as mm
+    torch.manual_seed(37)
+    model = mm.HGRNBitForCausalLM(mm.HGRNBitConfig(vocab_size=200, hidden_size=256, num_hidden_layers=2)).to(dev).train()
+    ids = torch.randint(0, 200, (2, 65), device=dev)
+    grads = []
+    for enabled in (False, True):
+        model.zero_grad(set_to_none=True)
+        loss = model(input_ids=ids, labels=ids).loss
+        with torch.autocast("cuda", torch.bfloat16, enabled=enabled):
+            loss.backward()
+        grads.append({n: p.grad.double() for n, p in model.named_parameters()})
+    for name, want in grads[0].items():
+        assert ((grads[1][name] - want).norm() / want.norm()).item() < 1e-2, name
