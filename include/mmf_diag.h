@@ -1,4 +1,4 @@
-/* libmmf_hip -- measuring aids (no counterpart in the reference; only bench.py binds them).
+/* libmmf_hip -- measuring aids (no counterpart in the reference; bench.py and the tests bind them).
  *
  * They are exported by the same library as the product entry points of mmf.h but are not part of the drop-in boundary:
  * nothing on a product path calls them.
@@ -24,6 +24,11 @@ extern "C" {
  *   and ternary weights (the switching activity, hence the power draw, of real operands) instead of constant ones. */
 int mmf_bitlinear_mfma_clock_sink(int64_t* sink, int64_t workgroups);
 int mmf_mfma_pipe_probe(int64_t steps, int64_t workgroups, int random_operands, int64_t* clocks, void* stream);
+
+/* mmf_bitlinear_mfma_plan: what mmf_bitlinear_mfma (config < 0; seg = 0), mmf_bitlinear_mfma_multi (seg: its seg_rows) or mmf_bitlinear_mfma_swiglu
+ *   launch for a shape: the rows of the first launch (M: the only one) and the kernels of the first and the second (-1: none), numbered as `config`
+ *   is.  Host code alone, no device. */
+int mmf_bitlinear_mfma_plan(int64_t M, int64_t K, int64_t N, int64_t seg, int swiglu, int64_t* first_rows, int* configs);
 
 /* mmf_decode_layers_traced: mmf_decode_layers (see mmf.h) built with its cycle trace, and with the hold-back of a link's
  *   first poll as an argument (`delay`, in units of about 64 cycles, 0..64).

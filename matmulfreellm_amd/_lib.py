@@ -90,6 +90,7 @@ SIGNATURES = {
     "mmf_rmsnorm_quant_multi": (_i32, [_ptr, _i64, _ptr, _f32, _ptr, _ptr, _ptr, _f32, _ptr, _ptr, _ptr, _i64, _i64, _i32, _i32, _ptr]),
     "mmf_rmsnorm_quant_multi_ahead": (_i32, [_ptr, _i64, _ptr, _f32, _ptr, _ptr, _ptr, _f32, _ptr, _ptr, _ptr, _i64, _i64, _ptr, _i64, _i32,
                                              _i32, _ptr]),
+    "mmf_bitlinear_mfma_plan": (_i32, [_i64, _i64, _i64, _i64, _i32, _ptr, _ptr]),
     "mmf_bitlinear_mfma_multi": (_i32, [_ptr, _i64, _ptr, _ptr, _ptr, _ptr, _i64, _ptr, _i64, _i64, _i64, _i64, _i32, _i32, _ptr]),
     "mmf_bitlinear_gemv_multi": (_i32, [_i32, _ptr, _i64, _ptr, _f32, _ptr, _ptr, _ptr, _f32, _ptr, _ptr, _i64, _ptr, _ptr, _ptr, _ptr,
                                         _i64, _i64, _i64, _i32, _i32, _ptr]),

@@ -1100,6 +1100,16 @@ inline MfmaChoice mfma_choice(int64_t M, int64_t N, int64_t Kp, bool swiglu) {
     return {MfmaPick::kTiles, t_tiles};
 }
 
+// The kernel of a choice (dispatch_mfma's numbers), and the columns of its tiles: 0 where they are never several segments' in one launch.
+inline int mfma_config(MfmaPick pick, int64_t M, int64_t N) {
+    if (pick == MfmaPick::kStream) return 5;
+    if (M <= 64) return M <= 32 ? 0 : 1;
+    return pick == MfmaPick::kSplit ? 18 : pick == MfmaPick::kNarrow ? 19 : N >= 512 ? 17 : 16;
+}
+inline int64_t mfma_tile_cols(int config) { return config == 5 ? 32 : config == 19 ? 128 : config == 16 || config == 18 ? 256 : config == 17 ? 512 : 0; }
+// tiles that suit segments with codes of their own (of seg columns; 0: one set of codes)
+inline bool mfma_suits(int config, int64_t N, int64_t seg) { return seg == 0 || N <= seg || (mfma_tile_cols(config) && seg % mfma_tile_cols(config) == 0); }
+
 // The rows of the first of two launches, or all of them: where the tiles' last round holds a few of them, its rows go in a launch of their own, most
 // often the stream's.  us, one launch / two (rows of the second): 2048 -> 6144, 1377 rows (528 split tiles; 33) 27.2 / 23.3, 2693 (5) 36.6 / 29.0, 5549 (109)
 // 59.6 / 54.5; gate and up to 5632 with swiglu, 3066 (122) 80.6 / 73.7, 715 (11) 26.3 / 25.2; 5632 -> 2048, 2096 (48) 32.6 / 27.7; 1536 -> 4608, 3586 (2)
@@ -1107,9 +1117,14 @@ inline MfmaChoice mfma_choice(int64_t M, int64_t N, int64_t Kp, bool swiglu) {
 // on average, 15 % more at most.  Where the estimate has to promise 7 % (10 % from 129 rows on; 3 % with swiglu, whose rounds take longer than
 // estimated) none took longer.  With 340 to 600 rows in the second two launches took between 12 % less and 12 % more (2048 -> 6144, 4843 (747)
 // 47.7 / 53.5; 6912 -> 2560, 5431 (567) 70.6 / 79.2).  The sums are integers and a row's do not depend on the others: the same bits.
+// Segments with codes of their own (seg columns) that do not suit a launch's tiles take a launch each, which no estimate covers: rows are cut only where all three
+// launches suit them (three of 2304, cut all the same / in one go: 1157 rows 53.1 / 27.9 us, 2445 61.8 / 47.8; of 1152, 2473 36.1 / 32.4).
 constexpr int64_t kCutRows = 320;
-inline int64_t mfma_first_rows(int64_t M, int64_t N, int64_t Kp, bool swiglu) {
-    const double whole = mfma_choice(M, N, Kp, swiglu).us;
+inline int64_t mfma_first_rows(int64_t M, int64_t N, int64_t Kp, int64_t seg, bool swiglu) {
+    auto suits = [&](const MfmaChoice& c, int64_t m) { return mfma_suits(mfma_config(c.pick, m, N), N, seg); };
+    const MfmaChoice all = mfma_choice(M, N, Kp, swiglu);
+    const double whole = all.us;
+    if (!suits(all, M)) return M;
     double least = whole;
     int64_t first = M;
     for (const int64_t cols : {256, 512}) {
@@ -1117,8 +1132,9 @@ inline int64_t mfma_first_rows(int64_t M, int64_t N, int64_t Kp, bool swiglu) {
         for (int64_t r = rounds - 1; r >= 1 && r >= rounds - 2; --r) {
             const int64_t m = 256 * r / across * 64;
             if (m < 64 || m >= M || M - m > kCutRows) continue;
-            const double us = mfma_choice(m, N, Kp, swiglu).us + mfma_choice(M - m, N, Kp, swiglu).us;
-            if (us < least && us < (swiglu ? 0.97 : M - m <= 128 ? 0.93 : 0.90) * whole) {
+            const MfmaChoice head = mfma_choice(m, N, Kp, swiglu), tail = mfma_choice(M - m, N, Kp, swiglu);
+            const double us = head.us + tail.us;
+            if (suits(head, m) && suits(tail, M - m) && us < least && us < (swiglu ? 0.97 : M - m <= 128 ? 0.93 : 0.90) * whole) {
                 least = us;
                 first = m;
             }
@@ -1147,23 +1163,16 @@ int dispatch_mfma(const MfmaArgs& a, int config, hipStream_t s, bool cut = true)
     //   15 / 16 / 17  256x256 / 128x256 / 64x512 tiles, A staged by DMA (17: every wave reads the whole activation
     //            tile from LDS and owns its own weight columns, so no weight block is fetched twice)
     if (config < 0) {
-        const int64_t first = cut ? mfma_first_rows(a.M, a.N, a.Kp, false) : a.M;
+        const int64_t first = cut ? mfma_first_rows(a.M, a.N, a.Kp, a.a_seg ? a.seg_rows : 0, false) : a.M;
         if (first < a.M) {
             if (const int rc = dispatch_mfma<T>(mfma_rows<T>(a, 0, first), -1, s, false)) return rc;
             return dispatch_mfma<T>(mfma_rows<T>(a, first, a.M - first), -1, s, false);
         }
-        const MfmaPick pick = mfma_choice(a.M, a.N, a.Kp, false).pick;
-        if (pick == MfmaPick::kStream) config = 5;
-        else if (a.M <= 32) config = 0;
-        else if (a.M <= 64) config = 1;
-        else if (pick == MfmaPick::kSplit) config = 18;
-        else if (pick == MfmaPick::kNarrow) config = 19;
-        else config = a.N >= 512 ? 17 : 16;
+        config = mfma_config(mfma_choice(a.M, a.N, a.Kp, false).pick, a.M, a.N);
     }
     if ((config == 18 || config == 19) && (a.Kp >> 7) % 2 != 0) return MMF_ERR_ARG;
     if (config == 5 && (a.Kp > 8192 || a.M > 65535 * 32)) return MMF_ERR_ARG;
-    const int64_t tile_cols = config == 5 ? 32 : config == 19 ? 128 : config == 16 || config == 18 ? 256 : config == 17 ? 512 : 0;
-    if (a.a_seg != 0 && a.N > a.seg_rows && (tile_cols == 0 || a.seg_rows % tile_cols != 0)) {
+    if (a.a_seg != 0 && !mfma_suits(config, a.N, a.seg_rows)) {
         // tiles that would straddle two segments (or tiles of the kernels that take one set of codes): a launch per segment
         for (int64_t n0 = 0; n0 < a.N; n0 += a.seg_rows) {
             const int64_t seg = n0 / a.seg_rows;
@@ -1195,7 +1204,7 @@ int dispatch_mfma(const MfmaArgs& a, int config, hipStream_t s, bool cut = true)
 
 template <typename T>
 int dispatch_mfma_swiglu(const MfmaArgs& a, hipStream_t s, bool cut = true) {
-    const int64_t first = cut ? mfma_first_rows(a.M, a.N, a.Kp, true) : a.M;
+    const int64_t first = cut ? mfma_first_rows(a.M, a.N, a.Kp, 0, true) : a.M;
     if (first < a.M) {
         if (const int rc = dispatch_mfma_swiglu<T>(mfma_rows<T>(a, 0, first), s, false)) return rc;
         return dispatch_mfma_swiglu<T>(mfma_rows<T>(a, first, a.M - first), s, false);
@@ -1263,6 +1272,19 @@ int mmf_mfma_pipe_probe(int64_t steps, int64_t workgroups, int random_operands, 
     mfma_pipe_probe_kernel<<<(unsigned)workgroups, 512, 0, stream>>>(steps, random_operands, reinterpret_cast<long long*>(clocks),
                                                                     reinterpret_cast<int*>(clocks + 2 * workgroups));
     MMF_CHECK_LAUNCH();
+    return 0;
+}
+
+int mmf_bitlinear_mfma_plan(int64_t M, int64_t K, int64_t N, int64_t seg, int swiglu, int64_t* first_rows, int* configs) {
+    if (M < 1 || K < 1 || N < 1 || N > 0x7fffffff || seg < 0 || !first_rows || !configs) return MMF_ERR_ARG;
+    const int64_t Kp = mmf_round_up(K, 128), first = mfma_first_rows(M, N, Kp, seg, swiglu != 0);
+    auto config = [&](int64_t m) {
+        const MfmaPick pick = mfma_choice(m, N, Kp, swiglu != 0).pick;
+        return !swiglu ? mfma_config(pick, m, N) : pick == MfmaPick::kStream ? 5 : pick == MfmaPick::kSplit ? 18 : 17;
+    };
+    *first_rows = first;
+    configs[0] = config(first);
+    configs[1] = first < M ? config(M - first) : -1;
     return 0;
 }
 

@@ -3,6 +3,8 @@ test_gpu_ops.py), with one row and with many behind the last whole round, a resi
 import pytest
 import torch
 
+from test_contraction_plan import plan
+
 pytestmark = pytest.mark.gpu
 
 
@@ -21,8 +23,9 @@ def _operands(dev, m, k, n, dtype, segments=1):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
 @pytest.mark.parametrize("m,k,n,pad,extra", [(1345, 2048, 6144, 0, None), (1377, 2048, 6112, 64, None), (1449, 2048, 6144, 0, "bias"),
-                                             (2096, 5632, 2048, 0, "addend"), (2368, 5632, 2048, 16, "addend"), (2743, 1024, 3072, 0, None)])
+                                             (2096, 5632, 2048, 0, "addend"), (2096, 5632, 2048, 16, "addend"), (2743, 1024, 3072, 0, None)])
 def test_rows_in_two_launches(dev, dtype, m, k, n, pad, extra):
+    assert plan(m, k, n)[0] < m
     L, lib, w, _, q, deq, qsum, wdeq = _operands(dev, m, k, n, dtype)
     other = torch.randn(m, n + pad, device=dev).to(dtype)
     bias = torch.randn(n, device=dev).to(dtype)
@@ -43,6 +46,7 @@ def test_rows_in_two_launches(dev, dtype, m, k, n, pad, extra):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("m,k,n,seg", [(1377, 2048, 6144, 2048), (1345, 2048, 6144, 2048), (1093, 2560, 7680, 2560), (2743, 1024, 3072, 1024)])
 def test_segments_with_codes_of_their_own(dev, dtype, m, k, n, seg):
+    assert plan(m, k, n, seg)[0] < m
     L, lib, w, stride, q, deq, qsum, wdeq = _operands(dev, m, k, n, dtype, n // seg)
 
     def run(config):
@@ -59,6 +63,7 @@ def test_segments_with_codes_of_their_own(dev, dtype, m, k, n, seg):
 @pytest.mark.parametrize("m,k,n", [(715, 2048, 11264), (705, 2048, 11264), (3066, 2048, 11264), (1848, 2560, 13824)])
 def test_swiglu_rows_in_two_launches(dev, dtype, m, k, n):
     """Against launches of 128 rows each, which are not cut."""
+    assert plan(m, k, n, 0, 1)[0] < m and plan(128, k, n, 0, 1)[0] == 128
     L, lib, w, _, q, deq, qsum, wdeq = _operands(dev, m, k, n, dtype)
     deq *= 1e-3                                                     # gates in the sigmoid's range
 

@@ -3,6 +3,8 @@ dispatch takes them the bits of the other tiles."""
 import pytest
 import torch
 
+from test_contraction_plan import plan
+
 pytestmark = pytest.mark.gpu
 
 
@@ -32,6 +34,7 @@ def test_narrow_tiles_vs_oracle(dev, dtype, m, k, n):
 def test_dispatch_to_narrow_tiles(dev, m, k, n):
     import matmulfreellm_amd.functional as F_
     from matmulfreellm_amd import _lib as L
+    assert 19 in plan(m, k, n)[1:]
     torch.manual_seed(m)
     pw = F_.ternarize_pack((torch.randn(n, k, device=dev) * 0.02).bfloat16())
     q = torch.randint(-127, 128, (L.load().mmf_codes_bytes(m, k, 1),), dtype=torch.int8, device=dev)
