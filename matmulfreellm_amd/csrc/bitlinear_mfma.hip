@@ -1058,8 +1058,9 @@ int launch_mfma(MfmaArgs a, hipStream_t s) {
 // 39.7 / 43.3, 6500 86.5 / 77.4; 2048 -> 2048 (16), 2002 rows 12.2 / 15.1, 3600 18.0 / 18.5; 2048 -> 6144, 2002 rows (768) 27.1 / 26.4.  Stream against split:
 // 1024 -> 5632, 300 rows 6.0 / 8.4, 700 9.9 / 9.4; 2048 -> 2048, 1203 rows 10.9 / 11.4, 1395 12.1 / 11.3.
 // Over 389 shapes, 66 to 8000 rows, the choice costs 0.01 % against the best of the three on average, 15 % at most (377 x 1536 -> 4608: 1.2 us).
-//   narrow tiles   (64 x 128, split like the others) where they give every CU at most one, or three in all; with rows of 2560 and more also instead of a
-//                  split one on nearly every CU.  us, best of the others / narrow: 5632 -> 2048, 700 rows 15.6 / 12.8, 1001 (256 narrow tiles) 19.0 / 13.9, 1377 (352)
+//   narrow tiles   (64 x 128, split like the others) where they give every CU at most one, or three in all; with rows of 2560 to 6144 also instead of a
+//                  split one on nearly every CU (481 to 512 of them: over 73 shapes 1.3 % less on average, from 10 % less to 4 % more, most where their last row of
+//                  tiles is nearly empty; rows of 6912 0.6 % more).  us, best of the others / narrow: 5632 -> 2048, 700 rows 15.6 / 12.8, 1001 (256 narrow tiles) 19.0 / 13.9, 1377 (352)
 //                  20.1 / 20.5, 2002 (512) 24.5 / 23.2, 2400 (608) 32.9 / 29.2; 2048 -> 2048, 830 rows 8.3 / 7.4, 1001 9.2 / 7.8, 1200 (304) 10.4 / 10.8, 2002
 //                  11.7 / 11.8; 2816 -> 1024, 1600 rows 11.9 / 8.4, 4022 (504) 16.4 / 14.5, 4100 (520) 19.7 / 17.4; 2560 -> 2560, 711 rows 11.3 / 8.4, 1491 (480) 13.0 / 13.2,
 //                  1966 (620) 20.3 / 18.4; 2048 -> 6144, 320 rows 9.3 / 7.6.  Weights that an XCD's L2 does not hold cost it more (6912 -> 2560, 580 rows 18.9 / 19.2,
@@ -1090,7 +1091,7 @@ inline MfmaChoice mfma_choice(int64_t M, int64_t N, int64_t Kp, bool swiglu) {
     if (!swiglu) {
         const int64_t narrow = mmf_ceil_div(M, 64) * mmf_ceil_div(N, 128);
         if (narrow <= 256) t_narrow = 3.9 + 0.17 * kb + (double)narrow / 256.0 * (0.3 + 0.045 * kb) + (N * Kp > 16 << 20 ? 0.1 * kb : 0.0);
-        else if (narrow > 480 && half <= 256 && KB >= 20) t_narrow = t_split - 0.1;
+        else if (narrow > 480 && half <= 256 && KB >= 20 && KB <= 48) t_narrow = t_split - 0.1;   // (instead of a split one, whatever that is estimated at)
         else if (narrow > 512 && narrow <= 768) t_narrow = 7.0 + 0.54 * kb;
     }
     if (KB % 2 != 0) t_split = t_narrow = 1e30;
