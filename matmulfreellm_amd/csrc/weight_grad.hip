@@ -45,9 +45,10 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 union Frag { v4s h[2]; v8b b; v8h f; };
 
 // 64 lanes x 16 bytes from `base` + off to LDS, lane order.  In assembly so that the compiler, which would answer the builtin with a wait
-// for every transfer in front of the next LDS read, does not see an LDS write in flight: the kernel waits itself.  No other
-// vector-memory operation is in flight beside these, and among themselves they complete in the order issued (what keeps no
-// order is a transfer and an ordinary load): the same bits as with waits for all of them, operands cold, warm and beside other traffic.
+// for every transfer in front of the next LDS read, does not see an LDS write in flight: the kernel waits itself, by a count of those that may
+// still be on their way.  Among themselves transfers complete in the order issued (what keeps no order is a transfer and an ordinary load); the 16-bit kernels
+// spill a register in front of the first of them (six or seven more behind the loop, none in it), and one more operation on its way can only make a
+// counted wait longer.  The same bits as with waits for all of them, operands cold, warm and beside other traffic.
 __device__ __forceinline__ void grad_dma(const void* base, uint32_t off, uint32_t lds) {
     const uint64_t b = (uint64_t)base;
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(b) : "memory");

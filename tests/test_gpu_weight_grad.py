@@ -46,6 +46,25 @@ def test_weight_gradients_are_the_products(dev, m, shapes, dtype):
         assert bool(((o.double() - want).abs() <= eps * want.abs() + m * 2.0 ** -24 * scale + 2.0 ** -25).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("m,shapes", [c for c in CASES if c[0] > 161])
+def test_many_rows_lose_no_bits_of_their_operands(dev, m, shapes, dtype):
+    """Sums of at most nine terms that are not zero, rows m // 8 apart: within half a unit of the rounding and nine of the sums', where m units of a full sum
+    would hide operands of 11 bits."""
+    g = torch.Generator().manual_seed(m)
+    apart = m // 8
+    pairs = []
+    for n, k in shapes:
+        y = torch.randn(m, k, generator=g) * (torch.arange(m)[:, None] % apart == torch.arange(k) % apart)
+        pairs.append((torch.randn(m, n, generator=g).to(dtype).to(dev), y.to(dtype).to(dev)))
+    rc, out, _ = grads(pairs, dtype)
+    assert rc == 0
+    eps = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -23}[dtype]
+    for (d, y), o in zip(pairs, out):
+        want, scale = d.double().t() @ y.double(), d.double().abs().t() @ y.double().abs()
+        assert bool(((o.double() - want).abs() <= eps * want.abs() + 9 * 2.0 ** -24 * scale + 2.0 ** -25).all())
+
+
 def test_not_a_number_reaches_its_row_and_column_only(dev):
     d, y = torch.ones(70, 264, dtype=torch.bfloat16, device=dev), torch.ones(70, 272, dtype=torch.bfloat16, device=dev)
     d[69, 263], y[3, 270] = float("nan"), float("inf")
