@@ -214,42 +214,13 @@ CHAIN_NORM, CHAIN_GATED, CHAIN_SWIGLU, CHAIN_RESNORM = 0, 1, 2, 3
 def _chain_bwd(kind, x, aux, w1, eps1, w2, eps2, dy, dres=None, dx=None, daux=None):
     """mmf_chain_bwd over [M, K] operands (column slices keep their row stride; dy [norms, M, K]):
     (dx, daux, y_quant [norms, M, K], weight gradients [(w1) + norms, K])."""
-    lib = L.load()
-    m, k = x.shape
-    n = len(w2)
-    dx = torch.empty(m, k, dtype=x.dtype, device=x.device) if dx is None else dx
-    rows = n + (kind != CHAIN_SWIGLU)
-    y = torch.empty(n, m, k, dtype=x.dtype, device=x.device)
-    part = torch.empty(lib.mmf_chain_bwd_groups(m) * rows * k, dtype=torch.float32, device=x.device)
-    dw = torch.empty(rows, k, dtype=w2[0].dtype, device=x.device)
-    w2p = (ctypes.c_void_p * 3)(*[w.data_ptr() for w in w2])
-    dyp = (ctypes.c_void_p * 3)(*[d.data_ptr() for d in dy])
-    L.check(lib.mmf_chain_bwd(kind, x.data_ptr(), x.stride(0), L.ptr(aux), aux.stride(0) if aux is not None else 0, L.ptr(w1), eps1, n, w2p,
-                              eps2, dyp, k, L.ptr(dres), dx.data_ptr(), dx.stride(0), L.ptr(daux),
-                              daux.stride(0) if daux is not None else 0, y.data_ptr(), part.data_ptr(), dw.data_ptr(), m, k,
-                              L.dtype_id(x.dtype), L.dtype_id(dw.dtype), L.stream()), "mmf_chain_bwd")
+    dx, y, dw = L.native().chain_backward(kind, x, aux, w1, eps1, tuple(w2), eps2, tuple(dy), dres, dx, daux, L.check)
     return dx, daux, y, dw
 
 
-def _dequantised(pw, dtype):
-    """t * wdeq of a packed weight as a dense [N, K] matrix (fusedbitnet.py:456-458), contiguous along N: dout @ W_q contracts there."""
-    w = torch.empty(pw.k, pw.n, dtype=dtype, device=pw.packed.device)
-    L.check(L.load().mmf_unpack_dequant_t(pw.packed.data_ptr(), pw.wdeq.data_ptr(), pw.seg_rows, pw.n, pw.k, w.data_ptr(), L.dtype_id(dtype),
-                                          L.stream()), "mmf_unpack_dequant_t")
-    return w.t()
-
-
 def _dense_weight(pw, dtype):
-    """The dense ternary weights for dout @ W_q, stored as that product and their unpacking take least time together.
-
-    16-bit products run faster with the contraction contiguous (_dequantised).  Single-precision ones take the same time either way, and
-    rows are written faster than columns: a 1024-wide step's 13 unpackings 126 us stored [K, N], 103 us stored [N, K]."""
-    if dtype != torch.float32:
-        return _dequantised(pw, dtype)
-    w = torch.empty(pw.n, pw.k, dtype=dtype, device=pw.packed.device)
-    L.check(L.load().mmf_unpack_dequant(pw.packed.data_ptr(), pw.wdeq.data_ptr(), pw.seg_rows, pw.n, pw.k, w.data_ptr(), L.dtype_id(dtype),
-                                        L.stream()), "mmf_unpack_dequant")
-    return w
+    """The dense ternary weights [N, K] for dout @ W_q."""
+    return L.native().dense_weight(pw.packed, pw.wdeq, pw.seg_rows, pw.n, pw.k, dtype, L.check)
 
 
 def _turns(dout, y):

@@ -1059,7 +1059,7 @@ int launch_mfma(MfmaArgs a, hipStream_t s) {
 // 1024 -> 5632, 300 rows 6.0 / 8.4, 700 9.9 / 9.4; 2048 -> 2048, 1203 rows 10.9 / 11.4, 1395 12.1 / 11.3.
 // Over 389 shapes, 66 to 8000 rows, the choice costs 0.01 % against the best of the three on average, 15 % at most (377 x 1536 -> 4608: 1.2 us).
 //   narrow tiles   (64 x 128, split like the others) where they give every CU at most one, or three in all; with rows of 2560 to 6144 also instead of a
-//                  split one on nearly every CU (481 to 512 of them: over 73 shapes 1.3 % less on average, from 10 % less to 4 % more, most where their last row of
+//                  split one on nearly every CU (481 to 512 of them: over 72 shapes 1.4 % less on average, from 10 % less to 4 % more, most where their last row of
 //                  tiles is nearly empty; rows of 6912 0.6 % more).  us, best of the others / narrow: 5632 -> 2048, 700 rows 15.6 / 12.8, 1001 (256 narrow tiles) 19.0 / 13.9, 1377 (352)
 //                  20.1 / 20.5, 2002 (512) 24.5 / 23.2, 2400 (608) 32.9 / 29.2; 2048 -> 2048, 830 rows 8.3 / 7.4, 1001 9.2 / 7.8, 1200 (304) 10.4 / 10.8, 2002
 //                  11.7 / 11.8; 2816 -> 1024, 1600 rows 11.9 / 8.4, 4022 (504) 16.4 / 14.5, 4100 (520) 19.7 / 17.4; 2560 -> 2560, 711 rows 11.3 / 8.4, 1491 (480) 13.0 / 13.2,

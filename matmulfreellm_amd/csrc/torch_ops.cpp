@@ -9,6 +9,7 @@
 #include <ATen/ATen.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -36,6 +37,17 @@ struct OnDevice {
 };
 struct Failed { int rc; const char* what; };
 void check(int rc, const char* what) { if (rc != 0) throw Failed{rc, what}; }
+// null, with the exception that `raise`, a caller's function of (code, name), makes of a failure
+PyObject* failed(const Failed& f, PyObject* raise) {
+    Py_XDECREF(PyObject_CallFunction(raise, "is", f.rc, f.what));
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, f.what);
+    return nullptr;
+}
+// None is an undefined tensor
+bool tensor_or_none(PyObject* o, Tensor& t) {
+    if (THPVariable_Check(o)) t = THPVariable_Unpack(o);
+    return THPVariable_Check(o) || o == Py_None;
+}
 
 struct NoGil {
     PyThreadState* state = PyEval_SaveThread();
@@ -153,9 +165,7 @@ PyObject* scan(PyObject*, PyObject* const* args, Py_ssize_t count) {
         NoGil nogil;
         out = ScanFn::apply(x, g, h0, final_state, chunk);
     } catch (const Failed& f) {
-        Py_XDECREF(PyObject_CallFunction(args[5], "is", f.rc, f.what));
-        if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, f.what);
-        return nullptr;
+        return failed(f, args[5]);
     }
     PyObject* o = THPVariable_Wrap(out[0]);
     PyObject* last = Py_None;
@@ -193,7 +203,9 @@ Chained chain(int kind, const Tensor& x, const Tensor& aux, const Tensor& w1, do
 }
 
 struct Packed { Tensor codes, wdeq; int64_t seg_rows, n, k; };
-// t * wdeq as a dense [N, K] matrix for dout @ W_q (autograd.py's _dense_weight): 16-bit types contiguous along N
+// t * wdeq as a dense [N, K] matrix for dout @ W_q (fusedbitnet.py:456-458), stored as that product and its unpacking take least time together.  16-bit
+// products run faster with the contraction, N, contiguous.  Single-precision ones take the same time either way, and rows are written faster than
+// columns: a 1024-wide step's 13 unpackings 126 us stored [K, N], 103 us stored [N, K].
 Tensor dense(const Packed& p, const at::TensorOptions& like) {
     const auto type = c10::typeMetaToScalarType(like.dtype());
     const bool rows = type == at::kFloat;
@@ -202,6 +214,64 @@ Tensor dense(const Packed& p, const at::TensorOptions& like) {
                                                              stream_of(w)),
           rows ? "mmf_unpack_dequant" : "mmf_unpack_dequant_t");
     return rows ? w : w.t();
+}
+
+// (kind, x, aux or None, w1 or None, eps1, norm weights, eps2, their gradients, dres or None, dx or None, daux or None, what raises for a return code) ->
+// (dx, y [norms, M, K], weight gradients [(w1) + norms, K]); daux is written where it is given
+PyObject* chain_backward(PyObject*, PyObject* const* args, Py_ssize_t count) {
+    HANDLE_TH_ERRORS
+    Tensor x, aux, w1, dres, dx, daux, w2[3], dy[3];
+    bool fits = count == 12 && THPVariable_Check(args[1]) && tensor_or_none(args[1], x) && tensor_or_none(args[2], aux) && tensor_or_none(args[3], w1) &&
+                PyTuple_Check(args[5]) && PyTuple_Check(args[7]) && tensor_or_none(args[8], dres) && tensor_or_none(args[9], dx) && tensor_or_none(args[10], daux);
+    const Py_ssize_t n = fits ? PyTuple_GET_SIZE(args[5]) : 0;
+    fits = fits && n >= 1 && n <= 3 && PyTuple_GET_SIZE(args[7]) == n && x.dim() == 2;
+    for (Py_ssize_t i = 0; fits && i < n; ++i) {
+        PyObject *w = PyTuple_GET_ITEM(args[5], i), *d = PyTuple_GET_ITEM(args[7], i);
+        fits = THPVariable_Check(w) && THPVariable_Check(d) && tensor_or_none(w, w2[i]) && tensor_or_none(d, dy[i]);
+    }
+    if (!fits) {
+        PyErr_SetString(PyExc_TypeError, "chain_backward takes (kind, x, aux, w1, eps1, w2, eps2, dy, dres, dx, daux, check)");
+        return nullptr;
+    }
+    const int kind = (int)PyLong_AsLong(args[0]);
+    const double eps1 = PyFloat_AsDouble(args[4]), eps2 = PyFloat_AsDouble(args[6]);
+    if (PyErr_Occurred()) return nullptr;
+    Chained c;
+    try {
+        NoGil nogil;
+        OnDevice on(x.get_device());
+        c = chain(kind, x, aux, w1, eps1, at::ArrayRef<Tensor>(w2, n), eps2, at::ArrayRef<Tensor>(dy, n), dres, dx, daux);
+    } catch (const Failed& f) {
+        return failed(f, args[11]);
+    }
+    PyObject *a = THPVariable_Wrap(c.dx), *b = THPVariable_Wrap(c.y), *w = THPVariable_Wrap(c.dw), *r = PyTuple_Pack(3, a, b, w);
+    Py_DECREF(a);
+    Py_DECREF(b);
+    Py_DECREF(w);
+    return r;
+    END_HANDLE_TH_ERRORS
+}
+
+// (codes, wdeq, seg_rows, n, k, dtype, what raises for a return code) -> [n, k]
+PyObject* dense_weight(PyObject*, PyObject* const* args, Py_ssize_t count) {
+    HANDLE_TH_ERRORS
+    if (count != 7 || !THPVariable_Check(args[0]) || !THPVariable_Check(args[1]) || !THPDtype_Check(args[5])) {
+        PyErr_SetString(PyExc_TypeError, "dense_weight takes (codes, wdeq, seg_rows, n, k, dtype, check)");
+        return nullptr;
+    }
+    const Packed p{THPVariable_Unpack(args[0]), THPVariable_Unpack(args[1]), PyLong_AsLongLong(args[2]), PyLong_AsLongLong(args[3]), PyLong_AsLongLong(args[4])};
+    if (PyErr_Occurred()) return nullptr;
+    const auto type = reinterpret_cast<THPDtype*>(args[5])->scalar_type;
+    Tensor w;
+    try {
+        NoGil nogil;
+        OnDevice on(p.codes.get_device());
+        w = dense(p, p.codes.options().dtype(type));
+    } catch (const Failed& f) {
+        return failed(f, args[6]);
+    }
+    return THPVariable_Wrap(std::move(w));
+    END_HANDLE_TH_ERRORS
 }
 
 // dout^T @ y of a block's BitLinears, [M, N] gradients and [M, K] de-quantised inputs; undefined where a gradient is.
@@ -360,9 +430,7 @@ PyObject* block_backward(PyObject*, PyObject* const* args, Py_ssize_t count) {
         grads[5] = down.dw;
         for (int i = 0; i < 6; ++i) grads[6 + i] = dw[i];
     } catch (const Failed& f) {
-        Py_XDECREF(PyObject_CallFunction(args[7], "is", f.rc, f.what));
-        if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, f.what);
-        return nullptr;
+        return failed(f, args[7]);
     }
     PyObject* r = PyTuple_New(12);
     for (int i = 0; r && i < 12; ++i) {
@@ -482,6 +550,8 @@ PyMethodDef methods[] = {
     {"structure_holds", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(structure_holds)), METH_FASTCALL, nullptr},
     {"parameters_hold", parameters_hold, METH_O, nullptr},
     {"bitlinear", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(bitlinear)), METH_FASTCALL, nullptr},
+    {"chain_backward", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(chain_backward)), METH_FASTCALL, nullptr},
+    {"dense_weight", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(dense_weight)), METH_FASTCALL, nullptr},
     {"block_backward", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(block_backward)), METH_FASTCALL, nullptr},
     {"scan", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(scan)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};

@@ -5,11 +5,19 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
+def _dequantised(pw, dtype):
+    """[N, K], stored [K, N]."""
+    from matmulfreellm_amd import _lib as L
+    w = torch.empty(pw.k, pw.n, dtype=dtype, device=pw.packed.device)
+    L.check(L.load().mmf_unpack_dequant_t(pw.packed.data_ptr(), pw.wdeq.data_ptr(), pw.seg_rows, pw.n, pw.k, w.data_ptr(), L.dtype_id(dtype),
+                                          L.stream()), "mmf_unpack_dequant_t")
+    return w.t()
+
+
 @pytest.mark.parametrize("n,k,seg", [(1, 4, 1), (7, 100, 7), (33, 131, 33), (96, 1024, 32), (40, 2056, 20), (64, 4100, 64)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_dense_weights_equal_unpacked_codes_times_scale(dev, n, k, seg, dtype):
     import matmulfreellm_amd.functional as F
-    from matmulfreellm_amd.autograd import _dequantised
     torch.manual_seed(n + k)
     pw = F.ternarize_pack(torch.randn(n, k, device=dev))
     codes = F.unpack_ternary(pw).float()
@@ -41,7 +49,6 @@ def test_both_layouts_of_the_dense_weights_hold_the_same_values(dev, n, k, seg, 
     """[N, K] and [K, N], at the edges of the row vectors, the workgroups' columns, the 16-input pieces and the segments."""
     import matmulfreellm_amd._lib as L
     import matmulfreellm_amd.functional as F
-    from matmulfreellm_amd.autograd import _dequantised
     torch.manual_seed(n * k)
     pw = F.ternarize_pack(torch.randn(n, k, device=dev))
     pw.wdeq, pw.seg_rows = torch.rand(-(-n // seg), device=dev) + 0.5, seg
