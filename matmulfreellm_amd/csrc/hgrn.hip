@@ -187,10 +187,10 @@ __global__ __launch_bounds__(64 * NW) void hgrn_recurrent_pipelined_kernel(const
 // a 128-byte line run on one XCD).  A turn requests and stores the same number of vectors whatever the tile, past the sequence's
 // ends through resources without records: the compiler then waits for one set of loads by count, where a store or load under a
 // branch made it wait for everything in flight, a trip to memory in every turn.  Wave 0 reads its steps a group ahead into two
-// sets of registers in turn, without copies between them.  bf16 in us, against branches, copies and the exact gate math: 8 x 2048 x 2048
-// 95 -> 63 (201 MB: 3.2 TB/s), 16 x 900 x 1024 42 -> 28, 2 x 1001 x 2048 24 -> 17, 3 x 459 x 2048 16 -> 12, 64 x 32 x 2048 23 -> 17, 4 x 300 x 1024
-// 9.5 -> 7.1, 1 x 77 x 1024 5.1 -> 4.7.  With few columns time is wave 0's own, 12 ns a step (1 x 2048 x 1024 40 -> 28; half as many channels a
-// workgroup: 28).  hgrn_gate_scan_kernel takes single channels (odd widths and strides, rows beyond 256 KiB), the kernel behind it pairs.
+// sets of registers in turn, without copies between them.  bf16 in us, against branches, copies and the exact gate math, operands in the last-level
+// cache: 8 x 2048 x 2048 95 -> 63, 16 x 900 x 1024 42 -> 28, 2 x 1001 x 2048 24 -> 17, 3 x 459 x 2048 16 -> 12, 64 x 32 x 2048 23 -> 17, 4 x 300 x 1024
+// 9.5 -> 7.1, 1 x 77 x 1024 5.1 -> 4.7; in memory 8 x 2048 x 2048 takes 74 to 79.  With few columns time is wave 0's own, 12 ns a step (1 x 2048 x 1024
+// 40 -> 28; half as many channels a workgroup: 28).  hgrn_gate_scan_kernel takes single channels (odd widths and strides, rows beyond 256 KiB), the kernel behind it pairs.
 struct GateScanArgs {
     const void* i; const void* f;       // rows [B * T, D], row strides ldi, ldf
     const float* lb; const uint8_t* mask;
@@ -385,11 +385,12 @@ __global__ __launch_bounds__(1024) void hgrn_gate_scan_kernel(GateScanArgs a) {
 
 // The same where rows and pointers allow two channels at once: a lane takes a pair of channels of one step, so a turn is one request each for i, f
 // and the store, and one LDS vector each way, instead of two, and the resources stand for the whole sequence: offsets advance by a vector add where the
-// bases of every tile took some 70 scalar operations a turn.  NP waves feed the one that walks: 15, or 8 for up to 512 steps, whose tiles of 64
-// are sooner ready.  us, single channels and pairs: 8 x 2048 x 2048 bf16 73.9 and 67.8 (2.97 TB/s), 8 x 512 x 2048 22.8 and 19.3, 16 x 1000 x 1024 38.1 and
-// 32.1, 64 x 32 x 2048 17.3 and 15.9, 3 x 459 x 2048 fp16 13.3 and 12.4, 1 x 77 x 1024 4.6 and 4.5; 1 x 2000 x 1024 28.3 and 28.1, the walk itself: 12.5 ns a step, two
-// dependent operations and one LDS access.  Where there are many columns the vector units bound it: with neither the test of the near forms nor
-// their fall-back 8 x 2048 x 2048 takes 42 us, without gate math 38.
+// bases of every tile took some 70 scalar operations a turn.  NP waves feed the one that walks: 15, or 8 for up to 512 steps in 16-channel workgroups,
+// whose tiles of 64 are sooner ready.  us, single channels / pairs, operands in memory (four sets in turn) and in the last-level cache: 8 x 2048 x 2048 bf16 79.2 / 58.0
+// (3.5 TB/s) and 56.4 / 47.7, 16 x 1000 x 1024 36.1 / 30.5 and 26.6 / 25.4; about the same in both: 8 x 512 x 2048 16.8 / 15.8, 64 x 32 x 2048 16.6 / 14.5, 3 x 459 x 2048
+// fp16 12.4 / 10.9, 1 x 77 x 1024 5.6 / 5.0; 1 x 2000 x 1024 27.6 / 27.4, the walk itself: 12.5 ns a step, two dependent operations and one LDS access.
+// Boxes differ by up to 17 % (8 x 2048 x 2048 in memory 73.9 / 67.8 on another).  Where there are many columns the vector units bound it: there, with
+// neither the test of the near forms nor their fall-back it took 42 us, without gate math 38.
 template <typename T, int CPW, int NP, bool MASK>
 __global__ __launch_bounds__(64 * (NP + 1)) void hgrn_gate_scan_pair_kernel(GateScanArgs a) {
     constexpr int CP = CPW / 2, SPW = 64 / CP, TT = NP * SPW, U = TT % 20 == 0 ? 10 : TT % 16 == 0 ? 8 : 5, e = (int)sizeof(T), kRsrcFlags = 0x00020000;
